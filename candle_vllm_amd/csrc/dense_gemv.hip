@@ -17,8 +17,10 @@
 // by index arithmetic here.
 #include "common.h"
 #include "scratch.h"
+#include "gemm_tile.h"
 #include "../../include/mi355_vllm.h"
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <utility>
 
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
@@ -802,13 +804,18 @@ static int dense_launch_gj(const DenseArgs& a, int gj, int nw, hipStream_t st) {
 }
 
 // ---- the 1..4-token launch of 4-bit weights (dense_small_kernel): -4 = this shape stays on dense_kernel
-static int g_tune_gemm_min_t = 96;     // tuning key 36: tokens from which a 16-bit projection takes the 128 x 128 MFMA GEMM
+// Tokens from which a 16-bit projection takes the MFMA GEMM of gemm_tile.h (tuning key 36; from 17 where the launch has 768 row tiles or pairs).
+// us per launch, streaming kernels against the GEMM: gate/up 28672 x 4096 T = 16 43.9 / 42.3, 32 47.0 / 42.3, 40 90.3 / 43.1 (two sweeps over
+// the weights from 33 tokens), 64 96.5 / 44.0; down 4096 x 14336 T = 32 28.5 / 28.6, 40 31.0 / 29.5, 64 64.9 / 32.3; wo 4096 x 4096
+// T = 16 9.3 / 13.7, 32 12.3 / 14.0, 40 16.1 / 13.7; 12288 x 2048 T = 32 17.0 / 12.9; at 5 .. 16 tokens either may win (16384 pairs of 3072: 18.7 / 22.1)
+enum { DENSE_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_T = 96 };
+static int g_tune_gemm_min_t = DENSE_GEMM_MIN_T;
 static int g_tune_gptq_gemm_off = 0;   // tuning key 39: 1 = 4-bit prompt steps run the decode kernel in 64-token chunks (A/B)
 static int g_tune_wide_nw = 4;         // tuning key 38: waves (row tiles) per workgroup of dense_wide_kernel: 2 | 4
 static int g_tune_wide_off = 0;        // tuning key 37: 1 = 16-bit launches with many row tiles stay on dense_kernel (A/B)
 static int g_tune_small_nw = 0;        // tuning key 30: waves per workgroup (0 = chosen from the k-blocks)
 static int g_tune_small_nw_big = 0;    // tuning key 35: the same for K > 8192
-static int g_tune_gemm_tall = 0;       // tuning key 30 bit 32 (round 4; measured SLOWER, stays off: bf16 prompt step of Llama-3-8B 53.7 k -> 51.5 k tok/s): the 256-token tile of the 16-bit prompt GEMM where it fills the chip twice
+static int g_tune_gemm_tall = 0;       // tuning key 30 bits 32, 64: the 16-bit prompt GEMM always takes its 256 x 256 tile and never splits K
 static int g_tune_small_off = 0;       // tuning key 31: 1 = keep 1..4 tokens on dense_kernel (A/B measurements)
 static int g_tune_gptq_wide_nosplit = 0;   // tuning key 30 bit 256: gate/up pairs of the 5..32-token 4-bit launches stay on one wave each (A/B)
 static int g_tune_gptq_wide_off = 0;   // tuning key 30 bit 128: 1 = 5..64-token launches of tiled 4-bit weights stay on dense_kernel (A/B; round 5)
@@ -816,7 +823,7 @@ static int g_tune_small_norope = 0;    // tuning key 34: 1 = RoPE and the cache 
 static int g_tune_small_nonorm = 0;    // tuning key 32: 1 = never norm on the way in (the host layer launches the norm separately)
 // tuning key 30 (product): bit mask of folded launches switched OFF -- 1 = the 1..4-token 4-bit kernel, 2 = no norm on the way in,
 // 4 = RoPE and the cache write in their own launch, 8 = the LDS-shared-activation 16-bit kernel, 16 = the one-pass 4-bit prompt GEMM;
-// 32 (switches ON) = the 256-token tile of the 16-bit prompt GEMM where it fills the chip twice, 32 | 64 = wherever that GEMM runs (tests).
+// 32, 64 (switch ON) = the 256 x 256 tile of the 16-bit prompt GEMM wherever that GEMM runs (tests).
 // Probe builds: 33 / 35 waves per workgroup of the 1..4-token kernel (hidden-sized K / long K), 36 tokens from which 16-bit
 // projections take the MFMA GEMM, 38 waves per workgroup of the LDS-shared-activation kernel.
 void mi355_dense_set_small(int key, int v) {
@@ -1074,18 +1081,158 @@ static int dense_dispatch(const DenseArgs& a, int wtype, int dt, hipStream_t st)
 }
 
 // ---- prompt steps (T >= 96, dense 16-bit weights): the matmul is compute-bound -> a hand-written MFMA GEMM
-// (`Linear::forward` on prompt chunks, linear.rs:124-172; packed gate_up of mlp.rs:324-352,440-458).  Both operands are
-// k-contiguous ("TN": x [T,K], W [N,K]), so a 16 x 16 x 32 A / B fragment is 16 contiguous bytes of a row:
-//   * workgroup tile 128 tokens x 128 weight rows, 4 waves as 2 x 2, wave tile 64 x 64 (4 x 4 accumulators), K in steps of 64;
-//   * both tiles go global -> LDS by DMA (`global_load_lds_dwordx4`, inline asm so that hipcc neither counts nor drains it:
-//     the DMA of K-step t+1 is in flight while step t is multiplied; one counted wait + one barrier per step), two LDS buffers;
-//   * LDS rows are 128 B (64 k): the 16-byte slot c of row r is stored at slot c ^ (r & 7) -- the swizzle is applied to the
-//     lane's GLOBAL source address (the DMA destination is lane-linear), fragment reads are conflict-free ds_read_b128;
+// (`Linear::forward` on prompt chunks, linear.rs:124-172; packed gate_up of mlp.rs:324-352,440-458) around the main loop of gemm_tile.h.
 //   * candle's rounding chain in the epilogue, from the f32 accumulators: round to the dtype, + bias (rounded), then
 //     + residual (rounded) or silu(gate) rounded * up rounded -- no separate chain kernel, no f32 / 16-bit staging of y;
-//   * SILU_MUL: the B tile holds 64 gate rows and the 64 matching up rows (pair_offset apart in W), every wave owns both halves
-//     of its 32 output columns, so gate and up meet in registers.
-// rocBLAS is no longer used on this path (round 2 called rocblas_gemm_ex here).
+//   * SILU_MUL: the weight tile holds BN / 2 gate rows and the matching up rows (pair_offset apart in W), fragments j and j + NF / 2 of a
+//     wave are the two halves of the same output columns, so gate and up meet in registers;
+//   * up to three matrices over one x (q, k, v) are one launch: their column tiles follow each other.
+struct DenseGemm3 {
+    DenseArgs a[3];
+    int32_t tiles[3], n_m;               // column tiles of each matrix (0: none), token tiles
+    int32_t splits, units_per_split;     // K in `splits` ranges (one matrix only) whose partial sums go to `part` [splits][token][N]
+    float* part;
+};
+// candle's rounding of one value by the hardware's conversion (the same round-to-nearest-even; a NaN keeps its sign)
+template <int DT> __device__ __forceinline__ uint32_t gemm_pack(float lo, float hi) {
+    if constexpr (DT == MI355_DTYPE_BF16) return cvt_pk_bf16(lo, hi);
+    else return (uint32_t)f2h<DT>(lo) | (uint32_t)f2h<DT>(hi) << 16;
+}
+template <int DT> __device__ __forceinline__ float gemm_rnd(float v) {
+    if constexpr (DT == MI355_DTYPE_BF16) return __uint_as_float(cvt_pk_bf16(v, 0.f) << 16);
+    else return rnd<DT>(v);
+}
+template <int DT, int EPI, int WM, int WN, int MF, int NF, int S, bool TILED>
+__global__ void __launch_bounds__(512, 2) dense_gemm_kernel(const DenseGemm3 g) {
+    typedef GemmTile<DT, WM, WN, MF, NF, S, TILED> Tile;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    const int n_tiles = g.n_m * (g.tiles[0] + g.tiles[1] + g.tiles[2]);
+    const int split = blockIdx.x / n_tiles;                              // the splits of a tile are as far apart as they can be: their reads do not meet
+    const GtPlace at = gt_place(blockIdx.x - split * n_tiles, g.n_m, g.tiles[0] + g.tiles[1] + g.tiles[2]);
+    int bn = at.n;
+    const int which = bn < g.tiles[0] ? 0 : bn < g.tiles[0] + g.tiles[1] ? 1 : 2;
+    if (which > 0) bn -= g.tiles[0];
+    if (which > 1) bn -= g.tiles[1];
+    const DenseArgs& a = g.a[which];
+    Tile tile(smem);
+    constexpr bool silu = EPI == MI355_EPI_SILU_MUL;
+    const int t0 = at.m * Tile::BM;
+    const int n_cols = silu ? a.pair_offset : a.N;                      // output columns
+    const int c0 = bn * (silu ? Tile::BN / 2 : Tile::BN);               // first output column of this tile
+    // weight row held by row j of the tile's weight side (clamped: rows beyond the matrix are multiplied and never stored)
+    auto wrow = [&](int j) {
+        int n = c0 + j, lim = a.N - 1;
+        if (silu) {
+            const int w = j / (NF * 16), in = j % (NF * 16), up = in >= NF * 8;
+            n = c0 + w * (NF * 8) + (up ? in - NF * 8 : in);
+            lim = a.pair_offset - 1;
+            n = (n > lim ? lim : n) + (up ? a.pair_offset : 0);
+            return n;
+        }
+        return n > lim ? lim : n;
+    };
+    const uint8_t* wb = static_cast<const uint8_t*>(a.w);
+    const uint8_t* a_base = static_cast<const uint8_t*>(a.x) + (size_t)t0 * a.ldx * 2;
+    uint32_t a_off[Tile::AR], b_off[Tile::BR];
+    const uint8_t* b_base[Tile::BR];
+#pragma unroll
+    for (int r = 0; r < Tile::AR; ++r) {
+        int row = tile.stage_row(r);
+        if (row > a.T - 1 - t0) row = a.T - 1 - t0;
+        a_off[r] = (uint32_t)row * (uint32_t)a.ldx * 2u + tile.stage_chunk();
+    }
+#pragma unroll
+    for (int r = 0; r < Tile::BR; ++r) {
+        if constexpr (TILED) {                                          // 8 KiB per (row tile, 256 k), 2 KiB per unit, 1 KiB per fragment
+            b_base[r] = wb + (size_t)(wrow(16 * tile.stage_tile(r)) >> 4) * (a.K >> 8) * 8192 + tile.stage_frag() * 1024;
+            b_off[r] = tile.lane * 16u;
+        } else {
+            const int first = wrow(8 * (tile.wave + 8 * r)), row = wrow(tile.stage_row(r));
+            b_base[r] = wb + (size_t)first * a.ldw * 2;
+            b_off[r] = (uint32_t)(row - first) * (uint32_t)a.ldw * 2u + tile.stage_chunk();
+        }
+    }
+    constexpr uint32_t b_step = TILED ? 2048u : 128u;
+    int units = a.K / 64;
+    if (g.splits > 1) {
+        const int u0 = split * g.units_per_split;
+        units = min(units - u0, g.units_per_split);
+        a_base += (size_t)u0 * 128;
+#pragma unroll
+        for (int r = 0; r < Tile::BR; ++r) b_base[r] += (size_t)u0 * b_step;
+    }
+    tile.run(a_base, a_off, b_base, b_off, b_step, units);
+    if (g.splits > 1) {                                                  // gptq_wide_epilogue_kernel adds the ranges in their order and rounds
+        float* part = g.part + (size_t)split * a.T * a.N;
+#pragma unroll
+        for (int i = 0; i < MF; ++i) {
+            const int t = t0 + tile.row(i);
+            if (t >= a.T) continue;
+#pragma unroll
+            for (int j = 0; j < NF; ++j) {
+                int col = c0 + tile.col(j);
+                if (silu) col = c0 + tile.wn * (NF * 8) + (j % (NF / 2)) * 16 + 4 * (tile.lane >> 4);
+                if (col >= n_cols) continue;
+                if (silu && j >= NF / 2) col += a.pair_offset;
+                *reinterpret_cast<f32x4_t*>(part + (size_t)t * a.N + col) = tile.acc[i][j];
+            }
+        }
+        return;
+    }
+    // ---- epilogue: four consecutive columns of one token per fragment
+    const uint16_t* bias = static_cast<const uint16_t*>(a.bias);
+    const uint16_t* resid = static_cast<const uint16_t*>(a.resid);
+    uint16_t* out = static_cast<uint16_t*>(a.out);
+    const bool wide = !((a.ldo & 3) | (n_cols & 3)) && !(((uintptr_t)out | (uintptr_t)resid) & 7);
+#pragma unroll
+    for (int i = 0; i < MF; ++i) {
+        const int t = t0 + tile.row(i);
+        if (t >= a.T) continue;
+#pragma unroll
+        for (int j = 0; j < (silu ? NF / 2 : NF); ++j) {
+            float o[4];
+            int col;
+            if (silu) {
+                col = c0 + tile.wn * (NF * 8) + j * 16 + 4 * (tile.lane >> 4);
+                if (col >= n_cols) continue;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float gv = gemm_rnd<DT>(tile.acc[i][j][v]), u = gemm_rnd<DT>(tile.acc[i][(j + NF / 2) % NF][v]);
+                    if (bias && col + v < n_cols) { gv = gemm_rnd<DT>(gv + h2f<DT>(bias[col + v])); u = gemm_rnd<DT>(u + h2f<DT>(bias[a.pair_offset + col + v])); }
+                    o[v] = gemm_rnd<DT>(gv / (1.f + __expf(-gv))) * u;        // silu(gate) * up (mlp.rs:457); the store rounds
+                }
+            } else {
+                col = c0 + tile.col(j);
+                if (col >= n_cols) continue;
+                uint16_t rr[4];
+                if (EPI == MI355_EPI_RESID) {
+                    const uint16_t* rp = resid + (size_t)t * a.ldo + col;
+                    if (wide) {
+                        const uint2 r2 = *reinterpret_cast<const uint2*>(rp);
+                        rr[0] = (uint16_t)r2.x; rr[1] = (uint16_t)(r2.x >> 16); rr[2] = (uint16_t)r2.y; rr[3] = (uint16_t)(r2.y >> 16);
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) rr[v] = col + v < n_cols ? rp[v] : (uint16_t)0;
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    o[v] = gemm_rnd<DT>(tile.acc[i][j][v]);
+                    if (bias && col + v < n_cols) o[v] = gemm_rnd<DT>(o[v] + h2f<DT>(bias[col + v]));
+                    if (EPI == MI355_EPI_RESID) o[v] = o[v] + h2f<DT>(rr[v]);
+                }
+            }
+            uint16_t* op = out + (size_t)t * a.ldo + col;
+            if (wide) {
+                *reinterpret_cast<uint2*>(op) = make_uint2(gemm_pack<DT>(o[0], o[1]), gemm_pack<DT>(o[2], o[3]));
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) if (col + v < n_cols) op[v] = (uint16_t)gemm_pack<DT>(o[v], 0.f);
+            }
+        }
+    }
+}
+
 template <int NP>
 __device__ __forceinline__ void dgemm_dma(const uint8_t* gsrc_lane, uint32_t lds_dst) {
     // NP x 1 KiB: lane l copies 16 B from its own source address (+ i * row_stride handled by the caller through separate calls)
@@ -1095,145 +1242,7 @@ __device__ __forceinline__ void dgemm_dma(const uint8_t* gsrc_lane, uint32_t lds
 }
 
 #define DG_BM 128
-#define DG_BN 128
 #define DG_BK 64
-// WR = wave rows: 2 = 128 tokens x 128 weight rows per workgroup (4 waves, two workgroups per CU), 4 = 256 x 128 (8 waves, one workgroup
-// per CU; round 4): at 128 x 128 the tile moves 32 KiB through L2 -> LDS per 2.1 MFLOP -- 15 B per kFLOP, ~10 TB/s at the measured 650
-// TFLOP/s, which is what the L2 -> CU path carried in every other measurement of this chip -- the taller tile moves 11.4.  Measured (round 4,
-// one box, alternated, T = 2048): 53.7 k tok/s with the 128 x 128 tile, 51.5 k with 256 x 128: L2 traffic is not what bounds it; the tall tile
-// stays a tested option (tuning key 30 bit 32; bit-identical outputs, tests/test_gpu_linear.py).  A ring of three K steps behind counted
-// waits (one workgroup per CU then) was measured too and removed: 53.0 k -> 41.2 k at 128 x 128, 47.5 k at 256 x 128 -- this GEMM lives on its
-// two workgroups per CU, not on prefetch depth.
-template <int DT, int WR = 2>
-__global__ void __launch_bounds__(128 * WR, WR == 2 ? 2 : 1) dense_gemm_kernel(const DenseArgs a) {
-    constexpr int BM = 64 * WR, NTHR = 128 * WR, AROUNDS = BM / (NTHR / 8), BROUNDS = DG_BN / (NTHR / 8);   // rows per staging round = NTHR / 8
-    constexpr uint32_t A_BYTES = BM * 128u, STAGE = A_BYTES + 16384u;
-    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];   // [2 buffers][A 16 / 32 KiB | B 16 KiB]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave >> 1, wc = wave & 1;
-    const int m16 = lane & 15, kg = lane >> 4;
-    const bool silu = a.epi == MI355_EPI_SILU_MUL;
-    // token tiles fastest: the workgroups that run together share their weight tile through L2
-    const int bm = blockIdx.x, bn = blockIdx.y;
-    const int t0 = bm * BM;
-    const int n_cols = silu ? a.pair_offset : a.N;                      // output columns
-    const int c0 = bn * (silu ? 64 : DG_BN);                            // first output column of this tile
-    // weight row held by LDS B-row j
-    auto wrow = [&](int j) {
-        int n = silu ? (j < 64 ? c0 + j : a.pair_offset + c0 + (j - 64)) : c0 + j;
-        const int lim = silu ? (j < 64 ? a.pair_offset - 1 : a.N - 1) : a.N - 1;
-        return n > lim ? lim : n;                                       // clamped: columns beyond the matrix are computed and never stored
-    };
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) void*)smem);
-    const uint8_t* xb = static_cast<const uint8_t*>(a.x);
-    const uint8_t* wb = static_cast<const uint8_t*>(a.w);
-    // staging: a round covers NTHR / 8 LDS rows (8 threads = the 8 slots of a row; one wave = 8 rows = 1 KiB); this thread's row / slot inside
-    // the round.  A takes AROUNDS rounds (BM rows), B BROUNDS (128 rows)
-    constexpr int RROWS = NTHR / 8, NWV = NTHR / 64;
-    const int srow = tid >> 3, sslot = tid & 7;
-    const uint8_t* asrc[AROUNDS];
-    const uint8_t* bsrc[BROUNDS];
-#pragma unroll
-    for (int r = 0; r < AROUNDS; ++r) {
-        const int row = RROWS * r + srow;
-        int t = t0 + row;
-        if (t > a.T - 1) t = a.T - 1;
-        asrc[r] = xb + ((size_t)t * a.ldx) * 2 + (size_t)((sslot ^ (row & 7)) * 16);
-    }
-#pragma unroll
-    for (int r = 0; r < BROUNDS; ++r) {
-        const int row = RROWS * r + srow;
-        if (a.wtiled) {
-            // the tiled image IS the fragment order: the B tile in LDS is a verbatim copy -- [n-tile 8][fragment 2][lane 64][16 B] --
-            // and every DMA instruction of a wave copies one contiguous KiB (piece p = NWV r + wave: n-tile p / 2, fragment p % 2 of
-            // this K step; 2 KiB per (n-tile, K step)).  (A first version kept the row-major LDS layout and gathered 16-byte chunks:
-            // 64 separate requests per instruction, prompt step 40.2 k -> 36.9 k tok/s.)
-            const int p = NWV * r + wave;
-            const int n = wrow(16 * (p >> 1));
-            bsrc[r] = wb + (((((size_t)(n >> 4) * (a.K >> 8)) * 8 + (p & 1)) * 64 + lane) << 4);
-        } else {
-            bsrc[r] = wb + ((size_t)wrow(row) * a.ldw) * 2 + (size_t)((sslot ^ (row & 7)) * 16);
-        }
-    }
-    const size_t bstep = a.wtiled ? 2048 : DG_BK * 2;                   // bytes per K step on the weight side
-    auto stage = [&](int kt, int buf) {
-        const uint32_t base = lds0 + (uint32_t)buf * STAGE + (uint32_t)wave * 1024u;
-#pragma unroll
-        for (int r = 0; r < AROUNDS; ++r) dgemm_dma<1>(asrc[r] + (size_t)kt * (DG_BK * 2), base + (uint32_t)r * (uint32_t)(RROWS * 128));
-#pragma unroll
-        for (int r = 0; r < BROUNDS; ++r) dgemm_dma<1>(bsrc[r] + (size_t)kt * bstep, base + A_BYTES + (uint32_t)r * (uint32_t)(RROWS * 128));
-    };
-    f32x4_t acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    // LDS byte offsets of this lane's fragments (without the K-step slot): A rows of the wave's four m-fragments, B rows of its
-    // four n-fragments (SILU_MUL: fragments 0, 1 = gate columns, 2, 3 = the same columns of up)
-    int arow[4], brow[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) arow[i] = wr * 64 + i * 16 + m16;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) brow[j] = silu ? ((j >> 1) * 64 + wc * 32 + (j & 1) * 16 + m16) : (wc * 64 + j * 16 + m16);
-    const int nkt = a.K / DG_BK;
-    stage(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    for (int kt = 0; kt < nkt; ++kt) {
-        const int buf = kt & 1;
-        if (kt + 1 < nkt) stage(kt + 1, buf ^ 1);                       // in flight while this step is multiplied
-        const uint8_t* A = smem + (size_t)buf * STAGE;
-        const uint8_t* B = A + A_BYTES;
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-            uint4 af[4], bf[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) af[i] = *reinterpret_cast<const uint4*>(A + (size_t)arow[i] * 128 + (size_t)(((s2 * 4 + kg) ^ (arow[i] & 7)) * 16));
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                bf[j] = a.wtiled ? *reinterpret_cast<const uint4*>(B + (size_t)((((brow[j] >> 4) * 2 + s2) * 64 + kg * 16 + m16) * 16))
-                                 : *reinterpret_cast<const uint4*>(B + (size_t)brow[j] * 128 + (size_t)(((s2 * 4 + kg) ^ (brow[j] & 7)) * 16));
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = mfma32<DT>(af[i], bf[j], acc[i][j]);
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // the next tile has landed (this wave's share of it)
-        __syncthreads();                                                // ... everyone's; and everyone is done reading `buf`
-    }
-    // ---- epilogue: the lane holds tokens 4 kg + v of every m-fragment for column m16 of every n-fragment
-    const uint16_t* bias = static_cast<const uint16_t*>(a.bias);
-    const uint16_t* resid = static_cast<const uint16_t*>(a.resid);
-    uint16_t* out = static_cast<uint16_t*>(a.out);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int t = t0 + wr * 64 + i * 16 + 4 * kg + v;
-            if (t >= a.T) continue;
-            if (silu) {
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int col = c0 + wc * 32 + j * 16 + m16;
-                    if (col >= n_cols) continue;
-                    float g = rnd<DT>(acc[i][j][v]), u = rnd<DT>(acc[i][j + 2][v]);
-                    if (bias) { g = rnd<DT>(g + h2f<DT>(bias[col])); u = rnd<DT>(u + h2f<DT>(bias[a.pair_offset + col])); }
-                    out[(size_t)t * a.ldo + col] = f2h<DT>(rnd<DT>(rnd<DT>(g / (1.f + __expf(-g))) * u));      // silu(gate) * up (mlp.rs:457)
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int col = c0 + wc * 64 + j * 16 + m16;
-                    if (col >= n_cols) continue;
-                    float o = rnd<DT>(acc[i][j][v]);
-                    if (bias) o = rnd<DT>(o + h2f<DT>(bias[col]));
-                    if (a.epi == MI355_EPI_RESID) o = rnd<DT>(o + h2f<DT>(resid[(size_t)t * a.ldo + col]));
-                    out[(size_t)t * a.ldo + col] = f2h<DT>(o);
-                }
-            }
-        }
-}
-
 // ---- prompt steps over the tiled 4-bit image: ONE pass over the weights instead of T / 64 passes of the decode
 // kernel.  Same 128 x 128 workgroup tile and the same activation staging (LDS-DMA, swizzled, double buffer) as dense_gemm_kernel; the
 // weights never touch LDS: word j of a lane in the tiled image holds exactly the 8 codes of its B fragment of MFMA step j (that is
@@ -1462,44 +1471,89 @@ static int gptq_prompt_gemm(const DenseArgs& a, int dt, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
-static int dense_prompt_gemm(const DenseArgs& a, int dt, hipStream_t st) {
-    if (a.K % DG_BK || a.T < 1 || a.N < 1) return (int)hipErrorNotSupported;
-    if ((a.ldx * 2) % 16 || (!a.wtiled && (a.ldw * 2) % 16)) return (int)hipErrorNotSupported;          // 16-byte DMA pieces
-    if (a.epi == MI355_EPI_SILU_MUL && (a.pair_offset <= 0 || a.N != 2 * a.pair_offset)) return (int)hipErrorNotSupported;
+template <int DT, int EPI, int WM, int WN, int MF, int NF, int S, bool TILED>
+static void dense_gemm_go(const DenseGemm3& g, hipStream_t st) {
+    typedef GemmTile<DT, WM, WN, MF, NF, S, TILED> Tile;
     static Mi355DevOnce attr_done;
     if (!attr_done.done()) {
-        (void)hipFuncSetAttribute((const void*)dense_gemm_kernel<MI355_DTYPE_BF16, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-        (void)hipFuncSetAttribute((const void*)dense_gemm_kernel<MI355_DTYPE_F16, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-        (void)hipFuncSetAttribute((const void*)dense_gemm_kernel<MI355_DTYPE_BF16, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-        (void)hipFuncSetAttribute((const void*)dense_gemm_kernel<MI355_DTYPE_F16, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+        (void)hipFuncSetAttribute((const void*)dense_gemm_kernel<DT, EPI, WM, WN, MF, NF, S, TILED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Tile::LDS);
         attr_done.set();
     }
-    const int n_cols = a.epi == MI355_EPI_SILU_MUL ? a.pair_offset : a.N;
-    const int cols_per_wg = a.epi == MI355_EPI_SILU_MUL ? 64 : DG_BN;
-    const int ncb = (n_cols + cols_per_wg - 1) / cols_per_wg;
-    // the 256-token tile (one 8-wave workgroup per CU) when it still fills the chip twice
-    const bool tall = g_tune_gemm_tall && ((g_tune_gemm_tall & 2) || (int64_t)((a.T + 255) / 256) * ncb >= 512);   // (bit 64 of key 30: wherever the GEMM runs -- tests)
-    if (tall) {
-        const dim3 grid((a.T + 255) / 256, ncb);
-        if (dt == MI355_DTYPE_BF16) hipLaunchKernelGGL((dense_gemm_kernel<MI355_DTYPE_BF16, 4>), grid, dim3(512), 96 * 1024, st, a);
-        else if (dt == MI355_DTYPE_F16) hipLaunchKernelGGL((dense_gemm_kernel<MI355_DTYPE_F16, 4>), grid, dim3(512), 96 * 1024, st, a);
-        else return (int)hipErrorNotSupported;
-        return (int)hipGetLastError();
+    hipLaunchKernelGGL((dense_gemm_kernel<DT, EPI, WM, WN, MF, NF, S, TILED>), dim3(g.n_m * (g.tiles[0] + g.tiles[1] + g.tiles[2]) * g.splits), dim3(512), Tile::LDS, st, g);
+}
+template <int DT, int EPI, bool TILED>
+static void dense_gemm_tile(const DenseGemm3& g, int which, hipStream_t st) {
+#define DG_GO(WM_, WN_, MF_, NF_, S_) dense_gemm_go<DT, EPI, WM_, WN_, MF_, NF_, S_, TILED>(g, st)
+    GT_TILES(which, DG_GO);
+#undef DG_GO
+}
+template <int DT, bool TILED>
+static void dense_gemm_epi(const DenseGemm3& g, int which, hipStream_t st) {
+    if (g.a[0].epi == MI355_EPI_SILU_MUL) dense_gemm_tile<DT, MI355_EPI_SILU_MUL, TILED>(g, which, st);
+    else if (g.a[0].epi == MI355_EPI_RESID) dense_gemm_tile<DT, MI355_EPI_RESID, TILED>(g, which, st);
+    else dense_gemm_tile<DT, MI355_EPI_STORE, TILED>(g, which, st);
+}
+// n matrices over the same x: all tiled or all row-major, one dtype
+static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) {
+    if (dt != MI355_DTYPE_BF16 && dt != MI355_DTYPE_F16) return (int)hipErrorNotSupported;
+    for (int i = 0; i < n; ++i) {
+        if (a[i].K % 64 || a[i].T < 1 || a[i].N < 1 || a[i].wtiled != a[0].wtiled || a[i].epi != a[0].epi) return (int)hipErrorNotSupported;
+        if ((a[i].ldx * 2) % 16 || (!a[i].wtiled && (a[i].ldw * 2) % 16)) return (int)hipErrorNotSupported;          // 16-byte DMA pieces
+        if (a[i].epi == MI355_EPI_SILU_MUL && (a[i].pair_offset <= 0 || a[i].N != 2 * a[i].pair_offset)) return (int)hipErrorNotSupported;
+        if (a[i].epi == MI355_EPI_SILU_MUL && a[i].wtiled && (a[i].pair_offset & 15)) return (int)hipErrorNotSupported;
+        if ((int64_t)a[i].ldx * 512 >= (1ll << 32) || (int64_t)a[i].ldw * 512 >= (1ll << 32)) return (int)hipErrorNotSupported;   // 32-bit offsets inside a tile
     }
-    const dim3 grid((a.T + DG_BM - 1) / DG_BM, ncb);
-    if (dt == MI355_DTYPE_BF16) hipLaunchKernelGGL((dense_gemm_kernel<MI355_DTYPE_BF16, 2>), grid, dim3(256), 64 * 1024, st, a);
-    else if (dt == MI355_DTYPE_F16) hipLaunchKernelGGL((dense_gemm_kernel<MI355_DTYPE_F16, 2>), grid, dim3(256), 64 * 1024, st, a);
-    else return (int)hipErrorNotSupported;
+    auto tiles = [&](const GtTile& t, DenseGemm3* g) {
+        int64_t cols = 0;
+        for (int i = 0; i < 3; ++i) {
+            const bool silu = i < n && a[i].epi == MI355_EPI_SILU_MUL;
+            const int c = i >= n ? 0 : silu ? (a[i].pair_offset + t.bn / 2 - 1) / (t.bn / 2) : (a[i].N + t.bn - 1) / t.bn;
+            if (g) g->tiles[i] = c;
+            cols += c;
+        }
+        return cols * ((a[0].T + t.bm - 1) / t.bm);
+    };
+    const int units = a[0].K / 64;
+    int64_t rows = 0;
+    for (int i = 0; i < n; ++i) rows += a[i].N;
+    // A split adds a write and a read of f32 partial sums and a launch; it needs whole groups of four columns.  us per launch (T x N x K) with
+    // the 128 x 128 tile of four waves and two buffers drained at every step, and now: 3001 x 28672 x 4096 742 / 580 (256 x 256; 192 x 256 570,
+    // 128 x 128 640), 3001 x 4096 x 14336 480 / 292 (192 x 256: exactly one round; 256 x 256 331), 2048 x 28672 x 4096 550 / 375,
+    // 2048 x 4096 x 14336 215 (128 x 128, two per CU), 700 x 4096 x 14336 94 (two ranges; one: 175), 96 x 4096 x 14336 33 (64-token tiles,
+    // eight ranges; one: 113), 64 x 28672 x 4096 96 / 44.
+    const int max_split = n == 1 && a[0].T <= 65535 && !(a[0].N & 3) && !(a[0].epi == MI355_EPI_SILU_MUL && (a[0].pair_offset & 3)) ? std::min(16, std::max(1, units / 8)) : 1;
+    GtChoice best = gt_pick([&](const GtTile& t) { return tiles(t, nullptr); }, units, (float)rows * (float)a[0].K * 2.f / 5.4e6f, max_split,
+                            (float)a[0].T * (float)a[0].N * 4.f / 4.5e6f, 31);
+    if (g_tune_gemm_tall) best = {0, 1};
+    DenseGemm3 g{};
+    for (int i = 0; i < 3; ++i) g.a[i] = a[i < n ? i : 0];
+    g.n_m = (a[0].T + kGtTiles[best.tile].bm - 1) / kGtTiles[best.tile].bm;
+    g.units_per_split = (units + best.splits - 1) / best.splits;
+    g.splits = (units + g.units_per_split - 1) / g.units_per_split;
+    if (g.splits > 1) {
+        void* p = nullptr;
+        if (mi355_scratch_get(&p, MI355_SCR_GPTQ_WIDE, (size_t)g.splits * a[0].T * a[0].N * sizeof(float), st, false)) { g.splits = 1; g.units_per_split = units; }
+        g.part = static_cast<float*>(p);
+    }
+    if (tiles(kGtTiles[best.tile], &g) * g.splits > 0x7FFFFFFF) return (int)hipErrorNotSupported;
+    if (dt == MI355_DTYPE_BF16) { if (a[0].wtiled) dense_gemm_epi<MI355_DTYPE_BF16, true>(g, best.tile, st); else dense_gemm_epi<MI355_DTYPE_BF16, false>(g, best.tile, st); }
+    else { if (a[0].wtiled) dense_gemm_epi<MI355_DTYPE_F16, true>(g, best.tile, st); else dense_gemm_epi<MI355_DTYPE_F16, false>(g, best.tile, st); }
+    if (g.splits > 1) {
+        const int n_out = a[0].epi == MI355_EPI_SILU_MUL ? a[0].pair_offset : a[0].N;
+        const dim3 grid((n_out + 255) / 256, a[0].T);
+        if (dt == MI355_DTYPE_BF16) hipLaunchKernelGGL((gptq_wide_epilogue_kernel<MI355_DTYPE_BF16>), grid, dim3(256), 0, st, a[0], g.part, a[0].N, g.splits, a[0].T);
+        else hipLaunchKernelGGL((gptq_wide_epilogue_kernel<MI355_DTYPE_F16>), grid, dim3(256), 0, st, a[0], g.part, a[0].N, g.splits, a[0].T);
+    }
     return (int)hipGetLastError();
 }
 
 // SILU_MUL with more than 32 tokens, or any T > 64: run in token chunks
 static int dense_run(DenseArgs a, int wtype, int dt, hipStream_t st) {
-    if (wtype == DW_DENSE && a.T >= g_tune_gemm_min_t) {
-        const int rc = dense_prompt_gemm(a, dt, st);
+    if (wtype == DW_DENSE && (a.T >= g_tune_gemm_min_t || (g_tune_gemm_min_t == DENSE_GEMM_MIN_T && a.T > 16 && (a.epi == MI355_EPI_SILU_MUL ? a.pair_offset : a.N) >= 16 * 768))) {
+        const int rc = dense_prompt_gemm(&a, 1, dt, st);
         if (rc != (int)hipErrorNotSupported) return rc;                    // odd strides / K: keep streaming in token chunks
     }
-    if (wtype == DW_GPTQ4T && a.T >= g_tune_gemm_min_t) {
+    if (wtype == DW_GPTQ4T && a.T >= std::max(g_tune_gemm_min_t, (int)GPTQ_GEMM_MIN_T)) {
         const int rc = gptq_prompt_gemm(a, dt, st);
         if (rc != (int)hipErrorNotSupported) return rc;                    // groups of 32, odd strides: token chunks of the decode kernel
     }
@@ -1911,7 +1965,8 @@ int mi355_internal_linear3(void* const* outs, const void* x, const void* const* 
                            const void* const* biases, const int32_t* ns, int32_t num_tokens, int32_t k, int32_t group_size,
                            int32_t is_gptq, int32_t dtype, const void* norm_w, float norm_eps, const float* ss_in, const void* rope,
                            int64_t stream) {
-    if (num_tokens < 1 || num_tokens > 64 || (k & 255)) return -4;
+    const bool prompt = num_tokens >= g_tune_gemm_min_t && (is_gptq == 0 || is_gptq == 3) && !norm_w && !rope;   // one GEMM launch for the three
+    if (num_tokens < 1 || (num_tokens > 64 && !prompt) || (k & 255)) return -4;
     const DenseRope* rp = static_cast<const DenseRope*>(rope);
     DenseArgs a[3];
     for (int i = 0; i < 3; ++i) {
@@ -1927,6 +1982,10 @@ int mi355_internal_linear3(void* const* outs, const void* x, const void* const* 
         }
     }
     hipStream_t st = (hipStream_t)stream;
+    if (prompt) {
+        const int rc = dense_prompt_gemm(a, 3, dtype, st);
+        return rc == (int)hipErrorNotSupported ? -4 : rc;
+    }
     if (dtype == MI355_DTYPE_BF16)
         return is_gptq == 2 ? dense3_launch_dt<MI355_DTYPE_BF16, DW_GPTQ4T>(a, rp, st)
                : is_gptq == 1 ? dense3_launch_dt<MI355_DTYPE_BF16, DW_GPTQ4>(a, rp, st) : dense3_launch_dt<MI355_DTYPE_BF16, DW_DENSE>(a, rp, st);

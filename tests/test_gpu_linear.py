@@ -68,6 +68,46 @@ def test_linear_matches_oracle(cv, dt, T, N, K):
               mag=G.linear16(x, w, None, dt))
 
 
+@pytest.mark.parametrize("T,N,K", [(33, 288, 2304), (65, 160, 4096),                          # 64-token tiles, K in ranges; one token into the next tile
+                                   (130, 96, 8192),                                            # K in ranges over three token tiles
+                                   (900, 8192, 128),                                           # 128 x 128 tiles, exactly two per CU
+                                   (1530, 8192, 128),                                          # 192 x 256 tiles, exactly one per CU, ragged tokens
+                                   (1540, 8208, 128)])                                         # 256 x 256 tiles, ragged both ways
+def test_linear_prompt_gemm_every_tile(cv, T, N, K):
+    """16-bit prompt GEMM where its dispatch takes each of its tiles and K splits: row-major and tiled weights alike bit for bit, and within the
+    op's bound of the oracle (tokens and rows at the tile's edges and at the matrix's)"""
+    from candle_vllm_amd._lib import lib
+    dt, st = "bf16", torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(T + N + K)
+    x, w = G.round_dt(rng.normal(0, 1, (T, K)), dt), G.round_dt(rng.normal(0, 0.05, (N, K)), dt)
+    b, res = G.round_dt(rng.normal(0, 0.2, N), dt), G.round_dt(rng.normal(0, 1, (T, N)), dt)
+    xd, wd, bd, rd = dev16(x, dt), dev16(w, dt), dev16(b, dt), dev16(res, dt)
+    tiled = None
+    if K % 256 == 0:
+        tiled = torch.empty_like(wd)
+        assert lib.mi355_dense_tile_repack(wd.data_ptr(), tiled.data_ptr(), N, K, K, st) == 0
+    rows = np.unique(np.concatenate([np.arange(0, T, max(1, T // 40)), [t for e in (63, 64, 127, 128, 191, 192, 255, 256) for t in (e, T - 1 - e) if 0 <= t < T], [T - 1]])).astype(np.int64)
+    I = N // 2
+    for epi, bias, resid, n_out in ((0, bd, None, N), (1, None, rd, N), (2, None, None, I)):
+        outs = []
+        for fn, img in ((lib.mi355_linear, wd), (lib.mi355_linear_tiled, tiled)):
+            if img is None:
+                continue
+            out = torch.full((T, n_out), float("nan"), dtype=torch.bfloat16, device="cuda")
+            assert fn(out.data_ptr(), xd.data_ptr(), img.data_ptr(), bias.data_ptr() if bias is not None else None,
+                      resid.data_ptr() if resid is not None else None, T, N, K, 2, epi, st) == 0
+            outs.append(host16(out, dt))
+        assert len(outs) == 1 or np.array_equal(outs[0], outs[1])
+        y = G.linear16(x[rows], w, None, dt)
+        if epi == 0:
+            check_ulp(outs[0][rows], G.linear16(x[rows], w, b, dt), dt, what="linear+bias", ulps=2.01, mag=y)
+        elif epi == 1:
+            check_ulp(outs[0][rows], G.round_dt(y + res[rows], dt), dt, what="linear+resid", ulps=2.01, mag=y)
+        else:
+            check_ulp(outs[0][rows], G.silu_mul16(y[:, :I], y[:, I:], dt), dt, ulps=3.0, what="silu(gate)*up")
+        assert np.isfinite(outs[0]).all()
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("T,N,K", [(256, 384, 1024), (300, 200, 576), (97, 130, 64), (700, 128, 256)])
 def test_linear_prompt_gemm_tall_tile(cv, dt, T, N, K):
