@@ -11,6 +11,7 @@
 
 #include "common.h"
 #include "hybrid_device.h"
+#include "gemm_tile.h"
 #include "../../include/mi355_hybrid.h"
 
 namespace {
@@ -72,8 +73,9 @@ template <int B> __device__ __forceinline__ void lin_store(const LinArgs& p, int
     }
     p.out[(size_t)t * p.ldo + n] = v;
 }
+__device__ __forceinline__ float lin_glu(const LinArgs& p, float g, float u) { return (p.act == MI355_HYB_ACT_GELU ? gelu_tanhf_(g) : siluf_(g)) * u; }
 __device__ __forceinline__ void lin_store_glu(const LinArgs& p, int t, int c, float g, float u) {
-    const float v = (p.act == MI355_HYB_ACT_GELU ? gelu_tanhf_(g) : siluf_(g)) * u;
+    const float v = lin_glu(p, g, u);
     if (p.out16) reinterpret_cast<uint16_t*>(p.out)[(size_t)t * p.ldo + c] = f32_to_bf16(v);
     else p.out[(size_t)t * p.ldo + c] = v;
 }
@@ -246,6 +248,88 @@ template <int B> __global__ __launch_bounds__(256) void linear_bf16_lds_kernel(L
                 if (t < p.T) lin_store<B>(p, t, n, acc[i][j][v] + bias);
             }
     }
+}
+
+// The same products where K is a multiple of 64, on the main loop of gemm_tile.h (128 x 128 tiles, 32-wide K steps through registers in the
+// kernel above reached 400 - 740 TFLOP/s at 2100 tokens).
+struct LinGrid { int n_m, n_n; };
+template <int B, int WM, int WN, int MF, int NF, int S> __global__ __launch_bounds__(512, 2) void linear_bf16_gemm_kernel(LinArgs p, LinGrid grid) {
+    typedef GemmTile<MI355_DTYPE_BF16, WM, WN, MF, NF, S, false> Tile;
+    extern __shared__ __align__(1024) uint8_t lin_smem[];
+    const GtPlace at = gt_place(blockIdx.x, grid.n_m, grid.n_n);
+    const int t0 = at.m * Tile::BM, n0 = at.n * Tile::BN;
+    lin_batch<uint16_t, B>(p, n0);
+    int64_t w_off;
+    if (!lin_group(p, t0, w_off)) return;
+    Tile tile(lin_smem);
+    const uint8_t* a_base = static_cast<const uint8_t*>(p.a) + (p.row_src ? 0 : (size_t)t0 * p.lda * 2);
+    const uint8_t* wb = reinterpret_cast<const uint8_t*>(static_cast<const uint16_t*>(p.w) + w_off);
+    uint32_t a_off[Tile::AR], b_off[Tile::BR];
+    const uint8_t* b_base[Tile::BR];
+#pragma unroll
+    for (int r = 0; r < Tile::AR; ++r) {
+        const int t = min(t0 + tile.stage_row(r), p.T - 1);              // rows beyond the last are multiplied and never stored
+        a_off[r] = (uint32_t)(p.row_src ? p.row_src[t] : t - t0) * (uint32_t)p.lda * 2u + tile.stage_chunk();
+    }
+#pragma unroll
+    for (int r = 0; r < Tile::BR; ++r) {
+        const int first = min(n0 + 8 * (tile.wave + 8 * r), p.N - 1), row = min(n0 + tile.stage_row(r), p.N - 1);
+        b_base[r] = wb + (size_t)first * p.K * 2;
+        b_off[r] = (uint32_t)(row - first) * (uint32_t)p.K * 2u + tile.stage_chunk();
+    }
+    tile.run(a_base, a_off, b_base, b_off, 128u, p.K / 64);
+    const bool wide = !(p.ldo & 3) && !((uintptr_t)p.out & 15);          // (N is a multiple of 16)
+#pragma unroll
+    for (int i = 0; i < MF; ++i) {
+        const int t = t0 + tile.row(i);
+        if (t >= p.T) continue;
+        if constexpr (B == LIN_GLU_BUILD) {
+#pragma unroll
+            for (int j = 0; j < NF; j += 2) {
+                const int n = n0 + tile.wn * NF * 16 + j * 16, c = n / 2 + 4 * (tile.lane >> 4);
+                if (n >= p.N) continue;
+                if (wide && p.out16) {
+                    float v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = lin_glu(p, tile.acc[i][j][e], tile.acc[i][j + 1][e]);
+                    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p.out) + (size_t)t * p.ldo + c) = make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) lin_store_glu(p, t, c + e, tile.acc[i][j][e], tile.acc[i][j + 1][e]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NF; ++j) {
+                const int n = n0 + tile.col(j);
+                if (n >= p.N) continue;
+                f32x4_t v = tile.acc[i][j];
+                if (p.bias) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] += p.bias[n + e];
+                }
+                if (wide && B != LIN_EPI_BUILD) *reinterpret_cast<f32x4_t*>(p.out + (size_t)t * p.ldo + n) = v;
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) lin_store<B>(p, t, n + e, v[e]);
+                }
+            }
+        }
+    }
+}
+template <int B> static void linear_gemm_launch(const LinArgs& p, int which, int n_m, int nz, hipStream_t st) {
+    const LinGrid grid{n_m, (p.N + kGtTiles[which].bn - 1) / kGtTiles[which].bn};
+#define LIN_GO(WM_, WN_, MF_, NF_, S_) do { \
+        typedef GemmTile<MI355_DTYPE_BF16, WM_, WN_, MF_, NF_, S_, false> Tile_; \
+        static Mi355DevOnce attr_; \
+        if (!attr_.done()) { (void)hipFuncSetAttribute((const void*)linear_bf16_gemm_kernel<B, WM_, WN_, MF_, NF_, S_>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Tile_::LDS); attr_.set(); } \
+        linear_bf16_gemm_kernel<B, WM_, WN_, MF_, NF_, S_><<<dim3(grid.n_m * grid.n_n, 1, nz), 512, Tile_::LDS, st>>>(p, grid); } while (0)
+    GT_TILES(which, LIN_GO);
+#undef LIN_GO
+}
+// operands the GEMM's 16-byte pieces and 32-bit offsets reach (rows: of `a`, as far as they are known)
+static bool linear_gemm_ok(const LinArgs& p, bool a_f32, int64_t a_rows) {
+    return !a_f32 && p.a_vec && p.w_vec && p.K % 64 == 0 && p.N % 16 == 0 && a_rows * p.lda * 2 < (1ll << 32) && (int64_t)p.K * 2 * 256 < (1ll << 32);
 }
 
 // Up to 16 tokens, bf16 weights: the product is a stream over the weights.  A workgroup owns 16 weight rows; its NW waves take the
@@ -1965,6 +2049,11 @@ static int linear_launch(float* out, int32_t ldo, int64_t o_bs, const void* a, i
         const dim3 grid(glu ? n / 32 : (n + 15) / 16, 1, nz);
         if (k >= 2048) { if (af) LIN_EPI_(p, (linear_bf16_stream_kernel<float, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); else LIN_EPI(p, (linear_bf16_stream_kernel<uint16_t, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); }
         else { if (af) LIN_EPI_(p, (linear_bf16_stream_kernel<float, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); else LIN_EPI(p, (linear_bf16_stream_kernel<uint16_t, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); }
+    } else if (linear_gemm_ok(p, af, T)) {
+        // (segments end at multiples of 128 columns: only the tiles of that width have one left operand each)
+        const GtChoice c = gt_pick([&](const GtTile& t) { return (int64_t)((T + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch; }, k / 64,
+                                   (float)n * (float)k * 2.f * (float)batch / 5.4e6f, 1, 0.f, seg ? 28 : 31);
+        LIN_EPI(p, (linear_gemm_launch<EPI>(p, c.tile, (T + kGtTiles[c.tile].bm - 1) / kGtTiles[c.tile].bm, nz, st_)));
     } else if (T > 32 && !af && p.a_vec && p.w_vec && k % 32 == 0) {
         LIN_EPI(p, (linear_bf16_lds_kernel<EPI><<<dim3((n + 127) / 128, (T + 127) / 128, nz), 256, 0, st_>>>(p)));
     } else if (T <= 32) {
@@ -2548,6 +2637,10 @@ static int grouped_launch(void* out, int32_t out_dtype, int32_t ldo, const void*
         const dim3 grid(glu ? n / 32 : (n + 15) / 16, n_blocks, 1);
         if (k >= 2048) { if (af) LIN_EPI2_(p, (linear_bf16_stream_kernel<float, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); else LIN_EPI2(p, (linear_bf16_stream_kernel<uint16_t, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); }
         else { if (af) LIN_EPI2_(p, (linear_bf16_stream_kernel<float, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); else LIN_EPI2(p, (linear_bf16_stream_kernel<uint16_t, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); }
+    } else if ((block_rows == 64 || block_rows == 128) && linear_gemm_ok(p, af, p.T)) {
+        // the tile as tall as a block: 64 tokens, or 128 (two workgroups per CU where the blocks fill the chip, else one with more buffers)
+        const int which = block_rows == 64 ? 4 : (int64_t)n_blocks * ((n + 127) / 128) > mi355_num_cus() ? 2 : 3;
+        LIN_EPI2(p, (linear_gemm_launch<EPI>(p, which, n_blocks, 1, st_)));
     } else if (block_rows == 64) {
         const dim3 grid(glu ? (n + 127) / 128 : (n + 63) / 64, n_blocks, 1);
         if (af) LIN_EPI2_(p, (linear_bf16_tile_kernel<float, 4, EPI><<<grid, 256, 0, st_>>>(p))); else LIN_EPI2(p, (linear_bf16_tile_kernel<uint16_t, 4, EPI><<<grid, 256, 0, st_>>>(p)));

@@ -109,6 +109,32 @@ def _paged(k, v, block_size, rng, n_blocks):
     return kp, vp, table, slots
 
 
+@pytest.mark.parametrize("T,n,k", [(17, 48, 64), (65, 272, 640),          # 64-token tiles, six buffers: one unit, ten; one token into the next tile
+                                   (900, 8192, 128),                      # 128 x 128 tiles, exactly two per CU
+                                   (1530, 8192, 128), (1540, 8208, 192)]) # 192 x 256 and 256 x 256 tiles, ragged
+def test_linear_every_gemm_tile(lib, T, n, k):
+    """bf16 products of more than 16 tokens where the dispatch takes each of its tiles, plain, with bias, and as a gate/up pair.  Products of
+    bf16 values are exact in f32, so the bound is that of an f32 sum of k terms: 2^-24 k sum |a w|"""
+    g = torch.Generator(device="cuda").manual_seed(T + n + k)
+    a = torch.randn((T, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn((n, k), generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randn((n,), generator=g, device="cuda")
+    ref, mag = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    bound = 2.0 ** -24 * (k + 2) * (mag + b.double().abs()) + 1e-30
+    for bias in (None, b):
+        out = torch.full((T, n), float("nan"), device="cuda")
+        ok(lib.mi355_hyb_linear(out.data_ptr(), n, a.data_ptr(), BF16, k, w.data_ptr(), bias.data_ptr() if bias is not None else None, T, n, k, BF16, _st()))
+        assert bool(((out.double() - ref - (0 if bias is None else bias.double())).abs() <= bound).all())
+    if n % 32 == 0:                                                       # 16 gate rows, their 16 up rows, ...
+        out = torch.full((T, n // 2), float("nan"), device="cuda")
+        ok(lib.mi355_hyb_linear_glu(out.data_ptr(), F32, n // 2, a.data_ptr(), k, w.data_ptr(), T, n // 2, k, 1, BF16, _st()))
+        gu = ref.view(T, n // 32, 2, 16)
+        want = (torch.nn.functional.silu(gu[:, :, 0]) * gu[:, :, 1]).reshape(T, n // 2)
+        bg = bound.view(T, n // 32, 2, 16)                                # |silu'| <= 1.1, |silu(g)| <= |g|; expf and the division: 2^-21 of the value
+        lim = (1.1 * bg[:, :, 0] * gu[:, :, 1].abs() + bg[:, :, 1] * (gu[:, :, 0].abs() + 1)).reshape(T, n // 2) + 2.0 ** -21 * want.abs() + 1e-6
+        assert bool(((out.double() - want).abs() <= lim).all())
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("H_,G,d,vd,window,sink,bs,big", [(4, 2, 32, 48, 20, True, 16, False), (3, 3, 24, 24, 0, False, 8, False),
                                                          (2, 1, 80, 130, 70, True, 32, False), (1, 1, 16, 16, 1, True, 4, False),
