@@ -1386,139 +1386,6 @@ template <int TAPS, int NW> __global__ __launch_bounds__(64 * NW) void norm_conv
     }
 }
 
-// ------------------------------------------------------------------------------------------------------------ gated delta rule
-struct DeltaArgs {
-    float* o; float* state; int64_t state_stride;
-    const float* qkv; int ldq;
-    const float* proj; int ldp, b_off;
-    const float* decay_in; int ldd, decay_channels;
-    const float* a_log; const float* dt_bias;
-    const uint32_t* ctx; const uint32_t* cu_q; const int32_t* slots;
-    int H, G, d, vd; float unit_eps;
-};
-// Everything of the rule that does not depend on the state is computed for all new tokens at once, one wave per (token, head):
-// prep [T, P] = unit q times d^-1/2 and unit k per q/k head, the decays per head (or per head and key channel), beta per head.
-__global__ __launch_bounds__(64) void delta_prep_kernel(DeltaArgs p, float* prep, int P, int T) {
-    const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-    const int d = p.d, hpg = p.H / p.G, g = h / hpg;
-    float* out = prep + (size_t)t * P;
-    const int q_off = 0, k_off = p.G * d, g_off = 2 * p.G * d, dd = p.decay_channels ? d : 1, b_off = g_off + p.H * dd;
-    if (h % hpg == 0) {
-        const float* row = p.qkv + (size_t)t * p.ldq;
-        float qq = 0.f, kk = 0.f;
-        for (int i = lane; i < d; i += 64) { const float a = row[g * d + i], b = row[p.G * d + g * d + i]; qq += a * a; kk += b * b; }
-        qq = wave_sum(qq); kk = wave_sum(kk);
-        const float qi = (1.f / sqrtf((float)d)) / sqrtf(qq + p.unit_eps), ki = 1.f / sqrtf(kk + p.unit_eps);
-        for (int i = lane; i < d; i += 64) {
-            out[q_off + g * d + i] = row[g * d + i] * qi;
-            out[k_off + g * d + i] = row[p.G * d + g * d + i] * ki;
-        }
-    }
-    const float a_rate = expf(p.a_log[h]);
-    if (p.decay_channels) {
-        for (int i = lane; i < d; i += 64) {
-            const int ch = h * d + i;
-            out[g_off + ch] = expf(-a_rate * softplusf_(p.decay_in[(size_t)t * p.ldd + ch] + p.dt_bias[ch]));
-        }
-    } else if (lane == 0) {
-        out[g_off + h] = expf(-a_rate * softplusf_(p.decay_in[(size_t)t * p.ldd + h] + p.dt_bias[h]));
-    }
-    if (lane == 0) out[b_off + h] = sigmoidf_(p.proj[(size_t)t * p.ldp + p.b_off + h]);
-}
-
-// The scan.  A workgroup of 256 threads owns 256 / LPC columns of one (sequence, head)'s state S [d, vd]; LPC neighbouring lanes share
-// a column, each holding DP = ceil(d / LPC) of its rows in registers, and walk the new tokens in order:
-//   S <- diag(g) S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q
-// (the two sums over d are finished by lane exchanges among the LPC lanes).  The walk is a chain of dependent steps, so its time per
-// token is the latency of one step: the more lanes share a column the shorter the step (LPC = 16 at d >= 64).  q, k, g of CH tokens
-// at a time sit in LDS, rows padded so that the parts fall into different banks; the next CH tokens are fetched into registers
-// while the current ones are used.
-template <int DP, int LPC, int CH> __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaArgs p, const float* __restrict__ prep, int P) {
-    constexpr int RS = DP + 4, ROW = LPC * DP, TOT = CH * ROW, NPT = (TOT + 255) / 256, CPB = 256 / LPC;
-    __shared__ __align__(16) float sq[2][CH][LPC][RS], sk[2][CH][LPC][RS], sg[2][CH][LPC][RS];
-    __shared__ float sb[2][CH], sgh[2][CH];
-    const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-    const int col = blockIdx.z * CPB + tid / LPC, part = tid % LPC;
-    const int d = p.d, vd = p.vd, g = h / (p.H / p.G);
-    const int tb = (int)p.cu_q[s], te = (int)p.cu_q[s + 1];
-    if (te <= tb) return;
-    const int start_pos = (int)p.ctx[s] - (te - tb);
-    const bool own = col < vd, chan = p.decay_channels != 0;
-    float* stt = p.state + (size_t)p.slots[s] * p.state_stride + (size_t)h * d * vd;
-    float S[DP];
-#pragma unroll
-    for (int r = 0; r < DP; ++r) { const int i = part * DP + r; S[r] = (own && i < d && start_pos > 0) ? stt[(size_t)i * vd + col] : 0.f; }
-    const int q_off = g * d, k_off = p.G * d + g * d, g_off = 2 * p.G * d + (chan ? h * d : h), b_off = 2 * p.G * d + p.H * (chan ? d : 1) + h;
-    const int v_col = 2 * p.G * d + h * vd + col;
-    float rq[NPT], rk[NPT], rg[NPT], rv[CH], rbeta = 0.f, rgh = 1.f;
-    auto fetch = [&](int t0) {
-#pragma unroll
-        for (int n = 0; n < NPT; ++n) {
-            const int idx = tid + n * 256, c = idx / ROW, ii = idx - c * ROW, t = t0 + c;
-            const bool ok_ = idx < TOT && t < te && ii < d;
-            const float* row = prep + (size_t)(ok_ ? t : tb) * P;
-            rq[n] = ok_ ? row[q_off + ii] : 0.f;
-            rk[n] = ok_ ? row[k_off + ii] : 0.f;
-            rg[n] = (ok_ && chan) ? row[g_off + ii] : 1.f;
-        }
-#pragma unroll
-        for (int c = 0; c < CH; ++c) rv[c] = (own && t0 + c < te) ? p.qkv[(size_t)(t0 + c) * p.ldq + v_col] : 0.f;
-        if (tid < CH && t0 + tid < te) {
-            rbeta = prep[(size_t)(t0 + tid) * P + b_off];
-            rgh = chan ? 1.f : prep[(size_t)(t0 + tid) * P + g_off];
-        }
-    };
-    auto stage = [&](int buf) {
-#pragma unroll
-        for (int n = 0; n < NPT; ++n) {
-            const int idx = tid + n * 256;
-            if (idx < TOT) {
-                const int c = idx / ROW, ii = idx - c * ROW, pp = ii / DP, r = ii - pp * DP;
-                sq[buf][c][pp][r] = rq[n]; sk[buf][c][pp][r] = rk[n]; sg[buf][c][pp][r] = rg[n];
-            }
-        }
-        if (tid < CH) { sb[buf][tid] = rbeta; sgh[buf][tid] = rgh; }
-    };
-    fetch(tb);
-    stage(0);
-    __syncthreads();
-    int buf = 0;
-    for (int t0 = tb; t0 < te; t0 += CH, buf ^= 1) {
-        float vc[CH];
-#pragma unroll
-        for (int c = 0; c < CH; ++c) vc[c] = rv[c];
-        const bool more = t0 + CH < te;
-        if (more) fetch(t0 + CH);
-        const int cn = min(CH, te - t0);
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            if (c < cn) {
-                float kv = 0.f;
-                if (chan) {
-#pragma unroll
-                    for (int r = 0; r < DP; ++r) { S[r] *= sg[buf][c][part][r]; kv = fmaf(S[r], sk[buf][c][part][r], kv); }
-                } else {
-                    const float gh = sgh[buf][c];
-#pragma unroll
-                    for (int r = 0; r < DP; ++r) { S[r] *= gh; kv = fmaf(S[r], sk[buf][c][part][r], kv); }
-                }
-                kv = column_sum<LPC>(kv);
-                const float u = sb[buf][c] * (vc[c] - kv);
-                float o = 0.f;
-#pragma unroll
-                for (int r = 0; r < DP; ++r) { S[r] = fmaf(sk[buf][c][part][r], u, S[r]); o = fmaf(S[r], sq[buf][c][part][r], o); }
-                o = column_sum<LPC>(o);
-                if (own && part == 0) p.o[((size_t)(t0 + c) * p.H + h) * vd + col] = o;
-            }
-        }
-        if (more) stage(buf ^ 1);
-        __syncthreads();
-    }
-    if (own)
-#pragma unroll
-        for (int r = 0; r < DP; ++r) { const int i = part * DP + r; if (i < d) stt[(size_t)i * vd + col] = S[r]; }
-}
-
 // out = o / rms(o) * w * gate * out_scale, one wave per (token, head); head h's weights start at w + h w_ld
 template <typename TO> __global__ __launch_bounds__(256) void gated_norm_kernel(TO* out, int ldo, int out_off, const float* o, const float* w,
                                                                               const float* gate_in, int ldg, int gate, int H, int vd, int w_ld,
@@ -2365,38 +2232,6 @@ int mi355_hyb_conv_state_update(float* conv_state, int64_t state_stride, const f
     ConvArgs p{nullptr, proj, ldp, off, nullptr, conv_state, state_stride, context_lens, cu_seqlens_q, state_slots, nullptr, channels, taps, 0, 0, 0, nullptr};
     const int n = num_seqs * channels;
     conv_state_update_kernel<<<(n + 255) / 256, 256, 0, to_stream(stream)>>>(p, num_seqs);
-    LAUNCH_OK(); return 0;
-}
-
-int mi355_hyb_delta_rule_scratch_floats(int32_t num_tokens, int32_t heads, int32_t kv_heads, int32_t dim, int32_t decay_channels) {
-    return num_tokens * (2 * kv_heads * dim + heads * (decay_channels ? dim : 1) + heads);
-}
-
-int mi355_hyb_delta_rule(float* o, float* state, int64_t state_stride, const float* qkv, int32_t ldq, const float* proj, int32_t ldp,
-                         int32_t b_off, const float* decay_in, int32_t ldd, int32_t decay_channels, const float* a_log,
-                         const float* dt_bias, const uint32_t* context_lens, const uint32_t* cu_seqlens_q, const int32_t* state_slots,
-                         int32_t num_seqs, int32_t num_tokens, int32_t heads, int32_t kv_heads, int32_t dim, int32_t vdim, float unit_eps,
-                         float* scratch, int64_t stream) {
-    if (!o || !state || !qkv || !proj || !decay_in || !a_log || !dt_bias || !context_lens || !cu_seqlens_q || !state_slots || !scratch) return -1;
-    if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || dim > 256 || vdim <= 0) return -1;
-    if (num_seqs <= 0 || num_tokens <= 0) return 0;
-    DeltaArgs p{o, state, state_stride, qkv, ldq, proj, ldp, b_off, decay_in, ldd, decay_channels, a_log, dt_bias,
-                context_lens, cu_seqlens_q, state_slots, heads, kv_heads, dim, vdim, unit_eps};
-    hipStream_t s_ = to_stream(stream);
-    const int P = 2 * kv_heads * dim + heads * (decay_channels ? dim : 1) + heads;
-    delta_prep_kernel<<<dim3(num_tokens, heads), 64, 0, s_>>>(p, scratch, P, num_tokens);
-    LAUNCH_OK();
-    if (dim < 64) {
-        const dim3 grid(num_seqs, heads, (vdim + 63) / 64);
-        if (dim <= 16) delta_scan_kernel<4, 4, 8><<<grid, 256, 0, s_>>>(p, scratch, P);
-        else if (dim <= 32) delta_scan_kernel<8, 4, 8><<<grid, 256, 0, s_>>>(p, scratch, P);
-        else delta_scan_kernel<16, 4, 8><<<grid, 256, 0, s_>>>(p, scratch, P);
-    } else {
-        const dim3 grid(num_seqs, heads, (vdim + 15) / 16);
-        if (dim <= 64) delta_scan_kernel<4, 16, 8><<<grid, 256, 0, s_>>>(p, scratch, P);
-        else if (dim <= 128) delta_scan_kernel<8, 16, 8><<<grid, 256, 0, s_>>>(p, scratch, P);
-        else delta_scan_kernel<16, 16, 8><<<grid, 256, 0, s_>>>(p, scratch, P);
-    }
     LAUNCH_OK(); return 0;
 }
 

@@ -303,6 +303,42 @@ def test_delta_rule_portions_and_state(lib, Hh, G, d, vd, per_channel):
     assert np.abs(S - S_want).max() < 2e-5 * max(1.0, np.abs(S_want).max())
 
 
+@pytest.mark.parametrize("Hh,G,d,vd,per_channel", [(2, 1, 16, 32, False), (3, 3, 48, 16, True), (2, 2, 64, 64, True), (4, 2, 128, 48, True), (1, 1, 208, 16, False)])
+def test_delta_rule_by_pieces(lib, Hh, G, d, vd, per_channel):
+    """portions of prompts (64 tokens and more: pieces of 16) of three sequences in one call, cut so that pieces end inside and at the ends of
+    portions, continued from the slots' states; decays from almost 1 to almost 0.  The bound is the walk's (test above)"""
+    _gpu()
+    rng = np.random.default_rng(Hh * 11 + d)
+    lens, cuts = [161, 64, 240], [[97, 64], [1, 63], [16, 224]]                # tokens of a sequence, of its two portions
+    C, ldp, nd, stride = 2 * G * d + Hh * vd, Hh + 1, Hh * d if per_channel else Hh, Hh * d * vd + 5
+    a_log, dtb = rng.standard_normal(Hh).astype(np.float32), rng.standard_normal(nd).astype(np.float32)
+    seqs, want = [], []
+    for T in lens:
+        qkv, proj, pre = (rng.standard_normal((T, n)).astype(np.float32) for n in (C, ldp, nd))
+        pre[:, ::3] = 6 * pre[:, ::3]
+        q = H.unit_heads(qkv[:, :G * d].astype(np.float64).reshape(T, G, d), 1e-6) * d ** -0.5
+        k = H.unit_heads(qkv[:, G * d:2 * G * d].astype(np.float64).reshape(T, G, d), 1e-6)
+        g = H.decay(a_log.astype(np.float64)[None, :, None], pre.astype(np.float64).reshape(T, Hh, -1), dtb.astype(np.float64).reshape(1, Hh, -1)) * np.ones((1, 1, d))
+        want.append(H.gated_delta_rule(q, k, qkv[:, 2 * G * d:].astype(np.float64).reshape(T, Hh, vd), H.sigmoid(proj[:, 1:].astype(np.float64)), g))
+        seqs.append((qkv, proj, pre))
+    state = dev(rng.standard_normal((4, stride)))
+    for part in (0, 1):
+        rows = [(0, c[0]) if part == 0 else (c[0], c[0] + c[1]) for c in cuts]
+        qkv, proj, pre = (np.concatenate([s[i][lo:hi] for s, (lo, hi) in zip(seqs, rows)]) for i in range(3))
+        n, cu = len(qkv), np.cumsum([0] + [hi - lo for lo, hi in rows])
+        o = torch.full((n, Hh, vd), float("nan"), device="cuda")
+        scratch = torch.zeros(lib.mi355_hyb_delta_rule_scratch_floats(n, Hh, G, d, int(per_channel)), device="cuda")
+        assert (n // 3 >= 48) == (part == 1)                                # the first call walks, the second goes by pieces
+        ok(lib.mi355_hyb_delta_rule(o.data_ptr(), state.data_ptr(), stride, P(qkv), C, P(proj), ldp, 1, P(pre), nd, int(per_channel), P(a_log), P(dtb),
+                                    P([hi for _, hi in rows], np.int32), P(cu, np.int32), P([2, 0, 3], np.int32), 3, n, Hh, G, d, vd, 1e-6, scratch.data_ptr(), _st()))
+        for i, (lo, hi) in enumerate(rows):
+            w = want[i][0]
+            assert np.abs(o[cu[i]:cu[i + 1]].cpu().numpy() - w[lo:hi]).max() < 2e-5 * max(1.0, np.abs(w).max())
+    S = state.cpu().numpy()
+    for slot, (_, w) in zip((2, 0, 3), want):
+        assert np.abs(S[slot, :Hh * d * vd].reshape(Hh, d, vd) - w).max() < 2e-5 * max(1.0, np.abs(w).max())
+
+
 def test_gated_norm_and_mingru(lib):
     _gpu()
     rng = np.random.default_rng(9)
