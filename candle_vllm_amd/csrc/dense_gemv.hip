@@ -808,7 +808,9 @@ static int dense_launch_gj(const DenseArgs& a, int gj, int nw, hipStream_t st) {
 // us per launch, streaming kernels against the GEMM: gate/up 28672 x 4096 T = 16 43.9 / 42.3, 32 47.0 / 42.3, 40 90.3 / 43.1 (two sweeps over
 // the weights from 33 tokens), 64 96.5 / 44.0; down 4096 x 14336 T = 32 28.5 / 28.6, 40 31.0 / 29.5, 64 64.9 / 32.3; wo 4096 x 4096
 // T = 16 9.3 / 13.7, 32 12.3 / 14.0, 40 16.1 / 13.7; 12288 x 2048 T = 32 17.0 / 12.9; at 5 .. 16 tokens either may win (16384 pairs of 3072: 18.7 / 22.1)
-enum { DENSE_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_T = 96 };
+// 4-bit, against token chunks of the decode kernels: down 3584 x 18944 T = 32 21.6 / 27.4, 33 29.1 / 28.1, 49 72.7 / 29.1; 4608 x 3584 T = 33 20.8 / 16.0;
+// wo 3584 x 3584 33 14.8 / 15.0, 64 19.2 / 16.5; gate/up 37888 x 3584 48 42.1 / 54.5, 64 48.3 / 58.3, 65 64.3 / 58.8
+enum { DENSE_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_PAIR_T = 65 };
 static int g_tune_gemm_min_t = DENSE_GEMM_MIN_T;
 static int g_tune_gptq_gemm_off = 0;   // tuning key 39: 1 = 4-bit prompt steps run the decode kernel in 64-token chunks (A/B)
 static int g_tune_wide_nw = 4;         // tuning key 38: waves (row tiles) per workgroup of dense_wide_kernel: 2 | 4
@@ -1102,6 +1104,65 @@ template <int DT> __device__ __forceinline__ float gemm_rnd(float v) {
     if constexpr (DT == MI355_DTYPE_BF16) return __uint_as_float(cvt_pk_bf16(v, 0.f) << 16);
     else return rnd<DT>(v);
 }
+// Epilogue of the prompt GEMMs: acc[i][j][v] is token t_first + 16 i, column col_first + 16 j + v (SILU_MUL: fragments j and j + NF / 2 are gate
+// and up of the same columns): four consecutive columns of one token per fragment
+template <int DT, int EPI, int MF, int NF>
+__device__ __forceinline__ void gemm_store(const DenseArgs& a, const f32x4_t (&acc)[MF][NF], const int t_first, const int col_first) {
+    constexpr bool silu = EPI == MI355_EPI_SILU_MUL;
+    const int n_cols = silu ? a.pair_offset : a.N;
+    const uint16_t* bias = static_cast<const uint16_t*>(a.bias);
+    const uint16_t* resid = static_cast<const uint16_t*>(a.resid);
+    uint16_t* out = static_cast<uint16_t*>(a.out);
+    const bool wide = !((a.ldo & 3) | (n_cols & 3)) && !(((uintptr_t)out | (uintptr_t)resid) & 7);
+#pragma unroll
+    for (int i = 0; i < MF; ++i) {
+        const int t = t_first + 16 * i;
+        if (t >= a.T) continue;
+#pragma unroll
+        for (int j = 0; j < (silu ? NF / 2 : NF); ++j) {
+            float o[4];
+            int col;
+            if (silu) {
+                col = col_first + 16 * j;
+                if (col >= n_cols) continue;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float gv = gemm_rnd<DT>(acc[i][j][v]), u = gemm_rnd<DT>(acc[i][(j + NF / 2) % NF][v]);
+                    if (bias && col + v < n_cols) { gv = gemm_rnd<DT>(gv + h2f<DT>(bias[col + v])); u = gemm_rnd<DT>(u + h2f<DT>(bias[a.pair_offset + col + v])); }
+                    o[v] = gemm_rnd<DT>(gv / (1.f + __expf(-gv))) * u;        // silu(gate) * up (mlp.rs:457); the store rounds
+                }
+            } else {
+                col = col_first + 16 * j;
+                if (col >= n_cols) continue;
+                uint16_t rr[4];
+                if (EPI == MI355_EPI_RESID) {
+                    const uint16_t* rp = resid + (size_t)t * a.ldo + col;
+                    if (wide) {
+                        const uint2 r2 = *reinterpret_cast<const uint2*>(rp);
+                        rr[0] = (uint16_t)r2.x; rr[1] = (uint16_t)(r2.x >> 16); rr[2] = (uint16_t)r2.y; rr[3] = (uint16_t)(r2.y >> 16);
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) rr[v] = col + v < n_cols ? rp[v] : (uint16_t)0;
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    o[v] = gemm_rnd<DT>(acc[i][j][v]);
+                    if (bias && col + v < n_cols) o[v] = gemm_rnd<DT>(o[v] + h2f<DT>(bias[col + v]));
+                    if (EPI == MI355_EPI_RESID) o[v] = o[v] + h2f<DT>(rr[v]);
+                }
+            }
+            uint16_t* op = out + (size_t)t * a.ldo + col;
+            if (wide) {
+                *reinterpret_cast<uint2*>(op) = make_uint2(gemm_pack<DT>(o[0], o[1]), gemm_pack<DT>(o[2], o[3]));
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) if (col + v < n_cols) op[v] = (uint16_t)gemm_pack<DT>(o[v], 0.f);
+            }
+        }
+    }
+}
+
 template <int DT, int EPI, int WM, int WN, int MF, int NF, int S, bool TILED>
 __global__ void __launch_bounds__(512, 2) dense_gemm_kernel(const DenseGemm3 g) {
     typedef GemmTile<DT, WM, WN, MF, NF, S, TILED> Tile;
@@ -1179,295 +1240,100 @@ __global__ void __launch_bounds__(512, 2) dense_gemm_kernel(const DenseGemm3 g) 
         }
         return;
     }
-    // ---- epilogue: four consecutive columns of one token per fragment
-    const uint16_t* bias = static_cast<const uint16_t*>(a.bias);
-    const uint16_t* resid = static_cast<const uint16_t*>(a.resid);
-    uint16_t* out = static_cast<uint16_t*>(a.out);
-    const bool wide = !((a.ldo & 3) | (n_cols & 3)) && !(((uintptr_t)out | (uintptr_t)resid) & 7);
-#pragma unroll
-    for (int i = 0; i < MF; ++i) {
-        const int t = t0 + tile.row(i);
-        if (t >= a.T) continue;
-#pragma unroll
-        for (int j = 0; j < (silu ? NF / 2 : NF); ++j) {
-            float o[4];
-            int col;
-            if (silu) {
-                col = c0 + tile.wn * (NF * 8) + j * 16 + 4 * (tile.lane >> 4);
-                if (col >= n_cols) continue;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    float gv = gemm_rnd<DT>(tile.acc[i][j][v]), u = gemm_rnd<DT>(tile.acc[i][(j + NF / 2) % NF][v]);
-                    if (bias && col + v < n_cols) { gv = gemm_rnd<DT>(gv + h2f<DT>(bias[col + v])); u = gemm_rnd<DT>(u + h2f<DT>(bias[a.pair_offset + col + v])); }
-                    o[v] = gemm_rnd<DT>(gv / (1.f + __expf(-gv))) * u;        // silu(gate) * up (mlp.rs:457); the store rounds
-                }
-            } else {
-                col = c0 + tile.col(j);
-                if (col >= n_cols) continue;
-                uint16_t rr[4];
-                if (EPI == MI355_EPI_RESID) {
-                    const uint16_t* rp = resid + (size_t)t * a.ldo + col;
-                    if (wide) {
-                        const uint2 r2 = *reinterpret_cast<const uint2*>(rp);
-                        rr[0] = (uint16_t)r2.x; rr[1] = (uint16_t)(r2.x >> 16); rr[2] = (uint16_t)r2.y; rr[3] = (uint16_t)(r2.y >> 16);
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) rr[v] = col + v < n_cols ? rp[v] : (uint16_t)0;
-                    }
-                }
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    o[v] = gemm_rnd<DT>(tile.acc[i][j][v]);
-                    if (bias && col + v < n_cols) o[v] = gemm_rnd<DT>(o[v] + h2f<DT>(bias[col + v]));
-                    if (EPI == MI355_EPI_RESID) o[v] = o[v] + h2f<DT>(rr[v]);
-                }
-            }
-            uint16_t* op = out + (size_t)t * a.ldo + col;
-            if (wide) {
-                *reinterpret_cast<uint2*>(op) = make_uint2(gemm_pack<DT>(o[0], o[1]), gemm_pack<DT>(o[2], o[3]));
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) if (col + v < n_cols) op[v] = (uint16_t)gemm_pack<DT>(o[v], 0.f);
-            }
-        }
-    }
+    gemm_store<DT, EPI, MF, NF>(a, tile.acc, t0 + tile.row(0), c0 + (silu ? tile.wn * NF * 8 : tile.wn * NF * 16) + 4 * (tile.lane >> 4));
 }
 
-template <int NP>
-__device__ __forceinline__ void dgemm_dma(const uint8_t* gsrc_lane, uint32_t lds_dst) {
-    // NP x 1 KiB: lane l copies 16 B from its own source address (+ i * row_stride handled by the caller through separate calls)
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(gsrc_lane), "s"(lds_dst) : "memory");
+#include "gptq_gemm.inc"
+template <int DT, int EPI, bool SYM, int XG, int WM, int WN, int MF, int NF, int S>
+static void gptq_gemm_go(const GptqGemm& g, hipStream_t st) {
+    constexpr int BM = WM * MF * 16, BN = WN * NF * 16;
+    constexpr uint32_t lds = S * (BM * 256u + BN * 64u) + (S + 1) * (GG_UNIT / XG) * (1024u + BN * 4u);
+    static_assert(lds <= 160 * 1024, "a CU's LDS");
+    static Mi355DevOnce attr_done;
+    if (!attr_done.done()) {
+        (void)hipFuncSetAttribute((const void*)gptq_gemm_kernel<DT, EPI, SYM, XG, WM, WN, MF, NF, S>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        attr_done.set();
+    }
+    hipLaunchKernelGGL((gptq_gemm_kernel<DT, EPI, SYM, XG, WM, WN, MF, NF, S>), dim3(g.n_m * (g.tiles[0] + g.tiles[1] + g.tiles[2]) * g.splits), dim3(512), lds, st, g);
 }
-
-#define DG_BM 128
-#define DG_BK 64
-// ---- prompt steps over the tiled 4-bit image: ONE pass over the weights instead of T / 64 passes of the decode
-// kernel.  Same 128 x 128 workgroup tile and the same activation staging (LDS-DMA, swizzled, double buffer) as dense_gemm_kernel; the
-// weights never touch LDS: word j of a lane in the tiled image holds exactly the 8 codes of its B fragment of MFMA step j (that is
-// what the tile order is), so a wave fetches one dwordx4 per n-fragment and 128 k and unpacks it in registers (128+q / 1024+q by one
-// AND-OR, code pairs (q_i, q_i+4): the A fragment is permuted to match on its way out of LDS).  The accumulators run over one
-// quantisation group (a multiple of 64 k); at its end  y += s_g (acc - (OFF + z) xsum_g)  with the per-token group sums of x from a
-// ones-MFMA (as the decode kernels) and (scale, zero point) from a panel staged in LDS once per workgroup: inside the K loop the only
-// global traffic is the activation DMA and the weight ring -- a load that hipcc can see next to the invisible DMA makes it wait for
-// everything (first version: scales and a pre-computed xsum array fetched at every group end, 2.1-2.4 us per K step, 214-306 TFLOP/s).
-#define GG_NF 2
-static_assert(GG_NF == 2, "the counted wait in gptq_gemm_kernel leaves GG_NF loads in flight");
-template <int DT, int GPK>
-__global__ void __launch_bounds__(256) gptq_gemm_kernel(const DenseArgs a) {
-    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];   // [3 buffers][A 16 KiB]: the DMA runs two K steps ahead
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave >> 1, wc = wave & 1;
-    const int m16 = lane & 15, kg = lane >> 4;
-    const bool silu = a.epi == MI355_EPI_SILU_MUL;
-    const int bm = blockIdx.x, bn = blockIdx.y;
-    const int t0 = bm * DG_BM;
-    const int n_cols = silu ? a.pair_offset : a.N;
-    // 128 tokens x 64 columns per workgroup (SILU_MUL: 32 gate + the same 32 up columns): 4 m-fragments x 2 n-fragments per wave --
-    // with 4 n-fragments the group accumulators, the running sums and the weight ring need more than 256 VGPRs
-    const int c0 = bn * (silu ? 32 : 64);
-    const int nkb = a.K >> 8, gs = a.group_size;
-    // n-fragment j of this wave: first column (clamped to the matrix: columns beyond it are computed and never stored)
-    int fcol[GG_NF];
-#pragma unroll
-    for (int j = 0; j < GG_NF; ++j) {
-        int n = silu ? ((j ? a.pair_offset : 0) + c0 + wc * 16) : (c0 + wc * 32 + j * 16);
-        const int lim = silu ? ((j ? a.N : a.pair_offset) - 16) : a.N - 16;
-        fcol[j] = n > lim ? lim : n;
+static constexpr GtTile kGgTiles[] = {{128, 256, 1, 2.0f}, {128, 128, 1, 1.2f}, {64, 128, 1, 0.9f}};   // us: a unit of 128 k
+template <int DT, int EPI, bool SYM, int XG>
+static void gptq_gemm_tile(const GptqGemm& g, int which, hipStream_t st) {
+    switch (which) {
+        case 0: if constexpr (XG == GG_UNIT) gptq_gemm_go<DT, EPI, SYM, XG, 2, 4, 4, 4, 3>(g, st); break;   // (groups of 64: 8 .. 31 registers too many)
+        case 1: gptq_gemm_go<DT, EPI, SYM, XG, 2, 4, 4, 2, 3>(g, st); break;
+        default: gptq_gemm_go<DT, EPI, SYM, XG, 2, 4, 2, 2, 5>(g, st); break;
     }
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) void*)smem);
-    const uint8_t* xb = static_cast<const uint8_t*>(a.x);
-    const int srow = tid >> 3, sslot = tid & 7;
-    const uint8_t* asrc[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int row = 32 * r + srow;
-        int t = t0 + row;
-        if (t > a.T - 1) t = a.T - 1;
-        asrc[r] = xb + ((size_t)t * a.ldx) * 2 + (size_t)((sslot ^ (row & 7)) * 16);
-    }
-    // ---- (scale, zero point) panel of this workgroup's 64 columns, all groups: u32 = zero point (f32 bits >> 16, an exact small
-    // integer) << 16 | scale bits; panel[g][wave-column wc][fragment j][m16]
-    uint32_t* panel = reinterpret_cast<uint32_t*>(smem + 3 * 16384);
-    {
-        const int ng = a.K / gs;
-        const uint16_t* sc16p = static_cast<const uint16_t*>(a.scales);
-        for (int e = tid; e < ng * 64; e += 256) {
-            const int g = e >> 6, lc = e & 63, pwc = lc >> 5, pj = (lc >> 4) & 1, pm = lc & 15;
-            int n = silu ? ((pj ? a.pair_offset : 0) + c0 + pwc * 16) : (c0 + pwc * 32 + pj * 16);
-            const int lim = silu ? ((pj ? a.N : a.pair_offset) - 16) : a.N - 16;
-            const int col = (n > lim ? lim : n) + pm;
-            const uint32_t sb = sc16p[(size_t)g * a.N + marlin_scale_pos(col, a.sperm)];
-            const float z = zero_point(a, g, col);
-            panel[e] = (__float_as_uint(z) & 0xFFFF0000u) | sb;
-        }
-    }
-    auto stage = [&](int kt, int buf) {
-        const uint32_t base = lds0 + (uint32_t)buf * 16384u + (uint32_t)wave * 1024u;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dgemm_dma<1>(asrc[r] + (size_t)kt * (DG_BK * 2), base + (uint32_t)r * 4096u);
-    };
-    // weights: one dwordx4 per n-fragment and 128 k: [tile][k-block][half][lane][4 words]
-    const dg_u32x4* wbase[GG_NF];
-#pragma unroll
-    for (int j = 0; j < GG_NF; ++j) wbase[j] = reinterpret_cast<const dg_u32x4*>(a.w) + ((size_t)(fcol[j] >> 4) * nkb * 2) * 64 + lane;
-    dg_u32x4 wq[2][GG_NF];
-    auto wload = [&](int slot, int h128) {                               // h128 = index of the 128-k half (2 per k-block)
-#pragma unroll
-        for (int j = 0; j < GG_NF; ++j) wq[slot][j] = __builtin_nontemporal_load(wbase[j] + (size_t)h128 * 64);
-    };
-    constexpr uint32_t KOFF = (DT == MI355_DTYPE_BF16) ? 0x43004300u : 0x64006400u;
-    constexpr float OFF = (DT == MI355_DTYPE_BF16) ? 128.f : 1024.f;
-    uint32_t nib = 0x000F000Fu;
-    asm volatile("" : "+v"(nib));
-    constexpr uint32_t ONE2 = (DT == MI355_DTYPE_BF16) ? 0x3F803F80u : 0x3C003C00u;
-    const uint4 ones = make_uint4(ONE2, ONE2, ONE2, ONE2);
-    f32x4_t xs[4];                                                       // group sums of x per token (every column of a ones-MFMA holds them)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) xs[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    f32x4_t acc[4][GG_NF], y[4][GG_NF];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < GG_NF; ++j) { acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f}; y[i][j] = acc[i][j]; }
-    int arow[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) arow[i] = wr * 64 + i * 16 + m16;
-    const int nkt = a.K / DG_BK;
-    const int nh = a.K >> 7;
-    // A K step is 16 MFMAs per wave -- far less than a memory round trip -- so the activation tiles run TWO steps ahead through three
-    // buffers and the end-of-step wait is counted: only the tile of the NEXT step has to have landed (measured with a two-buffer,
-    // wait-for-everything loop: 2.4 us per K step, 214-306 TFLOP/s)
-    stage(0, 0);
-    if (nkt > 1) stage(1, 1);
-    wload(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    // One k-block (256 k = 4 K steps = 2 weight halves) per iteration of the run-time loop, its four steps unrolled: buffer, ring slot
-    // and word indices are compile-time (a run-time slot index put the weight ring into scratch), and so is the position of the
-    // per-group update (GPK = K steps per group: 1 / 2 / 4; 0 = whole k-blocks, the update sits behind a loop over the group's
-    // k-blocks).  With the update under a run-time condition inside one flat loop hipcc parked y in the accumulation registers and
-    // moved 200 registers per K step back and forth (v_accvgpr_read / write: as many issue cycles as the MFMAs).
-    auto update = [&](const int g) {
-#pragma unroll
-        for (int j = 0; j < GG_NF; ++j) {
-            const uint32_t pz = panel[g * 64 + wc * 32 + j * 16 + m16];
-            const float sg = h2f<DT>((uint16_t)(pz & 0xFFFF));
-            const float cg = -(OFF + __uint_as_float(pz & 0xFFFF0000u)) * sg;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) y[i][j][v] += sg * acc[i][j][v] + cg * xs[i][v];
-                acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) xs[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    };
-#define GG_STEP(S_) do { \
-        constexpr int s_ = (S_); \
-        const int kt = 4 * kb + s_; \
-        const bool snext = kt + 2 < nkt; \
-        if (snext) stage(kt + 2, (kt + 2) % 3); \
-        constexpr bool wstep = !(s_ & 1); \
-        const bool wnext = wstep && 2 * kb + (s_ >> 1) + 1 < nh; \
-        if (wnext) wload(((s_ >> 1) & 1) ^ 1, 2 * kb + (s_ >> 1) + 1); \
-        const uint8_t* A = smem + (size_t)(kt % 3) * 16384; \
-        _Pragma("unroll") for (int s2 = 0; s2 < 2; ++s2) { \
-            uint4 af[4]; \
-            _Pragma("unroll") for (int i = 0; i < 4; ++i) { \
-                const uint4 v = *reinterpret_cast<const uint4*>(A + (size_t)arow[i] * 128 + (size_t)(((s2 * 4 + kg) ^ (arow[i] & 7)) * 16)); \
-                af[i].x = __builtin_amdgcn_perm(v.z, v.x, 0x05040100u); \
-                af[i].y = __builtin_amdgcn_perm(v.z, v.x, 0x07060302u); \
-                af[i].z = __builtin_amdgcn_perm(v.w, v.y, 0x05040100u); \
-                af[i].w = __builtin_amdgcn_perm(v.w, v.y, 0x07060302u); \
-                xs[i] = mfma32<DT>(af[i], ones, xs[i]); \
-            } \
-            _Pragma("unroll") for (int j = 0; j < GG_NF; ++j) { \
-                const dg_u32x4 wv = wq[(s_ >> 1) & 1][j]; \
-                const uint32_t w = ((s_ & 1) * 2 + s2) == 0 ? wv.x : ((s_ & 1) * 2 + s2) == 1 ? wv.y : ((s_ & 1) * 2 + s2) == 2 ? wv.z : wv.w; \
-                uint4 b; \
-                b.x = (w & nib) | KOFF; b.y = ((w >> 4) & nib) | KOFF; b.z = ((w >> 8) & nib) | KOFF; b.w = ((w >> 12) & nib) | KOFF; \
-                _Pragma("unroll") for (int i = 0; i < 4; ++i) acc[i][j] = mfma32<DT>(af[i], b, acc[i][j]); \
-            } \
-        } \
-        /* the tile of step kt + 1 (DMA issued one step ago) must have landed; younger than it: the weight loads of the previous step \
-           (odd steps) or of this one (even steps), and this step's DMA */ \
-        { \
-            const int younger = (snext ? 4 : 0) + ((wstep ? wnext : wprev) ? GG_NF : 0); \
-            if (younger >= 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); \
-            else if (younger == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); \
-            else if (younger == 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); \
-            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); \
-        } \
-        wprev = wnext; \
-        __syncthreads(); \
-        if constexpr (GPK == 1 || (GPK == 2 && (s_ & 1)) || (GPK == 4 && s_ == 3)) update(kt / (GPK ? GPK : 1)); \
-    } while (0)
-    bool wprev = false;
-    if constexpr (GPK != 0) {
-        for (int kb = 0; kb < nkb; ++kb) { GG_STEP(0); GG_STEP(1); GG_STEP(2); GG_STEP(3); }
-    } else {
-        const int kb_per_group = gs >> 8;
-        for (int g = 0; g < nkb / kb_per_group; ++g) {
-            for (int kbi = 0; kbi < kb_per_group; ++kbi) { const int kb = g * kb_per_group + kbi; GG_STEP(0); GG_STEP(1); GG_STEP(2); GG_STEP(3); }
-            update(g);
-        }
-    }
-#undef GG_STEP
-    // ---- epilogue (as dense_gemm_kernel): the lane holds tokens 4 kg + v of every m-fragment for column m16 of every n-fragment
-    const uint16_t* bias = static_cast<const uint16_t*>(a.bias);
-    const uint16_t* resid = static_cast<const uint16_t*>(a.resid);
-    uint16_t* out = static_cast<uint16_t*>(a.out);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int t = t0 + wr * 64 + i * 16 + 4 * kg + v;
-            if (t >= a.T) continue;
-            if (silu) {
-                const int col = c0 + wc * 16 + m16;
-                if (col < n_cols) {
-                    float g = rnd<DT>(y[i][0][v]), u = rnd<DT>(y[i][1][v]);
-                    if (bias) { g = rnd<DT>(g + h2f<DT>(bias[col])); u = rnd<DT>(u + h2f<DT>(bias[a.pair_offset + col])); }
-                    out[(size_t)t * a.ldo + col] = f2h<DT>(rnd<DT>(rnd<DT>(g / (1.f + __expf(-g))) * u));
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < GG_NF; ++j) {
-                    const int col = c0 + wc * 32 + j * 16 + m16;
-                    if (col >= n_cols) continue;
-                    float o = rnd<DT>(y[i][j][v]);
-                    if (bias) o = rnd<DT>(o + h2f<DT>(bias[col]));
-                    if (a.epi == MI355_EPI_RESID) o = rnd<DT>(o + h2f<DT>(resid[(size_t)t * a.ldo + col]));
-                    out[(size_t)t * a.ldo + col] = f2h<DT>(o);
-                }
-            }
-        }
 }
-static int gptq_prompt_gemm(const DenseArgs& a, int dt, hipStream_t st) {
+template <int DT, bool SYM, int XG>
+static void gptq_gemm_epi(const GptqGemm& g, int which, hipStream_t st) {
+    if (g.a[0].epi == MI355_EPI_SILU_MUL) gptq_gemm_tile<DT, MI355_EPI_SILU_MUL, SYM, XG>(g, which, st);
+    else if (g.a[0].epi == MI355_EPI_RESID) gptq_gemm_tile<DT, MI355_EPI_RESID, SYM, XG>(g, which, st);
+    else gptq_gemm_tile<DT, MI355_EPI_STORE, SYM, XG>(g, which, st);
+}
+template <int DT>
+static int gptq_gemm_dt(const GptqGemm& g, uint16_t* xp, float* xs, int which, hipStream_t st) {
+    const DenseArgs& a = g.a[0];
+    const int xg = a.group_size % GG_UNIT ? 64 : GG_UNIT;
+    int64_t xb = ((int64_t)a.T * (a.K >> 3) + 255) / 256, pb[3], all = xb;
+    for (int i = 0; i < 3; ++i) { pb[i] = g.tiles[i] ? ((int64_t)(a.K / a.group_size) * g.a[i].N + 255) / 256 : 0; all += pb[i]; }
+    if (all > 0x7FFFFFFF) return (int)hipErrorNotSupported;
+    if (xg == 64) hipLaunchKernelGGL((gptq_gemm_prep_kernel<DT, 64>), dim3((unsigned)all), dim3(256), 0, st, g, xp, xs, (int)xb, (int)pb[0], (int)pb[1]);
+    else hipLaunchKernelGGL((gptq_gemm_prep_kernel<DT, 128>), dim3((unsigned)all), dim3(256), 0, st, g, xp, xs, (int)xb, (int)pb[0], (int)pb[1]);
+    const bool sym = a.zmode == MI355_ZERO_SYM8 || !a.qzeros;
+    if (xg == 64) { if (sym) gptq_gemm_epi<DT, true, 64>(g, which, st); else gptq_gemm_epi<DT, false, 64>(g, which, st); }
+    else { if (sym) gptq_gemm_epi<DT, true, 128>(g, which, st); else gptq_gemm_epi<DT, false, 128>(g, which, st); }
+    return (int)hipGetLastError();
+}
+// n matrices over the same x, of one group size and zero mode
+static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) {
+    const DenseArgs& a = ms[0];
     const int gs = a.group_size;
-    if (g_tune_gptq_gemm_off || (a.K & 255) || (a.N & 15) || a.T < 4 || gs < 64 || (gs % 64) || (a.K % gs)) return (int)hipErrorNotSupported;
-    if ((a.ldx * 2) % 16 || ((uintptr_t)a.x & 15)) return (int)hipErrorNotSupported;
-    if (a.epi == MI355_EPI_SILU_MUL && (a.pair_offset <= 0 || a.N != 2 * a.pair_offset || (a.pair_offset & 15))) return (int)hipErrorNotSupported;
-    const int n_cols = a.epi == MI355_EPI_SILU_MUL ? a.pair_offset : a.N;
-    const int cols_per_wg = a.epi == MI355_EPI_SILU_MUL ? 32 : 64;
-    const dim3 grid((a.T + DG_BM - 1) / DG_BM, (n_cols + cols_per_wg - 1) / cols_per_wg);
-    const size_t lds = 3 * 16384 + (size_t)(a.K / gs) * 64 * sizeof(uint32_t);
-    if (lds > 152 * 1024) return (int)hipErrorNotSupported;
-    const int gpk = gs == 64 ? 1 : gs == 128 ? 2 : gs == 256 ? 4 : 0;
-    if (gpk == 0 && (gs % 256)) return (int)hipErrorNotSupported;
-#define GG_GO(DT_, GPK_) do { \
-        static bool attr_ = false; \
-        if (!attr_) { (void)hipFuncSetAttribute((const void*)gptq_gemm_kernel<DT_, GPK_>, hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024); attr_ = true; } \
-        hipLaunchKernelGGL((gptq_gemm_kernel<DT_, GPK_>), grid, dim3(256), lds, st, a); } while (0)
-#define GG_DT(DT_) do { if (gpk == 1) GG_GO(DT_, 1); else if (gpk == 2) GG_GO(DT_, 2); else if (gpk == 4) GG_GO(DT_, 4); else GG_GO(DT_, 0); } while (0)
-    if (dt == MI355_DTYPE_BF16) GG_DT(MI355_DTYPE_BF16);
-    else if (dt == MI355_DTYPE_F16) GG_DT(MI355_DTYPE_F16);
-#undef GG_DT
-#undef GG_GO
-    else return (int)hipErrorNotSupported;
+    const bool silu = a.epi == MI355_EPI_SILU_MUL;
+    if (dt != MI355_DTYPE_BF16 && dt != MI355_DTYPE_F16) return (int)hipErrorNotSupported;
+    if (g_tune_gptq_gemm_off || (a.K & 255) || a.T < 4 || gs < 64 || (gs % 64) || (a.K % gs) || (gs > 128 && gs % 128)) return (int)hipErrorNotSupported;
+    if ((a.ldx * 2) % 16 || ((uintptr_t)a.x & 15) || (int64_t)a.K * 512 >= (1ll << 32)) return (int)hipErrorNotSupported;
+    int64_t rows = 0, words = 0;
+    for (int i = 0; i < n; ++i) {
+        if ((ms[i].N & 15) || ms[i].epi != a.epi || ms[i].zmode != a.zmode || !ms[i].qzeros != !a.qzeros) return (int)hipErrorNotSupported;
+        rows += ms[i].N;
+        words += ((int64_t)(a.K / gs) * ms[i].N + 63) / 64 * 64;
+    }
+    if (silu && (a.pair_offset <= 0 || a.N != 2 * a.pair_offset || (a.pair_offset & 15))) return (int)hipErrorNotSupported;
+    GptqGemm g{};
+    auto tiles = [&](const GtTile& t) {
+        int64_t c = 0;
+        for (int i = 0; i < n; ++i) c += g.tiles[i] = silu ? (a.pair_offset + t.bn / 2 - 1) / (t.bn / 2) : (ms[i].N + t.bn - 1) / t.bn;
+        return c * ((a.T + t.bm - 1) / t.bm);
+    };
+    // us per launch (Qwen2-7B's layers, groups of 128; the 128 x 64 kernel that unpacked 128 k per wave and step, then this one): gate/up 37888 x 3584
+    // at 700 tokens 695 / 236, at 2048 2030 / 560; down 3584 x 18944 at 700 470 / 118 (three ranges), at 64 (chunks of the decode kernel) 78 / 30
+    // (64-token tiles, eight ranges), at 96 102 / 36.
+    const int units = a.K / GG_UNIT;
+    const GtChoice best = gt_pick(tiles, units, (float)rows * (float)a.K / 2.f / 5.0e6f, n == 1 && a.T <= 65535 ? std::min(16, std::max(1, units / 4)) : 1,
+                                  (float)a.T * (float)a.N * 4.f / 4.5e6f, gs % GG_UNIT ? 6 : 7, kGgTiles, 3);
+    const GtTile& t = kGgTiles[best.tile];
+    for (int i = 0; i < 3; ++i) g.a[i] = ms[i < n ? i : 0];
+    g.n_m = (a.T + t.bm - 1) / t.bm; g.t_pad = (a.T + 255) / 256 * 256 + 256;   // (a DMA of the sums reads 256 tokens from the tile's first)
+    g.units_per_split = (units + best.splits - 1) / best.splits;
+    g.splits = (units + g.units_per_split - 1) / g.units_per_split;
+    if (tiles(t) * g.splits > 0x7FFFFFFF) return (int)hipErrorNotSupported;
+    // workspace: permuted x | sums | panels | partial sums
+    const size_t xp_b = (size_t)a.T * a.K * 2, xs_b = (size_t)(a.K / 64) * g.t_pad * 4, pn_b = (size_t)words * 4;
+    const size_t pt_b = g.splits > 1 ? (size_t)g.splits * a.T * a.N * 4 : 0;
+    void* ws = nullptr;
+    if (mi355_scratch_get(&ws, MI355_SCR_GPTQ_GEMM, xp_b + xs_b + pn_b + pt_b, st, false)) return (int)hipErrorNotSupported;   // (no room while a stream is captured: token chunks)
+    uint8_t* base = static_cast<uint8_t*>(ws);
+    uint16_t* xp = reinterpret_cast<uint16_t*>(base);
+    float* xs = reinterpret_cast<float*>(base + xp_b);
+    uint32_t* panel = reinterpret_cast<uint32_t*>(base + xp_b + xs_b);
+    g.xp = xp; g.xs = xs; g.part = reinterpret_cast<float*>(base + xp_b + xs_b + pn_b);
+    for (int i = 0; i < n; ++i) { g.panel[i] = panel; panel += ((int64_t)(a.K / gs) * ms[i].N + 63) / 64 * 64; }
+    const int rc = dt == MI355_DTYPE_BF16 ? gptq_gemm_dt<MI355_DTYPE_BF16>(g, xp, xs, best.tile, st) : gptq_gemm_dt<MI355_DTYPE_F16>(g, xp, xs, best.tile, st);
+    if (rc || g.splits <= 1) return rc;
+    const dim3 grid(((silu ? a.pair_offset : a.N) + 255) / 256, a.T);
+    if (dt == MI355_DTYPE_BF16) hipLaunchKernelGGL((gptq_wide_epilogue_kernel<MI355_DTYPE_BF16>), grid, dim3(256), 0, st, a, g.part, a.N, g.splits, a.T);
+    else hipLaunchKernelGGL((gptq_wide_epilogue_kernel<MI355_DTYPE_F16>), grid, dim3(256), 0, st, a, g.part, a.N, g.splits, a.T);
     return (int)hipGetLastError();
 }
 
@@ -1553,8 +1419,8 @@ static int dense_run(DenseArgs a, int wtype, int dt, hipStream_t st) {
         const int rc = dense_prompt_gemm(&a, 1, dt, st);
         if (rc != (int)hipErrorNotSupported) return rc;                    // odd strides / K: keep streaming in token chunks
     }
-    if (wtype == DW_GPTQ4T && a.T >= std::max(g_tune_gemm_min_t, (int)GPTQ_GEMM_MIN_T)) {
-        const int rc = gptq_prompt_gemm(a, dt, st);
+    if (wtype == DW_GPTQ4T && a.T >= (a.epi == MI355_EPI_SILU_MUL ? GPTQ_GEMM_MIN_PAIR_T : GPTQ_GEMM_MIN_T)) {
+        const int rc = gptq_prompt_gemm(&a, 1, dt, st);
         if (rc != (int)hipErrorNotSupported) return rc;                    // groups of 32, odd strides: token chunks of the decode kernel
     }
     const int chunk = a.epi == MI355_EPI_SILU_MUL ? 32 : 64;
@@ -1965,7 +1831,7 @@ int mi355_internal_linear3(void* const* outs, const void* x, const void* const* 
                            const void* const* biases, const int32_t* ns, int32_t num_tokens, int32_t k, int32_t group_size,
                            int32_t is_gptq, int32_t dtype, const void* norm_w, float norm_eps, const float* ss_in, const void* rope,
                            int64_t stream) {
-    const bool prompt = num_tokens >= g_tune_gemm_min_t && (is_gptq == 0 || is_gptq == 3) && !norm_w && !rope;   // one GEMM launch for the three
+    const bool prompt = !norm_w && !rope && (is_gptq == 2 ? num_tokens >= GPTQ_GEMM_MIN_T : is_gptq != 1 && num_tokens >= g_tune_gemm_min_t);   // one GEMM launch for the three
     if (num_tokens < 1 || (num_tokens > 64 && !prompt) || (k & 255)) return -4;
     const DenseRope* rp = static_cast<const DenseRope*>(rope);
     DenseArgs a[3];
@@ -1983,8 +1849,9 @@ int mi355_internal_linear3(void* const* outs, const void* x, const void* const* 
     }
     hipStream_t st = (hipStream_t)stream;
     if (prompt) {
-        const int rc = dense_prompt_gemm(a, 3, dtype, st);
-        return rc == (int)hipErrorNotSupported ? -4 : rc;
+        const int rc = is_gptq == 2 ? gptq_prompt_gemm(a, 3, dtype, st) : dense_prompt_gemm(a, 3, dtype, st);
+        if (rc != (int)hipErrorNotSupported) return rc;
+        if (num_tokens > 64) return -4;
     }
     if (dtype == MI355_DTYPE_BF16)
         return is_gptq == 2 ? dense3_launch_dt<MI355_DTYPE_BF16, DW_GPTQ4T>(a, rp, st)

@@ -173,15 +173,15 @@ static constexpr GtTile kGtTiles[] = {{256, 256, 1, 1.46f}, {192, 256, 1, 1.28f}
 struct GtChoice { int tile, splits; };
 // tiles(t): workgroups of the launch with tile t; stream_us: the weights' read; part_us: write or read of one range's partial sums
 template <class F>
-static inline GtChoice gt_pick(F tiles, int units, float stream_us, int max_split, float part_us, unsigned allowed) {
+static inline GtChoice gt_pick(F tiles, int units, float stream_us, int max_split, float part_us, unsigned allowed, const GtTile* table = kGtTiles, int n_table = 5) {
     const int cus = mi355_num_cus();
     GtChoice best{-1, 1};
     float cost = 0.f;
-    for (int i = 0; i < 5; ++i)
+    for (int i = 0; i < n_table; ++i)
         for (int s = 1; s <= max_split; ++s) {
             if (!(allowed >> i & 1)) continue;
-            const int64_t wgs = (int64_t)cus * kGtTiles[i].per_cu, rounds = (tiles(kGtTiles[i]) * s + wgs - 1) / wgs;
-            const float t = (float)rounds * (float)((units + s - 1) / s + 2) * kGtTiles[i].us;
+            const int64_t wgs = (int64_t)cus * table[i].per_cu, rounds = (tiles(table[i]) * s + wgs - 1) / wgs;
+            const float t = (float)rounds * (float)((units + s - 1) / s + 2) * table[i].us;
             const float c = (t > stream_us ? t : stream_us) + (s > 1 ? 5.f + part_us * (float)(s + 1) : 0.f);
             if (best.tile < 0 || c < cost) { best = {i, s}; cost = c; }
         }

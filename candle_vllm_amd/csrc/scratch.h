@@ -15,6 +15,7 @@ enum {
     MI355_SCR_COMM = 9,          // one-shot all-reduce staging
     MI355_SCR_GPTQ_WIDE = 10,    // 5..64-token launches of tiled 4-bit weights: split-K partial sums (gptq_wide.inc)
     MI355_SCR_PF_FP8 = 11,       // prompt attention over an e4m3 cache: the sequences' blocks as bf16 + their block table (prefill_attention.hip)
+    MI355_SCR_GPTQ_GEMM = 13,    // 4-bit prompt GEMM: permuted x, its sums, scale panel, split-K partial sums (gptq_gemm.inc)
     MI355_SCR_DELTA = 12,        // delta rule by pieces: the pieces' records (hybrid_delta.hip)
 };
 

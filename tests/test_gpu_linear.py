@@ -446,6 +446,32 @@ def test_gptq_prompt_gemm_one_pass(cv, dt, T, N, K, gs, mode):
     check_ulp(y0, ref, dt, ulps=ulps, what="decode kernel in chunks", mag=mag)
 
 
+@pytest.mark.parametrize("T,N,K,gs,mode", [(33, 272, 4352, 128, "resid"), (65, 48, 2048, 64, "zp"),   # 64-token tiles, K in ranges; one token into the next
+                                           (65, 160, 768, 256, "silu"), (300, 4176, 256, 128, "zp"),   # ... pairs; 128 x 128
+                                           (900, 8192, 256, 128, "store"), (1100, 8224, 512, 512, "silu")])   # 128 x 256: exactly one per CU; ragged
+def test_gptq_prompt_gemm_every_tile(cv, T, N, K, gs, mode):
+    """the one-pass 4-bit prompt GEMM where its dispatch takes each of its tiles and K ranges, tokens at the tiles' edges, at the oracle's bound"""
+    dt = "bf16"
+    rng = np.random.default_rng(T + N + K)
+    q, s = _gptq_case(rng, K, N, gs, dt)
+    x = G.round_dt(rng.normal(0, 1, (T, K)), dt)
+    z = rng.integers(1, 17, (K // gs, N)) if mode == "zp" else None
+    kw = {"qzeros": dev_u32(G.gptq_pack_zeros(z)), "zero_mode": cv.ZERO_GPTQ_PLUS1} if z is not None else {}
+    lin = cv.GPTQLinear(dev_u32(G.gptq_pack(q)), dev16(s, dt), gs, **kw)
+    rows = np.unique([t for e in range(0, T, 64) for t in (e, e + 1, e + 63, T - 1) if t < T])
+    res = G.round_dt(rng.normal(0, 1, (T, N)), dt)
+    y = G.gptq_linear(x[rows], G.gptq_dequant(q, s, z, gs), None, dt)
+    if mode == "silu":
+        got, ref, ulps, mag = lin.forward(dev16(x, dt), epilogue=cv.EPI_SILU_MUL), G.silu_mul16(y[:, :N // 2], y[:, N // 2:], dt), 3.0, None
+    elif mode == "resid":
+        got, ref, ulps, mag = lin.forward(dev16(x, dt), epilogue=cv.EPI_RESID, residual=dev16(res, dt)), G.round_dt(y + res[rows], dt), 2.01, y
+    else:
+        got, ref, ulps, mag = lin.forward(dev16(x, dt)), y, 1.01, None
+    got = host16(got, dt)
+    assert np.isfinite(got).all()
+    check_ulp(got[rows], ref, dt, ulps=ulps, what="gptq prompt GEMM", mag=mag)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("T,N,K,gs,mode", [(32, 1184, 3584, 128, "store"), (32, 3584, 3584, 128, "resid"), (9, 224, 2048, 64, "store"),
                                            (48, 512, 4864, 256, "bias"), (17, 2 * 4736, 1792, 128, "silu"), (32, 2 * 608, 3584, 128, "silu"),
