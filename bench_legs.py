@@ -101,7 +101,7 @@ def leg_bf16_b32(steps=16, warmup=3):
 
 def leg_bf16_prompt(T=2048):
     """one prompt step of T tokens through the 16-bit host layer (dense_model.cpp): Llama-3-8B bf16, every projection on the
-    hand-written 128 x 128 MFMA GEMM (dense_gemv.hip dense_gemm_kernel), prefill attention, cache write -- tokens/s and the useful
+    hand-written MFMA GEMM (dense_gemv.hip dense_gemm_kernel), prefill attention, cache write -- tokens/s and the useful
     TFLOP/s of the weight GEMMs (2 * parameters * T; attention's flops not counted)"""
     import torch
     from candle_vllm_amd import dense_model as DM

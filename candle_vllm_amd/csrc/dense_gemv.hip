@@ -1082,7 +1082,7 @@ static int dense_dispatch(const DenseArgs& a, int wtype, int dt, hipStream_t st)
     return -2;
 }
 
-// ---- prompt steps (T >= 96, dense 16-bit weights): the matmul is compute-bound -> a hand-written MFMA GEMM
+// ---- prompt steps (T >= DENSE_GEMM_MIN_T, dense 16-bit weights): the matmul is compute-bound -> a hand-written MFMA GEMM
 // (`Linear::forward` on prompt chunks, linear.rs:124-172; packed gate_up of mlp.rs:324-352,440-458) around the main loop of gemm_tile.h.
 //   * candle's rounding chain in the epilogue, from the f32 accumulators: round to the dtype, + bias (rounded), then
 //     + residual (rounded) or silu(gate) rounded * up rounded -- no separate chain kernel, no f32 / 16-bit staging of y;
@@ -1295,7 +1295,7 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     if ((a.ldx * 2) % 16 || ((uintptr_t)a.x & 15) || (int64_t)a.K * 512 >= (1ll << 32)) return (int)hipErrorNotSupported;
     int64_t rows = 0, words = 0;
     for (int i = 0; i < n; ++i) {
-        if ((ms[i].N & 15) || ms[i].epi != a.epi || ms[i].zmode != a.zmode || !ms[i].qzeros != !a.qzeros) return (int)hipErrorNotSupported;
+        if ((ms[i].N & 15) || ((uintptr_t)ms[i].w & 15) || ms[i].epi != a.epi || ms[i].zmode != a.zmode || !ms[i].qzeros != !a.qzeros) return (int)hipErrorNotSupported;
         rows += ms[i].N;
         words += ((int64_t)(a.K / gs) * ms[i].N + 63) / 64 * 64;
     }
@@ -1364,7 +1364,7 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     if (dt != MI355_DTYPE_BF16 && dt != MI355_DTYPE_F16) return (int)hipErrorNotSupported;
     for (int i = 0; i < n; ++i) {
         if (a[i].K % 64 || a[i].T < 1 || a[i].N < 1 || a[i].wtiled != a[0].wtiled || a[i].epi != a[0].epi) return (int)hipErrorNotSupported;
-        if ((a[i].ldx * 2) % 16 || (!a[i].wtiled && (a[i].ldw * 2) % 16)) return (int)hipErrorNotSupported;          // 16-byte DMA pieces
+        if ((a[i].ldx * 2) % 16 || (!a[i].wtiled && (a[i].ldw * 2) % 16) || (((uintptr_t)a[i].x | (uintptr_t)a[i].w) & 15)) return (int)hipErrorNotSupported;   // 16-byte DMA pieces
         if (a[i].epi == MI355_EPI_SILU_MUL && (a[i].pair_offset <= 0 || a[i].N != 2 * a[i].pair_offset)) return (int)hipErrorNotSupported;
         if (a[i].epi == MI355_EPI_SILU_MUL && a[i].wtiled && (a[i].pair_offset & 15)) return (int)hipErrorNotSupported;
         if ((int64_t)a[i].ldx * 512 >= (1ll << 32) || (int64_t)a[i].ldw * 512 >= (1ll << 32)) return (int)hipErrorNotSupported;   // 32-bit offsets inside a tile

@@ -2219,7 +2219,7 @@ struct TuningInit {
         // probe builds: every key has a live value from the start (the defaults of the variables the setters write: a scoped
         // set / restore of a never-set key used to "restore" 0, which several setters ignore and which switches others off)
         static const int32_t kProbeDefaults[][2] = {{0, 0}, {1, 0}, {2, 0}, {10, 1024}, {11, 2}, {12, 96}, {14, 1}, {15, 0}, {16, 4096}, {17, 2}, {18, 0},
-                                                    {20, 0}, {21, 8}, {22, 0}, {23, 0}, {33, 0}, {34, 0}, {35, 0}, {36, 96}, {37, 0}, {38, 4},
+                                                    {20, 0}, {21, 8}, {22, 0}, {23, 0}, {33, 0}, {34, 0}, {35, 0}, {36, 33}, {37, 0}, {38, 4},
                                                     {42, 1}, {49, 0}};
         for (const auto& kv : kProbeDefaults) { g_tune_shadow[kv[0]] = kv[1]; g_tune_shadow_set[kv[0]] = true; }
 #endif

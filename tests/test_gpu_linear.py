@@ -108,6 +108,21 @@ def test_linear_prompt_gemm_every_tile(cv, T, N, K):
         assert np.isfinite(outs[0]).all()
 
 
+@pytest.mark.parametrize("T", [17, 33, 100])
+@pytest.mark.parametrize("off_x,off_w", [(4, 0), (0, 4)])
+def test_linear_prompt_operands_off_the_16_byte_grid(cv, T, off_x, off_w):
+    """x or w that do not start on 16 bytes stay with the kernels that read them element-aligned: same bound (the GEMM copies 16-byte pieces)"""
+    from candle_vllm_amd._lib import lib
+    dt, N, K, st = "bf16", 96, 512, torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(T + 8 * off_x + off_w)
+    x, w = G.round_dt(rng.normal(0, 1, (T, K)), dt), G.round_dt(rng.normal(0, 0.05, (N, K)), dt)
+    xd, wd = (torch.zeros(v.size + 8, dtype=torch.bfloat16, device="cuda") for v in (x, w))
+    xd[off_x:off_x + x.size], wd[off_w:off_w + w.size] = dev16(x, dt).flatten(), dev16(w, dt).flatten()
+    out = torch.empty((T, N), dtype=torch.bfloat16, device="cuda")
+    assert lib.mi355_linear(out.data_ptr(), xd[off_x:].data_ptr(), wd[off_w:].data_ptr(), None, None, T, N, K, 2, 0, st) == 0
+    check_ulp(host16(out, dt), G.linear16(x, w, None, dt), dt, what="unaligned operands")
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("T,N,K", [(256, 384, 1024), (300, 200, 576), (97, 130, 64), (700, 128, 256)])
 def test_linear_prompt_gemm_tall_tile(cv, dt, T, N, K):
