@@ -78,6 +78,34 @@ def test_reshape_and_cache_bit_exact(cv, flash, Hkv, D, bs):
     assert np.array_equal(bf16_bits(vcd), vc)
 
 
+@pytest.mark.parametrize("T,Hkv,D,bs", [(63, 2, 128, 16), (64, 8, 128, 64), (65, 1, 8, 16), (143, 3, 80, 32), (200, 4, 64, 7)])
+@pytest.mark.parametrize("shift", [0, 4])                         # values in front of the rows: on the 16-byte grid, off it
+def test_reshape_and_cache_prompt_rows_bit_exact(cv, lib, T, Hkv, D, bs, shift):
+    """16-bit paged rows of prompts, groups of 16 tokens per workgroup: runs of slots that start and end anywhere in a block, pads, a ragged last group,
+    rows off the 16-byte grid (the kernel of one token per workgroup) -- bit for bit, and nothing else written"""
+    rng = np.random.default_rng(T + D + shift)
+    NB = (T + 3 * bs) // bs + 4
+    ks, vs = O.kv_cache_shapes(NB, bs, Hkv, D, 2, False)
+    kc, vc = rng.integers(0, 65536, ks).astype(np.uint16), rng.integers(0, 65536, vs).astype(np.uint16)
+    k, v = rng.integers(0, 65536, (T, Hkv, D)).astype(np.uint16), rng.integers(0, 65536, (T, Hkv, D)).astype(np.uint16)
+    cut = T // 3                                                  # two sequences: runs of slots from 3 and, behind a gap, on
+    slots = np.concatenate([np.arange(3, 3 + cut), np.arange(cut + 5 + bs, cut + 5 + bs + T - cut)]).astype(np.int64)
+    slots[[5, T - 2]] = -1
+    kcd, vcd = bf16_dev(kc), bf16_dev(vc)
+    rows = []
+    for a in (k, v):
+        buf = torch.zeros(a.size + 8, dtype=torch.bfloat16, device="cuda")
+        buf[shift:shift + a.size] = bf16_dev(a).flatten()
+        rows.append(buf[shift:])
+    slots_d = dev(slots)
+    rc = lib.mi355_reshape_and_cache(rows[0].data_ptr(), rows[1].data_ptr(), kcd.data_ptr(), vcd.data_ptr(), slots_d.data_ptr(), T, Hkv, D, bs, 2,
+                                     cv.KV_PAGED, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    O.reshape_and_cache(k, v, kc, vc, slots, False)
+    assert np.array_equal(bf16_bits(kcd), kc) and np.array_equal(bf16_bits(vcd), vc)
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_copy_blocks_bit_exact(cv, dtype):
     rng = np.random.default_rng(2)
