@@ -198,6 +198,26 @@ def test_rope_inplace(cv, interleaved, H, Hkv, D, rot):
     assert rel_err(qd.cpu().numpy(), rq) < 1e-6 and rel_err(kd.cpu().numpy(), rk) < 1e-6
 
 
+@pytest.mark.parametrize("interleaved", [True, False])
+@pytest.mark.parametrize("T,H,Hkv,D,rot", [(64, 32, 8, 128, 128), (77, 3, 1, 80, 16), (130, 5, 2, 64, 32), (200, 1, 1, 16, 16)])
+def test_rope_prompt_rows_equal_few_rows(cv, T, H, Hkv, D, rot, interleaved):
+    """bf16 rows of prompts, eight pairs per thread == the same rows in calls of at most 50 tokens (one pair per thread), bit for bit, the values
+    behind the rotated part untouched -- and within a bf16 rounding of the oracle"""
+    rng = np.random.default_rng(T + D)
+    q, k = rng.normal(size=(T, H, D)).astype(np.float32), rng.normal(size=(T, Hkv, D)).astype(np.float32)
+    pos = rng.integers(0, 300, T).astype(np.int64)
+    cos, sin = O.rope_tables(500000.0, rot, 300)
+    cd, sd, pd = dev(cos), dev(sin), dev(pos)
+    qw, kw = dev(q, torch.bfloat16), dev(k, torch.bfloat16)
+    want = O.rope_apply(qw.float().cpu().numpy(), cos, sin, pos, interleaved, rot)
+    qf, kf = qw.clone(), kw.clone()
+    cv.FusedRope.apply_inplace_partial(qw, kw, cd, sd, pd, interleaved, rot)
+    for t in range(0, T, 50):
+        cv.FusedRope.apply_inplace_partial(qf[t:t + 50], kf[t:t + 50], cd, sd, pd[t:t + 50], interleaved, rot)
+    assert torch.equal(qw.view(torch.int16), qf.view(torch.int16)) and torch.equal(kw.view(torch.int16), kf.view(torch.int16))
+    assert np.abs(qw.float().cpu().numpy() - want).max() <= 2 ** -8 * np.abs(want).max()
+
+
 def test_silu_mul_add_cast_embedding_argmax(cv):
     rng = np.random.default_rng(7)
     g = rng.normal(0, 3, (5, 14336)).astype(np.float32)
