@@ -152,7 +152,12 @@ template <int DP, int LPC, int CH> __global__ __launch_bounds__(256) void delta_
 //   S <- diag(G_16) S + K_hat^T U,  K_hat[s] = k_s prod_(s < r) g_r
 // so that everything but U, O and S is known for all pieces at once: `prepare` makes W = (I + A)^-1 diag(beta) K_G and X = (I + A)^-1 diag(beta) V
 // by forward substitution, and the scan is U = X - W S and the two lines below it, on the f32 matrix cores.  Only products of decays are
-// formed, never their quotients: nothing over- or underflows that the walk keeps.  What bounds it: the chain over the pieces, about 24
+// formed, never their quotients: nothing over- or underflows that the walk keeps.
+// What is summed enters what it is added to by one rounding (forward substitution, K_hat^T U into the state, M U), the unit vectors' factors are
+// rounded once, and the decays' products G are formed in 64 bits.  Error against 64 bits (2-norm) of outputs / state, 16 heads of 128, 2048 tokens:
+// walk 1.81e-7 / 1.55e-7, pieces with every step in f32 and sums run on from their start 1.95e-7 / 1.76e-7, as here 1.46e-7 / 1.25e-7;
+// 200 tokens 1.77 / 1.59, 1.85 / 1.71, 1.26 / 1.18; at the same time (195 us; 64-wide heads 163 -> 167).
+// What bounds it: the chain over the pieces, about 24
 // f32 MFMAs of 32 cycles and one barrier each (0.88 us per 16 tokens against 0.36 us per ONE token of the walk); `prepare` (83 us for 2048
 // tokens) the logarithms and exponentials of the decays and the walks of the keys inside a piece.
 // A record per (piece, head), in the order the scan's lanes read it, 16 B each: W, Q_G [d / 16][lane = 16 (c % 16 / 4) + t][c % 4],
@@ -163,9 +168,24 @@ __host__ __device__ __forceinline__ int64_t delta_rec_floats(int d, int vd) { re
 // pieces of sequence s start at number cu_q[s] / 16 + s: room for every sequence's last, shorter piece without a table
 __device__ __forceinline__ int delta_first_piece(const uint32_t* cu_q, int s) { return (int)(cu_q[s] / DPC) + s; }
 
+// x / sqrt(s), rounded about once: the f32 root and quotient with one step of Newton's method in 64 bits, as the sum of two f32
+// (where that step has no value, s = 0 or infinite, the quotient stands)
+struct DeltaRoot { float hi, lo; };
+__device__ __forceinline__ DeltaRoot delta_rsqrt(double s) {
+    const float y = 1.f / sqrtf((float)s);
+    const double e = fma(-s * (double)y, (double)y, 1.), z = fma(0.5 * (double)y, e, (double)y);
+    if (!(fabs(e) < 1.)) return {y, 0.f};
+    return {(float)z, (float)(z - (double)(float)z)};
+}
+__device__ __forceinline__ float delta_scaled(float x, const DeltaRoot& r) { return fmaf(x, r.hi, x * r.lo); }
+
 template <int DP> __global__ __launch_bounds__(256, 3) void delta_piece_prepare_kernel(DeltaArgs p, DeltaPieces q) {
     constexpr int D = 16 * DP, RS = D + 4;                             // channels of a row, rounded up; floats per LDS row
     __shared__ __align__(16) float sq[DPC][RS], sk[DPC][RS], sg[DPC][RS];
+    // 2^25 (decay - sg), 11 bits of it: a decay is at most 1, so this is too.  (Not for 256 channels: three workgroups of 52 KB fill a CU's LDS,
+    // and two took 154 us instead of 139 for 8 x 128 tokens; the error is below the walk's there without it)
+    constexpr bool LOW = DP <= 8;
+    __shared__ __align__(16) _Float16 sl[LOW ? DPC : 1][RS];
     __shared__ float sA[DPC][DPC], sb[DPC], sM[DPC][DPC];
     const int piece = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, row = tid >> 4, part = tid & 15;
     const int d = p.d, vd = p.vd, g = h / (p.H / p.G);
@@ -187,21 +207,23 @@ template <int DP> __global__ __launch_bounds__(256, 3) void delta_piece_prepare_
             qq += qv[r] * qv[r]; kk += kv[r] * kv[r];
         }
         qq = column_sum<16>(qq); kk = column_sum<16>(kk);
-        const float qi = (1.f / sqrtf((float)d)) / sqrtf(qq + p.unit_eps), ki = 1.f / sqrtf(kk + p.unit_eps);
+        const DeltaRoot qi = delta_rsqrt((double)d * ((double)qq + (double)p.unit_eps)), ki = delta_rsqrt((double)kk + (double)p.unit_eps);
         const float rate = expf(p.a_log[h]);
-        float gh = 1.f;
-        if (!p.decay_channels && live) gh = expf(-rate * softplusf_(p.decay_in[(size_t)t * p.ldd + h] + p.dt_bias[h]));
+        double gh = 1.;
+        if (!p.decay_channels && live) gh = exp((double)(-rate * softplusf_(p.decay_in[(size_t)t * p.ldd + h] + p.dt_bias[h])));
 #pragma unroll
         for (int r = 0; r < DP; ++r) {
             const int i = part + 16 * r;
-            sq[row][i] = qv[r] * qi; sk[row][i] = kv[r] * ki;
+            sq[row][i] = delta_scaled(qv[r], qi); sk[row][i] = delta_scaled(kv[r], ki);
         }
 #pragma unroll 2
         for (int r = 0; r < DP; ++r) {                                   // (all at once they take the registers of two more waves)
             const int i = part + 16 * r;
-            float gv = gh;
-            if (p.decay_channels && live && i < d) gv = expf(-rate * softplusf_(p.decay_in[(size_t)t * p.ldd + h * d + i] + p.dt_bias[h * d + i]));
-            sg[row][i] = gv;
+            double gv = gh;
+            if (p.decay_channels && live && i < d) gv = exp((double)(-rate * softplusf_(p.decay_in[(size_t)t * p.ldd + h * d + i] + p.dt_bias[h * d + i])));
+            const float gf = (float)gv;
+            sg[row][i] = gf;
+            if constexpr (LOW) sl[row][i] = (_Float16)((float)(gv - (double)gf) * 0x1p25f);
         }
         if (part == 0) sb[row] = live ? sigmoidf_(p.proj[(size_t)t * p.ldp + p.b_off + h]) : 0.f;
     }
@@ -238,25 +260,27 @@ template <int DP> __global__ __launch_bounds__(256, 3) void delta_piece_prepare_
     // ---- a column of K_G or V per thread: forward substitution
     for (int c = tid; c < d + vd; c += 256) {
         const bool key = c < d;
-        float x[DPC], G = 1.f;
+        float x[DPC];
+        double G = 1.;
 #pragma unroll
         for (int t = 0; t < DPC; ++t) {
-            float v;
+            float v, a = 0.f;
             if (key) {
-                G *= sg[t][c];
-                v = sk[t][c] * G;
-                rec[DPC * (size_t)d + (size_t)(c >> 4) * 256 + (16 * ((c & 15) >> 2) + t) * 4 + (c & 3)] = sq[t][c] * G;
+                G *= LOW ? (double)sg[t][c] + (double)((float)sl[LOW ? t : 0][c] * 0x1p-25f) : (double)sg[t][c];
+                const float Gf = (float)G;
+                v = sk[t][c] * Gf;
+                rec[DPC * (size_t)d + (size_t)(c >> 4) * 256 + (16 * ((c & 15) >> 2) + t) * 4 + (c & 3)] = sq[t][c] * Gf;
             } else {
                 v = t0 + t < te ? p.qkv[(size_t)(t0 + t) * p.ldq + 2 * p.G * d + h * vd + (c - d)] : 0.f;
             }
             v *= sb[t];
             if (t & 1) asm volatile("" ::: "memory");                    // two rows of A in registers at a time, not all of them (172 registers: half the waves)
 #pragma unroll
-            for (int r = 0; r < t; ++r) v = fmaf(-sA[t][r], x[r], v);
-            x[t] = v;
+            for (int r = 0; r < t; ++r) a = fmaf(sA[t][r], x[r], a);
+            x[t] = v - a;                                                // (the sum by itself: its roundings are smaller than v's)
         }
         if (key) {
-            rec[3 * DPC * (size_t)d + c] = G;
+            rec[3 * DPC * (size_t)d + c] = (float)G;
 #pragma unroll
             for (int t = 0; t < DPC; ++t) rec[(size_t)(c >> 4) * 256 + (16 * ((c & 15) >> 2) + t) * 4 + (c & 3)] = x[t];
         } else {
@@ -295,9 +319,11 @@ template <int ND, bool FULL> __global__ __launch_bounds__(320) void delta_piece_
             const f32x4_t U = r.x - sum4(sw[i & 1]), m = r.m;
             fetch(r, i + 3);
             meet();                                                      // Q_G S of piece i (and W S of piece i + 1)
-            f32x4_t o = sum4(so[i & 1]);
+            f32x4_t qs = sum4(so[i & 1]), o = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            asm volatile("" : "+v"(qs));                                 // in hand first: these products are not on the chain, and a wave that is shares their SIMD
 #pragma unroll
-            for (int v = 0; v < 4; ++v) o = __builtin_amdgcn_mfma_f32_16x16x4f32(m[v], U[v], o, 0, 0, 0);
+            for (int v = 0; v < 4; ++v) o = __builtin_amdgcn_mfma_f32_16x16x4f32(m[v], U[v], o, 0, 0, 0);   // (the sum by itself, as the state's)
+            o += qs;
             const int t = tb + i * DPC + 4 * kg;
 #pragma unroll
             for (int v = 0; v < 4; ++v)
@@ -357,12 +383,16 @@ template <int ND, bool FULL> __global__ __launch_bounds__(320) void delta_piece_
             for (int j = 0; j < ND; ++j) po[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.qg[j][v], S[j][v], po[j], 0, 0, 0);
         const f32x4_t U = r.x - ((a0 + a1) + (a2 + a3));
 #pragma unroll
-        for (int j = 0; j < ND; ++j)
-            if (own[j]) S[j] *= r.gd[j];
+        for (int j = 0; j < ND; ++j) pw[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int j = 0; j < ND; ++j) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(own[j] ? r.kh[j][v] : 0.f, U[v], S[j], 0, 0, 0);
+            for (int j = 0; j < ND; ++j) pw[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.kh[j][v], U[v], pw[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < ND; ++j)
+            if (own[j])                                                  // (the sum by itself: one rounding of the state per piece)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) S[j][v] = fmaf(S[j][v], r.gd[j][v], pw[j][v]);
 #pragma unroll
         for (int j = 1; j < ND; ++j) po[0] += po[j];
         so[i & 1][wave][lane] = po[0];

@@ -339,6 +339,33 @@ def test_delta_rule_by_pieces(lib, Hh, G, d, vd, per_channel):
         assert np.abs(S[slot, :Hh * d * vd].reshape(Hh, d, vd) - w).max() < 2e-5 * max(1.0, np.abs(w).max())
 
 
+@pytest.mark.parametrize("Hh,d,vd,per_channel", [(4, 64, 64, True), (4, 128, 128, True), (2, 256, 256, True), (4, 128, 64, False)])
+def test_delta_rule_by_pieces_is_no_further_from_64_bits_than_the_walk(lib, Hh, d, vd, per_channel):
+    """one call over 320 tokens (pieces of 16) against the same tokens in calls of 32 (the walk): 2-norm of the error of outputs and state"""
+    _gpu()
+    rng = np.random.default_rng(Hh * 13 + d)
+    T, C, nd, stride = 320, 2 * Hh * d + Hh * vd, Hh * d if per_channel else Hh, Hh * d * vd
+    qkv, proj, pre = (rng.standard_normal((T, n)).astype(np.float32) for n in (C, Hh, nd))
+    a_log, dtb = (0.5 * rng.standard_normal(Hh)).astype(np.float32), (0.5 * rng.standard_normal(nd) - 3).astype(np.float32)
+    x = qkv.astype(np.float64)
+    q, k = (H.unit_heads(x[:, i * Hh * d:(i + 1) * Hh * d].reshape(T, Hh, d), 1e-6) for i in (0, 1))
+    g = H.decay(a_log.astype(np.float64)[None, :, None], pre.astype(np.float64).reshape(T, Hh, -1), dtb.astype(np.float64).reshape(1, Hh, -1)) * np.ones((1, 1, d))
+    want = H.gated_delta_rule(q * d ** -0.5, k, x[:, 2 * Hh * d:].reshape(T, Hh, vd), H.sigmoid(proj.astype(np.float64)), g)
+    err = []
+    for step in (T, 32):
+        state, outs = torch.zeros((1, stride), device="cuda"), []
+        for lo in range(0, T, step):
+            o = torch.empty((step, Hh, vd), device="cuda")
+            scratch = torch.zeros(lib.mi355_hyb_delta_rule_scratch_floats(step, Hh, Hh, d, int(per_channel)), device="cuda")
+            ok(lib.mi355_hyb_delta_rule(o.data_ptr(), state.data_ptr(), stride, P(qkv[lo:lo + step]), C, P(proj[lo:lo + step]), Hh, 0, P(pre[lo:lo + step]), nd,
+                                        int(per_channel), P(a_log), P(dtb), P([lo + step], np.int32), P([0, step], np.int32), P([0], np.int32), 1, step, Hh, Hh,
+                                        d, vd, 1e-6, scratch.data_ptr(), _st()))
+            outs.append(o.cpu().numpy())
+        got = (np.concatenate(outs), state.cpu().numpy().reshape(Hh, d, vd))
+        err.append([np.linalg.norm(a - b) / np.linalg.norm(b) for a, b in zip(got, want)])
+    assert err[0][0] <= err[1][0] and err[0][1] <= err[1][1], err
+
+
 def test_gated_norm_and_mingru(lib):
     _gpu()
     rng = np.random.default_rng(9)
