@@ -323,6 +323,20 @@ template <int ND, bool FULL> __global__ __launch_bounds__(320) void delta_piece_
             asm volatile("" : "+v"(qs));                                 // in hand first: these products are not on the chain, and a wave that is shares their SIMD
 #pragma unroll
             for (int v = 0; v < 4; ++v) o = __builtin_amdgcn_mfma_f32_16x16x4f32(m[v], U[v], o, 0, 0, 0);   // (the sum by itself, as the state's)
+            if (__any(o[0] != o[0])) {
+                // The zeros of M are no zeros times an infinity or a NaN: tokens in front of such a U are summed without it, as the walk does.
+                // (a U behind the first token that is not finite leaves a NaN in the first row, whose M is zero there: one comparison sees them all)
+                o = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s2 = 0; s2 < DPC; ++s2) {
+                    const float us = __shfl(U[s2 & 3], 16 * (s2 >> 2) + m16);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float ms = __shfl(m[s2 & 3], 16 * (s2 >> 2) + 4 * kg + v);
+                        if (s2 <= 4 * kg + v) o[v] = fmaf(ms, us, o[v]);
+                    }
+                }
+            }
             o += qs;
             const int t = tb + i * DPC + 4 * kg;
 #pragma unroll
@@ -381,7 +395,11 @@ template <int ND, bool FULL> __global__ __launch_bounds__(320) void delta_piece_
         for (int v = 0; v < 4; ++v)
 #pragma unroll
             for (int j = 0; j < ND; ++j) po[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.qg[j][v], S[j][v], po[j], 0, 0, 0);
-        const f32x4_t U = r.x - ((a0 + a1) + (a2 + a3));
+        f32x4_t U = r.x - ((a0 + a1) + (a2 + a3));
+        if (i == n - 1) {                                                // rows beyond the portion: nothing times a state that is not finite
+#pragma unroll
+            for (int v = 0; v < 4; ++v) if (tb + i * DPC + 4 * kg + v >= te) U[v] = 0.f;
+        }
 #pragma unroll
         for (int j = 0; j < ND; ++j) pw[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -366,6 +366,41 @@ def test_delta_rule_by_pieces_is_no_further_from_64_bits_than_the_walk(lib, Hh, 
     assert err[0][0] <= err[1][0] and err[0][1] <= err[1][1], err
 
 
+@pytest.mark.parametrize("what,at", [("v", 37), ("k", 37), ("pre", 41), ("proj", 32), ("v", 99), ("state", 0)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_delta_rule_by_pieces_not_finite(lib, what, at, value):
+    """an infinity or NaN of one token, in the middle of a piece, at its start or in the last token of a portion that ends inside a piece (100 tokens),
+    or in the state before: what the walk (the same tokens in calls of 20) keeps finite the pieces keep finite, infinities of the state stay infinities"""
+    _gpu()
+    rng = np.random.default_rng(at)
+    T, Hh, d, vd = 100, 2, 32, 48
+    C, nd, stride = 2 * Hh * d + Hh * vd, Hh * d, Hh * d * vd
+    qkv, proj, pre = (rng.standard_normal((T, n)).astype(np.float32) for n in (C, Hh, nd))
+    a_log, dtb, S0 = rng.standard_normal(Hh).astype(np.float32), rng.standard_normal(nd).astype(np.float32), rng.standard_normal((1, stride)).astype(np.float32)
+    if what == "state":
+        S0[0, 5 * vd + 7] = value
+    else:
+        {"v": qkv[:, 2 * Hh * d + 5:], "k": qkv[:, Hh * d + 3:], "pre": pre[:, 9:], "proj": proj}[what][at, 0] = value
+    res = []
+    for step in (T, 20):
+        state, outs = dev(S0), []
+        for lo in range(0, T, step):
+            o = torch.empty((step, Hh, vd), device="cuda")
+            scratch = torch.zeros(lib.mi355_hyb_delta_rule_scratch_floats(step, Hh, Hh, d, 1), device="cuda")
+            ok(lib.mi355_hyb_delta_rule(o.data_ptr(), state.data_ptr(), stride, P(qkv[lo:lo + step]), C, P(proj[lo:lo + step]), Hh, 0, P(pre[lo:lo + step]), nd, 1,
+                                        P(a_log), P(dtb), P([lo + step + 1], np.int32), P([0, step], np.int32), P([0], np.int32), 1, step, Hh, Hh, d, vd, 1e-6,
+                                        scratch.data_ptr(), _st()))
+            outs.append(o.cpu().numpy())
+        res.append((np.concatenate(outs), state.cpu().numpy()))
+    for got, want in zip(*res):
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isfinite(got), fin)
+        assert np.abs(got[fin] - want[fin]).max(initial=0) < 2e-5 * max(1.0, np.abs(want[fin]).max(initial=0))
+    if at == T - 1:
+        got, want = res[0][1], res[1][1]
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+
+
 def test_gated_norm_and_mingru(lib):
     _gpu()
     rng = np.random.default_rng(9)
