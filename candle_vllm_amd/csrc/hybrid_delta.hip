@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <math.h>
+#include <algorithm>
 
 #include "common.h"
 #include "hybrid_device.h"
@@ -163,7 +164,7 @@ template <int DP, int LPC, int CH> __global__ __launch_bounds__(256) void delta_
 // A record per (piece, head), in the order the scan's lanes read it, 16 B each: W, Q_G [d / 16][lane = 16 (c % 16 / 4) + t][c % 4],
 // K_hat [d / 16][lane = 16 (t / 4) + c % 16][t % 4], G_16 [d], M [lane = 16 (s / 4) + t][s % 4], X [vd / 16][lane = 16 (t / 4) + c % 16][t % 4].
 constexpr int DPC = 16;
-struct DeltaPieces { float* rec; int n_seqs; int64_t rec_floats; };
+struct DeltaPieces { float* rec; int n_seqs; int64_t rec_floats; int first, count; };   // this launch's window of piece numbers; rec holds theirs
 __host__ __device__ __forceinline__ int64_t delta_rec_floats(int d, int vd) { return 3 * DPC * (int64_t)d + d + DPC * DPC + DPC * (int64_t)vd; }
 // pieces of sequence s start at number cu_q[s] / 16 + s: room for every sequence's last, shorter piece without a table
 __device__ __forceinline__ int delta_first_piece(const uint32_t* cu_q, int s) { return (int)(cu_q[s] / DPC) + s; }
@@ -187,7 +188,7 @@ template <int DP> __global__ __launch_bounds__(256, 3) void delta_piece_prepare_
     constexpr bool LOW = DP <= 8;
     __shared__ __align__(16) _Float16 sl[LOW ? DPC : 1][RS];
     __shared__ float sA[DPC][DPC], sb[DPC], sM[DPC][DPC];
-    const int piece = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, row = tid >> 4, part = tid & 15;
+    const int piece = q.first + (int)blockIdx.x, h = blockIdx.y, tid = threadIdx.x, row = tid >> 4, part = tid & 15;
     const int d = p.d, vd = p.vd, g = h / (p.H / p.G);
     int s = 0;
     while (s + 1 < q.n_seqs && delta_first_piece(p.cu_q, s + 1) <= piece) ++s;
@@ -228,7 +229,7 @@ template <int DP> __global__ __launch_bounds__(256, 3) void delta_piece_prepare_
         if (part == 0) sb[row] = live ? sigmoidf_(p.proj[(size_t)t * p.ldp + p.b_off + h]) : 0.f;
     }
     __syncthreads();
-    float* rec = q.rec + ((size_t)piece * p.H + h) * q.rec_floats;
+    float* rec = q.rec + ((size_t)blockIdx.x * p.H + h) * q.rec_floats;
     // ---- A, M, K_hat: row s's key walks on through the decays (16 lanes per row, DP channels each)
     {
         float x[DP];
@@ -300,10 +301,12 @@ template <int ND, bool FULL> __global__ __launch_bounds__(320) void delta_piece_
     const int s = blockIdx.x / p.H, h = blockIdx.x % p.H, ct = blockIdx.y, lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), m16 = lane & 15, kg = lane >> 4;
     const int d = p.d, vd = p.vd, nd = d >> 4;
-    const int tb = (int)p.cu_q[s], te = (int)p.cu_q[s + 1];
+    // this sequence's tokens in the window: from piece `skip` of it (its state is in the slot by then), n pieces
+    const int cu0 = (int)p.cu_q[s], cu1 = (int)p.cu_q[s + 1], first = delta_first_piece(p.cu_q, s) - q.first, skip = max(-first, 0);
+    const int tb = cu0 + skip * DPC, te = min(cu1, cu0 + (q.count - first) * DPC);
     if (te <= tb) return;
-    const int n = (te - tb + DPC - 1) / DPC, start_pos = (int)p.ctx[s] - (te - tb);
-    const float* rec0 = q.rec + ((size_t)delta_first_piece(p.cu_q, s) * p.H + h) * q.rec_floats;
+    const int n = (te - tb + DPC - 1) / DPC, start_pos = (int)p.ctx[s] - (cu1 - cu0) + skip;
+    const float* rec0 = q.rec + ((size_t)(first + skip) * p.H + h) * q.rec_floats;
     const size_t rstep = (size_t)p.H * q.rec_floats, m_at = 3 * DPC * (size_t)d + d + lane * 4, x_at = 3 * DPC * (size_t)d + d + DPC * DPC + (size_t)ct * 256 + lane * 4;
     auto ld4 = [](const float* a) { return *reinterpret_cast<const f32x4_t*>(a); };
     auto meet = [] {                                                     // own LDS accesses done; everyone's
@@ -436,6 +439,7 @@ template <int ND, bool FULL> __global__ __launch_bounds__(320) void delta_piece_
 }
 
 constexpr int DELTA_MIN_TOKENS = 64, DELTA_MIN_PER_SEQ = 48;
+constexpr int64_t DELTA_WINDOW_BYTES = 256ll << 20;
 
 }  // namespace
 
@@ -459,18 +463,21 @@ int mi355_hyb_delta_rule(float* o, float* state, int64_t state_stride, const flo
     // Whole 16-row tiles and portions of prompts: by pieces.  us per call, walk / pieces, 16 heads of 128 x 128: one sequence of 32 tokens 20 / 25,
     // 64 31 / 27, 200 82 / 38, 2048 740 / 200; two sequences of 1050 402 / 150; 8 sequences of 16 21 / 32 (64 each: 35 / 38); 32 heads of 64 x 64,
     // 64 tokens 25 / 20, 2048 590 / 170; 8 heads of 256 x 256, 64 tokens 44 / 48, 200 112 / 64, 2048 1019 / 310
-    if (dim % 16 == 0 && vdim % 16 == 0 && num_tokens >= DELTA_MIN_TOKENS && num_tokens / num_seqs >= DELTA_MIN_PER_SEQ && vdim <= 65535 * 16) {
-        const int64_t pieces = num_tokens / DPC + num_seqs, rec = delta_rec_floats(dim, vdim);
+    // Their records take 8.6 KB per token and 16 heads of 128: windows of at most 256 MiB (7 800 such tokens), one behind the other, with the state in
+    // its slot in between
+    const int64_t pieces = num_tokens / DPC + num_seqs, piece_bytes = heads * delta_rec_floats(dim, vdim) * 4, window = std::min(pieces, DELTA_WINDOW_BYTES / piece_bytes);
+    if (dim % 16 == 0 && vdim % 16 == 0 && num_tokens >= DELTA_MIN_TOKENS && num_tokens / num_seqs >= DELTA_MIN_PER_SEQ && vdim <= 65535 * 16 && window > 0) {
         void* ws = nullptr;
-        if (pieces * heads * rec * 4 <= (int64_t)4 << 30 && heads <= 65535 &&
-            mi355_scratch_get(&ws, MI355_SCR_DELTA, (size_t)(pieces * heads * rec) * 4, s_, false) == 0) {   // (no room while a stream is captured: the walk)
-            const DeltaPieces q{static_cast<float*>(ws), num_seqs, rec};
-            const dim3 pg((unsigned)pieces, heads), sg(num_seqs * heads, vdim / 16);
+        if (heads <= 65535 && mi355_scratch_get(&ws, MI355_SCR_DELTA, (size_t)(window * piece_bytes), s_, false, (size_t)DELTA_WINDOW_BYTES) == 0) {   // (no room while a stream is captured: the walk)
+            for (int64_t first = 0; first < pieces; first += window) {
+                const DeltaPieces q{static_cast<float*>(ws), num_seqs, delta_rec_floats(dim, vdim), (int)first, (int)std::min(window, pieces - first)};
+                const dim3 pg((unsigned)q.count, heads), sg(num_seqs * heads, vdim / 16);
 #define DELTA_SCAN(ND) do { if (dim == 64 * (ND)) delta_piece_scan_kernel<ND, true><<<sg, 320, 0, s_>>>(p, q); else delta_piece_scan_kernel<ND, false><<<sg, 320, 0, s_>>>(p, q); } while (0)
-            if (dim <= 64) { delta_piece_prepare_kernel<4><<<pg, 256, 0, s_>>>(p, q); DELTA_SCAN(1); }
-            else if (dim <= 128) { delta_piece_prepare_kernel<8><<<pg, 256, 0, s_>>>(p, q); DELTA_SCAN(2); }
-            else { delta_piece_prepare_kernel<16><<<pg, 256, 0, s_>>>(p, q); DELTA_SCAN(4); }
+                if (dim <= 64) { delta_piece_prepare_kernel<4><<<pg, 256, 0, s_>>>(p, q); DELTA_SCAN(1); }
+                else if (dim <= 128) { delta_piece_prepare_kernel<8><<<pg, 256, 0, s_>>>(p, q); DELTA_SCAN(2); }
+                else { delta_piece_prepare_kernel<16><<<pg, 256, 0, s_>>>(p, q); DELTA_SCAN(4); }
 #undef DELTA_SCAN
+            }
             LAUNCH_OK(); return 0;
         }
     }

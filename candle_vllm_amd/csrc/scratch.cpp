@@ -3,16 +3,18 @@
 // Why: the kernels' internal scratch (arrival tickets of the fused attention merge, arg-max slots, the activation image
 // and split-K partials of the wide mat-mul path, the dense path's staging buffer) used to be process-wide statics --
 // two streams raced on the same tickets, a second device faulted on a buffer allocated on the first, and growing a
-// buffer freed memory a captured hipGraph still pointed to (ADVICE r1).  Rules here:
+// buffer freed memory a captured hipGraph still pointed to.  Rules here:
 //   * a buffer belongs to the stream that asked for it (the reference runs one model per process and stream; two models
 //     on two streams now get two buffers);
 //   * growing never frees: the old allocation is retired (kept until mi355_scratch_release_all), because a graph captured
-//     earlier may replay launches that hold its address.  Sizes double, so the retired total stays below the live size;
+//     earlier may replay launches that hold its address.  Sizes double (up to the most a caller names), so the retired total stays
+//     below the live size (below twice the named limit);
 //   * nothing is allocated while the stream is capturing (hipMalloc would break the capture): the caller gets
 //     hipErrorStreamCaptureUnsupported and the host layer's eager warm-up step does the growth.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -28,7 +30,7 @@ std::map<std::tuple<int, hipStream_t, int>, Buf> g_live;
 std::vector<std::pair<int, void*>> g_retired;          // (device, pointer)
 }  // namespace
 
-int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool zero_on_create) {
+int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool zero_on_create, size_t most) {
     if (!out) return (int)hipErrorInvalidValue;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -39,7 +41,7 @@ int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool ze
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
         return (int)hipErrorStreamCaptureUnsupported;
-    const size_t want = b.p ? bytes * 2 : bytes;
+    const size_t want = b.p ? std::max(bytes, std::min(bytes * 2, most)) : bytes;
     void* p = nullptr;
     e = hipMalloc(&p, want);
     if (e != hipSuccess) return (int)e;

@@ -21,7 +21,8 @@ enum {
 
 // *out = a device buffer of >= bytes owned by (current device, st, key).  zero_on_create: the buffer is cleared (on `st`)
 // when it is first created or grown.  Returns hipErrorStreamCaptureUnsupported when growth would be needed mid-capture.
-int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool zero_on_create);
+// `most`: what a caller asks for at most; a buffer that grows is doubled, but not beyond this.
+int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool zero_on_create, size_t most = (size_t)-1);
 extern "C" void mi355_scratch_release_all(void);
 
 // void FFI entry points record their first failure here (mi355_last_error / mi355_clear_error in the header)

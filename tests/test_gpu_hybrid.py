@@ -366,6 +366,38 @@ def test_delta_rule_by_pieces_is_no_further_from_64_bits_than_the_walk(lib, Hh, 
     assert err[0][0] <= err[1][0] and err[0][1] <= err[1][1], err
 
 
+def test_delta_rule_by_pieces_in_windows(lib):
+    """more pieces than the workspace holds records of (256 MiB: 61 of 64 heads of 256 x 256): windows that begin inside a sequence and at the start of
+    one, against the walk of the same tokens -- the same bound as the walk against 64 bits"""
+    _gpu()
+    Hh, d, lens = 64, 256, [700, 400, 1, 260]
+    T, n, stride = sum(lens), len(lens), Hh * d * d
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    qkv, proj, pre = (torch.randn(T, c, device="cuda", generator=gen) for c in (3 * Hh * d, Hh, Hh * d))
+    a_log, dtb, S0 = 0.5 * torch.randn(Hh, device="cuda", generator=gen), torch.randn(Hh * d, device="cuda", generator=gen) - 2, torch.randn(n, stride, device="cuda", generator=gen)
+    cu = np.cumsum([0] + lens)
+
+    def call(o, state, lo, hi, ctx, starts, slots):
+        scratch = torch.empty(lib.mi355_hyb_delta_rule_scratch_floats(hi - lo, Hh, Hh, d, 1), device="cuda")
+        ok(lib.mi355_hyb_delta_rule(o[lo:].data_ptr(), state.data_ptr(), stride, qkv[lo:].data_ptr(), 3 * Hh * d, proj[lo:].data_ptr(), Hh, 0, pre[lo:].data_ptr(), Hh * d, 1,
+                                    a_log.data_ptr(), dtb.data_ptr(), P(ctx, np.int32), P(starts, np.int32), P(slots, np.int32), len(slots), hi - lo, Hh, Hh, d, d, 1e-6,
+                                    scratch.data_ptr(), _st()))
+    got, want, S, Sw = torch.full((T, Hh * d), float("nan"), device="cuda"), torch.empty(T, Hh * d, device="cuda"), S0.clone(), S0.clone()
+    def taken():                                                            # of the card's memory, beside what torch keeps
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free - torch.cuda.memory_reserved()
+    before = taken()
+    call(got, S, 0, T, [lens[0] + 9, lens[1], lens[2], lens[3] + 1], cu, range(n))               # the second and third begin from nothing
+    assert taken() - before <= (256 + 8) << 20
+    for i in range(n):
+        for lo in range(cu[i], cu[i + 1], 63):
+            hi = min(lo + 63, cu[i + 1])
+            call(want, Sw, lo, hi, [hi - cu[i] + (9, 0, 0, 1)[i]], [0, hi - lo], [i])
+    assert float((got - want).abs().max()) < 2e-5 * max(1.0, float(want.abs().max()))
+    assert float((S - Sw).abs().max()) < 2e-5 * max(1.0, float(Sw.abs().max()))
+
+
 @pytest.mark.parametrize("what,at", [("v", 37), ("k", 37), ("pre", 41), ("proj", 32), ("v", 99), ("state", 0)])
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 def test_delta_rule_by_pieces_not_finite(lib, what, at, value):
