@@ -28,6 +28,7 @@ struct Buf { void* p = nullptr; size_t bytes = 0; };
 std::mutex g_mu;
 std::map<std::tuple<int, hipStream_t, int>, Buf> g_live;
 std::vector<std::pair<int, void*>> g_retired;          // (device, pointer)
+std::atomic<size_t> g_limit{(size_t)-1};               // largest allocation (mi355_internal_scratch_limit)
 }  // namespace
 
 int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool zero_on_create, size_t most) {
@@ -41,9 +42,15 @@ int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool ze
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
         return (int)hipErrorStreamCaptureUnsupported;
-    const size_t want = b.p ? std::max(bytes, std::min(bytes * 2, most)) : bytes;
+    size_t want = b.p ? std::max(bytes, std::min(bytes * 2, most)) : bytes;
     void* p = nullptr;
-    e = hipMalloc(&p, want);
+    auto allocate = [&](size_t n) {
+        const hipError_t rc = hipMalloc(&p, n <= g_limit.load() ? n : (size_t)1 << 60);
+        if (rc != hipSuccess) (void)hipGetLastError();      // the caller has another way: its launches must not find this error behind them
+        return rc;
+    };
+    e = allocate(want);
+    if (e != hipSuccess && want > bytes) e = allocate(want = bytes);
     if (e != hipSuccess) return (int)e;
     if (zero_on_create) {
         e = hipMemsetAsync(p, 0, want, st);                 // ordered before the first launch on `st` that uses it
@@ -54,6 +61,9 @@ int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool ze
     *out = p;
     return 0;
 }
+
+// Tests: an allocation above `bytes` fails the way one does on a full card (-1: none).
+extern "C" void mi355_internal_scratch_limit(int64_t bytes) { g_limit.store(bytes < 0 ? (size_t)-1 : (size_t)bytes); }
 
 // Sticky error of the `void` entry points (the reference's FFI symbols return nothing, src/backend/gptq.rs:115-194,
 // cache.rs:127-162): the first failure since the last clear is kept until the host reads it.
