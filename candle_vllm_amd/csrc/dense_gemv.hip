@@ -969,30 +969,29 @@ static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
             }
             const int kps = (nkb_w + ks - 1) / ks;
             ks = (nkb_w + kps - 1) / kps;
-            float* part = nullptr;
             const int tpad = mt * 16, ldp = a.N;
-            if (ks > 1) {
-                void* pp = nullptr;
-                if (mi355_scratch_get(&pp, MI355_SCR_GPTQ_WIDE, (size_t)ks * tpad * ldp * sizeof(float), st, false)) return -1;
-                part = static_cast<float*>(pp);
-            }
-            const dim3 grid(gx, ks), block(64 * nwv);
-            const size_t lds = (size_t)2 * mt * 16 * DWD_LDX * 2;
+            void* pp = nullptr;
+            const bool room = ks == 1 || mi355_scratch_get(&pp, MI355_SCR_GPTQ_WIDE, (size_t)ks * tpad * ldp * sizeof(float), st, false) == 0;
+            float* part = static_cast<float*>(pp);
+            if (room) {                                                 // (else dense_kernel below)
+                const dim3 grid(gx, ks), block(64 * nwv);
+                const size_t lds = (size_t)2 * mt * 16 * DWD_LDX * 2;
 #define DWD_GO2(MT_, R_, NW_) do { \
-                static bool attr = false; \
-                if (!attr) { (void)hipFuncSetAttribute((const void*)dense_wide_kernel<DT, MT_, R_, NW_>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024); attr = true; } \
-                hipLaunchKernelGGL((dense_wide_kernel<DT, MT_, R_, NW_>), grid, block, lds, st, a, part, ldp, kps); } while (0)
+                    static bool attr = false; \
+                    if (!attr) { (void)hipFuncSetAttribute((const void*)dense_wide_kernel<DT, MT_, R_, NW_>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024); attr = true; } \
+                    hipLaunchKernelGGL((dense_wide_kernel<DT, MT_, R_, NW_>), grid, block, lds, st, a, part, ldp, kps); } while (0)
 #define DWD_GO(MT_, R_) do { if (nwv == 2) DWD_GO2(MT_, R_, 2); else DWD_GO2(MT_, R_, 4); } while (0)
-            if (pair) { if (mt == 1) DWD_GO(1, 2); else DWD_GO(2, 2); }
-            else switch (mt) { case 1: DWD_GO(1, 1); break; case 2: DWD_GO(2, 1); break; case 3: DWD_GO(3, 1); break; default: DWD_GO(4, 1); break; }
+                if (pair) { if (mt == 1) DWD_GO(1, 2); else DWD_GO(2, 2); }
+                else switch (mt) { case 1: DWD_GO(1, 1); break; case 2: DWD_GO(2, 1); break; case 3: DWD_GO(3, 1); break; default: DWD_GO(4, 1); break; }
 #undef DWD_GO2
 #undef DWD_GO
-            if (hipGetLastError() != hipSuccess) return -1;
-            if (ks > 1) {
-                hipLaunchKernelGGL((gptq_wide_epilogue_kernel<DT>), dim3((a.N + 255) / 256, a.T), dim3(256), 0, st, a, part, ldp, ks, tpad);
                 if (hipGetLastError() != hipSuccess) return -1;
+                if (ks > 1) {
+                    hipLaunchKernelGGL((gptq_wide_epilogue_kernel<DT>), dim3((a.N + 255) / 256, a.T), dim3(256), 0, st, a, part, ldp, ks, tpad);
+                    if (hipGetLastError() != hipSuccess) return -1;
+                }
+                return 0;
             }
-            return 0;
         }
     }
     int gj = 8;

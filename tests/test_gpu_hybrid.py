@@ -366,6 +366,34 @@ def test_delta_rule_by_pieces_is_no_further_from_64_bits_than_the_walk(lib, Hh, 
     assert err[0][0] <= err[1][0] and err[0][1] <= err[1][1], err
 
 
+def test_delta_rule_no_room_for_the_pieces(lib):
+    """where the pieces' records cannot be allocated (a new stream, on which every allocation fails as on a full card) the tokens are walked"""
+    _gpu()
+    import ctypes
+    lib.mi355_internal_scratch_limit.argtypes = [ctypes.c_int64]
+    T, Hh, d = 96, 2, 32
+    C, stride = 3 * Hh * d, Hh * d * d
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    qkv, proj, pre, a_log, dtb = (torch.randn(*s, device="cuda", generator=gen) for s in ((T, C), (T, Hh), (T, Hh * d), (Hh,), (Hh * d,)))
+    ctx, cu, slot = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([T], [0, T], [0]))
+    scratch = torch.zeros(lib.mi355_hyb_delta_rule_scratch_floats(T, Hh, Hh, d, 1), device="cuda")
+    torch.cuda.synchronize()
+    res = []
+    for limit in (0, -1):
+        o, state = torch.full((T, Hh * d), float("nan"), device="cuda"), torch.zeros(1, stride, device="cuda")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(torch.cuda.Stream()):
+            lib.mi355_internal_scratch_limit(limit)
+            try:
+                ok(lib.mi355_hyb_delta_rule(o.data_ptr(), state.data_ptr(), stride, qkv.data_ptr(), C, proj.data_ptr(), Hh, 0, pre.data_ptr(), Hh * d, 1, a_log.data_ptr(),
+                                            dtb.data_ptr(), ctx.data_ptr(), cu.data_ptr(), slot.data_ptr(), 1, T, Hh, Hh, d, d, 1e-6, scratch.data_ptr(), _st()))
+            finally:
+                lib.mi355_internal_scratch_limit(-1)
+        res.append((o, state))
+    for a, b in zip(*res):
+        assert float((a - b).abs().max()) < 2e-5 * max(1.0, float(b.abs().max()))
+
+
 def test_delta_rule_by_pieces_in_windows(lib):
     """more pieces than the workspace holds records of (256 MiB: 61 of 64 heads of 256 x 256): windows that begin inside a sequence and at the start of
     one, against the walk of the same tokens -- the same bound as the walk against 64 bits"""

@@ -542,3 +542,31 @@ def test_wide_16bit_kernel_few_tiles_long_k_split(cv, dt, T, N, K, tiled):
     check_ulp(y, G.round_dt(full + res, dt), dt, what="split-K wide kernel + bias + residual", ulps=3.01, mag=np.maximum(np.abs(full), np.abs(G.linear16(x, w, None, dt))))
     y2 = host16(cv.Linear(dev16(w, dt), tiled=tiled).forward(dev16(x, dt)), dt)
     check_ulp(y2, G.linear16(x, w, None, dt), dt, what="split-K wide kernel")
+
+
+@pytest.mark.parametrize("kind,T,N,K", [("16-bit", 96, 96, 8192), ("16-bit", 9, 256, 8192), ("4-bit", 100, 64, 8192), ("4-bit", 33, 64, 8192)])
+def test_no_room_for_a_workspace(cv, kind, T, N, K):
+    """launches that split K or prepare their operands, where the workspace cannot be allocated (a new stream, on which every allocation fails as on a full
+    card): another way to the same result at the same bound, and no error behind it"""
+    import ctypes
+    from candle_vllm_amd._lib import lib
+    lib.mi355_internal_scratch_limit.argtypes = [ctypes.c_int64]
+    rng = np.random.default_rng(T + N + K)
+    x = G.round_dt(rng.normal(0, 1, (T, K)), "bf16")
+    if kind == "4-bit":
+        q, s = _gptq_case(rng, K, N, 128, "bf16")
+        lin, ref = cv.GPTQLinear(dev_u32(G.gptq_pack(q)), dev16(s, "bf16"), 128), G.gptq_linear(x, G.gptq_dequant(q, s, None, 128), None, "bf16")
+    else:
+        w = G.round_dt(rng.normal(0, 0.02, (N, K)), "bf16")
+        lin, ref = cv.Linear(dev16(w, "bf16"), tiled=True), G.linear16(x, w, None, "bf16")
+    xd = dev16(x, "bf16")
+    torch.cuda.synchronize()
+    for limit in (0, -1):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            lib.mi355_internal_scratch_limit(limit)
+            try:
+                y = lin.forward(xd)
+            finally:
+                lib.mi355_internal_scratch_limit(-1)
+            torch.cuda.current_stream().synchronize()
+            check_ulp(host16(y, "bf16"), ref, "bf16", what=f"{kind}, limit {limit}")
