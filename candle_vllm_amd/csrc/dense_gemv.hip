@@ -810,7 +810,7 @@ static int dense_launch_gj(const DenseArgs& a, int gj, int nw, hipStream_t st) {
 // T = 16 9.3 / 13.7, 32 12.3 / 14.0, 40 16.1 / 13.7; 12288 x 2048 T = 32 17.0 / 12.9; at 5 .. 16 tokens either may win (16384 pairs of 3072: 18.7 / 22.1)
 // 4-bit, against token chunks of the decode kernels: down 3584 x 18944 T = 32 21.6 / 27.4, 33 29.1 / 28.1, 49 72.7 / 29.1; 4608 x 3584 T = 33 20.8 / 16.0;
 // wo 3584 x 3584 33 14.8 / 15.0, 64 19.2 / 16.5; gate/up 37888 x 3584 48 42.1 / 54.5, 64 48.3 / 58.3, 65 64.3 / 58.8
-enum { DENSE_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_PAIR_T = 65 };
+enum { DENSE_GEMM_MIN_T = 33, DENSE_GEMM_ANY_T = 96, GPTQ_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_PAIR_T = 65 };
 static int g_tune_gemm_min_t = DENSE_GEMM_MIN_T;
 static int g_tune_gptq_gemm_off = 0;   // tuning key 39: 1 = 4-bit prompt steps run the decode kernel in 64-token chunks (A/B)
 static int g_tune_wide_nw = 4;         // tuning key 38: waves (row tiles) per workgroup of dense_wide_kernel: 2 | 4
@@ -1290,7 +1290,7 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     const int gs = a.group_size;
     const bool silu = a.epi == MI355_EPI_SILU_MUL;
     if (dt != MI355_DTYPE_BF16 && dt != MI355_DTYPE_F16) return (int)hipErrorNotSupported;
-    if (g_tune_gptq_gemm_off || (a.K & 255) || a.T < 4 || gs < 64 || (gs % 64) || (a.K % gs) || (gs > 128 && gs % 128)) return (int)hipErrorNotSupported;
+    if (g_tune_gptq_gemm_off || (a.K & 255) || a.T < 4 || gs < 64 || (gs % 64) || (a.K % gs) || (gs > 128 && gs % 256)) return (int)hipErrorNotSupported;   // (the groups of the token chunks, but 32)
     if ((a.ldx * 2) % 16 || ((uintptr_t)a.x & 15) || (int64_t)a.K * 512 >= (1ll << 32)) return (int)hipErrorNotSupported;
     int64_t rows = 0, words = 0;
     for (int i = 0; i < n; ++i) {
@@ -1414,7 +1414,10 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
 
 // SILU_MUL with more than 32 tokens, or any T > 64: run in token chunks
 static int dense_run(DenseArgs a, int wtype, int dt, hipStream_t st) {
-    if (wtype == DW_DENSE && (a.T >= g_tune_gemm_min_t || (g_tune_gemm_min_t == DENSE_GEMM_MIN_T && a.T > 16 && (a.epi == MI355_EPI_SILU_MUL ? a.pair_offset : a.N) >= 16 * 768))) {
+    // (rows and k that are not whole tiles of the streaming kernels are served from DENSE_GEMM_ANY_T tokens, and refused below)
+    const bool whole = !(a.N & 15) && !(a.K & 255);
+    if (wtype == DW_DENSE && (a.T >= DENSE_GEMM_ANY_T || whole) &&
+        (a.T >= g_tune_gemm_min_t || (g_tune_gemm_min_t == DENSE_GEMM_MIN_T && a.T > 16 && (a.epi == MI355_EPI_SILU_MUL ? a.pair_offset : a.N) >= 16 * 768))) {
         const int rc = dense_prompt_gemm(&a, 1, dt, st);
         if (rc != (int)hipErrorNotSupported) return rc;                    // odd strides / K: keep streaming in token chunks
     }

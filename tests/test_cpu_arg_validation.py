@@ -127,6 +127,21 @@ def test_malformed_quantised_matmul_descriptors_are_refused(L):
     assert lib.mi355_qweight_repack(p, p, 8, 16, 256) != 0
 
 
+@pytest.mark.parametrize("T", [5, 32, 33, 40, 95])
+def test_linear_shapes_of_no_kernel_are_refused(L, T):
+    """rows and k that are not whole tiles (16 rows, 256 k) below 96 tokens, and 4-bit groups that are neither 32, 64, 128 nor a multiple of 256 at any
+    number of tokens: -2, before any launch"""
+    lib = L.lib
+    one = ctypes.c_uint64(0)
+    p = (ctypes.addressof(one) + 15) & ~15
+    for n, k in ((64, 64), (64, 576), (72, 512), (12296, 512), (130, 1024)):
+        for epi in (0, 2):
+            assert lib.mi355_linear(p, p, p, None, None, T, n, k, BF16, epi, 0) == -2
+    for t in (T, T + 100):
+        for k, gs in ((768, 384), (1280, 640), (768, 192), (512, 16)):
+            assert lib.mi355_gptq_linear_tiled(p, p, p, p, None, 0, 0, None, None, t, 64, k, gs, BF16, 0, 0) == -2
+
+
 def test_constructors_refuse_bad_configurations(L):
     lib = L.lib
     assert not lib.mi355_llama_create(None)
