@@ -1412,14 +1412,29 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     return (int)hipGetLastError();
 }
 
+// x or w of a prompt that do not start on 16 bytes: the GEMM over copies that do (a pass over each, against a sweep of the weights per 64 tokens)
+static int dense_prompt_gemm_staged(const DenseArgs& a, int dt, hipStream_t st) {
+    DenseArgs c = a;
+    const size_t x_b = ((size_t)(a.T - 1) * a.ldx + a.K) * 2, w_b = ((size_t)(a.N - 1) * a.ldw + a.K) * 2, x_room = (x_b + 255) & ~(size_t)255;
+    const bool x_off = (uintptr_t)a.x & 15, w_off = (uintptr_t)a.w & 15;
+    void* ws = nullptr;
+    if ((!x_off && !w_off) || a.K % 64 || mi355_scratch_get(&ws, MI355_SCR_DENSE_WS, x_room + (w_off ? w_b : 0), st, false)) return (int)hipErrorNotSupported;
+    uint8_t* base = static_cast<uint8_t*>(ws);
+    hipError_t e = hipSuccess;
+    if (x_off) { e = hipMemcpyAsync(base, a.x, x_b, hipMemcpyDeviceToDevice, st); c.x = base; }
+    if (w_off && e == hipSuccess) { e = hipMemcpyAsync(base + x_room, a.w, w_b, hipMemcpyDeviceToDevice, st); c.w = base + x_room; }
+    return e != hipSuccess ? (int)e : dense_prompt_gemm(&c, 1, dt, st);
+}
+
 // SILU_MUL with more than 32 tokens, or any T > 64: run in token chunks
 static int dense_run(DenseArgs a, int wtype, int dt, hipStream_t st) {
     // (rows and k that are not whole tiles of the streaming kernels are served from DENSE_GEMM_ANY_T tokens, and refused below)
     const bool whole = !(a.N & 15) && !(a.K & 255);
     if (wtype == DW_DENSE && (a.T >= DENSE_GEMM_ANY_T || whole) &&
         (a.T >= g_tune_gemm_min_t || (g_tune_gemm_min_t == DENSE_GEMM_MIN_T && a.T > 16 && (a.epi == MI355_EPI_SILU_MUL ? a.pair_offset : a.N) >= 16 * 768))) {
-        const int rc = dense_prompt_gemm(&a, 1, dt, st);
-        if (rc != (int)hipErrorNotSupported) return rc;                    // odd strides / K: keep streaming in token chunks
+        int rc = dense_prompt_gemm(&a, 1, dt, st);
+        if (rc == (int)hipErrorNotSupported && a.T >= DENSE_GEMM_ANY_T) rc = dense_prompt_gemm_staged(a, dt, st);
+        if (rc != (int)hipErrorNotSupported) return rc;                    // odd K, few tokens off the 16-byte grid: keep streaming in token chunks
     }
     if (wtype == DW_GPTQ4T && a.T >= (a.epi == MI355_EPI_SILU_MUL ? GPTQ_GEMM_MIN_PAIR_T : GPTQ_GEMM_MIN_T)) {
         const int rc = gptq_prompt_gemm(&a, 1, dt, st);

@@ -11,7 +11,7 @@ enum {
     MI355_SCR_QMM_PART = 5,      // wide mat-mul path: split-K partial sums
     MI355_SCR_QMM_TICKET = 6,    // wide mat-mul path: split-K arrival tickets (zero-initialised, self-cleaning)
     MI355_SCR_QMP_WS = 7,        // prompt-step GEMM: quantised activation image
-    MI355_SCR_DENSE_WS = 8,      // dense / GPTQ path staging
+    MI355_SCR_DENSE_WS = 8,      // 16-bit prompt GEMM: copies of operands that do not start on 16 bytes
     MI355_SCR_COMM = 9,          // one-shot all-reduce staging
     MI355_SCR_GPTQ_WIDE = 10,    // 5..64-token launches of tiled 4-bit weights: split-K partial sums (gptq_wide.inc)
     MI355_SCR_PF_FP8 = 11,       // prompt attention over an e4m3 cache: the sequences' blocks as bf16 + their block table (prefill_attention.hip)

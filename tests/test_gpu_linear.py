@@ -123,6 +123,21 @@ def test_linear_prompt_operands_off_the_16_byte_grid(cv, T, off_x, off_w):
     check_ulp(host16(out, dt), G.linear16(x, w, None, dt), dt, what="unaligned operands")
 
 
+@pytest.mark.parametrize("T,N,K", [(96, 72, 576), (150, 130, 64), (100, 96, 512)])
+@pytest.mark.parametrize("off_x,off_w", [(4, 0), (0, 1), (3, 4)])
+def test_linear_prompt_operands_off_the_grid_of_any_shape(cv, T, N, K, off_x, off_w):
+    """from 96 tokens any rows and any k that is a multiple of 64 are served, also from operands that do not start on 16 bytes"""
+    from candle_vllm_amd._lib import lib
+    dt, st = "bf16", torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(T + 8 * off_x + off_w)
+    x, w, res = G.round_dt(rng.normal(0, 1, (T, K)), dt), G.round_dt(rng.normal(0, 0.05, (N, K)), dt), G.round_dt(rng.normal(0, 1, (T, N)), dt)
+    xd, wd = (torch.zeros(v.size + 8, dtype=torch.bfloat16, device="cuda") for v in (x, w))
+    xd[off_x:off_x + x.size], wd[off_w:off_w + w.size] = dev16(x, dt).flatten(), dev16(w, dt).flatten()
+    out, rd, y = torch.empty((T, N), dtype=torch.bfloat16, device="cuda"), dev16(res, dt), G.linear16(x, w, None, dt)
+    assert lib.mi355_linear(out.data_ptr(), xd[off_x:].data_ptr(), wd[off_w:].data_ptr(), None, rd.data_ptr(), T, N, K, 2, 1, st) == 0
+    check_ulp(host16(out, dt), G.round_dt(y + res, dt), dt, ulps=2.01, what="unaligned operands", mag=y)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("T,N,K", [(256, 384, 1024), (300, 200, 576), (97, 130, 64), (700, 128, 256)])
 def test_linear_prompt_gemm_tall_tile(cv, dt, T, N, K):
