@@ -139,7 +139,7 @@ extern "C" int mi355_reshape_and_cache(const void* k, const void* v, void* key_c
     } else if (layout == MI355_KV_PAGED) {
         if (head_dim % (16 / elem_size)) return (int)hipErrorInvalidValue;
         // (from 64 tokens: 3.8 us both ways there, 4.2 / 3.7 at 128.  Fewer are decode batches: no neighbouring slots to gather.  16-byte loads and K stores)
-        if (elem_size == 2 && num_tokens >= 4 * RC_TOKENS && num_kv_heads > 0 && (((uintptr_t)k | (uintptr_t)v | (uintptr_t)key_cache) & 15) == 0) {
+        if (elem_size == 2 && num_tokens >= 4 * RC_TOKENS && row > 0 && (((uintptr_t)k | (uintptr_t)v | (uintptr_t)key_cache) & 15) == 0) {
             hipLaunchKernelGGL(reshape_and_cache_paged16_kernel, dim3((num_tokens + RC_TOKENS - 1) / RC_TOKENS, (row / 8 + 15) / 16), dim3(256), 0, st, (const uint16_t*)k,
                                (const uint16_t*)v, (uint16_t*)key_cache, (uint16_t*)value_cache, slot_mapping, num_tokens, num_kv_heads, head_dim, block_size);
             return (int)hipGetLastError();

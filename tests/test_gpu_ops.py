@@ -106,6 +106,13 @@ def test_reshape_and_cache_prompt_rows_bit_exact(cv, lib, T, Hkv, D, bs, shift):
     assert np.array_equal(bf16_bits(kcd), kc) and np.array_equal(bf16_bits(vcd), vc)
 
 
+def test_reshape_and_cache_rows_of_no_values(cv, lib):
+    """nothing to write is no error, at few tokens and at many"""
+    slots = dev(np.arange(64, dtype=np.int64))
+    for T in (3, 64):
+        assert lib.mi355_reshape_and_cache(None, None, None, None, slots.data_ptr(), T, 2, 0, 16, 2, cv.KV_PAGED, torch.cuda.current_stream().cuda_stream) == 0
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_copy_blocks_bit_exact(cv, dtype):
     rng = np.random.default_rng(2)
