@@ -1284,7 +1284,23 @@ static int gptq_gemm_dt(const GptqGemm& g, uint16_t* xp, float* xs, int which, h
     else { if (sym) gptq_gemm_epi<DT, true, 128>(g, which, st); else gptq_gemm_epi<DT, false, 128>(g, which, st); }
     return (int)hipGetLastError();
 }
-// n matrices over the same x, of one group size and zero mode
+// The workspaces of the prompt GEMMs are kept, so they are bounded: partial sums of at most 128 MiB, and of a 4-bit prompt at most 128 MiB of permuted
+// x and its sums at a time (3 328 tokens of 18 944, 19 712 of 3 584; a launch of that many is at its rate, and the panel in front of each costs 1 % of it)
+constexpr int64_t GEMM_PART_BYTES = 128ll << 20, GPTQ_GEMM_X_BYTES = 128ll << 20;
+static int gemm_max_split(const DenseArgs& a, int most) {
+    return (int)std::min<int64_t>(std::min(16, most), std::max<int64_t>(1, GEMM_PART_BYTES / ((int64_t)a.T * a.N * 4)));
+}
+static int gptq_gemm_slab(int k) { return (int)std::max<int64_t>(1, GPTQ_GEMM_X_BYTES / ((int64_t)k * 2 + k / 16) / 256) * 256; }
+// rows t0 .. of a launch of T tokens, at most n of them
+static DenseArgs dense_rows(const DenseArgs& a, int t0, int n) {
+    DenseArgs c = a;
+    c.T = a.T - t0 < n ? a.T - t0 : n;
+    c.x = static_cast<const uint16_t*>(a.x) + (size_t)t0 * a.ldx;
+    c.out = static_cast<uint16_t*>(a.out) + (size_t)t0 * a.ldo;
+    if (a.resid) c.resid = static_cast<const uint16_t*>(a.resid) + (size_t)t0 * a.ldo;
+    return c;
+}
+// n matrices over the same x, of one group size and zero mode; at most gptq_gemm_slab(K) tokens
 static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) {
     const DenseArgs& a = ms[0];
     const int gs = a.group_size;
@@ -1309,7 +1325,7 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     // at 700 tokens 695 / 236, at 2048 2030 / 560; down 3584 x 18944 at 700 470 / 118 (three ranges), at 64 (chunks of the decode kernel) 78 / 30
     // (64-token tiles, eight ranges), at 96 102 / 36.
     const int units = a.K / GG_UNIT;
-    const GtChoice best = gt_pick(tiles, units, (float)rows * (float)a.K / 2.f / 5.0e6f, n == 1 && a.T <= 65535 ? std::min(16, std::max(1, units / 4)) : 1,
+    const GtChoice best = gt_pick(tiles, units, (float)rows * (float)a.K / 2.f / 5.0e6f, n == 1 && a.T <= 65535 ? gemm_max_split(a, std::max(1, units / 4)) : 1,
                                   (float)a.T * (float)a.N * 4.f / 4.5e6f, gs % GG_UNIT ? 6 : 7, kGgTiles, 3);
     const GtTile& t = kGgTiles[best.tile];
     for (int i = 0; i < 3; ++i) g.a[i] = ms[i < n ? i : 0];
@@ -1321,7 +1337,7 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     const size_t xp_b = (size_t)a.T * a.K * 2, xs_b = (size_t)(a.K / 64) * g.t_pad * 4, pn_b = (size_t)words * 4;
     const size_t pt_b = g.splits > 1 ? (size_t)g.splits * a.T * a.N * 4 : 0;
     void* ws = nullptr;
-    if (mi355_scratch_get(&ws, MI355_SCR_GPTQ_GEMM, xp_b + xs_b + pn_b + pt_b, st, false)) return (int)hipErrorNotSupported;   // (no room while a stream is captured: token chunks)
+    if (mi355_scratch_get(&ws, MI355_SCR_GPTQ_GEMM, xp_b + xs_b + pn_b + pt_b, st, false, (size_t)(GPTQ_GEMM_X_BYTES + GEMM_PART_BYTES))) return (int)hipErrorNotSupported;   // (no room while a stream is captured: token chunks)
     uint8_t* base = static_cast<uint8_t*>(ws);
     uint16_t* xp = reinterpret_cast<uint16_t*>(base);
     float* xs = reinterpret_cast<float*>(base + xp_b);
@@ -1386,7 +1402,7 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     // 128 x 128 640), 3001 x 4096 x 14336 480 / 292 (192 x 256: exactly one round; 256 x 256 331), 2048 x 28672 x 4096 550 / 375,
     // 2048 x 4096 x 14336 215 (128 x 128, two per CU), 700 x 4096 x 14336 94 (two ranges; one: 175), 96 x 4096 x 14336 33 (64-token tiles,
     // eight ranges; one: 113), 64 x 28672 x 4096 96 / 44.
-    const int max_split = n == 1 && a[0].T <= 65535 && !(a[0].N & 3) && !(a[0].epi == MI355_EPI_SILU_MUL && (a[0].pair_offset & 3)) ? std::min(16, std::max(1, units / 8)) : 1;
+    const int max_split = n == 1 && a[0].T <= 65535 && !(a[0].N & 3) && !(a[0].epi == MI355_EPI_SILU_MUL && (a[0].pair_offset & 3)) ? gemm_max_split(a[0], std::max(1, units / 8)) : 1;
     GtChoice best = gt_pick([&](const GtTile& t) { return tiles(t, nullptr); }, units, (float)rows * (float)a[0].K * 2.f / 5.4e6f, max_split,
                             (float)a[0].T * (float)a[0].N * 4.f / 4.5e6f, 31);
     if (g_tune_gemm_tall) best = {0, 1};
@@ -1397,7 +1413,7 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     g.splits = (units + g.units_per_split - 1) / g.units_per_split;
     if (g.splits > 1) {
         void* p = nullptr;
-        if (mi355_scratch_get(&p, MI355_SCR_GPTQ_WIDE, (size_t)g.splits * a[0].T * a[0].N * sizeof(float), st, false)) { g.splits = 1; g.units_per_split = units; }
+        if (mi355_scratch_get(&p, MI355_SCR_GPTQ_WIDE, (size_t)g.splits * a[0].T * a[0].N * sizeof(float), st, false, (size_t)GEMM_PART_BYTES)) { g.splits = 1; g.units_per_split = units; }
         g.part = static_cast<float*>(p);
     }
     if (tiles(kGtTiles[best.tile], &g) * g.splits > 0x7FFFFFFF) return (int)hipErrorNotSupported;
@@ -1437,6 +1453,12 @@ static int dense_run(DenseArgs a, int wtype, int dt, hipStream_t st) {
         if (rc != (int)hipErrorNotSupported) return rc;                    // odd K, few tokens off the 16-byte grid: keep streaming in token chunks
     }
     if (wtype == DW_GPTQ4T && a.T >= (a.epi == MI355_EPI_SILU_MUL ? GPTQ_GEMM_MIN_PAIR_T : GPTQ_GEMM_MIN_T)) {
+        const int slab = gptq_gemm_slab(a.K);
+        if (a.T > slab) {
+            for (int t0 = 0; t0 < a.T; t0 += slab)
+                if (const int rc = dense_run(dense_rows(a, t0, slab), wtype, dt, st)) return rc;
+            return 0;
+        }
         const int rc = gptq_prompt_gemm(&a, 1, dt, st);
         if (rc != (int)hipErrorNotSupported) return rc;                    // groups of 32, odd strides: token chunks of the decode kernel
     }
@@ -1444,12 +1466,7 @@ static int dense_run(DenseArgs a, int wtype, int dt, hipStream_t st) {
     const int T = a.T;
     if (T < 1) return -2;
     for (int t0 = 0; t0 < T; t0 += chunk) {
-        DenseArgs c = a;
-        c.T = T - t0 < chunk ? T - t0 : chunk;
-        c.x = static_cast<const uint16_t*>(a.x) + (size_t)t0 * a.ldx;
-        c.out = static_cast<uint16_t*>(a.out) + (size_t)t0 * a.ldo;
-        if (a.resid) c.resid = static_cast<const uint16_t*>(a.resid) + (size_t)t0 * a.ldo;
-        const int rc = dense_dispatch(c, wtype, dt, st);
+        const int rc = dense_dispatch(dense_rows(a, t0, chunk), wtype, dt, st);
         if (rc) return rc;
     }
     return 0;
@@ -1866,7 +1883,12 @@ int mi355_internal_linear3(void* const* outs, const void* x, const void* const* 
     }
     hipStream_t st = (hipStream_t)stream;
     if (prompt) {
-        const int rc = is_gptq == 2 ? gptq_prompt_gemm(a, 3, dtype, st) : dense_prompt_gemm(a, 3, dtype, st);
+        int rc = 0;
+        const int slab = is_gptq == 2 ? gptq_gemm_slab(k) : num_tokens;
+        for (int t0 = 0; t0 < num_tokens && rc == 0; t0 += slab) {
+            const DenseArgs c[3] = {dense_rows(a[0], t0, slab), dense_rows(a[1], t0, slab), dense_rows(a[2], t0, slab)};
+            rc = is_gptq == 2 ? gptq_prompt_gemm(c, 3, dtype, st) : dense_prompt_gemm(c, 3, dtype, st);
+        }
         if (rc != (int)hipErrorNotSupported) return rc;
         if (num_tokens > 64) return -4;
     }

@@ -502,6 +502,30 @@ def test_gptq_prompt_gemm_every_tile(cv, T, N, K, gs, mode):
     check_ulp(got[rows], ref, dt, ulps=ulps, what="gptq prompt GEMM", mag=mag)
 
 
+def test_gptq_prompt_gemm_in_slabs(cv):
+    """more tokens than the permuted copy of x has room for (128 MiB: 3 328 of 18 944): slabs of tokens, rows at their borders against the product in 64
+    bits, residual in place; and the memory taken"""
+    T, N, K, gs = 8000, 48, 18944, 128
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    q = torch.randint(0, 16, (K, N), generator=gen, device="cuda", dtype=torch.int32)
+    packed = sum((q.view(K // 8, 8, N)[:, i] << (4 * i)) for i in range(8)).contiguous()
+    s = (torch.rand(K // gs, N, generator=gen, device="cuda") * 0.004 + 0.002).to(torch.bfloat16)
+    x, out = (torch.randn(*sh, generator=gen, device="cuda").to(torch.bfloat16) for sh in ((T, K), (T, N)))
+    rows = torch.tensor(sorted({0, 1, 255, 256, 3327, 3328, 3329, 6655, 6656, T - 1}), device="cuda")
+    y = x[rows].double() @ ((q.double() - 8).view(K // gs, gs, N) * s.double()[:, None]).view(K, N)
+    mag, want = y.abs(), y.to(torch.bfloat16).double() + out[rows].double()
+    lin = cv.GPTQLinear(packed, s, gs)
+
+    def taken():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free - torch.cuda.memory_reserved()
+    before = taken()
+    got = lin.forward(x, epilogue=cv.EPI_RESID, residual=out)
+    assert taken() - before <= (256 + 8) << 20                    # with room for partial sums
+    check_ulp(got[rows].double().cpu().numpy(), want.cpu().numpy(), "bf16", ulps=2.01, what="slabs", mag=mag.cpu().numpy())
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("T,N,K,gs,mode", [(32, 1184, 3584, 128, "store"), (32, 3584, 3584, 128, "resid"), (9, 224, 2048, 64, "store"),
                                            (48, 512, 4864, 256, "bias"), (17, 2 * 4736, 1792, 128, "silu"), (32, 2 * 608, 3584, 128, "silu"),
