@@ -971,6 +971,7 @@ static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
             ks = (nkb_w + kps - 1) / kps;
             const int tpad = mt * 16, ldp = a.N;
             void* pp = nullptr;
+            Mi355ScratchTurn turn(MI355_SCR_GPTQ_WIDE, st);
             const bool room = ks == 1 || mi355_scratch_get(&pp, MI355_SCR_GPTQ_WIDE, (size_t)ks * tpad * ldp * sizeof(float), st, false) == 0;
             float* part = static_cast<float*>(pp);
             if (room) {                                                 // (else dense_kernel below)
@@ -1337,6 +1338,7 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     const size_t xp_b = (size_t)a.T * a.K * 2, xs_b = (size_t)(a.K / 64) * g.t_pad * 4, pn_b = (size_t)words * 4;
     const size_t pt_b = g.splits > 1 ? (size_t)g.splits * a.T * a.N * 4 : 0;
     void* ws = nullptr;
+    Mi355ScratchTurn turn(MI355_SCR_GPTQ_GEMM, st);
     if (mi355_scratch_get(&ws, MI355_SCR_GPTQ_GEMM, xp_b + xs_b + pn_b + pt_b, st, false, (size_t)(GPTQ_GEMM_X_BYTES + GEMM_PART_BYTES))) return (int)hipErrorNotSupported;   // (no room while a stream is captured: token chunks)
     uint8_t* base = static_cast<uint8_t*>(ws);
     uint16_t* xp = reinterpret_cast<uint16_t*>(base);
@@ -1411,6 +1413,7 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     g.n_m = (a[0].T + kGtTiles[best.tile].bm - 1) / kGtTiles[best.tile].bm;
     g.units_per_split = (units + best.splits - 1) / best.splits;
     g.splits = (units + g.units_per_split - 1) / g.units_per_split;
+    Mi355ScratchTurn turn(MI355_SCR_GPTQ_WIDE, st);
     if (g.splits > 1) {
         void* p = nullptr;
         if (mi355_scratch_get(&p, MI355_SCR_GPTQ_WIDE, (size_t)g.splits * a[0].T * a[0].N * sizeof(float), st, false, (size_t)GEMM_PART_BYTES)) { g.splits = 1; g.units_per_split = units; }
@@ -1434,6 +1437,7 @@ static int dense_prompt_gemm_staged(const DenseArgs& a, int dt, hipStream_t st) 
     const size_t x_b = ((size_t)(a.T - 1) * a.ldx + a.K) * 2, w_b = ((size_t)(a.N - 1) * a.ldw + a.K) * 2, x_room = (x_b + 255) & ~(size_t)255;
     const bool x_off = (uintptr_t)a.x & 15, w_off = (uintptr_t)a.w & 15;
     void* ws = nullptr;
+    Mi355ScratchTurn turn(MI355_SCR_GPTQ_WIDE, st);                     // (the GEMM's, which takes it again)
     if ((!x_off && !w_off) || a.K % 64 || mi355_scratch_get(&ws, MI355_SCR_DENSE_WS, x_room + (w_off ? w_b : 0), st, false)) return (int)hipErrorNotSupported;
     uint8_t* base = static_cast<uint8_t*>(ws);
     hipError_t e = hipSuccess;

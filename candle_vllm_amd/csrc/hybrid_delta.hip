@@ -468,6 +468,7 @@ int mi355_hyb_delta_rule(float* o, float* state, int64_t state_stride, const flo
     const int64_t pieces = num_tokens / DPC + num_seqs, piece_bytes = heads * delta_rec_floats(dim, vdim) * 4, window = std::min(pieces, DELTA_WINDOW_BYTES / piece_bytes);
     if (dim % 16 == 0 && vdim % 16 == 0 && num_tokens >= DELTA_MIN_TOKENS && num_tokens / num_seqs >= DELTA_MIN_PER_SEQ && vdim <= 65535 * 16 && window > 0) {
         void* ws = nullptr;
+        Mi355ScratchTurn turn(MI355_SCR_DELTA, s_);
         if (heads <= 65535 && mi355_scratch_get(&ws, MI355_SCR_DELTA, (size_t)(window * piece_bytes), s_, false, (size_t)DELTA_WINDOW_BYTES) == 0) {   // (no room while a stream is captured: the walk)
             for (int64_t first = 0; first < pieces; first += window) {
                 const DeltaPieces q{static_cast<float*>(ws), num_seqs, delta_rec_floats(dim, vdim), (int)first, (int)std::min(window, pieces - first)};

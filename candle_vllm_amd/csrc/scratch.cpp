@@ -62,6 +62,11 @@ int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool ze
     return 0;
 }
 
+// A fixed set of locks, shared by the (stream, key) pairs that fall on the same one: held for the time of a few launches.
+namespace { std::recursive_mutex g_turns[64]; }
+Mi355ScratchTurn::Mi355ScratchTurn(int key, hipStream_t st) : slot_((int)((((uintptr_t)st >> 4) * 31 + (uintptr_t)key) % 64)) { g_turns[slot_].lock(); }
+Mi355ScratchTurn::~Mi355ScratchTurn() { g_turns[slot_].unlock(); }
+
 // Tests: an allocation above `bytes` fails the way one does on a full card (-1: none).
 extern "C" void mi355_internal_scratch_limit(int64_t bytes) { g_limit.store(bytes < 0 ? (size_t)-1 : (size_t)bytes); }
 

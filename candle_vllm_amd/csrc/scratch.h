@@ -25,5 +25,18 @@ enum {
 int mi355_scratch_get(void** out, int key, size_t bytes, hipStream_t st, bool zero_on_create, size_t most = (size_t)-1);
 extern "C" void mi355_scratch_release_all(void);
 
+// Launches that hand a buffer on to each other (a producer and its consumers) are enqueued under one of these, from before mi355_scratch_get until
+// the last of them: two host threads on one stream then take turns with it, instead of one's producer running between the other's two.  A thread
+// takes turns of one (stream, key) at a time; it may take that one again.
+class Mi355ScratchTurn {
+public:
+    Mi355ScratchTurn(int key, hipStream_t st);
+    ~Mi355ScratchTurn();
+    Mi355ScratchTurn(const Mi355ScratchTurn&) = delete;
+    Mi355ScratchTurn& operator=(const Mi355ScratchTurn&) = delete;
+private:
+    int slot_;
+};
+
 // void FFI entry points record their first failure here (mi355_last_error / mi355_clear_error in the header)
 void mi355_note_error(int code);

@@ -21,6 +21,8 @@ inline hipError_t hipGetLastError() { const hipError_t e = last_error; last_erro
 """
 HEAD = r"""
 #include <stdio.h>
+#include <thread>
+#include <vector>
 #include "scratch.h"
 size_t room, last_request; hipError_t last_error;
 #define CHECK(c) do { if (!(c)) { printf("line %d: %s\n", __LINE__, #c); return 1; } } while (0)
@@ -59,3 +61,16 @@ def test_growth_doubles_up_to_the_most_and_takes_what_is_asked_where_that_is_all
     room = 1500;
     CHECK(mi355_scratch_get(&b, 7, 1200, st, false) == 0 && last_request == 1200 && a != b && last_error == hipSuccess);
     """)
+
+
+def test_launches_of_two_threads_on_one_stream_take_turns(tmp_path):
+    """what a thread enqueues inside a turn is not interleaved with another's (`queue` stands for the stream: a data race without the turn, which the thread
+    sanitizer reports as well as the order does)"""
+    run(tmp_path, """
+    std::vector<int> queue;
+    auto work = [&](int me) { for (int i = 0; i < 2000; ++i) { Mi355ScratchTurn turn(12, st); { Mi355ScratchTurn again(12, st); queue.push_back(me); } std::this_thread::yield(); queue.push_back(me); } };
+    std::thread one(work, 1), two(work, 2);
+    one.join(); two.join();
+    CHECK(queue.size() == 8000);
+    for (size_t i = 0; i < queue.size(); i += 2) CHECK(queue[i] == queue[i + 1]);
+    """, "-fsanitize=thread")

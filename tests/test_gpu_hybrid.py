@@ -394,6 +394,35 @@ def test_delta_rule_no_room_for_the_pieces(lib):
         assert float((a - b).abs().max()) < 2e-5 * max(1.0, float(b.abs().max()))
 
 
+def test_delta_rule_two_threads_on_one_stream(lib):
+    """the pieces' records pass from one launch to the next: two threads on one stream, each with its own inputs, have the results they have alone"""
+    _gpu()
+    import threading
+    T, Hh, d = 200, 2, 64
+    C, stride = 3 * Hh * d, Hh * d * d
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    ctx, cu, slot = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([T], [0, T], [0]))
+    ins = [[torch.randn(*s, device="cuda", generator=gen) for s in ((T, C), (T, Hh), (T, Hh * d), (Hh,), (Hh * d,))] for _ in range(2)]
+    scratch = [torch.zeros(lib.mi355_hyb_delta_rule_scratch_floats(T, Hh, Hh, d, 1), device="cuda") for _ in range(2)]
+    outs = [[(torch.zeros(T, Hh * d, device="cuda"), torch.zeros(1, stride, device="cuda")) for _ in range(101)] for _ in range(2)]
+    st = _st()
+
+    def call(i, n):
+        (qkv, proj, pre, a_log, dtb), (o, state) = ins[i], outs[i][n]
+        assert lib.mi355_hyb_delta_rule(o.data_ptr(), state.data_ptr(), stride, qkv.data_ptr(), C, proj.data_ptr(), Hh, 0, pre.data_ptr(), Hh * d, 1, a_log.data_ptr(),
+                                        dtb.data_ptr(), ctx.data_ptr(), cu.data_ptr(), slot.data_ptr(), 1, T, Hh, Hh, d, d, 1e-6, scratch[i].data_ptr(), st) == 0
+    call(0, 0)
+    call(1, 0)
+    torch.cuda.synchronize()
+    go = threading.Barrier(2)
+    threads = [threading.Thread(target=lambda i=i: (go.wait(), [call(i, n) for n in range(1, 101)])) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    torch.cuda.synchronize()
+    for res in outs:
+        assert all(torch.equal(a, b) for r in res[1:] for a, b in zip(r, res[0]))
+
+
 def test_delta_rule_by_pieces_in_windows(lib):
     """more pieces than the workspace holds records of (256 MiB: 61 of 64 heads of 256 x 256): windows that begin inside a sequence and at the start of
     one, against the walk of the same tokens -- the same bound as the walk against 64 bits"""

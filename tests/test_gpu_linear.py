@@ -609,3 +609,30 @@ def test_no_room_for_a_workspace(cv, kind, T, N, K):
                 lib.mi355_internal_scratch_limit(-1)
             torch.cuda.current_stream().synchronize()
             check_ulp(host16(y, "bf16"), ref, "bf16", what=f"{kind}, limit {limit}")
+
+
+@pytest.mark.parametrize("kind,T,N,K", [("4-bit", 130, 64, 4096), ("16-bit", 96, 96, 4096), ("16-bit", 9, 256, 8192)])
+def test_two_threads_on_one_stream(cv, kind, T, N, K):
+    """launches that hand a workspace on to each other, from two threads on one stream, each over its own x: every result is the one it has alone, bit for bit"""
+    import threading
+    rng = np.random.default_rng(T + N)
+    if kind == "4-bit":
+        q, s = _gptq_case(rng, K, N, 128, "bf16")
+        lin = cv.GPTQLinear(dev_u32(G.gptq_pack(q)), dev16(s, "bf16"), 128)
+    else:
+        lin = cv.Linear(dev16(G.round_dt(rng.normal(0, 0.02, (N, K)), "bf16"), "bf16"), tiled=True)
+    xs = [torch.randn(T, K, device="cuda").to(torch.bfloat16) for _ in range(2)]
+    alone = [lin.forward(x) for x in xs]
+    torch.cuda.synchronize()
+    got = [[], []]
+    go = threading.Barrier(2)
+
+    def work(i):
+        go.wait()
+        got[i] = [lin.forward(xs[i]) for _ in range(300)]
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == 300 and all(torch.equal(y.view(torch.int16), alone[i].view(torch.int16)) for y in got[i])
