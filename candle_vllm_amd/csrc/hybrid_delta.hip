@@ -438,7 +438,7 @@ template <int ND, bool FULL> __global__ __launch_bounds__(320) void delta_piece_
         }
 }
 
-constexpr int DELTA_MIN_TOKENS = 64, DELTA_MIN_PER_SEQ = 48;
+constexpr int DELTA_MIN_TOKENS = 64, DELTA_MIN_TOKENS_WIDE = 80, DELTA_MIN_PER_SEQ = 48;
 constexpr int64_t DELTA_WINDOW_BYTES = 256ll << 20;
 
 }  // namespace
@@ -460,13 +460,16 @@ int mi355_hyb_delta_rule(float* o, float* state, int64_t state_stride, const flo
     DeltaArgs p{o, state, state_stride, qkv, ldq, proj, ldp, b_off, decay_in, ldd, decay_channels, a_log, dt_bias,
                 context_lens, cu_seqlens_q, state_slots, heads, kv_heads, dim, vdim, unit_eps};
     hipStream_t s_ = to_stream(stream);
-    // Whole 16-row tiles and portions of prompts: by pieces.  us per call, walk / pieces, 16 heads of 128 x 128: one sequence of 32 tokens 20 / 25,
-    // 64 31 / 27, 200 82 / 38, 2048 740 / 200; two sequences of 1050 402 / 150; 8 sequences of 16 21 / 32 (64 each: 35 / 38); 32 heads of 64 x 64,
-    // 64 tokens 25 / 20, 2048 590 / 170; 8 heads of 256 x 256, 64 tokens 44 / 48, 200 112 / 64, 2048 1019 / 310
+    // Whole 16-row tiles and portions of prompts: by pieces.  us per call, walk / pieces.  16 heads of 128 x 128: one portion of 64 tokens 32 / 27, 200 81 / 37,
+    // 2048 740 / 195; two of 1050 396 / 145; 4 of 64 40 / 39, 8 of 64 56 / 57, 8 of 400 246 / 230; one of 500 beside 7 single tokens 266 / 89.  32 heads of
+    // 64: 64 tokens 25 / 20, 2048 590 / 174.  8 heads of 256: 64 tokens 44 / 48, 80 51 / 49, 200 111 / 63, 2048 1018 / 310.
+    // The lengths are on the device; what is known here is their mean.  Portions that fill the chip by themselves would be walked a little faster (16 of 50
+    // 79 / 102, 16 of 100 135 / 158), but a batch of the same mean with one long portion in it would take three times as long, so the mean decides
     // Their records take 8.6 KB per token and 16 heads of 128: windows of at most 256 MiB (7 800 such tokens), one behind the other, with the state in
     // its slot in between
-    const int64_t pieces = num_tokens / DPC + num_seqs, piece_bytes = heads * delta_rec_floats(dim, vdim) * 4, window = std::min(pieces, DELTA_WINDOW_BYTES / piece_bytes);
-    if (dim % 16 == 0 && vdim % 16 == 0 && num_tokens >= DELTA_MIN_TOKENS && num_tokens / num_seqs >= DELTA_MIN_PER_SEQ && vdim <= 65535 * 16 && window > 0) {
+    const int64_t pieces = num_tokens / DPC + num_seqs, piece_bytes = heads * delta_rec_floats(dim, vdim) * 4, room = DELTA_WINDOW_BYTES / piece_bytes;
+    if (dim % 16 == 0 && vdim % 16 == 0 && num_tokens >= (dim > 128 ? DELTA_MIN_TOKENS_WIDE : DELTA_MIN_TOKENS) && num_tokens / num_seqs >= DELTA_MIN_PER_SEQ && vdim <= 65535 * 16 && room > 0) {
+        const int64_t windows = (pieces + room - 1) / room, window = (pieces + windows - 1) / windows;             // of one size: the scan of a short one is as long
         void* ws = nullptr;
         Mi355ScratchTurn turn(MI355_SCR_DELTA, s_);
         if (heads <= 65535 && mi355_scratch_get(&ws, MI355_SCR_DELTA, (size_t)(window * piece_bytes), s_, false, (size_t)DELTA_WINDOW_BYTES) == 0) {   // (no room while a stream is captured: the walk)
