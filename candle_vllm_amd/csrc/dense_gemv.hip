@@ -1346,6 +1346,7 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     uint32_t* panel = reinterpret_cast<uint32_t*>(base + xp_b + xs_b);
     g.xp = xp; g.xs = xs; g.part = reinterpret_cast<float*>(base + xp_b + xs_b + pn_b);
     for (int i = 0; i < n; ++i) { g.panel[i] = panel; panel += ((int64_t)(a.K / gs) * ms[i].N + 63) / 64 * 64; }
+    gt_last_launch = 100 * best.tile + g.splits;
     const int rc = dt == MI355_DTYPE_BF16 ? gptq_gemm_dt<MI355_DTYPE_BF16>(g, xp, xs, best.tile, st) : gptq_gemm_dt<MI355_DTYPE_F16>(g, xp, xs, best.tile, st);
     if (rc || g.splits <= 1) return rc;
     const dim3 grid(((silu ? a.pair_offset : a.N) + 255) / 256, a.T);
@@ -1420,6 +1421,7 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
         g.part = static_cast<float*>(p);
     }
     if (tiles(kGtTiles[best.tile], &g) * g.splits > 0x7FFFFFFF) return (int)hipErrorNotSupported;
+    gt_last_launch = 100 * best.tile + g.splits;
     if (dt == MI355_DTYPE_BF16) { if (a[0].wtiled) dense_gemm_epi<MI355_DTYPE_BF16, true>(g, best.tile, st); else dense_gemm_epi<MI355_DTYPE_BF16, false>(g, best.tile, st); }
     else { if (a[0].wtiled) dense_gemm_epi<MI355_DTYPE_F16, true>(g, best.tile, st); else dense_gemm_epi<MI355_DTYPE_F16, false>(g, best.tile, st); }
     if (g.splits > 1) {

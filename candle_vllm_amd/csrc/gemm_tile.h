@@ -34,6 +34,13 @@ __device__ __forceinline__ void gt_dma(const uint8_t* base, uint32_t off, uint32
                  : "=&s"(keep) : "s"(dst), "v"(off), "s"(base) : "memory");
 }
 
+// the same from 64-bit addresses
+__device__ __forceinline__ void gt_dma(const uint8_t* src, uint32_t dst) {
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "s"(dst), "v"(src) : "memory");
+}
+
 // a value every lane holds alike, in scalar registers (what the compiler works out through a division is in vector registers)
 __device__ __forceinline__ const uint8_t* gt_uniform(const uint8_t* p) {
     const uint64_t v = (uint64_t)(uintptr_t)p;
@@ -88,8 +95,10 @@ struct GemmTile {
         if (n < NF) f.b[n] = *reinterpret_cast<const uint4*>(smem + buf + (TILED ? b_rd + (half ? 1024u : 0u) : (b_rd ^ (half ? 64u : 0u))) + (size_t)n * 2048);
         else f.a[n - NF] = *reinterpret_cast<const uint4*>(smem + buf + (a_rd ^ (half ? 64u : 0u)) + (size_t)(n - NF) * 2048);
     }
-    // a_base + a_off[r]: source of DMA instruction r in unit 0 (units are 128 B apart); b_base[r] + b_off[r] likewise, b_step bytes apart
-    __device__ __forceinline__ void run(const uint8_t* a_src, const uint32_t (&a_off)[AR], const uint8_t* const (&b_src)[BR],
+    // a_base + a_off[r]: source of DMA instruction r in unit 0 (units are 128 B apart); b_base[r] + b_off[r] likewise, b_step bytes apart.
+    // Offsets of 64 bits: rows gathered from anywhere
+    template <class AOff>
+    __device__ __forceinline__ void run(const uint8_t* a_src, const AOff (&a_off)[AR], const uint8_t* const (&b_src)[BR],
                                         const uint32_t (&b_off)[BR], uint32_t b_step, int units) {
         const uint8_t* a_base = gt_uniform(a_src);
         const uint8_t* b_base[BR];
@@ -102,6 +111,7 @@ struct GemmTile {
         auto dma = [&](int u, uint32_t buf, int n) {                      // instruction n of unit u into the buffer at `buf`
             const uint32_t dst = lds0 + buf + (uint32_t)wave * 1024u;
             if (n < BR) gt_dma(b_base[n] + (size_t)u * b_step, b_off[n], dst + A_BYTES + (uint32_t)n * 8192u);
+            else if constexpr (sizeof(AOff) == 8) gt_dma(a_base + (size_t)u * 128 + a_off[n - BR], dst + (uint32_t)(n - BR) * 8192u);
             else gt_dma(a_base + (size_t)u * 128, a_off[n - BR], dst + (uint32_t)(n - BR) * 8192u);
         };
         Frags f0, f1;
@@ -171,6 +181,8 @@ static constexpr GtTile kGtTiles[] = {{256, 256, 1, 1.46f}, {192, 256, 1, 1.28f}
     case 0: CALL(2, 4, 8, 4, 2); break; case 1: CALL(2, 4, 6, 4, 2); break; case 2: CALL(2, 4, 4, 2, 2); break; \
     case 3: CALL(2, 4, 4, 2, 4); break; default: CALL(2, 4, 2, 2, 6); break; } } while (0)
 struct GtChoice { int tile, splits; };
+// tile and K ranges of this thread's last launch, 100 tile + ranges (tests: mi355_internal_last_gemm)
+inline thread_local int gt_last_launch = -1;
 // tiles(t): workgroups of the launch with tile t; stream_us: the weights' read; part_us: write or read of one range's partial sums
 template <class F>
 static inline GtChoice gt_pick(F tiles, int units, float stream_us, int max_split, float part_us, unsigned allowed, const GtTile* table = kGtTiles, int n_table = 5) {

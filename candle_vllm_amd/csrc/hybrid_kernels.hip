@@ -7,6 +7,7 @@
 // ctx[s] - that many cached ones; a portion that starts at position 0 starts from zero state whatever its slot holds.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include <math.h>
 
 #include "common.h"
@@ -253,7 +254,8 @@ template <int B> __global__ __launch_bounds__(256) void linear_bf16_lds_kernel(L
 // The same products where K is a multiple of 64, on the main loop of gemm_tile.h (128 x 128 tiles, 32-wide K steps through registers in the
 // kernel above reached 400 - 740 TFLOP/s at 2100 tokens).
 struct LinGrid { int n_m, n_n; };
-template <int B, int WM, int WN, int MF, int NF, int S> __global__ __launch_bounds__(512, 2) void linear_bf16_gemm_kernel(LinArgs p, LinGrid grid) {
+// GATHER: rows of `a` by row_src
+template <int B, int WM, int WN, int MF, int NF, int S, bool GATHER> __global__ __launch_bounds__(512, 2) void linear_bf16_gemm_kernel(LinArgs p, LinGrid grid) {
     typedef GemmTile<MI355_DTYPE_BF16, WM, WN, MF, NF, S, false> Tile;
     extern __shared__ __align__(1024) uint8_t lin_smem[];
     const GtPlace at = gt_place(blockIdx.x, grid.n_m, grid.n_n);
@@ -262,14 +264,16 @@ template <int B, int WM, int WN, int MF, int NF, int S> __global__ __launch_boun
     int64_t w_off;
     if (!lin_group(p, t0, w_off)) return;
     Tile tile(lin_smem);
-    const uint8_t* a_base = static_cast<const uint8_t*>(p.a) + (p.row_src ? 0 : (size_t)t0 * p.lda * 2);
+    const uint8_t* a_base = static_cast<const uint8_t*>(p.a) + (GATHER ? 0 : (size_t)t0 * p.lda * 2);
     const uint8_t* wb = reinterpret_cast<const uint8_t*>(static_cast<const uint16_t*>(p.w) + w_off);
-    uint32_t a_off[Tile::AR], b_off[Tile::BR];
+    std::conditional_t<GATHER, uint64_t, uint32_t> a_off[Tile::AR];      // the rows of a tile are at most 255 apart, gathered ones any distance
+    uint32_t b_off[Tile::BR];
     const uint8_t* b_base[Tile::BR];
 #pragma unroll
     for (int r = 0; r < Tile::AR; ++r) {
         const int t = min(t0 + tile.stage_row(r), p.T - 1);              // rows beyond the last are multiplied and never stored
-        a_off[r] = (uint32_t)(p.row_src ? p.row_src[t] : t - t0) * (uint32_t)p.lda * 2u + tile.stage_chunk();
+        if constexpr (GATHER) a_off[r] = (uint64_t)(uint32_t)p.row_src[t] * (uint64_t)p.lda * 2u + tile.stage_chunk();
+        else a_off[r] = (uint32_t)(t - t0) * (uint32_t)p.lda * 2u + tile.stage_chunk();
     }
 #pragma unroll
     for (int r = 0; r < Tile::BR; ++r) {
@@ -319,17 +323,23 @@ template <int B, int WM, int WN, int MF, int NF, int S> __global__ __launch_boun
 }
 template <int B> static void linear_gemm_launch(const LinArgs& p, int which, int n_m, int nz, hipStream_t st) {
     const LinGrid grid{n_m, (p.N + kGtTiles[which].bn - 1) / kGtTiles[which].bn};
-#define LIN_GO(WM_, WN_, MF_, NF_, S_) do { \
+#define LIN_GO_(G_, WM_, WN_, MF_, NF_, S_) do { \
         typedef GemmTile<MI355_DTYPE_BF16, WM_, WN_, MF_, NF_, S_, false> Tile_; \
         static Mi355DevOnce attr_; \
-        if (!attr_.done()) { (void)hipFuncSetAttribute((const void*)linear_bf16_gemm_kernel<B, WM_, WN_, MF_, NF_, S_>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Tile_::LDS); attr_.set(); } \
-        linear_bf16_gemm_kernel<B, WM_, WN_, MF_, NF_, S_><<<dim3(grid.n_m * grid.n_n, 1, nz), 512, Tile_::LDS, st>>>(p, grid); } while (0)
-    GT_TILES(which, LIN_GO);
+        if (!attr_.done()) { (void)hipFuncSetAttribute((const void*)linear_bf16_gemm_kernel<B, WM_, WN_, MF_, NF_, S_, G_>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Tile_::LDS); attr_.set(); } \
+        linear_bf16_gemm_kernel<B, WM_, WN_, MF_, NF_, S_, G_><<<dim3(grid.n_m * grid.n_n, 1, nz), 512, Tile_::LDS, st>>>(p, grid); } while (0)
+#define LIN_GO(...) LIN_GO_(false, __VA_ARGS__)
+#define LIN_GATHER(WM_, WN_, MF_, NF_, S_) do { if constexpr ((WM_) * (MF_) * 16 <= 128 && B != LIN_SEG_BUILD) LIN_GO_(true, WM_, WN_, MF_, NF_, S_); } while (0)   // (a grouped product's tiles)
+    gt_last_launch = 100 * which + 1;
+    if (p.row_src) GT_TILES(which, LIN_GATHER);
+    else GT_TILES(which, LIN_GO);
+#undef LIN_GATHER
 #undef LIN_GO
+#undef LIN_GO_
 }
-// operands the GEMM's 16-byte pieces and 32-bit offsets reach (rows: of `a`, as far as they are known)
-static bool linear_gemm_ok(const LinArgs& p, bool a_f32, int64_t a_rows) {
-    return !a_f32 && p.a_vec && p.w_vec && p.K % 64 == 0 && p.N % 16 == 0 && a_rows * p.lda * 2 < (1ll << 32) && (int64_t)p.K * 2 * 256 < (1ll << 32);
+// operands the GEMM's 16-byte pieces and its 32-bit offsets inside a tile reach
+static bool linear_gemm_ok(const LinArgs& p, bool a_f32) {
+    return !a_f32 && p.a_vec && p.w_vec && p.K % 64 == 0 && p.N % 16 == 0 && (int64_t)p.lda * 512 < (1ll << 32) && (int64_t)p.K * 512 < (1ll << 32);
 }
 
 // Up to 16 tokens, bf16 weights: the product is a stream over the weights.  A workgroup owns 16 weight rows; its NW waves take the
@@ -1916,7 +1926,7 @@ static int linear_launch(float* out, int32_t ldo, int64_t o_bs, const void* a, i
         const dim3 grid(glu ? n / 32 : (n + 15) / 16, 1, nz);
         if (k >= 2048) { if (af) LIN_EPI_(p, (linear_bf16_stream_kernel<float, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); else LIN_EPI(p, (linear_bf16_stream_kernel<uint16_t, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); }
         else { if (af) LIN_EPI_(p, (linear_bf16_stream_kernel<float, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); else LIN_EPI(p, (linear_bf16_stream_kernel<uint16_t, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); }
-    } else if (linear_gemm_ok(p, af, T)) {
+    } else if (linear_gemm_ok(p, af)) {
         // (segments end at multiples of 128 columns: only the tiles of that width have one left operand each)
         const GtChoice c = gt_pick([&](const GtTile& t) { return (int64_t)((T + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch; }, k / 64,
                                    (float)n * (float)k * 2.f * (float)batch / 5.4e6f, 1, 0.f, seg ? 28 : 31);
@@ -1932,6 +1942,9 @@ static int linear_launch(float* out, int32_t ldo, int64_t o_bs, const void* a, i
     }
     LAUNCH_OK(); return 0;
 }
+
+// which GEMM tile this thread's last product took (100 tile + K ranges), -1: none since the last call
+int mi355_internal_last_gemm(void) { const int v = gt_last_launch; gt_last_launch = -1; return v; }
 
 int mi355_hyb_linear(float* out, int32_t ldo, const void* a, int32_t a_dtype, int32_t lda, const void* w, const float* bias,
                      int32_t T, int32_t n, int32_t k, int32_t dtype, int64_t stream) {
@@ -2472,7 +2485,7 @@ static int grouped_launch(void* out, int32_t out_dtype, int32_t ldo, const void*
         const dim3 grid(glu ? n / 32 : (n + 15) / 16, n_blocks, 1);
         if (k >= 2048) { if (af) LIN_EPI2_(p, (linear_bf16_stream_kernel<float, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); else LIN_EPI2(p, (linear_bf16_stream_kernel<uint16_t, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); }
         else { if (af) LIN_EPI2_(p, (linear_bf16_stream_kernel<float, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); else LIN_EPI2(p, (linear_bf16_stream_kernel<uint16_t, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); }
-    } else if ((block_rows == 64 || block_rows == 128) && linear_gemm_ok(p, af, p.T)) {
+    } else if ((block_rows == 64 || block_rows == 128) && linear_gemm_ok(p, af)) {
         // the tile as tall as a block: 64 tokens, or 128 (two workgroups per CU where the blocks fill the chip, else one with more buffers)
         const int which = block_rows == 64 ? 4 : (int64_t)n_blocks * ((n + 127) / 128) > mi355_num_cus() ? 2 : 3;
         LIN_EPI2(p, (linear_gemm_launch<EPI>(p, which, n_blocks, 1, st_)));

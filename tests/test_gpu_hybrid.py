@@ -263,6 +263,69 @@ def test_conv_silu_portions_and_state(lib, taps):
     assert np.abs(np.concatenate(got_b) - want_b).max() < 5e-6
 
 
+@pytest.mark.parametrize("block_rows,blocks,n,tile", [(64, 5, 160, 4), (128, 3, 160, 3), (128, 130, 160, 2)])
+@pytest.mark.parametrize("k", [640, 704])
+@pytest.mark.parametrize("gather", [False, True])
+def test_grouped_products_of_many_units(lib, block_rows, blocks, n, tile, k, gather):
+    """the grouped products on each of the GEMM's tiles over ten and eleven units of 64 k (all of its buffers refilled), blocks that end inside a tile and
+    one that is empty, rows in place or gathered, plain, with an activation and as gate and up -- against 64 bits"""
+    _gpu()
+    gen = torch.Generator(device="cuda").manual_seed(k + blocks)
+    R, E = block_rows * blocks, 3
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen)          # noqa: E731
+    a, w = rnd(R if not gather else 300, k + 8).to(torch.bfloat16), (rnd(E, n, k) / math.sqrt(k)).to(torch.bfloat16)
+    src = torch.randint(0, 300, (R,), device="cuda", generator=gen, dtype=torch.int32) if gather else torch.arange(R, device="cuda", dtype=torch.int32)
+    expert = torch.arange(blocks, device="cuda") % E
+    end = torch.arange(1, blocks + 1, device="cuda") * block_rows - torch.arange(blocks, device="cuda") % 7 * 5
+    end[1] = block_rows                                                     # nothing in the second block
+    table = torch.stack([expert, end], 1).int().contiguous()
+    live = (torch.arange(R, device="cuda") < end.repeat_interleave(block_rows))
+    z = torch.cat([a[src[b * block_rows:(b + 1) * block_rows].long(), :k].double() @ w[expert[b]].double().t() for b in range(blocks)])
+    pt = src.data_ptr() if gather else None
+    for act, glu in ((0, False), (1, False), (1, True)):
+        want = (torch.nn.functional.silu(z.view(R, -1, 2, 16)[:, :, 0]) * z.view(R, -1, 2, 16)[:, :, 1]).reshape(R, -1) if glu else torch.nn.functional.silu(z) if act else z
+        out = torch.full((R, n), 7.0, device="cuda")
+        if glu:
+            ok(lib.mi355_hyb_linear_grouped_glu(out.data_ptr(), F32, n, a.data_ptr(), k + 8, pt, w.data_ptr(), n * k, table.data_ptr(), block_rows, blocks, n // 2, k, 1, BF16, _st()))
+        else:
+            ok(lib.mi355_hyb_linear_grouped_act(out.data_ptr(), F32, n, a.data_ptr(), BF16, k + 8, pt, w.data_ptr(), n * k, table.data_ptr(), block_rows, blocks, n, k, act, BF16, _st()))
+        assert lib.mi355_internal_last_gemm() == 100 * tile + 1
+        got = out[:, :want.shape[1]]
+        assert bool((out[~live] == 7).all()) and bool((out[:, want.shape[1]:] == 7).all())
+        assert float((got[live].double() - want[live]).abs().max()) < 3e-5 * max(1.0, float(want[live].abs().max()))
+
+
+def test_grouped_product_of_rows_far_apart(lib):
+    """rows gathered from an operand of more than 4 GiB"""
+    _gpu()
+    k, n, rows = 2048, 32, (1 << 20) + 300
+    a = torch.empty(rows, k, device="cuda", dtype=torch.bfloat16)
+    src = torch.tensor([5, rows - 1, 17, rows - 200] + [i % 64 for i in range(60)], device="cuda", dtype=torch.int32)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    a[:512] = torch.randn(512, k, device="cuda", generator=gen).to(torch.bfloat16)
+    a[-512:] = torch.randn(512, k, device="cuda", generator=gen).to(torch.bfloat16)
+    w = (torch.randn(1, n, k, device="cuda", generator=gen) / math.sqrt(k)).to(torch.bfloat16)
+    table, out = torch.tensor([[0, 64]], device="cuda", dtype=torch.int32), torch.empty(64, n, device="cuda")
+    ok(lib.mi355_hyb_linear_grouped(out.data_ptr(), n, a.data_ptr(), BF16, k, src.data_ptr(), w.data_ptr(), n * k, table.data_ptr(), 64, 1, n, k, BF16, _st()))
+    want = a[src.long()].double() @ w[0].double().t()
+    assert float((out.double() - want).abs().max()) < 3e-5 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("T,segs,tile", [(40, (128, 256), 4), (1030, (1280, 1280), 3), (1030, (3072, 1024), 2)])
+def test_segmented_products_of_many_units(lib, T, segs, tile):
+    """column segments with a left operand each, on each of the GEMM's 128-column tiles over eleven units of 64 k -- against 64 bits"""
+    _gpu()
+    k, n, first = 704, sum(segs), 1
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    a = torch.randn(first + len(segs), T, k + 8, device="cuda", generator=gen).to(torch.bfloat16)
+    w, b = (torch.randn(n, k, device="cuda", generator=gen) / math.sqrt(k)).to(torch.bfloat16), torch.randn(n, device="cuda", generator=gen)
+    rows, out, ends = np.array(segs, np.int32), torch.empty(T, n, device="cuda"), np.cumsum((0,) + segs)
+    ok(lib.mi355_hyb_linear_segments(out.data_ptr(), n, a.data_ptr(), BF16, k + 8, T * (k + 8), first, w.data_ptr(), b.data_ptr(), rows.ctypes.data, len(segs), T, n, k, BF16, _st()))
+    assert lib.mi355_internal_last_gemm() == 100 * tile + 1
+    want = torch.cat([a[first + i, :, :k].double() @ w[ends[i]:ends[i + 1]].double().t() for i in range(len(segs))], 1) + b.double()
+    assert float((out.double() - want).abs().max()) < 3e-5 * max(1.0, float(want.abs().max()))
+
+
 @pytest.mark.parametrize("Hh,G,d,vd,per_channel", [(2, 1, 32, 32, False), (3, 3, 20, 70, True), (4, 2, 64, 16, True), (1, 1, 128, 300, False),
                                                   (2, 2, 136, 64, True)])
 def test_delta_rule_portions_and_state(lib, Hh, G, d, vd, per_channel):
