@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(512) dense3r_kernel(const DenseArgs a0, const 
     else dense_body<DT, WTYPE, MT, 1, GJ>(a2, bx - t0 - t1, &rp);
 }
 
-// ------------------------------------------------------------------------------------------------ 5..64 tokens x 16-bit weights, many row tiles
+// ------------------------------------------------------------------------------------------------ 5..16 tokens x 16-bit weights, many row tiles; 5..32, long K
 // dense_body gives a workgroup ONE row tile (or gate/up pair) and lets its waves split K: every wave then fetches its own copy of
 // the activations of its k-blocks -- at 32 tokens 16 KB of x (from L2) for every 8 KB of weights, and all of a k-block's loads are
 // requested, waited for and consumed before the next k-block's go out (measured on BASELINE configs[2], Llama-3-8B bf16 at batch
@@ -955,8 +955,8 @@ static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
         // k-blocks plus the epilogue launch is not faster than its one launch)
         const int wtiles = (pair ? a.pair_offset : a.N) / 16;
         const int nkb_w = a.K >> 8;
-        const bool many = wtiles >= 4 * 192, longk = !pair && nkb_w >= 32 && mt <= 3;
-        if (!g_tune_wide_off && a.T > 4 && (many || longk) && (!pair || mt <= 2) && !((uintptr_t)a.x & 15) && !(a.ldx & 7) &&
+        const bool many = wtiles >= 4 * 192 && mt == 1, longk = !pair && nkb_w >= 32 && mt <= 2;   // (more tokens: the prompt GEMM, dense_run)
+        if (!g_tune_wide_off && a.T > 4 && (many || longk) && !((uintptr_t)a.x & 15) && !(a.ldx & 7) &&
             !((uintptr_t)a.w & 15) && (a.wtiled || !(a.ldw & 7))) {
             const int nwv = many ? (g_tune_wide_nw == 2 ? 2 : 4) : 4;
             const int gx = (wtiles + nwv - 1) / nwv;
@@ -982,8 +982,7 @@ static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
                     if (!attr) { (void)hipFuncSetAttribute((const void*)dense_wide_kernel<DT, MT_, R_, NW_>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024); attr = true; } \
                     hipLaunchKernelGGL((dense_wide_kernel<DT, MT_, R_, NW_>), grid, block, lds, st, a, part, ldp, kps); } while (0)
 #define DWD_GO(MT_, R_) do { if (nwv == 2) DWD_GO2(MT_, R_, 2); else DWD_GO2(MT_, R_, 4); } while (0)
-                if (pair) { if (mt == 1) DWD_GO(1, 2); else DWD_GO(2, 2); }
-                else switch (mt) { case 1: DWD_GO(1, 1); break; case 2: DWD_GO(2, 1); break; case 3: DWD_GO(3, 1); break; default: DWD_GO(4, 1); break; }
+                if (pair) DWD_GO(1, 2); else if (mt == 1) DWD_GO(1, 1); else DWD_GO(2, 1);
 #undef DWD_GO2
 #undef DWD_GO
                 if (hipGetLastError() != hipSuccess) return -1;

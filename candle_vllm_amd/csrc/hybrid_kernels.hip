@@ -328,7 +328,7 @@ template <int B> static void linear_gemm_launch(const LinArgs& p, int which, int
         static Mi355DevOnce attr_; \
         if (!attr_.done()) { (void)hipFuncSetAttribute((const void*)linear_bf16_gemm_kernel<B, WM_, WN_, MF_, NF_, S_, G_>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Tile_::LDS); attr_.set(); } \
         linear_bf16_gemm_kernel<B, WM_, WN_, MF_, NF_, S_, G_><<<dim3(grid.n_m * grid.n_n, 1, nz), 512, Tile_::LDS, st>>>(p, grid); } while (0)
-#define LIN_GO(...) LIN_GO_(false, __VA_ARGS__)
+#define LIN_GO(WM_, WN_, MF_, NF_, S_) do { if constexpr ((WN_) * (NF_) * 16 == 128 || B != LIN_SEG_BUILD) LIN_GO_(false, WM_, WN_, MF_, NF_, S_); } while (0)   // (segments: 128 columns)
 #define LIN_GATHER(WM_, WN_, MF_, NF_, S_) do { if constexpr ((WM_) * (MF_) * 16 <= 128 && B != LIN_SEG_BUILD) LIN_GO_(true, WM_, WN_, MF_, NF_, S_); } while (0)   // (a grouped product's tiles)
     gt_last_launch = 100 * which + 1;
     if (p.row_src) GT_TILES(which, LIN_GATHER);
