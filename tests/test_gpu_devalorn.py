@@ -160,7 +160,7 @@ def test_step_between_two_layers_over_portions(lib, dtype, W, mixes, top):
 @pytest.mark.parametrize("T,k,segs,first", [(3, 40, (128, 128, 256), 0), (1, 2080, (256, 128), 1), (20, 72, (128, 128), 0), (50, 33, (128, 384), 1), (130, 64, (256, 128, 128), 0),
                                             (70, 40, (128,) * 8, 0)])
 def test_products_whose_segments_read_different_operands(lib, dtype, T, k, segs, first):
-    """every product kernel (stream, tile, LDS tile, f32): segment i of the columns multiplies operand first + i"""
+    """stream, tile, LDS tile and f32 kernels, one unit of the GEMM (many units: test_gpu_hybrid.py): segment i of the columns multiplies operand first + i"""
     _gpu()
     rng = np.random.default_rng(k)
     n, stride = sum(segs), T * (k + 8)

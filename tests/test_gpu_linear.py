@@ -52,7 +52,7 @@ def check_ulp(got, ref, dt, ulps=1.01, what="", mag=None):
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("T,N,K", [(1, 256, 512), (5, 48, 256), (16, 1024, 1024), (17, 64, 768), (33, 128, 512),
                                    (64, 96, 256), (70, 32, 512), (128, 64, 512), (200, 48, 256),
-                                   (256, 384, 1024), (300, 200, 576), (97, 130, 64)])   # >= 96 tokens: the hand-written 128 x 128 MFMA GEMM (ragged T / N tiles, one K step)
+                                   (256, 384, 1024), (300, 200, 576), (97, 130, 64)])   # >= 33 tokens: the MFMA GEMM (ragged T / N tiles, one K step)
 def test_linear_matches_oracle(cv, dt, T, N, K):
     rng = np.random.default_rng(T * 1000 + N)
     x = G.round_dt(rng.normal(0, 1, (T, K)), dt)
@@ -68,12 +68,13 @@ def test_linear_matches_oracle(cv, dt, T, N, K):
               mag=G.linear16(x, w, None, dt))
 
 
-@pytest.mark.parametrize("T,N,K", [(33, 288, 2304), (65, 160, 4096),                          # 64-token tiles, K in ranges; one token into the next tile
-                                   (130, 96, 8192),                                            # K in ranges over three token tiles
-                                   (900, 8192, 128),                                           # 128 x 128 tiles, exactly two per CU
-                                   (1530, 8192, 128),                                          # 192 x 256 tiles, exactly one per CU, ragged tokens
-                                   (1540, 8208, 128)])                                         # 256 x 256 tiles, ragged both ways
-def test_linear_prompt_gemm_every_tile(cv, T, N, K):
+@pytest.mark.parametrize("T,N,K,launch", [(33, 288, 2304, 404), (65, 160, 4096, 408),          # 64-token tiles, K in 4 and 8 ranges; one token into the next tile
+                                          (130, 96, 8192, 416),                                # K in 16 ranges over three token tiles
+                                          (900, 8192, 128, 201),                               # 128 x 128 tiles, exactly two per CU
+                                          (1030, 2560, 704, 301),                              # 128 x 128 tiles, one per CU
+                                          (1530, 8192, 128, 101),                              # 192 x 256 tiles, exactly one per CU, ragged tokens
+                                          (1540, 8208, 128, 1)])                               # 256 x 256 tiles, ragged both ways
+def test_linear_prompt_gemm_every_tile(cv, T, N, K, launch):
     """16-bit prompt GEMM where its dispatch takes each of its tiles and K splits: row-major and tiled weights alike bit for bit, and within the
     op's bound of the oracle (tokens and rows at the tile's edges and at the matrix's)"""
     from candle_vllm_amd._lib import lib
@@ -96,6 +97,7 @@ def test_linear_prompt_gemm_every_tile(cv, T, N, K):
             out = torch.full((T, n_out), float("nan"), dtype=torch.bfloat16, device="cuda")
             assert fn(out.data_ptr(), xd.data_ptr(), img.data_ptr(), bias.data_ptr() if bias is not None else None,
                       resid.data_ptr() if resid is not None else None, T, N, K, 2, epi, st) == 0
+            assert lib.mi355_internal_last_gemm() == launch       # 100 tile + K ranges
             outs.append(host16(out, dt))
         assert len(outs) == 1 or np.array_equal(outs[0], outs[1])
         y = G.linear16(x[rows], w, None, dt)
@@ -141,10 +143,10 @@ def test_linear_prompt_operands_off_the_grid_of_any_shape(cv, T, N, K, off_x, of
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("T,N,K", [(256, 384, 1024), (300, 200, 576), (97, 130, 64), (700, 128, 256)])
 def test_linear_prompt_gemm_tall_tile(cv, dt, T, N, K):
-    """the 256 x 128 tile of the 16-bit prompt GEMM (8 waves, tuning key 30 bits 32 | 64 = wherever the GEMM runs): the same rounding chain as
-    the 128 x 128 tile -- bit for bit (same K order per output element) -- and within the op's bound of the oracle; plain, tiled-image and
+    """the 256 x 256 tile of the 16-bit prompt GEMM (tuning key 30 bits 32 | 64 = wherever the GEMM runs): the same as the 64-token tile these launches
+    take by themselves -- bit for bit (K in one range, the same order per output element) -- and within the op's bound of the oracle; plain, residual and
     SiLU * up launches, ragged token / column tiles"""
-    from candle_vllm_amd import tuning
+    from candle_vllm_amd import lib, tuning
     rng = np.random.default_rng(T * 7 + N)
     x = G.round_dt(rng.normal(0, 1, (T, K)), dt)
     w = G.round_dt(rng.normal(0, 0.05, (N, K)), dt)
@@ -160,8 +162,10 @@ def test_linear_prompt_gemm_tall_tile(cv, dt, T, N, K):
         return y, y2, y3
 
     base = run()
+    assert lib.mi355_internal_last_gemm() == 401
     with tuning(30, 32 | 64):
         tall = run()
+    assert lib.mi355_internal_last_gemm() == 1
     for a_, b_ in zip(base, tall):
         assert np.array_equal(np.asarray(a_), np.asarray(b_))
     check_ulp(tall[0], G.linear16(x, w, b, dt), dt, what="linear+bias", ulps=2.01, mag=G.linear16(x, w, None, dt))
@@ -378,10 +382,10 @@ def test_small_batch_4bit_kernel_shapes(cv, T, N, K, gs, tiled):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
-@pytest.mark.parametrize("T,N,K,pair", [(32, 12304, 512, False), (9, 12288, 256, False), (64, 12320, 768, False), (48, 12288, 512, False),
-                                        (32, 12304, 512, True), (5, 12288, 256, True), (20, 12320, 768, True)])
+@pytest.mark.parametrize("T,N,K,pair", [(16, 12304, 512, False), (9, 12288, 256, False), (13, 12320, 768, False), (6, 12288, 512, False),
+                                        (16, 12304, 512, True), (5, 12288, 256, True), (11, 12320, 768, True)])
 def test_wide_16bit_kernel_many_row_tiles(cv, dt, T, N, K, pair):
-    """5..64 tokens against >= 768 row tiles (gate/up, lm_head shapes): the LDS-shared-activation kernel (one row tile or gate/up
+    """5..16 tokens against >= 768 row tiles (gate/up, lm_head shapes): the LDS-shared-activation kernel (one row tile or gate/up
     pair per wave, 2-slot weight ring; a tile count that is not a multiple of 4 leaves surplus waves), against the oracle -- and
     the K-split kernel on the same inputs (tuning key 37) to the same bound"""
     from candle_vllm_amd import lib
@@ -396,8 +400,10 @@ def test_wide_16bit_kernel_many_row_tiles(cv, dt, T, N, K, pair):
         ref, mag, ulps = G.linear16(x, w, None, dt), None, 1.01
     lin = cv.Linear(dev16(w, dt))
     kw = {"epilogue": cv.EPI_SILU_MUL} if pair else {}
+    lib.mi355_internal_last_gemm()
     y = host16(lin.forward(dev16(x, dt), **kw), dt)
     check_ulp(y, ref, dt, ulps=ulps, what="wide 16-bit kernel", mag=mag)
+    assert lib.mi355_internal_last_gemm() == -1                   # not the prompt GEMM
     from candle_vllm_amd import tuning
     with tuning(30, 8):                                           # key 30 bit 3: the LDS-shared-activation kernel off
         y0 = host16(lin.forward(dev16(x, dt), **kw), dt)
@@ -423,8 +429,8 @@ def test_dense_tile_repack_bit_exact(cv):
                                         (32, 12304, 512, False), (20, 12320, 256, True), (3, 96, 512, True),
                                         (130, 208, 512, False), (257, 336, 1024, True), (97, 144, 256, False)])
 def test_linear_over_the_tiled_weight_image(cv, dt, T, N, K, pair):
-    """mi355_linear_tiled through all three 16-bit kernels (K-split streaming kernel, LDS-shared-activation kernel at >= 768 row tiles,
-    128 x 128 MFMA GEMM from 96 tokens) == the oracle == the row-major result to the same bound"""
+    """mi355_linear_tiled through the 16-bit kernels (K-split streaming kernel; MFMA GEMM from 33 tokens, at >= 768 row tiles from 17) == the oracle ==
+    the row-major result to the same bound"""
     rng = np.random.default_rng(T * 7 + N + K)
     x = G.round_dt(rng.normal(0, 1, (T, K)), dt)
     if pair:
@@ -445,7 +451,7 @@ def test_linear_over_the_tiled_weight_image(cv, dt, T, N, K, pair):
                                            (200, 48, 512, -1, "sym"), (128, 80, 768, 128, "zp"), (161, 144, 512, 128, "silu"),
                                            (97, 32, 256, 128, "resid")])
 def test_gptq_prompt_gemm_one_pass(cv, dt, T, N, K, gs, mode):
-    """>= 96 tokens over the tiled 4-bit image: the one-pass MFMA GEMM (weights unpacked in registers, per-group scale / offset with
+    """>= 96 tokens over the tiled 4-bit image: the one-pass MFMA GEMM (weights unpacked from LDS, per-group scale / offset with
     the prep launch's group sums of x; ragged token and column tiles, groups of 64 / 128 / 256 / whole K, zero points, the fused
     epilogues) == the oracle == the decode kernel in 64-token chunks (tuning key 39) to the same bound"""
     from candle_vllm_amd import tuning
@@ -476,10 +482,10 @@ def test_gptq_prompt_gemm_one_pass(cv, dt, T, N, K, gs, mode):
     check_ulp(y0, ref, dt, ulps=ulps, what="decode kernel in chunks", mag=mag)
 
 
-@pytest.mark.parametrize("T,N,K,gs,mode", [(33, 272, 4352, 128, "resid"), (65, 48, 2048, 64, "zp"),   # 64-token tiles, K in ranges; one token into the next
-                                           (65, 160, 768, 256, "silu"), (300, 4176, 256, 128, "zp"),   # ... pairs; 128 x 128
-                                           (900, 8192, 256, 128, "store"), (1100, 8224, 512, 512, "silu")])   # 128 x 256: exactly one per CU; ragged
-def test_gptq_prompt_gemm_every_tile(cv, T, N, K, gs, mode):
+@pytest.mark.parametrize("T,N,K,gs,mode,launch", [(33, 272, 4352, 128, "resid", 207), (65, 48, 2048, 64, "zp", 204),   # 64-token tiles, K in 7 and 4 ranges
+                                                  (65, 160, 768, 256, "silu", 201), (300, 4176, 256, 128, "zp", 201),   # ... in one; pairs; one token into the next
+                                                  (900, 8192, 256, 128, "store", 1), (1100, 8224, 512, 512, "silu", 101)])   # 128 x 256: exactly one per CU; 128 x 128, ragged
+def test_gptq_prompt_gemm_every_tile(cv, T, N, K, gs, mode, launch):
     """the one-pass 4-bit prompt GEMM where its dispatch takes each of its tiles and K ranges, tokens at the tiles' edges, at the oracle's bound"""
     dt = "bf16"
     rng = np.random.default_rng(T + N + K)
@@ -497,6 +503,8 @@ def test_gptq_prompt_gemm_every_tile(cv, T, N, K, gs, mode):
         got, ref, ulps, mag = lin.forward(dev16(x, dt), epilogue=cv.EPI_RESID, residual=dev16(res, dt)), G.round_dt(y + res[rows], dt), 2.01, y
     else:
         got, ref, ulps, mag = lin.forward(dev16(x, dt)), y, 1.01, None
+    from candle_vllm_amd import lib
+    assert lib.mi355_internal_last_gemm() == launch               # 100 tile + K ranges
     got = host16(got, dt)
     assert np.isfinite(got).all()
     check_ulp(got[rows], ref, dt, ulps=ulps, what="gptq prompt GEMM", mag=mag)
@@ -531,7 +539,7 @@ def test_gptq_prompt_gemm_in_slabs(cv):
                                            (48, 512, 4864, 256, "bias"), (17, 2 * 4736, 1792, 128, "silu"), (32, 2 * 608, 3584, 128, "silu"),
                                            (5, 64, 18944, 128, "resid"), (33, 4096, 256, 128, "store")])
 def test_gptq_wide_kernel_5_to_48_tokens(cv, dt, T, N, K, gs, mode):
-    """round 5 (csrc/gptq_wide.inc): 5..48 tokens over the tiled 4-bit image with the activations shared through LDS -- many-tile launches
+    """csrc/gptq_wide.inc: 5..48 tokens over the tiled 4-bit image with the activations shared through LDS -- many-tile launches
     in one sweep (gate/up as pairs per wave, SiLU * up from the accumulators), few-tile launches split over K with the partial sums added
     by the epilogue launch (Qwen2-7B's wo / down shapes: 14 and 74 k-blocks), a single k-block, ragged last workgroups.  Against the oracle
     at the bound of the 16-token-tile kernel it replaces, and against that kernel itself (tuning key 30 bit 128)."""
@@ -556,18 +564,22 @@ def test_gptq_wide_kernel_5_to_48_tokens(cv, dt, T, N, K, gs, mode):
         if mode == "bias":
             ulps = 2.01
     magkw = {"mag": full} if mode == "resid" else ({"mag": G.gptq_linear(x, G.gptq_dequant(q, s, None, gs), None, dt)} if mode == "bias" else {})
-    y = host16(lin.forward(dev16(x, dt), **kw), dt)
+    from candle_vllm_amd import lib
+    lib.mi355_internal_last_gemm()
+    with tuning(30, 16):                                           # key 30 bit 16: the prompt GEMM off, which takes 33 tokens and more
+        y = host16(lin.forward(dev16(x, dt), **kw), dt)
     check_ulp(y, ref, dt, ulps=ulps, what="gptq wide kernel", **magkw)
-    with tuning(30, 128):                                          # key 30 bit 128: the wide kernel off
+    with tuning(30, 16 | 128):                                     # bit 128: the wide kernel off
         y0 = host16(lin.forward(dev16(x, dt), **kw), dt)
+    assert lib.mi355_internal_last_gemm() == -1
     check_ulp(y0, ref, dt, ulps=ulps, what="16-token-tile kernel", **magkw)
     assert np.abs(y - y0).max() <= 3 * (2.0 ** -8 if dt == "bf16" else 2.0 ** -11) * max(1.0, np.abs(ref).max())
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
-@pytest.mark.parametrize("T,N,K,tiled", [(32, 256, 8192, True), (20, 336, 14336, True), (48, 64, 8448, False), (9, 4096, 8192, True)])
+@pytest.mark.parametrize("T,N,K,tiled", [(32, 256, 8192, True), (20, 336, 14336, True), (31, 64, 8448, False), (9, 4096, 8192, True)])
 def test_wide_16bit_kernel_few_tiles_long_k_split(cv, dt, T, N, K, tiled):
-    """round 5: few-tile 16-bit launches with a long K (down_proj of a batch-32 step: 256 tiles x 56 k-blocks at Llama-3-8B) take the
+    """5..32 tokens: few-tile 16-bit launches with a long K (down_proj of a batch-32 step: 256 tiles x 56 k-blocks at Llama-3-8B) take the
     LDS-shared-activation sweep split over K across workgroups; the partial sums meet in the epilogue launch (split order), which applies
     bias / residual and the rounding chain.  Against the oracle at the bound of the kernel it replaces, bias + residual included."""
     rng = np.random.default_rng(T + N + K)
@@ -579,8 +591,11 @@ def test_wide_16bit_kernel_few_tiles_long_k_split(cv, dt, T, N, K, tiled):
     y = host16(lin.forward(dev16(x, dt), epilogue=cv.EPI_RESID, residual=dev16(res, dt)), dt)
     full = G.linear16(x, w, b, dt)
     check_ulp(y, G.round_dt(full + res, dt), dt, what="split-K wide kernel + bias + residual", ulps=3.01, mag=np.maximum(np.abs(full), np.abs(G.linear16(x, w, None, dt))))
+    from candle_vllm_amd import lib
+    lib.mi355_internal_last_gemm()
     y2 = host16(cv.Linear(dev16(w, dt), tiled=tiled).forward(dev16(x, dt)), dt)
     check_ulp(y2, G.linear16(x, w, None, dt), dt, what="split-K wide kernel")
+    assert lib.mi355_internal_last_gemm() == -1                   # not the prompt GEMM
 
 
 @pytest.mark.parametrize("kind,T,N,K", [("16-bit", 96, 96, 8192), ("16-bit", 9, 256, 8192), ("4-bit", 100, 64, 8192), ("4-bit", 33, 64, 8192)])
