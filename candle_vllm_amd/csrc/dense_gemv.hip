@@ -933,6 +933,12 @@ static int dense_small3_launch(const DenseArgs (&a)[3], const DenseRope* rp, hip
     }
 }
 
+// waves per workgroup of dense_kernel: K split so that tiles * waves covers the chip several times, capped by the k-blocks
+static int dense_waves(int tiles, int nkb, int mt) {
+    int nw = 8;
+    while (nw > 1 && (nw > nkb || (size_t)tiles * nw > 256 * 32)) nw >>= 1;
+    return mt >= 3 && nw > 4 ? 4 : nw;
+}
 #include "gptq_wide.inc"   // 5..64 tokens x tiled 4-bit weights: LDS-shared activations, split-K for few-tile launches
 template <int DT, int WTYPE>
 static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
@@ -1002,12 +1008,7 @@ static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
         else if (a.group_size == 32) gj = 1;
         else return -2;
     }
-    // waves per workgroup: split K so that tiles * waves covers the chip several times, capped by the k-blocks
-    const int tiles = (pair ? a.pair_offset : a.N) / 16;
-    const int nkb = a.K >> 8;
-    int nw = 8;
-    while (nw > 1 && (nw > nkb || (size_t)tiles * nw > 256 * 32)) nw >>= 1;
-    if (mt >= 3 && nw > 4) nw = 4;
+    const int nw = dense_waves((pair ? a.pair_offset : a.N) / 16, a.K >> 8, mt);
 #define DG_CASE(MT_, R_) return dense_launch_gj<DT, WTYPE, MT_, R_>(a, gj, nw, st)
     if (pair) {
         switch (mt) { case 1: DG_CASE(1, 2); case 2: DG_CASE(2, 2); default: return -3; }
@@ -1041,9 +1042,7 @@ static int dense3_launch_dt(const DenseArgs (&a)[3], const DenseRope* rp, hipStr
     }
     const int t0 = a[0].N / 16, t1 = a[1].N / 16, t2 = a[2].N / 16, tiles = t0 + t1 + t2;
     const int nkb = a[0].K >> 8;
-    int nw = 8;
-    while (nw > 1 && (nw > nkb || (size_t)tiles * nw > 256 * 32)) nw >>= 1;
-    if (mt >= 3 && nw > 4) nw = 4;
+    const int nw = dense_waves(tiles, nkb, mt);
     if (rp) {
         DenseArgs b[3] = {a[0], a[1], a[2]};
         b[0].rope_mode = 1; b[1].rope_mode = 2; b[2].rope_mode = 3;
@@ -1300,6 +1299,35 @@ static DenseArgs dense_rows(const DenseArgs& a, int t0, int n) {
     if (a.resid) c.resid = static_cast<const uint16_t*>(a.resid) + (size_t)t0 * a.ldo;
     return c;
 }
+// us that the streaming kernels take for one matrix and 33 .. 64 tokens, from what their time follows: the k-blocks in a row of the slowest wave.
+//   * gptq_wide_kernel, K in one range: 4.3 + 1.29 a block (512 .. 12288 rows x 1024 9.4 .. 9.8, 16384 x 8192 45.7; more waves per CU are slower by 6 % each);
+//     K in ranges (and an epilogue launch that adds them): the rounds of two workgroups per CU, the last range's share of a second round
+//     counted as far as its workgroups are a quarter of the CUs (4096 x 14336: 7 blocks 22.3, 4608: 14 31.8; 4608 x 11008: 6 + 1 22.9);
+//   * dense_kernel: its waves' share of K, once per round of the row tiles over the CUs (4096 rows x 2048 33 tokens 9.3, 48 10.3, 64 12.1; 8192 x 2048 13.1,
+//     15.7, 18.6).
+// With gptq_gemm_us it picks the faster side, or one within 5 %, at 748 of 759 measured sizes (512 .. 32000 rows, k of 256 .. 18944, groups, zero points, epilogues)
+static float gptq_stream_us(const DenseArgs& a) {
+    const int cus = mi355_num_cus(), tiles = a.N / 16, nkb = a.K >> 8, mt = (a.T + 15) / 16;
+    if (gptq_wide_takes(a)) {
+        const GptqWideSplit w = gptq_wide_split(tiles, nkb, cus);
+        if (w.ks == 1) return 4.3f + (float)nkb * (1.29f + 0.08f * (float)(w.nw - 4)) * (float)((w.gx + cus - 1) / cus);
+        const int wgs = w.gx * w.ks, over = wgs - 2 * cus;
+        const float sweep = (float)w.kps + (over > 0 ? (float)(nkb - w.kps * (w.ks - 1)) * std::min(1.f, 4.f * (float)over / (float)cus) : 0.f);
+        const float one = 5.f + 0.3f * (float)w.ks + 1.3f * sweep, two = 12.f + 1.55f * sweep;      // one workgroup per CU, two
+        return one + (two - one) * std::min(1.f, std::max(0.f, 2.f * (float)(wgs - cus) / (float)cus));
+    }
+    const int nw = dense_waves(tiles, nkb, mt), blocks = (nkb + nw - 1) / nw, rounds = (tiles + cus - 1) / cus;
+    const float t1 = mt <= 3 ? 2.93f + 0.018f * (float)(a.T - 33) : 3.95f + 0.02f * (float)(a.T - 49);    // a block, one tile per CU
+    const float t2 = mt <= 3 ? 2.53f + 0.036f * (float)(a.T - 33) : 3.6f;                                  // a block and a tile of several
+    const bool small = a.group_size < 128, zp = a.qzeros && a.zmode != MI355_ZERO_SYM8;                     // more scales, zero points to unpack
+    const float f = (small ? 1.05f : 1.f) * (!zp ? 1.f : small ? 1.25f : 1.1f);
+    return 3.3f + f * (float)blocks * (rounds == 1 ? t1 : t2 * (float)rounds) + (a.epi == MI355_EPI_RESID ? (mt <= 3 ? 1.f : 1.7f) : 0.f);
+}
+// the GEMM's, from its choice: beside the rounds there are the launch in front, the partial sums and their launch, and a start on cold weights
+static float gptq_gemm_us(const GtChoice& c, int T, float weights_us) {
+    const float cold = std::min(1.7f, weights_us);
+    return c.splits == 1 ? 0.88f * c.us + 3.5f + cold : c.us + 0.2f * (float)(c.splits - 1) + 1.9f * cold + 0.03f * (float)(T - 33);
+}
 // n matrices over the same x, of one group size and zero mode; at most gptq_gemm_slab(K) tokens
 static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) {
     const DenseArgs& a = ms[0];
@@ -1325,8 +1353,13 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     // at 700 tokens 695 / 236, at 2048 2030 / 560; down 3584 x 18944 at 700 470 / 118 (three ranges), at 64 (chunks of the decode kernel) 78 / 30
     // (64-token tiles, eight ranges), at 96 102 / 36.
     const int units = a.K / GG_UNIT;
-    const GtChoice best = gt_pick(tiles, units, (float)rows * (float)a.K / 2.f / 5.0e6f, n == 1 && a.T <= 65535 ? gemm_max_split(a, std::max(1, units / 4)) : 1,
+    const float weights_us = (float)rows * (float)a.K / 2.f / 5.0e6f;
+    const GtChoice best = gt_pick(tiles, units, weights_us, n == 1 && a.T <= 65535 ? gemm_max_split(a, std::max(1, units / 4)) : 1,
                                   (float)a.T * (float)a.N * 4.f / 4.5e6f, gs % GG_UNIT ? 6 : 7, kGgTiles, 3);
+    // To 64 tokens one matrix is also one sweep of the streaming kernels.  us, streaming / this (33 tokens unless given): 4096 x 512 7.0 / 8.9, x 1024 9.6 / 11.8,
+    // x 2048 9.3 / 12.8, x 4096 15.5 / 15.8, x 5120 18.4 / 17.7, x 14336 22.3 / 24.7; 2048 x 14336 18.7 / 19.2, 1024 x 14336 48 tokens 15.7 / 21.6; 4608 x 14336 31.8 / 25.9;
+    // 16384 x 2048 15.1 / 18.9, x 8192 45.7 / 37.9; 28672 x 8192 51 / 58; 64 tokens 4096 x 1024 8.0 / 12.2, 2048 x 3072 16.3 / 12.5
+    if (n == 1 && a.T <= 64 && !silu && gptq_stream_us(a) <= gptq_gemm_us(best, a.T, weights_us)) return (int)hipErrorNotSupported;
     const GtTile& t = kGgTiles[best.tile];
     for (int i = 0; i < 3; ++i) g.a[i] = ms[i < n ? i : 0];
     g.n_m = (a.T + t.bm - 1) / t.bm; g.t_pad = (a.T + 255) / 256 * 256 + 256;   // (a DMA of the sums reads 256 tokens from the tile's first)
@@ -1407,7 +1440,7 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     const int max_split = n == 1 && a[0].T <= 65535 && !(a[0].N & 3) && !(a[0].epi == MI355_EPI_SILU_MUL && (a[0].pair_offset & 3)) ? gemm_max_split(a[0], std::max(1, units / 8)) : 1;
     GtChoice best = gt_pick([&](const GtTile& t) { return tiles(t, nullptr); }, units, (float)rows * (float)a[0].K * 2.f / 5.4e6f, max_split,
                             (float)a[0].T * (float)a[0].N * 4.f / 4.5e6f, 31);
-    if (g_tune_gemm_tall) best = {0, 1};
+    if (g_tune_gemm_tall) best = {0, 1, 0.f};
     DenseGemm3 g{};
     for (int i = 0; i < 3; ++i) g.a[i] = a[i < n ? i : 0];
     g.n_m = (a[0].T + kGtTiles[best.tile].bm - 1) / kGtTiles[best.tile].bm;

@@ -180,22 +180,21 @@ static constexpr GtTile kGtTiles[] = {{256, 256, 1, 1.46f}, {192, 256, 1, 1.28f}
 #define GT_TILES(which, CALL) do { switch (which) { \
     case 0: CALL(2, 4, 8, 4, 2); break; case 1: CALL(2, 4, 6, 4, 2); break; case 2: CALL(2, 4, 4, 2, 2); break; \
     case 3: CALL(2, 4, 4, 2, 4); break; default: CALL(2, 4, 2, 2, 6); break; } } while (0)
-struct GtChoice { int tile, splits; };
+struct GtChoice { int tile, splits; float us; };
 // tile and K ranges of this thread's last launch, 100 tile + ranges (tests: mi355_internal_last_gemm)
 inline thread_local int gt_last_launch = -1;
 // tiles(t): workgroups of the launch with tile t; stream_us: the weights' read; part_us: write or read of one range's partial sums
 template <class F>
 static inline GtChoice gt_pick(F tiles, int units, float stream_us, int max_split, float part_us, unsigned allowed, const GtTile* table = kGtTiles, int n_table = 5) {
     const int cus = mi355_num_cus();
-    GtChoice best{-1, 1};
-    float cost = 0.f;
+    GtChoice best{-1, 1, 0.f};
     for (int i = 0; i < n_table; ++i)
         for (int s = 1; s <= max_split; ++s) {
             if (!(allowed >> i & 1)) continue;
             const int64_t wgs = (int64_t)cus * table[i].per_cu, rounds = (tiles(table[i]) * s + wgs - 1) / wgs;
             const float t = (float)rounds * (float)((units + s - 1) / s + 2) * table[i].us;
             const float c = (t > stream_us ? t : stream_us) + (s > 1 ? 5.f + part_us * (float)(s + 1) : 0.f);
-            if (best.tile < 0 || c < cost) { best = {i, s}; cost = c; }
+            if (best.tile < 0 || c < best.us) best = {i, s, c};
         }
     return best;
 }

@@ -510,6 +510,27 @@ def test_gptq_prompt_gemm_every_tile(cv, T, N, K, gs, mode, launch):
     check_ulp(got[rows], ref, dt, ulps=ulps, what="gptq prompt GEMM", mag=mag)
 
 
+@pytest.mark.parametrize("T,N,K,gs,zp,gemm", [(33, 512, 256, 128, False, False), (64, 1024, 1024, 128, False, False), (48, 4096, 2048, 128, False, False),
+                                              (33, 2048, 2048, 64, True, False), (64, 4096, 1536, 128, True, False), (40, 12304, 512, 128, False, False),
+                                              (48, 512, 8192, 128, False, False), (33, 2560, 8192, 256, False, False),      # K in ranges, one and two workgroups per CU
+                                              (33, 2048, 4096, 128, False, True), (64, 2048, 3072, 128, False, True), (48, 4608, 2048, 128, False, True),
+                                              (33, 512, 8192, 64, False, True)])
+def test_gptq_33_to_64_tokens_take_the_faster_kernel(cv, T, N, K, gs, zp, gemm):
+    """4-bit products of 33 to 64 tokens: the streaming kernels where they are faster than the prompt GEMM with its launch in front, both at the op's bound"""
+    from candle_vllm_amd import lib
+    dt = "bf16"
+    rng = np.random.default_rng(T + N + K)
+    q, s = _gptq_case(rng, K, N, gs, dt)
+    x = G.round_dt(rng.normal(0, 1, (T, K)), dt)
+    z = rng.integers(1, 17, (K // gs, N)) if zp else None
+    kw = {"qzeros": dev_u32(G.gptq_pack_zeros(z)), "zero_mode": cv.ZERO_GPTQ_PLUS1} if zp else {}
+    lin = cv.GPTQLinear(dev_u32(G.gptq_pack(q)), dev16(s, dt), gs, **kw)
+    lib.mi355_internal_last_gemm()
+    y = host16(lin.forward(dev16(x, dt)), dt)
+    assert (lib.mi355_internal_last_gemm() >= 0) == gemm
+    check_ulp(y, G.gptq_linear(x, G.gptq_dequant(q, s, z, gs), None, dt), dt, ulps=1.01, what="gptq linear")
+
+
 def test_gptq_prompt_gemm_in_slabs(cv):
     """more tokens than the permuted copy of x has room for (128 MiB: 3 328 of 18 944): slabs of tokens, rows at their borders against the product in 64
     bits, residual in place; and the memory taken"""
