@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(512) dense3r_kernel(const DenseArgs a0, const 
     else dense_body<DT, WTYPE, MT, 1, GJ>(a2, bx - t0 - t1, &rp);
 }
 
-// ------------------------------------------------------------------------------------------------ 5..16 tokens x 16-bit weights, many row tiles; 5..32, long K
+// ------------------------------------------------------------------------------------------------ 5..32 tokens x 16-bit weights, many row tiles (pairs: 5..16); 5..48, long K
 // dense_body gives a workgroup ONE row tile (or gate/up pair) and lets its waves split K: every wave then fetches its own copy of
 // the activations of its k-blocks -- at 32 tokens 16 KB of x (from L2) for every 8 KB of weights, and all of a k-block's loads are
 // requested, waited for and consumed before the next k-block's go out (measured on BASELINE configs[2], Llama-3-8B bf16 at batch
@@ -810,6 +810,7 @@ static int dense_launch_gj(const DenseArgs& a, int gj, int nw, hipStream_t st) {
 // T = 16 9.3 / 13.7, 32 12.3 / 14.0, 40 16.1 / 13.7; 12288 x 2048 T = 32 17.0 / 12.9; at 5 .. 16 tokens either may win (16384 pairs of 3072: 18.7 / 22.1)
 // 4-bit, against token chunks of the decode kernels: down 3584 x 18944 T = 32 21.6 / 27.4, 33 29.1 / 28.1, 49 72.7 / 29.1; 4608 x 3584 T = 33 20.8 / 16.0;
 // wo 3584 x 3584 33 14.8 / 15.0, 64 19.2 / 16.5; gate/up 37888 x 3584 48 42.1 / 54.5, 64 48.3 / 58.3, 65 64.3 / 58.8
+// (to 64 tokens the sizes decide: dense_streams, gptq_prompt_gemm)
 enum { DENSE_GEMM_MIN_T = 33, DENSE_GEMM_ANY_T = 96, GPTQ_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_PAIR_T = 65 };
 static int g_tune_gemm_min_t = DENSE_GEMM_MIN_T;
 static int g_tune_gptq_gemm_off = 0;   // tuning key 39: 1 = 4-bit prompt steps run the decode kernel in 64-token chunks (A/B)
@@ -961,10 +962,10 @@ static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
         // k-blocks plus the epilogue launch is not faster than its one launch)
         const int wtiles = (pair ? a.pair_offset : a.N) / 16;
         const int nkb_w = a.K >> 8;
-        const bool many = wtiles >= 4 * 192 && mt == 1, longk = !pair && nkb_w >= 32 && mt <= 2;   // (more tokens: the prompt GEMM, dense_run)
+        const bool many = wtiles >= 4 * 192 && (mt == 1 || (mt == 2 && !pair)), longk = !pair && nkb_w >= 32 && mt <= 3;   // (more tokens: the prompt GEMM, dense_run)
         if (!g_tune_wide_off && a.T > 4 && (many || longk) && !((uintptr_t)a.x & 15) && !(a.ldx & 7) &&
             !((uintptr_t)a.w & 15) && (a.wtiled || !(a.ldw & 7))) {
-            const int nwv = many ? (g_tune_wide_nw == 2 ? 2 : 4) : 4;
+            const int nwv = many && g_tune_wide_nw == 2 ? 2 : 4;
             const int gx = (wtiles + nwv - 1) / nwv;
             int ks = 1;
             if (!many) {
@@ -988,7 +989,7 @@ static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
                     if (!attr) { (void)hipFuncSetAttribute((const void*)dense_wide_kernel<DT, MT_, R_, NW_>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024); attr = true; } \
                     hipLaunchKernelGGL((dense_wide_kernel<DT, MT_, R_, NW_>), grid, block, lds, st, a, part, ldp, kps); } while (0)
 #define DWD_GO(MT_, R_) do { if (nwv == 2) DWD_GO2(MT_, R_, 2); else DWD_GO2(MT_, R_, 4); } while (0)
-                if (pair) DWD_GO(1, 2); else if (mt == 1) DWD_GO(1, 1); else DWD_GO(2, 1);
+                if (pair) DWD_GO(1, 2); else if (mt == 1) DWD_GO(1, 1); else if (mt == 2) DWD_GO(2, 1); else DWD_GO2(3, 1, 4);
 #undef DWD_GO2
 #undef DWD_GO
                 if (hipGetLastError() != hipSuccess) return -1;
@@ -1480,11 +1481,30 @@ static int dense_prompt_gemm_staged(const DenseArgs& a, int dt, hipStream_t st) 
     return e != hipSuccess ? (int)e : dense_prompt_gemm(&c, 1, dt, st);
 }
 
+// 16-bit products that the streaming kernels make sooner than the GEMM, of those it would take below 65 tokens (33 .. 64; 17 .. 32 against 768 row tiles).  With
+// one row tile per CU they take a wave's share of K, the GEMM at least one unit per 64 k in one workgroup or the partial sums' launch.  us, streaming / GEMM:
+// 33 tokens 4096 x 1024 6.6 / 9.6, x 2048 9.4 / 12.2, x 3072 11.7 / 13.9, x 5120 16.7 / 16.1; 2048 x 512 4.8 / 6.0, x 2048 8.8 / 9.9, x 3072 11.1 / 10.7; 48 tokens 4096 x 3072
+// 13.4 / 14.5, 2048 x 2048 9.9 / 10.2; 64 tokens 4096 x 2048 12.8 / 13.4, x 3072 16.6 / 15.1, 1024 x 1024 7.6 / 7.9, x 1536 9.9 / 9.5; two tiles per CU, 33 tokens 8192 x 1024
+// 9.2 / 10.1, x 2048 14.9 / 13.4, 49 x 1024 11.4 / 10.6; a long K in ranges (LDS-shared activations) 33 tokens 1024 x 8192 13.8 / 14.7, 48 14.0 / 15.8, 64 x 8192
+// 12.4 / 11.1, 2048 x 14336 22.1 / 20.2, row-major 1024 x 11008 18.6 / 16.2; 32 tokens 12288 x 512 7.3 / 8.1, x 1536 13.3 / 14.2, x 2048 17.6 / 17.5.  At k = 256 the GEMM (4096: 5.1 / 4.9, 64 tokens
+// 6.7 / 5.3).  Row-major weights cost the streaming kernels 0.5 .. 2: 33 tokens 4096 x 2048 11.4 / 12.4, 49 13.4 / 13.4, 2048 x 1024 6.4 / 7.8, 64 8.4 / 8.3
+static bool dense_streams(const DenseArgs& a) {
+    if (a.T > 64 || a.epi == MI355_EPI_SILU_MUL || (a.N & 15) || (a.K & 255) || a.K < 512) return false;
+    const int cus = mi355_num_cus(), tiles = a.N / 16;
+    if (a.T > 32 && a.T <= 48 && a.wtiled && tiles >= 32 && tiles * 4 <= cus && a.K >= 8192) return true;
+    const int T = a.epi == MI355_EPI_RESID ? a.T + 8 : a.T;              // (a residual adds 1 to the streaming kernels, nothing to the GEMM)
+    int most;
+    if (a.T <= 32) most = 1536;
+    else if (tiles > cus) most = tiles <= 2 * cus && T <= 40 ? 1536 : 0;
+    else if (tiles > cus / 2) most = T <= 48 ? (a.wtiled ? 3072 : 2048) : T > 64 ? 1536 : a.wtiled ? 2048 : 1024;
+    else most = T <= 48 && a.wtiled ? 2048 : T > 64 ? 0 : 1024;
+    return a.K <= most;
+}
 // SILU_MUL with more than 32 tokens, or any T > 64: run in token chunks
 static int dense_run(DenseArgs a, int wtype, int dt, hipStream_t st) {
     // (rows and k that are not whole tiles of the streaming kernels are served from DENSE_GEMM_ANY_T tokens, and refused below)
     const bool whole = !(a.N & 15) && !(a.K & 255);
-    if (wtype == DW_DENSE && (a.T >= DENSE_GEMM_ANY_T || whole) &&
+    if (wtype == DW_DENSE && (a.T >= DENSE_GEMM_ANY_T || whole) && !(g_tune_gemm_min_t == DENSE_GEMM_MIN_T && !g_tune_gemm_tall && dense_streams(a)) &&
         (a.T >= g_tune_gemm_min_t || (g_tune_gemm_min_t == DENSE_GEMM_MIN_T && a.T > 16 && (a.epi == MI355_EPI_SILU_MUL ? a.pair_offset : a.N) >= 16 * 768))) {
         int rc = dense_prompt_gemm(&a, 1, dt, st);
         if (rc == (int)hipErrorNotSupported && a.T >= DENSE_GEMM_ANY_T) rc = dense_prompt_gemm_staged(a, dt, st);

@@ -13,7 +13,7 @@ enum {
     MI355_SCR_QMP_WS = 7,        // prompt-step GEMM: quantised activation image
     MI355_SCR_DENSE_WS = 8,      // 16-bit prompt GEMM: copies of operands that do not start on 16 bytes
     MI355_SCR_COMM = 9,          // one-shot all-reduce staging
-    MI355_SCR_GPTQ_WIDE = 10,    // split-K partial sums: 5..48-token launches of tiled 4-bit weights, 5..32-token and prompt launches of 16-bit weights
+    MI355_SCR_GPTQ_WIDE = 10,    // split-K partial sums: 5..48-token launches of tiled 4-bit and of 16-bit weights, prompt launches of 16-bit weights
     MI355_SCR_PF_FP8 = 11,       // prompt attention over an e4m3 cache: the sequences' blocks as bf16 + their block table (prefill_attention.hip)
     MI355_SCR_GPTQ_GEMM = 13,    // 4-bit prompt GEMM: permuted x, its sums, scale panel, split-K partial sums (gptq_gemm.inc)
     MI355_SCR_DELTA = 12,        // delta rule by pieces: the pieces' records (hybrid_delta.hip)

@@ -52,7 +52,7 @@ def check_ulp(got, ref, dt, ulps=1.01, what="", mag=None):
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("T,N,K", [(1, 256, 512), (5, 48, 256), (16, 1024, 1024), (17, 64, 768), (33, 128, 512),
                                    (64, 96, 256), (70, 32, 512), (128, 64, 512), (200, 48, 256),
-                                   (256, 384, 1024), (300, 200, 576), (97, 130, 64)])   # >= 33 tokens: the MFMA GEMM (ragged T / N tiles, one K step)
+                                   (256, 384, 1024), (300, 200, 576), (97, 130, 64)])   # (64, 96, 256) and more tokens: the MFMA GEMM (ragged T / N tiles, one K step)
 def test_linear_matches_oracle(cv, dt, T, N, K):
     rng = np.random.default_rng(T * 1000 + N)
     x = G.round_dt(rng.normal(0, 1, (T, K)), dt)
@@ -508,6 +508,23 @@ def test_gptq_prompt_gemm_every_tile(cv, T, N, K, gs, mode, launch):
     got = host16(got, dt)
     assert np.isfinite(got).all()
     check_ulp(got[rows], ref, dt, ulps=ulps, what="gptq prompt GEMM", mag=mag)
+
+
+@pytest.mark.parametrize("T,N,K,gemm", [(33, 4096, 1024, False), (48, 2048, 2048, False), (64, 4096, 2048, False), (64, 1024, 1024, False), (40, 4112, 512, False),
+                                        (17, 12288, 512, False), (32, 12304, 1536, False), (33, 1024, 8192, False), (48, 528, 8448, False),  # K in ranges
+                                        (48, 48, 8448, True),
+                                        (49, 2048, 2048, True), (64, 4096, 3072, True), (41, 4112, 512, True), (33, 512, 256, True), (32, 12288, 2048, True)])
+def test_linear_17_to_64_tokens_take_the_faster_kernel(cv, T, N, K, gemm):
+    """16-bit products of 17 to 64 tokens: the streaming kernels to the sizes where the prompt GEMM becomes the faster one, both at the op's bound"""
+    from candle_vllm_amd import lib
+    dt = "bf16"
+    rng = np.random.default_rng(T + N + K)
+    x, w, b = G.round_dt(rng.normal(0, 1, (T, K)), dt), G.round_dt(rng.normal(0, 0.05, (N, K)), dt), G.round_dt(rng.normal(0, 0.2, N), dt)
+    lin = cv.Linear(dev16(w, dt), dev16(b, dt), tiled=True)
+    lib.mi355_internal_last_gemm()
+    y = host16(lin.forward(dev16(x, dt)), dt)
+    assert (lib.mi355_internal_last_gemm() >= 0) == gemm
+    check_ulp(y, G.linear16(x, w, b, dt), dt, what="linear+bias", ulps=2.01, mag=G.linear16(x, w, None, dt))
 
 
 @pytest.mark.parametrize("T,N,K,gs,zp,gemm", [(33, 512, 256, 128, False, False), (64, 1024, 1024, 128, False, False), (48, 4096, 2048, 128, False, False),
