@@ -1923,13 +1923,14 @@ int mi355_internal_linear3(void* const* outs, const void* x, const void* const* 
                            const void* const* biases, const int32_t* ns, int32_t num_tokens, int32_t k, int32_t group_size,
                            int32_t is_gptq, int32_t dtype, const void* norm_w, float norm_eps, const float* ss_in, const void* rope,
                            int64_t stream) {
-    // One GEMM launch for the three, or the streaming kernel over all their row tiles (to 64 tokens).  us, streaming / GEMM (q + k + v rows x k): 16-bit
-    // 2048 + 2 x 512 x 2048 33 tokens 9.9 / 11.0, 48 10.6 / 11.2, 52 11.6 / 11.3; the same x 4096 13.6 / 17.5, 16.0 / 17.8, 17.9 / 17.9; 2560 + 2 x 1024 x 2560 15.9 / 13.0;
-    // 4096 + 2 x 1024 x 4096 23.8 / 17.8.  4-bit (its GEMM has a launch in front) 2048 + 2 x 512 x 4096 64 tokens 20.6 / 29.9; 3584 + 2 x 512 x 3584 48 24.8 / 27.1,
-    // 52 29.0 / 27.2, groups of 64 29.3 / 30.8, 60 31.2 / 30.9; 5120 + 2 x 1024 x 5120 48 33.9 / 36.1, 52 39.5 / 36.3; 3 x 4096 x 4096 33 34.6 / 29.9
+    // One GEMM launch for the three (K in one range), or the streaming kernel over all their row tiles (to 64 tokens).  us, streaming / GEMM, weights from HBM
+    // (q + k + v rows x k): 16-bit 2048 + 2 x 512 x 2048 33 tokens 9.3 / 11.0, 49 11.4 / 16.0, 64 12.9 / 17.0; 3 x 2048 x 2048 33 14.5 / 16.0, 48 17.3 / 16.9; 4096 + 2 x 1024
+    // x 1024 33 9.3 / 10.1, 48 10.7 / 10.5, x 4096 33 24.1 / 27.9, 48 29.4 / 29.3, 49 31.5 / 29.3; 5120 + 2 x 1024 x 5120 40 32.5 / 36.8, 48 36.6 / 38.2, 56 42.3 / 39.3; 3 x 2048 x 512 33
+    // 6.5 / 6.3, 3 x 4096 x 4096 34.9 / 30.4, 8192 + 2 x 1024 x 8192 62.9 / 54.0.  4-bit (its GEMM has a launch in front) 2048 + 2 x 512 x 4096 64 tokens 20.6 / 29.9; 3584 + 2 x 512 x
+    // 3584 48 24.8 / 27.1, 52 29.0 / 27.2, groups of 64 29.3 / 30.8, 60 31.2 / 30.9; 4096 + 2 x 1024 x 1024 49 11.0 / 12.3, 64 12.3 / 12.6; 3 x 4096 x 4096 33 34.6 / 31.2
     const int64_t rows3 = ns ? (int64_t)ns[0] + ns[1] + ns[2] : 0;
-    const int gemm_t = is_gptq == 2 ? (rows3 < 4096 ? 65 : rows3 >= 10240 ? (int)GPTQ_GEMM_MIN_T : group_size > 0 && group_size < 128 ? 57 : 49)
-                                    : std::max(g_tune_gemm_min_t, rows3 < 4096 ? 49 : 0);
+    const int gemm_t = is_gptq == 2 ? (rows3 < 4096 ? 65 : rows3 >= 10240 ? (k <= 1024 ? 49 : (int)GPTQ_GEMM_MIN_T) : k <= 1024 ? 65 : group_size > 0 && group_size < 128 ? 57 : 49)
+                                    : std::max(g_tune_gemm_min_t, rows3 < 4096 ? 65 : rows3 < 10240 && k >= 1024 ? 48 : 0);
     const bool prompt = !norm_w && !rope && is_gptq != 1 && num_tokens >= gemm_t;
     if (num_tokens < 1 || (num_tokens > 64 && !prompt) || (k & 255)) return -4;
     const DenseRope* rp = static_cast<const DenseRope*>(rope);

@@ -548,6 +548,41 @@ def test_gptq_33_to_64_tokens_take_the_faster_kernel(cv, T, N, K, gs, zp, gemm):
     check_ulp(y, G.gptq_linear(x, G.gptq_dequant(q, s, z, gs), None, dt), dt, ulps=1.01, what="gptq linear")
 
 
+@pytest.mark.parametrize("T,ns,K,bits,gemm", [(64, (2048, 512, 512), 512, 16, False), (47, (2048, 2048, 2048), 1024, 16, False), (48, (2048, 2048, 2048), 1024, 16, True),
+                                              (33, (2048, 2048, 2048), 512, 16, True), (64, (2048, 2048, 2048), 512, 4, False), (49, (4096, 4096, 4096), 512, 4, True),
+                                              (48, (4096, 4096, 4096), 512, 4, False), (49, (2048, 2048, 2048), 1280, 4, True)])
+def test_three_products_take_the_faster_kernel(cv, T, ns, K, bits, gemm):
+    """q, k and v in one launch, 16-bit and 4-bit: streaming kernel or prompt GEMM by rows, k and tokens; within the op's bound of the products in 64 bits"""
+    import ctypes
+    from candle_vllm_amd import lib
+    gen, st = torch.Generator(device="cuda").manual_seed(T + K), torch.cuda.current_stream().cuda_stream
+    x, out, ws, ss, refs = torch.randn(T, K, generator=gen, device="cuda").to(torch.bfloat16), [], [], [], []
+    for n in ns:
+        out.append(torch.full((T, n), float("nan"), device="cuda", dtype=torch.bfloat16))
+        if bits == 16:
+            w = (torch.randn(n, K, generator=gen, device="cuda") * 0.05).to(torch.bfloat16)
+            img = torch.empty_like(w)
+            assert lib.mi355_dense_tile_repack(w.data_ptr(), img.data_ptr(), n, K, K, st) == 0
+            wd = w.double().T
+        else:
+            q = torch.randint(0, 16, (K, n), generator=gen, device="cuda", dtype=torch.int32)
+            packed = sum((q.view(K // 8, 8, n)[:, i] << (4 * i)) for i in range(8)).contiguous()
+            img = torch.empty_like(packed)
+            assert lib.mi355_gptq_tile_repack(packed.data_ptr(), img.data_ptr(), K, n, 0, st) == 0
+            ss.append((torch.rand(K // 128, n, generator=gen, device="cuda") * 0.01 + 0.002).to(torch.bfloat16))
+            wd = ((q.double() - 8).view(K // 128, 128, n) * ss[-1].double()[:, None]).view(K, n)
+        ws.append(img)
+        refs.append(x.double() @ wd)
+    p3 = lambda ts: (ctypes.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    fn = lib.mi355_internal_linear3
+    fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_int32] * 5 + [ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64]
+    lib.mi355_internal_last_gemm()
+    assert fn(p3(out), x.data_ptr(), p3(ws), p3(ss) if ss else None, None, (ctypes.c_int32 * 3)(*ns), T, K, 128, 3 if bits == 16 else 2, 2, None, 0.0, None, None, st) == 0
+    assert (lib.mi355_internal_last_gemm() >= 0) == gemm
+    for o, r in zip(out, refs):
+        check_ulp(o.double().cpu().numpy(), r.to(torch.bfloat16).double().cpu().numpy(), "bf16", ulps=1.01, what="one of three", mag=r.abs().cpu().numpy())
+
+
 def test_gptq_prompt_gemm_in_slabs(cv):
     """more tokens than the permuted copy of x has room for (128 MiB: 3 328 of 18 944): slabs of tokens, rows at their borders against the product in 64
     bits, residual in place; and the memory taken"""
