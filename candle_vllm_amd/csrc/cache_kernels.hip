@@ -64,23 +64,28 @@ __global__ void __launch_bounds__(256) reshape_and_cache_paged_kernel(
 // that neighbouring lanes are neighbouring slots of a sequence -- K leaves in runs of 256 bytes, V in runs of 32 -- whatever the slots are:
 // each lane writes its own token's slot.  us per call, 8 heads of 128, blocks of 64, one token per workgroup / this: 3001 tokens in a row 21.4 / 8.3
 // (24.6 MB moved: 3.0 TB/s), 8192 52.4 / 19.9, 700 7.9 / 3.8; 3001 scattered slots 43.3 / 41.0.
+// Few tokens of few heads are a handful of such workgroups, and eight stores to V one behind the other are what the call waits for: there a lane copies 2
+// values (W) and four times the workgroups share them.  us, one token per workgroup / 8 values / 2 values: 64 scattered tokens (a decoding batch), 1 head of 128
+// 2.3 / 3.3 / 2.4, 4 heads 2.8 / 3.4 / 2.7, 8 heads 3.7 / 3.8 / 3.1; 256, 4 heads 4.0 / 4.5 / 3.9; in a row 2.2 .. 2.4 both ways there, and beyond a workgroup of 8 values
+// on every fourth CU 400, 8 heads 2.5 / 3.0, 1000, 4 heads 2.6 / 3.2
 #define RC_TOKENS 16
+template <int W>
 __global__ void __launch_bounds__(256) reshape_and_cache_paged16_kernel(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, uint16_t* __restrict__ kc,
                                                                         uint16_t* __restrict__ vc, const int64_t* __restrict__ slot_mapping, int num_tokens,
                                                                         int num_kv_heads, int head_dim, int block_size) {
-    const int t = blockIdx.x * RC_TOKENS + (threadIdx.x & 15), c = blockIdx.y * 16 + (threadIdx.x >> 4);      // c: 8 values of the row
+    struct alignas(2 * W) Piece { uint32_t w[W / 2]; };
+    const int t = blockIdx.x * RC_TOKENS + (threadIdx.x & 15), c = blockIdx.y * 16 + (threadIdx.x >> 4);      // c: W values of the row
     const int row = num_kv_heads * head_dim;
-    if (t >= num_tokens || c * 8 >= row) return;
+    if (t >= num_tokens || c * W >= row) return;
     const int64_t slot = slot_mapping[t];
     if (slot < 0) return;
-    const uint4 kq = *reinterpret_cast<const uint4*>(k + (int64_t)t * row + c * 8), vq = *reinterpret_cast<const uint4*>(v + (int64_t)t * row + c * 8);
+    const Piece kq = *reinterpret_cast<const Piece*>(k + (int64_t)t * row + c * W), vq = *reinterpret_cast<const Piece*>(v + (int64_t)t * row + c * W);
     const int64_t blk = slot / block_size, off = slot % block_size;
-    const int h = c * 8 / head_dim, d = c * 8 % head_dim;                   // head_dim % 8 == 0: one head
-    *reinterpret_cast<uint4*>(kc + (((blk * num_kv_heads + h) * (head_dim / 8) + d / 8) * block_size + off) * 8) = kq;
+    const int h = c * W / head_dim, d = c * W % head_dim;                   // head_dim % 8 == 0: one head
+    *reinterpret_cast<Piece*>(kc + (((blk * num_kv_heads + h) * (head_dim / 8) + d / 8) * block_size + off) * 8 + d % 8) = kq;
     uint16_t* const vp = vc + ((blk * num_kv_heads + h) * head_dim + d) * (int64_t)block_size + off;
-    const uint32_t w[4] = {vq.x, vq.y, vq.z, vq.w};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) vp[(int64_t)i * block_size] = (uint16_t)(w[i >> 1] >> (16 * (i & 1)));
+    for (int i = 0; i < W; ++i) vp[(int64_t)i * block_size] = (uint16_t)(vq.w[i >> 1] >> (16 * (i & 1)));
 }
 
 // fp8 KV cache (`--kvcache-dtype fp8`, src/main.rs:263-267; K layout x = 16, cache_engine.rs:304-311): bf16 k, v are
@@ -138,10 +143,15 @@ extern "C" int mi355_reshape_and_cache(const void* k, const void* v, void* key_c
 #undef LAUNCH
     } else if (layout == MI355_KV_PAGED) {
         if (head_dim % (16 / elem_size)) return (int)hipErrorInvalidValue;
-        // (from 64 tokens: 3.8 us both ways there, 4.2 / 3.7 at 128.  Fewer are decode batches: no neighbouring slots to gather.  16-byte loads and K stores)
+        // (from 64 tokens: in a row, 8 heads 3.4 / 2.2.  Fewer are decode batches: no neighbouring slots to gather.  16-byte loads and K stores)
         if (elem_size == 2 && num_tokens >= 4 * RC_TOKENS && row > 0 && (((uintptr_t)k | (uintptr_t)v | (uintptr_t)key_cache) & 15) == 0) {
-            hipLaunchKernelGGL(reshape_and_cache_paged16_kernel, dim3((num_tokens + RC_TOKENS - 1) / RC_TOKENS, (row / 8 + 15) / 16), dim3(256), 0, st, (const uint16_t*)k,
-                               (const uint16_t*)v, (uint16_t*)key_cache, (uint16_t*)value_cache, slot_mapping, num_tokens, num_kv_heads, head_dim, block_size);
+            const int groups = (num_tokens + RC_TOKENS - 1) / RC_TOKENS, per = (row / 8 + 15) / 16;
+#define LAUNCH16(W, PIECES)                                                                                            \
+    hipLaunchKernelGGL(reshape_and_cache_paged16_kernel<W>, dim3(groups, PIECES), dim3(256), 0, st, (const uint16_t*)k, \
+                       (const uint16_t*)v, (uint16_t*)key_cache, (uint16_t*)value_cache, slot_mapping, num_tokens, num_kv_heads, head_dim, block_size)
+            if ((int64_t)groups * per * 4 <= mi355_num_cus()) LAUNCH16(2, (row / 2 + 15) / 16);
+            else LAUNCH16(8, per);
+#undef LAUNCH16
             return (int)hipGetLastError();
         }
 #define LAUNCH(T)                                                                                      \

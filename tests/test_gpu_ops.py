@@ -106,6 +106,24 @@ def test_reshape_and_cache_prompt_rows_bit_exact(cv, lib, T, Hkv, D, bs, shift):
     assert np.array_equal(bf16_bits(kcd), kc) and np.array_equal(bf16_bits(vcd), vc)
 
 
+@pytest.mark.parametrize("T,Hkv,D,bs", [(64, 1, 8, 16), (64, 1, 128, 64), (65, 4, 128, 64), (128, 8, 128, 32), (129, 8, 128, 32), (1024, 1, 128, 16), (1025, 1, 128, 16),
+                                        (70, 3, 72, 7)])
+def test_reshape_and_cache_scattered_rows_bit_exact(cv, T, Hkv, D, bs):
+    """tokens that each have a block of their own (a large decoding batch), on both sides of the line between 2 and 8 values per lane"""
+    rng = np.random.default_rng(T + D)
+    NB = T // 2 + 9
+    ks, vs = O.kv_cache_shapes(NB, bs, Hkv, D, 2, False)
+    kc, vc = rng.integers(0, 65536, ks).astype(np.uint16), rng.integers(0, 65536, vs).astype(np.uint16)
+    k, v = rng.integers(0, 65536, (T, Hkv, D)).astype(np.uint16), rng.integers(0, 65536, (T, Hkv, D)).astype(np.uint16)
+    slots = rng.permutation(NB * bs)[:T].astype(np.int64)
+    slots[[3, T - 1]] = -1
+    kcd, vcd = bf16_dev(kc), bf16_dev(vc)
+    cv.reshape_and_cache(bf16_dev(k), bf16_dev(v), kcd, vcd, dev(slots))
+    O.reshape_and_cache(k, v, kc, vc, slots, False)
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_bits(kcd), kc) and np.array_equal(bf16_bits(vcd), vc)
+
+
 def test_reshape_and_cache_rows_of_no_values(cv, lib):
     """nothing to write is no error, at few tokens and at many"""
     slots = dev(np.arange(64, dtype=np.int64))
