@@ -810,7 +810,7 @@ static int dense_launch_gj(const DenseArgs& a, int gj, int nw, hipStream_t st) {
 // T = 16 9.3 / 13.7, 32 12.3 / 14.0, 40 16.1 / 13.7; 12288 x 2048 T = 32 17.0 / 12.9; at 5 .. 16 tokens either may win (16384 pairs of 3072: 18.7 / 22.1)
 // 4-bit, against token chunks of the decode kernels: down 3584 x 18944 T = 32 21.6 / 27.4, 33 29.1 / 28.1, 49 72.7 / 29.1; 4608 x 3584 T = 33 20.8 / 16.0;
 // wo 3584 x 3584 33 14.8 / 15.0, 64 19.2 / 16.5; gate/up 37888 x 3584 48 42.1 / 54.5, 64 48.3 / 58.3, 65 64.3 / 58.8
-// (to 64 tokens the sizes decide: dense_streams, gptq_prompt_gemm)
+// (to 64 tokens the sizes decide: dense_streams, gptq_stream_us)
 enum { DENSE_GEMM_MIN_T = 33, DENSE_GEMM_ANY_T = 96, GPTQ_GEMM_MIN_T = 33, GPTQ_GEMM_MIN_PAIR_T = 65 };
 static int g_tune_gemm_min_t = DENSE_GEMM_MIN_T;
 static int g_tune_gptq_gemm_off = 0;   // tuning key 39: 1 = 4-bit prompt steps run the decode kernel in 64-token chunks (A/B)
@@ -1410,6 +1410,31 @@ static void dense_gemm_epi(const DenseGemm3& g, int which, hipStream_t st) {
     else if (g.a[0].epi == MI355_EPI_RESID) dense_gemm_tile<DT, MI355_EPI_RESID, TILED>(g, which, st);
     else dense_gemm_tile<DT, MI355_EPI_STORE, TILED>(g, which, st);
 }
+// Whether the streaming kernels make a 16-bit product sooner than the GEMM in its choice c, of those it would take below 65 tokens (33 .. 64; 17 .. 32 against 768
+// row tiles).  With a row tile or two per CU they need one launch and a wave's share of K; the GEMM walks all units in one workgroup, or there is the partial sums'
+// launch.  Both times as they were measured with the weights in HBM: the side taken is the faster one or within 5 % at 1064 of 1098 sizes (512 .. 32000 rows,
+// k of 256 .. 18944, both layouts, with and without a residual).  us, streaming / GEMM: 33 tokens 4096 x 1024 6.6 / 9.6, x 2048 9.4 / 12.2, x 3072 11.7 / 13.9, x 5120
+// 16.7 / 16.1; 2048 x 512 4.8 / 6.0, x 2048 8.8 / 9.9, x 3072 11.1 / 10.7; 48 tokens 4096 x 3072 13.4 / 14.5; 64 tokens 4096 x 1024 8.5 / 10.6, x 3072 16.6 / 15.1; two tiles per CU
+// 33 tokens 8192 x 1024 9.2 / 10.1, 64 12.6 / 11.1; a residual adds 1 .. 2 to the streaming kernels and next to nothing to the GEMM, row-major weights 0.5 .. 2; a long K in ranges
+// (few rows, activations shared through LDS) 48 tokens 1024 x 8192 14.0 / 15.8, 64 x 8192 12.4 / 11.1, row-major 1024 x 11008 19.0 / 16.9; 32 tokens 12288 x 512 7.3 / 8.1, x 1536
+// 13.3 / 14.2, x 2048 17.6 / 17.5, row-major 12288 x 1024 11.8 / 10.7
+static bool dense_streams(const DenseArgs& a, const GtChoice& c, float weights_us) {
+    if (a.T > 64 || a.epi == MI355_EPI_SILU_MUL || (a.N & 15) || (a.K & 255)) return false;
+    const int cus = mi355_num_cus(), tiles = a.N / 16, nkb = a.K >> 8, mt = (a.T + 15) / 16, rounds = (tiles + cus - 1) / cus;
+    if (a.T <= 32) return a.K >= 512 && a.K <= (a.wtiled ? 1536 : tiles <= 4 * cus ? 512 : 0);
+    if (mt == 3 && a.wtiled && a.K >= 8192 && tiles >= 32 && tiles * 4 <= cus) return true;
+    if (rounds > 2) return false;
+    const bool resid = a.epi == MI355_EPI_RESID;
+    const int nw = dense_waves(tiles, nkb, mt);
+    const float blocks = 0.5f * (float)((nkb + nw - 1) / nw) + 0.5f * (float)nkb / (float)nw;         // the slowest wave's, and the mean
+    const float block = (mt == 3 ? 2.46f + 0.04f * (float)(a.T - 33) : 3.3f + 0.04f * (float)(a.T - 49)) + (a.wtiled ? 0.f : 0.7f);
+    const float stream = 3.5f - (nw == 2 ? 1.5f : nw == 1 ? 1.4f : 0.f) + (rounds == 2 ? 0.8f : 0.3f * (float)a.N / 4096.f) +
+                         block * (rounds == 2 ? 2.05f : 1.f) * blocks + (resid ? mt == 3 ? 1.35f : 1.75f : 0.f);
+    const float cold = 1.3f * std::min(weights_us, 3.f);                                              // what of the weights' first bytes nothing hides
+    const float gemm = c.splits == 1 ? 0.67f * c.us + 2.4f + cold + 0.02f * (float)(a.T - 33) + (resid ? 0.5f : 0.f)
+                                     : 0.95f * c.us - (c.splits <= 3 ? 0.9f : 1.6f) + cold + 0.21f * (float)(c.splits - 1) + 0.03f * (float)(a.T - 33) + (resid ? 0.15f : 0.f);
+    return stream <= gemm;
+}
 // n matrices over the same x: all tiled or all row-major, one dtype
 static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) {
     if (dt != MI355_DTYPE_BF16 && dt != MI355_DTYPE_F16) return (int)hipErrorNotSupported;
@@ -1439,8 +1464,10 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     // 2048 x 4096 x 14336 215 (128 x 128, two per CU), 700 x 4096 x 14336 94 (two ranges; one: 175), 96 x 4096 x 14336 33 (64-token tiles,
     // eight ranges; one: 113), 64 x 28672 x 4096 96 / 44.
     const int max_split = n == 1 && a[0].T <= 65535 && !(a[0].N & 3) && !(a[0].epi == MI355_EPI_SILU_MUL && (a[0].pair_offset & 3)) ? gemm_max_split(a[0], std::max(1, units / 8)) : 1;
-    GtChoice best = gt_pick([&](const GtTile& t) { return tiles(t, nullptr); }, units, (float)rows * (float)a[0].K * 2.f / 5.4e6f, max_split,
+    const float weights_us = (float)rows * (float)a[0].K * 2.f / 5.4e6f;
+    GtChoice best = gt_pick([&](const GtTile& t) { return tiles(t, nullptr); }, units, weights_us, max_split,
                             (float)a[0].T * (float)a[0].N * 4.f / 4.5e6f, 31);
+    if (n == 1 && g_tune_gemm_min_t == DENSE_GEMM_MIN_T && !g_tune_gemm_tall && dense_streams(a[0], best, weights_us)) return (int)hipErrorNotSupported;
     if (g_tune_gemm_tall) best = {0, 1, 0.f};
     DenseGemm3 g{};
     for (int i = 0; i < 3; ++i) g.a[i] = a[i < n ? i : 0];
@@ -1481,30 +1508,11 @@ static int dense_prompt_gemm_staged(const DenseArgs& a, int dt, hipStream_t st) 
     return e != hipSuccess ? (int)e : dense_prompt_gemm(&c, 1, dt, st);
 }
 
-// 16-bit products that the streaming kernels make sooner than the GEMM, of those it would take below 65 tokens (33 .. 64; 17 .. 32 against 768 row tiles).  With
-// one row tile per CU they take a wave's share of K, the GEMM at least one unit per 64 k in one workgroup or the partial sums' launch.  us, streaming / GEMM:
-// 33 tokens 4096 x 1024 6.6 / 9.6, x 2048 9.4 / 12.2, x 3072 11.7 / 13.9, x 5120 16.7 / 16.1; 2048 x 512 4.8 / 6.0, x 2048 8.8 / 9.9, x 3072 11.1 / 10.7; 48 tokens 4096 x 3072
-// 13.4 / 14.5, 2048 x 2048 9.9 / 10.2; 64 tokens 4096 x 2048 12.8 / 13.4, x 3072 16.6 / 15.1, 1024 x 1024 7.6 / 7.9, x 1536 9.9 / 9.5; two tiles per CU, 33 tokens 8192 x 1024
-// 9.2 / 10.1, x 2048 14.9 / 13.4, 49 x 1024 11.4 / 10.6; a long K in ranges (LDS-shared activations) 33 tokens 1024 x 8192 13.8 / 14.7, 48 14.0 / 15.8, 64 x 8192
-// 12.4 / 11.1, 2048 x 14336 22.1 / 20.2, row-major 1024 x 11008 18.6 / 16.2; 32 tokens 12288 x 512 7.3 / 8.1, x 1536 13.3 / 14.2, x 2048 17.6 / 17.5.  At k = 256 the GEMM (4096: 5.1 / 4.9, 64 tokens
-// 6.7 / 5.3).  Row-major weights cost the streaming kernels 0.5 .. 2: 33 tokens 4096 x 2048 11.4 / 12.4, 49 13.4 / 13.4, 2048 x 1024 6.4 / 7.8, 64 8.4 / 8.3
-static bool dense_streams(const DenseArgs& a) {
-    if (a.T > 64 || a.epi == MI355_EPI_SILU_MUL || (a.N & 15) || (a.K & 255) || a.K < 512) return false;
-    const int cus = mi355_num_cus(), tiles = a.N / 16;
-    if (a.T > 32 && a.T <= 48 && a.wtiled && tiles >= 32 && tiles * 4 <= cus && a.K >= 8192) return true;
-    const int T = a.epi == MI355_EPI_RESID ? a.T + 8 : a.T;              // (a residual adds 1 to the streaming kernels, nothing to the GEMM)
-    int most;
-    if (a.T <= 32) most = 1536;
-    else if (tiles > cus) most = tiles <= 2 * cus && T <= 40 ? 1536 : 0;
-    else if (tiles > cus / 2) most = T <= 48 ? (a.wtiled ? 3072 : 2048) : T > 64 ? 1536 : a.wtiled ? 2048 : 1024;
-    else most = T <= 48 && a.wtiled ? 2048 : T > 64 ? 0 : 1024;
-    return a.K <= most;
-}
 // SILU_MUL with more than 32 tokens, or any T > 64: run in token chunks
 static int dense_run(DenseArgs a, int wtype, int dt, hipStream_t st) {
     // (rows and k that are not whole tiles of the streaming kernels are served from DENSE_GEMM_ANY_T tokens, and refused below)
     const bool whole = !(a.N & 15) && !(a.K & 255);
-    if (wtype == DW_DENSE && (a.T >= DENSE_GEMM_ANY_T || whole) && !(g_tune_gemm_min_t == DENSE_GEMM_MIN_T && !g_tune_gemm_tall && dense_streams(a)) &&
+    if (wtype == DW_DENSE && (a.T >= DENSE_GEMM_ANY_T || whole) &&
         (a.T >= g_tune_gemm_min_t || (g_tune_gemm_min_t == DENSE_GEMM_MIN_T && a.T > 16 && (a.epi == MI355_EPI_SILU_MUL ? a.pair_offset : a.N) >= 16 * 768))) {
         int rc = dense_prompt_gemm(&a, 1, dt, st);
         if (rc == (int)hipErrorNotSupported && a.T >= DENSE_GEMM_ANY_T) rc = dense_prompt_gemm_staged(a, dt, st);
