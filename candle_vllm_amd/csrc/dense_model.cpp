@@ -486,7 +486,7 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
             const QLin &gq = L.gq[MI355_W_WQ], &gk = L.gq[MI355_W_WK], &gv = L.gq[MI355_W_WV];
             const bool all_q = gq.qw && gk.qw && gv.qw && gq.group == gk.group && gq.group == gv.group;
             const bool all_d = !gq.qw && !gk.qw && !gv.qw && L.wq && L.wk && L.wv;
-            if (all_q || all_d) {                                        // (from 33 tokens: the prompt GEMM over the three matrices)
+            if (all_q || all_d) {                                        // (prompts: the GEMM over the three matrices)
                 void* outs[3] = {m->q, m->k, m->v};
                 const void* ws[3] = {all_q ? (const void*)gq.qw : L.wq, all_q ? (const void*)gk.qw : L.wk, all_q ? (const void*)gv.qw : L.wv};
                 const void* sc[3] = {gq.scales, gk.scales, gv.scales};
