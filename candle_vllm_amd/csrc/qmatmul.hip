@@ -24,6 +24,7 @@
 #include "scratch.h"
 #include "../../include/mi355_vllm.h"
 #include <string.h>
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -1967,6 +1968,69 @@ static int g_tune_qpg_min = 96;                            // mi355_set_tuning(1
 static int g_tune_dbg = 0;                                 // mi355_set_tuning(2, v): probe / ablation modes (experiments only)
 
 #include "qmm_prefill.inc"
+#include "qmm_prompt_gemm.inc"
+
+template <int WT, int WM, int WN, int MG, int NG, int SA, bool QKV = false>
+static int qpw_go(const QmmArgs& r, const QpgImg& im, int n_slots, hipStream_t st) {
+    if constexpr (!QKV) if (r.epi == MI355_EPI_QKV_ROPE_CACHE) return qpw_go<WT, WM, WN, MG, NG, SA, true>(r, im, n_slots, st);
+    using L = QpwTile<WT, WM, WN, MG, NG, SA>;
+    static Mi355DevOnce once;
+    if (!once.done()) {
+        const hipError_t e = hipFuncSetAttribute((const void*)qpw_gemm_kernel<WT, WM, WN, MG, NG, SA, QKV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::LDS);
+        if (e != hipSuccess) return (int)e;
+        once.set();
+    }
+    QpwArgs w{};
+    w.n_slots = n_slots;
+    for (int s = 0; s < r.nseg; ++s) w.odd_rows |= r.seg[s].n_rows | r.seg[s].row0;
+    w.qkv_by_8 = r.epi == MI355_EPI_QKV_ROPE_CACHE && ((w.odd_rows | r.D) & 15) == 0 && (r.rot & 7) == 0 &&
+                 (((uintptr_t)r.q_out | (uintptr_t)r.kcache | (uintptr_t)r.vcache | (uintptr_t)r.cos_t | (uintptr_t)r.sin_t) & 15) == 0;
+    w.n_m = (r.B + L::BM - 1) / L::BM;
+    w.n_n = (n_slots + L::NT - 1) / L::NT;
+    hipLaunchKernelGGL((qpw_gemm_kernel<WT, WM, WN, MG, NG, SA, QKV>), dim3(w.n_m * w.n_n), dim3(512), (size_t)L::LDS, st, r, im, w);
+    return (int)hipGetLastError();
+}
+// tile of this thread's last prompt product (tests: which kernel ran)
+static thread_local int g_qpw_last = -1;
+extern "C" int32_t mi355_internal_last_qpw(void) { return g_qpw_last; }
+// Which kernel makes a prompt product: us per k-block and round of workgroups (one per CU; the 64 x 256 tile of qmm_prefill.inc: two), a full round and
+// one that leaves most of the chip idle (it runs at a higher clock).  Both sides measured at 19 sizes of 96 .. 4096 tokens for 14 matrices of 1024 x 4096 ..
+// 28672 x 4096: with the choice 1.09 x as fast on average as with 64 x 256 tiles alone (Q4_K up to 1.34 x, Q6_K 1.92 x), nowhere slower by more than 2 %.
+struct QpwChoice { int tile; float us; };
+static QpwChoice qpw_pick(int type, int T, int n_slots, int K, float old_extra_us) {
+    const int cus = mi355_num_cus(), nkb = K >> 8;
+    auto est = [&](int bm, int bn, int cap, float full, float light) {
+        const int wgs = ((T + bm - 1) / bm) * ((n_slots * 16 + bn - 1) / bn), left = wgs % cap;
+        // two workgroups per CU: up to half a round they have a CU each
+        const float last = !left ? 0.f : cap > cus ? (left <= cus ? light : full) : light + (full - light) * (float)left / (float)cap;
+        return (float)nkb * (full * (float)(wgs / cap) + last);
+    };
+    QpwChoice best{-1, 0.f};
+    auto take = [&](int tile, float us) {
+        if (tile >= 0) us += 4.f;                                     // a workgroup alone on its CU: nothing hides its first loads and its epilogue
+        if (best.us == 0.f || us < best.us) best = {tile, us};
+    };
+    if (type == MI355_GGML_Q4_K) {
+        take(-1, old_extra_us + est(64, 256, 2 * cus, 5.f, 3.4f));
+        take(0, est(256, 256, cus, 7.4f, 6.2f));
+        take(1, est(256, 128, cus, 4.6f, 3.9f));
+        take(2, est(192, 256, cus, 6.2f, 5.2f));
+    } else {
+        take(-1, old_extra_us + est(64, 256, cus, 4.3f, 3.95f));
+        take(1, est(256, 128, cus, 4.8f, 4.1f));
+    }
+    return best;
+}
+extern "C" int32_t mi355_internal_qpw_pick(int32_t type, int32_t T, int32_t n_slots, int32_t K) { return qpw_pick(type, T, n_slots, K, 0.f).tile; }   // tests
+template <int WT>
+static int qpw_launch(int tile, const QmmArgs& r, const QpgImg& im, int n_slots, hipStream_t st) {
+    g_qpw_last = WT == MI355_GGML_Q4_K ? tile : 10 + tile;
+    if constexpr (WT == MI355_GGML_Q4_K) {
+        if (tile == 0) return qpw_go<WT, 2, 4, 4, 2, 2>(r, im, n_slots, st);
+        if (tile == 2) return qpw_go<WT, 2, 4, 3, 2, 2>(r, im, n_slots, st);
+    }
+    return qpw_go<WT, 4, 2, 2, 2, 2>(r, im, n_slots, st);
+}
 
 // hand-written prompt-step GEMM (qmm_prefill.inc); returns hipErrorNotSupported for launches it does not cover (then the
 // caller keeps the library-GEMM path)
@@ -1979,11 +2043,30 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
     int n_slots = 0;
     for (int s = 0; s < a.nseg; ++s) n_slots += a.seg[s].n_tiles;
     const int T = a.B, K = a.K, ldp = n_slots * 16, nkb = K >> 8;
-    const int Tpad = (T + QPG_BM - 1) / QPG_BM * QPG_BM;
     const int parts = g_tune_exact_act ? 2 : 1;             // activation planes of the f16 image (mi355_set_tuning(24, 1) = hi + lo)
+    // the launches of this product, and the kernel of each (qpw_pick; -1: qmm_prefill.inc's): one of all rows, or q | k and a Q6_K v
+    bool all_q4 = true;
+    for (int s = 0; s < a.nseg; ++s) all_q4 = all_q4 && a.seg[s].type == MI355_GGML_Q4_K;
+    const bool one_q6 = a.nseg == 1 && !all_q4;
+    const bool epi_ok = a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID ||
+                        (a.epi == MI355_EPI_SILU_MUL && a.nseg == 2 && a.seg[0].n_tiles == a.seg[1].n_tiles && a.seg[0].n_rows == a.seg[1].n_rows);
+    const bool fuse = g_tune_qpg_fepi && parts == 1 && g_tune_qpg == 2, big = fuse && (size_t)K * (T + 512) * 2 < ((size_t)1 << 32);
+    const bool qkv = a.epi == MI355_EPI_QKV_ROPE_CACHE && a.nseg == 3 && a.seg[0].type == MI355_GGML_Q4_K && a.seg[1].type == MI355_GGML_Q4_K;
+    const int v_slots = qkv && a.seg[2].type == MI355_GGML_Q6_K ? a.seg[2].n_tiles : 0, slots4 = n_slots - v_slots;
+    const float c_pass = 3.f + (float)T * (float)ldp * 8e-6f / 4.f;      // us of a launch that reads the f32 sums back: kernels without the epilogue need it
+    int pick4 = -1, pick6 = -1;
+    g_qpw_last = -1;
+    if (big && !a.blk_tab && ((all_q4 && epi_ok) || qkv)) pick4 = qpw_pick(MI355_GGML_Q4_K, T, slots4, K, qkv && T < 1024 ? c_pass : 0.f).tile;
+    if (big && !a.blk_tab && (v_slots || (one_q6 && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID))))
+        pick6 = qpw_pick(MI355_GGML_Q6_K, T, v_slots ? v_slots : n_slots, K, v_slots || T >= 4096 ? 0.f : c_pass).tile;
+    // token rows of the image: whole tiles of whichever kernel reads it
+    const int Tpad = pick4 == 2 ? std::max((T + 191) / 192 * 192, (T + 255) / 256 * 256)
+                     : pick4 >= 0 || pick6 >= 0 ? (T + 255) / 256 * 256 : (T + QPG_BM - 1) / QPG_BM * QPG_BM;
     // (a block-table launch only exists with the epilogue in the store loop: no C buffer -- it would be 1.9 GB for a Mixtral chunk)
+    const int blk64 = (T + QPG_BM - 1) / QPG_BM * (QPG_BM / 64);   // token blocks of the 64-token kernels
     const size_t xa_b = (size_t)K * Tpad * 2 * parts, sf_b = (size_t)nkb * Tpad * 32, rs_b = (size_t)Tpad * 4, c_b = a.blk_tab ? 0 : (size_t)T * ldp * 4;
     void* ws = nullptr;
+    Mi355ScratchTurn turn(MI355_SCR_QMP_WS, st);            // from the image's launch to its readers'
     int rc = qmg_buf(&ws, MI355_SCR_QMP_WS, xa_b + sf_b + 2 * rs_b + c_b + 4096, st);
     if (rc) return rc;
     a.dbg = g_tune_dbg;                                     // ablation bits of the prompt-step GEMM (experiments only)
@@ -2022,15 +2105,12 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
     // EXPERIMENT (mi355_set_tuning(48, 1)): all segments Q4_K, one activation plane, the default wave tile, and an epilogue that is a
     // store / residual add / SiLU * up over two equal segments -> the GEMM writes the outputs itself, no C buffer, no epilogue launch
     {
-        bool all_q4 = true;
-        for (int s = 0; s < a.nseg; ++s) all_q4 = all_q4 && a.seg[s].type == MI355_GGML_Q4_K;
-        const bool epi_ok = a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID ||
-                            (a.epi == MI355_EPI_SILU_MUL && a.nseg == 2 && a.seg[0].n_tiles == a.seg[1].n_tiles && a.seg[0].n_rows == a.seg[1].n_rows);
         if (g_tune_qpg_fepi && all_q4 && epi_ok && parts == 1 && (g_tune_qpg == 0 || g_tune_qpg == 2)) {
             QmmArgs r = a;
             r.norm_w = nullptr;                                 // applied while the image was built
+            if (pick4 >= 0) return qpw_launch<MI355_GGML_Q4_K>(pick4, r, im, n_slots, st);
             if (g_tune_qpg == 2) {                              // 64 tokens x 256 rows per workgroup (waves 64 x 32), two workgroups per CU
-                const dim3 g_(Tpad / 64, (n_slots + 15) / 16), b_(512);
+                const dim3 g_(blk64, (n_slots + 15) / 16), b_(512);
                 if (a.blk_tab) hipLaunchKernelGGL((qpg_gemm_lds2_kernel<true, true>), g_, b_, (size_t)QPG2_BYTES, st, r, im, C, ldp, n_slots, 0);
                 else hipLaunchKernelGGL((qpg_gemm_lds2_kernel<true>), g_, b_, (size_t)QPG2_BYTES, st, r, im, C, ldp, n_slots, 0);
             } else {
@@ -2048,7 +2128,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
                 g_tune_qpg == 2 && g_tune_qpg_fepi) {
                 QmmArgs r = a;
                 r.norm_w = nullptr;
-                hipLaunchKernelGGL((qpg_gemm_q6k_lds_kernel<true, 2, true>), dim3(Tpad / 64, (n_slots + 15) / 16), dim3(512), (size_t)QPG6_LDS_BYTES, st, r, im, C,
+                hipLaunchKernelGGL((qpg_gemm_q6k_lds_kernel<true, 2, true>), dim3(blk64, (n_slots + 15) / 16), dim3(512), (size_t)QPG6_LDS_BYTES, st, r, im, C,
                                    ldp, n_slots, 0);
                 return (int)hipGetLastError();
             }
@@ -2068,15 +2148,15 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
 #define QPG_FUSE_QKV 1          // A/B builds: 0 = q | k | v through the C buffer and the epilogue launch (rounds 2-5)
 #endif
     // (from 1024 tokens: measured +0.7 % at 2048 and +1.2 % at 4096 tokens, -1.9 % at 512 -- profiles/r06_prompt_qkv_fused_ab.txt)
-    if (QPG_FUSE_QKV && T >= 1024 && g_tune_qpg_fepi && parts == 1 && g_tune_qpg == 2 && a.epi == MI355_EPI_QKV_ROPE_CACHE && a.nseg == 3 &&
-        a.seg[0].type == MI355_GGML_Q4_K && a.seg[1].type == MI355_GGML_Q4_K && (QPG_FUSE_Q6K || a.seg[2].type == MI355_GGML_Q4_K)) {
+    if (QPG_FUSE_QKV && (T >= 1024 || pick4 >= 0) && fuse && qkv && (QPG_FUSE_Q6K || !v_slots)) {
         const bool v4 = a.seg[2].type == MI355_GGML_Q4_K;
         QmmArgs r = a;
         r.norm_w = nullptr;                                         // applied while the image was built
         if (!v4) r.nseg = 2;
         int f_slots = 0;
         for (int q = 0; q < r.nseg; ++q) f_slots += r.seg[q].n_tiles;
-        hipLaunchKernelGGL((qpg_gemm_lds2_kernel<true>), dim3(Tpad / 64, (f_slots + 15) / 16), dim3(512), (size_t)QPG2_BYTES, st, r, im, C, ldp, f_slots, 0);
+        if (pick4 >= 0) { const int rcw = qpw_launch<MI355_GGML_Q4_K>(pick4, r, im, f_slots, st); if (rcw) return rcw; }
+        else hipLaunchKernelGGL((qpg_gemm_lds2_kernel<true>), dim3(blk64, (f_slots + 15) / 16), dim3(512), (size_t)QPG2_BYTES, st, r, im, C, ldp, f_slots, 0);
         if (v4) return (int)hipGetLastError();
         // v (Q6_K): its own GEMM with the fused store loop; q and k stay in the descriptor as EMPTY segments (no tiles) so that the value
         // segment keeps its role (2 = v: bf16 + cache scatter, no rotation) and its row offsets
@@ -2085,10 +2165,11 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
         rv.seg[0].n_tiles = 0; rv.seg[1].n_tiles = 0;
         // (one row tile per wave where two would leave CUs empty: 1024 rows x 2048 tokens = 128 workgroups of 256 rows)
         const int vt = a.seg[2].n_tiles;
-        if (QPG6_SPLIT_SMALL && (Tpad / 64) * ((vt + 15) / 16) < mi355_num_cus())
-            hipLaunchKernelGGL((qpg_gemm_q6k_lds_kernel<true, 1>), dim3(Tpad / 64, (vt + 7) / 8), dim3(512), (size_t)QPG6_LDS_BYTES, st, rv, im, C, ldp, vt, 0);
+        if (pick6 >= 0) return qpw_launch<MI355_GGML_Q6_K>(pick6, rv, im, vt, st);
+        if (QPG6_SPLIT_SMALL && blk64 * ((vt + 15) / 16) < mi355_num_cus())
+            hipLaunchKernelGGL((qpg_gemm_q6k_lds_kernel<true, 1>), dim3(blk64, (vt + 7) / 8), dim3(512), (size_t)QPG6_LDS_BYTES, st, rv, im, C, ldp, vt, 0);
         else
-            hipLaunchKernelGGL((qpg_gemm_q6k_lds_kernel<true>), dim3(Tpad / 64, (vt + 15) / 16), dim3(512), (size_t)QPG6_LDS_BYTES, st, rv, im, C, ldp, vt, 0);
+            hipLaunchKernelGGL((qpg_gemm_q6k_lds_kernel<true>), dim3(blk64, (vt + 15) / 16), dim3(512), (size_t)QPG6_LDS_BYTES, st, rv, im, C, ldp, vt, 0);
         return (int)hipGetLastError();
     }
     for (int s0 = 0, slot_base = 0; s0 < a.nseg;) {
@@ -2113,7 +2194,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
 #endif
                 default:                                                //  64 x 256, waves 64 x 32, two workgroups per CU; one activation plane: image and weights through LDS by DMA
                     if (parts == 1) {
-                        const dim3 g4(Tpad / 64, (run_slots + 15) / 16), b_(512);
+                        const dim3 g4(blk64, (run_slots + 15) / 16), b_(512);
                         hipLaunchKernelGGL((qpg_gemm_lds2_kernel<false>), g4, b_, (size_t)QPG2_BYTES, st, r, im, C, ldp, run_slots, slot_base);
                     } else {
                         QPG_GO(4, 2, 1, 8, false);                      // hi + lo planes ("exact" activations): the register-fed form
@@ -2123,7 +2204,11 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
 #undef QPG_GO
         } else {
             if (parts == 1 && g_tune_qpg == 2) {                        // Q6_K: 64 tokens x 256 rows per workgroup; token blocks fastest
-                const dim3 grid(Tpad / 64, (run_slots + 15) / 16);
+                const dim3 grid(blk64, (run_slots + 15) / 16);
+                if (pick6 >= 0 && one_q6) {
+                    r.norm_w = nullptr;
+                    return qpw_launch<MI355_GGML_Q6_K>(pick6, r, im, run_slots, st);
+                }
                 // the whole mat-mul is this one Q6_K run and its epilogue is a store / residual add: fused store loop, no C buffer, no launch
                 // (from 4096 tokens -- measured: +1.2 % at 4096, -0.2 % at 2048: profiles/r06_prompt_q6k_fused_ab.txt)
                 if (QPG_FUSE_Q6K && g_tune_qpg_fepi && T >= 4096 && s0 == 0 && s1 == a.nseg && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID)) {

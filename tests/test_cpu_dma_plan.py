@@ -140,3 +140,55 @@ def test_two_workgroup_kernel_counted_waits(lib):
         slack = _simulate_two_wg(plan, nkb)
         assert min(slack) >= 0 and min(slack) == 0, (nkb, slack[:12])
     assert set(_simulate_two_wg(plan, 16)[8:]) == {0}
+
+
+def _simulate_unpacked_once(plan, nkb):
+    """qpw_gemm_kernel: behind the barrier of chunk c (in the middle of step 2 c + 1) the image of chunk + 2, then headers and first planes of the
+    next k-block (c = 0) or its other planes (c = 1; one plane's room: of this k-block's successor, c = 3); the sums in front of chunk 2's image.
+    Everything of the prologue has landed before the loop, but for the second planes where they share the first ones' room."""
+    sa, ar, x1, x3, one, ut, waits = plan[0], plan[1], plan[2], plan[3], plan[4], plan[5], plan[6:]
+    assert sa == 2 and x1 >= 2 * ut and x3 == (0 if one else ut)
+    issued, retired = [], 0
+    if one:
+        issued += [("P1", 0)] * ut
+    slack = []
+    for kb in range(nkb):
+        for c in range(4):
+            retired = max(retired, len(issued) - waits[c])
+            kc = 4 * kb + c
+            need = [("I", kc + 1)] if kc + 1 >= sa else []            # read behind this barrier: the next chunk ...
+            if c == 0 and (one or kb > 0):
+                need.append(("P1", kb))                               # ... the second planes (step 1), ...
+            if c == 2 and kb + 1 < nkb:
+                need += [("H", kb + 1), ("P0", kb + 1)]               # ... the next k-block's headers and first planes (step 5), ...
+            if c == 3 and kb + 1 < nkb:
+                need.append(("S", kb + 1))                            # ... and its sums (end of step 7)
+            for n in need:
+                pos = [i for i, op in enumerate(issued) if op == n]
+                assert pos and max(pos) < retired, (plan, kb, c, n)
+            newest = max([i for i, op in enumerate(issued) if op in need], default=None)
+            if newest is not None:
+                slack.append(len(issued) - 1 - newest - waits[c])
+            if c == 2:
+                issued.append(("S", kb + 1))
+            issued += [("I", kc + sa)] * ar
+            if c == 0:
+                issued += [("H", kb + 1)] * (x1 - ut) + [("P0", kb + 1)] * ut
+            if c == (3 if one else 1):
+                issued += [("P1", kb + 1)] * ut
+    return slack
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2, 11])
+def test_unpacked_once_kernel_counted_waits(lib, tile):
+    f = lib.mi355_internal_qpw_dma_plan
+    f.restype, f.argtypes = ctypes.c_int32, [ctypes.c_int32, ctypes.c_void_p]
+    out = (ctypes.c_int32 * 10)()
+    assert f(tile, ctypes.addressof(out)) == 0
+    plan = list(out)
+    if tile == 11:                                                    # Q6_K: scales, d, and two planes (low half 0, high bits) in front of the last
+        assert plan[2] == 4 * plan[5]
+    for nkb in (1, 2, 3, 16, 56):
+        assert min(_simulate_unpacked_once(plan, nkb)) >= 0
+    # (chunk 3 waits for all: the sums went out ahead of the image that it needs)
+    assert max(_simulate_unpacked_once(plan, 16)) <= plan[5], plan

@@ -1,0 +1,156 @@
+"""The prompt products that unpack every weight once per workgroup (csrc/qmm_prompt_gemm.inc): each tile of both types, at tiles that end inside
+a token block, a row tile or the matrix, with every epilogue, against dequantised weights in 64 bits."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import candle_vllm_amd.ops as cv
+from oracle import kquants as kq
+
+pytestmark = pytest.mark.gpu
+Q4, Q6 = kq.GGML_Q4_K, kq.GGML_Q6_K
+# activations are rounded to f16 once (2^-12 of each, its share of a row's error about 2^-12 / sqrt(3) and, over the largest outputs, three times that)
+TOL = 5e-4
+
+
+def last_tile():
+    f = cv.lib.mi355_internal_last_qpw
+    f.restype = ctypes.c_int32
+    return f()
+
+
+def blocks(rng, n, k, kind, odd=True):
+    """native GGUF blocks of random codes; with `odd`, blocks of d = 0 (with and without a minimum), of a large minimum beside a tiny d, and, Q6_K, of d < 0"""
+    size = 144 if kind == Q4 else 210
+    b = rng.integers(0, 256, (n, k // 256, size), dtype=np.uint8)
+    d = rng.uniform(1e-4, 3e-4, (n, k // 256)).astype(np.float16)
+    m = rng.uniform(1e-4, 3e-3, (n, k // 256)).astype(np.float16)
+    if odd:
+        pick = rng.integers(0, 16, (n, k // 256))
+        d[pick == 0] = 0
+        m[pick == 0] *= rng.integers(0, 2, (pick == 0).sum()).astype(np.float16)
+        d[pick == 1] = 6e-7
+        d[pick == 2] = 2e-2 if kind == Q4 else -3e-4
+
+    def put(at, v):
+        b[:, :, at:at + 2] = v.view(np.uint8).reshape(n, k // 256, 2)
+    put(0 if kind == Q4 else 208, d)
+    if kind == Q4:
+        put(2, m)
+    return b
+
+
+def product(x, b, kind):
+    return x.double() @ torch.from_numpy(kq.dequantize(b, kind)).cuda().double().t()
+
+
+def close(got, want):
+    assert torch.isfinite(got).all()
+    return ((got.double() - want).abs().max() / want.abs().max()).item()
+
+
+@pytest.mark.parametrize("kind,T,N,K,tile", [(Q4, 385, 28628, 1024, 0), (Q4, 700, 16380, 1024, 2), (Q4, 1281, 4096, 2048, 1), (Q4, 1300, 4120, 2048, 1), (Q4, 4097, 2064, 1024, 2),
+                                             (Q4, 4001, 4084, 1024, 0), (Q4, 200, 512, 512, -1), (Q6, 1300, 4120, 1024, 11), (Q6, 1153, 4096, 512, 11), (Q6, 100, 2048, 8192, -1)])
+def test_store_and_residual(kind, T, N, K, tile):
+    rng = np.random.default_rng(T + N)
+    b = blocks(rng, N, K, kind)
+    m = cv.QMatMul(b, kind, "cuda")
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    x[T // 2] *= 3000.0                                               # a token that the image scales
+    want = product(x, b, kind)
+    rows = torch.cat([torch.arange(T // 2), torch.arange(T // 2 + 1, T)]).cuda()
+    bias = torch.randn(N, device="cuda")
+    got = m.forward(x)
+    assert last_tile() == tile
+    assert close(got[rows], want[rows]) < TOL and close(got[T // 2], want[T // 2]) < TOL
+    assert close(m.forward(x, bias)[rows], (want + bias)[rows]) < TOL
+    for pad in (0, 3):                                                # whole fours, and rows that are not
+        o = torch.randn(T, N + pad, device="cuda")
+        keep = o.clone()
+        d = cv.QmmDesc()
+        d.nseg, d.w_tiles[0], d.ggml_type[0], d.n_rows[0] = 1, m.tiles.data_ptr(), kind, N
+        d.x, d.x_dtype, d.ldx, d.k, d.num_tokens = x.data_ptr(), cv.DT_F32, K, K, T
+        d.epilogue, d.out, d.ldo, d.residual = cv.EPI_RESID, o.data_ptr(), N + pad, o.data_ptr()
+        assert cv.lib.mi355_qmatmul_fused(d, torch.cuda.current_stream().cuda_stream) == 0
+        assert close(o[rows, :N], (want + keep[:, :N].double())[rows]) < TOL
+        assert torch.equal(o[:, N:], keep[:, N:])
+
+
+@pytest.mark.parametrize("T,N,K,tile", [(385, 14314, 1024, 0), (700, 8190, 1024, 2), (1281, 2048, 2048, 1), (1300, 2060, 2048, 1)])
+def test_gate_up(T, N, K, tile):
+    rng = np.random.default_rng(T + N)
+    bg, bu = blocks(rng, N, K, Q4), blocks(rng, N, K, Q4)
+    g, u = cv.QMatMul(bg, Q4, "cuda"), cv.QMatMul(bu, Q4, "cuda")
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    nw = 1 + 0.1 * torch.randn(K, device="cuda")
+    xn = (x.double() * torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-5) * nw.double()).float()
+    want = torch.nn.functional.silu(product(xn, bg, Q4)) * product(xn, bu, Q4)
+    out = torch.empty(T, N, device="cuda")
+    cv.qmatmul_fused([g, u], x, epilogue=cv.EPI_SILU_MUL, out=out, norm_weight=nw, norm_eps=1e-5)
+    assert last_tile() == tile
+    assert close(out, want) < 2 * TOL                                 # two rounded factors
+
+
+# heads and rotated parts of whole eights (eight columns per lane) and not (a column per lane); values Q4_K and Q6_K; the three cache layouts
+@pytest.mark.parametrize("layout,D,rot,v_kind,H,Hkv,T,K", [("paged", 128, 128, Q6, 32, 8, 2049, 1024), ("paged", 64, 32, Q4, 64, 2, 2049, 1024), ("flash", 128, 128, Q4, 32, 4, 2049, 1024),
+                                                           ("fp8", 128, 64, Q4, 40, 4, 2049, 1024), ("paged", 80, 20, Q4, 60, 3, 2051, 1024), ("flash", 80, 20, Q6, 60, 3, 2051, 1024)])
+def test_qkv(layout, D, rot, v_kind, H, Hkv, T, K):
+    rng = np.random.default_rng(T + D)
+    kinds, heads = (Q4, Q4, v_kind), (H, Hkv, Hkv)
+    bs = [blocks(rng, n * D, K, t, odd=layout != "fp8") for n, t in zip(heads, kinds)]   # (e4m3 ends at 448)
+    ms = [cv.QMatMul(b, t, "cuda") for b, t in zip(bs, kinds)]
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    block = 16
+    pos = torch.from_numpy(rng.integers(0, 5000, T)).cuda()
+    slot = torch.from_numpy(rng.permutation(T + 64)[:T].astype(np.int64)).cuda()
+    slot[5] = -1                                                      # a token that the cache does not take
+    half = rot // 2
+    ang = torch.arange(5000, device="cuda").double()[:, None] * 10000.0 ** (-torch.arange(half, device="cuda").double() / half)
+    cos, sin = ang.cos().float().contiguous(), ang.sin().float().contiguous()
+    nb = (T + 64 + block - 1) // block
+    x16 = 16 if layout == "fp8" else 8
+    dt = torch.uint8 if layout == "fp8" else torch.bfloat16
+    if layout == "flash":
+        kc, vc = (torch.zeros(nb, block, Hkv, D, dtype=dt, device="cuda") for _ in range(2))
+    else:
+        kc, vc = torch.zeros(nb, Hkv, D // x16, block, x16, dtype=dt, device="cuda"), torch.zeros(nb, Hkv, D, block, dtype=dt, device="cuda")
+    q_out = torch.zeros(T, H * D, dtype=torch.bfloat16, device="cuda")
+    bias = torch.randn(sum(heads) * D, device="cuda") * 0.1
+    d = cv.QmmDesc()
+    d.nseg = 3
+    for i, (m, n, t) in enumerate(zip(ms, heads, kinds)):
+        d.w_tiles[i], d.ggml_type[i], d.n_rows[i] = m.tiles.data_ptr(), t, n * D
+    d.x, d.x_dtype, d.ldx, d.k, d.num_tokens = x.data_ptr(), cv.DT_F32, K, K, T
+    d.epilogue, d.bias, d.cos_table, d.sin_table, d.positions, d.slot_mapping = cv.EPI_QKV_ROPE_CACHE, bias.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), slot.data_ptr()
+    d.q_out, d.key_cache, d.value_cache = q_out.data_ptr(), kc.data_ptr(), vc.data_ptr()
+    d.num_heads, d.num_kv_heads, d.head_dim, d.rotary_dim, d.block_size = H, Hkv, D, rot, block
+    d.kv_layout = {"paged": cv.KV_PAGED, "flash": cv.KV_FLASH, "fp8": 2}[layout]
+    assert cv.lib.mi355_qmatmul_fused(d, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert last_tile() >= 0
+    parts = torch.split(torch.cat([product(x, b, t) for b, t in zip(bs, kinds)], 1) + bias, [n * D for n in heads], 1)
+
+    def turned(y):
+        y = y.view(T, -1, D).clone()
+        c, s = cos[pos].double()[:, None], sin[pos].double()[:, None]
+        a, b = y[..., 0:rot:2].clone(), y[..., 1:rot:2].clone()
+        y[..., 0:rot:2], y[..., 1:rot:2] = a * c - b * s, a * s + b * c
+        return y
+    tol = TOL + 2.0 ** -8 if layout != "fp8" else TOL + 2.0 ** -3     # bf16's rounding; e4m3's
+    assert close(q_out, turned(parts[0]).reshape(T, -1)) < TOL + 2.0 ** -8
+    ok = slot >= 0
+    blk, off = slot[ok] // block, slot[ok] % block
+    if layout == "flash":
+        k, v = kc[blk, off], vc[blk, off]
+    else:
+        k, v = kc[blk, :, :, off].reshape(int(ok.sum()), Hkv, D), vc[blk, :, :, off]
+        if layout == "fp8":
+            k, v = k.view(torch.float8_e4m3fn).float(), v.contiguous().view(torch.float8_e4m3fn).float()
+    assert close(k.float(), turned(parts[1])[ok]) < tol
+    assert close(v.float(), parts[2].view(T, Hkv, D)[ok]) < tol
+    untouched = torch.ones(nb * block, dtype=torch.bool, device="cuda")
+    untouched[slot[ok]] = False
+    flat = kc.view(nb * block, -1) if layout == "flash" else kc.permute(0, 3, 1, 2, 4).reshape(nb * block, -1)
+    assert (flat[untouched].float() == 0).all()
