@@ -346,21 +346,33 @@ __global__ void __launch_bounds__(64) prefill_attn_generic_kernel(const PrefillP
 }
 
 // ------------------------------------------------------------------------------------------------
-// EXPERIMENT (tuning key 47 = 1; bf16, head_dim 128, keys from the PAGED cache, block size 16 / 32 / 64): prompt attention with K / V
-// through LDS by DMA.  prefill_attn_kernel above gives every wave its own K / V fragments straight from global memory: 128 queries of
+// bf16, head_dim 128, keys from the PAGED cache, block size 16 / 32 / 64: prompt attention with K / V through LDS by DMA (tuning key 47).
+// prefill_attn_kernel above gives every wave its own K / V fragments straight from global memory: 128 queries of
 // ONE head per workgroup, so a 2048-token prompt reads every K / V tile 16 x 4 (GQA) times out of L2 -- 432 us per layer at
-// Llama-3-8B shapes, 79 TFLOP/s.  Here a workgroup is 64 queries x the (up to) four heads of a GQA group: wave w owns head w, the four
-// waves share every K / V byte through the stage ring of paged_attn_lds_kernel (64-token stages, global_load_lds_dwordx4 three stages
-// ahead, counted vmcnt, one barrier per stage, the same conflict-free layouts -- pa_lds_layout.h), and a wave has the whole register
-// file: Q (4 query tiles x 4 k-steps), K of the stage (16 fragments, read once for the four query tiles), O (4 x 8 accumulators).
+// Llama-3-8B shapes, 79 TFLOP/s.  Here a workgroup is 32 queries x the (up to) four heads of a GQA group: wave w owns head w, the four
+// waves share every K / V byte through a ring of two 64-token stages (global_load_lds_dwordx4 one stage
+// ahead, counted vmcnt, one barrier per stage, the same conflict-free layouts -- pa_lds_layout.h).
 //   S^T = K . Q^T per (key tile, query tile): the lane owns ONE query per query tile -- running max / sum are per-lane scalars;
 //   O   = P . V  with P as the A operand (hi + lo bf16 pieces, as prefill_attn_kernel: the 1e-3 logit bound is against exact
-//         softmax) and the V row fragment as B: 192 MFMAs per wave and stage.
+//         softmax) and the V row fragment as B: 96 MFMAs per wave and stage.
+// What bounds it: MFMAs (1.5 x the useful ones: P in two pieces) beside the vector work of the softmax, which two waves per SIMD hide from each
+// other -- two workgroups per CU by LDS (64 KiB) AND by registers (231, none of them accumulation registers that the rescaling would have
+// to copy).  One wave per SIMD (299 registers) took 111 us for 2048 tokens x 32 heads, this 83; 4096 queries behind 4096 keys 1220 us in
+// 64-query workgroups, one per CU, and 670 here (615 useful TFLOP/s).  Its share: the scale inside the exponent's multiply-add, v_exp_f32 as
+// it is, O rescaled only where a maximum moved, values beyond the context cleared once in LDS, maxima across lanes by permlane swaps.
 // Causal masks only on the stages the diagonal crosses; exp2 domain and softcap as prefill_attn_kernel.
-template <int R, int QT = 4>
-__global__ void __launch_bounds__(256, 1) prefill_attn_lds_kernel(const PrefillParams p, const uint32_t* __restrict__ btab,
+// the largest of the four values that lanes c, c + 16, c + 32, c + 48 hold, in all of them
+__device__ __forceinline__ float pfl_max_over_rows(float x) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+constexpr int PFL_STAGES = 2, PFL_QT = 2;                            // stages of the ring, query tiles of 16 per workgroup
+__global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillParams p, const uint32_t* __restrict__ btab,
                                                                    const uint32_t* __restrict__ clens, const uint32_t* __restrict__ cuq) {
-    constexpr int D = 128, NC = 4, NDT = 8;
+    constexpr int D = 128, NC = 4, NDT = 8, R = PFL_STAGES, QT = PFL_QT;
     constexpr uint32_t STAGE_B = 32768u;
     extern __shared__ __attribute__((aligned(1024))) uint8_t pfl_smem[];
     // QT = query tiles of 16 per workgroup.  Grid: x = head group (fastest), y = query block, HEAVIEST FIRST (the last block of a prompt sees
@@ -453,20 +465,30 @@ __global__ void __launch_bounds__(256, 1) prefill_attn_lds_kernel(const PrefillP
     }
     for (int i = 0; i < ns; ++i) {
         {
-            const int ahead = min(ns, i + R - 1) - (i + 1);
-            if (ahead >= 3) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-            else if (ahead == 2) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-            else if (ahead == 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            static_assert(R == 2, "the stage requested in the iteration before is the only one under way");
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __syncthreads();
         if (i + R - 1 < ns) {
             issue(i + R - 1, ent);
             if (i + R < ns) load_ent(i + R, ent);
         }
-        if (!active) continue;                                        // uniform per wave; the barrier is at the top of the loop
-        const uint8_t* Kb = pfl_smem + (size_t)(i % R) * STAGE_B;
+        uint8_t* Kb = pfl_smem + (size_t)(i % R) * STAGE_B;
         const int tb = 64 * i;
+        if (tb + 64 > ctx) {                                          // the last stage: values at or beyond ctx hold arbitrary bits, cleared here (the stage is in LDS, no DMA aims at it)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int piece = ((int)threadIdx.x >> 7) * 4 + q, first = tb + 32 * (piece >> 2) + 8 * (piece & 3);
+                uint4* const at = reinterpret_cast<uint4*>(Kb + pal_v_read_off((int)threadIdx.x & 127, piece >> 2, piece & 3));
+                uint32_t m[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m[e] = (first + 2 * e < ctx ? 0x0000FFFFu : 0u) | (first + 2 * e + 1 < ctx ? 0xFFFF0000u : 0u);
+                const uint4 v = *at;
+                *at = make_uint4(v.x & m[0], v.y & m[1], v.z & m[2], v.w & m[3]);
+            }
+            __syncthreads();
+        }
+        if (!active) continue;                                        // uniform per wave; the barriers are above
         const bool diag = tb + 63 > cached + q0;                      // some query of the block does not see the whole stage
         // ---- K fragments of the stage: tile (ip, it), k-step j
         uint4 ka[2][2][NC];
@@ -493,20 +515,18 @@ __global__ void __launch_bounds__(256, 1) prefill_attn_lds_kernel(const PrefillP
 #pragma unroll
                     for (int v = 0; v < 4; ++v) x[ip][it][v] = acc[v];
                 }
-            if (p.softcap > 0.f) {                                    // one uniform branch for the sixteen logits of the query tile
+            // logits in units of log 2 are x sl; a softcap or a scale that is not positive is applied here (one uniform branch), else inside the exponent
+            float sl = p.scale_log2;
+            if (p.softcap > 0.f || !(sl > 0.f)) {
+                const bool cap = p.softcap > 0.f;
+                sl = 1.f;
 #pragma unroll
                 for (int ip = 0; ip < 2; ++ip)
 #pragma unroll
                     for (int it = 0; it < 2; ++it)
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) x[ip][it][v] = tanhf(x[ip][it][v] * p.scale / p.softcap) * p.softcap * 1.4426950408889634f;
-            } else {
-#pragma unroll
-                for (int ip = 0; ip < 2; ++ip)
-#pragma unroll
-                    for (int it = 0; it < 2; ++it)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) x[ip][it][v] *= p.scale_log2;
+                        for (int v = 0; v < 4; ++v)
+                            x[ip][it][v] = cap ? tanhf(x[ip][it][v] * p.scale / p.softcap) * p.softcap * 1.4426950408889634f : x[ip][it][v] * p.scale_log2;
             }
             if (diag) {
 #pragma unroll
@@ -523,10 +543,9 @@ __global__ void __launch_bounds__(256, 1) prefill_attn_lds_kernel(const PrefillP
                 for (int it = 0; it < 2; ++it)
 #pragma unroll
                     for (int v = 0; v < 4; ++v) tmax = fmaxf(tmax, x[ip][it][v]);
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-            const float m_new = fmaxf(m_run[qt], tmax);               // finite from the first stage on: key 0 is visible to every query
-            alpha[qt] = exp2f(m_run[qt] - m_new);
+            tmax = pfl_max_over_rows(tmax);
+            const float m_new = fmaxf(m_run[qt], tmax * sl);          // finite from the first stage on: key 0 is visible to every query
+            alpha[qt] = __builtin_amdgcn_exp2f(m_run[qt] - m_new);
             m_run[qt] = m_new;
             float psum = 0.f;
 #pragma unroll
@@ -535,7 +554,7 @@ __global__ void __launch_bounds__(256, 1) prefill_attn_lds_kernel(const PrefillP
 #pragma unroll
                 for (int it = 0; it < 2; ++it)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) { e8[4 * it + v] = exp2f(x[ip][it][v] - m_new); psum += e8[4 * it + v]; }
+                    for (int v = 0; v < 4; ++v) { e8[4 * it + v] = __builtin_amdgcn_exp2f(fmaf(x[ip][it][v], sl, -m_new)); psum += e8[4 * it + v]; }
                 const uint4 hi = make_uint4(cvt_pk_bf16(e8[0], e8[1]), cvt_pk_bf16(e8[2], e8[3]), cvt_pk_bf16(e8[4], e8[5]), cvt_pk_bf16(e8[6], e8[7]));
                 float r8[8];
 #pragma unroll
@@ -549,17 +568,16 @@ __global__ void __launch_bounds__(256, 1) prefill_attn_lds_kernel(const PrefillP
             l_run[qt] = fmaf(l_run[qt], alpha[qt], psum);             // this lane's share (keys 8kg.. of both pairs); summed over kg at the end
         }
         // ---- O = O * alpha + P . V : lane (channel 16 nt + c, queries 4kg+v of tile qt); query 4kg+v's alpha sits in lane 4kg+v
-        float av[QT][4];
+        // (where no query of a tile has a new maximum -- most stages -- alpha is 1 and the products with it are left out: the same bits)
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt)
+        for (int qt = 0; qt < QT; ++qt) {
+            if (__builtin_amdgcn_ballot_w64(alpha[qt] != 1.f) == 0) continue;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) av[qt][v] = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (4 * kg + v), __float_as_int(alpha[qt])));
-        uint32_t vm[2][4];                                            // keys at or beyond ctx hold arbitrary bits: cleared in the B fragment
+            for (int v = 0; v < 4; ++v) {
+                const float av = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (4 * kg + v), __float_as_int(alpha[qt])));
 #pragma unroll
-        for (int ip = 0; ip < 2; ++ip) {
-            const int tk = tb + 32 * ip + 8 * kg;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) vm[ip][e] = (tk + 2 * e < ctx ? 0x0000FFFFu : 0u) | (tk + 2 * e + 1 < ctx ? 0xFFFF0000u : 0u);
+                for (int nt = 0; nt < NDT; ++nt) o[qt][nt][v] *= av;
+            }
         }
 #pragma unroll
         for (int nt = 0; nt < NDT; ++nt) {
@@ -567,13 +585,10 @@ __global__ void __launch_bounds__(256, 1) prefill_attn_lds_kernel(const PrefillP
 #pragma unroll
             for (int ip = 0; ip < 2; ++ip) {
                 vv[ip] = *reinterpret_cast<const uint4*>(Kb + pal_v_read_off(16 * nt + c, ip, kg));
-                vv[ip].x &= vm[ip][0]; vv[ip].y &= vm[ip][1]; vv[ip].z &= vm[ip][2]; vv[ip].w &= vm[ip][3];
             }
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
                 f32x4_t on = o[qt][nt];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) on[v] *= av[qt][v];
 #pragma unroll
                 for (int ip = 0; ip < 2; ++ip) {
                     on = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, pb[qt][ip]), __builtin_bit_cast(bf16x8_t, vv[ip]), on, 0, 0, 0);
@@ -640,27 +655,14 @@ extern "C" int mi355_prefill_attention(void* out, const void* q, const void* k, 
     const bool mfma_ok = (head_dim == 64 || head_dim == 128) && (src != SRC_PAGED || block_size % 16 == 0);
     if (g_pf_lds && src == SRC_PAGED && dtype == MI355_DTYPE_BF16 && head_dim == 128 &&
         (block_size == 16 || block_size == 32 || block_size == 64)) {
-        // round 4 default (first run on hardware in round 4: its tests green, prompt step 21.8 k -> 23.7 k tok/s at T = 2048): 64 queries x the
-        // heads of a GQA group per workgroup, K / V through the LDS ring
         static Mi355DevOnce attr_done;
         if (!attr_done.done()) {
-            (void)hipFuncSetAttribute((const void*)prefill_attn_lds_kernel<4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 32768);
-            (void)hipFuncSetAttribute((const void*)prefill_attn_lds_kernel<2, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 32768);
+            (void)hipFuncSetAttribute((const void*)prefill_attn_lds_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PFL_STAGES * 32768);
             attr_done.set();
         }
         const int G = num_heads / num_kv_heads, hgs = num_kv_heads * ((G + 3) / 4);
-        // 64 queries per workgroup when that still gives two workgroups per CU to hand out heaviest first; else 32 (ring of two stages).
-        // Measured (round 4, Llama-3-8B prompt step, one box): T = 2048 (256 workgroups of 64 queries = one round, the launch lasts as long
-        // as its heaviest block) 37.8 k -> 39.8 k tok/s with 32-query blocks; T = 4096 38.9 k either way -- and 34.7 k before the grid was
-        // ordered heaviest block first.
-        const int64_t nwg64 = (int64_t)((max_seqlen_q + 63) / 64) * hgs * num_seqs;
-        if (nwg64 >= 512) {
-            dim3 grid(hgs, (max_seqlen_q + 63) / 64, num_seqs);
-            hipLaunchKernelGGL((prefill_attn_lds_kernel<4, 4>), grid, dim3(256), 4 * 32768, st, p, block_tables, context_lens, cu_seqlens_q);
-        } else {
-            dim3 grid(hgs, (max_seqlen_q + 31) / 32, num_seqs);
-            hipLaunchKernelGGL((prefill_attn_lds_kernel<2, 2>), grid, dim3(256), 2 * 32768, st, p, block_tables, context_lens, cu_seqlens_q);
-        }
+        const dim3 grid(hgs, (max_seqlen_q + 16 * PFL_QT - 1) / (16 * PFL_QT), num_seqs);
+        hipLaunchKernelGGL(prefill_attn_lds_kernel, grid, dim3(256), PFL_STAGES * 32768, st, p, block_tables, context_lens, cu_seqlens_q);
         return (int)hipGetLastError();
     }
     if (mfma_ok) {
@@ -726,7 +728,7 @@ void mi355_prefill_set_fp8_generic(int v) { g_pf_fp8_generic = v; }
 
 // Round 6: the e4m3 cache blocks of the sequences of a prompt step as bf16 (exact: 3 mantissa bits), in the bf16 cache layouts
 // K [NBt, Hkv, D/8, bs, 8] / V [NBt, Hkv, D, bs], temp block seq * max_blocks + i, with the table that says so -- so that the step's attention
-// runs through prefill_attn_lds_kernel (K / V through the LDS ring: 290 TFLOP/s on the Llama prompt step) instead of the register-fed
+// runs through prefill_attn_lds_kernel (K / V through the LDS ring) instead of the register-fed
 // prefill_attn_kernel<.., SRC_PAGED8> (110 TFLOP/s, 51 % of a 16 k-token Mixtral prompt: profiles/r06_moe_prompt_device_ab.txt).  One pass
 // over ctx x Hkv x D x 2 bytes per layer (33 MB read, 67 MB written at 16 k tokens: ~25 us next to 10 ms of attention).
 __global__ void __launch_bounds__(256) pf_fp8_blocks_to_bf16_kernel(uint16_t* __restrict__ tk, uint16_t* __restrict__ tv, uint32_t* __restrict__ tbt,

@@ -180,6 +180,26 @@ def test_prefill_lds_dma_kernel(cv, H, Hkv, bs):
     assert np.abs(soft - soft_base).max() <= 2 ** -7 * max(1.0, np.abs(soft_base).max())
 
 
+@pytest.mark.parametrize("factor", [1.0, 6.0, -1.0, 0.0])
+def test_prefill_lds_stage_ends_and_scales(cv, factor):
+    """contexts that end at both sides of a stage of 64 keys and of a 32-query workgroup (slots behind them hold NaN patterns), long ones whose
+    running maximum stands still over whole stages, and scales that do not fit the exponent's multiply-add: sharp, negative, zero"""
+    dt, H, Hkv, D, bs = "bf16", 8, 2, 128, 16
+    rng = np.random.default_rng(5)
+    lens, cached = [1, 31, 32, 33, 63, 64, 65, 16, 40], [0, 32, 31, 31, 1, 64, 0, 700, 1111]
+    q, k_all, v_all, kc, vc, meta = make_case(rng, lens, cached, H, Hkv, D, bs, dt, False)
+    scale = factor / np.sqrt(D)
+    pa = cv.PagedAttention(H, D, scale, Hkv)
+    im = cv.InputMetadata.from_oracle_meta(meta, "cuda", is_prefill=True)
+    kcd, vcd = (torch.from_numpy(a.view(np.int16)).cuda().view(TD[dt]) for a in (kc, vc))
+    got = host16(pa.prefill(dev16(np.concatenate(q), dt), None, None, kcd, vcd, im), dt)
+    assert np.isfinite(got).all()
+    o = 0
+    for i, l in enumerate(lens):
+        ref = O.prefill_attention(q[i], k_all[i], v_all[i], scale, cached=cached[i], rnd=lambda a: G.round_dt(a, dt))
+        assert np.abs(got[o:o + l] - ref).max() <= TOL[dt] * max(1.0, np.abs(ref).max()), f"seq {i}"
+        o += l
+
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("flash", [True, False])
