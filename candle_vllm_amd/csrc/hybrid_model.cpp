@@ -80,9 +80,9 @@ struct HLayer {
     int a_conv_channels() const { return (c.a_heads + c.a_kv_heads) * c.a_dim + c.a_kv_heads * c.a_vdim; }
     // elements of a token's row in the key / value pages (latent attention: one row [latent | rotated key part], no value pages)
     // gate and up rows are stored interleaved by 16 so that the activation is the product's epilogue: the experts', and the dense
-    // feed-forward's where its activation is silu or gelu
+    // feed-forward's
     bool glu_experts() const { return c.mlp_kind == 3 && !c.moe_relu2 && c.mlp_ff % 16 == 0; }
-    bool glu_dense() const { return (c.mlp_kind == 2 || c.mlp_kind == 6) && c.mlp_ff % 16 == 0; }
+    bool glu_dense() const { return (c.mlp_kind == 1 || c.mlp_kind == 2 || c.mlp_kind == 6) && c.mlp_ff % 16 == 0; }
     // a shared expert of the experts' size runs as one more group of the grouped products (and one more pair of every token)
     bool shared_merged() const { return c.mlp_kind == 3 && c.moe_shared_ff > 0 && c.moe_shared_ff == c.mlp_ff; }
     int k_row() const { return is_latent() ? c.a_kv_rank + c.a_rot_dim : c.a_kv_heads * c.a_dim; }
@@ -783,6 +783,8 @@ static int forward_enqueue(HModel* m, const uint32_t* tokens, const int64_t* pos
     // gate, up and activation of a dense feed-forward (kinds 1, 2, 6)
     auto dense_gate_up = [&](const HLayer& WL) -> int {
         const int ff = WL.c.mlp_ff, kind = WL.c.mlp_kind;
+        if (WL.glu_dense() && kind == 1)
+            return mi355_hyb_linear_clamped_glu(m->act, dt, ff, xin, W, WL.w[MI355_HW_MLP_GATE_UP].p, T, ff, W, WL.c.mlp_limit, WL.c.mlp_alpha, dt, stream);
         if (WL.glu_dense())
             return mi355_hyb_linear_glu(m->act, dt, ff, xin, W, WL.w[MI355_HW_MLP_GATE_UP].p, T, ff, W, kind == 2 ? MI355_HYB_ACT_GELU : MI355_HYB_ACT_SILU, dt,
                                         stream);

@@ -561,6 +561,9 @@ int mi355_hyb_linear_segments(float* out, int32_t ldo, const void* a, int32_t a_
  * [T, ldo] = act(gate) up; a and w are both (dt) */
 int mi355_hyb_linear_glu(void* out, int32_t out_dtype, int32_t ldo, const void* a, int32_t lda, const void* w, int32_t num_tokens, int32_t ff,
                          int32_t k, int32_t act, int32_t dtype, int64_t stream);
+/* the same with mi355_hyb_clamped_glu's activation */
+int mi355_hyb_linear_clamped_glu(void* out, int32_t out_dtype, int32_t ldo, const void* a, int32_t lda, const void* w, int32_t num_tokens, int32_t ff,
+                                 int32_t k, float limit, float alpha, int32_t dtype, int64_t stream);
 /* the same per block of a table (mi355_hyb_linear_grouped) */
 int mi355_hyb_linear_grouped_glu(void* out, int32_t out_dtype, int32_t ldo, const void* a, int32_t lda, const int32_t* row_token, const void* w,
                                  int64_t w_bs, const int32_t* block_table, int32_t block_rows, int32_t n_blocks, int32_t ff, int32_t k, int32_t act,

@@ -97,6 +97,47 @@ def test_norm_add_and_glu(lib):
     assert np.abs(out.cpu().numpy() - H.clamped_glu(g32[:, :ff], g32[:, ff:], 1.5, 1.702)).max() < 2e-6
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("T,ff,k", [(3, 16, 24), (1, 48, 2080), (12, 160, 2048), (20, 80, 40), (50, 112, 33), (130, 144, 64), (200, 64, 96), (65, 16, 32)])
+def test_clamped_gate_and_up_in_one_product(lib, dtype, T, ff, k):
+    """interleaved gate and up rows with the clamped activation behind the product, every product kernel, values on both sides of the limit, results in
+    f32 or bf16 -- against 64 bits.  An f32 sum of k products is within 3e-5 of the largest value; the activation's slope is at most 1.1 times (limit + 1) here"""
+    _gpu()
+    rng = np.random.default_rng(ff + k)
+    rnd = (lambda v: v.astype(np.float32).astype(np.float64)) if dtype == F32 else H.bf16_round
+    a, w = rnd(rng.standard_normal((T, k + 8))), rnd(rng.standard_normal((2 * ff, k)) * 1.5 / math.sqrt(k))
+    il, dw, da = dev_dt(np.zeros((2 * ff, k)), dtype), dev_dt(w, dtype), dev_dt(a, dtype)
+    ok(lib.mi355_hyb_interleave_gate_up(il.data_ptr(), dw.data_ptr(), 1, ff, k, dtype, _st()))
+    z = a[:, :k] @ w.T
+    want = H.clamped_glu(z[:, :ff], z[:, ff:], 1.25, 1.702)
+    for out_dt in ((F32,) if dtype == F32 else (F32, BF16)):
+        out = dev_dt(np.zeros((T, ff + 3)), out_dt)
+        ok(lib.mi355_hyb_linear_clamped_glu(out.data_ptr(), out_dt, ff + 3, da.data_ptr(), k + 8, il.data_ptr(), T, ff, k, 1.25, 1.702, dtype, _st()))
+        got = host_dt(out, out_dt)
+        assert np.abs(got[:, :ff] - want).max() < (8e-5 if out_dt == F32 else 8e-3) * max(1.0, np.abs(want).max()) and (got[:, ff:] == 0).all(), out_dt
+    assert lib.mi355_hyb_linear_clamped_glu(il.data_ptr(), dtype, ff, il.data_ptr(), k, il.data_ptr(), T, ff + 8, k, 1.25, 1.702, dtype, _st()) != 0
+
+
+@pytest.mark.parametrize("T,W,ld,skew", [(3, 4, 4, 0), (2, 1024, 1028, 0), (2, 1028, 1028, 0), (1, 2048, 2052, 0), (2, 3076, 3076, 0), (2, 4096, 4100, 0),   # one to four per thread
+                                         (2, 4100, 4100, 0), (2, 1022, 1024, 0), (2, 1024, 1026, 0), (2, 1024, 1024, 1)])                               # an element at a time
+@pytest.mark.parametrize("copy", [False, True])
+def test_norm_add_widths(lib, T, W, ld, skew, copy):
+    """the residual norm four elements at a time and one at a time, at the ends of their widths, with and without the bf16 copy; nothing beyond a row.
+    (an f32 sum of W squares and a handful of rounded operations on values of at most 8: 5e-6)"""
+    _gpu()
+    rng = np.random.default_rng(W + ld)
+    f = lambda *n: rng.standard_normal(n).astype(np.float32)                # noqa: E731
+    x, y, w = f(T, W), 3 * f(T, ld), f(W)
+    dx, dy, dw = torch.empty(T * W + 5, device="cuda").fill_(7.0), dev(np.concatenate([np.zeros(skew), y.ravel()])), dev(w)
+    dx[:T * W] = dev(x).view(-1)
+    xc = torch.zeros((T, W), dtype=torch.int16, device="cuda")
+    ok(lib.mi355_hyb_norm_add(dx.data_ptr(), xc.data_ptr() if copy else None, dy[skew:].data_ptr(), ld, dw.data_ptr(), T, W, 1e-5, _st()))
+    want = x + H.rms_norm(y[:, :W].astype(np.float64), w.astype(np.float64), 1e-5)
+    assert np.abs(dx[:T * W].cpu().numpy().reshape(T, W) - want).max() < 5e-6 and bool((dx[T * W:] == 7).all())
+    if copy:
+        assert np.array_equal(xc.cpu().numpy().view(np.uint16), bits(dx[:T * W].cpu().numpy().reshape(T, W)))
+
+
 def _paged(k, v, block_size, rng, n_blocks):
     """scatter k [Tk, G, d], v [Tk, G, vd] of one sequence into shuffled pages -> (k_pages, v_pages, block table, slot mapping)"""
     Tk = k.shape[0]
