@@ -494,6 +494,40 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* x, uint16_t* xcopy
     }
 }
 
+// The same, four elements at a time, V of them per thread (width <= 1024 V): y, x and w are requested together, so that a launch is one round trip
+// to memory and the sum.  (y, then x and w behind the sum, y a second time, took 7.3 us for 8 tokens of width 2048 and 20.3 for 2100; now 4.6 and 11.5).
+template <int V> __global__ __launch_bounds__(256) void norm_add4_kernel(float* x, uint16_t* xcopy, const float* y, int ldy, const float* w, int width, float eps) {
+    __shared__ float red[4];
+    const int t = blockIdx.x;
+    f32x4_t yv[V], xv[V], wv[V];
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const int i = (j * 256 + (int)threadIdx.x) * 4;
+        yv[j] = xv[j] = wv[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (i >= width) continue;
+        yv[j] = *reinterpret_cast<const f32x4_t*>(y + (size_t)t * ldy + i);
+        xv[j] = *reinterpret_cast<const f32x4_t*>(x + (size_t)t * width + i);
+        wv[j] = *reinterpret_cast<const f32x4_t*>(w + i);
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss += yv[j][e] * yv[j][e];
+    ss = block_sum(ss, red);
+    const float inv = 1.f / sqrtf(ss / (float)width + eps);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const int i = (j * 256 + (int)threadIdx.x) * 4;
+        if (i >= width) continue;
+        f32x4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = xv[j][e] + yv[j][e] * inv * wv[j][e];
+        *reinterpret_cast<f32x4_t*>(x + (size_t)t * width + i) = v;
+        if (xcopy) *reinterpret_cast<uint2*>(xcopy + (size_t)t * width + i) = make_uint2(cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]));
+    }
+}
+
 // rows[r] of x -> RMS norm with weight -> out (dt) [n_rows, width]   (the model's last norm, on the wanted rows only)
 template <typename TO> __global__ __launch_bounds__(256) void gather_norm_kernel(TO* out, const float* x, const int32_t* rows, const float* w, int width, float eps) {
     __shared__ float red[4];
@@ -1990,7 +2024,12 @@ int mi355_hyb_norm_add(float* x, void* xcopy, const float* y, int32_t ldy, const
                        int64_t stream) {
     if (!x || !y || !w || width <= 0 || ldy < width) return -1;
     if (T <= 0) return 0;
-    norm_add_kernel<<<T, 256, 0, to_stream(stream)>>>(x, (uint16_t*)xcopy, y, ldy, w, width, eps);
+    if (width <= 4096 && ((width | ldy) & 3) == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w) & 15) == 0 && ((uintptr_t)xcopy & 7) == 0) {
+        const int v = (width + 1023) / 1024;
+#define NORM_ADD_GO(V) norm_add4_kernel<V><<<T, 256, 0, to_stream(stream)>>>(x, (uint16_t*)xcopy, y, ldy, w, width, eps)
+        if (v == 1) NORM_ADD_GO(1); else if (v == 2) NORM_ADD_GO(2); else if (v == 3) NORM_ADD_GO(3); else NORM_ADD_GO(4);
+#undef NORM_ADD_GO
+    } else norm_add_kernel<<<T, 256, 0, to_stream(stream)>>>(x, (uint16_t*)xcopy, y, ldy, w, width, eps);
     LAUNCH_OK(); return 0;
 }
 
