@@ -304,6 +304,40 @@ def test_conv_silu_portions_and_state(lib, taps):
     assert np.abs(np.concatenate(got_b) - want_b).max() < 5e-6
 
 
+@pytest.mark.parametrize("C,T", [(1028, 1021), (12, 87383), (2048, 512)])
+@pytest.mark.parametrize("form", ["silu", "residual", "bias", "residual16"])
+def test_conv_rows_of_tokens(lib, C, T, form):
+    """the convolution that makes several tokens per thread equals the one of a value per thread (what an offset off the 16-byte grid takes) bit for bit:
+    sequences that begin and end inside a thread's tokens, of 1 .. 4 tokens and long ones, new ones and ones with 1, 2, 3 or more inputs in front"""
+    _gpu()
+    rng = np.random.default_rng(C)
+    lens, ctx = [], []
+    while sum(lens) < T:
+        n = int(rng.choice([1, 2, 3, 4, 5, 9, 40, 100]))
+        lens.append(min(n, T - sum(lens)))
+        ctx.append(lens[-1] + int(rng.choice([0, 0, 1, 2, 3, 50])))
+    n, taps, stride = len(lens), 4, C * 3 + 1
+    cu, sl = dev(np.concatenate([[0], np.cumsum(lens)]), np.int32), dev(rng.permutation(n), np.int32)
+    dctx, ts = dev(ctx, np.int32), torch.zeros(T, dtype=torch.int32, device="cuda")
+    ok(lib.mi355_hyb_token_seq(ts.data_ptr(), cu.data_ptr(), n, _st()))
+    u, w, b, state = dev(rng.standard_normal((T, C))), dev(rng.standard_normal((C, taps))), dev(rng.standard_normal(C)), dev(rng.standard_normal((n, stride)))
+    outs = []
+    for off in (4, 1):
+        proj = torch.zeros(T, C + 8, device="cuda")
+        proj[:, off:off + C] = u
+        out = torch.zeros(T, C, device="cuda", dtype=torch.bfloat16 if form == "residual16" else torch.float32)
+        where = (dctx.data_ptr(), cu.data_ptr(), sl.data_ptr(), ts.data_ptr(), n, T, C, taps)
+        if form == "silu":
+            ok(lib.mi355_hyb_conv_silu(out.data_ptr(), proj.data_ptr(), C + 8, off, w.data_ptr(), state.data_ptr(), stride, *where, _st()))
+        elif form == "bias":
+            ok(lib.mi355_hyb_conv_bias(out.data_ptr(), proj.data_ptr(), C + 8, off, w.data_ptr(), b.data_ptr(), state.data_ptr(), stride, *where, 1, _st()))
+        else:
+            ok(lib.mi355_hyb_conv_residual(out.data_ptr(), BF16 if form == "residual16" else F32, proj.data_ptr(), C + 8, off, w.data_ptr(), state.data_ptr(), stride,
+                                           *where, _st()))
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and bool((outs[0] != 0).any())
+
+
 @pytest.mark.parametrize("block_rows,blocks,n,tile", [(64, 5, 160, 4), (128, 3, 160, 3), (128, 130, 160, 2)])
 @pytest.mark.parametrize("k", [640, 704])
 @pytest.mark.parametrize("gather", [False, True])
