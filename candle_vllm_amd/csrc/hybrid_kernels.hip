@@ -1554,10 +1554,12 @@ template <typename TO, int UNR> __global__ __launch_bounds__(64) void mingru_ker
 
 // Long portions: S_t = (1 - z_t) S_(t-1) + z_t c_t is a composition of affine maps, so the portion is cut into NSEG segments, one wave
 // each: pass 1 reduces a segment to (A, B) with S_end = A S_start + B, the waves exchange (A, B) through LDS, every wave folds the
-// segments before its own into its starting state and walks its segment again writing the outputs.
-template <typename TO, int NSEG, int UNR> __global__ __launch_bounds__(64 * NSEG) void mingru_seg_kernel(GruArgs p) {
-    __shared__ float sA[NSEG][64], sB[NSEG][64];
-    const int s = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
+// segments before its own into its starting state and walks its segment again writing the outputs.  Bound by the five gates per value (each an exponential and
+// a division): LANES channels and NSEG segments per workgroup, so that a few sequences fill the card and a segment is short (two of 1050 tokens, width
+// 4096: 64 channels x 16 segments 133 us, 32 x 32 76).
+template <typename TO, int NSEG, int LANES, int UNR> __global__ __launch_bounds__(LANES * NSEG) void mingru_seg_kernel(GruArgs p) {
+    __shared__ float sA[NSEG][LANES], sB[NSEG][LANES];
+    const int s = blockIdx.y, lane = threadIdx.x % LANES, w = threadIdx.x / LANES, c = blockIdx.x * LANES + lane;
     const int tb = (int)p.cu_q[s], te = (int)p.cu_q[s + 1];
     if (te <= tb) return;
     const bool ok_ = c < p.width;
@@ -2384,8 +2386,14 @@ int mi355_hyb_mingru(void* out, int32_t out_dtype, float* state, int64_t state_s
     GruArgs p{out, state, state_stride, proj, ldp, z_off, x_off, g_off, context_lens, cu_seqlens_q, state_slots, width};
     const dim3 grid((width + 63) / 64, num_seqs);
     if (num_tokens >= 256) {                            // some portion may be long: segmented scan
-        if (out_dtype == MI355_DTYPE_F32) mingru_seg_kernel<float, 16, 4><<<grid, 1024, 0, to_stream(stream)>>>(p);
-        else mingru_seg_kernel<uint16_t, 16, 4><<<grid, 1024, 0, to_stream(stream)>>>(p);
+        // where 64 channels per workgroup do not fill the card and the sequences are long: 32.  us, 64 / 32 channels (sequences x tokens, width): 1 x 256, 1024
+        // 18.9 / 10.9, 8 x 256, 1024 20.0 / 12.6, 1 x 4096, 4096 277 / 142, 32 x 64, 256 6.8 / 5.5; 32 x 8, 256 4.2 / 5.7, 8 x 256, 4096 38.2 / 39.1, 64 x 16, 4096 33.5 / 45.7
+        if ((int64_t)grid.x * num_seqs <= mi355_num_cus() && num_tokens >= 64 * (int64_t)num_seqs) {
+            const dim3 narrow((width + 31) / 32, num_seqs);
+            if (out_dtype == MI355_DTYPE_F32) mingru_seg_kernel<float, 32, 32, 4><<<narrow, 1024, 0, to_stream(stream)>>>(p);
+            else mingru_seg_kernel<uint16_t, 32, 32, 4><<<narrow, 1024, 0, to_stream(stream)>>>(p);
+        } else if (out_dtype == MI355_DTYPE_F32) mingru_seg_kernel<float, 16, 64, 4><<<grid, 1024, 0, to_stream(stream)>>>(p);
+        else mingru_seg_kernel<uint16_t, 16, 64, 4><<<grid, 1024, 0, to_stream(stream)>>>(p);
         LAUNCH_OK(); return 0;
     }
     if (out_dtype == MI355_DTYPE_F32) mingru_kernel<float, 8><<<grid, 64, 0, to_stream(stream)>>>(p);
