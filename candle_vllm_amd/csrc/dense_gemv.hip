@@ -1466,7 +1466,7 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     const int max_split = n == 1 && a[0].T <= 65535 && !(a[0].N & 3) && !(a[0].epi == MI355_EPI_SILU_MUL && (a[0].pair_offset & 3)) ? gemm_max_split(a[0], std::max(1, units / 8)) : 1;
     const float weights_us = (float)rows * (float)a[0].K * 2.f / 5.4e6f;
     GtChoice best = gt_pick([&](const GtTile& t) { return tiles(t, nullptr); }, units, weights_us, max_split,
-                            (float)a[0].T * (float)a[0].N * 4.f / 4.5e6f, 31);
+                            (float)a[0].T * (float)a[0].N * 4.f / 4.5e6f, 63);
     if (n == 1 && g_tune_gemm_min_t == DENSE_GEMM_MIN_T && !g_tune_gemm_tall && dense_streams(a[0], best, weights_us)) return (int)hipErrorNotSupported;
     if (g_tune_gemm_tall) best = {0, 1, 0.f};
     DenseGemm3 g{};

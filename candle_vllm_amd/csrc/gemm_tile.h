@@ -174,23 +174,28 @@ struct GemmTile {
 // ---- which tile.  us: a unit of 64 k of one round (per_cu workgroups on every CU); the launch takes the tile and K split whose rounds end
 // first, never below the time of the weights' stream from HBM.  The 64- and 128-token tiles of one workgroup per CU have six and four
 // buffers: where a launch is a stream over the weights, what counts is the bytes under way.
+// 192 x 128 is for the launches whose 128 x 128 tiles are a little more than one per CU, which 256 x 256 ones leave half empty.  us, two 128 x 128
+// per CU / one 192 x 128 (f32 results): 2100 x 2048 x 2048 29.3 / 25.3, x 6144 73.8 / 59.2; 1100 x 4096 x 4096 50.1 / 44.4; 300 x 14336 x 4096 64.9 / 49.0;
+// where its second round is not full the pick stays: 1100 x 9216 x 2048 192 x 256 44.4 / 50.9, 1100 x 14336 x 4096 135.5 / 144.2.  From 16 units (k >= 1024) on:
+// below, a launch is mostly its start and its stores (2100 x 2048 x 128 9.3 / 8.5, x 704 15.7 / 13.2).  256 x 128 as a seventh tile won nowhere by more than 2 %.
 struct GtTile { int bm, bn, per_cu; float us; };
-static constexpr GtTile kGtTiles[] = {{256, 256, 1, 1.46f}, {192, 256, 1, 1.28f}, {128, 128, 2, 0.93f}, {128, 128, 1, 0.5f}, {64, 128, 1, 0.42f}};
-// CALL with the five tiles' template arguments, by number
+constexpr int GT_NARROW = 5;
+static constexpr GtTile kGtTiles[] = {{256, 256, 1, 1.46f}, {192, 256, 1, 1.28f}, {128, 128, 2, 0.93f}, {128, 128, 1, 0.5f}, {64, 128, 1, 0.42f}, {192, 128, 1, 0.72f}};
+// CALL with the six tiles' template arguments, by number
 #define GT_TILES(which, CALL) do { switch (which) { \
     case 0: CALL(2, 4, 8, 4, 2); break; case 1: CALL(2, 4, 6, 4, 2); break; case 2: CALL(2, 4, 4, 2, 2); break; \
-    case 3: CALL(2, 4, 4, 2, 4); break; default: CALL(2, 4, 2, 2, 6); break; } } while (0)
+    case 3: CALL(2, 4, 4, 2, 4); break; case 4: CALL(2, 4, 2, 2, 6); break; default: CALL(4, 2, 3, 4, 4); break; } } while (0)
 struct GtChoice { int tile, splits; float us; };
 // tile and K ranges of this thread's last launch, 100 tile + ranges (tests: mi355_internal_last_gemm)
 inline thread_local int gt_last_launch = -1;
 // tiles(t): workgroups of the launch with tile t; stream_us: the weights' read; part_us: write or read of one range's partial sums
 template <class F>
-static inline GtChoice gt_pick(F tiles, int units, float stream_us, int max_split, float part_us, unsigned allowed, const GtTile* table = kGtTiles, int n_table = 5) {
+static inline GtChoice gt_pick(F tiles, int units, float stream_us, int max_split, float part_us, unsigned allowed, const GtTile* table = kGtTiles, int n_table = 6) {
     const int cus = mi355_num_cus();
     GtChoice best{-1, 1, 0.f};
     for (int i = 0; i < n_table; ++i)
         for (int s = 1; s <= max_split; ++s) {
-            if (!(allowed >> i & 1)) continue;
+            if (!(allowed >> i & 1) || (i == GT_NARROW && units < 16)) continue;
             const int64_t wgs = (int64_t)cus * table[i].per_cu, rounds = (tiles(table[i]) * s + wgs - 1) / wgs;
             const float t = (float)rounds * (float)((units + s - 1) / s + 2) * table[i].us;
             const float c = (t > stream_us ? t : stream_us) + (s > 1 ? 5.f + part_us * (float)(s + 1) : 0.f);

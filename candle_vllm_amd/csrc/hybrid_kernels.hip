@@ -2036,7 +2036,7 @@ static int linear_launch(float* out, int32_t ldo, int64_t o_bs, const void* a, i
     } else if (linear_gemm_ok(p, af)) {
         // (segments end at multiples of 128 columns: only the tiles of that width have one left operand each)
         const GtChoice c = gt_pick([&](const GtTile& t) { return (int64_t)((T + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch; }, k / 64,
-                                   (float)n * (float)k * 2.f * (float)batch / 5.4e6f, 1, 0.f, seg ? 28 : 31);
+                                   (float)n * (float)k * 2.f * (float)batch / 5.4e6f, 1, 0.f, seg ? 60 : 63);
         LIN_EPI(p, (linear_gemm_launch<EPI>(p, c.tile, (T + kGtTiles[c.tile].bm - 1) / kGtTiles[c.tile].bm, nz, st_)));
     } else if (T > 32 && !af && p.a_vec && p.w_vec && k % 32 == 0) {
         LIN_EPI(p, (linear_bf16_lds_kernel<EPI><<<dim3((n + 127) / 128, (T + 127) / 128, nz), 256, 0, st_>>>(p)));

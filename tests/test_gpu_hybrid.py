@@ -401,6 +401,30 @@ def test_segmented_products_of_many_units(lib, T, segs, tile):
     assert float((out.double() - want).abs().max()) < 3e-5 * max(1.0, float(want.abs().max()))
 
 
+@pytest.mark.parametrize("T,segs,k", [(1153, (3072, 1024), 1024), (2100, (2048,), 2048)])
+def test_products_of_tall_narrow_tiles(lib, T, segs, k):
+    """the 192 x 128 tile: one token into its last tile and a ragged last one; a plain product, an activation, gate and up, column segments -- against 64 bits"""
+    _gpu()
+    gen, n = torch.Generator(device="cuda").manual_seed(T), sum(segs)
+    a = torch.randn(len(segs), T, k + 8, device="cuda", generator=gen).to(torch.bfloat16)
+    w, b = (torch.randn(n, k, device="cuda", generator=gen) / math.sqrt(k)).to(torch.bfloat16), torch.randn(n, device="cuda", generator=gen)
+    rows, ends, silu = np.array(segs, np.int32), np.cumsum((0,) + segs), torch.nn.functional.silu
+    z = a[0, :, :k].double() @ w.double().t()
+    zs = torch.cat([a[i, :, :k].double() @ w[ends[i]:ends[i + 1]].double().t() for i in range(len(segs))], 1)
+    head = (a.data_ptr(), BF16, k + 8)
+    out = torch.empty(T, n, device="cuda")
+    for want, call in ((z + b.double(), lambda: lib.mi355_hyb_linear(out.data_ptr(), n, *head, w.data_ptr(), b.data_ptr(), T, n, k, BF16, _st())),
+                       (zs + b.double(), lambda: lib.mi355_hyb_linear_segments(out.data_ptr(), n, *head, T * (k + 8), 0, w.data_ptr(), b.data_ptr(), rows.ctypes.data,
+                                                                               len(segs), T, n, k, BF16, _st())),
+                       ((silu(z.view(T, -1, 2, 16)[:, :, 0]) * z.view(T, -1, 2, 16)[:, :, 1]).reshape(T, -1),
+                        lambda: lib.mi355_hyb_linear_glu(out.data_ptr(), F32, n, a.data_ptr(), k + 8, w.data_ptr(), T, n // 2, k, 1, BF16, _st()))):
+        out.fill_(7.0)
+        ok(call())
+        assert lib.mi355_internal_last_gemm() == 501                        # 100 tile + K ranges
+        got = out[:, :want.shape[1]]
+        assert float((got.double() - want).abs().max()) < 3e-5 * max(1.0, float(want.abs().max())) and bool((out[:, want.shape[1]:] == 7).all())
+
+
 @pytest.mark.parametrize("Hh,G,d,vd,per_channel", [(2, 1, 32, 32, False), (3, 3, 20, 70, True), (4, 2, 64, 16, True), (1, 1, 128, 300, False),
                                                   (2, 2, 136, 64, True)])
 def test_delta_rule_portions_and_state(lib, Hh, G, d, vd, per_channel):

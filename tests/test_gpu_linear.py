@@ -68,6 +68,33 @@ def test_linear_matches_oracle(cv, dt, T, N, K):
               mag=G.linear16(x, w, None, dt))
 
 
+@pytest.mark.parametrize("T,N,K,epi", [(1153, 4096, 1024, 0), (2100, 2050, 2048, 0), (1344, 4080, 1280, 1), (1345, 4096, 1024, 2)])
+def test_linear_prompt_gemm_tall_narrow_tile(cv, T, N, K, epi):
+    """the prompt GEMM's 192 x 128 tile: one token into the last tile, ragged tokens and rows, each epilogue; row-major and tiled weights alike bit for bit, and
+    the sums within the op's bound of the oracle at the tiles' edges"""
+    from candle_vllm_amd._lib import lib
+    dt, st = "bf16", torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(T + N)
+    x, w, res = G.round_dt(rng.normal(0, 1, (T, K)), dt), G.round_dt(rng.normal(0, 0.05, (N, K)), dt), G.round_dt(rng.normal(0, 1, (T, N)), dt)
+    xd, wd, rd = dev16(x, dt), dev16(w, dt), dev16(res, dt)
+    images, outs = [(lib.mi355_linear, wd)], []
+    if N % 16 == 0 and K % 256 == 0:
+        images.append((lib.mi355_linear_tiled, torch.empty_like(wd)))
+        assert lib.mi355_dense_tile_repack(wd.data_ptr(), images[1][1].data_ptr(), N, K, K, st) == 0
+    for fn, img in images:
+        out = torch.full((T, N // 2 if epi == 2 else N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert fn(out.data_ptr(), xd.data_ptr(), img.data_ptr(), None, rd.data_ptr() if epi == 1 else None, T, N, K, 2, epi, st) == 0
+        assert lib.mi355_internal_last_gemm() == 501              # 100 tile + K ranges
+        outs.append(host16(out, dt))
+    assert all(np.array_equal(outs[0], o) for o in outs) and np.isfinite(outs[0]).all()
+    rows = np.unique([t for e in range(0, T, 192) for t in (e, e + 1, e + 95, e + 191, T - 1) if t < T])
+    y = G.linear16(x[rows], w, None, dt)
+    if epi == 2:
+        check_ulp(outs[0][rows], G.silu_mul16(y[:, :N // 2], y[:, N // 2:], dt), dt, ulps=3.0, what="silu(gate)*up")
+    else:
+        check_ulp(outs[0][rows], G.round_dt(y + res[rows], dt) if epi == 1 else y, dt, what="linear", ulps=2.01, mag=y)
+
+
 @pytest.mark.parametrize("T,N,K,launch", [(33, 288, 2304, 404), (65, 160, 4096, 408),          # 64-token tiles, K in 4 and 8 ranges; one token into the next tile
                                           (130, 96, 8192, 416),                                # K in 16 ranges over three token tiles
                                           (900, 8192, 128, 201),                               # 128 x 128 tiles, exactly two per CU
