@@ -87,6 +87,7 @@ struct DModel {
     void* comm = nullptr;                 // borrowed communicator (tp_world > 1, or a 1-rank plumbing test)
     uint16_t* lg_gather = nullptr;        // [W, B, V/W]
     // greedy decode loop on static device buffers (mi355_dense_decode_*): step inputs, sampled tokens, f32 logits
+    StepInputs in;                        // (the next pointers but d_next lead into it)
     uint32_t *d_tokens = nullptr, *d_ctx = nullptr, *d_bt = nullptr, *d_next = nullptr;
     int64_t *d_positions = nullptr, *d_slots = nullptr;
     float* d_logits = nullptr;
@@ -297,8 +298,8 @@ void mi355_dense_destroy(void* mp) {
         if (kv.second.graph) (void)hipGraphDestroy(kv.second.graph);
     }
     void* ps[] = {m->tok_embd, m->output_norm, m->output_norm_b, m->output, m->cos_t, m->sin_t, m->xs, m->xn, m->q, m->k, m->v, m->attn,
-                  m->h, m->lg16, m->pa_tmp, m->pa_max, m->pa_sum, m->ss, m->kv_slab, m->lg_gather, m->d_tokens, m->d_ctx, m->d_bt,
-                  m->d_next, m->d_positions, m->d_slots, m->d_logits};
+                  m->h, m->lg16, m->pa_tmp, m->pa_max, m->pa_sum, m->ss, m->kv_slab, m->lg_gather, m->d_next, m->d_logits};
+    m->in.destroy();
     for (void* p : ps) if (p) (void)hipFree(p);
     delete m;
 }
@@ -657,32 +658,26 @@ int mi355_dense_decode_begin(void* mp, const uint32_t* tokens_host, const uint32
         return (int)hipErrorInvalidValue;
     const mi355_dense_config& c = m->cfg;
     const int bs = c.block_size, W = c.tp_world > 1 ? c.tp_world : 1;
-    std::vector<int64_t> pos(batch), slot(batch);
     int ctx_max = 0;
     for (int b = 0; b < batch; ++b) {
         if (seq_lens_host[b] < 1) return (int)hipErrorInvalidValue;
-        pos[b] = (int64_t)seq_lens_host[b] - 1;
-        if (pos[b] / bs >= max_blocks) return (int)hipErrorInvalidValue;          // "Block table is too small"
-        slot[b] = (int64_t)block_tables_host[(size_t)b * max_blocks + pos[b] / bs] * bs + pos[b] % bs;
+        if (((int64_t)seq_lens_host[b] - 1) / bs >= max_blocks) return (int)hipErrorInvalidValue;          // "Block table is too small"
         ctx_max = std::max(ctx_max, (int)seq_lens_host[b]);
     }
     if (ctx_cap < ctx_max || ctx_cap > c.max_seq || ctx_max > max_blocks * bs) return (int)hipErrorInvalidValue;
     if (!m->d_tokens) {
         const size_t B = c.max_batch;
-        DHIP(hipMalloc((void**)&m->d_tokens, B * 4)); DHIP(hipMalloc((void**)&m->d_ctx, B * 4)); DHIP(hipMalloc((void**)&m->d_next, B * 4));
-        DHIP(hipMalloc((void**)&m->d_bt, B * c.max_blocks_per_seq * 4));
-        DHIP(hipMalloc((void**)&m->d_positions, B * 8)); DHIP(hipMalloc((void**)&m->d_slots, B * 8));
-        DHIP(hipMalloc((void**)&m->d_logits, B * (size_t)c.vocab * W * 4));
+        if (!m->d_next) DHIP(hipMalloc((void**)&m->d_next, B * 4));
+        if (!m->d_logits) DHIP(hipMalloc((void**)&m->d_logits, B * (size_t)c.vocab * W * 4));
+        if (!m->in.create(c.max_batch, c.max_blocks_per_seq)) { m->in.destroy(); return (int)hipErrorOutOfMemory; }
+        m->d_ctx = m->in.ctx(m->in.dev); m->d_bt = m->in.tables(m->in.dev);
+        m->d_positions = m->in.positions(m->in.dev); m->d_slots = m->in.slots(m->in.dev);
+        m->d_tokens = m->in.tokens(m->in.dev);
     }
     DCHECK(ensure_cap(m, batch));                          // everything that allocates happens here, never inside a captured step
     DCHECK(finalize_weights(m));
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    DHIP(hipMemcpyAsync(m->d_tokens, tokens_host, (size_t)batch * 4, hipMemcpyHostToDevice, st));
-    DHIP(hipMemcpyAsync(m->d_ctx, seq_lens_host, (size_t)batch * 4, hipMemcpyHostToDevice, st));
-    DHIP(hipMemcpyAsync(m->d_bt, block_tables_host, (size_t)batch * max_blocks * 4, hipMemcpyHostToDevice, st));
-    DHIP(hipMemcpyAsync(m->d_positions, pos.data(), (size_t)batch * 8, hipMemcpyHostToDevice, st));
-    DHIP(hipMemcpyAsync(m->d_slots, slot.data(), (size_t)batch * 8, hipMemcpyHostToDevice, st));
-    DHIP(hipStreamSynchronize(st));                        // host vectors go out of scope
+    DHIP(m->in.send(tokens_host, seq_lens_host, block_tables_host, batch, max_blocks, bs, st));
     m->cur_batch = batch; m->cur_max_blocks = max_blocks; m->cur_ctx_cap = ctx_cap; m->cur_ctx_max = ctx_max;
     return 0;
 }
@@ -701,6 +696,7 @@ int mi355_dense_decode_step(void* mp, int64_t stream) {
     DModel* m = static_cast<DModel*>(mp);
     if (!m || m->cur_batch < 1) return (int)hipErrorInvalidValue;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    DHIP(m->in.use_on(st));
     // this step attends over cur_ctx_max tokens, then advance_kernel looks up the slot of position cur_ctx_max: both must stay
     // inside the attention grid (ctx_cap), the block-table row and the RoPE tables
     if (m->cur_ctx_max > m->cur_ctx_cap || m->cur_ctx_max > m->cfg.max_seq ||
@@ -760,12 +756,11 @@ int mi355_dense_decode_read_tokens(void* mp, uint32_t* host_out, int64_t stream)
     DModel* m = static_cast<DModel*>(mp);
     if (!m || !host_out || m->cur_batch < 1) return (int)hipErrorInvalidValue;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    DHIP(hipMemcpyAsync(host_out, m->d_tokens, (size_t)m->cur_batch * 4, hipMemcpyDeviceToHost, st));
     uint32_t p2p_err = 0;
     const Comm* cm = static_cast<const Comm*>(m->comm);
     const bool p2p = cm && cm->p2p && cm->local;
     if (p2p) DHIP(hipMemcpyAsync(&p2p_err, &cm->local->err, 4, hipMemcpyDeviceToHost, st));
-    DHIP(hipStreamSynchronize(st));
+    DHIP(m->in.read_tokens(host_out, m->cur_batch, st));
     if (p2p && p2p_err != 0) return (int)hipErrorPeerAccessNotEnabled;     // a peer missed the spin bound: the step is invalid on this rank
     return 0;
 }

@@ -76,7 +76,8 @@ struct Model {
     void* kv_slab = nullptr;
     std::vector<void*> kcache, vcache;
     int num_blocks = 0;
-    // static step inputs (graph mode)
+    // static step inputs (graph mode); the pointers lead into `in`
+    StepInputs in;
     uint32_t* d_tokens = nullptr;
     int64_t* d_positions = nullptr;
     int64_t* d_slots = nullptr;
@@ -717,11 +718,9 @@ extern "C" void* mi355_llama_create(const mi355_llama_config* cfg) {
     alloc((void**)&m->pa_tmp, (size_t)B * H * m->pa_cap_partitions * D * 4);
     alloc((void**)&m->pa_max, (size_t)B * H * m->pa_cap_partitions * 4);
     alloc((void**)&m->pa_sum, (size_t)B * H * m->pa_cap_partitions * 4);
-    alloc((void**)&m->d_tokens, (size_t)B * 4);
-    alloc((void**)&m->d_positions, (size_t)B * 8);
-    alloc((void**)&m->d_slots, (size_t)B * 8);
-    alloc((void**)&m->d_ctx, (size_t)B * 4);
-    alloc((void**)&m->d_bt, (size_t)B * cfg->max_blocks_per_seq * 4);
+    if (!m->in.create(B, cfg->max_blocks_per_seq)) ok = false;
+    m->d_tokens = m->in.tokens(m->in.dev); m->d_ctx = m->in.ctx(m->in.dev); m->d_bt = m->in.tables(m->in.dev);
+    m->d_positions = m->in.positions(m->in.dev); m->d_slots = m->in.slots(m->in.dev);
     // RoPE tables (rotary_emb.rs:14-48): inv_freq f32, idx_theta = pos(f32) * inv_freq(f32), cos/sin in f32
     const int half = D / 2;
     std::vector<float> ct((size_t)cfg->max_seq * half), stb((size_t)cfg->max_seq * half);
@@ -770,9 +769,9 @@ extern "C" void mi355_llama_destroy(void* mp) {
     }
     free_qw(m->output);
     void* ptrs[] = {m->tok_embd, m->output_norm, m->cos_t, m->sin_t, m->xs, m->q, m->attn, m->h, m->logits,
-                    m->pa_tmp, m->pa_max, m->pa_sum, m->kv_slab, m->d_tokens, m->d_positions, m->d_slots,
-                    m->d_ctx, m->d_bt, m->logits_local, m->logits_gather, m->tp_y, m->p_tp_y, m->p_moe_xg, m->p_moe_perm, m->p_moe_inv, m->p_moe_tab, m->p_xs, m->p_q, m->p_attn, m->p_h,
+                    m->pa_tmp, m->pa_max, m->pa_sum, m->kv_slab, m->logits_local, m->logits_gather, m->tp_y, m->p_tp_y, m->p_moe_xg, m->p_moe_perm, m->p_moe_inv, m->p_moe_tab, m->p_xs, m->p_q, m->p_attn, m->p_h,
                     m->moe_ids, m->moe_w, m->moe_y, m->p_moe_ids, m->p_moe_w, m->p_moe_y, m->chain_sync, m->g_moe_xg, m->g_moe_h, m->g_moe_yg, m->g_moe_pos, m->g_moe_cnt};
+    m->in.destroy();
     if (m->comm && m->comm_owned) mi355_comm_destroy(m->comm);
     for (void* p : ptrs) if (p) (void)hipFree(p);
     delete m;
@@ -988,24 +987,16 @@ extern "C" int mi355_llama_decode_begin(void* mp, const uint32_t* tokens_host, c
     if (!m || batch < 1 || batch > m->cfg.max_batch || max_blocks < 1 || max_blocks > m->cfg.max_blocks_per_seq)
         return (int)hipErrorInvalidValue;
     const int bs = m->cfg.block_size;
-    std::vector<int64_t> pos(batch), slot(batch);
     for (int b = 0; b < batch; ++b) {
         if (seq_lens_host[b] < 1) return (int)hipErrorInvalidValue;
-        pos[b] = (int64_t)seq_lens_host[b] - 1;
-        if (pos[b] / bs >= max_blocks) return (int)hipErrorInvalidValue;          // "Block table is too small"
-        slot[b] = (int64_t)block_tables_host[(size_t)b * max_blocks + pos[b] / bs] * bs + pos[b] % bs;
+        if (((int64_t)seq_lens_host[b] - 1) / bs >= max_blocks) return (int)hipErrorInvalidValue;          // "Block table is too small"
     }
     // the greedy loop advances the context on the device: everything it will index is checked here and in decode_step
     int ctx_max = 0;
     for (int b = 0; b < batch; ++b) ctx_max = std::max(ctx_max, (int)seq_lens_host[b]);
     if (ctx_cap < ctx_max || ctx_cap > m->cfg.max_seq || ctx_max > max_blocks * bs) return (int)hipErrorInvalidValue;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    HCHECK(hipMemcpyAsync(m->d_tokens, tokens_host, (size_t)batch * 4, hipMemcpyHostToDevice, st));
-    HCHECK(hipMemcpyAsync(m->d_ctx, seq_lens_host, (size_t)batch * 4, hipMemcpyHostToDevice, st));
-    HCHECK(hipMemcpyAsync(m->d_bt, block_tables_host, (size_t)batch * max_blocks * 4, hipMemcpyHostToDevice, st));
-    HCHECK(hipMemcpyAsync(m->d_positions, pos.data(), (size_t)batch * 8, hipMemcpyHostToDevice, st));
-    HCHECK(hipMemcpyAsync(m->d_slots, slot.data(), (size_t)batch * 8, hipMemcpyHostToDevice, st));
-    HCHECK(hipStreamSynchronize(st));                     // host vectors go out of scope
+    HCHECK(m->in.send(tokens_host, seq_lens_host, block_tables_host, batch, max_blocks, bs, st));
     m->cur_batch = batch; m->cur_max_blocks = max_blocks; m->cur_ctx_cap = ctx_cap; m->cur_ctx_max = ctx_max;
     return 0;
 }
@@ -1053,6 +1044,7 @@ extern "C" int mi355_llama_decode_step(void* mp, int64_t stream) {
     Model* m = static_cast<Model*>(mp);
     if (!m || m->cur_batch < 1) return (int)hipErrorInvalidValue;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    HCHECK(m->in.use_on(st));
     // this step attends over cur_ctx_max tokens, then `advance_kernel` looks up the slot of position cur_ctx_max: both
     // must stay inside the attention grid (ctx_cap), the block-table row and the RoPE tables
     if (m->cur_ctx_max > m->cur_ctx_cap || m->cur_ctx_max > m->cfg.max_seq ||
@@ -1119,13 +1111,12 @@ extern "C" int mi355_llama_decode_read_tokens(void* mp, uint32_t* host_out, int6
     Model* m = static_cast<Model*>(mp);
     if (!m || m->cur_batch < 1) return (int)hipErrorInvalidValue;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    HCHECK(hipMemcpyAsync(host_out, m->d_tokens, (size_t)m->cur_batch * 4, hipMemcpyDeviceToHost, st));
     // the one-shot peer all-reduce's sticky error word rides along in the same synchronisation: a peer that missed the spin
     // bound poisoned that step's activations with NaN (comm.hip), and the tokens read here must not be used
     uint32_t p2p_err = 0;
     const bool p2p = m->use_comm && m->comm && m->comm->p2p && m->comm->local;
     if (p2p) HCHECK(hipMemcpyAsync(&p2p_err, &m->comm->local->err, 4, hipMemcpyDeviceToHost, st));
-    HCHECK(hipStreamSynchronize(st));
+    HCHECK(m->in.read_tokens(host_out, m->cur_batch, st));
     if (p2p && p2p_err != 0) return (int)hipErrorPeerAccessNotEnabled;   // "a peer was not there": the step is invalid on this rank
     return 0;
 }
@@ -1437,6 +1428,7 @@ extern "C" int mi355_llama_run_part(void* mp, int32_t layer, int32_t part, int64
     Model* m = static_cast<Model*>(mp);
     if (!m || m->cur_batch < 1 || part < PART_QKV || part > PART_EMBED) return (int)hipErrorInvalidValue;
     if (part <= PART_DOWN && (layer < 0 || layer >= m->cfg.n_layers)) return (int)hipErrorInvalidValue;
+    HCHECK(m->in.use_on(reinterpret_cast<hipStream_t>(stream)));
     const StepIn in{m->d_tokens, m->d_positions, m->d_slots, m->d_bt, m->d_ctx, m->cur_batch, m->cur_max_blocks, m->cur_ctx_cap,
                     m->xs, m->q, m->attn, m->h, m->moe_ids, m->moe_w, m->moe_y, m->tp_y, false, nullptr, 0, 0};
     return run_part(m, part <= PART_DOWN ? layer : 0, part, in, m->logits, stream);

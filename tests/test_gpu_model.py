@@ -99,6 +99,43 @@ def test_greedy_decode_loop_graph_equals_eager_equals_oracle(lib):
     assert _rel(last, ref_last) < 1e-3
 
 
+@pytest.mark.parametrize("graph", [False, True])
+def test_step_inputs_overtaken_and_on_another_stream(lib, graph):
+    """the loop's inputs travel behind the call: a second begin before the first is used (same and smaller batch, narrower tables), the step on a stream other
+    than the inputs', a stream being captured (refused, as a copy that a replay would send again) -- tokens of every step as when all is waited for"""
+    cfg, orc, gm, seqs, cache = _setup(lib, True)
+    bt = np.array([[3, 7, 9], [1, 5, 0]], np.uint32)
+    toks, lens = [s["tokens"][-1] for s in seqs], [len(s["tokens"]) for s in seqs]
+    one, two = torch.cuda.Stream(), torch.cuda.Stream()
+    a, b = one.cuda_stream, two.cuda_stream
+    gm.set_graph(graph)
+
+    def step(n, width, begin_on, step_on, first=None):
+        got = []
+        for _ in range(3 if graph else 1):                                  # eager, captured, replayed
+            if first is not None:
+                gm.decode_begin(*first, ctx_cap=32, stream=begin_on)
+            gm.decode_begin(toks[:n], lens[:n], np.ascontiguousarray(bt[:n, :width]), ctx_cap=32, stream=begin_on)
+            if first is None:
+                torch.cuda.synchronize()
+            gm.decode_step(step_on)
+            got.append(gm.read_tokens(step_on).tolist())
+        assert all(g == got[0] for g in got)
+        return got[0]
+
+    for n, width in ((2, 3), (1, 2)):
+        want = step(n, width, a, a)
+        other = ([5, 6], [9, 3], bt[::-1])
+        assert step(n, width, a, a, other) == want
+        assert step(n, width, a, b, other) == want
+    g = torch.cuda.CUDAGraph()
+    with pytest.raises(Exception):
+        with torch.cuda.graph(g, stream=one):
+            gm.decode_begin(toks, lens, bt, ctx_cap=32, stream=torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert step(2, 3, a, a) == step(2, 3, b, a, ([5, 6], [9, 3], bt[::-1]))
+
+
 def test_rccl_plumbing_single_rank(lib, monkeypatch):
     """The tensor-parallel code path (RCCL through dlopen: unique id, comm init, in-stream all-reduce of the
     residual stream, all-gather + transpose of the logits) with a 1-rank communicator must reproduce the
