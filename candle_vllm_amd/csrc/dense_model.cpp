@@ -87,8 +87,8 @@ struct DModel {
     void* comm = nullptr;                 // borrowed communicator (tp_world > 1, or a 1-rank plumbing test)
     uint16_t* lg_gather = nullptr;        // [W, B, V/W]
     // greedy decode loop on static device buffers (mi355_dense_decode_*): step inputs, sampled tokens, f32 logits
-    StepInputs in;                        // (the next pointers but d_next lead into it)
-    uint32_t *d_tokens = nullptr, *d_ctx = nullptr, *d_bt = nullptr, *d_next = nullptr;
+    StepInputs in;                        // (the next pointers lead into it)
+    uint32_t *d_tokens = nullptr, *d_ctx = nullptr, *d_bt = nullptr;
     int64_t *d_positions = nullptr, *d_slots = nullptr;
     float* d_logits = nullptr;
     int cur_batch = 0, cur_max_blocks = 0, cur_ctx_cap = 0, cur_ctx_max = 0;
@@ -298,7 +298,7 @@ void mi355_dense_destroy(void* mp) {
         if (kv.second.graph) (void)hipGraphDestroy(kv.second.graph);
     }
     void* ps[] = {m->tok_embd, m->output_norm, m->output_norm_b, m->output, m->cos_t, m->sin_t, m->xs, m->xn, m->q, m->k, m->v, m->attn,
-                  m->h, m->lg16, m->pa_tmp, m->pa_max, m->pa_sum, m->ss, m->kv_slab, m->lg_gather, m->d_next, m->d_logits};
+                  m->h, m->lg16, m->pa_tmp, m->pa_max, m->pa_sum, m->ss, m->kv_slab, m->lg_gather, m->d_logits};
     m->in.destroy();
     for (void* p : ps) if (p) (void)hipFree(p);
     delete m;
@@ -667,7 +667,6 @@ int mi355_dense_decode_begin(void* mp, const uint32_t* tokens_host, const uint32
     if (ctx_cap < ctx_max || ctx_cap > c.max_seq || ctx_max > max_blocks * bs) return (int)hipErrorInvalidValue;
     if (!m->d_tokens) {
         const size_t B = c.max_batch;
-        if (!m->d_next) DHIP(hipMalloc((void**)&m->d_next, B * 4));
         if (!m->d_logits) DHIP(hipMalloc((void**)&m->d_logits, B * (size_t)c.vocab * W * 4));
         if (!m->in.create(c.max_batch, c.max_blocks_per_seq)) { m->in.destroy(); return (int)hipErrorOutOfMemory; }
         m->d_ctx = m->in.ctx(m->in.dev); m->d_bt = m->in.tables(m->in.dev);
@@ -686,8 +685,9 @@ static int dense_record_step(DModel* m, int64_t stream) {
     DCHECK(mi355_dense_forward(m, m->d_tokens, m->d_positions, m->d_slots, m->d_bt, m->d_ctx, nullptr, B, B, 0, m->cur_max_blocks,
                                m->cur_ctx_cap, m->d_logits, stream));
     // greedy sample (`sample_argmax`, logits_processor.rs:92-95: first maximum), then the next step's inputs on the device
-    DCHECK(mi355_argmax_f32(m->d_next, m->d_logits, B, logits_width(m->cfg), stream));
-    hipLaunchKernelGGL(advance_kernel, dim3((B + 63) / 64), dim3(64), 0, reinterpret_cast<hipStream_t>(stream), m->d_tokens, m->d_next,
+    unsigned long long* next = nullptr;
+    DCHECK(mi355_internal_argmax_slots(&next, m->d_logits, B, logits_width(m->cfg), stream));
+    hipLaunchKernelGGL(advance_kernel, dim3((B + 63) / 64), dim3(64), 0, reinterpret_cast<hipStream_t>(stream), m->d_tokens, next,
                        m->d_positions, m->d_slots, m->d_ctx, m->d_bt, m->cur_max_blocks, m->cfg.block_size, B);
     return (int)hipGetLastError();
 }

@@ -1006,9 +1006,9 @@ static int record_step(Model* m, int64_t stream) {
     RCHECK(forward_decode(m, m->d_tokens, m->d_positions, m->d_slots, m->d_bt, m->d_ctx, B, m->cur_max_blocks,
                           m->cur_ctx_cap, m->logits, stream));
     // greedy sample, then prepare the next step's inputs on the device
-    uint32_t* next = reinterpret_cast<uint32_t*>(m->q);   // scratch: q is dead after the last layer
+    unsigned long long* next = nullptr;
     // under TP the lm_head holds pad_vocab / world rows; the gathered logits row is narrowed to the real vocabulary
-    RCHECK(mi355_argmax_f32(next, m->logits, B, m->use_comm ? m->cfg.vocab : m->output.n_rows, stream));
+    RCHECK(mi355_internal_argmax_slots(&next, m->logits, B, m->use_comm ? m->cfg.vocab : m->output.n_rows, stream));
     hipLaunchKernelGGL(advance_kernel, dim3((B + 63) / 64), dim3(64), 0, reinterpret_cast<hipStream_t>(stream),
                        m->d_tokens, next, m->d_positions, m->d_slots, m->d_ctx, m->d_bt, m->cur_max_blocks,
                        m->cfg.block_size, B);

@@ -5,12 +5,14 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string.h>
+#include "argmax_slots.h"
 
-static __global__ void advance_kernel(uint32_t* tokens, const uint32_t* next_tokens, int64_t* positions, int64_t* slots,
+// The sampled tokens come out of the argmax' slots here: a launch of 4 us less per step.
+static __global__ void advance_kernel(uint32_t* tokens, unsigned long long* sampled, int64_t* positions, int64_t* slots,
                                       uint32_t* ctx, const uint32_t* bt, int max_blocks, int block_size, int batch) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= batch) return;
-    tokens[b] = next_tokens[b];
+    tokens[b] = argmax_take(sampled + b);
     const uint32_t n = ctx[b] + 1;              // sequence length after appending the sampled token
     ctx[b] = n;
     const int64_t pos = (int64_t)n - 1;

@@ -68,6 +68,25 @@ def test_linear_matches_oracle(cv, dt, T, N, K):
               mag=G.linear16(x, w, None, dt))
 
 
+@pytest.mark.parametrize("B,V", [(1, 1), (1, 3), (3, 4), (2, 1020), (1, 1024), (5, 1027), (1, 4100), (33, 8192), (9, 32001), (1, 151936), (300, 2052)])
+@pytest.mark.parametrize("skew", [0, 1])
+def test_argmax_slices(cv, B, V, skew):
+    """the first of the largest logits of every row, whatever slice it is in: ties, NaN (never), infinities, rows of nothing else; rows on and off 16 bytes;
+    the slots are clear again for the next call"""
+    rng = np.random.default_rng(B + V)
+    x = np.round(rng.normal(0, 2, (B, V)), 1).astype(np.float32)            # many ties
+    x[rng.random((B, V)) < 0.05] = np.nan
+    x[0, V // 2] = np.inf
+    x[-1, :] = np.nan if V % 2 else -np.inf
+    buf = torch.empty(B * V + skew, device="cuda")
+    d = buf[skew:].view(B, V)
+    d.copy_(torch.from_numpy(x))
+    want = np.where(np.isnan(x).all(1), 0, np.argmax(np.where(np.isnan(x), -np.inf, x), 1))
+    want = np.where((np.nan_to_num(x, nan=-np.inf) == -np.inf).all(1) & ~np.isnan(x).all(1), np.argmax(~np.isnan(x), 1), want)
+    for _ in range(2):
+        assert np.array_equal(cv.argmax(d).cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("T,N,K,epi", [(1153, 4096, 1024, 0), (2100, 2050, 2048, 0), (1344, 4080, 1280, 1), (1345, 4096, 1024, 2)])
 def test_linear_prompt_gemm_tall_narrow_tile(cv, T, N, K, epi):
     """the prompt GEMM's 192 x 128 tile: one token into the last tile, ragged tokens and rows, each epilogue; row-major and tiled weights alike bit for bit, and
