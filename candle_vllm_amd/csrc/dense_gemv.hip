@@ -74,7 +74,10 @@ struct DenseArgs {
     // dense_small3r_kernel only (q / k / v of a decode step): RoPE and the KV-cache write in the projection's epilogue
     int32_t rope_mode;        // 0 none; 1 = q (rotate, store); 2 = k (rotate, store, write the key cache); 3 = v (store, write the value cache)
     float* ss_out;            // dense_small_kernel only: where this launch leaves [T][ldo/16] partial sums of squares of its output
+    struct DenseNormTail* tail;   // host only: the RmsNorm that reads this product's output, or null
 };
+// out [T][N] = RmsNorm(the product's output) * w, bf16; done: the launch made it (only split sums of few tokens do, resid_norm_tail)
+struct DenseNormTail { void* out; const void* w; float eps; bool done; };
 
 template <int DT> __device__ __forceinline__ float h2f(uint16_t h) {
     return DT == MI355_DTYPE_BF16 ? bf16_to_f32(h) : f16_bits_to_f32(h);
@@ -994,7 +997,8 @@ static int dense_launch_dt(const DenseArgs& a, hipStream_t st) {
 #undef DWD_GO
                 if (hipGetLastError() != hipSuccess) return -1;
                 if (ks > 1) {
-                    hipLaunchKernelGGL((gptq_wide_epilogue_kernel<DT>), dim3((a.N + 255) / 256, a.T), dim3(256), 0, st, a, part, ldp, ks, tpad);
+                    if (!resid_norm_tail<DT>(a, part, ldp, ks, tpad, st))
+                        hipLaunchKernelGGL((gptq_wide_epilogue_kernel<DT>), dim3((a.N + 255) / 256, a.T), dim3(256), 0, st, a, part, ldp, ks, tpad);
                     if (hipGetLastError() != hipSuccess) return -1;
                 }
                 return 0;
@@ -1867,6 +1871,22 @@ int mi355_linear(void* out, const void* x, const void* w, const void* bias, cons
     if (epilogue == MI355_EPI_SILU_MUL) { a.pair_offset = n / 2; a.ldo = n / 2; } else a.ldo = n;
     if (epilogue == MI355_EPI_RESID && !residual) return -2;
     return dense_run(a, DW_DENSE, dtype, (hipStream_t)stream);
+}
+
+/* a decode step's residual product and the RmsNorm behind it: out = residual + x . w^T as mi355_linear / _linear_tiled / _gptq_linear_tiled (kind 0, 1, 2; symmetric
+ * zero points); *normed != 0: norm_out holds the norm of out too (else the caller makes it).  Internal to the host layer. */
+int mi355_internal_resid_norm_linear(void* out, const void* x, const void* w, const void* scales, const void* residual, int32_t num_tokens, int32_t n, int32_t k,
+                                     int32_t group_size, int32_t kind, int32_t dtype, void* norm_out, const void* norm_w, float eps, int32_t* normed, int64_t stream) {
+    if (!residual || !norm_out || !norm_w || !normed || num_tokens < 1 || num_tokens > 32 || kind < 0 || kind > 2) return -1;
+    DenseNormTail tail{norm_out, norm_w, eps, false};
+    DenseArgs a{};
+    a.w = w; a.ldw = k; a.wtiled = kind == 1; a.scales = scales; a.zmode = kind == 2 ? MI355_ZERO_SYM8 : 0; a.sperm = SP_NONE;
+    a.group_size = (group_size <= 0 || group_size > k) ? k : group_size;
+    a.x = x; a.ldx = k; a.T = num_tokens; a.K = k; a.N = n; a.resid = residual; a.epi = MI355_EPI_RESID; a.out = out; a.ldo = n;
+    a.tail = &tail;
+    const int rc = dense_run(a, kind == 2 ? DW_GPTQ4T : DW_DENSE, dtype, (hipStream_t)stream);
+    *normed = tail.done;
+    return rc;
 }
 
 static int gptq_linear_impl(int wtype, void* out, const void* x, const void* qweight, const void* scales, const void* qzeros,

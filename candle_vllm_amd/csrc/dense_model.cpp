@@ -40,6 +40,9 @@ struct DenseRope {
     uint16_t* kcache; uint16_t* vcache;
     int32_t n_kv_heads, head_dim, block_size, flash;
 };
+extern "C" int mi355_internal_resid_norm_linear(void* out, const void* x, const void* w, const void* scales, const void* residual, int32_t num_tokens, int32_t n,
+                                                int32_t k, int32_t group_size, int32_t kind, int32_t dtype, void* norm_out, const void* norm_w, float eps,
+                                                int32_t* normed, int64_t stream);
 extern "C" int mi355_internal_gptq_small_linear(void* out, const void* x, const void* qweight_tiled, const void* scales, const void* bias,
                                                 const void* residual, const void* norm_w, float norm_eps, const float* ss_in, float* ss_out,
                                                 int32_t num_tokens, int32_t n, int32_t k, int32_t group_size, int32_t dtype,
@@ -229,13 +232,22 @@ int finalize_weights(DModel* m) {
 
 // xs += x . w^T (the residual epilogue of o_proj / down_proj).  With 4-bit weights and 1..4 tokens the launch also leaves the sums
 // of squares of the new xs rows in m->ss (*ss_valid), so the consumer's RmsNorm needs no launch of its own.
-int resid_linear(const DModel* m, const uint16_t* w, const QLin& g, const void* x, int T, int n, int k, bool* ss_valid, int64_t stream) {
-    *ss_valid = false;
+// next_norm != NULL: the RmsNorm weight that reads the new xs next; *normed: m->xn holds that norm already.
+int resid_linear(const DModel* m, const uint16_t* w, const QLin& g, const void* x, int T, int n, int k, const uint16_t* next_norm, bool* ss_valid, bool* normed,
+                 int64_t stream) {
+    *ss_valid = *normed = false;
     if (g.qw && T <= 4 && m->cfg.norm_type == 0) {
         const int rc = mi355_internal_gptq_small_linear(m->xs, x, g.qw, g.scales, nullptr, m->xs, nullptr, 0.f, nullptr, m->ss, T, n, k,
                                                         g.group, m->cfg.dtype, MI355_EPI_RESID, stream);
         if (rc == 0) { *ss_valid = true; return 0; }
         if (rc != -4) return rc;
+    }
+    if (next_norm && T <= 32 && m->cfg.norm_type == 0 && (g.qw || w)) {
+        int32_t done = 0;
+        const int rc = mi355_internal_resid_norm_linear(m->xs, x, g.qw ? (const void*)g.qw : (const void*)w, g.scales, m->xs, T, n, k, g.group, g.qw ? 2 : (int)m->tiled.count(w),
+                                                        m->cfg.dtype, m->xn, next_norm, m->cfg.rms_eps, &done, stream);
+        *normed = done != 0;
+        return rc;
     }
     return linear(m, w, g, m->xs, x, nullptr, m->xs, T, n, k, MI355_EPI_RESID, stream);
 }
@@ -475,7 +487,9 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
     if (window) DHIP(hipMemcpyAsync(m->xs, m->win_in, (size_t)T * hid * 2, hipMemcpyDeviceToDevice, st));
     else hipLaunchKernelGGL(embedding16_kernel, dim3(T), dim3(256), 0, st, m->xs, m->tok_embd, tokens, hid);
     bool ss_valid = false;                    // m->ss holds the sums of squares of the current xs rows
-    for (int l = window ? m->win_first : 0; l <= (window ? m->win_last : c.n_layers - 1); ++l) {
+    bool xn_ready = false;                    // m->xn holds the norm of the current xs that is read next
+    const int l_last = window ? m->win_last : c.n_layers - 1;
+    for (int l = window ? m->win_first : 0; l <= l_last; ++l) {
         DLayer& L = m->layers[l];
         if (!L.attn_norm || !L.ffn_norm) return (int)hipErrorInvalidValue;
         // x = rms_1(xs) (llama.rs:53-54), then the q,k,v projections (+bias) (attention.rs:597-607)
@@ -508,7 +522,7 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
                     }
                 }
                 if (rc3 != 0) {
-                    DCHECK(norm(m, m->xn, m->xs, L.attn_norm, L.attn_norm_b, T, stream));
+                    if (!xn_ready) DCHECK(norm(m, m->xn, m->xs, L.attn_norm, L.attn_norm_b, T, stream));
                     normed = true;
                     for (int pass = rope_ok ? 0 : 1; pass < 2 && rc3 != 0; ++pass) {
                         rc3 = mi355_internal_linear3(outs, m->xn, ws, sc, bs, ns, T, hid, gq.group, all_q ? 2 : (m->tiled.count(L.wq) ? 3 : 0), m->cfg.dtype, nullptr, 0.f, nullptr,
@@ -519,7 +533,7 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
                 }
             }
         }
-        if (rc3 != 0 && !normed) DCHECK(norm(m, m->xn, m->xs, L.attn_norm, L.attn_norm_b, T, stream));
+        if (rc3 != 0 && !normed && !xn_ready) DCHECK(norm(m, m->xn, m->xs, L.attn_norm, L.attn_norm_b, T, stream));
         if (rc3 != 0) {
         DCHECK(linear(m, L.wq, L.gq[MI355_W_WQ], m->q, m->xn, L.bq, nullptr, T, H * D, hid, MI355_EPI_STORE, stream));
         DCHECK(linear(m, L.wk, L.gq[MI355_W_WK], m->k, m->xn, L.bk, nullptr, T, Hkv * D, hid, MI355_EPI_STORE, stream));
@@ -587,7 +601,7 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
             DCHECK(mi355_comm_all_reduce(m->comm, m->xn, (int64_t)T * hid, dt, stream));
             hipLaunchKernelGGL(add16_kernel, dim3(add_grid), dim3(256), 0, st, m->xs, m->xn, (int64_t)T * hid, dt == MI355_DTYPE_BF16);
         } else {
-            DCHECK(resid_linear(m, L.wo, L.gq[MI355_W_WO], m->attn, T, hid, H * D, &ss_valid, stream));
+            DCHECK(resid_linear(m, L.wo, L.gq[MI355_W_WO], m->attn, T, hid, H * D, L.ffn_norm, &ss_valid, &xn_ready, stream));
         }
         // xs = down(silu(gate) * up) + residual                              llama.rs:59-61, mlp.rs:440-458
         int rc_gu = -4;
@@ -598,7 +612,7 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
             if (rc_gu != 0 && rc_gu != -4) return rc_gu;
         }
         if (rc_gu != 0) {
-        DCHECK(norm(m, m->xn, m->xs, L.ffn_norm, L.ffn_norm_b, T, stream));
+        if (!xn_ready) DCHECK(norm(m, m->xn, m->xs, L.ffn_norm, L.ffn_norm_b, T, stream));
         DCHECK(linear(m, L.gate_up, L.gq[MI355_W_W1], m->h, m->xn, nullptr, nullptr, T, 2 * I, hid, MI355_EPI_SILU_MUL, stream));
         }
         if (tp) {
@@ -606,7 +620,8 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
             DCHECK(mi355_comm_all_reduce(m->comm, m->xn, (int64_t)T * hid, dt, stream));
             hipLaunchKernelGGL(add16_kernel, dim3(add_grid), dim3(256), 0, st, m->xs, m->xn, (int64_t)T * hid, dt == MI355_DTYPE_BF16);
         } else {
-            DCHECK(resid_linear(m, L.w2, L.gq[MI355_W_W2], m->h, T, hid, I, &ss_valid, stream));
+            const uint16_t* next = l < l_last ? m->layers[l + 1].attn_norm : (prefill || window) ? nullptr : m->output_norm;
+            DCHECK(resid_linear(m, L.w2, L.gq[MI355_W_W2], m->h, T, hid, I, next, &ss_valid, &xn_ready, stream));
         }
     }
     if (window) {                                                           // the residual stream after the window's last layer
@@ -619,7 +634,7 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
         DHIP(hipMemcpyAsync(m->xs, m->xn, (size_t)num_seqs * hid * 2, hipMemcpyDeviceToDevice, st));
         last = m->xs;
     }
-    DCHECK(norm(m, m->xn, last, m->output_norm, m->output_norm_b, num_seqs, stream));
+    if (!xn_ready) DCHECK(norm(m, m->xn, last, m->output_norm, m->output_norm_b, num_seqs, stream));
     if (m->comm) {                                                          // VocabParallelLinear (distributed.rs:1632-1667)
         const int W = c.tp_world > 1 ? c.tp_world : 1;
         DCHECK(linear(m, m->output, QLin{}, m->lg16, m->xn, nullptr, nullptr, num_seqs, c.vocab, hid, MI355_EPI_STORE, stream));

@@ -68,6 +68,45 @@ def test_linear_matches_oracle(cv, dt, T, N, K):
               mag=G.linear16(x, w, None, dt))
 
 
+@pytest.mark.parametrize("T,N,K,kind,made", [(5, 16, 8192, 0, True), (8, 1040, 8192, 1, True), (16, 2064, 8192, 1, True), (32, 4096, 8192, 1, True), (20, 8192, 8192, 0, True),
+                                             (7, 8208, 8192, 1, False), (8, 2064, 1024, 1, False), (3, 1040, 8192, 1, False),     # too long a row; sums in one range
+                                             (5, 1040, 8192, 2, True), (16, 3584, 18944, 2, True), (32, 2064, 8192, 2, True), (16, 2064, 512, 2, False)])
+def test_residual_product_with_the_norm_behind_it(cv, T, N, K, kind, made):
+    """a residual product that also leaves the RmsNorm of its output: where the split sums' launch makes it, the output equals the plain product's to the bit and the
+    norm is the norm launch's of that output, up to the order of one f32 sum (an ulp where a value is on the edge of two)"""
+    import ctypes
+
+    from candle_vllm_amd._lib import lib
+    dt, st, rng = "bf16", torch.cuda.current_stream().cuda_stream, np.random.default_rng(T + N + kind)
+    x, res, nw = dev16(G.round_dt(rng.normal(0, 1, (T, K)), dt), dt), dev16(G.round_dt(rng.normal(0, 1, (T, N)), dt), dt), dev16(G.round_dt(rng.normal(1, 0.1, N), dt), dt)
+    want = torch.empty(T, N, dtype=torch.bfloat16, device="cuda")
+    sc = None
+    if kind == 2:
+        q, s = _gptq_case(rng, K, N, 128, dt)
+        lin = cv.GPTQLinear(dev_u32(G.gptq_pack(q)), dev16(s, dt), 128)
+        w, sc = lin.qweight, lin.scales
+        want = lin.forward(x, epilogue=cv.EPI_RESID, residual=res)
+    else:
+        w = dev16(G.round_dt(rng.normal(0, 0.02, (N, K)), dt), dt)
+        if kind == 1:
+            w, flat = torch.empty_like(w), w
+            assert lib.mi355_dense_tile_repack(flat.data_ptr(), w.data_ptr(), N, K, K, st) == 0
+        assert (lib.mi355_linear_tiled if kind else lib.mi355_linear)(want.data_ptr(), x.data_ptr(), w.data_ptr(), None, res.data_ptr(), T, N, K, 2, 1, st) == 0
+    out, normed, done = res.clone(), torch.full((T, N), 7.0, dtype=torch.bfloat16, device="cuda"), ctypes.c_int32(-1)
+    fused = lib.mi355_internal_resid_norm_linear
+    fused.argtypes = [ctypes.c_void_p] * 5 + [ctypes.c_int32] * 6 + [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p, ctypes.c_int64]
+    assert fused(out.data_ptr(), x.data_ptr(), w.data_ptr(), sc.data_ptr() if sc is not None else None, out.data_ptr(), T, N, K, 128, kind, 2,
+                                                normed.data_ptr(), nw.data_ptr(), 1e-5, ctypes.addressof(done), st) == 0
+    assert torch.equal(out, want.view(T, N)) and done.value == int(made)
+    if not made:
+        assert bool((normed == 7).all())
+        return
+    ref = torch.empty_like(normed)
+    assert lib.mi355_rms_norm(ref.data_ptr(), out.data_ptr(), nw.data_ptr(), T, N, 1e-5, 2, 2, st) == 0
+    a, b = normed.view(torch.int16).int(), ref.view(torch.int16).int()
+    assert int((a - b).abs().max()) <= 1 and float((a != b).float().mean()) < 0.01
+
+
 @pytest.mark.parametrize("B,V", [(1, 1), (1, 3), (3, 4), (2, 1020), (1, 1024), (5, 1027), (1, 4100), (33, 8192), (9, 32001), (1, 151936), (300, 2052)])
 @pytest.mark.parametrize("skew", [0, 1])
 def test_argmax_slices(cv, B, V, skew):
