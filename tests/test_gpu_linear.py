@@ -96,7 +96,7 @@ def test_residual_product_with_the_norm_behind_it(cv, T, N, K, kind, made):
     fused = lib.mi355_internal_resid_norm_linear
     fused.argtypes = [ctypes.c_void_p] * 5 + [ctypes.c_int32] * 6 + [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p, ctypes.c_int64]
     assert fused(out.data_ptr(), x.data_ptr(), w.data_ptr(), sc.data_ptr() if sc is not None else None, out.data_ptr(), T, N, K, 128, kind, 2,
-                                                normed.data_ptr(), nw.data_ptr(), 1e-5, ctypes.addressof(done), st) == 0
+                 normed.data_ptr(), nw.data_ptr(), 1e-5, ctypes.addressof(done), st) == 0
     assert torch.equal(out, want.view(T, N)) and done.value == int(made)
     if not made:
         assert bool((normed == 7).all())
