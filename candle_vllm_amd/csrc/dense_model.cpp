@@ -711,7 +711,6 @@ int mi355_dense_decode_step(void* mp, int64_t stream) {
     DModel* m = static_cast<DModel*>(mp);
     if (!m || m->cur_batch < 1) return (int)hipErrorInvalidValue;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    DHIP(m->in.use_on(st));
     // this step attends over cur_ctx_max tokens, then advance_kernel looks up the slot of position cur_ctx_max: both must stay
     // inside the attention grid (ctx_cap), the block-table row and the RoPE tables
     if (m->cur_ctx_max > m->cur_ctx_cap || m->cur_ctx_max > m->cfg.max_seq ||

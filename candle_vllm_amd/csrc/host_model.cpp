@@ -1044,7 +1044,6 @@ extern "C" int mi355_llama_decode_step(void* mp, int64_t stream) {
     Model* m = static_cast<Model*>(mp);
     if (!m || m->cur_batch < 1) return (int)hipErrorInvalidValue;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    HCHECK(m->in.use_on(st));
     // this step attends over cur_ctx_max tokens, then `advance_kernel` looks up the slot of position cur_ctx_max: both
     // must stay inside the attention grid (ctx_cap), the block-table row and the RoPE tables
     if (m->cur_ctx_max > m->cur_ctx_cap || m->cur_ctx_max > m->cfg.max_seq ||
@@ -1428,7 +1427,6 @@ extern "C" int mi355_llama_run_part(void* mp, int32_t layer, int32_t part, int64
     Model* m = static_cast<Model*>(mp);
     if (!m || m->cur_batch < 1 || part < PART_QKV || part > PART_EMBED) return (int)hipErrorInvalidValue;
     if (part <= PART_DOWN && (layer < 0 || layer >= m->cfg.n_layers)) return (int)hipErrorInvalidValue;
-    HCHECK(m->in.use_on(reinterpret_cast<hipStream_t>(stream)));
     const StepIn in{m->d_tokens, m->d_positions, m->d_slots, m->d_bt, m->d_ctx, m->cur_batch, m->cur_max_blocks, m->cur_ctx_cap,
                     m->xs, m->q, m->attn, m->h, m->moe_ids, m->moe_w, m->moe_y, m->tp_y, false, nullptr, 0, 0};
     return run_part(m, part <= PART_DOWN ? layer : 0, part, in, m->logits, stream);

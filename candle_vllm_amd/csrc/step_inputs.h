@@ -25,15 +25,13 @@ static __global__ void advance_kernel(uint32_t* tokens, unsigned long long* samp
 }
 
 // The static inputs of the greedy loop, one block of device memory (positions | slots | tokens | context lengths | block tables) behind one pinned
-// image of it.  A change of the batch is one copy that the step is queued behind.  (One copy per array from pageable memory and a wait: begin, step
-// and read of one sequence of a 1B model, eight layers, 346 us, 16 of a 4-bit 7B, seven layers, 752; one pinned copy each way and the wait 330 and 723; without it
-// 324 and 716.)  A stream other than the copy's waits for it on the host.
+// image of it: a change of the batch is one copy, and waits for it.  (Begin, step and read of one sequence of a 1B model, eight layers: 346 us with a
+// copy per array from pageable memory, 330 with one; 16 of a 4-bit 7B, seven layers, 752 and 723.  Without the wait 324 and 716, but then nothing orders
+// a step on another stream behind the copy -- one whose handle is the same (a per-thread stream of another thread, a new stream in a destroyed one's place) or
+// a graph of the step that the caller captured and replays where he likes.)
 struct StepInputs {
     uint8_t *dev = nullptr, *host = nullptr;
     int32_t batch = 0, blocks = 0;          // room
-    hipEvent_t sent = nullptr;
-    hipStream_t last = nullptr;
-    bool pending = false;
     size_t bytes() const { return (size_t)batch * (24 + 4 * (size_t)blocks); }
     int64_t* positions(uint8_t* p) const { return reinterpret_cast<int64_t*>(p); }
     int64_t* slots(uint8_t* p) const { return positions(p) + batch; }
@@ -42,28 +40,17 @@ struct StepInputs {
     uint32_t* tables(uint8_t* p) const { return ctx(p) + batch; }
     bool create(int max_batch, int max_blocks) {
         batch = max_batch; blocks = max_blocks;
-        return hipMalloc((void**)&dev, bytes()) == hipSuccess && hipHostMalloc((void**)&host, bytes() + (size_t)batch * 4, hipHostMallocDefault) == hipSuccess &&
-               hipEventCreateWithFlags(&sent, hipEventDisableTiming) == hipSuccess;
+        return hipMalloc((void**)&dev, bytes()) == hipSuccess && hipHostMalloc((void**)&host, bytes() + (size_t)batch * 4, hipHostMallocDefault) == hipSuccess;
     }
     void destroy() {
-        if (pending) (void)hipEventSynchronize(sent);
-        if (sent) (void)hipEventDestroy(sent);
         if (host) (void)hipHostFree(host);
         if (dev) (void)hipFree(dev);
-        dev = host = nullptr; sent = nullptr; pending = false;
+        dev = host = nullptr;
     }
-    hipError_t landed() {
-        if (!pending) return hipSuccess;
-        const hipError_t e = hipEventSynchronize(sent);
-        if (e == hipSuccess) pending = false;
-        return e;
-    }
-    // the inputs of a step over n sequences (checked by the caller: every position has a block in its table's row), in stream order
+    // the inputs of a step over n sequences (checked by the caller: every position has a block in its table's row), behind everything on `st`; waits for it
     hipError_t send(const uint32_t* toks, const uint32_t* lens, const uint32_t* bt, int n, int n_blocks, int block_size, hipStream_t st) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;     // the image is written once, a replay would send what it holds by then
         if (st && hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
-        hipError_t e = landed();                                     // the image is free again
-        if (e != hipSuccess) return e;
         for (int b = 0; b < n; ++b) {
             const int64_t pos = (int64_t)lens[b] - 1;
             positions(host)[b] = pos;
@@ -72,19 +59,15 @@ struct StepInputs {
             ctx(host)[b] = lens[b];
         }
         memcpy(tables(host), bt, (size_t)n * n_blocks * 4);
-        if ((e = hipMemcpyAsync(dev, host, (size_t)batch * 24 + (size_t)n * n_blocks * 4, hipMemcpyHostToDevice, st)) != hipSuccess) return e;
-        if ((e = hipEventRecord(sent, st)) != hipSuccess) { (void)hipStreamSynchronize(st); return e; }
-        last = st; pending = true;
-        return hipSuccess;
+        const hipError_t e = hipMemcpyAsync(dev, host, (size_t)batch * 24 + (size_t)n * n_blocks * 4, hipMemcpyHostToDevice, st);
+        return e == hipSuccess ? hipStreamSynchronize(st) : e;
     }
-    hipError_t use_on(hipStream_t st) { return pending && st != last ? landed() : hipSuccess; }
     // the tokens of the n sequences, behind everything on `st`; waits for it
     hipError_t read_tokens(uint32_t* out, int n, hipStream_t st) {
         uint32_t* pin = reinterpret_cast<uint32_t*>(host + bytes());
-        hipError_t e = use_on(st);
-        if (e == hipSuccess) e = hipMemcpyAsync(pin, tokens(dev), (size_t)n * 4, hipMemcpyDeviceToHost, st);
+        hipError_t e = hipMemcpyAsync(pin, tokens(dev), (size_t)n * 4, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e == hipSuccess) { pending = false; memcpy(out, pin, (size_t)n * 4); }
+        if (e == hipSuccess) memcpy(out, pin, (size_t)n * 4);
         return e;
     }
 };

@@ -519,7 +519,8 @@ int mi355_llama_forward_prefill(void* model, const uint32_t* tokens, const int64
                                 const uint32_t* context_lens, const uint32_t* cu_seqlens_q, int32_t num_seqs,
                                 int32_t num_tokens, int32_t max_seqlen_q, int32_t max_blocks, float* logits,
                                 int64_t stream);
-/* greedy decode loop on static device buffers; the step is replayed from a hipGraph when stream != 0 */
+/* greedy decode loop on static device buffers; the step is replayed from a hipGraph when stream != 0.  begin: behind everything on `stream`, and the
+ * inputs have landed when it returns (steps may follow on any stream); steps still running on another stream are the caller's to wait for */
 int mi355_llama_decode_begin(void* model, const uint32_t* tokens_host, const uint32_t* seq_lens_host,
                              const uint32_t* block_tables_host, int32_t batch, int32_t max_blocks, int32_t ctx_cap,
                              int64_t stream);

@@ -101,8 +101,9 @@ def test_greedy_decode_loop_graph_equals_eager_equals_oracle(lib):
 
 @pytest.mark.parametrize("graph", [False, True])
 def test_step_inputs_overtaken_and_on_another_stream(lib, graph):
-    """the loop's inputs travel behind the call: a second begin before the first is used (same and smaller batch, narrower tables), the step on a stream other
-    than the inputs', a stream being captured (refused, as a copy that a replay would send again) -- tokens of every step as when all is waited for"""
+    """the loop's inputs have landed when the call returns: a second begin before the first is used (same and smaller batch, narrower tables), the step on a stream
+    other than the inputs', in a graph that the caller captured and replays on any stream; a stream being captured (refused, as a copy that a replay would send
+    again) -- tokens of every step as when all is waited for"""
     cfg, orc, gm, seqs, cache = _setup(lib, True)
     bt = np.array([[3, 7, 9], [1, 5, 0]], np.uint32)
     toks, lens = [s["tokens"][-1] for s in seqs], [len(s["tokens"]) for s in seqs]
@@ -133,7 +134,22 @@ def test_step_inputs_overtaken_and_on_another_stream(lib, graph):
         with torch.cuda.graph(g, stream=one):
             gm.decode_begin(toks, lens, bt, ctx_cap=32, stream=torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
-    assert step(2, 3, a, a) == step(2, 3, b, a, ([5, 6], [9, 3], bt[::-1]))
+    want = step(2, 3, a, a)
+    assert want == step(2, 3, b, a, ([5, 6], [9, 3], bt[::-1]))
+    gm.set_graph(False)
+    gm.decode_begin(toks, lens, bt, ctx_cap=32, stream=a)
+    gm.decode_step(b)                                                       # (the stream runs one first: nothing is allocated in a capture)
+    torch.cuda.synchronize()
+    gm.decode_begin(toks, lens, bt, ctx_cap=32, stream=a)
+    own = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(own, stream=two):
+        gm.decode_step(torch.cuda.current_stream().cuda_stream)
+    for replay_on in (two, one, torch.cuda.Stream()):
+        gm.decode_begin([5, 6], [9, 3], np.ascontiguousarray(bt[::-1]), ctx_cap=32, stream=b)
+        gm.decode_begin(toks, lens, bt, ctx_cap=32, stream=a)
+        with torch.cuda.stream(replay_on):
+            own.replay()
+        assert gm.read_tokens(replay_on.cuda_stream).tolist() == want
 
 
 def test_rccl_plumbing_single_rank(lib, monkeypatch):
