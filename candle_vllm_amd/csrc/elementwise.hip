@@ -440,7 +440,8 @@ __global__ void argmax_stage2_kernel(uint32_t* __restrict__ out, unsigned long l
     if (b >= B) return;
     out[b] = argmax_take(slots + b);
 }
-// stage 1 alone: the rows' slots, for a kernel of the caller's that takes the winners (step_inputs.h)
+// stage 1 alone: the rows' slots, for a kernel of the caller's that takes the winners (step_inputs.h).  Where this returns 0 that kernel has to follow, whatever
+// error is pending: what stays in the slots would win the next call's rows.  The caller asks for the launches' error behind it.
 int mi355_internal_argmax_slots(unsigned long long** slots, const float* logits, int32_t batch, int32_t vocab, int64_t stream) {
     if (batch > ARGMAX_MAX_ROWS || vocab <= 0) return (int)hipErrorInvalidValue;
     hipStream_t st = to_stream(stream);
@@ -452,7 +453,7 @@ int mi355_internal_argmax_slots(unsigned long long** slots, const float* logits,
     const dim3 grid(splits < 64 ? splits : 64, batch);
     if (!(vocab & 3) && !((uintptr_t)logits & 15)) hipLaunchKernelGGL((argmax_stage1_kernel<true>), grid, dim3(256), 0, st, *slots, logits, vocab);
     else hipLaunchKernelGGL((argmax_stage1_kernel<false>), grid, dim3(256), 0, st, *slots, logits, vocab);
-    return (int)hipGetLastError();
+    return 0;
 }
 extern "C" int mi355_argmax_f32(uint32_t* out, const float* logits, int32_t batch, int32_t vocab, int64_t stream) {
     if (batch <= 0) return 0;

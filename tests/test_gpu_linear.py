@@ -126,6 +126,21 @@ def test_argmax_slices(cv, B, V, skew):
         assert np.array_equal(cv.argmax(d).cpu().numpy(), want)
 
 
+def test_argmax_behind_an_error_of_the_callers(cv):
+    """an error that an earlier call of the caller's left behind is reported, and costs neither this call's winners nor the next one's"""
+    import ctypes
+
+    from candle_vllm_amd._lib import lib
+    hip, st = ctypes.CDLL("libamdhip64.so.7"), torch.cuda.current_stream().cuda_stream
+    high, low, out = torch.zeros(3, 5000, device="cuda"), torch.zeros(3, 5000, device="cuda"), torch.full((3,), 7, dtype=torch.int32, device="cuda")
+    high[:, 40], low[:, 4000] = 2.0, 1.0
+    cv.argmax(low)
+    torch.cuda.synchronize()
+    assert hip.hipSetDevice(1 << 20) != 0                                   # (a number that no card has: the call is refused, and leaves its error)
+    assert lib.mi355_argmax_f32(out.data_ptr(), high.data_ptr(), 3, 5000, st) != 0
+    assert out.tolist() == [40] * 3 and cv.argmax(low).tolist() == [4000] * 3
+
+
 @pytest.mark.parametrize("T,N,K,epi", [(1153, 4096, 1024, 0), (2100, 2050, 2048, 0), (1344, 4080, 1280, 1), (1345, 4096, 1024, 2)])
 def test_linear_prompt_gemm_tall_narrow_tile(cv, T, N, K, epi):
     """the prompt GEMM's 192 x 128 tile: one token into the last tile, ragged tokens and rows, each epilogue; row-major and tiled weights alike bit for bit, and
