@@ -701,6 +701,7 @@ static int dense_record_step(DModel* m, int64_t stream) {
                                m->cur_ctx_cap, m->d_logits, stream));
     // greedy sample (`sample_argmax`, logits_processor.rs:92-95: first maximum), then the next step's inputs on the device
     unsigned long long* next = nullptr;
+    Mi355ScratchTurn turn(MI355_SCR_ARGMAX, reinterpret_cast<hipStream_t>(stream));
     DCHECK(mi355_internal_argmax_slots(&next, m->d_logits, B, logits_width(m->cfg), stream));
     hipLaunchKernelGGL(advance_kernel, dim3((B + 63) / 64), dim3(64), 0, reinterpret_cast<hipStream_t>(stream), m->d_tokens, next,
                        m->d_positions, m->d_slots, m->d_ctx, m->d_bt, m->cur_max_blocks, m->cfg.block_size, B);

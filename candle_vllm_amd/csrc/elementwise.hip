@@ -458,6 +458,7 @@ int mi355_internal_argmax_slots(unsigned long long** slots, const float* logits,
 extern "C" int mi355_argmax_f32(uint32_t* out, const float* logits, int32_t batch, int32_t vocab, int64_t stream) {
     if (batch <= 0) return 0;
     unsigned long long* slots = nullptr;
+    Mi355ScratchTurn turn(MI355_SCR_ARGMAX, to_stream(stream));
     const int rc = mi355_internal_argmax_slots(&slots, logits, batch, vocab, stream);
     if (rc) return rc;
     hipLaunchKernelGGL(argmax_stage2_kernel, dim3((batch + 255) / 256), dim3(256), 0, to_stream(stream), out, slots, batch);

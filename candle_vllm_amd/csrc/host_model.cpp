@@ -1007,6 +1007,7 @@ static int record_step(Model* m, int64_t stream) {
                           m->cur_ctx_cap, m->logits, stream));
     // greedy sample, then prepare the next step's inputs on the device
     unsigned long long* next = nullptr;
+    Mi355ScratchTurn turn(MI355_SCR_ARGMAX, reinterpret_cast<hipStream_t>(stream));
     // under TP the lm_head holds pad_vocab / world rows; the gathered logits row is narrowed to the real vocabulary
     RCHECK(mi355_internal_argmax_slots(&next, m->logits, B, m->use_comm ? m->cfg.vocab : m->output.n_rows, stream));
     hipLaunchKernelGGL(advance_kernel, dim3((B + 63) / 64), dim3(64), 0, reinterpret_cast<hipStream_t>(stream),

@@ -141,6 +141,24 @@ def test_argmax_behind_an_error_of_the_callers(cv):
     assert out.tolist() == [40] * 3 and cv.argmax(low).tolist() == [4000] * 3
 
 
+def test_argmax_two_threads_on_one_stream(cv):
+    """the winners pass from one launch to the next in the stream's slots: two threads on one stream, each over its own logits, have their own winners"""
+    import threading
+    xs = [torch.zeros(40, 3000, device="cuda") for _ in range(2)]
+    xs[0][:, 2900], xs[1][:, 17] = 1.0, 2.0
+    got, go = [[], []], threading.Barrier(2)
+
+    def work(i):
+        go.wait()
+        got[i] = [cv.argmax(xs[i]) for _ in range(400)]
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    torch.cuda.synchronize()
+    for i, at in enumerate((2900, 17)):
+        assert len(got[i]) == 400 and all(bool((g == at).all()) for g in got[i])
+
+
 @pytest.mark.parametrize("T,N,K,epi", [(1153, 4096, 1024, 0), (2100, 2050, 2048, 0), (1344, 4080, 1280, 1), (1345, 4096, 1024, 2)])
 def test_linear_prompt_gemm_tall_narrow_tile(cv, T, N, K, epi):
     """the prompt GEMM's 192 x 128 tile: one token into the last tile, ragged tokens and rows, each epilogue; row-major and tiled weights alike bit for bit, and
