@@ -1552,9 +1552,9 @@ template <typename TO, int UNR> __global__ __launch_bounds__(64) void mingru_ker
     stt[c] = S;
 }
 
-// Long portions: S_t = (1 - z_t) S_(t-1) + z_t c_t is a composition of affine maps, so the portion is cut into NSEG segments, one wave
-// each: pass 1 reduces a segment to (A, B) with S_end = A S_start + B, the waves exchange (A, B) through LDS, every wave folds the
-// segments before its own into its starting state and walks its segment again writing the outputs.  Bound by the five gates per value (each an exponential and
+// Long portions: S_t = (1 - z_t) S_(t-1) + z_t c_t is a composition of affine maps, so the portion is cut into NSEG segments, LANES threads
+// (a wave, or half of one) each: pass 1 reduces a segment to (A, B) with S_end = A S_start + B, the segments exchange (A, B) through LDS, every one folds
+// those before its own into its starting state and is walked again, writing the outputs.  Bound by the five gates per value (each an exponential and
 // a division): LANES channels and NSEG segments per workgroup, so that a few sequences fill the card and a segment is short (two of 1050 tokens, width
 // 4096: 64 channels x 16 segments 133 us, 32 x 32 76).
 template <typename TO, int NSEG, int LANES, int UNR> __global__ __launch_bounds__(LANES * NSEG) void mingru_seg_kernel(GruArgs p) {
@@ -1566,6 +1566,9 @@ template <typename TO, int NSEG, int LANES, int UNR> __global__ __launch_bounds_
     const int cc = ok_ ? c : 0;
     const int seg = (te - tb + NSEG - 1) / NSEG;
     const int lo = min(te, tb + w * seg), hi = min(te, lo + seg);
+    const int start_pos = (int)p.ctx[s] - (te - tb);
+    float* stt = p.state + (size_t)p.slots[s] * p.state_stride;
+    float S = (start_pos > 0 && ok_) ? stt[cc] : 0.f;                   // in front of the barrier: behind it the last segment may write it at any time
     float A = 1.f, B = 0.f;
     for (int t0 = lo; t0 < hi; t0 += UNR) {
         float z[UNR], u[UNR];
@@ -1581,9 +1584,6 @@ template <typename TO, int NSEG, int LANES, int UNR> __global__ __launch_bounds_
     }
     sA[w][lane] = A; sB[w][lane] = B;
     __syncthreads();
-    const int start_pos = (int)p.ctx[s] - (te - tb);
-    float* stt = p.state + (size_t)p.slots[s] * p.state_stride;
-    float S = (start_pos > 0 && ok_) ? stt[cc] : 0.f;
     for (int v = 0; v < w; ++v) S = sA[v][lane] * S + sB[v][lane];
     for (int t0 = lo; t0 < hi; t0 += UNR) {
         float z[UNR], u[UNR], gg[UNR];
