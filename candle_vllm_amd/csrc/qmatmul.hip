@@ -2060,14 +2060,24 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
     if (big && !a.blk_tab && (v_slots || (one_q6 && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID))))
         pick6 = qpw_pick(MI355_GGML_Q6_K, T, v_slots ? v_slots : n_slots, K, v_slots || T >= 4096 ? 0.f : c_pass).tile;
     // token rows of the image: whole tiles of whichever kernel reads it
-    const int Tpad = pick4 == 2 ? std::max((T + 191) / 192 * 192, (T + 255) / 256 * 256)
-                     : pick4 >= 0 || pick6 >= 0 ? (T + 255) / 256 * 256 : (T + QPG_BM - 1) / QPG_BM * QPG_BM;
-    // (a block-table launch only exists with the epilogue in the store loop: no C buffer -- it would be 1.9 GB for a Mixtral chunk)
     const int blk64 = (T + QPG_BM - 1) / QPG_BM * (QPG_BM / 64);   // token blocks of the 64-token kernels
-    const size_t xa_b = (size_t)K * Tpad * 2 * parts, sf_b = (size_t)nkb * Tpad * 32, rs_b = (size_t)Tpad * 4, c_b = a.blk_tab ? 0 : (size_t)T * ldp * 4;
+    int Tpad = pick4 == 2 ? std::max((T + 191) / 192 * 192, (T + 255) / 256 * 256)
+               : pick4 >= 0 || pick6 >= 0 ? (T + 255) / 256 * 256 : blk64 * 64;
+    // (a block-table launch only exists with the epilogue in the store loop: no C buffer -- it would be 1.9 GB for a Mixtral chunk)
+    const size_t c_b = a.blk_tab ? 0 : (size_t)T * ldp * 4;
+    size_t xa_b = 0, sf_b = 0, rs_b = 0;
     void* ws = nullptr;
     Mi355ScratchTurn turn(MI355_SCR_QMP_WS, st);            // from the image's launch to its readers'
-    int rc = qmg_buf(&ws, MI355_SCR_QMP_WS, xa_b + sf_b + 2 * rs_b + c_b + 4096, st);
+    auto room = [&]() {
+        xa_b = (size_t)K * Tpad * 2 * parts; sf_b = (size_t)nkb * Tpad * 32; rs_b = (size_t)Tpad * 4;
+        return qmg_buf(&ws, MI355_SCR_QMP_WS, xa_b + sf_b + 2 * rs_b + c_b + 4096, st);
+    };
+    int rc = room();
+    if (rc && Tpad > blk64 * 64) {                          // a full card, or a capture and a buffer that has room for the 64-token kernels' rows only
+        pick4 = pick6 = -1;
+        Tpad = blk64 * 64;
+        rc = room();
+    }
     if (rc) return rc;
     a.dbg = g_tune_dbg;                                     // ablation bits of the prompt-step GEMM (experiments only)
     uint8_t* base = static_cast<uint8_t*>(ws);

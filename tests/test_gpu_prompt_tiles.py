@@ -78,6 +78,37 @@ def test_store_and_residual(kind, T, N, K, tile):
         assert torch.equal(o[:, N:], keep[:, N:])
 
 
+@pytest.mark.parametrize("kind,T,N,K,tile", [(Q4, 1281, 4096, 2048, 1), (Q4, 4097, 2064, 1024, 2), (Q6, 1300, 4096, 1024, 11)])
+def test_no_room_for_whole_tiles(kind, T, N, K, tile):
+    """room for the image in whole 128 tokens but not in whole tiles: the 64-token kernels take the product -- on a full card, and in a capture, where the buffer of
+    an earlier product may not grow"""
+    rng = np.random.default_rng(T)
+    b = blocks(rng, N, K, kind)
+    m = cv.QMatMul(b, kind, "cuda")
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    want, rows = product(x, b, kind), (T + 127) // 128 * 128
+    room = rows * (2 * K + K // 256 * 32 + 8) + 4 * T * N + 4096
+    cv.lib.mi355_internal_scratch_limit.argtypes = [ctypes.c_int64]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        cv.lib.mi355_internal_scratch_limit(room)
+        try:
+            got = m.forward(x)
+        finally:
+            cv.lib.mi355_internal_scratch_limit(-1)
+        assert last_tile() == -1 and close(got, want) < TOL
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=torch.cuda.current_stream()):
+            captured = m.forward(x)
+        assert last_tile() == -1
+        for _ in range(3):
+            captured.zero_()
+            graph.replay()
+            assert torch.equal(captured, got)
+        assert close(m.forward(x), want) < TOL and last_tile() == tile
+
+
 @pytest.mark.parametrize("T,N,K,tile", [(385, 14314, 1024, 0), (700, 8190, 1024, 2), (1281, 2048, 2048, 1), (1300, 2060, 2048, 1)])
 def test_gate_up(T, N, K, tile):
     rng = np.random.default_rng(T + N)
