@@ -1970,13 +1970,13 @@ static int g_tune_dbg = 0;                                 // mi355_set_tuning(2
 #include "qmm_prefill.inc"
 #include "qmm_prompt_gemm.inc"
 
-template <int WT, int WM, int WN, int MG, int NG, int SA, bool QKV = false>
+template <int WT, int WM, int WN, int MG, bool QKV = false>
 static int qpw_go(const QmmArgs& r, const QpgImg& im, int n_slots, hipStream_t st) {
-    if constexpr (!QKV) if (r.epi == MI355_EPI_QKV_ROPE_CACHE) return qpw_go<WT, WM, WN, MG, NG, SA, true>(r, im, n_slots, st);
-    using L = QpwTile<WT, WM, WN, MG, NG, SA>;
+    if constexpr (!QKV) if (r.epi == MI355_EPI_QKV_ROPE_CACHE) return qpw_go<WT, WM, WN, MG, true>(r, im, n_slots, st);
+    using L = QpwTile<WT, WM, WN, MG>;
     static Mi355DevOnce once;
     if (!once.done()) {
-        const hipError_t e = hipFuncSetAttribute((const void*)qpw_gemm_kernel<WT, WM, WN, MG, NG, SA, QKV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::LDS);
+        const hipError_t e = hipFuncSetAttribute((const void*)qpw_gemm_kernel<WT, WM, WN, MG, QKV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L::LDS);
         if (e != hipSuccess) return (int)e;
         once.set();
     }
@@ -1987,7 +1987,7 @@ static int qpw_go(const QmmArgs& r, const QpgImg& im, int n_slots, hipStream_t s
                  (((uintptr_t)r.q_out | (uintptr_t)r.kcache | (uintptr_t)r.vcache | (uintptr_t)r.cos_t | (uintptr_t)r.sin_t) & 15) == 0;
     w.n_m = (r.B + L::BM - 1) / L::BM;
     w.n_n = (n_slots + L::NT - 1) / L::NT;
-    hipLaunchKernelGGL((qpw_gemm_kernel<WT, WM, WN, MG, NG, SA, QKV>), dim3(w.n_m * w.n_n), dim3(512), (size_t)L::LDS, st, r, im, w);
+    hipLaunchKernelGGL((qpw_gemm_kernel<WT, WM, WN, MG, QKV>), dim3(w.n_m * w.n_n), dim3(512), (size_t)L::LDS, st, r, im, w);
     return (int)hipGetLastError();
 }
 // tile of this thread's last prompt product (tests: which kernel ran)
@@ -2021,15 +2021,14 @@ static QpwChoice qpw_pick(int type, int T, int n_slots, int K, float old_extra_u
     }
     return best;
 }
-extern "C" int32_t mi355_internal_qpw_pick(int32_t type, int32_t T, int32_t n_slots, int32_t K) { return qpw_pick(type, T, n_slots, K, 0.f).tile; }   // tests
 template <int WT>
 static int qpw_launch(int tile, const QmmArgs& r, const QpgImg& im, int n_slots, hipStream_t st) {
     g_qpw_last = WT == MI355_GGML_Q4_K ? tile : 10 + tile;
     if constexpr (WT == MI355_GGML_Q4_K) {
-        if (tile == 0) return qpw_go<WT, 2, 4, 4, 2, 2>(r, im, n_slots, st);
-        if (tile == 2) return qpw_go<WT, 2, 4, 3, 2, 2>(r, im, n_slots, st);
+        if (tile == 0) return qpw_go<WT, 2, 4, 4>(r, im, n_slots, st);
+        if (tile == 2) return qpw_go<WT, 2, 4, 3>(r, im, n_slots, st);
     }
-    return qpw_go<WT, 4, 2, 2, 2, 2>(r, im, n_slots, st);
+    return qpw_go<WT, 4, 2, 2>(r, im, n_slots, st);
 }
 
 // hand-written prompt-step GEMM (qmm_prefill.inc); returns hipErrorNotSupported for launches it does not cover (then the
@@ -2112,8 +2111,8 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
     }
     if (a.blk_tab && g_tune_qpg != 2) return (int)hipErrorNotSupported;                   // only the LDS-fed kernel reads a block table
     hipLaunchKernelGGL(qpg_rowprep_kernel, dim3(Tpad), dim3(256), 0, st, a, im);          // row statistics + image, one launch (workgroup = token)
-    // EXPERIMENT (mi355_set_tuning(48, 1)): all segments Q4_K, one activation plane, the default wave tile, and an epilogue that is a
-    // store / residual add / SiLU * up over two equal segments -> the GEMM writes the outputs itself, no C buffer, no epilogue launch
+    // all segments Q4_K, one activation plane, and an epilogue that is a store / residual add / SiLU * up over two equal segments: the GEMM
+    // writes the outputs itself, no C buffer, no epilogue launch (mi355_set_tuning(48, 0) switches that off)
     {
         if (g_tune_qpg_fepi && all_q4 && epi_ok && parts == 1 && (g_tune_qpg == 0 || g_tune_qpg == 2)) {
             QmmArgs r = a;

@@ -111,7 +111,7 @@ def test_residual_product_with_the_norm_behind_it(cv, T, N, K, kind, made):
 @pytest.mark.parametrize("skew", [0, 1])
 def test_argmax_slices(cv, B, V, skew):
     """the first of the largest logits of every row, whatever slice it is in: ties, NaN (never), infinities, rows of nothing else; rows on and off 16 bytes;
-    the slots are clear again for the next call"""
+    the slots are clear again for the next call, whose logits are all below this one's, the largest of them last"""
     rng = np.random.default_rng(B + V)
     x = np.round(rng.normal(0, 2, (B, V)), 1).astype(np.float32)            # many ties
     x[rng.random((B, V)) < 0.05] = np.nan
@@ -122,8 +122,10 @@ def test_argmax_slices(cv, B, V, skew):
     d.copy_(torch.from_numpy(x))
     want = np.where(np.isnan(x).all(1), 0, np.argmax(np.where(np.isnan(x), -np.inf, x), 1))
     want = np.where((np.nan_to_num(x, nan=-np.inf) == -np.inf).all(1) & ~np.isnan(x).all(1), np.argmax(~np.isnan(x), 1), want)
+    below = torch.linspace(-9e3, -8e3, V, device="cuda").repeat(B, 1)
     for _ in range(2):
         assert np.array_equal(cv.argmax(d).cpu().numpy(), want)
+        assert bool((cv.argmax(below) == V - 1).all())
 
 
 def test_argmax_behind_an_error_of_the_callers(cv):
