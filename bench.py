@@ -330,7 +330,8 @@ def bench_prefill(gm, cfg, perm, blocks_per_seq, T=2048):
             "with_causal_attention_TFLOPs": round((gemm_flops + attn_flops) / dt / 1e12, 1),
             "flops_counted": "2 x (32 layers x %.1f M projection weights x T + lm_head x 1 token); attention's %.1f TFLOP reported separately"
                              % (layer_params / 1e6, attn_flops / 1e12),
-            "note": "hand-written quantised GEMM (csrc/qmm_prefill.inc): Q4_K/Q6_K unpacked in registers into f16 MFMA operands, "
+            "note": "hand-written quantised GEMMs: Q4_K/Q6_K unpacked into f16 MFMA operands, once per workgroup through LDS in tiles of up to "
+                    "256 x 256 (csrc/qmm_prompt_gemm.inc) or in registers (csrc/qmm_prefill.inc: few tokens, small matrices, experts), "
                     "no weight image in HBM, no library GEMM; activations ONE f16 plane with a power-of-two scale per (token, "
                     "k-block) = 1 MFMA pass (round 2: hi + lo planes, 2 passes; tuning key 24 restores them); whole prompt step "
                     "incl. prefill attention and epilogues"}

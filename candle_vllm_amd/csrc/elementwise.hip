@@ -391,9 +391,9 @@ extern "C" int mi355_embedding_f32(float* out, const float* table, const uint32_
 // Stage 1: grid (splits, B) workgroups reduce a slice each and atomicMax a packed 64-bit key
 //          (order-preserving value bits << 32 | ~index) into a per-row slot; stage 2 decodes and re-zeroes the
 //          slot, so the scratch is self-cleaning and the pair is safe to replay from a hipGraph.
-// Bound by its round trips and by the atomics of one row, which queue at one address: slices of 1024 logits or more, 64 at most and fewer where the rows
-// already fill the card, 16 bytes per load.  Both stages, 64 slices of a float per load / now: 32 x 32000 logits 15.9 / 6.9 us, 8 x 128256 10.5 / 7.9, 256 x 151936
-// 59 / 26; one row of 32000 6.8 / 6.4, of 151936 6.1 (32 slices of four floats: 7.3).
+// Bound by its round trips and by the atomics of one row, which queue at one address: a slice per 1024 logits and one more, 64 at most and fewer where the
+// rows already fill the card, 16 bytes per load.  Both stages, 64 slices of a float per load / now: 32 x 32000 logits 15.9 / 6.9 us, 8 x 128256 10.5 / 7.9,
+// 256 x 151936 59 / 26; one row of 32000 6.8 / 6.4, of 151936 6.1 (32 slices of four floats: 7.3).
 #define ARGMAX_MAX_ROWS 4096
 
 __device__ __forceinline__ unsigned long long argmax_key(float v, uint32_t idx) {

@@ -2031,7 +2031,7 @@ static int qpw_launch(int tile, const QmmArgs& r, const QpgImg& im, int n_slots,
     return qpw_go<WT, 4, 2, 2>(r, im, n_slots, st);
 }
 
-// hand-written prompt-step GEMM (qmm_prefill.inc); returns hipErrorNotSupported for launches it does not cover (then the
+// hand-written prompt-step GEMMs (qmm_prompt_gemm.inc, qmm_prefill.inc); returns hipErrorNotSupported for launches it does not cover (then the
 // caller keeps the library-GEMM path)
 static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
     QmmArgs a = a0;
@@ -2634,7 +2634,7 @@ int mi355_qmm_launch(QmmArgs a, int64_t stream) {
     }
     if (a.blk_tab && !(a.B >= g_tune_qpg_min && g_tune_prefill_gemm == 1)) return (int)hipErrorNotSupported;   // only the prompt GEMM reads a block table
     if (a.B >= g_tune_qpg_min && g_tune_prefill_gemm) {
-        // prompt step: the hand-written quantised GEMM (qmm_prefill.inc).  mi355_set_tuning(6, 2) = the first-generation path
+        // prompt step: the hand-written quantised GEMMs (qmm_prompt_gemm.inc, qmm_prefill.inc).  mi355_set_tuning(6, 2) = the first-generation path
         // (bf16 hi/lo weight image + three library GEMMs) for A/B runs; (6, 0) = stream the weights 32 tokens at a time.
 #ifdef MI355_QMM_PROBES
         if (g_tune_prefill_gemm == 2) {

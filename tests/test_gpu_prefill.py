@@ -150,7 +150,7 @@ def test_prefill_mixed_batch_cached_and_fresh_with_equal_maxima(cv):
 
 @pytest.mark.parametrize("H,Hkv,bs", [(8, 2, 64), (32, 8, 16), (28, 4, 32), (4, 4, 64), (8, 1, 16)])
 def test_prefill_lds_dma_kernel(cv, H, Hkv, bs):
-    """the default since round 4: prompt attention with K / V through the LDS ring (prefill_attn_lds_kernel): 64 queries x the heads of a GQA
+    """prompt attention with K / V through the LDS ring (prefill_attn_lds_kernel): 32 queries x the heads of a GQA
     group per workgroup -- chunked prefill, prefix hit, fresh prompts, blocks that end inside a stage, GQA groups of 1 / 4 / 7 / 8
     heads; against the oracle at the product kernel's bound AND against the product kernel itself (same hi + lo probabilities:
     the two agree to accumulation noise)"""
