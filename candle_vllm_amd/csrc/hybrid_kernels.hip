@@ -63,7 +63,7 @@ struct LinArgs {
     float glu_limit, glu_alpha;   // of LIN_ACT_CLAMPED
 };
 constexpr int LIN_ACT_CLAMPED = MI355_HYB_ACT_RELU2 + 1;   // g' sigmoid(alpha g') (u' + 1), g' = min(g, limit), u' = u within +- limit
-// (behind the gate/up product: 156 -> 168 us at 2100 tokens x 12288 x 2048, and the activation's own launch, 43 us there and 4.7 at 8 tokens, is gone)
+// (behind the gate/up product: 156 -> 168 us at 2100 tokens x 16384 x 2048, and the activation's own launch, 43 us there and 4.7 at 8 tokens, is gone)
 __device__ __forceinline__ float clamped_gluf_(float g, float u, float limit, float alpha) {
     g = fminf(g, limit);
     return g * sigmoidf_(alpha * g) * (fminf(fmaxf(u, -limit), limit) + 1.f);
