@@ -178,6 +178,10 @@ struct GemmTile {
 // per CU / one 192 x 128 (f32 results): 2100 x 2048 x 2048 29.3 / 25.3, x 6144 73.8 / 59.2; 1100 x 4096 x 4096 50.1 / 44.4; 300 x 14336 x 4096 64.9 / 49.0;
 // where its second round is not full the pick stays: 1100 x 9216 x 2048 192 x 256 44.4 / 50.9, 1100 x 14336 x 4096 135.5 / 144.2.  From 16 units (k >= 1024) on:
 // below, a launch is mostly its start and its stores (2100 x 2048 x 128 9.3 / 8.5, x 704 15.7 / 13.2).  256 x 128 as a seventh tile won nowhere by more than 2 %.
+// With K in ranges (16-bit results, us, without it / with it): in place of 256 x 256 tiles 933 x 2784 x 8448 61.7 / 53.3 (sixteen such sizes 0.83 .. 0.91 of the time); of the other
+// two-buffered ones up to four row tiles, 162 x 4272 x 8192 34.3 / 26.9, 373 x 3712 x 11264 46.5 / 42.1 (60 sizes 0.78 .. 0.99), and not beyond (1418 x 768 x 10496 42.4 / 38.8, but
+// 1094 x 1216 x 5888 31.4 / 34.5: 0.87 .. 1.10); never in place of tiles 3 and 4, whose rounds the sum below makes look 1 .. 5 % longer than its short ranges and which
+// are faster (185 x 6864 x 3072 16.8 / 22.9, 903 x 1136 x 7936 29.3 / 34.6, 960 x 2848 x 6400 40.9 / 45.6: 24 sizes 1.02 .. 1.37).
 struct GtTile { int bm, bn, per_cu; float us; };
 constexpr int GT_NARROW = 5;
 static constexpr GtTile kGtTiles[] = {{256, 256, 1, 1.46f}, {192, 256, 1, 1.28f}, {128, 128, 2, 0.93f}, {128, 128, 1, 0.5f}, {64, 128, 1, 0.42f}, {192, 128, 1, 0.72f}};
@@ -193,13 +197,19 @@ template <class F>
 static inline GtChoice gt_pick(F tiles, int units, float stream_us, int max_split, float part_us, unsigned allowed, const GtTile* table = kGtTiles, int n_table = 6) {
     const int cus = mi355_num_cus();
     GtChoice best{-1, 1, 0.f};
-    for (int i = 0; i < n_table; ++i)
-        for (int s = 1; s <= max_split; ++s) {
-            if (!(allowed >> i & 1) || (i == GT_NARROW && units < 16)) continue;
+    auto consider = [&](int i, int most) {
+        if (!(allowed >> i & 1)) return;
+        for (int s = 1; s <= most; ++s) {
             const int64_t wgs = (int64_t)cus * table[i].per_cu, rounds = (tiles(table[i]) * s + wgs - 1) / wgs;
             const float t = (float)rounds * (float)((units + s - 1) / s + 2) * table[i].us;
             const float c = (t > stream_us ? t : stream_us) + (s > 1 ? 5.f + part_us * (float)(s + 1) : 0.f);
             if (best.tile < 0 || c < best.us) best = {i, s, c};
         }
+    };
+    for (int i = 0; i < n_table; ++i) if (i != GT_NARROW) consider(i, max_split);
+    if (n_table > GT_NARROW && units >= 16) {
+        const bool ranges = best.tile == 0 || (best.tile > 0 && best.tile < 3 && tiles(GtTile{table[GT_NARROW].bm, 1 << 30, 1, 0.f}) <= 4);
+        consider(GT_NARROW, ranges ? max_split : 1);
+    }
     return best;
 }

@@ -193,7 +193,9 @@ def test_linear_prompt_gemm_tall_narrow_tile(cv, T, N, K, epi):
                                           (900, 8192, 128, 201),                               # 128 x 128 tiles, exactly two per CU
                                           (1030, 2560, 704, 301),                              # 128 x 128 tiles, one per CU
                                           (1530, 8192, 128, 101),                              # 192 x 256 tiles, exactly one per CU, ragged tokens
-                                          (1540, 8208, 128, 1)])                               # 256 x 256 tiles, ragged both ways
+                                          (1540, 8208, 128, 1),                                # 256 x 256 tiles, ragged both ways
+                                          (162, 4256, 8192, 507),                              # 192 x 128 tiles, K in 7 ranges, where a two-buffered tile's are longer
+                                          (185, 6880, 3072, 401), (903, 1152, 7936, 303)])     # ... and never where the tiles of six or four buffers serve
 def test_linear_prompt_gemm_every_tile(cv, T, N, K, launch):
     """16-bit prompt GEMM where its dispatch takes each of its tiles and K splits: row-major and tiled weights alike bit for bit, and within the
     op's bound of the oracle (tokens and rows at the tile's edges and at the matrix's)"""
