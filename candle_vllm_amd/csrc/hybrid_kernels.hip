@@ -1419,8 +1419,10 @@ static void conv_launch(const ConvArgs& p, hipStream_t st) {
     constexpr int RT = 8;
     const int cols = (p.C + 1023) / 1024, rows = (p.T + RT - 1) / RT;
     // us, this / a value per thread (channels x tokens): 1024 x 512 7.4 / 5.0, 6144 x 128 7.7 / 6.8, 1024 x 1024 7.7 / 7.9, 6144 x 256 8.1 / 10.9, 8192 x 1024 17.3 / 47.5:
-    // the lines cross near 2^20 values, below which the launch is its chain of look-ups
-    if (p.taps == 4 && ((p.C | p.ldp | p.off) & 3) == 0 && p.T <= RT * 65535 && (int64_t)p.T * p.C >= 1 << 20 &&
+    // the lines cross near 2^20 values, below which the launch is its chain of look-ups.  Fewer than 128 channels leave half of a workgroup idle and more: 128 x 8193
+    // 7.3 / 7.5, 96 x 10923 7.7 / 7.5, 64 x 16385 8.0 / 7.5, x 49152 18.2 / 19.2; 48 x 65536 22 / 19.3, 4 x 262145 65 / 6.3
+    const int64_t from = p.C >= 128 ? 1 << 20 : p.C >= 64 ? 3 << 20 : INT64_MAX;
+    if (p.taps == 4 && ((p.C | p.ldp | p.off) & 3) == 0 && p.T <= RT * 65535 && (int64_t)p.T * p.C >= from &&
         (((uintptr_t)p.proj | (uintptr_t)p.out | (uintptr_t)p.bias) & 15) == 0 && ((uintptr_t)p.out_bf16 & 7) == 0)
         conv_silu_rows_kernel<4, RT><<<dim3(cols, rows), 256, 0, st>>>(p);
     else conv_silu_kernel<<<(unsigned)(((int64_t)p.T * p.C + 255) / 256), 256, 0, st>>>(p);

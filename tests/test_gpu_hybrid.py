@@ -304,7 +304,7 @@ def test_conv_silu_portions_and_state(lib, taps):
     assert np.abs(np.concatenate(got_b) - want_b).max() < 5e-6
 
 
-@pytest.mark.parametrize("C,T", [(1028, 1021), (12, 87383), (2048, 512)])
+@pytest.mark.parametrize("C,T", [(1028, 1021), (12, 87383), (2048, 512), (132, 7944), (64, 49153)])
 @pytest.mark.parametrize("form", ["silu", "residual", "bias", "residual16"])
 def test_conv_rows_of_tokens(lib, C, T, form):
     """the convolution that makes several tokens per thread equals the one of a value per thread (what an offset off the 16-byte grid takes) bit for bit:
