@@ -2388,9 +2388,13 @@ int mi355_hyb_mingru(void* out, int32_t out_dtype, float* state, int64_t state_s
     GruArgs p{out, state, state_stride, proj, ldp, z_off, x_off, g_off, context_lens, cu_seqlens_q, state_slots, width};
     const dim3 grid((width + 63) / 64, num_seqs);
     if (num_tokens >= 256) {                            // some portion may be long: segmented scan
-        // where 64 channels per workgroup do not fill the card and the sequences are long: 32.  us, 64 / 32 channels (sequences x tokens, width): 1 x 256, 1024
-        // 18.9 / 10.9, 8 x 256, 1024 20.0 / 12.6, 1 x 4096, 4096 277 / 142, 32 x 64, 256 6.8 / 5.5; 32 x 8, 256 4.2 / 5.7, 8 x 256, 4096 38.2 / 39.1, 64 x 16, 4096 33.5 / 45.7
-        if ((int64_t)grid.x * num_seqs <= mi355_num_cus() && num_tokens >= 64 * (int64_t)num_seqs) {
+        // 32 channels per workgroup where 64 leave half of the card idle and the sequences are long, 64 tokens on average.  us, 64 / 32 channels (sequences x tokens, width):
+        // 1 x 256, 1024 18.9 / 10.9, 8 x 256, 1024 20.0 / 12.6, 1 x 4096, 4096 277 / 142, 100 x 64, 64 6.5 / 5.1; 32 x 8, 256 4.2 / 5.7, 64 x 16, 4096 33.5 / 45.7.  With more than
+        // half of the card at work both take about as long, but for one long sequence among short ones (2000 and 7 x 1 tokens, 2048 133 / 70): 32 from 96 tokens on average in rows of
+        // whole 128-byte lines (4 x 1024, 2560 70.6 / 64.9; 16 x 64, 1024 6.9 / 7.5; off the lines, 3 x 512, 5000 43.1 / 46.1).  Over the card's width 64 (8 x 256, 4096 38.2 / 39.1)
+        const int64_t wide = (int64_t)grid.x * num_seqs;
+        const bool lines = ((ldp | z_off | x_off | g_off) & 31) == 0 && ((uintptr_t)proj & 127) == 0;
+        if (2 * wide <= mi355_num_cus() ? num_tokens >= 64 * (int64_t)num_seqs : wide <= mi355_num_cus() && lines && num_tokens >= 96 * (int64_t)num_seqs) {
             const dim3 narrow((width + 31) / 32, num_seqs);
             if (out_dtype == MI355_DTYPE_F32) mingru_seg_kernel<float, 32, 32, 4><<<narrow, 1024, 0, to_stream(stream)>>>(p);
             else mingru_seg_kernel<uint16_t, 32, 32, 4><<<narrow, 1024, 0, to_stream(stream)>>>(p);

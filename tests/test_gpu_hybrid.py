@@ -680,30 +680,35 @@ def test_gated_norm_and_mingru(lib):
         assert np.abs(state.cpu().numpy()[2, :width] - S_want).max() < 2e-5
 
 
-@pytest.mark.parametrize("width,lens,narrow", [(70, (300, 0, 1, 33, 97), True), (33, (257, 64), True), (5440, (260, 1, 65), True),     # 32 channels per workgroup
-                                               (70, (17, 0, 1, 250, 5, 3), False), (64, (16,) * 16, False), (5506, (260, 1, 65), False)])   # 64: short ones, many channels
+@pytest.mark.parametrize("width,lens,off,narrow", [(70, (300, 0, 1, 33, 97), 1, True), (33, (257, 64), 1, True), (2688, (260, 1, 65), 1, True),     # 32 channels per workgroup
+                                                   (4096, (300, 1, 1), 0, True),                                                             # more channels, in rows of whole lines
+                                                   (70, (17, 0, 1, 250, 5, 3), 1, False), (64, (16,) * 16, 1, False),                        # 64: short ones on average,
+                                                   (2752, (260, 1, 65), 1, False), (4096, (255, 1, 1), 0, False), (5506, (260, 1, 65), 0, False)])   # ... many channels
 @pytest.mark.parametrize("out_dt", [F32, BF16])
-def test_mingru_segments_of_several_sequences(lib, width, lens, narrow, out_dt):
+def test_mingru_segments_of_several_sequences(lib, width, lens, off, narrow, out_dt):
     """both segmented scans: sequences of no token, of fewer tokens than segments and long ones, new ones and ones that go on from a state, widths off the
     workgroups' channels; outputs and states, nothing beyond a row or of an idle sequence's state.  (the f32 walk of at most 300 gates: 2e-5, as the plain scan)"""
     _gpu()
     T, n = sum(lens), len(lens)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    assert T >= 256 and ((width + 63) // 64 * n <= cus and T >= 64 * n) == narrow       # (the launch's rule, on a card of 256 CUs)
+    wide, ldp = (width + 63) // 64 * n, 3 * width + off
+    by_32 = T >= 64 * n if 2 * wide <= cus else wide <= cus and ldp % 32 == 0 and width % 32 == 0 and T >= 96 * n
+    assert T >= 256 and by_32 == narrow                                     # (the launch's rule, on a card of 256 CUs)
     rng = np.random.default_rng(width + n)
     f = lambda a: np.asarray(a).astype(np.float32).astype(np.float64)       # noqa: E731
-    proj, old = f(2 * rng.standard_normal((T, 3 * width + 1))), f(rng.standard_normal((n + 1, width + 4)))
+    proj, old = f(2 * rng.standard_normal((T, ldp))), f(rng.standard_normal((n + 1, width + 4)))
     before, slots = rng.choice([0, 0, 1, 70], n), rng.permutation(n + 1)[:n]
     before[0] = 70
     cu = np.concatenate([[0], np.cumsum(lens)])
     state, out = dev(old), dev_dt(np.full((T * width + 5,), 7.0), out_dt)
-    ok(lib.mi355_hyb_mingru(out.data_ptr(), out_dt, state.data_ptr(), width + 4, P(proj), 3 * width + 1, 1, 1 + width, 1 + 2 * width,
+    ok(lib.mi355_hyb_mingru(out.data_ptr(), out_dt, state.data_ptr(), width + 4, P(proj), ldp, off, off + width, off + 2 * width,
                             P(before + np.array(lens), np.int32), P(cu, np.int32), P(slots, np.int32), n, T, width, _st()))
     got, S_got = host_dt(out, out_dt), state.cpu().numpy()
     for i in range(n):
         p = proj[cu[i]:cu[i + 1]]
-        want, S = H.min_gru(p[:, 1:1 + width], p[:, 1 + width:1 + 2 * width], old[slots[i], :width] if before[i] else None)
-        want = want * H.silu(p[:, 1 + 2 * width:1 + 3 * width])
+        z, x, g = (p[:, off + j * width:off + (j + 1) * width] for j in range(3))
+        want, S = H.min_gru(z, x, old[slots[i], :width] if before[i] else None)
+        want = want * H.silu(g)
         y = got[cu[i] * width:cu[i + 1] * width].reshape(-1, width)
         assert (np.abs(y - want) <= 2e-5 + (0 if out_dt == F32 else 2.0 ** -8) * np.abs(want)).all()
         assert np.abs(S_got[slots[i], :width] - (S if lens[i] else old[slots[i], :width])).max() < 2e-5
