@@ -610,11 +610,13 @@ template <typename TO> __global__ void gelu_glu_kernel(TO* out, const float* gu,
     st<TO>(out, (size_t)i, gelu_tanhf_(gu[t * 2 * ff + j]) * gu[t * 2 * ff + ff + j]);
 }
 
-template <typename TO> __global__ void clamped_glu_kernel(TO* out, const float* gu, int64_t n, int ff, float limit, float alpha) {
+// IL: gu holds 16 gate columns, their 16 up columns, the next 16 gate columns, ...
+template <typename TO, bool IL> __global__ void clamped_glu_kernel(TO* out, const float* gu, int64_t n, int ff, float limit, float alpha) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int64_t t = i / ff; const int j = (int)(i - t * ff);
-    st<TO>(out, (size_t)i, clamped_gluf_(gu[t * 2 * ff + j], gu[t * 2 * ff + ff + j], limit, alpha));
+    const int64_t g = t * 2 * ff + (IL ? (j & ~15) + j : j);
+    st<TO>(out, (size_t)i, clamped_gluf_(gu[g], gu[g + (IL ? 16 : ff)], limit, alpha));
 }
 
 // ------------------------------------------------------------------------------------------------------------ attention
@@ -2108,14 +2110,22 @@ int mi355_hyb_gather_norm(void* out, int32_t out_dtype, const float* x, const in
     LAUNCH_OK(); return 0;
 }
 
-int mi355_hyb_clamped_glu(void* out, int32_t out_dtype, const float* gu, int32_t T, int32_t ff, float limit, float alpha, int64_t stream) {
-    if (!out || !gu || ff <= 0 || !is_dt(out_dtype)) return -1;
+static int clamped_glu_launch(bool il, void* out, int32_t out_dtype, const float* gu, int32_t T, int32_t ff, float limit, float alpha, int64_t stream) {
+    if (!out || !gu || ff <= 0 || (il && ff % 16) || !is_dt(out_dtype)) return -1;
     const int64_t n = (int64_t)T * ff;
     if (n <= 0) return 0;
     const unsigned grid = (unsigned)((n + 255) / 256);
-    if (out_dtype == MI355_DTYPE_F32) clamped_glu_kernel<float><<<grid, 256, 0, to_stream(stream)>>>((float*)out, gu, n, ff, limit, alpha);
-    else clamped_glu_kernel<uint16_t><<<grid, 256, 0, to_stream(stream)>>>((uint16_t*)out, gu, n, ff, limit, alpha);
+#define CLAMPED_GLU_GO(TO, IL) clamped_glu_kernel<TO, IL><<<grid, 256, 0, to_stream(stream)>>>((TO*)out, gu, n, ff, limit, alpha)
+    if (out_dtype == MI355_DTYPE_F32) { if (il) CLAMPED_GLU_GO(float, true); else CLAMPED_GLU_GO(float, false); }
+    else if (il) CLAMPED_GLU_GO(uint16_t, true); else CLAMPED_GLU_GO(uint16_t, false);
+#undef CLAMPED_GLU_GO
     LAUNCH_OK(); return 0;
+}
+int mi355_hyb_clamped_glu(void* out, int32_t out_dtype, const float* gu, int32_t T, int32_t ff, float limit, float alpha, int64_t stream) {
+    return clamped_glu_launch(false, out, out_dtype, gu, T, ff, limit, alpha, stream);
+}
+int mi355_hyb_clamped_glu_interleaved(void* out, int32_t out_dtype, const float* gu, int32_t T, int32_t ff, float limit, float alpha, int64_t stream) {
+    return clamped_glu_launch(true, out, out_dtype, gu, T, ff, limit, alpha, stream);
 }
 
 int mi355_hyb_attn_prepare(void* q_out, void* k_pages, void* v_pages, const float* proj, int32_t ldp, int32_t q_off, int32_t k_off,
@@ -2644,6 +2654,19 @@ int mi355_hyb_linear_clamped_glu(void* out, int32_t out_dtype, int32_t ldo, cons
     if (!is_dt(out_dtype)) return -1;
     return linear_launch(static_cast<float*>(out), ldo, 0, a, dtype, lda, 0, w, 0, nullptr, T, 2 * ff, k, 1, dtype, stream, LIN_ACT_CLAMPED, 0,
                          out_dtype == MI355_DTYPE_BF16, nullptr, 1, limit, alpha);
+}
+// Whether a bf16 model's clamped gate/up is one launch, or the product over the same interleaved rows and mi355_hyb_clamped_glu_interleaved.  Up to 16 tokens stream the
+// weights, 32 rows per workgroup in one launch and 16 in the other: what counts is how the rows divide over the CUs and, at few of them, the activation's launch.
+// us on cold weights, one launch / two (tokens, ff, k):
+//   to 8 tokens, as many rows on the fullest CU either way: 8, 8192, 2048 18.5 / 20.5; 4, 3072, 2048 11.6 / 11.9; 1, 12288, 4096 41.1 / 42.1 -- but 4, 3584, 3072 16.2 / 14.7,
+//   where few rows wait for many columns; more rows on it with one: 4, 1024, 4096 17.5 / 14.6; 1, 5632, 4096 25.3 / 22.3
+//   9 to 16, where one launch reads x half as often: 16, 5632, 4096 32.1 / 32.1; 16, 2304, 4096 20.3 / 20.7; only below half a card it is slower, 16, 2048, 4096 19.9 / 16.5
+//   k to 1024: 8, 2048, 1024 10.5 / 10.8.  More tokens: one (2100, 8192, 2048 168 / 199)
+int32_t mi355_internal_hyb_clamped_fused(int32_t T, int32_t ff, int32_t k, int32_t dtype) {
+    if (T > 16 || k <= 1024 || dtype != MI355_DTYPE_BF16) return 1;
+    const int cus = mi355_num_cus(), one = ff / 16, two = ff / 8;
+    if (T > 8) return two > cus;
+    return 2 * ((one + cus - 1) / cus) <= (two + cus - 1) / cus && (k <= 2048 || two > 2 * cus);
 }
 int mi355_hyb_interleave_gate_up(void* out, const void* in, int32_t matrices, int32_t ff, int32_t k, int32_t dtype, int64_t stream) {
     if (!out || !in || out == in || matrices <= 0 || ff <= 0 || ff % 16 || k <= 0 || !is_dt(dtype)) return -1;

@@ -32,6 +32,7 @@
 
 extern "C" {
 int mi355_hyb_token_seq(int32_t*, const uint32_t*, int32_t, int64_t);
+int32_t mi355_internal_hyb_clamped_fused(int32_t T, int32_t ff, int32_t k, int32_t dtype);
 int mi355_hyb_bf16_to_f32(float*, const uint16_t*, int64_t, int64_t);
 int mi355_hyb_fill_f32(float*, float, int64_t, int64_t);
 int mi355_hyb_embed(float*, void*, const void*, const uint32_t*, int32_t, int32_t, int32_t, int32_t, int64_t);
@@ -783,6 +784,10 @@ static int forward_enqueue(HModel* m, const uint32_t* tokens, const int64_t* pos
     // gate, up and activation of a dense feed-forward (kinds 1, 2, 6)
     auto dense_gate_up = [&](const HLayer& WL) -> int {
         const int ff = WL.c.mlp_ff, kind = WL.c.mlp_kind;
+        if (WL.glu_dense() && kind == 1 && !mi355_internal_hyb_clamped_fused(T, ff, W, dt)) {
+            HCHECK(mi355_hyb_linear(m->gu, 2 * ff, xin, xin_dt, W, WL.w[MI355_HW_MLP_GATE_UP].p, nullptr, T, 2 * ff, W, dt, stream));
+            return mi355_hyb_clamped_glu_interleaved(m->act, dt, m->gu, T, ff, WL.c.mlp_limit, WL.c.mlp_alpha, stream);
+        }
         if (WL.glu_dense() && kind == 1)
             return mi355_hyb_linear_clamped_glu(m->act, dt, ff, xin, W, WL.w[MI355_HW_MLP_GATE_UP].p, T, ff, W, WL.c.mlp_limit, WL.c.mlp_alpha, dt, stream);
         if (WL.glu_dense())

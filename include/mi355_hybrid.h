@@ -655,6 +655,9 @@ int mi355_hyb_mingru(void* out, int32_t out_dtype, float* state, int64_t state_s
 /* out (dt_out) [T, ff] = g sigmoid(alpha g) (u + 1), g = min(gu[:, j], limit), u = clamp(gu[:, ff + j], -limit, limit) */
 int mi355_hyb_clamped_glu(void* out, int32_t out_dtype, const float* gu, int32_t num_tokens, int32_t ff, float limit, float alpha,
                           int64_t stream);
+/* the same of a product over mi355_hyb_interleave_gate_up's rows: 16 gate columns, their 16 up columns, the next 16 gate columns, ... (ff a multiple of 16) */
+int mi355_hyb_clamped_glu_interleaved(void* out, int32_t out_dtype, const float* gu, int32_t num_tokens, int32_t ff, float limit, float alpha,
+                                      int64_t stream);
 
 #ifdef __cplusplus
 }
