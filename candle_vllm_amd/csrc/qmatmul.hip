@@ -1995,7 +1995,8 @@ static thread_local int g_qpw_last = -1;
 extern "C" int32_t mi355_internal_last_qpw(void) { return g_qpw_last; }
 // Which kernel makes a prompt product: us per k-block and round of workgroups (one per CU; the 64 x 256 tile of qmm_prefill.inc: two), a full round and
 // one that leaves most of the chip idle (it runs at a higher clock).  Both sides measured at 19 sizes of 96 .. 4096 tokens for 14 matrices of 1024 x 4096 ..
-// 28672 x 4096: with the choice 1.09 x as fast on average as with 64 x 256 tiles alone (Q4_K up to 1.34 x, Q6_K 1.92 x), nowhere slower by more than 2 %.
+// 28672 x 4096: with the choice 1.09 x as fast on average as with 64 x 256 tiles alone (Q4_K up to 1.34 x, Q6_K 1.92 x); 270 drawn products and 190 q | k | v of
+// 96 .. 4500 tokens: 0.48 .. 1.03 of their time.
 struct QpwChoice { int tile; float us; };
 static QpwChoice qpw_pick(int type, int T, int n_slots, int K, float old_extra_us) {
     const int cus = mi355_num_cus(), nkb = K >> 8;
