@@ -2,7 +2,7 @@
 // block engine's pages, the gated delta rule and the minGRU over the block engine's state slots, the short causal convolution in
 // front of the delta rule, and the f32-residual glue around them.  Numerics: residual stream, norms, scores, probabilities,
 // decays, gates of a recurrence and all recurrent state are f32; MI355_DTYPE_BF16 keeps matrices, K/V pages and the operands of
-// a matrix product in bf16 (matrix cores, f32 accumulation), MI355_DTYPE_F32 multiplies with f32 FMAs.
+// a matrix product in bf16 (matrix cores, f32 accumulation), MI355_DTYPE_F32 multiplies in f32 (the matrix cores' f32 mode).
 // One step function serves prompts, portions of prompts and decoded tokens: a sequence brings cu_q[s+1] - cu_q[s] new tokens behind
 // ctx[s] - that many cached ones; a portion that starts at position 0 starts from zero state whatever its slot holds.
 #include <hip/hip_runtime.h>
@@ -407,52 +407,210 @@ template <typename TA, int NW, int UNR, int B> __global__ __launch_bounds__(64 *
     }
 }
 
-// f32 weights and operands: plain FMAs in f32 (no reduced-precision matrix mode).  64 x 64 tile, 16-wide K steps through LDS,
-// every thread owns 4 tokens x 4 columns.
-template <int B> __global__ __launch_bounds__(256) void linear_f32_kernel(LinArgs p) {
-    __shared__ float As[16][68], Ws[16][68];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int n0 = blockIdx.x * 64, t0 = blockIdx.y * 64;
+// ---- f32 weights and operands, on the matrix cores' f32 mode (every product and sum in f32; no reduced-precision operand) ----
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+// 4 consecutive operands of a row, zero beyond `kend`
+__device__ __forceinline__ float4 frag4(const float* row, int k, int kend, bool vec_ok) {
+    if (vec_ok && k + 4 <= kend) return *reinterpret_cast<const float4*>(row + k);
+    float4 f;
+    f.x = k < kend ? row[k] : 0.f; f.y = k + 1 < kend ? row[k + 1] : 0.f;
+    f.z = k + 2 < kend ? row[k + 2] : 0.f; f.w = k + 3 < kend ? row[k + 3] : 0.f;
+    return f;
+}
+
+// Few tokens: a stream over the weights, as the bf16 kernel above.  A workgroup owns 16 weight rows (GLU: a gate and an up tile) and 16 MT tokens; its NW
+// waves take 16 UNR columns in turn and add their partial tiles through LDS.  Lane (m16, kg) loads four consecutive k of its row: matrix instruction j
+// of a step multiplies element j of every lane, so a step is 16 columns in another order on both sides alike.
+template <int NW, int UNR, int MT, int B> __global__ __launch_bounds__(64 * NW) void linear_f32_stream_kernel(LinArgs p) {
+    constexpr int NC = B == LIN_GLU_BUILD ? 2 : 1;
+    __shared__ float part[NW][NC * MT * 4][64];
+    lin_batch<float, B>(p, blockIdx.x * 16);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m16 = lane & 15, kg = lane >> 4;
+    const int n = blockIdx.x * 16 * NC + m16, t0 = blockIdx.y * 16 * MT;
+    const bool nok = n < p.N;
+    const float* wrow = static_cast<const float*>(p.w) + (int64_t)blockIdx.z * p.w_bs + (size_t)(nok ? n : 0) * p.K;
+    const float* arow[MT];
+    bool aok[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        aok[m] = t0 + 16 * m + m16 < p.T;
+        arow[m] = static_cast<const float*>(p.a) + (size_t)(aok[m] ? t0 + 16 * m + m16 : 0) * p.lda;
+    }
+    f32x4_t acc[NC][MT];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[c][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave * 16 * UNR; k0 < p.K; k0 += NW * 16 * UNR) {
+        float4 a[MT][UNR], b[NC][UNR];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) {
+            const int k = k0 + 16 * u + 4 * kg;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) b[c][u] = (nok && k < p.K) ? frag4(wrow + (size_t)(16 * c) * p.K, k, p.K, p.w_vec) : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int m = 0; m < MT; ++m) a[m][u] = (aok[m] && k < p.K) ? frag4(arow[m], k, p.K, p.a_vec) : float4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int u = 0; u < UNR; ++u)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        acc[c][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float*>(&a[m][u])[j],
+                                                                         reinterpret_cast<const float*>(&b[c][u])[j], acc[c][m], 0, 0, 0);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) part[wave][(c * MT + m) * 4 + v][lane] = acc[c][m][v];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 256 * MT; i += 64 * NW) {
+        const int q = i >> 6, l = i & 63;                            // q = 4 m + v
+        float s[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            s[c] = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) s[c] += part[w][c * MT * 4 + q][l];
+        }
+        const int t = t0 + 16 * (q >> 2) + 4 * (l >> 4) + (q & 3), col = blockIdx.x * 16 * NC + (l & 15);
+        if (col >= p.N || t >= p.T) continue;
+        if (B == LIN_GLU_BUILD) lin_store_glu(p, t, blockIdx.x * 16 + (l & 15), s[0], s[NC - 1]);
+        else lin_store<B>(p, t, col, s[0] + (p.bias ? p.bias[col] : 0.f));
+    }
+}
+
+// More tokens: tiles of 64 MF tokens x 64 NF columns, KS groups of four waves that take the 16-wide K slices in turn (KS = 2 where the tiles are few) and
+// add up through LDS at the end.  A slice goes from global memory into registers PF slices ahead, then into one of two LDS buffers (rows of 16 + 4 floats:
+// the eight rows that a ds_read_b128 serves at a time start on different banks), from where every wave multiplies its quarter by 32x32x2 instructions --
+// again with four consecutive k per lane, one to an instruction.
+template <int MF, int NF, int KS, int PF, int B> __global__ __launch_bounds__(256 * KS) void linear_f32_gemm_kernel(LinArgs p) {
+    constexpr int BM = 64 * MF, BN = 64 * NF, ROWS = BM + BN, LD = 20, NL = ROWS / 64;   // NL float4 per thread and slice
+    constexpr int TILE = KS * 2 * ROWS * LD, RED = KS > 1 ? (KS - 1) * BM * BN : 1;
+    __shared__ float smem[TILE > RED ? TILE : RED];
+    const int tid = threadIdx.x & 255, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, c32 = lane & 31, h = lane >> 5, wm = wave >> 1, wn = wave & 1;
+    const int n0 = blockIdx.x * BN, t0 = blockIdx.y * BM;
     lin_batch<float, B>(p, n0);
     int64_t w_off;
     if (!lin_group(p, t0, w_off)) return;
-    const float* A = static_cast<const float*>(p.a);
-    const float* W = static_cast<const float*>(p.w) + w_off;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < p.K; k0 += 16) {
+    // thread (row r, k quarter) of a slice: rows r = tid / 4 + 64 i of [tokens | columns]
+    const int kq = 4 * (tid & 3);
+    const float* src[NL];
+    bool ok[NL];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = threadIdx.x + r * 256;            // 1024 elements of each 64 x 16 tile
-            const int row = idx >> 4, kk = idx & 15;
-            const int k = k0 + kk;
-            As[kk][row] = (t0 + row < p.T && k < p.K) ? A[(size_t)lin_row(p, t0 + row) * p.lda + k] : 0.f;
-            Ws[kk][row] = (n0 + row < p.N && k < p.K) ? W[(size_t)(n0 + row) * p.K + k] : 0.f;
+    for (int i = 0; i < NL; ++i) {
+        const int r = (tid >> 2) + 64 * i;
+        if (i < MF) {
+            ok[i] = t0 + r < p.T;
+            src[i] = static_cast<const float*>(p.a) + (size_t)(ok[i] ? lin_row(p, t0 + r) : 0) * p.lda;
+        } else {
+            ok[i] = n0 + r - BM < p.N;
+            src[i] = static_cast<const float*>(p.w) + w_off + (size_t)(ok[i] ? n0 + r - BM : 0) * p.K;
         }
-        __syncthreads();
+    }
+    float4 reg[PF][NL];
+    auto fetch = [&](float4 (&to)[NL], int slice) {
+        const int k = 16 * slice + kq;
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            float a[4], w[4];
+        for (int i = 0; i < NL; ++i) to[i] = (ok[i] && k < p.K) ? frag4(src[i], k, p.K, i < MF ? p.a_vec : p.w_vec) : float4{0.f, 0.f, 0.f, 0.f};
+    };
+    f32x16_t acc[MF][NF];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) { a[i] = As[kk][ty * 4 + i]; w[i] = Ws[kk][tx * 4 + i]; }
+    for (int m = 0; m < MF; ++m)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int n = 0; n < NF; ++n)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
+            for (int v = 0; v < 16; ++v) acc[m][n][v] = 0.f;
+    const int slices = (p.K + 15) / 16, rounds = (slices + KS - 1) / KS;   // (the last slices of a group past K are zeros)
+    float* base = smem + grp * 2 * ROWS * LD;
+#pragma unroll
+    for (int u = 0; u < PF; ++u) fetch(reg[u], u * KS + grp);
+    for (int r0 = 0; r0 < rounds; r0 += PF) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            if (r0 + u < rounds) {                                         // (the same for every wave)
+                float* buf = base + ((r0 + u) & 1) * ROWS * LD;
+#pragma unroll
+                for (int i = 0; i < NL; ++i) *reinterpret_cast<float4*>(buf + ((tid >> 2) + 64 * i) * LD + kq) = reg[u][i];
+                fetch(reg[u], (r0 + u + PF) * KS + grp);
+                __syncthreads();
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    float4 a[MF], b[NF];
+#pragma unroll
+                    for (int m = 0; m < MF; ++m) a[m] = *reinterpret_cast<const float4*>(buf + (wm * 32 * MF + 32 * m + c32) * LD + 8 * s + 4 * h);
+#pragma unroll
+                    for (int n = 0; n < NF; ++n) b[n] = *reinterpret_cast<const float4*>(buf + (BM + wn * 32 * NF + 32 * n + c32) * LD + 8 * s + 4 * h);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int m = 0; m < MF; ++m)
+#pragma unroll
+                            for (int n = 0; n < NF; ++n)
+                                acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(reinterpret_cast<const float*>(&a[m])[j],
+                                                                                 reinterpret_cast<const float*>(&b[n])[j], acc[m][n], 0, 0, 0);
+                }
+            }
         }
+    }
+    if (KS > 1) {
+        __syncthreads();                                                   // every wave is done with the slices
+        if (grp)
+#pragma unroll
+            for (int m = 0; m < MF; ++m)
+#pragma unroll
+                for (int n = 0; n < NF; ++n)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) smem[(((grp - 1) * 4 + wave) * MF * NF * 16 + (m * NF + n) * 16 + v) * 64 + lane] = acc[m][n][v];
         __syncthreads();
+        if (grp) return;
+#pragma unroll
+        for (int g = 0; g < KS - 1; ++g)
+#pragma unroll
+            for (int m = 0; m < MF; ++m)
+#pragma unroll
+                for (int n = 0; n < NF; ++n)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[m][n][v] += smem[((g * 4 + wave) * MF * NF * 16 + (m * NF + n) * 16 + v) * 64 + lane];
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int t = t0 + ty * 4 + i;
-        if (B != LIN_GLU_BUILD && t >= p.T) continue;
+    for (int m = 0; m < MF; ++m)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (B == LIN_GLU_BUILD) {                                       // the up column of a gate column is four threads further
-                const float up = __shfl_xor(acc[i][j], 4);
-                if (!(tx & 4) && n < p.N && t < p.T) lin_store_glu(p, t, (n & ~31) / 2 + (n & 15), acc[i][j], up);
-            } else if (n < p.N) lin_store<B>(p, t, n, acc[i][j] + (p.bias ? p.bias[n] : 0.f));
+        for (int n = 0; n < NF; ++n) {
+            const int col = n0 + wn * 32 * NF + 32 * n + c32;
+            const float bias = (B != LIN_GLU_BUILD && p.bias && col < p.N) ? p.bias[col] : 0.f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int t = t0 + wm * 32 * MF + 32 * m + 8 * (v >> 2) + 4 * h + (v & 3);
+                if (B == LIN_GLU_BUILD) {                                   // the up column of a gate column is 16 lanes further
+                    const float up = __shfl_xor(acc[m][n][v], 16);
+                    if (!(c32 & 16) && col < p.N && t < p.T) lin_store_glu(p, t, (col & ~31) / 2 + (col & 15), acc[m][n][v], up);
+                } else if (col < p.N && t < p.T) lin_store<B>(p, t, col, acc[m][n][v] + bias);
+            }
         }
+}
+
+// f32 products by the number of 64 x 64 tiles: under half a card's worth (and up to 32 tokens) the streaming kernel, 16 or 32 tokens to a workgroup; then the
+// tiles, three groups of waves to a tile up to two tiles per unit, two beyond.  us, the FMA kernel that took all of them before / this one / the other side of the line:
+// 2 tokens 2048 x 8192 1290 / 29;  2 tokens 32000 x 2048 396 / 55;  300 tokens x 16384 (gate/up) x 2048 412 / 198;  100 tokens 2048 x 8192 stream 102, tiles 175;
+// 200 tokens 46 and 48 (2048 x 2048);  130 tokens 3072 x 3072 tiles 70, stream 72;  500 tokens 2048 x 8192 three groups 177, two 190;  2048 tokens 9360 x 2048
+// two groups 693 (113 TFLOP/s of 157), three 744, tiles of 128 x 128 692.
+template <int B> static void linear_f32_launch(const LinArgs& p, unsigned nz, hipStream_t st) {
+    const int T = p.T, n = p.N, cus = mi355_num_cus();
+    const int64_t cols = B == LIN_GLU_BUILD ? n / 32 : (n + 15) / 16, tiles = (int64_t)((n + 63) / 64) * ((T + 63) / 64) * nz;
+    if (T <= 32 || 2 * tiles <= cus) {
+        if (T <= 16 || cols * ((T + 31) / 32) * nz < cus) linear_f32_stream_kernel<16, 2, 1, B><<<dim3((unsigned)cols, (T + 15) / 16, nz), 1024, 0, st>>>(p);
+        else linear_f32_stream_kernel<16, 2, 2, B><<<dim3((unsigned)cols, (T + 31) / 32, nz), 1024, 0, st>>>(p);
+    } else {
+        const dim3 grid((n + 63) / 64, (T + 63) / 64, nz);
+        if (tiles <= 2 * cus) linear_f32_gemm_kernel<1, 1, 3, 2, B><<<grid, 768, 0, st>>>(p);
+        else linear_f32_gemm_kernel<1, 1, 2, 2, B><<<grid, 512, 0, st>>>(p);
     }
 }
 
@@ -2026,7 +2184,9 @@ static int linear_launch(float* out, int32_t ldo, int64_t o_bs, const void* a, i
     const unsigned nz = (unsigned)batch;
     if (dtype == MI355_DTYPE_F32) {
         if (a_dtype != MI355_DTYPE_F32) return -1;
-        LIN_EPI(p, (linear_f32_kernel<EPI><<<dim3((n + 63) / 64, (T + 63) / 64, nz), 256, 0, st_>>>(p)));
+        p.w_vec = (k % 4 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 4 == 0);
+        p.a_vec = (lda % 4 == 0) && ((uintptr_t)a % 16 == 0) && (a_bs % 4 == 0);
+        LIN_EPI(p, (linear_f32_launch<EPI>(p, nz, st_)));
         LAUNCH_OK(); return 0;
     }
     const int a_bytes = a_dtype == MI355_DTYPE_F32 ? 4 : 2;
@@ -2606,7 +2766,9 @@ static int grouped_launch(void* out, int32_t out_dtype, int32_t ldo, const void*
     hipStream_t st_ = to_stream(stream);
     if (dtype == MI355_DTYPE_F32) {
         if (a_dtype != MI355_DTYPE_F32 || block_rows != 64) return -1;
-        LIN_EPI2(p, (linear_f32_kernel<EPI><<<dim3((n + 63) / 64, n_blocks, 1), 256, 0, st_>>>(p)));
+        p.w_vec = (k % 4 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 4 == 0);
+        p.a_vec = (lda % 4 == 0) && ((uintptr_t)a % 16 == 0);
+        LIN_EPI2(p, (linear_f32_gemm_kernel<1, 1, 2, 2, EPI><<<dim3((n + 63) / 64, n_blocks, 1), 512, 0, st_>>>(p)));
         LAUNCH_OK(); return 0;
     }
     const int a_bytes = a_dtype == MI355_DTYPE_F32 ? 4 : 2;

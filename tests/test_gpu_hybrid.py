@@ -79,6 +79,54 @@ def test_linear(lib, dtype, a_f32, T, n, k):
     assert np.all(got[:, n:] == 7.0)                                       # columns beyond n are not touched
 
 
+# every form of the f32 products (16 and 32 tokens to a workgroup, tiles by three and by two groups of waves) and of the bf16 stream (8 and 16 waves; more tiles
+# than units with few and with more tokens), with rows, columns and k that fill neither tile nor slice, aligned operands and not
+@pytest.mark.parametrize("dtype,T,n,k,skew", [
+    (F32, 1, 17, 2051, 0), (F32, 16, 4112, 520, 0), (F32, 21, 40, 1000, 1), (F32, 48, 2063, 519, 0), (F32, 33, 4100, 64, 0), (F32, 65, 48, 4096, 0),
+    (F32, 130, 3090, 516, 0), (F32, 300, 2100, 63, 1), (F32, 1030, 2180, 200, 0), (F32, 1031, 2179, 33, 0),
+    (BF16, 1, 100, 520, 0), (BF16, 8, 4090, 2088, 0), (BF16, 9, 4090, 1032, 0), (BF16, 16, 20, 4103, 1), (BF16, 4, 5000, 512, 0), (BF16, 5, 5000, 1000, 0), (BF16, 16, 9001, 513, 1)])
+def test_linear_forms(lib, dtype, T, n, k, skew):
+    """against 64 bits, within what any order of k f32 products and sums stays in: (k + 2) 2^-24 sum |a w|.  The product's own rows only: a NaN row, an infinite
+    one and one of products below the normal numbers leave the others alone"""
+    _gpu()
+    torch.manual_seed(T + n + k)
+    td = torch.float32 if dtype == F32 else torch.bfloat16
+    a, w = torch.randn(T * (k + 8) + 8, device="cuda").to(td)[skew:], (torch.randn(n * k + 8, device="cuda") * k ** -0.5).to(td)[skew:]
+    A, W, b = a[:T * (k + 8)].view(T, k + 8)[:, :k], w[:n * k].view(n, k), torch.randn(n, device="cuda")
+    if T > 4:
+        A[1, k - 1], A[2, 0] = float("nan"), float("inf")
+        A[3] *= 2.0 ** -100
+        W[5 % n] = W[5 % n] * 2.0 ** -30
+    out = torch.full((T, n + 3), 7.0, device="cuda")
+    ok(lib.mi355_hyb_linear(out.data_ptr(), n + 3, A.data_ptr(), dtype, k + 8, W.data_ptr(), b.data_ptr(), T, n, k, dtype, _st()))
+    want, bound = A.double() @ W.double().t() + b.double(), (k + 2) * 2.0 ** -24 * (A.double().abs() @ W.double().abs().t() + b.double().abs()) + 1e-44
+    keep = [t for t in range(T) if T <= 4 or t not in (1, 2)]
+    assert ((out[keep, :n].double() - want[keep]).abs() <= bound[keep]).all()
+    assert (out[:, n:] == 7.0).all()
+    if T > 4:
+        assert out[1, :n].isnan().all() and not out[2, :n].isfinite().any()
+        none = torch.zeros(n, device="cuda")
+        ok(lib.mi355_hyb_linear(out.data_ptr(), n + 3, A.data_ptr(), dtype, k + 8, W.data_ptr(), none.data_ptr(), T, n, k, dtype, _st()))
+        small = A[3].double() @ W[5 % n].double()                           # about 2^-130
+        assert abs(out[3, 5 % n].item() - small.item()) <= k * 2.0 ** -148, (out[3, 5 % n].item(), small.item())
+
+
+@pytest.mark.parametrize("T,ff,k", [(1, 48, 520), (8, 4112, 512), (9, 4112, 1028), (20, 48, 200), (40, 2064, 100), (130, 1040, 516), (300, 2064, 68)])
+@pytest.mark.parametrize("dtype", [F32, BF16])
+def test_gate_and_up_forms(lib, dtype, T, ff, k):
+    """interleaved gate/up products in every form, against 64 bits: an f32 sum is within (k + 2) 2^-24 sum |a w|, and silu(g) u moves by at most 1.1 |u| dg + |g| du"""
+    _gpu()
+    torch.manual_seed(T + ff + k)
+    td = torch.float32 if dtype == F32 else torch.bfloat16
+    a, w = torch.randn(T, k, device="cuda").to(td), (torch.randn(2 * ff, k, device="cuda") * k ** -0.5).to(td)
+    out = torch.full((T, ff + 3), 7.0, device="cuda")
+    ok(lib.mi355_hyb_linear_glu(out.data_ptr(), F32, ff + 3, a.data_ptr(), k, w.data_ptr(), T, ff, k, 1, dtype, _st()))
+    z, e = ((x.view(T, ff // 16, 2, 16) for x in (a.double() @ w.double().t(), (k + 2) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t()))))
+    g, u, dg, du = z[:, :, 0], z[:, :, 1], e[:, :, 0], e[:, :, 1]
+    want, bound = torch.nn.functional.silu(g) * u, 1.1 * u.abs() * dg + g.abs() * du + 1e-6 * (1 + (g * u).abs())
+    assert ((out[:, :ff].double() - want.reshape(T, ff)).abs() <= bound.reshape(T, ff)).all() and (out[:, ff:] == 7.0).all()
+
+
 def test_norm_add_and_glu(lib):
     _gpu()
     rng = np.random.default_rng(1)
