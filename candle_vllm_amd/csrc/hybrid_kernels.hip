@@ -407,6 +407,28 @@ template <typename TA, int NW, int UNR, int B> __global__ __launch_bounds__(64 *
     }
 }
 
+// How many waves a row tile gets and how much each has in flight.  What bounds a tile is its waves' round trips to memory, so tiles that leave compute units
+// idle get up to 16 waves; where every unit has several, fewer waves with less each, which the units take up one behind the other.  us on cold weights with
+// four waves of four steps (the only form before) / with the form chosen here, at 1, 8 and 16 tokens:
+//   up to a tile per unit   2048 x 2048 5.9 6.7 / 4.8 5.8;  2048 x 8192 21.0 22.7 / 12.2 15.4;  4096 x 4096 12.7 13.6 14.3 / 9.0 10.1 11.5;  4096 x 14336 39 42 44 / 24 30 34
+//   up to two               8192 x 1024 5.6 6.2 / 5.0 6.2;  5120 x 5120 18.2 20.1 25.5 / 15.8 20.1 25.5 (from five tokens on two steps lose: 22.5 27.3)
+//   more                    12288 x 2048 13.2 15.8 / 13.0 15.0;  32000 x 2048 29.1 36.2 / 27.6 33.4
+//   gate/up pairs           8192 x 2048 12.2 13.2 13.3 / 10.3 12.0 12.6;  16384 x 2048 17.4 19.6 / 16.9 18.4;  11264 x 4096 26.1 29.4 32.3 / 25.0 26.8 29.1
+// Below 512 columns there is nothing to split (2048 x 256 2.9 at 8 tokens with two waves of two steps, 3.0 with 16 waves), at 512 it begins to pay: 3.6 / 3.0.
+template <typename TA, int B> static void linear_stream_launch(const LinArgs& p, dim3 grid, hipStream_t st) {
+    const int64_t tiles = (int64_t)grid.x * grid.z;
+    const int cus = mi355_num_cus();
+    if (p.K < 512) linear_bf16_stream_kernel<TA, 2, 2, B><<<grid, 128, 0, st>>>(p);
+    else if (B == LIN_GLU_BUILD) {
+        if (tiles <= cus) linear_bf16_stream_kernel<TA, 8, 4, B><<<grid, 512, 0, st>>>(p);
+        else linear_bf16_stream_kernel<TA, 4, 2, B><<<grid, 256, 0, st>>>(p);
+    } else if (tiles <= cus) {
+        if (p.T <= 8) linear_bf16_stream_kernel<TA, 16, 2, B><<<grid, 1024, 0, st>>>(p);
+        else linear_bf16_stream_kernel<TA, 8, 4, B><<<grid, 512, 0, st>>>(p);
+    } else if (p.T <= 4 || tiles > 2 * cus) linear_bf16_stream_kernel<TA, 8, 2, B><<<grid, 512, 0, st>>>(p);
+    else linear_bf16_stream_kernel<TA, 4, 4, B><<<grid, 256, 0, st>>>(p);
+}
+
 // ---- f32 weights and operands, on the matrix cores' f32 mode (every product and sum in f32; no reduced-precision operand) ----
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 // 4 consecutive operands of a row, zero beyond `kend`
@@ -2195,8 +2217,7 @@ static int linear_launch(float* out, int32_t ldo, int64_t o_bs, const void* a, i
     const bool af = a_dtype == MI355_DTYPE_F32;
     if (T <= 16) {
         const dim3 grid(glu ? n / 32 : (n + 15) / 16, 1, nz);
-        if (k >= 2048) { if (af) LIN_EPI_(p, (linear_bf16_stream_kernel<float, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); else LIN_EPI(p, (linear_bf16_stream_kernel<uint16_t, 4, 4, EPI><<<grid, 256, 0, st_>>>(p))); }
-        else { if (af) LIN_EPI_(p, (linear_bf16_stream_kernel<float, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); else LIN_EPI(p, (linear_bf16_stream_kernel<uint16_t, 2, 2, EPI><<<grid, 128, 0, st_>>>(p))); }
+        if (af) LIN_EPI_(p, (linear_stream_launch<float, EPI>(p, grid, st_))); else LIN_EPI(p, (linear_stream_launch<uint16_t, EPI>(p, grid, st_)));
     } else if (linear_gemm_ok(p, af)) {
         // (segments end at multiples of 128 columns: only the tiles of that width have one left operand each)
         const GtChoice c = gt_pick([&](const GtTile& t) { return (int64_t)((T + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch; }, k / 64,
@@ -2820,10 +2841,11 @@ int mi355_hyb_linear_clamped_glu(void* out, int32_t out_dtype, int32_t ldo, cons
 // Whether a bf16 model's clamped gate/up is one launch, or the product over the same interleaved rows and mi355_hyb_clamped_glu_interleaved.  Up to 16 tokens stream the
 // weights, 32 rows per workgroup in one launch and 16 in the other: what counts is how the rows divide over the CUs and, at few of them, the activation's launch.
 // us on cold weights, one launch / two (tokens, ff, k):
-//   to 8 tokens, as many rows on the fullest CU either way: 8, 8192, 2048 18.5 / 20.5; 4, 3072, 2048 11.6 / 11.9; 1, 12288, 4096 41.1 / 42.1 -- but 4, 3584, 3072 16.2 / 14.7,
-//   where few rows wait for many columns; more rows on it with one: 4, 1024, 4096 17.5 / 14.6; 1, 5632, 4096 25.3 / 22.3
-//   9 to 16, where one launch reads x half as often: 16, 5632, 4096 32.1 / 32.1; 16, 2304, 4096 20.3 / 20.7; only below half a card it is slower, 16, 2048, 4096 19.9 / 16.5
-//   k to 1024: 8, 2048, 1024 10.5 / 10.8.  More tokens: one (2100, 8192, 2048 168 / 199)
+//   to 8 tokens, as many rows on the fullest CU either way: 8, 8192, 2048 18.6 / 20.7; 4, 3072, 2048 10.3 / 11.2 -- but 4, 2048, 3072 12.2 / 10.4,
+//   where few rows wait for many columns; more rows on it with one: 4, 1024, 4096 12.2 / 10.1; 1, 5632, 4096 26.3 / 24.6
+//   9 to 16, where one launch reads x half as often: 16, 5632, 4096 30.9 / 33.0; 16, 2304, 4096 18.1 / 20.8; only below half a card it is slower, 16, 2048, 4096 17.7 / 14.4
+//   k to 1024: 8, 2048, 1024 6.2 / 6.7.  More tokens: one (2100, 8192, 2048 168 / 199)
+// Over 144 sizes (k 2048 ... 5120) what it picks is on average 0.5 % behind the faster side, at most 13 % (1, 2048, 2048: 7.1 for two launches, 7.9).
 int32_t mi355_internal_hyb_clamped_fused(int32_t T, int32_t ff, int32_t k, int32_t dtype) {
     if (T > 16 || k <= 1024 || dtype != MI355_DTYPE_BF16) return 1;
     const int cus = mi355_num_cus(), one = ff / 16, two = ff / 8;
