@@ -1991,20 +1991,43 @@ static int qpw_go(const QmmArgs& r, const QpgImg& im, int n_slots, hipStream_t s
     return (int)hipGetLastError();
 }
 // tile of this thread's last prompt product (tests: which kernel ran)
-static thread_local int g_qpw_last = -1;
+static thread_local int g_qpw_last = -1, g_qpg_split_last = 1;
 extern "C" int32_t mi355_internal_last_qpw(void) { return g_qpw_last; }
+extern "C" int32_t mi355_internal_last_qpg_split(void) { return g_qpg_split_last; }   // ranges of K
 // Which kernel makes a prompt product: us per k-block and round of workgroups (one per CU; the 64 x 256 tile of qmm_prefill.inc: two), a full round and
 // one that leaves most of the chip idle (it runs at a higher clock).  Both sides measured at 19 sizes of 96 .. 4096 tokens for 14 matrices of 1024 x 4096 ..
 // 28672 x 4096: with the choice 1.09 x as fast on average as with 64 x 256 tiles alone (Q4_K up to 1.34 x, Q6_K 1.92 x); 270 drawn products and 190 q | k | v of
 // 96 .. 4500 tokens: 0.48 .. 1.03 of their time.
 struct QpwChoice { int tile; float us; };
+// us per k-block of `wgs` workgroups
+static float qpw_rounds(int wgs, int cap, float full, float light) {
+    const int cus = mi355_num_cus(), left = wgs % cap;
+    // two workgroups per CU: up to half a round they have a CU each
+    const float last = !left ? 0.f : cap > cus ? (left <= cus ? light : full) : light + (full - light) * (float)left / (float)cap;
+    return full * (float)(wgs / cap) + last;
+}
+// us of a launch of qmm_prefill.inc's 64 x 256 tiles over all of K
+static float qpg_tiles_us(int type, int T, int n_slots, int nkb) {
+    const int wgs = ((T + 63) / 64) * ((n_slots + 15) / 16);
+    return (float)nkb * (type == MI355_GGML_Q4_K ? qpw_rounds(wgs, 2 * mi355_num_cus(), 5.f, 3.4f) : qpw_rounds(wgs, mi355_num_cus(), 4.3f, 3.95f));
+}
+// Few tokens: those tiles with K in ks ranges, whose sums the epilogue's launch adds up.  A workgroup walks its k-blocks at the pace of its own round trips
+// (2.3 us each, alone on its CU or not), so a product of 48 workgroups and 32 k-blocks took 95 us with most of the chip idle.  us of both launches, fitted to
+// 1 000 launches of 33 .. 1400 tokens (error 8 %): per round and k-block, 3 per round, 4 for the second launch beyond what a fused epilogue costs, and the sums'
+// traffic.  What it picks is 1 % behind the fastest number of ranges.  us, one range / the picked ranges: 8192 -> 2048 at 96 tokens Q4_K 95 / 26, Q6_K 134 / 30;
+// 14336 -> 4096 at 130 tokens 157 / 56, 227 / 77; q | k | v of 2048 (v in Q6_K) at 320 tokens 72 / 41.  Beyond 1024 tokens the tiles fill the chip.
+static float qpg_split_us(int T, int slots4, int slots6, int nkb, int ks) {
+    const int cus = mi355_num_cus(), blocks = (T + 63) / 64, kbs = (nkb + ks - 1) / ks;
+    const int w4 = blocks * ((slots4 + 15) / 16) * ks, w6 = blocks * ((slots6 + 15) / 16) * ks;
+    float us = 4.f + (float)T * (float)((slots4 + slots6) * 16) * 1e-6f * (2.6f + 1.25f * (float)ks);
+    if (w4) us += (float)kbs * qpw_rounds(w4, 2 * cus, 3.9f, 2.25f) + 3.f * (float)((w4 + 2 * cus - 1) / (2 * cus));
+    if (w6) us += (float)kbs * qpw_rounds(w6, cus, 3.8f, 3.8f) + 3.f * (float)((w6 + cus - 1) / cus);
+    return us;
+}
 static QpwChoice qpw_pick(int type, int T, int n_slots, int K, float old_extra_us) {
     const int cus = mi355_num_cus(), nkb = K >> 8;
     auto est = [&](int bm, int bn, int cap, float full, float light) {
-        const int wgs = ((T + bm - 1) / bm) * ((n_slots * 16 + bn - 1) / bn), left = wgs % cap;
-        // two workgroups per CU: up to half a round they have a CU each
-        const float last = !left ? 0.f : cap > cus ? (left <= cus ? light : full) : light + (full - light) * (float)left / (float)cap;
-        return (float)nkb * (full * (float)(wgs / cap) + last);
+        return (float)nkb * qpw_rounds(((T + bm - 1) / bm) * ((n_slots * 16 + bn - 1) / bn), cap, full, light);
     };
     QpwChoice best{-1, 0.f};
     auto take = [&](int tile, float us) {
@@ -2012,12 +2035,12 @@ static QpwChoice qpw_pick(int type, int T, int n_slots, int K, float old_extra_u
         if (best.us == 0.f || us < best.us) best = {tile, us};
     };
     if (type == MI355_GGML_Q4_K) {
-        take(-1, old_extra_us + est(64, 256, 2 * cus, 5.f, 3.4f));
+        take(-1, old_extra_us + qpg_tiles_us(type, T, n_slots, nkb));
         take(0, est(256, 256, cus, 7.4f, 6.2f));
         take(1, est(256, 128, cus, 4.6f, 3.9f));
         take(2, est(192, 256, cus, 6.2f, 5.2f));
     } else {
-        take(-1, old_extra_us + est(64, 256, cus, 4.3f, 3.95f));
+        take(-1, old_extra_us + qpg_tiles_us(type, T, n_slots, nkb));
         take(1, est(256, 128, cus, 4.8f, 4.1f));
     }
     return best;
@@ -2056,15 +2079,32 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
     const float c_pass = 3.f + (float)T * (float)ldp * 8e-6f / 4.f;      // us of a launch that reads the f32 sums back: kernels without the epilogue need it
     int pick4 = -1, pick6 = -1;
     g_qpw_last = -1;
-    if (big && !a.blk_tab && ((all_q4 && epi_ok) || qkv)) pick4 = qpw_pick(MI355_GGML_Q4_K, T, slots4, K, qkv && T < 1024 ? c_pass : 0.f).tile;
-    if (big && !a.blk_tab && (v_slots || (one_q6 && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID))))
-        pick6 = qpw_pick(MI355_GGML_Q6_K, T, v_slots ? v_slots : n_slots, K, v_slots || T >= 4096 ? 0.f : c_pass).tile;
+    float whole_us = 0.f;
+    if (big && !a.blk_tab && ((all_q4 && epi_ok) || qkv)) {
+        const QpwChoice c = qpw_pick(MI355_GGML_Q4_K, T, slots4, K, qkv && T < 1024 ? c_pass : 0.f);
+        pick4 = c.tile; whole_us += c.us;
+    }
+    if (big && !a.blk_tab && (v_slots || (one_q6 && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID)))) {
+        const QpwChoice c = qpw_pick(MI355_GGML_Q6_K, T, v_slots ? v_slots : n_slots, K, v_slots || T >= 4096 ? 0.f : c_pass);
+        pick6 = c.tile; whole_us += c.us;
+    }
+    if (T < g_tune_qpg_min && !a.blk_tab && whole_us == 0.f) return (int)hipErrorNotSupported;
+    int ks = 1;
+    if (fuse && !a.blk_tab && whole_us > 0.f && T <= 1024) {
+        const int s6 = one_q6 ? n_slots : v_slots;
+        float best = 0.95f * whole_us;
+        for (int q = 2; q <= std::min(nkb, 16); ++q) {
+            const float us = qpg_split_us(T, n_slots - s6, s6, nkb, q);
+            if (us < best) { best = us; ks = q; }
+        }
+        if (ks > 1) pick4 = pick6 = -1;
+    }
     // token rows of the image: whole tiles of whichever kernel reads it
-    const int blk64 = (T + QPG_BM - 1) / QPG_BM * (QPG_BM / 64);   // token blocks of the 64-token kernels
+    const int blk64 = parts == 1 ? (T + 63) / 64 : (T + QPG_BM - 1) / QPG_BM * (QPG_BM / 64);   // token blocks of the 64-token kernels
     int Tpad = pick4 == 2 ? std::max((T + 191) / 192 * 192, (T + 255) / 256 * 256)
                : pick4 >= 0 || pick6 >= 0 ? (T + 255) / 256 * 256 : blk64 * 64;
     // (a block-table launch only exists with the epilogue in the store loop: no C buffer -- it would be 1.9 GB for a Mixtral chunk)
-    const size_t c_b = a.blk_tab ? 0 : (size_t)T * ldp * 4;
+    size_t c_b = a.blk_tab ? 0 : (size_t)T * ldp * 4 * ks;
     size_t xa_b = 0, sf_b = 0, rs_b = 0;
     void* ws = nullptr;
     Mi355ScratchTurn turn(MI355_SCR_QMP_WS, st);            // from the image's launch to its readers'
@@ -2078,7 +2118,10 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
         Tpad = blk64 * 64;
         rc = room();
     }
+    if (rc && T < g_tune_qpg_min) return (int)hipErrorNotSupported;   // the 32-token launches, which need less
+    if (rc && ks > 1) { c_b /= ks; ks = 1; rc = room(); }   // ... and for one set of sums
     if (rc) return rc;
+    g_qpg_split_last = ks;
     a.dbg = g_tune_dbg;                                     // ablation bits of the prompt-step GEMM (experiments only)
     uint8_t* base = static_cast<uint8_t*>(ws);
     QpgImg im;
@@ -2115,7 +2158,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
     // all segments Q4_K, one activation plane, and an epilogue that is a store / residual add / SiLU * up over two equal segments: the GEMM
     // writes the outputs itself, no C buffer, no epilogue launch (mi355_set_tuning(48, 0) switches that off)
     {
-        if (g_tune_qpg_fepi && all_q4 && epi_ok && parts == 1 && (g_tune_qpg == 0 || g_tune_qpg == 2)) {
+        if (g_tune_qpg_fepi && all_q4 && epi_ok && parts == 1 && ks == 1 && (g_tune_qpg == 0 || g_tune_qpg == 2)) {
             QmmArgs r = a;
             r.norm_w = nullptr;                                 // applied while the image was built
             if (pick4 >= 0) return qpw_launch<MI355_GGML_Q4_K>(pick4, r, im, n_slots, st);
@@ -2158,7 +2201,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
 #define QPG_FUSE_QKV 1          // A/B builds: 0 = q | k | v through the C buffer and the epilogue launch (rounds 2-5)
 #endif
     // (from 1024 tokens: measured +0.7 % at 2048 and +1.2 % at 4096 tokens, -1.9 % at 512 -- profiles/r06_prompt_qkv_fused_ab.txt)
-    if (QPG_FUSE_QKV && (T >= 1024 || pick4 >= 0) && fuse && qkv && (QPG_FUSE_Q6K || !v_slots)) {
+    if (QPG_FUSE_QKV && (T >= 1024 || pick4 >= 0) && fuse && ks == 1 && qkv && (QPG_FUSE_Q6K || !v_slots)) {
         const bool v4 = a.seg[2].type == MI355_GGML_Q4_K;
         QmmArgs r = a;
         r.norm_w = nullptr;                                         // applied while the image was built
@@ -2204,7 +2247,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
 #endif
                 default:                                                //  64 x 256, waves 64 x 32, two workgroups per CU; one activation plane: image and weights through LDS by DMA
                     if (parts == 1) {
-                        const dim3 g4(blk64, (run_slots + 15) / 16), b_(512);
+                        const dim3 g4(blk64, (run_slots + 15) / 16, ks), b_(512);
                         hipLaunchKernelGGL((qpg_gemm_lds2_kernel<false>), g4, b_, (size_t)QPG2_BYTES, st, r, im, C, ldp, run_slots, slot_base);
                     } else {
                         QPG_GO(4, 2, 1, 8, false);                      // hi + lo planes ("exact" activations): the register-fed form
@@ -2214,14 +2257,14 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
 #undef QPG_GO
         } else {
             if (parts == 1 && g_tune_qpg == 2) {                        // Q6_K: 64 tokens x 256 rows per workgroup; token blocks fastest
-                const dim3 grid(blk64, (run_slots + 15) / 16);
+                const dim3 grid(blk64, (run_slots + 15) / 16, ks);
                 if (pick6 >= 0 && one_q6) {
                     r.norm_w = nullptr;
                     return qpw_launch<MI355_GGML_Q6_K>(pick6, r, im, run_slots, st);
                 }
                 // the whole mat-mul is this one Q6_K run and its epilogue is a store / residual add: fused store loop, no C buffer, no launch
                 // (from 4096 tokens -- measured: +1.2 % at 4096, -0.2 % at 2048: profiles/r06_prompt_q6k_fused_ab.txt)
-                if (QPG_FUSE_Q6K && g_tune_qpg_fepi && T >= 4096 && s0 == 0 && s1 == a.nseg && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID)) {
+                if (QPG_FUSE_Q6K && g_tune_qpg_fepi && T >= 4096 && ks == 1 && s0 == 0 && s1 == a.nseg && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID)) {
                     r.norm_w = nullptr;
                     hipLaunchKernelGGL((qpg_gemm_q6k_lds_kernel<true>), grid, dim3(512), (size_t)QPG6_LDS_BYTES, st, r, im, C, ldp, run_slots, 0);
                     return (int)hipGetLastError();
@@ -2240,7 +2283,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
         s0 = s1;
     }
     a.norm_w = nullptr;                                     // applied while the image was built
-    hipLaunchKernelGGL(qmm_epilogue_kernel, dim3((ldp + 255) / 256, T), dim3(256), 0, st, a, C, ldp, 1, T, (const float*)nullptr,
+    hipLaunchKernelGGL(qmm_epilogue_kernel, dim3((ldp + 255) / 256, T), dim3(256), 0, st, a, C, ldp, ks, T, (const float*)nullptr,
                        QmgChainOut{nullptr, nullptr, nullptr, 0, 0, 0, 0}, (const float*)im.row_scale);
     return (int)hipGetLastError();
 }
@@ -2634,7 +2677,12 @@ int mi355_qmm_launch(QmmArgs a, int64_t stream) {
         return qmm_launch_bt<1>(a, R, wt, n_wg, NW, st);
     }
     if (a.blk_tab && !(a.B >= g_tune_qpg_min && g_tune_prefill_gemm == 1)) return (int)hipErrorNotSupported;   // only the prompt GEMM reads a block table
-    if (a.B >= g_tune_qpg_min && g_tune_prefill_gemm) {
+    // From 33 tokens, where its kernels of one activation plane run, the prompt GEMM with K in ranges is sooner than the 32-token launches one behind the other
+    // (2048 wide, 66 tokens, us a product: q | k | v 34 -> 21, gate/up 46 -> 29, down 40 -> 26), except just above 32 tokens with a Q6_K matrix (33 tokens: 20 and 26)
+    bool q6 = false;
+    for (int s = 0; s < a.nseg; ++s) q6 = q6 || a.seg[s].type == MI355_GGML_Q6_K;
+    const bool few = a.B > (q6 ? 36 : 32) && !g_tune_exact_act && g_tune_qpg == 2 && g_tune_qpg_fepi && !a.rows_dev && g_tune_prefill_gemm == 1;
+    if ((a.B >= g_tune_qpg_min && g_tune_prefill_gemm) || few) {
         // prompt step: the hand-written quantised GEMMs (qmm_prompt_gemm.inc, qmm_prefill.inc).  mi355_set_tuning(6, 2) = the first-generation path
         // (bf16 hi/lo weight image + three library GEMMs) for A/B runs; (6, 0) = stream the weights 32 tokens at a time.
 #ifdef MI355_QMM_PROBES

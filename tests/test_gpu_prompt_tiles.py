@@ -185,3 +185,99 @@ def test_qkv(layout, D, rot, v_kind, H, Hkv, T, K):
     untouched[slot[ok]] = False
     flat = kc.view(nb * block, -1) if layout == "flash" else kc.permute(0, 3, 1, 2, 4).reshape(nb * block, -1)
     assert (flat[untouched].float() == 0).all()
+
+
+def last_split():
+    f = cv.lib.mi355_internal_last_qpg_split
+    f.restype = ctypes.c_int32
+    return f()
+
+
+# K in ranges: a token in a block of its own, blocks that end inside, rows that fill neither tile nor workgroup, k-blocks that the ranges do not divide
+@pytest.mark.parametrize("kind,T,N,K", [(Q4, 33, 2048, 2048), (Q4, 64, 530, 8192), (Q4, 65, 4096, 4096), (Q4, 129, 3072, 8192), (Q4, 300, 1024, 2816), (Q4, 500, 2048, 8192),
+                                        (Q6, 37, 2048, 8192), (Q6, 64, 4100, 2048), (Q6, 95, 424, 1024), (Q6, 130, 4096, 14336), (Q6, 700, 512, 3328)])
+def test_ranges_of_k(kind, T, N, K):
+    rng = np.random.default_rng(T + N)
+    b = blocks(rng, N, K, kind)
+    m = cv.QMatMul(b, kind, "cuda")
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    x[T // 2] *= 3000.0                                               # tokens that the image scales down and up
+    x[T // 3] *= 1e-7
+    want, bias = product(x, b, kind), torch.randn(N, device="cuda")
+    for got, ref in ((m.forward(x), want), (m.forward(x, bias), want + bias)):
+        assert last_split() > 1
+        for t in (T // 2, T // 3):
+            assert close(got[t], ref[t]) < TOL
+        rest = [t for t in range(T) if t not in (T // 2, T // 3)]
+        assert close(got[rest], ref[rest]) < TOL
+    o = torch.randn(T, N + 3, device="cuda")
+    keep = o.clone()
+    d = cv.QmmDesc()
+    d.nseg, d.w_tiles[0], d.ggml_type[0], d.n_rows[0] = 1, m.tiles.data_ptr(), kind, N
+    d.x, d.x_dtype, d.ldx, d.k, d.num_tokens = x.data_ptr(), cv.DT_F32, K, K, T
+    d.epilogue, d.out, d.ldo, d.residual = cv.EPI_RESID, o.data_ptr(), N + 3, o.data_ptr()
+    assert cv.lib.mi355_qmatmul_fused(d, torch.cuda.current_stream().cuda_stream) == 0
+    assert close(o[rest, :N], (want + keep[:, :N].double())[rest]) < TOL and torch.equal(o[:, N:], keep[:, N:])
+
+
+@pytest.mark.parametrize("T,N,K", [(33, 2048, 2048), (66, 8192, 3072), (90, 500, 4096)])
+def test_gate_up_ranges_of_k(T, N, K):
+    rng = np.random.default_rng(T + N)
+    bg, bu = blocks(rng, N, K, Q4, odd=False), blocks(rng, N, K, Q4, odd=False)
+    g, u = cv.QMatMul(bg, Q4, "cuda"), cv.QMatMul(bu, Q4, "cuda")
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    nw = 1 + 0.1 * torch.randn(K, device="cuda")
+    xn = (x.double() * torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + 1e-5) * nw.double()).float()
+    want = torch.nn.functional.silu(product(xn, bg, Q4)) * product(xn, bu, Q4)
+    out = torch.empty(T, N, device="cuda")
+    cv.qmatmul_fused([g, u], x, epilogue=cv.EPI_SILU_MUL, out=out, norm_weight=nw, norm_eps=1e-5)
+    assert last_split() > 1
+    assert close(out, want) < 2 * TOL                                 # two rounded factors
+
+
+@pytest.mark.parametrize("v_kind,T", [(Q4, 40), (Q6, 40), (Q4, 161), (Q6, 320)])
+def test_qkv_ranges_of_k(v_kind, T):
+    H, Hkv, D, K, block = 16, 4, 128, 2048, 16
+    rng = np.random.default_rng(T)
+    kinds, heads = (Q4, Q4, v_kind), (H, Hkv, Hkv)
+    bs = [blocks(rng, n * D, K, t) for n, t in zip(heads, kinds)]
+    ms = [cv.QMatMul(b, t, "cuda") for b, t in zip(bs, kinds)]
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    pos, slot = torch.from_numpy(rng.integers(0, 500, T)).cuda(), torch.from_numpy(rng.permutation(T + 64)[:T].astype(np.int64)).cuda()
+    slot[5] = -1
+    ang = torch.arange(500, device="cuda").double()[:, None] * 10000.0 ** (-torch.arange(D // 2, device="cuda").double() / (D // 2))
+    nb = (T + 64 + block - 1) // block
+    kc, vc = torch.zeros(nb, Hkv, D // 8, block, 8, dtype=torch.bfloat16, device="cuda"), torch.zeros(nb, Hkv, D, block, dtype=torch.bfloat16, device="cuda")
+    q_out = torch.zeros(T, H * D, dtype=torch.bfloat16, device="cuda")
+    cv.qmatmul_fused(ms, x, epilogue=cv.EPI_QKV_ROPE_CACHE, rope=dict(cos=ang.cos().float().contiguous(), sin=ang.sin().float().contiguous(), positions=pos, slot_mapping=slot,
+                                                                     q_out=q_out, key_cache=kc, value_cache=vc, num_heads=H, num_kv_heads=Hkv, head_dim=D, rotary_dim=D))
+    assert last_split() > 1
+    y = [product(x, b, t).view(T, -1, D) for b, t in zip(bs, kinds)]
+    c, s = ang.cos()[pos][:, None], ang.sin()[pos][:, None]
+    turned = [torch.stack([z[..., 0::2] * c - z[..., 1::2] * s, z[..., 0::2] * s + z[..., 1::2] * c], dim=-1).reshape(T, -1, D) for z in y[:2]]
+    ok = slot >= 0
+    blk, off = slot[ok] // block, slot[ok] % block
+    for got, want in ((q_out.view(T, H, D), turned[0]), (kc[blk, :, :, off].reshape(-1, Hkv, D), turned[1][ok]), (vc[blk, :, :, off], y[2][ok])):
+        assert close(got.float(), want) < TOL + 2.0 ** -8                 # bf16's rounding
+
+
+def test_ranges_of_k_without_room():
+    """no room for the sums of several ranges: one range from 96 tokens on, the 32-token launches below"""
+    rng = np.random.default_rng(3)
+    K, N = 4096, 2048
+    b = blocks(rng, N, K, Q4)
+    m = cv.QMatMul(b, Q4, "cuda")
+    cv.lib.mi355_internal_scratch_limit.argtypes = [ctypes.c_int64]
+    for T, splits in ((200, 1), (80, None)):
+        x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+        want = product(x, b, Q4)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(torch.cuda.Stream()):
+            cv.lib.mi355_internal_scratch_limit(4200000)                  # 200 tokens: image 2.2 MB, sums of a range 1.6 MB
+            try:
+                got = m.forward(x)
+                assert splits is None or last_split() == splits
+            finally:
+                cv.lib.mi355_internal_scratch_limit(-1)
+            assert close(got, want) < TOL
+            assert close(m.forward(x), want) < TOL and last_split() > 1
