@@ -149,7 +149,8 @@ extern "C" int mi355_internal_moe_scatter_combine_to_image(float* ys, const floa
 extern "C" int mi355_internal_pa_stream_reduce_to_image(void* out, const float* tmp_out, const float* max_logits, const float* exp_sums,
                                                         const uint32_t* context_lens, int32_t B, int32_t H, int32_t W, int32_t slots,
                                                         int64_t stream);                                                     // qmatmul.hip
-extern "C" int mi355_pa_stream_auto(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size);   // paged_attention.hip
+extern "C" int32_t mi355_internal_pa_plan(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_context_len,
+                                          int32_t kv8, int32_t slots, int32_t* partition_size);   // paged_attention.hip
 int g_host_ps_override = 0;     // experiments: mi355_set_tuning(5, partition_size)
 // MI355_MOE_PROMPT_DEVICE=0: prompt steps of a mixture-of-experts model sort their (token, slot) pairs on the host again (rounds 2-5; A/B runs)
 static const int g_moe_prompt_device = []() { const char* e = getenv("MI355_MOE_PROMPT_DEVICE"); return e && e[0] == '0' ? 0 : 1; }();
@@ -502,24 +503,24 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
         int ps = choose_partition(B, Hkv, in.ctx_cap);
         if (ps > 0) ps = 32;   // MFMA kernel: 32-token partitions, 4 per workgroup (measured at batch 32: 32 -> 4937, 64 -> 4784, 128 -> ~4500 tok/s)
         // >= 64 (sequence, kv head) pairs: the balanced LDS-DMA stream over the e4m3fn cache (round 5), as on the bf16 cache
-        if (ps > 0 && mi355_pa_stream_auto(B, H, Hkv, D, c.block_size)) ps = 64;
+        const int cap = ps > 0 ? mi355_internal_pa_plan(B, H, Hkv, D, c.block_size, in.ctx_cap, 1, m->pa_cap_partitions, &ps) : in.ctx_cap;
         if (g_host_ps_override > 0 && ps > 0) ps = g_host_ps_override;
-        if (ps > 0 && (in.ctx_cap + ps - 1) / ps > m->pa_cap_partitions) return (int)hipErrorInvalidValue;
+        if (ps > 0 && (cap + ps - 1) / ps > m->pa_cap_partitions) return (int)hipErrorInvalidValue;
         if (in.ctx_cap > c.max_seq) return (int)hipErrorInvalidValue;
         if (ps == 64 && B >= 9 && B <= 32 && !(H & 1) && !m->use_comm) {
             // as on the bf16 cache below: the merge of the stream's partials also stages wo's activation image
             int32_t w = 0;
             RCHECK(mi355_internal_paged_attention_fp8_partials(in.attn, m->pa_sum, m->pa_max, m->pa_tmp, in.q, m->kcache[l], m->vcache[l], in.bt,
-                                                               in.ctx, B, H, Hkv, D, c.block_size, in.max_blocks, in.ctx_cap, ps, scale, 0.f, 1.f, 1.f,
+                                                               in.ctx, B, H, Hkv, D, c.block_size, in.max_blocks, cap, ps, scale, 0.f, 1.f, 1.f,
                                                                st, &w));
             if (w == 0) return 0;                                     // the launch did not take the stream: it is complete
-            const int max_partitions = (in.ctx_cap + ps - 1) / ps < 1 ? 1 : (in.ctx_cap + ps - 1) / ps;
+            const int max_partitions = (cap + ps - 1) / ps < 1 ? 1 : (cap + ps - 1) / ps;
             const int rc = mi355_internal_pa_stream_reduce_to_image(in.attn, m->pa_tmp, m->pa_max, m->pa_sum, in.ctx, B, H, w, max_partitions, st);
             if (rc != -4) return rc;
             return mi355_internal_pa_stream_reduce(in.attn, m->pa_tmp, m->pa_max, m->pa_sum, in.ctx, B, H, w, max_partitions, st);
         }
         return mi355_paged_attention_fp8(in.attn, m->pa_sum, m->pa_max, m->pa_tmp, in.q, m->kcache[l], m->vcache[l], in.bt, in.ctx,
-                                         B, H, Hkv, D, c.block_size, in.max_blocks, in.ctx_cap, ps, scale, 0.f, 1.f, 1.f, st);
+                                         B, H, Hkv, D, c.block_size, in.max_blocks, cap, ps, scale, 0.f, 1.f, 1.f, st);
     }
     if (part == PART_ATTN && in.is_prefill) {
         // --- K4: every key (cached prefix + this chunk, just written by the QKV epilogue) comes from the cache
@@ -538,10 +539,11 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
         int ps = choose_partition(B, Hkv, in.ctx_cap);
         if (ps > 0 && c.kv_layout == MI355_KV_PAGED) ps = 32;   // MFMA kernel: 32-token partitions, 4 per workgroup (measured at batch 32: 32 -> 4937, 64 -> 4784, 128 -> ~4500 tok/s)
         // >= 64 (sequence, kv head) pairs: 64-token stages through the balanced LDS-DMA stream (round 4: 5987 -> 6177 tok/s at batch 32)
-        if (ps > 0 && c.kv_layout == MI355_KV_PAGED && mi355_pa_stream_auto(B, H, Hkv, D, c.block_size)) ps = 64;
+        const int cap = ps > 0 && c.kv_layout == MI355_KV_PAGED
+            ? mi355_internal_pa_plan(B, H, Hkv, D, c.block_size, in.ctx_cap, 0, m->pa_cap_partitions, &ps) : in.ctx_cap;
         if (g_host_ps_override > 0 && ps > 0) ps = g_host_ps_override;
         const float scale = 1.0f / sqrtf((float)D);
-        if (ps > 0 && (in.ctx_cap + ps - 1) / ps > m->pa_cap_partitions) return (int)hipErrorInvalidValue;
+        if (ps > 0 && (cap + ps - 1) / ps > m->pa_cap_partitions) return (int)hipErrorInvalidValue;
         if (in.ctx_cap > c.max_seq) return (int)hipErrorInvalidValue;
         if (ps == 0)
             return mi355_paged_attention_v1(in.attn, in.q, m->kcache[l], m->vcache[l], in.bt, in.ctx, B, H, Hkv, D,
@@ -552,16 +554,16 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
             // image (qmatmul.hip mi355_internal_pa_stream_reduce_to_image): one launch instead of merge + staging
             int32_t w = 0;
             RCHECK(mi355_internal_paged_attention_v2_partials(in.attn, m->pa_sum, m->pa_max, m->pa_tmp, in.q, m->kcache[l], m->vcache[l], in.bt,
-                                                              in.ctx, B, H, Hkv, D, c.block_size, in.max_blocks, in.ctx_cap, ps, scale, 0.f,
+                                                              in.ctx, B, H, Hkv, D, c.block_size, in.max_blocks, cap, ps, scale, 0.f,
                                                               c.kv_layout, MI355_DTYPE_BF16, st, &w));
             if (w == 0) return 0;                                     // the launch did not take the stream: it is complete
-            const int max_partitions = (in.ctx_cap + ps - 1) / ps < 1 ? 1 : (in.ctx_cap + ps - 1) / ps;
+            const int max_partitions = (cap + ps - 1) / ps < 1 ? 1 : (cap + ps - 1) / ps;
             const int rc = mi355_internal_pa_stream_reduce_to_image(in.attn, m->pa_tmp, m->pa_max, m->pa_sum, in.ctx, B, H, w, max_partitions, st);
             if (rc != -4) return rc;
             return mi355_internal_pa_stream_reduce(in.attn, m->pa_tmp, m->pa_max, m->pa_sum, in.ctx, B, H, w, max_partitions, st);
         }
         return mi355_paged_attention_v2(in.attn, m->pa_sum, m->pa_max, m->pa_tmp, in.q, m->kcache[l], m->vcache[l],
-                                        in.bt, in.ctx, B, H, Hkv, D, c.block_size, in.max_blocks, in.ctx_cap, ps,
+                                        in.bt, in.ctx, B, H, Hkv, D, c.block_size, in.max_blocks, cap, ps,
                                         scale, 0.f, c.kv_layout, MI355_DTYPE_BF16, st);
     }
     if (part == PART_WO || part == PART_DOWN) {

@@ -435,7 +435,8 @@ __global__ void __launch_bounds__(256) paged_attn_paged_layout_kernel(const PAPa
 //   * all K and V loads of the partition are issued before the first MFMA.
 // one partition [t0, t1) of (sequence b, kv head hk) on one wave: unnormalised O (lane: channel 16nt + (lane&15), heads
 // 4(lane>>4)+v), the partition's row maxima m and bf16-rounded probability sums lsum (valid in lane == head)
-template <int D32, int NT, bool KV8>
+// P32: the probabilities keep 16 bits of mantissa and more -- each as a bf16 and the bf16 of what that leaves, two instructions for P.V -- and their sum is f32's
+template <int D32, int NT, bool KV8, bool P32 = false>
 __device__ __forceinline__ void pa_mfma_partition(const PAParams& p, const int b, const int hk, const int t0, const int t1,
                                                   const int lane, f32x4_t (&o)[2 * D32], float& m, float& lsum, const int blk_s = -1) {
     constexpr int D = 32 * D32, NTD = D / 16;
@@ -544,7 +545,7 @@ __device__ __forceinline__ void pa_mfma_partition(const PAParams& p, const int b
     m = fmaxf(m, __shfl_xor(m, 16, 64));
     m = fmaxf(m, __shfl_xor(m, 32, 64));
     lsum = 0.f;
-    uint2 pf[NT];
+    uint2 pf[NT], pl[P32 ? NT : 1];
 #pragma unroll
     for (int it = 0; it < NT; ++it) {
         const int tokb = t0 + 32 * (it >> 1) + 8 * kg + 4 * (it & 1);
@@ -552,6 +553,11 @@ __device__ __forceinline__ void pa_mfma_partition(const PAParams& p, const int b
 #pragma unroll
         for (int v = 0; v < 4; ++v) pr[v] = (tokb + v < t1) ? __expf(sc[it][v] - m) : 0.f;
         pf[it] = make_uint2(cvt_pk_bf16(pr[0], pr[1]), cvt_pk_bf16(pr[2], pr[3]));
+        if constexpr (P32) {
+            pl[it] = make_uint2(cvt_pk_bf16(pr[0] - bf16lo_to_f32(pf[it].x), pr[1] - bf16hi_to_f32(pf[it].x)),
+                                cvt_pk_bf16(pr[2] - bf16lo_to_f32(pf[it].y), pr[3] - bf16hi_to_f32(pf[it].y)));
+            lsum += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+        } else
         // the normaliser must match what the MFMA sums: the bf16-rounded probabilities
         lsum += (bf16lo_to_f32(pf[it].x) + bf16hi_to_f32(pf[it].x)) + (bf16lo_to_f32(pf[it].y) + bf16hi_to_f32(pf[it].y));
     }
@@ -592,6 +598,9 @@ __device__ __forceinline__ void pa_mfma_partition(const PAParams& p, const int b
             }
             o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, pa),
                                                             __builtin_bit_cast(bf16x8_t, vv), o[nt], 0, 0, 0);
+            if constexpr (P32)
+                o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, make_uint4(pl[2 * ip].x, pl[2 * ip].y, pl[2 * ip + 1].x, pl[2 * ip + 1].y)),
+                                                                __builtin_bit_cast(bf16x8_t, vv), o[nt], 0, 0, 0);
         }
     }
 }
@@ -816,7 +825,8 @@ extern "C" int mi355_debug_set_pa_timestamps(void* dev_ptr) { return (int)hipMem
 #define PA_TL_FLUSH() ((void)0)
 #endif
 
-template <int D32, int NT, bool KV8 = false, int WPB = 1>
+// ONE: the workgroup's WPB partitions are all of the sequence -- it writes the outputs itself, with probabilities as P32 keeps them
+template <int D32, int NT, bool KV8 = false, int WPB = 1, bool ONE = false>
 __global__ void __launch_bounds__(64 * WPB) paged_attn_mfma_kernel(const PAParams p) {
     PA_TL_DECL;
     PA_TL(0);
@@ -827,7 +837,8 @@ __global__ void __launch_bounds__(64 * WPB) paged_attn_mfma_kernel(const PAParam
     const int part = blockIdx.z * WPB + wave;
     // a context longer than the launch was sized for is truncated to the grid (the host layer refuses such a step): the
     // partition count below must match the launched grid or the fused merge's ticket never completes
-    const int t0 = part * p.partition_size;
+    const int psize = ONE ? 32 : p.partition_size;                  // (ONE: p.partition_size holds the most tokens of a context)
+    const int t0 = part * psize;
     // looped chunks: the table entries of this wave's chunk go out before the context length is known -- lane l asks for entry
     // t0 / bs + l (clamped to the row: entries beyond the context hold no block id and are never used).  A relaxed atomic load: a
     // plain one is sunk below the context-length branch by the compiler, back into the dependent chain.
@@ -842,18 +853,23 @@ __global__ void __launch_bounds__(64 * WPB) paged_attn_mfma_kernel(const PAParam
     // constant address space, in flight together with the context length (the table was written by an earlier launch / copy)
     int blk_s = -1;
     if constexpr (PA_SCALAR_TABLE && NT == 2) {
-        if ((p.block_size & 31) == 0 && p.partition_size == 32) {
+        if ((p.block_size & 31) == 0 && psize == 32) {
             typedef const uint32_t __attribute__((address_space(4))) * cbt_t;
             const int q0 = min(t0 / p.block_size, p.max_blocks - 1);
             blk_s = (int)*reinterpret_cast<cbt_t>(reinterpret_cast<uintptr_t>(p.block_tables + (int64_t)b * p.max_blocks + q0));
         }
     }
-    const int ctx = min((int)p.context_lens[b], p.max_partitions * p.partition_size);
-    if (blockIdx.z * WPB * p.partition_size >= ctx) return;        // uniform for the workgroup
+    const int ctx = min((int)p.context_lens[b], ONE ? p.partition_size : p.max_partitions * p.partition_size);
+    const int G = p.H / p.Hkv;
+    if constexpr (ONE) {
+        if (ctx <= 0) {                                             // nothing cached: zeros
+            for (int i = threadIdx.x; i < G * D; i += 64 * WPB) static_cast<uint16_t*>(p.out)[((int64_t)b * p.H + hk * G) * D + i] = 0;
+            return;
+        }
+    } else if (blockIdx.z * WPB * p.partition_size >= ctx) return;  // uniform for the workgroup
     PA_TL(1);
     const bool live = t0 < ctx;
-    const int t1 = min(ctx, t0 + p.partition_size);
-    const int G = p.H / p.Hkv;
+    const int t1 = min(ctx, t0 + psize);
     const int c = lane & 15, kg = lane >> 4;
     extern __shared__ __attribute__((aligned(16))) float pa_smem[];   // WPB > 1 only
     f32x4_t o[NTD];
@@ -862,7 +878,7 @@ __global__ void __launch_bounds__(64 * WPB) paged_attn_mfma_kernel(const PAParam
     for (int nt = 0; nt < NTD; ++nt) o[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     if (live) {
         if constexpr (NT == 0) pa_mfma_chunk<D32, KV8>(p, b, hk, t0, t1, lane, btv, o, m, lsum);  // partition = a chunk of 32-token pairs, looped
-        else pa_mfma_partition<D32, NT, KV8>(p, b, hk, t0, t1, lane, o, m, lsum, blk_s);
+        else pa_mfma_partition<D32, NT, KV8, ONE>(p, b, hk, t0, t1, lane, o, m, lsum, blk_s);
     }
 #ifdef MI355_PA_TIMELINE
     asm volatile("" ::"v"(o[0][0]), "v"(lsum));
@@ -901,7 +917,7 @@ __global__ void __launch_bounds__(64 * WPB) paged_attn_mfma_kernel(const PAParam
             }
             const float outv = (den > 0.f ? val / den : 0.f) * vs;
             const int h = hk * G + g;
-            if (p.max_partitions > 1) {
+            if (!ONE && p.max_partitions > 1) {
                 const int64_t pi = ((int64_t)b * p.H + h) * p.max_partitions + pslot;
                 if (p.arrive) {
                     __hip_atomic_store(p.tmp_out + pi * D + d, outv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -917,7 +933,7 @@ __global__ void __launch_bounds__(64 * WPB) paged_attn_mfma_kernel(const PAParam
                 static_cast<uint16_t*>(p.out)[((int64_t)b * p.H + h) * D + d] = f32_to_bf16(outv);
             }
         }
-        if (p.max_partitions <= 1 || p.arrive == nullptr) return;
+        if (ONE || p.max_partitions <= 1 || p.arrive == nullptr) return;
         PA_TL(4);
         // fused merge, workgroup form: every wave drains its write-through stores, one thread takes the ticket, the
         // last workgroup merges with one WAVE per query head (64 lanes x D/64 channels)
@@ -1790,6 +1806,27 @@ static int launch_mfma(const PAParams& p, int B, int P, int wpb, hipStream_t st)
     return wpb == 4 ? launch_mfma_w<D32, 4>(p, B, P, st) : launch_mfma_w<D32, 1>(p, B, P, st);
 }
 
+// Short contexts (a caller's bound of up to 512 tokens): one workgroup per (sequence, kv head), a wave to 32 tokens, outputs from its own merge.  What bounds it
+// is one chain of round trips (length, table, K and V, merge in LDS); a second launch for the merge, or a thread to a token, only made it longer.
+// us, before / now, 24 heads over 8: three sequences of up to 146 tokens 39.5 / 4.7 (a thread per token, one token after the other for V), 250 tokens 11.6 / 5.0 (one wave),
+// 500 tokens 9.2 / 8.1 (partitions and a reduce launch); 32 sequences of up to 300 tokens 42.8 / 8.4 (the stream).  Error against 64 bits 1.7e-3, the bf16 outputs'
+// own (a thread per token 1.7e-3, the others 2.0e-3).
+static int pa_one_waves(int H, int Hkv, int D, int tokens) {          // 0: not served
+    const int n = (tokens + 31) / 32, waves = n <= 4 ? 4 : n <= 8 ? 8 : 16;
+    return n <= 16 && (size_t)waves * (H / Hkv) * (D + 2) * sizeof(float) <= 64 * 1024 ? waves : 0;
+}
+static bool pa_one_shape_ok(int H, int Hkv, int D, int block_size) {
+    return (D == 128 || D == 64) && Hkv > 0 && H % Hkv == 0 && H / Hkv <= 16 && block_size % 16 == 0;
+}
+template <int D32, bool KV8>
+static void launch_mfma_one(const PAParams& p, int B, int waves, hipStream_t st) {
+    const size_t per_wave = (size_t)(p.H / p.Hkv) * (32 * D32 + 2) * sizeof(float);
+    const dim3 grid(p.Hkv, B), block(64 * waves);
+    if (waves == 4) hipLaunchKernelGGL((paged_attn_mfma_kernel<D32, 2, KV8, 4, true>), grid, block, 4 * per_wave, st, p);
+    else if (waves == 8) hipLaunchKernelGGL((paged_attn_mfma_kernel<D32, 2, KV8, 8, true>), grid, block, 8 * per_wave, st, p);
+    else hipLaunchKernelGGL((paged_attn_mfma_kernel<D32, 2, KV8, 16, true>), grid, block, 16 * per_wave, st, p);
+}
+
 // ------------------------------------------------------------------------------------------------ launchers
 template <int LPT, int KVT, bool PART>
 static int launch_flash_g(const PAParams& p, int B, int P, hipStream_t st) {
@@ -1835,6 +1872,27 @@ extern "C" int mi355_pa_stream_auto(int32_t num_seqs, int32_t num_heads, int32_t
     return (g_pa_loop == 3 || (int64_t)num_seqs * num_kv_heads >= PA_STREAM_MIN_PAIRS) ? 1 : 0;
 }
 
+// workgroups per kv head of the stream: one per CU (bf16), two (e4m3 and up to 8 query heads per kv head)
+static int pa_stream_most(int H, int Hkv, bool kv8) {
+    const int W = (kv8 ? (H / Hkv > 8 ? 256 : 512) : PAS_RING <= 2 ? 512 : 256) / Hkv;
+    return W < 1 ? 1 : W > 64 ? 64 : W;
+}
+// What the step drivers pass for a PAGED bf16 launch of contexts up to max_context_len: *partition_size (in: theirs, > 0) and, returned, the context length that sizes
+// the launch.  Short contexts: 32, one workgroup each.  The stream: 64, and a context long enough that every compute unit gets a share -- its workgroups per kv head
+// are as many as the caller has partial slots for, and 16 sequences of 2500 tokens (4 kv heads) left 96 of 256 without one: 24.4 -> 21.8 us; 17 sequences of 584
+// tokens 25.0 -> 15.5 (28 heads), 24.4 -> 15.7 (24 over 8, e4m3).  slots: partials per (sequence, head) that the driver's buffers hold
+extern "C" int32_t mi355_internal_pa_plan(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_context_len,
+                                          int32_t kv8, int32_t slots, int32_t* partition_size) {
+    if (pa_one_shape_ok(num_heads, num_kv_heads, head_dim, block_size) && pa_one_waves(num_heads, num_kv_heads, head_dim, max_context_len)) {
+        *partition_size = 32;
+        return max_context_len;
+    }
+    if (!mi355_pa_stream_auto(num_seqs, num_heads, num_kv_heads, head_dim, block_size)) return max_context_len;
+    *partition_size = 64;
+    const int W = pa_stream_most(num_heads, num_kv_heads, kv8 != 0);
+    return W <= slots && max_context_len < 64 * W ? 64 * W : max_context_len;
+}
+
 static int pa_dispatch(PAParams p, int B, int P, int layout, int dtype, int64_t stream) {
     if (B <= 0) return 0;
     if (p.H % p.Hkv || (p.D & 7) || p.D > 256) return (int)hipErrorInvalidValue;
@@ -1842,6 +1900,14 @@ static int pa_dispatch(PAParams p, int B, int P, int layout, int dtype, int64_t 
     hipStream_t st = to_stream(stream);
     int rc, wpb = 1;
     if (p.kv8 && (layout != MI355_KV_PAGED || dtype != MI355_DTYPE_BF16 || (p.D % 16))) return (int)hipErrorInvalidValue;
+    const int one = layout == MI355_KV_PAGED && dtype == MI355_DTYPE_BF16 && pa_one_shape_ok(p.H, p.Hkv, p.D, p.block_size) && g_pa_wpb == 0 &&
+                            (P == 1 || p.partition_size == 32) ? pa_one_waves(p.H, p.Hkv, p.D, P * p.partition_size) : 0;
+    if (one) {
+        p.partition_size *= P;                                       // the most tokens of a context
+        if (p.D == 128) p.kv8 ? launch_mfma_one<4, true>(p, B, one, st) : launch_mfma_one<4, false>(p, B, one, st);
+        else p.kv8 ? launch_mfma_one<2, true>(p, B, one, st) : launch_mfma_one<2, false>(p, B, one, st);
+        return (int)hipGetLastError();
+    }
     if (layout == MI355_KV_FLASH) {
         if (P > 1)
             rc = (dtype == MI355_DTYPE_BF16) ? launch_flash<MI355_DTYPE_BF16, true>(p, B, P, st)
@@ -1865,10 +1931,7 @@ static int pa_dispatch(PAParams p, int B, int P, int layout, int dtype, int64_t 
             (void)hipFuncSetAttribute((const void*)paged_attn_stream_kernel<PAS_R8, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, PAS_R8 * 16384 + 16384 + 32768);
             attr_done.set();
         }
-        int W = (G > 8 ? 256 : 512) / p.Hkv;
-        if (W < 1) W = 1;
-        if (W > 64) W = 64;
-        if (W > P) W = P;
+        const int W = std::min(pa_stream_most(p.H, p.Hkv, true), P);
         hipLaunchKernelGGL((paged_attn_stream_kernel<PAS_R8, true, true>), dim3(W, p.Hkv), dim3(256), shm8, st, p, B, p.block_tables, p.context_lens);
         if (g_pa_stream_noreduce) { g_pa_stream_last_w = W; return (int)hipGetLastError(); }   // the caller merges
         hipLaunchKernelGGL(paged_attn_stream_reduce_kernel, dim3(p.H, B), dim3(128), 0, st, p.out, p.tmp_out, p.max_logits, p.exp_sums,
@@ -1887,10 +1950,7 @@ static int pa_dispatch(PAParams p, int B, int P, int layout, int dtype, int64_t 
             (void)hipFuncSetAttribute((const void*)paged_attn_stream_kernel<PAS_R, PAS_TS != 0>, hipFuncAttributeMaxDynamicSharedMemorySize, PAS_R * 32768 + 16384);
             attr_done.set();
         }
-        int W = (PAS_RING <= 2 ? 512 : 256) / p.Hkv;                  // two workgroups per CU fit with a ring of two stages only
-        if (W < 1) W = 1;
-        if (W > 64) W = 64;
-        if (W > P) W = P;
+        const int W = std::min(pa_stream_most(p.H, p.Hkv, false), P);
         hipLaunchKernelGGL((paged_attn_stream_kernel<PAS_R, PAS_TS != 0>), dim3(W, p.Hkv), dim3(256), PAS_R * 32768 + 16384, st, p, B, p.block_tables,
                            p.context_lens);
         if (g_pa_stream_noreduce) { g_pa_stream_last_w = W; return (int)hipGetLastError(); }   // the caller merges (mi355_internal_pa_stream_partials)
