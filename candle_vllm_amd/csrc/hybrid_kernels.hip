@@ -7,6 +7,7 @@
 // ctx[s] - that many cached ones; a portion that starts at position 0 starts from zero state whatever its slot holds.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
 #include <type_traits>
 #include <math.h>
 
@@ -61,6 +62,7 @@ struct LinArgs {
     // gate/up pairs: the rows of w come as 16 gate rows, their 16 up rows, the next 16 gate rows, ...; out [T, N / 2] = act(gate) up
     int glu;
     float glu_limit, glu_alpha;   // of LIN_ACT_CLAMPED
+    int ldw;                // elements between two rows of w (K, and more where the launch's z are ranges of a longer row)
 };
 constexpr int LIN_ACT_CLAMPED = MI355_HYB_ACT_RELU2 + 1;   // g' sigmoid(alpha g') (u' + 1), g' = min(g, limit), u' = u within +- limit
 // (behind the gate/up product: 156 -> 168 us at 2100 tokens x 16384 x 2048, and the activation's own launch, 43 us there and 4.7 at 8 tokens, is gone)
@@ -127,7 +129,7 @@ template <typename TA, int MT, int B> __global__ __launch_bounds__(256) void lin
     const int t0 = blockIdx.y * (16 * MT);
     int64_t w_off;
     if (!lin_group(p, t0, w_off)) return;
-    const uint16_t* wrow = static_cast<const uint16_t*>(p.w) + w_off + (size_t)(n < p.N ? n : 0) * p.K;
+    const uint16_t* wrow = static_cast<const uint16_t*>(p.w) + w_off + (size_t)(n < p.N ? n : 0) * p.ldw;
     const TA* arow[MT];
     bool aok[MT];
 #pragma unroll
@@ -146,7 +148,7 @@ template <typename TA, int MT, int B> __global__ __launch_bounds__(256) void lin
         const int k = k0 + 8 * kg;
         uint4 b[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) b[c] = nok ? frag8<uint16_t>(wrow + (size_t)(16 * c) * p.K, k, p.K, p.w_vec) : uint4{0, 0, 0, 0};
+        for (int c = 0; c < NC; ++c) b[c] = nok ? frag8<uint16_t>(wrow + (size_t)(16 * c) * p.ldw, k, p.K, p.w_vec) : uint4{0, 0, 0, 0};
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             const uint4 a = aok[i] ? frag8<TA>(arow[i], k, p.K, p.a_vec) : uint4{0, 0, 0, 0};
@@ -190,7 +192,7 @@ template <int B> __global__ __launch_bounds__(256) void linear_bf16_lds_kernel(L
         const int t = t0 + r0 + 64 * j, n = n0 + r0 + 64 * j;
         aok[j] = t < p.T; wok[j] = n < p.N;
         asrc[j] = A + (size_t)(aok[j] ? lin_row(p, t) : 0) * p.lda + ch * 8;
-        wsrc[j] = W + (size_t)(wok[j] ? n : 0) * p.K + ch * 8;
+        wsrc[j] = W + (size_t)(wok[j] ? n : 0) * p.ldw + ch * 8;
     }
     uint4 ra[2], rw[2];
     auto fetch = [&](int k0) {
@@ -288,8 +290,8 @@ template <int B, int WM, int WN, int MF, int NF, int S, bool GATHER> __global__ 
 #pragma unroll
     for (int r = 0; r < Tile::BR; ++r) {
         const int first = min(n0 + 8 * (tile.wave + 8 * r), p.N - 1), row = min(n0 + tile.stage_row(r), p.N - 1);
-        b_base[r] = wb + (size_t)first * p.K * 2;
-        b_off[r] = (uint32_t)(row - first) * (uint32_t)p.K * 2u + tile.stage_chunk();
+        b_base[r] = wb + (size_t)first * p.ldw * 2;
+        b_off[r] = (uint32_t)(row - first) * (uint32_t)p.ldw * 2u + tile.stage_chunk();
     }
     tile.run(a_base, a_off, b_base, b_off, 128u, p.K / 64);
     const bool wide = !(p.ldo & 3) && !((uintptr_t)p.out & 15);          // (N is a multiple of 16)
@@ -349,7 +351,7 @@ template <int B> static void linear_gemm_launch(const LinArgs& p, int which, int
 }
 // operands the GEMM's 16-byte pieces and its 32-bit offsets inside a tile reach
 static bool linear_gemm_ok(const LinArgs& p, bool a_f32) {
-    return !a_f32 && p.a_vec && p.w_vec && p.K % 64 == 0 && p.N % 16 == 0 && (int64_t)p.lda * 512 < (1ll << 32) && (int64_t)p.K * 512 < (1ll << 32);
+    return !a_f32 && p.a_vec && p.w_vec && p.K % 64 == 0 && p.N % 16 == 0 && (int64_t)p.lda * 512 < (1ll << 32) && (int64_t)p.ldw * 512 < (1ll << 32);
 }
 
 // Up to 16 tokens, bf16 weights: the product is a stream over the weights.  A workgroup owns 16 weight rows; its NW waves take the
@@ -364,7 +366,7 @@ template <typename TA, int NW, int UNR, int B> __global__ __launch_bounds__(64 *
     int64_t w_off;
     if (!lin_group(p, t0, w_off)) return;
     const bool nok = n < p.N, aok = t0 + m16 < p.T;
-    const uint16_t* wrow = static_cast<const uint16_t*>(p.w) + w_off + (size_t)(nok ? n : 0) * p.K;
+    const uint16_t* wrow = static_cast<const uint16_t*>(p.w) + w_off + (size_t)(nok ? n : 0) * p.ldw;
     const TA* arow = static_cast<const TA*>(p.a) + (size_t)(aok ? lin_row(p, t0 + m16) : 0) * p.lda;
     f32x4_t acc[NC];
 #pragma unroll
@@ -375,7 +377,7 @@ template <typename TA, int NW, int UNR, int B> __global__ __launch_bounds__(64 *
         for (int u = 0; u < UNR; ++u) {
             const int k = k0 + u * 32 + 8 * kg;
 #pragma unroll
-            for (int c = 0; c < NC; ++c) b[c][u] = (nok && k < p.K) ? frag8<uint16_t>(wrow + (size_t)(16 * c) * p.K, k, p.K, p.w_vec) : uint4{0, 0, 0, 0};
+            for (int c = 0; c < NC; ++c) b[c][u] = (nok && k < p.K) ? frag8<uint16_t>(wrow + (size_t)(16 * c) * p.ldw, k, p.K, p.w_vec) : uint4{0, 0, 0, 0};
             a[u] = (aok && k < p.K) ? frag8<TA>(arow, k, p.K, p.a_vec) : uint4{0, 0, 0, 0};
         }
 #pragma unroll
@@ -450,7 +452,7 @@ template <int NW, int UNR, int MT, int B> __global__ __launch_bounds__(64 * NW) 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m16 = lane & 15, kg = lane >> 4;
     const int n = blockIdx.x * 16 * NC + m16, t0 = blockIdx.y * 16 * MT;
     const bool nok = n < p.N;
-    const float* wrow = static_cast<const float*>(p.w) + (int64_t)blockIdx.z * p.w_bs + (size_t)(nok ? n : 0) * p.K;
+    const float* wrow = static_cast<const float*>(p.w) + (int64_t)blockIdx.z * p.w_bs + (size_t)(nok ? n : 0) * p.ldw;
     const float* arow[MT];
     bool aok[MT];
 #pragma unroll
@@ -469,7 +471,7 @@ template <int NW, int UNR, int MT, int B> __global__ __launch_bounds__(64 * NW) 
         for (int u = 0; u < UNR; ++u) {
             const int k = k0 + 16 * u + 4 * kg;
 #pragma unroll
-            for (int c = 0; c < NC; ++c) b[c][u] = (nok && k < p.K) ? frag4(wrow + (size_t)(16 * c) * p.K, k, p.K, p.w_vec) : float4{0.f, 0.f, 0.f, 0.f};
+            for (int c = 0; c < NC; ++c) b[c][u] = (nok && k < p.K) ? frag4(wrow + (size_t)(16 * c) * p.ldw, k, p.K, p.w_vec) : float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int m = 0; m < MT; ++m) a[m][u] = (aok[m] && k < p.K) ? frag4(arow[m], k, p.K, p.a_vec) : float4{0.f, 0.f, 0.f, 0.f};
         }
@@ -533,7 +535,7 @@ template <int MF, int NF, int KS, int PF, int B> __global__ __launch_bounds__(25
             src[i] = static_cast<const float*>(p.a) + (size_t)(ok[i] ? lin_row(p, t0 + r) : 0) * p.lda;
         } else {
             ok[i] = n0 + r - BM < p.N;
-            src[i] = static_cast<const float*>(p.w) + w_off + (size_t)(ok[i] ? n0 + r - BM : 0) * p.K;
+            src[i] = static_cast<const float*>(p.w) + w_off + (size_t)(ok[i] ? n0 + r - BM : 0) * p.ldw;
         }
     }
     float4 reg[PF][NL];
@@ -674,9 +676,12 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* x, uint16_t* xcopy
     }
 }
 
+constexpr int PARTS_MOST = 8;
 // The same, four elements at a time, V of them per thread (width <= 1024 V): y, x and w are requested together, so that a launch is one round trip
 // to memory and the sum.  (y, then x and w behind the sum, y a second time, took 7.3 us for 8 tokens of width 2048 and 20.3 for 2100; now 4.6 and 11.5).
-template <int V> __global__ __launch_bounds__(256) void norm_add4_kernel(float* x, uint16_t* xcopy, const float* y, int ldy, const float* w, int width, float eps) {
+// SUM: y is the sum of `parts` sets of rows, `part` elements apart (a product's ranges of K)
+template <int V, bool SUM> __global__ __launch_bounds__(256) void norm_add4_kernel(float* x, uint16_t* xcopy, const float* y, int ldy, const float* w, int width, float eps,
+                                                                                   int64_t part, int parts) {
     __shared__ float red[4];
     const int t = blockIdx.x;
     f32x4_t yv[V], xv[V], wv[V];
@@ -689,6 +694,13 @@ template <int V> __global__ __launch_bounds__(256) void norm_add4_kernel(float* 
         yv[j] = *reinterpret_cast<const f32x4_t*>(y + (size_t)t * ldy + i);
         xv[j] = *reinterpret_cast<const f32x4_t*>(x + (size_t)t * width + i);
         wv[j] = *reinterpret_cast<const f32x4_t*>(w + i);
+        if (SUM) {
+            f32x4_t more[PARTS_MOST - 1];                                // all requested before the first is added
+#pragma unroll
+            for (int p = 1; p < PARTS_MOST; ++p) more[p - 1] = p < parts ? *reinterpret_cast<const f32x4_t*>(y + p * part + (size_t)t * ldy + i) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int p = 1; p < PARTS_MOST; ++p) yv[j] += more[p - 1];
+        }
     }
 #pragma unroll
     for (int j = 0; j < V; ++j)
@@ -2188,11 +2200,11 @@ struct LinSegments { int32_t n, first; int64_t a_stride; const int32_t* rows; };
 static int linear_launch(float* out, int32_t ldo, int64_t o_bs, const void* a, int32_t a_dtype, int32_t lda, int64_t a_bs, const void* w,
                          int64_t w_bs, const float* bias, int32_t T, int32_t n, int32_t k, int32_t batch, int32_t dtype, int64_t stream,
                          int32_t act = 0, int32_t act_cols = 0, int32_t out16 = 0, const LinSegments* seg = nullptr, int32_t glu = 0,
-                         float glu_limit = 0.f, float glu_alpha = 0.f) {
+                         float glu_limit = 0.f, float glu_alpha = 0.f, int32_t ldw = 0) {
     if (!out || !a || !w || T < 0 || n <= 0 || k <= 0 || ldo < (glu ? n / 2 : n) || lda < k || batch <= 0 || batch > 65535 || !is_dt(dtype) || !is_dt(a_dtype)) return -1;
     if (T == 0) return 0;
     LinArgs p{out, ldo, a, lda, w, bias, T, n, k, 0, 0, a_bs, w_bs, o_bs};
-    p.act = act; p.act_cols = act_cols; p.out16 = out16; p.glu = glu; p.glu_limit = glu_limit; p.glu_alpha = glu_alpha;
+    p.act = act; p.act_cols = act_cols; p.out16 = out16; p.glu = glu; p.glu_limit = glu_limit; p.glu_alpha = glu_alpha; p.ldw = ldw ? ldw : k;
     if (glu && (n % 32 || a_dtype != dtype || bias)) return -1;
     if (seg) {
         if (seg->n < 1 || seg->n > LIN_MAX_SEG || seg->first < 0 || seg->a_stride < 0 || !seg->rows || batch != 1 || act || out16) return -1;
@@ -2206,13 +2218,13 @@ static int linear_launch(float* out, int32_t ldo, int64_t o_bs, const void* a, i
     const unsigned nz = (unsigned)batch;
     if (dtype == MI355_DTYPE_F32) {
         if (a_dtype != MI355_DTYPE_F32) return -1;
-        p.w_vec = (k % 4 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 4 == 0);
+        p.w_vec = (p.ldw % 4 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 4 == 0);
         p.a_vec = (lda % 4 == 0) && ((uintptr_t)a % 16 == 0) && (a_bs % 4 == 0);
         LIN_EPI(p, (linear_f32_launch<EPI>(p, nz, st_)));
         LAUNCH_OK(); return 0;
     }
     const int a_bytes = a_dtype == MI355_DTYPE_F32 ? 4 : 2;
-    p.w_vec = (k % 8 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 8 == 0);
+    p.w_vec = (p.ldw % 8 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 8 == 0);
     p.a_vec = ((size_t)lda * a_bytes % 16 == 0) && ((uintptr_t)a % 16 == 0) && ((size_t)a_bs * a_bytes % 16 == 0);
     const bool af = a_dtype == MI355_DTYPE_F32;
     if (T <= 16) {
@@ -2242,6 +2254,39 @@ int mi355_hyb_linear(float* out, int32_t ldo, const void* a, int32_t a_dtype, in
                      int32_t T, int32_t n, int32_t k, int32_t dtype, int64_t stream) {
     return linear_launch(out, ldo, 0, a, a_dtype, lda, 0, w, 0, bias, T, n, k, 1, dtype, stream);
 }
+// How many ranges of K a product [T, k] x [n, k] whose sums mi355_internal_hyb_norm_add_parts takes is made in, of at most `most`: few row tiles, each walking all of
+// K, leave the chip idle.  us of product and norm, one range / the picked ones (bf16 unless said): 8 tokens 2048 x 8192 19.5 / 16.3, x 4096 12.2 / 10.3; 48 tokens
+// x 8192 55 / 17, 164 53 / 21, 400 49 / 28, x 2048 15.3 / 10.8 at 48; 3072 x 8192 at 256 54 / 32; f32 8 tokens 2048 x 8192 34 / 25, 100 tokens 106 / 52.  To 16 tokens: up to a
+// row tile per unit, 1024 columns a range; beyond: the rounds of the tiles (gt_pick) and what the sums cost the norm.  Over 150 sizes 1 % behind the best number.
+int32_t mi355_internal_hyb_parts(int32_t T, int32_t n, int32_t k, int32_t dtype, int32_t most) {
+    const int cus = mi355_num_cus(), top = std::min(most, PARTS_MOST);
+    auto fits = [&](int s) { return s <= top && k % (64 * s) == 0; };
+    if (T < 1 || (n & 15)) return 1;
+    if (dtype == MI355_DTYPE_F32 || T <= 16) {
+        const int64_t tiles = T <= 32 ? n / 16 : (int64_t)((n + 63) / 64) * ((T + 63) / 64);
+        if (dtype == MI355_DTYPE_F32 && T <= 32 && tiles >= cus) return 1;
+        for (int s = 8; s > 1; s >>= 1) {
+            const bool full = dtype == MI355_DTYPE_F32 ? T > 32 ? tiles * s > 4 * cus : s == 8 && tiles * s > 2 * cus : s == 8 || tiles * s > cus || k / s < 1024;
+            if (!full && fits(s)) return s;
+        }
+        return 1;
+    }
+    int best = 1;
+    float best_us = 0.f;
+    for (int s : {1, 2, 3, 4, 8}) {
+        if (!fits(s)) continue;
+        const GtChoice c = gt_pick([&](const GtTile& t) { return (int64_t)((T + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * s; }, k / s / 64, (float)n * (float)k * 2.f / 5.4e6f, 1, 0.f, 63);
+        const float us = c.us + (s > 1 ? 1.f + 2.4e-6f * (float)T * (float)n * (float)(s - 1) : 0.f);
+        if (s == 1 || us < best_us) { best = s; best_us = us; }
+    }
+    return best;
+}
+// mi355_hyb_linear with K in `parts` ranges: out holds that many sets of sums, `part` elements apart, for mi355_internal_hyb_norm_add_parts
+int mi355_internal_hyb_linear_parts(float* out, int64_t part, int32_t parts, const void* a, int32_t a_dtype, int32_t lda, const void* w, int32_t T, int32_t n,
+                                    int32_t k, int32_t dtype, int64_t stream) {
+    if (parts < 1 || parts > PARTS_MOST || k % (64 * parts) || lda < k || (part & 3)) return -1;
+    return linear_launch(out, n, part, a, a_dtype, lda, k / parts, w, k / parts, nullptr, T, n, k / parts, parts, dtype, stream, 0, 0, 0, nullptr, 0, 0.f, 0.f, k);
+}
 int mi355_hyb_linear_act(void* out, int32_t out_dtype, int32_t ldo, const void* a, int32_t a_dtype, int32_t lda, const void* w, const float* bias,
                          int32_t T, int32_t n, int32_t k, int32_t act, int32_t act_cols, int32_t dtype, int64_t stream) {
     if (act < 0 || act > MI355_HYB_ACT_RELU2 || act_cols < 0 || !is_dt(out_dtype)) return -1;
@@ -2269,15 +2314,29 @@ int mi355_hyb_embed(float* x, void* xcopy, const void* table, const uint32_t* id
     LAUNCH_OK(); return 0;
 }
 
+int mi355_internal_hyb_norm_add_parts(float* x, void* xcopy, const float* y, int32_t ldy, int64_t part, int32_t parts, const float* w, int32_t T, int32_t width,
+                                      float eps, int64_t stream);
+static bool norm_add_by_4(const float* x, const void* xcopy, const float* y, int32_t ldy, const float* w, int32_t width) {
+    return width <= 4096 && ((width | ldy) & 3) == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w) & 15) == 0 && ((uintptr_t)xcopy & 7) == 0;
+}
 int mi355_hyb_norm_add(float* x, void* xcopy, const float* y, int32_t ldy, const float* w, int32_t T, int32_t width, float eps,
                        int64_t stream) {
-    if (!x || !y || !w || width <= 0 || ldy < width) return -1;
+    return mi355_internal_hyb_norm_add_parts(x, xcopy, y, ldy, 0, 1, w, T, width, eps, stream);
+}
+// mi355_hyb_norm_add of the sum of `parts` (1 .. 8) sets of rows, `part` elements apart
+int mi355_internal_hyb_norm_add_parts(float* x, void* xcopy, const float* y, int32_t ldy, int64_t part, int32_t parts, const float* w, int32_t T, int32_t width,
+                                      float eps, int64_t stream) {
+    if (!x || !y || !w || width <= 0 || ldy < width || parts < 1 || parts > PARTS_MOST || (parts > 1 && (part & 3))) return -1;
+    const bool by_4 = norm_add_by_4(x, xcopy, y, ldy, w, width);
+    if (parts > 1 && !by_4) return -1;
     if (T <= 0) return 0;
-    if (width <= 4096 && ((width | ldy) & 3) == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w) & 15) == 0 && ((uintptr_t)xcopy & 7) == 0) {
+    if (by_4) {
         const int v = (width + 1023) / 1024;
-#define NORM_ADD_GO(V) norm_add4_kernel<V><<<T, 256, 0, to_stream(stream)>>>(x, (uint16_t*)xcopy, y, ldy, w, width, eps)
+#define NORM_ADD_GO_(V, SUM) norm_add4_kernel<V, SUM><<<T, 256, 0, to_stream(stream)>>>(x, (uint16_t*)xcopy, y, ldy, w, width, eps, part, parts)
+#define NORM_ADD_GO(V) do { if (parts > 1) NORM_ADD_GO_(V, true); else NORM_ADD_GO_(V, false); } while (0)
         if (v == 1) NORM_ADD_GO(1); else if (v == 2) NORM_ADD_GO(2); else if (v == 3) NORM_ADD_GO(3); else NORM_ADD_GO(4);
 #undef NORM_ADD_GO
+#undef NORM_ADD_GO_
     } else norm_add_kernel<<<T, 256, 0, to_stream(stream)>>>(x, (uint16_t*)xcopy, y, ldy, w, width, eps);
     LAUNCH_OK(); return 0;
 }
@@ -2783,17 +2842,17 @@ static int grouped_launch(void* out, int32_t out_dtype, int32_t ldo, const void*
     if (n_blocks <= 0) return 0;
     if (n_blocks > 65535) return -1;
     LinArgs p{static_cast<float*>(out), ldo, a, lda, w, nullptr, n_blocks * block_rows, n, k, 0, 0, 0, w_bs, 0, block_table, row_token, block_rows};
-    p.act = act; p.act_cols = n; p.glu = glu; p.out16 = out_dtype == MI355_DTYPE_BF16;
+    p.act = act; p.act_cols = n; p.glu = glu; p.out16 = out_dtype == MI355_DTYPE_BF16; p.ldw = k;
     hipStream_t st_ = to_stream(stream);
     if (dtype == MI355_DTYPE_F32) {
         if (a_dtype != MI355_DTYPE_F32 || block_rows != 64) return -1;
-        p.w_vec = (k % 4 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 4 == 0);
+        p.w_vec = (p.ldw % 4 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 4 == 0);
         p.a_vec = (lda % 4 == 0) && ((uintptr_t)a % 16 == 0);
         LIN_EPI2(p, (linear_f32_gemm_kernel<1, 1, 2, 2, EPI><<<dim3((n + 63) / 64, n_blocks, 1), 512, 0, st_>>>(p)));
         LAUNCH_OK(); return 0;
     }
     const int a_bytes = a_dtype == MI355_DTYPE_F32 ? 4 : 2;
-    p.w_vec = (k % 8 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 8 == 0);
+    p.w_vec = (p.ldw % 8 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 8 == 0);
     p.a_vec = ((size_t)lda * a_bytes % 16 == 0) && ((uintptr_t)a % 16 == 0);
     const bool af = a_dtype == MI355_DTYPE_F32;
     if (block_rows == 16) {

@@ -32,6 +32,11 @@
 
 extern "C" {
 int mi355_hyb_token_seq(int32_t*, const uint32_t*, int32_t, int64_t);
+int32_t mi355_internal_hyb_parts(int32_t T, int32_t n, int32_t k, int32_t dtype, int32_t most);
+int mi355_internal_hyb_linear_parts(float* out, int64_t part, int32_t parts, const void* a, int32_t a_dtype, int32_t lda, const void* w, int32_t T, int32_t n,
+                                    int32_t k, int32_t dtype, int64_t stream);
+int mi355_internal_hyb_norm_add_parts(float* x, void* xcopy, const float* y, int32_t ldy, int64_t part, int32_t parts, const float* w, int32_t T, int32_t width,
+                                      float eps, int64_t stream);
 int32_t mi355_internal_hyb_clamped_fused(int32_t T, int32_t ff, int32_t k, int32_t dtype);
 int mi355_hyb_bf16_to_f32(float*, const uint16_t*, int64_t, int64_t);
 int mi355_hyb_fill_f32(float*, float, int64_t, int64_t);
@@ -99,6 +104,7 @@ struct HModel {
     int num_blocks = 0;
     // activations (grow-only)
     int cap_t = 0, cap_out = 0;
+    size_t y_rows = 0;               // rows that `y` holds
     float *prep = nullptr, *x = nullptr, *proj = nullptr, *aux1 = nullptr, *aux2 = nullptr, *conv = nullptr, *o = nullptr, *y = nullptr, *gu = nullptr;
     void *xcopy = nullptr, *q = nullptr, *mix = nullptr, *act = nullptr, *xn = nullptr, *att = nullptr;
     int32_t* tok_seq = nullptr;
@@ -414,7 +420,9 @@ int ensure_capacity(HModel* m, int T, int n_out, int n_seqs) {
         HCHECK(grow(m->conv, t * (size_t)m->max_conv * 4));
         HCHECK(grow(m->o, t * (size_t)m->max_o * 4));
         HCHECK(grow(m->prep, t * (size_t)m->max_prep * 4));
-        HCHECK(grow(m->y, t * W * 4));
+        // (room for a product's sums in several ranges of K: up to 8, and 4096 rows in all; one set of rows where the card has no more)
+        m->y_rows = std::max<size_t>(t, std::min<size_t>(8 * t, 4096));
+        if (grow(m->y, m->y_rows * W * 4)) { (void)hipGetLastError(); m->y_rows = t; HCHECK(grow(m->y, t * W * 4)); }
         HCHECK(grow(m->gu, t * (size_t)m->max_ff * 2 * 4));
         HCHECK(grow(m->xcopy, t * W * 2));
         HCHECK(grow(m->q, t * (size_t)m->max_q * m->esize()));
@@ -1003,12 +1011,20 @@ static int forward_enqueue(HModel* m, const uint32_t* tokens, const int64_t* pos
         if (c.mixer == MI355_HYB_MIX_MINGRU)
             HCHECK(mi355_hyb_mingru(m->mix, dt, m->state + L.state_off, m->slot_floats, m->proj, ldp, L.off[0], L.off[1], L.off[2],
                                     context_lens, cu_seqlens_q, state_slots, num_seqs, T, c.g_width, stream));
+        // the products in front of a residual(): K in as many ranges as their few tiles want, the sums added by the norm's launch
+        int parts = 1;
+        const bool by_parts = !pair && !copies && !parallel && m->cfg.residual_form != 1 && W <= 4096 && W % 16 == 0;
+        auto residual_product = [&](const void* a, int k, const void* w) -> int {
+            parts = by_parts ? mi355_internal_hyb_parts(T, W, k, dt, (int)std::min<size_t>(m->y_rows / (size_t)T, 8)) : 1;
+            if (parts == 1) return mi355_hyb_linear(m->y, W, a, dt, k, w, nullptr, T, W, k, dt, stream);
+            return mi355_internal_hyb_linear_parts(m->y, TW, parts, a, dt, k, w, T, W, k, dt, stream);
+        };
         auto residual = [&](int norm_slot) -> int {
             if (m->cfg.residual_form == 1)
                 return mi355_hyb_resid_norm(m->x, xcopy, m->y, W, f(norm_slot), T, W, m->cfg.norm_groups, m->cfg.resid_alpha, eps, stream);
-            return mi355_hyb_norm_add(m->x, xcopy, m->y, W, f(norm_slot), T, W, eps, stream);
+            return mi355_internal_hyb_norm_add_parts(m->x, xcopy, m->y, W, TW, parts, f(norm_slot), T, W, eps, stream);
         };
-        HCHECK(mi355_hyb_linear(m->y, W, m->mix, dt, L.out_k, WL.w[MI355_HW_OUT_PROJ].p, nullptr, T, W, L.out_k, dt, stream));
+        HCHECK(residual_product(m->mix, L.out_k, WL.w[MI355_HW_OUT_PROJ].p));
         if (pair) {
             if (c.mlp_kind == 3) HCHECK(run_experts(c, WL));
             else if (c.mlp_kind == 4 || c.mlp_kind == 5) {
@@ -1092,7 +1108,7 @@ static int forward_enqueue(HModel* m, const uint32_t* tokens, const int64_t* pos
         } else if (c.mlp_kind) {
             if (sandwich) HCHECK(mi355_hyb_pre_norm(m->pre, dt, m->x, f(MI355_HW_PRE_NORM2), T, W, eps, stream));
             HCHECK(dense_gate_up(WL));
-            HCHECK(mi355_hyb_linear(m->y, W, m->act, dt, c.mlp_ff, WL.w[MI355_HW_MLP_DOWN].p, nullptr, T, W, c.mlp_ff, dt, stream));
+            HCHECK(residual_product(m->act, c.mlp_ff, WL.w[MI355_HW_MLP_DOWN].p));
             HCHECK(residual(MI355_HW_NORM2));
         }
         }

@@ -3,6 +3,7 @@ its C entry point, then whole Sogodra models through the step engine -- whole pr
 down to two tokens, unequal batches against each request alone, pages and state slots that are freed and used again, keys at page
 borders and at the edges of the window, the first tokens, long decoding, odd sizes -- and greedy generation through run_engine and
 the scheduler.  Configurations and weights are made here."""
+import ctypes
 import math
 
 import numpy as np
@@ -125,6 +126,38 @@ def test_gate_and_up_forms(lib, dtype, T, ff, k):
     g, u, dg, du = z[:, :, 0], z[:, :, 1], e[:, :, 0], e[:, :, 1]
     want, bound = torch.nn.functional.silu(g) * u, 1.1 * u.abs() * dg + g.abs() * du + 1e-6 * (1 + (g * u).abs())
     assert ((out[:, :ff].double() - want.reshape(T, ff)).abs() <= bound.reshape(T, ff)).all() and (out[:, ff:] == 7.0).all()
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("T,n,k", [(1, 2048, 2048), (8, 1024, 4096), (16, 2048, 8192), (17, 48, 512), (40, 2048, 8192), (100, 3072, 3072), (333, 2048, 1536), (65, 4096, 6144)])
+def test_products_in_ranges_of_k_and_their_norm(lib, dtype, T, n, k):
+    """a residual product in every number of ranges that K divides into, the picked one among them, and the norm that adds them: as one range to (k + 2) 2^-24 sum |a w|,
+    and x + norm(y) w of the sum to 2^-20 of its values; sums of other calls are not read"""
+    _gpu()
+    i32, i64, vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p
+    lp, na, pick = lib.mi355_internal_hyb_linear_parts, lib.mi355_internal_hyb_norm_add_parts, lib.mi355_internal_hyb_parts
+    lp.argtypes, na.argtypes = [vp, i64, i32, vp, i32, i32, vp, i32, i32, i32, i32, i64], [vp, vp, vp, i32, i64, i32, vp, i32, i32, ctypes.c_float, i64]
+    torch.manual_seed(T + n + k)
+    td = torch.float32 if dtype == F32 else torch.bfloat16
+    a, w, g = torch.randn(T, k + 8, device="cuda").to(td), (torch.randn(n, k, device="cuda") * k ** -0.5).to(td), 1 + 0.1 * torch.randn(n, device="cuda")
+    want, bound = a[:, :k].double() @ w.double().t(), (k + 2) * 2.0 ** -24 * (a[:, :k].double().abs() @ w.double().abs().t())
+    x0 = torch.randn(T, n, device="cuda")
+    picked = pick(T, n, k, dtype, 8)
+    assert picked == 1 or k % (64 * picked) == 0
+    for parts in sorted({1, 2, 3, 4, 8, picked}):
+        if k % (64 * parts):
+            assert lp(x0.data_ptr(), T * n, parts, a.data_ptr(), dtype, k + 8, w.data_ptr(), T, n, k, dtype, _st()) != 0
+            continue
+        y = torch.full((9, T, n), float("nan"), device="cuda")
+        ok(lp(y.data_ptr(), T * n, parts, a.data_ptr(), dtype, k + 8, w.data_ptr(), T, n, k, dtype, _st()))
+        s = y[:parts].double().sum(0)
+        assert ((s - want).abs() <= bound).all() and y[parts:].isnan().all()
+        x, xc = x0.clone(), torch.zeros(T, n, dtype=torch.int16, device="cuda")
+        ok(na(x.data_ptr(), xc.data_ptr(), y.data_ptr(), n, T * n, parts, g.data_ptr(), T, n, 1e-5, _st()))
+        ref = x0.double() + s * torch.rsqrt((s * s).mean(1, keepdim=True) + 1e-5) * g.double()
+        assert ((x.double() - ref).abs() <= 2.0 ** -20 * (1 + ref.abs())).all()
+        assert torch.equal(xc, x.bfloat16().view(torch.int16))
+    assert na(x.data_ptr(), None, y.data_ptr(), n, T * n, 9, g.data_ptr(), T, n, 1e-5, _st()) != 0
 
 
 def test_norm_add_and_glu(lib):
