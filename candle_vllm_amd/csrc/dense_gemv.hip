@@ -76,7 +76,7 @@ struct DenseArgs {
     float* ss_out;            // dense_small_kernel only: where this launch leaves [T][ldo/16] partial sums of squares of its output
     struct DenseNormTail* tail;   // host only: the RmsNorm that reads this product's output, or null
 };
-// out [T][N] = RmsNorm(the product's output) * w, bf16; done: the launch made it (only split sums of few tokens do, resid_norm_tail)
+// out [T][N] = RmsNorm(the product's output) * w, bf16; done: the launch made it (only split sums do, resid_norm_tail)
 struct DenseNormTail { void* out; const void* w; float eps; bool done; };
 
 template <int DT> __device__ __forceinline__ float h2f(uint16_t h) {
@@ -1095,8 +1095,9 @@ static int dense_dispatch(const DenseArgs& a, int wtype, int dt, hipStream_t st)
 struct DenseGemm3 {
     DenseArgs a[3];
     int32_t tiles[3], n_m;               // column tiles of each matrix (0: none), token tiles
-    int32_t splits, units_per_split;     // K in `splits` ranges (one matrix only) whose partial sums go to `part` [splits][token][N]
+    int32_t splits, units_per_split;     // K in `splits` ranges whose partial sums go to `part` [splits][token][ldp], a matrix's from column col0 on
     float* part;
+    int32_t ldp, col0[3];
 };
 // candle's rounding of one value by the hardware's conversion (the same round-to-nearest-even; a NaN keeps its sign)
 template <int DT> __device__ __forceinline__ uint32_t gemm_pack(float lo, float hi) {
@@ -1227,7 +1228,7 @@ __global__ void __launch_bounds__(512, 2) dense_gemm_kernel(const DenseGemm3 g) 
     }
     tile.run(a_base, a_off, b_base, b_off, b_step, units);
     if (g.splits > 1) {                                                  // gptq_wide_epilogue_kernel adds the ranges in their order and rounds
-        float* part = g.part + (size_t)split * a.T * a.N;
+        float* part = g.part + (size_t)split * a.T * g.ldp + g.col0[which];
 #pragma unroll
         for (int i = 0; i < MF; ++i) {
             const int t = t0 + tile.row(i);
@@ -1238,7 +1239,7 @@ __global__ void __launch_bounds__(512, 2) dense_gemm_kernel(const DenseGemm3 g) 
                 if (silu) col = c0 + tile.wn * (NF * 8) + (j % (NF / 2)) * 16 + 4 * (tile.lane >> 4);
                 if (col >= n_cols) continue;
                 if (silu && j >= NF / 2) col += a.pair_offset;
-                *reinterpret_cast<f32x4_t*>(part + (size_t)t * a.N + col) = tile.acc[i][j];
+                *reinterpret_cast<f32x4_t*>(part + (size_t)t * g.ldp + col) = tile.acc[i][j];
             }
         }
         return;
@@ -1291,8 +1292,8 @@ static int gptq_gemm_dt(const GptqGemm& g, uint16_t* xp, float* xs, int which, h
 // The workspaces of the prompt GEMMs are kept, so they are bounded: partial sums of at most 128 MiB, and of a 4-bit prompt at most 128 MiB of permuted
 // x and its sums at a time (3 328 tokens of 18 944, 19 712 of 3 584; a launch of that many is at its rate, and the panel in front of each costs 1 % of it)
 constexpr int64_t GEMM_PART_BYTES = 128ll << 20, GPTQ_GEMM_X_BYTES = 128ll << 20;
-static int gemm_max_split(const DenseArgs& a, int most) {
-    return (int)std::min<int64_t>(std::min(16, most), std::max<int64_t>(1, GEMM_PART_BYTES / ((int64_t)a.T * a.N * 4)));
+static int gemm_max_split(const DenseArgs& a, int64_t rows, int most) {
+    return (int)std::min<int64_t>(std::min(16, most), std::max<int64_t>(1, GEMM_PART_BYTES / ((int64_t)a.T * rows * 4)));
 }
 static int gptq_gemm_slab(int k) { return (int)std::max<int64_t>(1, GPTQ_GEMM_X_BYTES / ((int64_t)k * 2 + k / 16) / 256) * 256; }
 // rows t0 .. of a launch of T tokens, at most n of them
@@ -1302,7 +1303,68 @@ static DenseArgs dense_rows(const DenseArgs& a, int t0, int n) {
     c.x = static_cast<const uint16_t*>(a.x) + (size_t)t0 * a.ldx;
     c.out = static_cast<uint16_t*>(a.out) + (size_t)t0 * a.ldo;
     if (a.resid) c.resid = static_cast<const uint16_t*>(a.resid) + (size_t)t0 * a.ldo;
+    if (c.T < a.T) c.tail = nullptr;                                   // (its buffer starts with the first row)
     return c;
+}
+// The sums of q | k | v in ranges of K, RoPE (halves) and the cache write: four pairs of q or k or four channels of v per thread, units of a token one behind the other.
+// The products' own rounding, then rope_kernel's and the cache's: what the launches that it stands for do.  Three small products with K in ranges and this launch
+// in place of the products over all of K, RoPE and the cache write, us: 4608 x 3584 in 4 bits, 50 tokens 17.1 for 37.8; 3072 x 2048 in 16 bits, 99 tokens 15.9 for 22.9.
+__global__ void __launch_bounds__(256) sum3_rope_cache_kernel(const DenseGemm3 g, const DenseRope rp, const int n_units) {
+    constexpr int DT = MI355_DTYPE_BF16;
+    const int u = blockIdx.x * 256 + threadIdx.x;
+    if (u >= n_units) return;
+    const int D = rp.head_dim, half = D >> 1, G = rp.n_kv_heads, H = g.a[0].N / D, qk = (H + G) * (half >> 2), per_tok = qk + G * (D >> 2);
+    const int t = u / per_tok, r = u - t * per_tok;
+    const int64_t slot = rp.slots[t];
+    const int64_t blk = slot >= 0 ? slot / rp.block_size : 0;
+    const int off = slot >= 0 ? (int)(slot % rp.block_size) : 0;
+    const size_t step = (size_t)g.a[0].T * g.ldp;
+    const int h = r < qk ? r / (half >> 2) : 0, m = r >= qk ? 2 : h < H ? 0 : 1;
+    const int col = r < qk ? (m ? h - H : h) * D + (r - h * (half >> 2)) * 4 : (r - qk) * 4;   // in matrix m
+    const int second = m < 2 ? half : 0;
+    const float* p = g.part + (size_t)t * g.ldp + g.col0[m] + col;
+    f32x4_t x = {0.f, 0.f, 0.f, 0.f}, y = x;
+#pragma unroll 8
+    for (int s = 0; s < g.splits; ++s, p += step) {
+        x += *reinterpret_cast<const f32x4_t*>(p);
+        y += *reinterpret_cast<const f32x4_t*>(p + second);
+    }
+    const uint16_t* bias = static_cast<const uint16_t*>(g.a[m].bias);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        x[i] = gemm_rnd<DT>(x[i]); y[i] = gemm_rnd<DT>(y[i]);
+        if (bias) { x[i] = gemm_rnd<DT>(x[i] + h2f<DT>(bias[col + i])); y[i] = gemm_rnd<DT>(y[i] + h2f<DT>(bias[col + second + i])); }
+    }
+    if (m == 2) {
+        if (slot < 0) return;
+        const int hh = col / D, d = col - hh * D;
+        if (rp.flash) *reinterpret_cast<uint2*>(rp.vcache + (slot * G + hh) * D + d) = make_uint2(pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]));
+        else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rp.vcache[((blk * G + hh) * D + d + i) * (int64_t)rp.block_size + off] = f32_to_bf16(x[i]);
+        }
+        return;
+    }
+    const int hh = col / D, j = col - hh * D;
+    const float4 c = *reinterpret_cast<const float4*>(rp.cos_t + rp.positions[t] * half + j), s = *reinterpret_cast<const float4*>(rp.sin_t + rp.positions[t] * half + j);
+    const float cc[4] = {c.x, c.y, c.z, c.w}, ss[4] = {s.x, s.y, s.z, s.w};
+    float o[4], o2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rope_rotate(x[i], y[i], cc[i], ss[i], o[i], o2[i]);
+    uint16_t *pa, *pb;
+    if (m == 0) { pa = static_cast<uint16_t*>(g.a[0].out) + (size_t)t * g.a[0].ldo + col; pb = pa + half; }
+    else if (slot < 0) return;
+    else if (rp.flash) { pa = rp.kcache + (slot * G + hh) * D + j; pb = pa + half; }
+    else { pa = rp.kcache + (((blk * G + hh) * (D / 8) + j / 8) * rp.block_size + off) * 8 + j % 8; pb = pa + (int64_t)(half / 8) * rp.block_size * 8; }
+    *reinterpret_cast<uint2*>(pa) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+    *reinterpret_cast<uint2*>(pb) = make_uint2(pack_bf16x2(o2[0], o2[1]), pack_bf16x2(o2[2], o2[3]));
+}
+// Whether the launch above takes the sums of these three, and its units
+static int64_t sum3_units(const DenseArgs* a, const DenseRope& rp, int dt) {
+    if (dt != MI355_DTYPE_BF16 || rp.head_dim % 16 || a[0].N % rp.head_dim || a[1].N != rp.n_kv_heads * rp.head_dim || a[2].N != a[1].N) return 0;
+    if (((uintptr_t)a[0].out | (uintptr_t)rp.kcache | (uintptr_t)rp.vcache | (uintptr_t)rp.cos_t | (uintptr_t)rp.sin_t) & 15 || a[0].ldo % 8 || rp.block_size < 1) return 0;
+    const int64_t units = (int64_t)a[0].T * ((a[0].N + a[1].N) / 8 + a[2].N / 4);
+    return units < (1ll << 31) - 256 ? units : 0;
 }
 // us that the streaming kernels take for one matrix and 33 .. 64 tokens, from what their time follows: the k-blocks in a row of the slowest wave.
 //   * gptq_wide_kernel, K in one range: 4.3 + 1.29 a block (512 .. 12288 rows x 1024 9.4 .. 9.8, 16384 x 8192 45.7; more waves per CU are slower by 6 % each);
@@ -1334,7 +1396,8 @@ static float gptq_gemm_us(const GtChoice& c, int T, float weights_us) {
     return c.splits == 1 ? 0.88f * c.us + 3.5f + cold : c.us + 0.2f * (float)(c.splits - 1) + 1.9f * cold + 0.03f * (float)(T - 33);
 }
 // n matrices over the same x, of one group size and zero mode; at most gptq_gemm_slab(K) tokens
-static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) {
+// (rope, three matrices: K may go in ranges, and then RoPE and the cache write are done too, *roped)
+static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st, const DenseRope* rope = nullptr, bool* roped = nullptr) {
     const DenseArgs& a = ms[0];
     const int gs = a.group_size;
     const bool silu = a.epi == MI355_EPI_SILU_MUL;
@@ -1359,8 +1422,13 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     // (64-token tiles, eight ranges), at 96 102 / 36.
     const int units = a.K / GG_UNIT;
     const float weights_us = (float)rows * (float)a.K / 2.f / 5.0e6f;
-    const GtChoice best = gt_pick(tiles, units, weights_us, n == 1 && a.T <= 65535 ? gemm_max_split(a, std::max(1, units / 4)) : 1,
-                                  (float)a.T * (float)a.N * 4.f / 4.5e6f, gs % GG_UNIT ? 6 : 7, kGgTiles, 3);
+    const float part_us = (float)a.T * 4.f / 4.5e6f;
+    GtChoice best = gt_pick(tiles, units, weights_us, n == 1 && a.T <= 65535 ? gemm_max_split(a, a.N, std::max(1, units / 4)) : 1, part_us * (float)a.N, gs % GG_UNIT ? 6 : 7, kGgTiles, 3);
+    const int64_t units3 = n == 3 && rope ? sum3_units(ms, *rope, dt) : 0;
+    if (units3) {
+        const GtChoice c = gt_pick(tiles, units, weights_us, gemm_max_split(a, rows, std::max(1, units / 4)), part_us * (float)rows, gs % GG_UNIT ? 6 : 7, kGgTiles, 3);
+        if (c.splits > 1) best = c;
+    }
     // To 64 tokens one matrix is also one sweep of the streaming kernels.  us, streaming / this (33 tokens unless given): 4096 x 512 7.0 / 8.9, x 1024 9.6 / 11.8,
     // x 2048 9.3 / 12.8, x 4096 15.5 / 15.8, x 5120 18.4 / 17.7, x 14336 22.3 / 24.7; 2048 x 14336 18.7 / 19.2, 1024 x 14336 48 tokens 15.7 / 21.6; 4608 x 14336 31.8 / 25.9;
     // 16384 x 2048 15.1 / 18.9, x 8192 45.7 / 37.9; 28672 x 8192 51 / 58; 64 tokens 4096 x 1024 8.0 / 12.2, 2048 x 3072 16.3 / 12.5
@@ -1373,10 +1441,13 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     if (tiles(t) * g.splits > 0x7FFFFFFF) return (int)hipErrorNotSupported;
     // workspace: permuted x | sums | panels | partial sums
     const size_t xp_b = (size_t)a.T * a.K * 2, xs_b = (size_t)(a.K / 64) * g.t_pad * 4, pn_b = (size_t)words * 4;
-    const size_t pt_b = g.splits > 1 ? (size_t)g.splits * a.T * a.N * 4 : 0;
+    g.ldp = n == 1 ? a.N : (int)rows;
+    for (int i = 1; i < n; ++i) g.col0[i] = g.col0[i - 1] + ms[i - 1].N;
+    const size_t pt_b = g.splits > 1 ? (size_t)g.splits * a.T * g.ldp * 4 : 0;
     void* ws = nullptr;
     Mi355ScratchTurn turn(MI355_SCR_GPTQ_GEMM, st);
-    if (mi355_scratch_get(&ws, MI355_SCR_GPTQ_GEMM, xp_b + xs_b + pn_b + pt_b, st, false, (size_t)(GPTQ_GEMM_X_BYTES + GEMM_PART_BYTES))) return (int)hipErrorNotSupported;   // (no room while a stream is captured: token chunks)
+    if (mi355_scratch_get(&ws, MI355_SCR_GPTQ_GEMM, xp_b + xs_b + pn_b + pt_b, st, false, (size_t)(GPTQ_GEMM_X_BYTES + GEMM_PART_BYTES)))
+        return n == 3 && pt_b ? gptq_prompt_gemm(ms, n, dt, st) : (int)hipErrorNotSupported;   // (no room while a stream is captured: token chunks)
     uint8_t* base = static_cast<uint8_t*>(ws);
     uint16_t* xp = reinterpret_cast<uint16_t*>(base);
     float* xs = reinterpret_cast<float*>(base + xp_b);
@@ -1386,6 +1457,15 @@ static int gptq_prompt_gemm(const DenseArgs* ms, int n, int dt, hipStream_t st) 
     gt_last_launch = 100 * best.tile + g.splits;
     const int rc = dt == MI355_DTYPE_BF16 ? gptq_gemm_dt<MI355_DTYPE_BF16>(g, xp, xs, best.tile, st) : gptq_gemm_dt<MI355_DTYPE_F16>(g, xp, xs, best.tile, st);
     if (rc || g.splits <= 1) return rc;
+    if (n == 3) {
+        DenseGemm3 s{};
+        for (int i = 0; i < 3; ++i) { s.a[i] = ms[i]; s.col0[i] = g.col0[i]; }
+        s.splits = g.splits; s.part = g.part; s.ldp = g.ldp;
+        hipLaunchKernelGGL(sum3_rope_cache_kernel, dim3((unsigned)((units3 + 255) / 256)), dim3(256), 0, st, s, *rope, (int)units3);
+        *roped = true;
+        return (int)hipGetLastError();
+    }
+    if (dt == MI355_DTYPE_BF16 && resid_norm_tail<MI355_DTYPE_BF16>(a, g.part, a.N, g.splits, a.T, st)) return (int)hipGetLastError();
     const dim3 grid(((silu ? a.pair_offset : a.N) + 255) / 256, a.T);
     if (dt == MI355_DTYPE_BF16) hipLaunchKernelGGL((gptq_wide_epilogue_kernel<MI355_DTYPE_BF16>), grid, dim3(256), 0, st, a, g.part, a.N, g.splits, a.T);
     else hipLaunchKernelGGL((gptq_wide_epilogue_kernel<MI355_DTYPE_F16>), grid, dim3(256), 0, st, a, g.part, a.N, g.splits, a.T);
@@ -1440,7 +1520,7 @@ static bool dense_streams(const DenseArgs& a, const GtChoice& c, float weights_u
     return stream <= gemm;
 }
 // n matrices over the same x: all tiled or all row-major, one dtype
-static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) {
+static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st, const DenseRope* rope = nullptr, bool* roped = nullptr) {   // (rope: as gptq_prompt_gemm)
     if (dt != MI355_DTYPE_BF16 && dt != MI355_DTYPE_F16) return (int)hipErrorNotSupported;
     for (int i = 0; i < n; ++i) {
         if (a[i].K % 64 || a[i].T < 1 || a[i].N < 1 || a[i].wtiled != a[0].wtiled || a[i].epi != a[0].epi) return (int)hipErrorNotSupported;
@@ -1467,13 +1547,21 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     // 128 x 128 640), 3001 x 4096 x 14336 480 / 292 (192 x 256: exactly one round; 256 x 256 331), 2048 x 28672 x 4096 550 / 375,
     // 2048 x 4096 x 14336 215 (128 x 128, two per CU), 700 x 4096 x 14336 94 (two ranges; one: 175), 96 x 4096 x 14336 33 (64-token tiles,
     // eight ranges; one: 113), 64 x 28672 x 4096 96 / 44.
-    const int max_split = n == 1 && a[0].T <= 65535 && !(a[0].N & 3) && !(a[0].epi == MI355_EPI_SILU_MUL && (a[0].pair_offset & 3)) ? gemm_max_split(a[0], std::max(1, units / 8)) : 1;
+    const int max_split = n == 1 && a[0].T <= 65535 && !(a[0].N & 3) && !(a[0].epi == MI355_EPI_SILU_MUL && (a[0].pair_offset & 3)) ? gemm_max_split(a[0], a[0].N, std::max(1, units / 8)) : 1;
     const float weights_us = (float)rows * (float)a[0].K * 2.f / 5.4e6f;
     GtChoice best = gt_pick([&](const GtTile& t) { return tiles(t, nullptr); }, units, weights_us, max_split,
                             (float)a[0].T * (float)a[0].N * 4.f / 4.5e6f, 63);
     if (n == 1 && g_tune_gemm_min_t == DENSE_GEMM_MIN_T && !g_tune_gemm_tall && dense_streams(a[0], best, weights_us)) return (int)hipErrorNotSupported;
+    const int64_t units3 = n == 3 && rope ? sum3_units(a, *rope, dt) : 0;
+    if (units3) {
+        const GtChoice c = gt_pick([&](const GtTile& t) { return tiles(t, nullptr); }, units, weights_us, gemm_max_split(a[0], rows, std::max(1, units / 8)),
+                                   (float)a[0].T * (float)rows * 4.f / 4.5e6f, 63);
+        if (c.splits > 1) best = c;
+    }
     if (g_tune_gemm_tall) best = {0, 1, 0.f};
     DenseGemm3 g{};
+    g.ldp = n == 1 ? a[0].N : (int)rows;
+    for (int i = 1; i < n; ++i) g.col0[i] = g.col0[i - 1] + a[i - 1].N;
     for (int i = 0; i < 3; ++i) g.a[i] = a[i < n ? i : 0];
     g.n_m = (a[0].T + kGtTiles[best.tile].bm - 1) / kGtTiles[best.tile].bm;
     g.units_per_split = (units + best.splits - 1) / best.splits;
@@ -1481,14 +1569,18 @@ static int dense_prompt_gemm(const DenseArgs* a, int n, int dt, hipStream_t st) 
     Mi355ScratchTurn turn(MI355_SCR_GPTQ_WIDE, st);
     if (g.splits > 1) {
         void* p = nullptr;
-        if (mi355_scratch_get(&p, MI355_SCR_GPTQ_WIDE, (size_t)g.splits * a[0].T * a[0].N * sizeof(float), st, false, (size_t)GEMM_PART_BYTES)) { g.splits = 1; g.units_per_split = units; }
+        if (mi355_scratch_get(&p, MI355_SCR_GPTQ_WIDE, (size_t)g.splits * a[0].T * g.ldp * sizeof(float), st, false, (size_t)GEMM_PART_BYTES)) { g.splits = 1; g.units_per_split = units; }
         g.part = static_cast<float*>(p);
     }
     if (tiles(kGtTiles[best.tile], &g) * g.splits > 0x7FFFFFFF) return (int)hipErrorNotSupported;
     gt_last_launch = 100 * best.tile + g.splits;
     if (dt == MI355_DTYPE_BF16) { if (a[0].wtiled) dense_gemm_epi<MI355_DTYPE_BF16, true>(g, best.tile, st); else dense_gemm_epi<MI355_DTYPE_BF16, false>(g, best.tile, st); }
     else { if (a[0].wtiled) dense_gemm_epi<MI355_DTYPE_F16, true>(g, best.tile, st); else dense_gemm_epi<MI355_DTYPE_F16, false>(g, best.tile, st); }
-    if (g.splits > 1) {
+    if (g.splits > 1 && n == 3) {
+        hipLaunchKernelGGL(sum3_rope_cache_kernel, dim3((unsigned)((units3 + 255) / 256)), dim3(256), 0, st, g, *rope, (int)units3);
+        *roped = true;
+    } else if (g.splits > 1 && dt == MI355_DTYPE_BF16 && resid_norm_tail<MI355_DTYPE_BF16>(a[0], g.part, a[0].N, g.splits, a[0].T, st)) {
+    } else if (g.splits > 1) {
         const int n_out = a[0].epi == MI355_EPI_SILU_MUL ? a[0].pair_offset : a[0].N;
         const dim3 grid((n_out + 255) / 256, a[0].T);
         if (dt == MI355_DTYPE_BF16) hipLaunchKernelGGL((gptq_wide_epilogue_kernel<MI355_DTYPE_BF16>), grid, dim3(256), 0, st, a[0], g.part, a[0].N, g.splits, a[0].T);
@@ -1873,11 +1965,11 @@ int mi355_linear(void* out, const void* x, const void* w, const void* bias, cons
     return dense_run(a, DW_DENSE, dtype, (hipStream_t)stream);
 }
 
-/* a decode step's residual product and the RmsNorm behind it: out = residual + x . w^T as mi355_linear / _linear_tiled / _gptq_linear_tiled (kind 0, 1, 2; symmetric
+/* a residual product and the RmsNorm behind it: out = residual + x . w^T as mi355_linear / _linear_tiled / _gptq_linear_tiled (kind 0, 1, 2; symmetric
  * zero points); *normed != 0: norm_out holds the norm of out too (else the caller makes it).  Internal to the host layer. */
 int mi355_internal_resid_norm_linear(void* out, const void* x, const void* w, const void* scales, const void* residual, int32_t num_tokens, int32_t n, int32_t k,
                                      int32_t group_size, int32_t kind, int32_t dtype, void* norm_out, const void* norm_w, float eps, int32_t* normed, int64_t stream) {
-    if (!residual || !norm_out || !norm_w || !normed || num_tokens < 1 || num_tokens > 32 || kind < 0 || kind > 2) return -1;
+    if (!residual || !norm_out || !norm_w || !normed || num_tokens < 1 || kind < 0 || kind > 2) return -1;
     DenseNormTail tail{norm_out, norm_w, eps, false};
     DenseArgs a{};
     a.w = w; a.ldw = k; a.wtiled = kind == 1; a.scales = scales; a.zmode = kind == 2 ? MI355_ZERO_SYM8 : 0; a.sperm = SP_NONE;
@@ -1941,6 +2033,10 @@ int mi355_gptq_linear_tiled(void* out, const void* x, const void* qweight_tiled,
                             n, k, group_size, dtype, epilogue, stream);
 }
 
+int mi355_internal_linear3_prompt(void* const* outs, const void* x, const void* const* ws, const void* const* scales,
+                                  const void* const* biases, const int32_t* ns, int32_t num_tokens, int32_t k, int32_t group_size,
+                                  int32_t is_gptq, int32_t dtype, const void* norm_w, float norm_eps, const float* ss_in, const void* rope,
+                                  const void* prompt_rope, int32_t* roped, int64_t stream);
 /* q, k, v projections (plain store epilogue, optional bias) in one launch; returns -4 when the shapes do not qualify
  * (the caller then issues three mi355_linear / mi355_gptq_linear calls).  norm_w != NULL: x is the residual stream and the
  * launch applies RmsNorm(norm_w, eps) on the way in, inv from the producer's sums of squares `ss_in` (1..4 tokens of 4-bit
@@ -1951,6 +2047,15 @@ int mi355_internal_linear3(void* const* outs, const void* x, const void* const* 
                            const void* const* biases, const int32_t* ns, int32_t num_tokens, int32_t k, int32_t group_size,
                            int32_t is_gptq, int32_t dtype, const void* norm_w, float norm_eps, const float* ss_in, const void* rope,
                            int64_t stream) {
+    return mi355_internal_linear3_prompt(outs, x, ws, scales, biases, ns, num_tokens, k, group_size, is_gptq, dtype, norm_w, norm_eps, ss_in, rope, nullptr, nullptr, stream);
+}
+/* the same for a prompt step (rope NULL): *roped != 0: the launch also rotated q and wrote the rotated k and v into the cache as prompt_rope says (k's and v's outs are not
+ * written then); else the caller does */
+int mi355_internal_linear3_prompt(void* const* outs, const void* x, const void* const* ws, const void* const* scales,
+                                  const void* const* biases, const int32_t* ns, int32_t num_tokens, int32_t k, int32_t group_size,
+                                  int32_t is_gptq, int32_t dtype, const void* norm_w, float norm_eps, const float* ss_in, const void* rope,
+                                  const void* prompt_rope, int32_t* roped, int64_t stream) {
+    if (roped) *roped = 0;
     // One GEMM launch for the three (K in one range), or the streaming kernel over all their row tiles (to 64 tokens).  us, streaming / GEMM, weights from HBM
     // (q + k + v rows x k): 16-bit 2048 + 2 x 512 x 2048 33 tokens 9.3 / 11.0, 49 11.4 / 16.0, 64 12.9 / 17.0; 3 x 2048 x 2048 33 14.5 / 16.0, 48 17.3 / 16.9; 4096 + 2 x 1024
     // x 1024 33 9.3 / 10.1, 48 10.7 / 10.5, x 4096 33 24.1 / 27.9, 48 29.4 / 29.3, 49 31.5 / 29.3; 5120 + 2 x 1024 x 5120 40 32.5 / 36.8, 48 36.6 / 38.2, 56 42.3 / 39.3; 3 x 2048 x 512 33
@@ -1979,10 +2084,13 @@ int mi355_internal_linear3(void* const* outs, const void* x, const void* const* 
     if (prompt) {
         int rc = 0;
         const int slab = is_gptq == 2 ? gptq_gemm_slab(k) : num_tokens;
+        const DenseRope* pr = slab >= num_tokens && roped ? static_cast<const DenseRope*>(prompt_rope) : nullptr;
+        bool did = false;
         for (int t0 = 0; t0 < num_tokens && rc == 0; t0 += slab) {
             const DenseArgs c[3] = {dense_rows(a[0], t0, slab), dense_rows(a[1], t0, slab), dense_rows(a[2], t0, slab)};
-            rc = is_gptq == 2 ? gptq_prompt_gemm(c, 3, dtype, st) : dense_prompt_gemm(c, 3, dtype, st);
+            rc = is_gptq == 2 ? gptq_prompt_gemm(c, 3, dtype, st, pr, &did) : dense_prompt_gemm(c, 3, dtype, st, pr, &did);
         }
+        if (roped) *roped = did;
         if (rc != (int)hipErrorNotSupported) return rc;
         if (num_tokens > 64) return -4;
     }

@@ -33,6 +33,10 @@ extern "C" int mi355_internal_linear3(void* const* outs, const void* x, const vo
                                       const void* const* biases, const int32_t* ns, int32_t num_tokens, int32_t k,
                                       int32_t group_size, int32_t is_gptq, int32_t dtype, const void* norm_w, float norm_eps,
                                       const float* ss_in, const void* rope, int64_t stream);
+extern "C" int mi355_internal_linear3_prompt(void* const* outs, const void* x, const void* const* ws, const void* const* scales,
+                                      const void* const* biases, const int32_t* ns, int32_t num_tokens, int32_t k,
+                                      int32_t group_size, int32_t is_gptq, int32_t dtype, const void* norm_w, float norm_eps,
+                                      const float* ss_in, const void* rope, const void* prompt_rope, int32_t* roped, int64_t stream);
 // mirror of dense_gemv.hip's DenseRope: RoPE + KV-cache write in the epilogue of the q/k/v launch
 struct DenseRope {
     const float* cos_t; const float* sin_t;
@@ -243,7 +247,7 @@ int resid_linear(const DModel* m, const uint16_t* w, const QLin& g, const void* 
         if (rc == 0) { *ss_valid = true; return 0; }
         if (rc != -4) return rc;
     }
-    if (next_norm && T <= 32 && m->cfg.norm_type == 0 && (g.qw || w)) {
+    if (next_norm && m->cfg.norm_type == 0 && (g.qw || w)) {
         int32_t done = 0;
         const int rc = mi355_internal_resid_norm_linear(m->xs, x, g.qw ? (const void*)g.qw : (const void*)w, g.scales, m->xs, T, n, k, g.group, g.qw ? 2 : (int)m->tiled.count(w),
                                                         m->cfg.dtype, m->xn, next_norm, m->cfg.rms_eps, &done, stream);
@@ -526,10 +530,13 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
                     if (!xn_ready) DCHECK(norm(m, m->xn, m->xs, L.attn_norm, L.attn_norm_b, T, stream));
                     normed = true;
                     for (int pass = rope_ok ? 0 : 1; pass < 2 && rc3 != 0; ++pass) {
-                        rc3 = mi355_internal_linear3(outs, m->xn, ws, sc, bs, ns, T, hid, gq.group, all_q ? 2 : (m->tiled.count(L.wq) ? 3 : 0), m->cfg.dtype, nullptr, 0.f, nullptr,
-                                                     pass == 0 ? &rp : nullptr, stream);
+                        // (a prompt with a bf16 cache and full, non-interleaved rotary: the launch that adds ranges of K does RoPE and the cache write too)
+                        int32_t done = 0;
+                        const bool prompt_rope = prefill && !c.kv_fp8 && c.rotary_dim == D && !c.rope_interleaved;
+                        rc3 = mi355_internal_linear3_prompt(outs, m->xn, ws, sc, bs, ns, T, hid, gq.group, all_q ? 2 : (m->tiled.count(L.wq) ? 3 : 0), m->cfg.dtype, nullptr, 0.f,
+                                                            nullptr, pass == 0 ? &rp : nullptr, prompt_rope ? &rp : nullptr, &done, stream);
                         if (rc3 != 0 && rc3 != -4) return rc3;
-                        roped = rc3 == 0 && pass == 0;
+                        roped = rc3 == 0 && (pass == 0 || done);
                     }
                 }
             }
@@ -570,7 +577,7 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
                                                  cap, ps, scale, 0.f, 1.f, 1.f, stream));
             }
         } else {
-        if (!fused_rc)
+        if (!fused_rc)                                                  // (RoPE and the cache write go together in every launch that does one)
         DCHECK(mi355_reshape_and_cache(m->k, m->v, m->kcache[l], m->vcache[l], slot_mapping, T, Hkv, D, c.block_size, 2,
                                        c.kv_layout, stream));
         if (prefill) {

@@ -846,3 +846,68 @@ def test_two_threads_on_one_stream(cv, kind, T, N, K):
     torch.cuda.synchronize()
     for i in range(2):
         assert len(got[i]) == 300 and all(torch.equal(y.view(torch.int16), alone[i].view(torch.int16)) for y in got[i])
+
+
+# K in ranges: prompts whose tiles leave units idle, in 16 and 4 bits, both cache layouts, biases, heads of 64, 128 and 80, tokens that the cache does not take
+@pytest.mark.parametrize("T,H,G_,D,K,bits,flash,bias", [(66, 16, 4, 128, 2048, 16, False, False), (99, 16, 4, 128, 2048, 16, True, True), (359, 16, 4, 64, 4096, 16, False, False),
+                                                         (50, 28, 4, 128, 3584, 4, False, True), (133, 28, 4, 128, 3584, 4, True, False), (150, 14, 2, 64, 4096, 4, False, True),
+                                                         (70, 8, 2, 80, 2048, 16, False, True)])
+def test_three_products_in_ranges_of_k_with_rope_and_cache(cv, T, H, G_, D, K, bits, flash, bias):
+    """q, rotated, and the rotated k and v in the cache by the launch that adds the ranges: each within the bf16 steps of its rounding chain (product, bias, rotation) of
+    64 bits, the cache's other slots untouched"""
+    import ctypes
+    from candle_vllm_amd import lib
+    gen, st = torch.Generator(device="cuda").manual_seed(T + K), torch.cuda.current_stream().cuda_stream
+    ns, bs = (H * D, G_ * D, G_ * D), 32
+    x, out, ws, ss, refs, bb = torch.randn(T, K, generator=gen, device="cuda").to(torch.bfloat16), [], [], [], [], []
+    for n in ns:
+        out.append(torch.full((T, n), float("nan"), device="cuda", dtype=torch.bfloat16))
+        bb.append(torch.randn(n, generator=gen, device="cuda").to(torch.bfloat16))
+        if bits == 16:
+            w = (torch.randn(n, K, generator=gen, device="cuda") * 0.05).to(torch.bfloat16)
+            img = torch.empty_like(w)
+            assert lib.mi355_dense_tile_repack(w.data_ptr(), img.data_ptr(), n, K, K, st) == 0
+            wd = w.double().T
+        else:
+            q = torch.randint(0, 16, (K, n), generator=gen, device="cuda", dtype=torch.int32)
+            packed = sum((q.view(K // 8, 8, n)[:, i] << (4 * i)) for i in range(8)).contiguous()
+            img = torch.empty_like(packed)
+            assert lib.mi355_gptq_tile_repack(packed.data_ptr(), img.data_ptr(), K, n, 0, st) == 0
+            ss.append((torch.rand(K // 128, n, generator=gen, device="cuda") * 0.01 + 0.002).to(torch.bfloat16))
+            wd = ((q.double() - 8).view(K // 128, 128, n) * ss[-1].double()[:, None]).view(K, n)
+        ws.append(img)
+        refs.append(x.double() @ wd + (bb[-1].double() if bias else 0))
+    nb = (T + 40) // bs + 1
+    shape = (nb, bs, G_, D) if flash else (nb, G_, D // 8, bs, 8)
+    kc, vc = torch.full(shape, 7.0, device="cuda", dtype=torch.bfloat16), torch.full(shape if flash else (nb, G_, D, bs), 7.0, device="cuda", dtype=torch.bfloat16)
+    pos = torch.randint(0, 500, (T,), generator=gen, device="cuda")
+    slot = torch.randperm(nb * bs, device="cuda")[:T]
+    slot[3] = -1
+    ang = torch.arange(500, device="cuda").double()[:, None] * 10000.0 ** (-torch.arange(D // 2, device="cuda").double() / (D // 2))
+    cos, sin = ang.cos().float().contiguous(), ang.sin().float().contiguous()
+
+    class Rope(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_void_p) for n in ("cos", "sin", "pos", "slots", "kc", "vc")] + [(n, ctypes.c_int32) for n in ("kv", "d", "bs", "flash")]
+    rope = Rope(cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), slot.data_ptr(), kc.data_ptr(), vc.data_ptr(), G_, D, bs, int(flash))
+    p3 = lambda ts: (ctypes.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    fn = lib.mi355_internal_linear3_prompt
+    fn.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_int32] * 5 + [ctypes.c_void_p, ctypes.c_float] + [ctypes.c_void_p] * 4 + [ctypes.c_int64]
+    done = ctypes.c_int32(-1)
+    lib.mi355_internal_last_gemm()
+    assert fn(p3(out), x.data_ptr(), p3(ws), p3(ss) if ss else None, p3(bb) if bias else None, (ctypes.c_int32 * 3)(*ns), T, K, 128, 3 if bits == 16 else 2, 2, None, 0.0, None, None,
+              ctypes.byref(rope), ctypes.byref(done), st) == 0
+    assert lib.mi355_internal_last_gemm() % 100 > 1 and done.value == 1
+    c, s = ang.cos()[pos][:, None], ang.sin()[pos][:, None]
+
+    def turned(y):
+        a, b = y.view(T, -1, D)[..., :D // 2], y.view(T, -1, D)[..., D // 2:]
+        return torch.cat([a * c - b * s, b * c + a * s], -1), torch.cat([a.abs() + b.abs()] * 2, -1)
+    flat = (lambda t: t.reshape(nb * bs, G_, D)) if flash else (lambda t: (t.permute(0, 3, 1, 2, 4) if t.dim() == 5 else t.permute(0, 3, 1, 2)).reshape(nb * bs, G_, D))
+    ok = slot >= 0
+    for got, (want, mag) in ((out[0].view(T, H, D), turned(refs[0])), (flat(kc)[slot[ok]], [v[ok] for v in turned(refs[1])]),
+                             (flat(vc)[slot[ok]], (refs[2].view(T, G_, D)[ok], refs[2].view(T, G_, D)[ok].abs()))):
+        # product, bias and rotation are rounded to bf16 each: 2^-8 of the largest value in the chain at most (the sums of K products in f32 are far below)
+        assert ((got.double() - want).abs() <= 3.0 * 2.0 ** -8 * (mag + (0 if not bias else 8.0)) + 1e-6).all()
+    rest = torch.ones(nb * bs, dtype=torch.bool, device="cuda")
+    rest[slot[ok]] = False
+    assert (flat(kc)[rest] == 7).all() and (flat(vc)[rest] == 7).all()
