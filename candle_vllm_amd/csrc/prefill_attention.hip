@@ -369,10 +369,16 @@ __device__ __forceinline__ float pfl_max_over_rows(float x) {
     r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-constexpr int PFL_STAGES = 2, PFL_QT = 2;                            // stages of the ring, query tiles of 16 per workgroup
-__global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillParams p, const uint32_t* __restrict__ btab,
+// Launches that leave CUs idle take smaller tiles (QT = 1: 16 queries, 126 registers, half the chain of MFMAs and softmax per stage) and KG = 2
+// groups of four waves that take the stages in turn, each through a ring of its own, and meet at the end: maxima, sums and O of the second group
+// go through LDS to the first, rescaled in f32 as at any stage.  What bounds such a launch is the longest chain of stages, about 2.2 us each for 32
+// queries, 1.5 for 16 and 0.9 in two groups (66 tokens behind 700 cached: 29.2, 21.2, 17.0 us): mi355_internal_prefill_form picks.
+constexpr int PFL_STAGES = 2;                                        // stages of a ring
+// QT query tiles of 16 per workgroup, KG groups of four waves
+template <int QT, int KG>
+__global__ void __launch_bounds__(256 * KG, 2) prefill_attn_lds_kernel(const PrefillParams p, const uint32_t* __restrict__ btab,
                                                                    const uint32_t* __restrict__ clens, const uint32_t* __restrict__ cuq) {
-    constexpr int D = 128, NC = 4, NDT = 8, R = PFL_STAGES, QT = PFL_QT;
+    constexpr int D = 128, NC = 4, NDT = 8, R = PFL_STAGES;
     constexpr uint32_t STAGE_B = 32768u;
     extern __shared__ __attribute__((aligned(1024))) uint8_t pfl_smem[];
     // QT = query tiles of 16 per workgroup.  Grid: x = head group (fastest), y = query block, HEAVIEST FIRST (the last block of a prompt sees
@@ -380,7 +386,7 @@ __global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillP
     const int qb = (int)gridDim.y - 1 - (int)blockIdx.y, seq = blockIdx.z;
     const int G = p.H / p.Hkv, HG = (G + 3) >> 2;                     // head groups of up to four query heads per kv head
     const int hk = (int)blockIdx.x / HG, hg = (int)blockIdx.x % HG;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) & 3), grp = KG > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)) : 0;
     const int c = lane & 15, kg = lane >> 4;
     const int bs = p.block_size, bs_shift = __ffs(bs) - 1, E = 64 >> bs_shift;
     const int q_begin = (int)cuq[seq], qlen = (int)cuq[seq + 1] - q_begin;
@@ -392,7 +398,7 @@ __global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillP
     const bool active = hw < G;                                       // this wave has a head (all waves copy and meet at the barriers)
     const int h = hk * G + (active ? hw : 0);
     const int kend = min(ctx, cached + min(q0 + 16 * QT, qlen));           // keys this block can see (exclusive)
-    const int ns = (kend + 63) >> 6;
+    const int ns = (kend + 63) >> 6, trips = (ns + KG - 1) / KG, mine = (ns - grp + KG - 1) / KG;   // stages: all, of the longest group, of this one (grp, grp + KG, ..)
     const int nblk = (ctx + bs - 1) >> bs_shift;
     // ---- Q fragments (B operand: lane = query c of tile qt, k = d 32j + 8kg ..) and the query's position
     uint4 qf[QT][NC];
@@ -411,19 +417,22 @@ __global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillP
     // the compiler's wait for these loads must come before the first DMA goes out (it knows nothing of the DMA queue)
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) asm volatile("" : "+v"(qf[qt][0].x), "+v"(qf[qt][1].x), "+v"(qf[qt][2].x), "+v"(qf[qt][3].x));
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) void*)pfl_smem);
+    uint8_t* const ring = pfl_smem + grp * (R * STAGE_B);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) void*)ring);
     const uint8_t* kc8 = static_cast<const uint8_t*>(p.k);
     const uint8_t* vc8 = static_cast<const uint8_t*>(p.v);
     const int ktok = pal_dma_token(0, lane);
-    auto load_ent = [&](int st, int (&ent)[4]) {
+    auto load_ent = [&](int i, int (&ent)[4]) {                        // of this group's stage i
+        const int st = i * KG + grp;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int idx = min(st * E + min(e, E - 1), nblk - 1);
             ent[e] = (int)btab[(int64_t)seq * p.max_blocks + idx];
         }
     };
-    auto issue = [&](int st, const int (&ent)[4]) {
-        const uint32_t dst = lds0 + (uint32_t)(st % R) * STAGE_B + (uint32_t)wave * 8192u;
+    auto issue = [&](int i, const int (&ent)[4]) {
+        const int st = i * KG + grp;
+        const uint32_t dst = lds0 + (uint32_t)(i % R) * STAGE_B + (uint32_t)wave * 8192u;
         auto block_of = [&](int tok) {
             const int e = tok >> bs_shift;
             return (int64_t)(e == 0 ? ent[0] : (e == 1 ? ent[1] : (e == 2 ? ent[2] : ent[3])));
@@ -453,8 +462,8 @@ __global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillP
     int ent[4];
 #pragma unroll
     for (int st = 0; st < R - 1; ++st)
-        if (st < ns) { load_ent(st, ent); issue(st, ent); }
-    if (R - 1 < ns) load_ent(R - 1, ent);
+        if (st < mine) { load_ent(st, ent); issue(st, ent); }
+    if (R - 1 < mine) load_ent(R - 1, ent);
     float m_run[QT], l_run[QT];
     f32x4_t o[QT][NDT];
 #pragma unroll
@@ -463,32 +472,34 @@ __global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillP
 #pragma unroll
         for (int nt = 0; nt < NDT; ++nt) o[qt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-    for (int i = 0; i < ns; ++i) {
+    for (int i = 0; i < trips; ++i) {
         {
             static_assert(R == 2, "the stage requested in the iteration before is the only one under way");
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __syncthreads();
-        if (i + R - 1 < ns) {
+        if (i + R - 1 < mine) {
             issue(i + R - 1, ent);
-            if (i + R < ns) load_ent(i + R, ent);
+            if (i + R < mine) load_ent(i + R, ent);
         }
-        uint8_t* Kb = pfl_smem + (size_t)(i % R) * STAGE_B;
-        const int tb = 64 * i;
-        if (tb + 64 > ctx) {                                          // the last stage: values at or beyond ctx hold arbitrary bits, cleared here (the stage is in LDS, no DMA aims at it)
+        uint8_t* Kb = ring + (size_t)(i % R) * STAGE_B;
+        const int tb = 64 * (i * KG + grp);
+        if (i == trips - 1 && 64 * ns > ctx) {                        // (uniform for the workgroup)
+            if (i < mine && tb + 64 > ctx) {                          // the last stage: values at or beyond ctx hold arbitrary bits, cleared here (the stage is in LDS, no DMA aims at it)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int piece = ((int)threadIdx.x >> 7) * 4 + q, first = tb + 32 * (piece >> 2) + 8 * (piece & 3);
-                uint4* const at = reinterpret_cast<uint4*>(Kb + pal_v_read_off((int)threadIdx.x & 127, piece >> 2, piece & 3));
-                uint32_t m[4];
+                for (int q = 0; q < 4; ++q) {
+                    const int piece = (((int)threadIdx.x & 255) >> 7) * 4 + q, first = tb + 32 * (piece >> 2) + 8 * (piece & 3);
+                    uint4* const at = reinterpret_cast<uint4*>(Kb + pal_v_read_off((int)threadIdx.x & 127, piece >> 2, piece & 3));
+                    uint32_t m[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) m[e] = (first + 2 * e < ctx ? 0x0000FFFFu : 0u) | (first + 2 * e + 1 < ctx ? 0xFFFF0000u : 0u);
-                const uint4 v = *at;
-                *at = make_uint4(v.x & m[0], v.y & m[1], v.z & m[2], v.w & m[3]);
+                    for (int e = 0; e < 4; ++e) m[e] = (first + 2 * e < ctx ? 0x0000FFFFu : 0u) | (first + 2 * e + 1 < ctx ? 0xFFFF0000u : 0u);
+                    const uint4 v = *at;
+                    *at = make_uint4(v.x & m[0], v.y & m[1], v.z & m[2], v.w & m[3]);
+                }
             }
             __syncthreads();
         }
-        if (!active) continue;                                        // uniform per wave; the barriers are above
+        if (!active || i >= mine) continue;                           // uniform per wave; the barriers are above
         const bool diag = tb + 63 > cached + q0;                      // some query of the block does not see the whole stage
         // ---- K fragments of the stage: tile (ip, it), k-step j
         uint4 ka[2][2][NC];
@@ -544,7 +555,8 @@ __global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillP
 #pragma unroll
                     for (int v = 0; v < 4; ++v) tmax = fmaxf(tmax, x[ip][it][v]);
             tmax = pfl_max_over_rows(tmax);
-            const float m_new = fmaxf(m_run[qt], tmax * sl);          // finite from the first stage on: key 0 is visible to every query
+            float m_new = fmaxf(m_run[qt], tmax * sl);                // finite from the first stage on: key 0 is visible to every query (of group 0)
+            if (KG > 1 && m_new == -INFINITY) m_new = 0.f;            // (no key of this group's is visible, and none of its later ones: nothing, at any scale)
             alpha[qt] = __builtin_amdgcn_exp2f(m_run[qt] - m_new);
             m_run[qt] = m_new;
             float psum = 0.f;
@@ -598,16 +610,53 @@ __global__ void __launch_bounds__(256, 2) prefill_attn_lds_kernel(const PrefillP
             }
         }
     }
+    float l_all[QT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) { l_all[qt] = l_run[qt] + __shfl_xor(l_run[qt], 16); l_all[qt] += __shfl_xor(l_all[qt], 32); }
+    if constexpr (KG > 1) {
+        // ---- the groups' states of (head, query): maxima, sums and O of group 1 .. through LDS to group 0
+        constexpr int PER = QT * (NDT * 4 + 2);
+        static_assert((KG - 1) * 4 * PER * 256 <= KG * R * (int)STAGE_B, "the rings' LDS");
+        float* const sm = reinterpret_cast<float*>(pfl_smem) + lane;
+        __syncthreads();                                              // every wave is done with the stages
+        if (grp) {
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) {
+                float* const at = sm + (((grp - 1) * 4 + wave) * PER + qt * (NDT * 4 + 2)) * 64;
+                at[0] = m_run[qt]; at[64] = l_all[qt];
+#pragma unroll
+                for (int nt = 0; nt < NDT; ++nt)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) at[(2 + nt * 4 + v) * 64] = o[qt][nt][v];
+            }
+        }
+        __syncthreads();
+        if (grp) return;
+#pragma unroll
+        for (int g = 1; g < KG; ++g)
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) {
+                const float* const at = sm + (((g - 1) * 4 + wave) * PER + qt * (NDT * 4 + 2)) * 64;
+                const float mg = at[0], lg = at[64], mx = lg > 0.f ? fmaxf(m_run[qt], mg) : m_run[qt];   // (nothing there: its maximum says nothing)
+                const float wa = __builtin_amdgcn_exp2f(m_run[qt] - mx), wb = lg > 0.f ? __builtin_amdgcn_exp2f(mg - mx) : 0.f;
+                m_run[qt] = mx;
+                l_all[qt] = l_all[qt] * wa + lg * wb;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float va = __shfl(wa, 4 * kg + v), vb = __shfl(wb, 4 * kg + v);
+#pragma unroll
+                    for (int nt = 0; nt < NDT; ++nt) o[qt][nt][v] = o[qt][nt][v] * va + at[(2 + nt * 4 + v) * 64] * vb;
+                }
+            }
+    }
     if (!active) return;
     // ---- epilogue: rows (queries 4kg+v of tile qt) need the sums of lane (4kg+v)
     uint16_t* out16 = static_cast<uint16_t*>(p.out);
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
-        float lt = l_run[qt] + __shfl_xor(l_run[qt], 16);
-        lt += __shfl_xor(lt, 32);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const float lq = __shfl(lt, 4 * kg + v);
+            const float lq = __shfl(l_all[qt], 4 * kg + v);
             const int ql = q0 + 16 * qt + 4 * kg + v;
             if (ql >= qlen) continue;
             const float inv = 1.f / lq;
@@ -630,6 +679,36 @@ static void prefill_launch_src(const PrefillParams& p, int src, dim3 grid, hipSt
     }
 }
 
+template <int QT, int KG>
+static void pfl_launch(const PrefillParams& p, int hgs, int num_seqs, int max_seqlen_q, const uint32_t* block_tables, const uint32_t* context_lens, const uint32_t* cu_seqlens_q,
+                       hipStream_t st) {
+    constexpr int LDS = KG * PFL_STAGES * 32768;
+    static Mi355DevOnce attr_done;
+    if (!attr_done.done()) {
+        (void)hipFuncSetAttribute((const void*)prefill_attn_lds_kernel<QT, KG>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        attr_done.set();
+    }
+    hipLaunchKernelGGL((prefill_attn_lds_kernel<QT, KG>), dim3(hgs, (max_seqlen_q + 16 * QT - 1) / (16 * QT), num_seqs), dim3(256 * KG), LDS, st, p, block_tables, context_lens, cu_seqlens_q);
+}
+/* 10 * QT + KG of the LDS kernel's form, from what the host knows of a launch (contexts are on the device).  Times in us, 32 heads, 8 kv heads;
+ * "21 / 11 / 12 / 22" are the forms:
+ *  - 16-query workgroups fit one per CU: eight waves on one tile, since nothing else would use the CU (381 tokens behind 450: 31.6 / 23.8 /
+ *    19.6 / 27.0; 99 tokens 9.5 / 7.1 / 7.0 / 10.3); a table of one stage has nothing to share out (32 tokens 7.5 / 5.6 / 6.3 / 9.2).
+ *  - two per CU (the LDS of form 11): as many waves without a merge (200 tokens x 4 12.9 / 12.2 / 14.6); from 512 tokens on the queries' key
+ *    counts differ so much that half as many stages in the longest chain win (1024 tokens 37.5 / 29.5 / 26.5, 512 x 2 22.7 / 20.6 / 19.1).
+ *  - up to three: the small tiles' finer tail is worth their second read of K and V if prompts are not short (300 x 4 21.9 / 15.6, 1200 tokens
+ *    45.1 / 35.3, 1200 behind 1200 88.3 / 88.0; 60 x 20 11.6 / 12.1).
+ *  - behind that K and V are read by as few workgroups as possible; only where all 32-query workgroups of long prompts are on the chip at once
+ *    the longest chain is what ends it, and two groups halve that (2048 tokens 74.5 / 69.7 / 82.8 / 64.6, behind 2048 168.8 / 180.2 / 206.5 /
+ *    159.8; but 2300 tokens 84.8 / 83.7 / 104.9 / 87.2, 250 x 8 behind 250 34.9 / 36.6 / 45.4 / 39.0). */
+extern "C" int mi355_internal_prefill_form(int32_t num_heads, int32_t num_kv_heads, int32_t num_seqs, int32_t max_seqlen_q, int32_t max_blocks_per_seq, int32_t block_size) {
+    const int64_t cus = mi355_num_cus(), hgs = (int64_t)num_kv_heads * ((num_heads / num_kv_heads + 3) / 4) * num_seqs;
+    const int64_t n16 = hgs * (((int64_t)max_seqlen_q + 15) / 16), n32 = hgs * (((int64_t)max_seqlen_q + 31) / 32);
+    if (n16 <= cus) return (int64_t)max_blocks_per_seq * block_size <= 64 ? 11 : 12;
+    if (n16 <= 2 * cus) return max_seqlen_q >= 512 ? 12 : 11;
+    if (2 * n32 <= 3 * cus && max_seqlen_q >= 128) return 11;
+    return n32 <= 2 * cus && max_seqlen_q >= 1024 ? 22 : 21;
+}
 extern "C" int mi355_prefill_attention(void* out, const void* q, const void* k, const void* v, const void* key_cache,
                                        const void* value_cache, const uint32_t* block_tables, const uint32_t* context_lens,
                                        const uint32_t* cu_seqlens_q, int32_t num_seqs, int32_t max_seqlen_q,
@@ -655,14 +734,10 @@ extern "C" int mi355_prefill_attention(void* out, const void* q, const void* k, 
     const bool mfma_ok = (head_dim == 64 || head_dim == 128) && (src != SRC_PAGED || block_size % 16 == 0);
     if (g_pf_lds && src == SRC_PAGED && dtype == MI355_DTYPE_BF16 && head_dim == 128 &&
         (block_size == 16 || block_size == 32 || block_size == 64)) {
-        static Mi355DevOnce attr_done;
-        if (!attr_done.done()) {
-            (void)hipFuncSetAttribute((const void*)prefill_attn_lds_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PFL_STAGES * 32768);
-            attr_done.set();
-        }
         const int G = num_heads / num_kv_heads, hgs = num_kv_heads * ((G + 3) / 4);
-        const dim3 grid(hgs, (max_seqlen_q + 16 * PFL_QT - 1) / (16 * PFL_QT), num_seqs);
-        hipLaunchKernelGGL(prefill_attn_lds_kernel, grid, dim3(256), PFL_STAGES * 32768, st, p, block_tables, context_lens, cu_seqlens_q);
+        const int form = mi355_internal_prefill_form(num_heads, num_kv_heads, num_seqs, max_seqlen_q, max_blocks_per_seq, block_size);
+        const auto launch = form == 11 ? pfl_launch<1, 1> : form == 12 ? pfl_launch<1, 2> : form == 22 ? pfl_launch<2, 2> : pfl_launch<2, 1>;
+        launch(p, hgs, num_seqs, max_seqlen_q, block_tables, context_lens, cu_seqlens_q, st);
         return (int)hipGetLastError();
     }
     if (mfma_ok) {

@@ -201,6 +201,38 @@ def test_prefill_lds_stage_ends_and_scales(cv, factor):
         o += l
 
 
+@pytest.mark.parametrize("form,H,Hkv,lens,cached", [
+    (11, 8, 2, [1, 17, 64], [63, 3, 0]),                              # one stage of keys, full tables
+    (12, 5, 1, [15, 16, 17, 33, 1], [49, 113, 128, 640, 255]),        # two groups of waves: 1, 2, 3, 11 and 4 stages, queries that see nothing of the second group's
+    (12, 4, 4, [900, 70], [0, 130]),                                  # long prompts on up to two workgroups a CU
+    (11, 32, 8, [130] * 3 + [129, 1], [0, 62, 63, 64, 0]),
+    (22, 12, 4, [2000, 65], [0, 1]),
+    (21, 32, 8, [65] * 26, [0, 63] * 13)])
+def test_prefill_forms(cv, form, H, Hkv, lens, cached):
+    """the forms of the LDS kernel (queries per workgroup, groups of waves that share the stages out) at the edges of tiles and stages, slots
+    behind the contexts NaN patterns; against softmax in 64 bits.  A bf16 output is within 2^-8 of its value; what goes before it (products
+    in f32, probabilities in two bf16 pieces: 2^-16 of the largest |value| that they weigh) is far below."""
+    dt, D, bs = "bf16", 128, 16
+    rng = np.random.default_rng(form + H)
+    q, k_all, v_all, kc, vc, meta = make_case(rng, lens, cached, H, Hkv, D, bs, dt, False)
+    im = cv.InputMetadata.from_oracle_meta(meta, "cuda", is_prefill=True)
+    from candle_vllm_amd import _lib
+    assert _lib.lib.mi355_internal_prefill_form(H, Hkv, len(lens), max(lens), im.block_tables.shape[1], bs) == form
+    scale = 1.0 / np.sqrt(D)
+    pa = cv.PagedAttention(H, D, scale, Hkv)
+    kcd, vcd = (torch.from_numpy(a.view(np.int16)).cuda().view(TD[dt]) for a in (kc, vc))
+    got = host16(pa.prefill(dev16(np.concatenate(q), dt), None, None, kcd, vcd, im), dt)
+    o = 0
+    for i, l in enumerate(lens):
+        k, v = (torch.from_numpy(a[i].astype(np.float64)).cuda().repeat_interleave(H // Hkv, 1).permute(1, 0, 2) for a in (k_all, v_all))
+        s = torch.from_numpy(q[i].astype(np.float64)).cuda().permute(1, 0, 2) @ k.transpose(1, 2).contiguous() * scale
+        hide = torch.arange(cached[i] + l, device="cuda")[None] > torch.arange(l, device="cuda")[:, None] + cached[i]
+        ref = (torch.softmax(s.masked_fill(hide, float("-inf")), -1) @ v.contiguous()).permute(1, 0, 2).cpu().numpy()
+        bound = 2.0 ** -8 * np.abs(ref) + 2.0 ** -14 * np.abs(v_all[i]).max()
+        assert (np.abs(got[o:o + l] - ref) <= bound).all(), f"seq {i}: {np.abs(got[o:o + l] - ref).max()}"
+        o += l
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("flash", [True, False])
 @pytest.mark.parametrize("H,Hkv,D,bs,window", [(8, 2, 128, 64, 100), (4, 4, 64, 16, 7), (4, 2, 80, 16, 33), (8, 2, 128, 16, 4096)])
