@@ -6,6 +6,7 @@ import numpy as np
 import torch
 
 from ._lib import lib, DenseConfig
+from .model import step_inputs
 from .ops import _check, KV_FLASH, KV_PAGED  # noqa: F401
 
 W_SLOTS = {"wq": 0, "wk": 1, "wv": 2, "wo": 3, "w1": 4, "w2": 5, "w3": 6, "attn_norm": 7, "ffn_norm": 8,
@@ -174,23 +175,14 @@ class DenseLlama:
 
     def forward(self, meta, is_prefill=False, stream=None, sync=True):
         """meta: dict from oracle.ops.prepare_decode / prepare_prompt or BlockEngine.prepare_*  -> logits f32"""
-        dev = "cuda"
         n = len(meta["context_lens"])
         T = len(meta["input_ids"])
-        tok = torch.from_numpy(np.asarray(meta["input_ids"]).astype(np.int64).astype(np.int32)).to(dev)
-        pos = torch.from_numpy(np.asarray(meta["positions"]).astype(np.int64)).to(dev)
-        slots = torch.from_numpy(np.asarray(meta["slot_mapping"]).astype(np.int64)).to(dev)
-        bt = torch.from_numpy(np.asarray(meta["block_tables"]).astype(np.int64).astype(np.int32)).contiguous().to(dev)
-        ctx = torch.from_numpy(np.asarray(meta["context_lens"]).astype(np.int64).astype(np.int32)).to(dev)
-        cu = None
-        if is_prefill:
-            cu = torch.from_numpy(np.asarray(meta["cu_seqlens_q"]).astype(np.int64).astype(np.int32)).to(dev)
+        dev, tok, pos, slots, bt, ctx, cu = step_inputs(meta, is_prefill)
         logits = torch.empty((n, self.logits_width()),
-                             dtype=torch.float32, device=dev)
+                             dtype=torch.float32, device=dev.device)
         st = torch.cuda.current_stream().cuda_stream if stream is None else stream
-        _check(lib.mi355_dense_forward(self.h, tok.data_ptr(), pos.data_ptr(), slots.data_ptr(), bt.data_ptr(),
-                                       ctx.data_ptr(), cu.data_ptr() if cu is not None else None, n, T,
-                                       int(meta.get("max_seqlen_q", 0)), bt.shape[1], int(meta["max_context_len"]),
+        _check(lib.mi355_dense_forward(self.h, tok, pos, slots, bt, ctx, cu, n, T,
+                                       int(meta.get("max_seqlen_q", 0)), np.shape(meta["block_tables"])[1], int(meta["max_context_len"]),
                                        logits.data_ptr(), st), "dense_forward")
         if sync:
             torch.cuda.synchronize()

