@@ -25,6 +25,7 @@
 
 #include "../../include/mi355_vllm.h"
 #include "comm.h"
+#include "prompt_image.h"
 #include "step_inputs.h"
 
 #define HCHECK(expr)                                   \
@@ -110,6 +111,7 @@ struct Model {
     int32_t* moe_ids = nullptr; float* moe_w = nullptr; float* moe_y = nullptr;
     int32_t* p_moe_ids = nullptr; float* p_moe_w = nullptr; float* p_moe_y = nullptr;
     // grouped experts on prompt steps: gathered rows in expert order + the permutation and its inverse
+    Mi355PromptImage p_img;          // prompt steps of up to 1024 tokens: the next product's activation image (qmatmul.hip qpg_sum_image_kernel)
     float* p_moe_xg = nullptr; int32_t* p_moe_perm = nullptr; int32_t* p_moe_inv = nullptr;
     int32_t* p_moe_tab = nullptr;    // block table of the device-grouped prompt path: {expert, row end} per 64-row block
     // decode steps with many (token, slot) pairs: experts grouped on the device, `g_cap` rows per expert (host_model.cpp run_part)
@@ -151,6 +153,7 @@ extern "C" int mi355_internal_pa_stream_reduce_to_image(void* out, const float* 
                                                         int64_t stream);                                                     // qmatmul.hip
 extern "C" int32_t mi355_internal_pa_plan(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_context_len,
                                           int32_t kv8, int32_t slots, int32_t* partition_size);   // paged_attention.hip
+extern "C" int mi355_internal_qmatmul_prompt(const mi355_qmm_desc* d, Mi355PromptImage* io, int64_t stream);   // qmatmul.hip
 int g_host_ps_override = 0;     // experiments: mi355_set_tuning(5, partition_size)
 // MI355_MOE_PROMPT_DEVICE=0: prompt steps of a mixture-of-experts model sort their (token, slot) pairs on the host again (rounds 2-5; A/B runs)
 static const int g_moe_prompt_device = []() { const char* e = getenv("MI355_MOE_PROMPT_DEVICE"); return e && e[0] == '0' ? 0 : 1; }();
@@ -289,6 +292,10 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
     const bool lead = c.tp_rank == 0;                              // the rank that carries the residual into the sum
     mi355_qmm_desc d;
     memset(&d, 0, sizeof(d));
+    // a prompt step's products hand the next one its activation image where nothing comes between them
+    const bool hand_on = in.is_prefill && m->p_img.buf && !m->use_comm && c.n_expert <= 1 && part != PART_HEAD;
+    auto product = [&](mi355_qmm_desc& p) { return hand_on ? mi355_internal_qmatmul_prompt(&p, &m->p_img, st) : mi355_qmatmul_fused(&p, st); };
+    if (part == PART_EMBED) { m->p_img.valid = false; m->p_img.eps = c.rms_eps; }
     if (part == PART_EMBED) return mi355_embedding_f32(in.xs, m->tok_embd, in.tokens, B, hid, st);
     if (part == PART_HEAD) {
         // --- output_norm + lm_head -> logits f32       (quantized_llama.rs:500-505; vocab-parallel under TP)
@@ -491,7 +498,7 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
     if (part == PART_QKV) {
         // --- attention_norm + wq|wk|wv + interleaved RoPE + bf16 cast + cache scatter
         dense_desc(m, l, PART_QKV, in, logits, d);
-        return mi355_qmatmul_fused(&d, st);
+        return product(d);
     }
     if (part == PART_ATTN && c.kv_layout == MI355_KV_PAGED_FP8) {
         // `--kvcache-dtype fp8` (is_fp8_keys, attention.rs:896): every key comes back from the e4m3fn cache
@@ -570,13 +577,14 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
         // --- wo(y.to_dtype(F32)) + residual (+ all-reduce)   (attention.rs:1004-1009, quantized_llama.rs:464)
         // --- w2 + residual (+ all-reduce)                     (quantized_llama.rs:37-42, 470)
         dense_desc(m, l, part, in, logits, d);
-        RCHECK(mi355_qmatmul_fused(&d, st));
+        if (hand_on && part == PART_DOWN && l + 1 == c.n_layers) d.chain_next = 0;      // the last tokens' rows follow, in another buffer
+        RCHECK(product(d));
         return all_reduce_xs(m, in.xs, in.tp_y, B, st);
     }
     if (part == PART_GATEUP) {
         // --- ffn_norm + w1|w3 + silu*mul              (quantized_llama.rs:33-37, 468)
         dense_desc(m, l, PART_GATEUP, in, logits, d);
-        return mi355_qmatmul_fused(&d, st);
+        return product(d);
     }
     return (int)hipErrorInvalidValue;
 }
@@ -771,7 +779,7 @@ extern "C" void mi355_llama_destroy(void* mp) {
     }
     free_qw(m->output);
     void* ptrs[] = {m->tok_embd, m->output_norm, m->cos_t, m->sin_t, m->xs, m->q, m->attn, m->h, m->logits,
-                    m->pa_tmp, m->pa_max, m->pa_sum, m->kv_slab, m->logits_local, m->logits_gather, m->tp_y, m->p_tp_y, m->p_moe_xg, m->p_moe_perm, m->p_moe_inv, m->p_moe_tab, m->p_xs, m->p_q, m->p_attn, m->p_h,
+                    m->pa_tmp, m->pa_max, m->pa_sum, m->kv_slab, m->logits_local, m->logits_gather, m->tp_y, m->p_tp_y, m->p_moe_xg, m->p_moe_perm, m->p_moe_inv, m->p_moe_tab, m->p_img.buf, m->p_xs, m->p_q, m->p_attn, m->p_h,
                     m->moe_ids, m->moe_w, m->moe_y, m->p_moe_ids, m->p_moe_w, m->p_moe_y, m->chain_sync, m->g_moe_xg, m->g_moe_h, m->g_moe_yg, m->g_moe_pos, m->g_moe_cnt};
     m->in.destroy();
     if (m->comm && m->comm_owned) mi355_comm_destroy(m->comm);
@@ -908,9 +916,10 @@ extern "C" int64_t mi355_llama_kv_bytes_per_tensor(void* mp) {
 
 static int ensure_prefill_cap(Model* m, int T) {
     if (T <= m->p_cap) return 0;
-    void* old[] = {m->p_xs, m->p_q, m->p_attn, m->p_h, m->p_tp_y};
+    void* old[] = {m->p_xs, m->p_q, m->p_attn, m->p_h, m->p_tp_y, m->p_img.buf};
     HCHECK(hipDeviceSynchronize());
     for (void* p : old) if (p) (void)hipFree(p);
+    m->p_img = Mi355PromptImage();
     m->p_xs = nullptr; m->p_q = nullptr; m->p_attn = nullptr; m->p_h = nullptr; m->p_tp_y = nullptr; m->p_cap = 0;
     const int H = local_heads(m), D = m->cfg.head_dim;
     const int cap = (T + 255) / 256 * 256;
@@ -922,6 +931,12 @@ static int ensure_prefill_cap(Model* m, int T) {
     const size_t moe_pad = m->cfg.n_expert > 1 ? (size_t)64 * (m->cfg.n_expert + 2) : 0;
     HCHECK(hipMalloc((void**)&m->p_h, ((size_t)cap * KE + moe_pad) * m->cfg.intermediate * 4));
     if (m->use_comm) HCHECK(hipMalloc((void**)&m->p_tp_y, (size_t)cap * m->cfg.hidden * 4));
+    if (!m->use_comm && m->cfg.n_expert <= 1) {
+        // (29 MiB at most for 14336 columns; without it every product builds its own image)
+        const size_t n = Mi355PromptImage::need(std::min(cap, (int)Mi355PromptImage::MAX_ROWS), std::max(m->cfg.hidden, m->cfg.intermediate));
+        if (hipMalloc((void**)&m->p_img.buf, n) == hipSuccess) m->p_img.bytes = n;
+        else { (void)hipGetLastError(); m->p_img.buf = nullptr; }
+    }
     if (m->cfg.n_expert > 1) {
         void* oldm[] = {m->p_moe_ids, m->p_moe_w, m->p_moe_y, m->p_moe_xg, m->p_moe_perm, m->p_moe_inv, m->p_moe_tab};
         for (void* p : oldm) if (p) (void)hipFree(p);

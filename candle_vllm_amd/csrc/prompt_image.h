@@ -1,0 +1,19 @@
+// The activation image of a prompt step's next quantised product, handed from one product to the next by the model that runs them (no look-up by
+// address: the model owns the buffer and passes it to both calls).
+#pragma once
+#include <cstddef>
+#include <cstdint>
+
+struct Mi355PromptImage {
+    uint8_t* buf = nullptr;          // device memory of the owner
+    size_t bytes = 0;
+    bool valid = false;              // an image is there: of `live` rows and K columns, normalised with `norm`, in a layout of `rows` rows
+    int32_t live = 0, rows = 0, K = 0;
+    int32_t half = 0;                // which of two sets of the rows' factors it has: a product reads its own behind its GEMM, where the next image goes over the last
+    const float* norm = nullptr;
+    float eps = 0.f;                 // of every norm that an image is made with (the owner's; a product's descriptor has only its own)
+    bool next = false;               // the call's output is the next call's x: leave its image
+    static constexpr int MAX_ROWS = 1024;
+    // two sets of two floats a row, the f16 image, its sub-block sums
+    static size_t need(size_t rows, size_t k) { return (size_t)MAX_ROWS * 16 + rows * (k * 2 + k / 256 * 32); }
+};

@@ -22,6 +22,7 @@
 //     interleaved RoPE + bf16 cast + paged-cache scatter (K7 + K1).
 #include "common.h"
 #include "scratch.h"
+#include "prompt_image.h"
 #include "../../include/mi355_vllm.h"
 #include <string.h>
 #include <algorithm>
@@ -2057,7 +2058,7 @@ static int qpw_launch(int tile, const QmmArgs& r, const QpgImg& im, int n_slots,
 
 // hand-written prompt-step GEMMs (qmm_prompt_gemm.inc, qmm_prefill.inc); returns hipErrorNotSupported for launches it does not cover (then the
 // caller keeps the library-GEMM path)
-static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
+static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, const bool staged) {
     QmmArgs a = a0;
     a.paired = 0;
     for (int s = 0; s < a.nseg; ++s)
@@ -2130,6 +2131,17 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
     im.row_inv = im.row_scale + Tpad;
     im.Tpad = Tpad;
     im.parts = parts;
+    auto image_at = [](uint8_t* p, int half, int rows, int k) {
+        QpgImg q;
+        q.row_scale = reinterpret_cast<float*>(p) + half * 2 * Mi355PromptImage::MAX_ROWS;
+        q.row_inv = q.row_scale + Mi355PromptImage::MAX_ROWS;
+        q.xa = p + (size_t)Mi355PromptImage::MAX_ROWS * 16; q.sfrag = q.xa + (size_t)k * rows * 2;
+        q.Tpad = rows; q.parts = 1;
+        return q;
+    };
+    // the product before has built the image (qpg_sum_image_kernel), with at least the rows that this product's tiles read
+    const bool have_image = staged && parts == 1 && !a.blk_tab && Tpad <= io->rows;
+    if (have_image) im = image_at(io->buf, io->half, io->rows, K);
     float* C = reinterpret_cast<float*>(base + xa_b + sf_b + 2 * rs_b);
     static Mi355DevOnce attr_done;
     if (!attr_done.done()) {
@@ -2154,7 +2166,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
         attr_done.set();
     }
     if (a.blk_tab && g_tune_qpg != 2) return (int)hipErrorNotSupported;                   // only the LDS-fed kernel reads a block table
-    hipLaunchKernelGGL(qpg_rowprep_kernel, dim3(Tpad), dim3(256), 0, st, a, im);          // row statistics + image, one launch (workgroup = token)
+    if (!have_image) hipLaunchKernelGGL(qpg_rowprep_kernel, dim3(Tpad), dim3(256), 0, st, a, im);          // row statistics + image, one launch (workgroup = token)
     // all segments Q4_K, one activation plane, and an epilogue that is a store / residual add / SiLU * up over two equal segments: the GEMM
     // writes the outputs itself, no C buffer, no epilogue launch (mi355_set_tuning(48, 0) switches that off)
     {
@@ -2283,6 +2295,31 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st) {
         s0 = s1;
     }
     a.norm_w = nullptr;                                     // applied while the image was built
+    if (io && io->next && parts == 1 && !a.bias) {
+        // one launch for the epilogue and the next product's image, where a row of outputs is a row of that product's x
+        const int Kn = a.next_k, rows = T <= 192 ? (T + 63) / 64 * 64 : (T + 255) / 256 * 256;   // whole 64-token blocks, from 193 tokens whole tiles of 256 (qpw_pick may take them)
+        const bool one = a.epi == MI355_EPI_RESID && a.nseg == 1 && a.seg[0].n_rows == Kn && a.seg[0].row0 == 0;
+        const bool two = a.epi == MI355_EPI_SILU_MUL && a.nseg == 2 && a.seg[0].n_rows == Kn && a.seg[1].n_rows == Kn && a.seg[0].n_tiles == a.seg[1].n_tiles;
+        const uintptr_t align = (uintptr_t)a.out | (one ? (uintptr_t)a.resid : 0);
+        if ((one || two) && Kn > 0 && (Kn & 255) == 0 && Kn <= (a.next_norm_w ? 8192 : 16384) && a.ldo == Kn && (align & 15) == 0 && rows <= Mi355PromptImage::MAX_ROWS && Mi355PromptImage::need(rows, Kn) <= io->bytes) {
+            const int half = have_image ? io->half ^ 1 : 0;          // im's factors are read here, and to's image lies over im's
+            const QpgImg to = image_at(io->buf, half, rows, Kn);
+            const size_t row_lds = a.next_norm_w ? (size_t)Kn * 4 : 0;
+            if (one) hipLaunchKernelGGL((qpg_sum_image_kernel<false>), dim3(rows), dim3(512), row_lds, st, a, C, ldp, ks, (const float*)im.row_scale, to, a.next_norm_w, io->eps);
+            else hipLaunchKernelGGL((qpg_sum_image_kernel<true>), dim3(rows), dim3(512), row_lds, st, a, C, ldp, ks, (const float*)im.row_scale, to, a.next_norm_w, io->eps);
+            const hipError_t e = hipGetLastError();
+            if (e == hipSuccess) { io->valid = true; io->live = T; io->rows = rows; io->K = Kn; io->half = half; io->norm = a.next_norm_w; }
+            return (int)e;
+        }
+    }
+    if (a.epi == MI355_EPI_QKV_ROPE_CACHE && !a.bias && a.nseg == 3 && a.D % (a.kv_layout == MI355_KV_PAGED_FP8 ? 16 : 8) == 0 && a.rot % 8 == 0 &&
+        (((uintptr_t)a.q_out | (uintptr_t)a.kcache | (uintptr_t)a.vcache | (uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0) {
+        const int64_t units = (int64_t)T * (a.Hq + 2 * a.Hkv) * (a.D / 8);
+        if (units < (1ll << 31) - 256) {
+            hipLaunchKernelGGL(qpg_qkv_sum_kernel, dim3((uint32_t)((units + 255) / 256)), dim3(256), 0, st, a, C, ldp, ks, (const float*)im.row_scale, (int)units);
+            return (int)hipGetLastError();
+        }
+    }
     hipLaunchKernelGGL(qmm_epilogue_kernel, dim3((ldp + 255) / 256, T), dim3(256), 0, st, a, C, ldp, ks, T, (const float*)nullptr,
                        QmgChainOut{nullptr, nullptr, nullptr, 0, 0, 0, 0}, (const float*)im.row_scale);
     return (int)hipGetLastError();
@@ -2600,7 +2637,9 @@ static bool qmg_wide_one_launch(int B) {
     return B > 8 && B <= 8 * QMW_MAXMT && !g_tune_exact_act && !g_qmm_exact && !(B >= g_tune_qpg_min && g_tune_prefill_gemm);
 }
 
-int mi355_qmm_launch(QmmArgs a, int64_t stream) {
+int mi355_qmm_launch(QmmArgs a, int64_t stream, Mi355PromptImage* io = nullptr) {
+    const bool staged = io && io->valid && io->live == a.B && io->K == a.K && io->norm == a.norm_w && a.x_dtype == MI355_DTYPE_F32 && a.ldx == a.K;
+    if (io) io->valid = false;                                        // taken now or never
     {   // images staged WITHOUT backing activations (fused MoE staging) may only be consumed by the grouped 9..32-token launch they were
         // built for; any other route would read rows nobody wrote.  qw1_launch checks the remaining fields (tile height, k, norm, groups)
         QmgStream& qs0 = qmg_stream(to_stream(stream));
@@ -2692,7 +2731,7 @@ int mi355_qmm_launch(QmmArgs a, int64_t stream) {
         } else
 #endif
         {
-            const int rcq = qpg_launch(a, st);
+            const int rcq = qpg_launch(a, st, io, staged);
             if (rcq != (int)hipErrorNotSupported || a.blk_tab) return rcq;
         }
     }
@@ -2883,6 +2922,16 @@ extern "C" int mi355_qmatmul_fused(const mi355_qmm_desc* d, int64_t stream) {
     const int rc = qmm_args_from_desc(d, a);
     if (rc) return rc;
     return mi355_qmm_launch(a, stream);
+}
+
+/* internal (host_model.cpp): mi355_qmatmul_fused of a prompt step's model, which hands the activation image on in `io`: the call before left it there if
+ * io->valid, and this one leaves the next call's if chain_next is set and its own sums are added up by a launch of their own (io->valid says so) */
+extern "C" int mi355_internal_qmatmul_prompt(const mi355_qmm_desc* d, Mi355PromptImage* io, int64_t stream) {
+    QmmArgs a{};
+    const int rc = qmm_args_from_desc(d, a);
+    if (rc) { io->valid = false; return rc; }
+    io->next = d->chain_next != 0;
+    return mi355_qmm_launch(a, stream, io);
 }
 
 #ifdef MI355_QMM_PROBES

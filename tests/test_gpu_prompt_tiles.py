@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import candle_vllm_amd.ops as cv
+from candle_vllm_amd.model import KV_PAGED_FP8
 from oracle import kquants as kq
 
 pytestmark = pytest.mark.gpu
@@ -281,3 +282,101 @@ def test_ranges_of_k_without_room():
                 cv.lib.mi355_internal_scratch_limit(-1)
             assert close(got, want) < TOL
             assert close(m.forward(x), want) < TOL and last_split() > 1
+
+
+class PromptImage(ctypes.Structure):
+    """csrc/prompt_image.h"""
+    _fields_ = [("buf", ctypes.c_void_p), ("bytes", ctypes.c_size_t), ("valid", ctypes.c_bool), ("live", ctypes.c_int32), ("rows", ctypes.c_int32),
+                ("K", ctypes.c_int32), ("half", ctypes.c_int32), ("norm", ctypes.c_void_p), ("eps", ctypes.c_float), ("next", ctypes.c_bool)]
+
+
+@pytest.mark.parametrize("T,hid,inter,kinds,staged", [(40, 2048, 8192, (Q4, Q4, Q4), 2), (65, 3072, 8192, (Q6, Q4, Q6), 2), (193, 2048, 4096, (Q4, Q4, Q6), 2),
+                                                      (34, 1024, 16640, (Q4, Q4, Q4), 1)])
+def test_image_handed_on(T, hid, inter, kinds, staged):
+    """wo (residual) -> gate/up -> down as a prompt step runs them, the image handed on (after wo, and after gate/up up to 16384 columns) against every
+    product building its own: the same bits (the sums, also that of the squares, have the same order)"""
+    rng = np.random.default_rng(T)
+    shapes = ((hid, hid, kinds[0]), (inter, hid, kinds[1]), (inter, hid, kinds[1]), (hid, inter, kinds[2]))
+    ms = [cv.QMatMul(blocks(rng, n, k, t, odd=False), t, "cuda") for n, k, t in shapes]
+    attn = torch.from_numpy(rng.normal(0, 1, (T, hid)).astype(np.float32)).cuda().bfloat16()
+    start = torch.from_numpy(rng.normal(0, 1, (T, hid)).astype(np.float32)).cuda()
+    norm = 1 + 0.1 * torch.randn(hid, device="cuda")
+    fn = cv.lib.mi355_internal_qmatmul_prompt
+    fn.argtypes, fn.restype = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64], ctypes.c_int
+    room = 16384 + (T + 255) // 256 * 256 * (inter * 2 + inter // 256 * 32)
+    buf = torch.full((room,), 255, dtype=torch.uint8, device="cuda")              # NaN patterns: what is read has been written
+    results = []
+    for hand_on in (False, True):
+        xs, h = start.clone(), torch.empty(T, inter, device="cuda")
+        io = PromptImage(buf.data_ptr(), room, eps=0.3)                          # (an eps that shows)
+        seen = []
+        for x, ws, nw, epi, out in ((attn, ms[:1], None, cv.EPI_RESID, xs), (xs, ms[1:3], norm, cv.EPI_SILU_MUL, h), (h, ms[3:], None, cv.EPI_RESID, xs)):
+            d = _desc(x, ws, nw, epi, out)
+            d.chain_next, d.chain_next_k = int(hand_on and x is not h), out.shape[1]
+            d.chain_next_norm = norm.data_ptr() if x is attn else None
+            assert fn(ctypes.byref(d), ctypes.byref(io), torch.cuda.current_stream().cuda_stream) == 0
+            seen.append(bool(io.valid))
+            if x is attn:
+                first = xs.clone()
+        assert seen == [hand_on, hand_on and staged == 2, False]
+        results.append((first, h, xs))
+    torch.cuda.synchronize()
+    (f0, h0, x0), (f1, h1, x1) = results
+    assert torch.isfinite(x0).all() and torch.equal(f0, f1) and torch.equal(h0, h1) and torch.equal(x0, x1)
+
+
+def _desc(x, ws, nw, epi, out):
+    from candle_vllm_amd._lib import QmmDesc
+    d = QmmDesc()
+    d.nseg = len(ws)
+    for i, w in enumerate(ws):
+        d.w_tiles[i], d.ggml_type[i], d.n_rows[i] = w.tiles.data_ptr(), w.ggml_type, w.n
+    d.x, d.x_dtype = x.data_ptr(), cv.DT_F32 if x.dtype == torch.float32 else cv.DT_BF16
+    d.ldx = d.k = x.shape[1]
+    d.num_tokens, d.norm_weight, d.norm_eps = x.shape[0], nw.data_ptr() if nw is not None else None, 0.3 if nw is not None else 0.0
+    d.epilogue, d.out, d.ldo, d.residual = epi, out.data_ptr(), out.shape[1], out.data_ptr() if epi == cv.EPI_RESID else None
+    return d
+
+
+@pytest.mark.parametrize("layout,D,rot,T", [("flash", 128, 64, 65), ("fp8", 128, 128, 40), ("paged", 72, 24, 130), ("fp8", 64, 32, 97), ("paged", 64, 64, 33)])
+def test_qkv_sums_by_eights(layout, D, rot, T):
+    """the launch that adds the ranges up, turns q and k and writes the cache eight columns at a time: every layout, rotated parts that end inside
+    a head, heads that are no whole row tiles' multiple, tokens without a slot; one rounding to bf16 (2^-8), for an e4m3 cache one more (2^-4)"""
+    H, Hkv, K, block = 8, 2, 2048, 16
+    rng = np.random.default_rng(T)
+    heads = (H, Hkv, Hkv)
+    bs = [blocks(rng, n * D, K, Q4, odd=False) for n in heads]
+    ms = [cv.QMatMul(b, Q4, "cuda") for b in bs]
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    pos, slot = torch.from_numpy(rng.integers(0, 500, T)).cuda(), torch.from_numpy(rng.permutation(T + 64)[:T].astype(np.int64)).cuda()
+    slot[::7] = -1
+    ang = torch.arange(500, device="cuda").double()[:, None] * 10000.0 ** (-torch.arange(rot // 2, device="cuda").double() / (rot // 2))
+    nb = (T + 64 + block - 1) // block
+    x16 = 16 if layout == "fp8" else 8
+    dt = torch.uint8 if layout == "fp8" else torch.bfloat16
+    kc = torch.zeros((nb, block, Hkv, D) if layout == "flash" else (nb, Hkv, D // x16, block, x16), dtype=dt, device="cuda")
+    vc = torch.zeros((nb, block, Hkv, D) if layout == "flash" else (nb, Hkv, D, block), dtype=dt, device="cuda")
+    q_out = torch.zeros(T, H * D, dtype=torch.bfloat16, device="cuda")
+    cos, sin = ang.cos().float().contiguous(), ang.sin().float().contiguous()
+    d = _desc(x, ms, None, cv.EPI_QKV_ROPE_CACHE, q_out)
+    d.out, d.ldo = None, 0
+    d.cos_table, d.sin_table, d.positions, d.slot_mapping = (v.data_ptr() for v in (cos, sin, pos, slot))
+    d.q_out, d.key_cache, d.value_cache = q_out.data_ptr(), kc.data_ptr(), vc.data_ptr()
+    d.num_heads, d.num_kv_heads, d.head_dim, d.rotary_dim, d.block_size = H, Hkv, D, rot, block
+    d.kv_layout = {"flash": cv.KV_FLASH, "paged": cv.KV_PAGED, "fp8": KV_PAGED_FP8}[layout]
+    assert cv.lib.mi355_qmatmul_fused(ctypes.byref(d), torch.cuda.current_stream().cuda_stream) == 0
+    assert last_split() > 1
+    y = [product(x, b, Q4).view(T, -1, D) for b in bs]
+    c, s = ang.cos()[pos][:, None], ang.sin()[pos][:, None]
+    turned = [torch.cat([torch.stack([z[..., 0:rot:2] * c - z[..., 1:rot:2] * s, z[..., 0:rot:2] * s + z[..., 1:rot:2] * c], dim=-1).reshape(T, -1, rot), z[..., rot:]], -1) for z in y[:2]]
+    ok = slot >= 0
+    blk, off = slot[ok] // block, slot[ok] % block
+    if layout == "fp8":
+        kc, vc = kc.view(torch.float8_e4m3fn).float(), vc.view(torch.float8_e4m3fn).float()
+        big = max(turned[1].abs().max(), y[2].abs().max()).item()
+        assert big < 448, big                                         # nothing saturates
+    gk = kc[blk, off] if layout == "flash" else kc[blk, :, :, off].reshape(-1, Hkv, D)
+    gv = vc[blk, off] if layout == "flash" else vc[blk, :, :, off]
+    cache_tol = TOL + 2.0 ** -8 + (2.0 ** -4 if layout == "fp8" else 0)
+    for got, want, tol in ((q_out.view(T, H, D), turned[0], TOL + 2.0 ** -8), (gk, turned[1][ok], cache_tol), (gv, y[2][ok], cache_tol)):
+        assert close(got.float(), want) < tol
