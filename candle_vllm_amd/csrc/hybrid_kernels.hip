@@ -2637,7 +2637,10 @@ int mi355_hyb_mingru(void* out, int32_t out_dtype, float* state, int64_t state_s
     if (num_seqs <= 0) return 0;
     GruArgs p{out, state, state_stride, proj, ldp, z_off, x_off, g_off, context_lens, cu_seqlens_q, state_slots, width};
     const dim3 grid((width + 63) / 64, num_seqs);
-    if (num_tokens >= 256) {                            // some portion may be long: segmented scan
+    // The segmented scan, unless the sequences are a few tokens each: the walk takes 0.24 us a token (width 2048, walk / segments, us: 1 x 8 3.9 / 3.4, 1 x 164
+    // 42.2 / 9.1, 2 x 96 26.1 / 6.3, 8 x 24 8.1 / 4.7).  With more workgroups than CUs eight tokens are as quick one by one (16 x 8 4.2 / 4.4, 16 x 12 5.6 / 5.1;
+    // 4096 wide 16 x 12 6.5 / 8.7, 8 x 16 6.8 / 6.3).
+    if (num_tokens >= 256 || num_tokens >= ((int64_t)grid.x * num_seqs <= mi355_num_cus() ? 8 : 16) * (int64_t)num_seqs) {
         // 32 channels per workgroup where 64 leave half of the card idle and the sequences are long, 64 tokens on average.  us, 64 / 32 channels (sequences x tokens, width):
         // 1 x 256, 1024 18.9 / 10.9, 8 x 256, 1024 20.0 / 12.6, 1 x 4096, 4096 277 / 142, 100 x 64, 64 6.5 / 5.1; 32 x 8, 256 4.2 / 5.7, 64 x 16, 4096 33.5 / 45.7.  With more than
         // half of the card at work both take about as long, but for one long sequence among short ones (2000 and 7 x 1 tokens, 2048 133 / 70): 32 from 96 tokens on average in rows of
