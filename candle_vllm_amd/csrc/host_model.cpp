@@ -26,6 +26,7 @@
 #include "../../include/mi355_vllm.h"
 #include "comm.h"
 #include "prompt_image.h"
+#include "scratch.h"
 #include "step_inputs.h"
 
 #define HCHECK(expr)                                   \
@@ -153,6 +154,8 @@ extern "C" int mi355_internal_pa_stream_reduce_to_image(void* out, const float* 
                                                         int64_t stream);                                                     // qmatmul.hip
 extern "C" int32_t mi355_internal_pa_plan(int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_context_len,
                                           int32_t kv8, int32_t slots, int32_t* partition_size);   // paged_attention.hip
+extern "C" int mi355_internal_moe_combine_parts(float* ys, const float* parts, int32_t ks, int32_t rows, int32_t ldp, const float* scale, const float* weights,
+                                                const int32_t* inv, int32_t num_tokens, int32_t hidden, int32_t top_k, int64_t stream);   // moe.hip
 extern "C" int mi355_internal_qmatmul_prompt(const mi355_qmm_desc* d, Mi355PromptImage* io, int64_t stream);   // qmatmul.hip
 int g_host_ps_override = 0;     // experiments: mi355_set_tuning(5, partition_size)
 // MI355_MOE_PROMPT_DEVICE=0: prompt steps of a mixture-of-experts model sort their (token, slot) pairs on the host again (rounds 2-5; A/B runs)
@@ -355,8 +358,14 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
                 dn.x = in.h; dn.x_dtype = MI355_DTYPE_F32; dn.ldx = I; dn.k = I; dn.num_tokens = rows;
                 dn.epilogue = MI355_EPI_STORE; dn.out = in.moe_y; dn.ldo = hid;
                 dn.group_block_table = m->p_moe_tab;
-                RCHECK(mi355_qmatmul_fused(&dn, st));
-                RCHECK(mi355_moe_scatter_combine(in.xs, in.moe_y, in.moe_w, m->p_moe_inv, B, hid, K, st));
+                Mi355ScratchTurn turn(MI355_SCR_QMP_WS, reinterpret_cast<hipStream_t>(st));      // the product's sums lie there until the launch behind it has read them
+                Mi355PromptImage sums;
+                sums.want_parts = true;
+                RCHECK(mi355_internal_qmatmul_prompt(&dn, &sums, st));
+                if (sums.ks > 1)
+                    RCHECK(mi355_internal_moe_combine_parts(in.xs, sums.parts, sums.ks, rows, sums.ldp, sums.scale, in.moe_w, m->p_moe_inv, B, hid, K, st));
+                else
+                    RCHECK(mi355_moe_scatter_combine(in.xs, in.moe_y, in.moe_w, m->p_moe_inv, B, hid, K, st));
                 m->moe_grouped_done = true;
                 return 0;
             }

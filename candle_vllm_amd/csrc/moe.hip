@@ -220,6 +220,37 @@ extern "C" int mi355_moe_gather(float* dst, const float* src, const int32_t* per
     hipLaunchKernelGGL(moe_gather_kernel, dim3((hidden / 4 + 255) / 256, num_pairs), dim3(256), 0, to_stream(stream), dst, src, perm, top_k, hidden);
     return (int)hipGetLastError();
 }
+// the same behind a down product that left sums of ks ranges of K: added in their order, scaled by the row's factor as its epilogue would have, four
+// columns per thread
+__global__ void __launch_bounds__(256) moe_combine_parts_kernel(float* __restrict__ ys, const float* __restrict__ parts, const int ks, const int rows, const int ldp,
+                                                                const float* __restrict__ scale, const float* __restrict__ wts, const int32_t* __restrict__ inv,
+                                                                const int hidden, const int K) {
+    const int t = blockIdx.y, i = (blockIdx.x * 256 + (int)threadIdx.x) * 4;
+    if (i >= hidden) return;
+    float4 acc = *reinterpret_cast<const float4*>(ys + (size_t)t * hidden + i);          // residual (quantized_llama.rs:470)
+    for (int j = 0; j < K; ++j) {
+        const int row = inv[t * K + j];
+        const float w = wts[(size_t)t * K + j], rs = scale[row];
+        const float* p = parts + (size_t)row * ldp + i;
+        float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int z = 0; z < ks; ++z, p += (size_t)rows * ldp) {
+            const float4 v = *reinterpret_cast<const float4*>(p);
+            s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+        }
+        acc.x = fmaf(w, s.x * rs, acc.x); acc.y = fmaf(w, s.y * rs, acc.y); acc.z = fmaf(w, s.z * rs, acc.z); acc.w = fmaf(w, s.w * rs, acc.w);
+    }
+    *reinterpret_cast<float4*>(ys + (size_t)t * hidden + i) = acc;
+}
+/* internal (host_model.cpp) */
+extern "C" int mi355_internal_moe_combine_parts(float* ys, const float* parts, int32_t ks, int32_t rows, int32_t ldp, const float* scale, const float* weights,
+                                                const int32_t* inv, int32_t num_tokens, int32_t hidden, int32_t top_k, int64_t stream) {
+    if (num_tokens <= 0) return 0;
+    if (!ys || !parts || !scale || !weights || !inv || ks < 1 || (hidden & 3) || (ldp & 3) || ldp < hidden) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(moe_combine_parts_kernel, dim3((hidden + 1023) / 1024, num_tokens), dim3(256), 0, to_stream(stream), ys, parts, ks, rows, ldp, scale, weights, inv,
+                       hidden, top_k);
+    return (int)hipGetLastError();
+}
 extern "C" int mi355_moe_scatter_combine(float* ys, const float* y_sorted, const float* weights, const int32_t* inv, int32_t num_tokens,
                                          int32_t hidden, int32_t top_k, int64_t stream) {
     if (num_tokens <= 0) return 0;

@@ -13,6 +13,11 @@ struct Mi355PromptImage {
     const float* norm = nullptr;
     float eps = 0.f;                 // of every norm that an image is made with (the owner's; a product's descriptor has only its own)
     bool next = false;               // the call's output is the next call's x: leave its image
+    // a grouped product of a mixture's down projection (group_block_table): its sums of `ks` ranges of K instead of outputs, where that is quicker (0: outputs)
+    bool want_parts = false;
+    int32_t ks = 0, ldp = 0;
+    const float* parts = nullptr;    // [ks][num_tokens][ldp], in scratch: read by the caller's next launch, in the same turn of (MI355_SCR_QMP_WS, stream)
+    const float* scale = nullptr;    // [num_tokens]
     static constexpr int MAX_ROWS = 1024;
     // two sets of two floats a row, the f16 image, its sub-block sums
     static size_t need(size_t rows, size_t k) { return (size_t)MAX_ROWS * 16 + rows * (k * 2 + k / 256 * 32); }

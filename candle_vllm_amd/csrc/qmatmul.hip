@@ -2100,12 +2100,23 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
         }
         if (ks > 1) pick4 = pick6 = -1;
     }
+    // The down product of a mixture's experts, whose sums the combining launch adds up (moe.hip): 2.6 us a k-block, one range of K after the other on
+    // (blocks x 16) workgroups.  14336 -> 4096, eight experts, two per token, us: 57 tokens 145 -> 88 (three ranges), 115 147 -> 101 (four), 300 238 -> 156,
+    // 994 405 -> 353 (two); 2000 698 -> 663, which the sums' way through memory uses up: up to 4096 rows.
+    const bool to_parts = io && io->want_parts && T <= 4096 && fuse && a.blk_tab && a.nseg == 1 && a.epi == MI355_EPI_STORE && !a.bias && (ldp & 3) == 0 && a.seg[0].n_rows == ldp;
+    if (to_parts) {
+        float best = 0.95f * qpg_tiles_us(a.seg[0].type, T, n_slots, nkb);
+        for (int q = 2; q <= std::min(nkb, 8); ++q) {
+            const float us = qpg_split_us(T, all_q4 ? n_slots : 0, all_q4 ? 0 : n_slots, nkb, q);
+            if (us < best && (size_t)T * ldp * 4 * q <= (size_t)256 << 20) { best = us; ks = q; }
+        }
+    }
     // token rows of the image: whole tiles of whichever kernel reads it
     const int blk64 = parts == 1 ? (T + 63) / 64 : (T + QPG_BM - 1) / QPG_BM * (QPG_BM / 64);   // token blocks of the 64-token kernels
     int Tpad = pick4 == 2 ? std::max((T + 191) / 192 * 192, (T + 255) / 256 * 256)
                : pick4 >= 0 || pick6 >= 0 ? (T + 255) / 256 * 256 : blk64 * 64;
     // (a block-table launch only exists with the epilogue in the store loop: no C buffer -- it would be 1.9 GB for a Mixtral chunk)
-    size_t c_b = a.blk_tab ? 0 : (size_t)T * ldp * 4 * ks;
+    size_t c_b = a.blk_tab && ks == 1 ? 0 : (size_t)T * ldp * 4 * ks;
     size_t xa_b = 0, sf_b = 0, rs_b = 0;
     void* ws = nullptr;
     Mi355ScratchTurn turn(MI355_SCR_QMP_WS, st);            // from the image's launch to its readers'
@@ -2120,7 +2131,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
         rc = room();
     }
     if (rc && T < g_tune_qpg_min) return (int)hipErrorNotSupported;   // the 32-token launches, which need less
-    if (rc && ks > 1) { c_b /= ks; ks = 1; rc = room(); }   // ... and for one set of sums
+    if (rc && ks > 1) { c_b = a.blk_tab ? 0 : c_b / ks; ks = 1; rc = room(); }   // ... and for one set of sums
     if (rc) return rc;
     g_qpg_split_last = ks;
     a.dbg = g_tune_dbg;                                     // ablation bits of the prompt-step GEMM (experiments only)
@@ -2158,6 +2169,8 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
         (void)hipFuncSetAttribute((const void*)qpg_gemm_lds2_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
         (void)hipFuncSetAttribute((const void*)qpg_gemm_lds2_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
         (void)hipFuncSetAttribute((const void*)qpg_gemm_lds2_kernel<true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+        (void)hipFuncSetAttribute((const void*)qpg_gemm_lds2_kernel<false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+        (void)hipFuncSetAttribute((const void*)qpg_gemm_q6k_lds_kernel<false, 2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipFuncSetAttribute((const void*)qpg_gemm_q6k_kernel<2, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
         (void)hipFuncSetAttribute((const void*)qpg_gemm_q6k_lds_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipFuncSetAttribute((const void*)qpg_gemm_q6k_lds_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -2185,6 +2198,15 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
                 hipLaunchKernelGGL((qpg_gemm_kernel<MI355_GGML_Q4_K, 2, 4, 1, 8, false, 1, true>), g_, b_, sh_, st, r, im, C, ldp, n_slots, 0);
 #endif
             }
+            return (int)hipGetLastError();
+        }
+        if (a.blk_tab && ks > 1) {
+            QmmArgs r = a;
+            r.norm_w = nullptr;
+            const dim3 g_(blk64, (n_slots + 15) / 16, ks);
+            if (all_q4) hipLaunchKernelGGL((qpg_gemm_lds2_kernel<false, true>), g_, dim3(512), (size_t)QPG2_BYTES, st, r, im, C, ldp, n_slots, 0);
+            else hipLaunchKernelGGL((qpg_gemm_q6k_lds_kernel<false, 2, true>), g_, dim3(512), (size_t)QPG6_LDS_BYTES, st, r, im, C, ldp, n_slots, 0);
+            io->ks = ks; io->ldp = ldp; io->parts = C; io->scale = im.row_scale;
             return (int)hipGetLastError();
         }
         if (a.blk_tab) {
@@ -2930,6 +2952,7 @@ extern "C" int mi355_internal_qmatmul_prompt(const mi355_qmm_desc* d, Mi355Promp
     QmmArgs a{};
     const int rc = qmm_args_from_desc(d, a);
     if (rc) { io->valid = false; return rc; }
+    io->ks = 0;
     io->next = d->chain_next != 0;
     return mi355_qmm_launch(a, stream, io);
 }

@@ -287,7 +287,8 @@ def test_ranges_of_k_without_room():
 class PromptImage(ctypes.Structure):
     """csrc/prompt_image.h"""
     _fields_ = [("buf", ctypes.c_void_p), ("bytes", ctypes.c_size_t), ("valid", ctypes.c_bool), ("live", ctypes.c_int32), ("rows", ctypes.c_int32),
-                ("K", ctypes.c_int32), ("half", ctypes.c_int32), ("norm", ctypes.c_void_p), ("eps", ctypes.c_float), ("next", ctypes.c_bool)]
+                ("K", ctypes.c_int32), ("half", ctypes.c_int32), ("norm", ctypes.c_void_p), ("eps", ctypes.c_float), ("next", ctypes.c_bool), ("want_parts", ctypes.c_bool),
+                ("ks", ctypes.c_int32), ("ldp", ctypes.c_int32), ("parts", ctypes.c_void_p), ("scale", ctypes.c_void_p)]
 
 
 @pytest.mark.parametrize("T,hid,inter,kinds,staged", [(40, 2048, 8192, (Q4, Q4, Q4), 2), (65, 3072, 8192, (Q6, Q4, Q6), 2), (193, 2048, 4096, (Q4, Q4, Q6), 2),
@@ -380,3 +381,53 @@ def test_qkv_sums_by_eights(layout, D, rot, T):
     cache_tol = TOL + 2.0 ** -8 + (2.0 ** -4 if layout == "fp8" else 0)
     for got, want, tol in ((q_out.view(T, H, D), turned[0], TOL + 2.0 ** -8), (gk, turned[1][ok], cache_tol), (gv, y[2][ok], cache_tol)):
         assert close(got.float(), want) < tol
+
+
+@pytest.mark.parametrize("kind,counts", [(Q4, (5, 64, 0, 65)), (Q6, (1, 0, 130, 63)), (Q4, (0, 0, 0, 1))])
+def test_down_of_experts_in_ranges_of_k(kind, counts):
+    """a mixture's down product over its block table, sums of ranges of K and the launch that adds them into the residual: experts without rows, of one row,
+    of whole blocks and of one row more; against dequantised weights in 64 bits, every row of the sums that belongs to a pair"""
+    E, K, hid, top = len(counts), 4096, 512, 2
+    rng = np.random.default_rng(sum(counts))
+    bs = [blocks(rng, hid, K, kind, odd=False) for _ in range(E)]
+    ms = [cv.QMatMul(b, kind, "cuda") for b in bs]
+    slab = torch.cat([m.tiles.view(torch.uint8).reshape(-1) for m in ms])
+    first, table, rows_of = 0, [], []
+    for e, c in enumerate(counts):
+        nb = -(-c // 64)
+        table += [(e, 64 * first + c)] * nb
+        rows_of += [(e, 64 * first + i) for i in range(c)]
+        first += nb
+    table += [(0, 0)] * 3                                             # blocks behind the last expert's: nothing to do
+    T = 64 * len(table)
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    out = torch.empty(T, hid, device="cuda")
+    tab = torch.tensor(table, dtype=torch.int32, device="cuda")
+    d = _desc(x, ms[:1], None, cv.EPI_STORE, out)
+    d.w_tiles[0], d.moe_expert_stride[0], d.group_block_table = slab.data_ptr(), slab.numel() // E, tab.data_ptr()
+    fn = cv.lib.mi355_internal_qmatmul_prompt
+    fn.argtypes, fn.restype = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64], ctypes.c_int
+    st = torch.cuda.current_stream().cuda_stream
+    io = PromptImage(want_parts=True)
+    assert fn(ctypes.byref(d), ctypes.byref(io), st) == 0 and io.ks > 1
+    order = rng.permutation(len(rows_of))
+    pairs = (len(rows_of) // top) * top
+    toks = max(1, pairs // top)
+    picked = [rows_of[order[i % len(rows_of)]] for i in range(toks * top)]
+    inv = torch.tensor([r for _, r in picked], dtype=torch.int32, device="cuda")
+    w = torch.from_numpy(rng.uniform(0.1, 1, toks * top).astype(np.float32)).cuda()
+    ys0 = torch.from_numpy(rng.normal(0, 1, (toks, hid)).astype(np.float32)).cuda()
+    ys = ys0.clone()
+    comb = cv.lib.mi355_internal_moe_combine_parts
+    vp, i32 = ctypes.c_void_p, ctypes.c_int32
+    comb.argtypes, comb.restype = [vp, vp, i32, i32, i32, vp, vp, vp, i32, i32, i32, ctypes.c_int64], ctypes.c_int
+    assert comb(ys.data_ptr(), io.parts, io.ks, T, io.ldp, io.scale, w.data_ptr(), inv.data_ptr(), toks, hid, top, st) == 0
+    want = ys0.double()
+    for p, (e, r) in enumerate(picked):
+        want[p // top] += w[p].double() * product(x[r:r + 1], bs[e], kind)[0]
+    assert close(ys, want) < TOL
+    d2 = _desc(x, ms[:1], None, cv.EPI_STORE, out)                    # the call without the wish: outputs, as before
+    d2.w_tiles[0], d2.moe_expert_stride[0], d2.group_block_table = d.w_tiles[0], d.moe_expert_stride[0], d.group_block_table
+    assert cv.lib.mi355_qmatmul_fused(ctypes.byref(d2), st) == 0
+    for e, r in picked[:8]:
+        assert close(out[r], product(x[r:r + 1], bs[e], kind)[0]) < 2 * TOL
