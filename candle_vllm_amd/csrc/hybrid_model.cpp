@@ -33,6 +33,9 @@
 extern "C" {
 int mi355_hyb_token_seq(int32_t*, const uint32_t*, int32_t, int64_t);
 int32_t mi355_internal_hyb_parts(int32_t T, int32_t n, int32_t k, int32_t dtype, int32_t most);
+int mi355_internal_hyb_conv_step(float* out, const float* proj, int32_t ldp, int32_t off, const float* w, const float* bias, float* conv_state, int64_t state_stride,
+                                 const uint32_t* context_lens, const uint32_t* cu_seqlens_q, const int32_t* state_slots, const int32_t* tok_seq, int32_t num_seqs,
+                                 int32_t T, int32_t channels, int32_t taps, int32_t act, int64_t stream);   // hybrid_kernels.hip
 int mi355_internal_hyb_linear_parts(float* out, int64_t part, int32_t parts, const void* a, int32_t a_dtype, int32_t lda, const void* w, int32_t T, int32_t n,
                                     int32_t k, int32_t dtype, int64_t stream);
 int mi355_internal_hyb_norm_add_parts(float* x, void* xcopy, const float* y, int32_t ldy, int64_t part, int32_t parts, const float* w, int32_t T, int32_t width,
@@ -926,10 +929,8 @@ static int forward_enqueue(HModel* m, const uint32_t* tokens, const int64_t* pos
         if (L.is_conv_attn()) {
             const int C = L.a_conv_channels(), H = c.a_heads, G = c.a_kv_heads;
             float* conv_state = m->state + L.conv_off;
-            HCHECK(mi355_hyb_conv(m->conv, m->proj, ldp, L.off[P_AQ], f(MI355_HW_A_CONV), conv_state, m->slot_floats, context_lens,
-                                  cu_seqlens_q, state_slots, m->tok_seq, num_seqs, T, C, c.a_conv, 0, stream));
-            HCHECK(mi355_hyb_conv_state_update(conv_state, m->slot_floats, m->proj, ldp, L.off[P_AQ], context_lens, cu_seqlens_q,
-                                               state_slots, num_seqs, C, c.a_conv, stream));
+            HCHECK(mi355_internal_hyb_conv_step(m->conv, m->proj, ldp, L.off[P_AQ], f(MI355_HW_A_CONV), nullptr, conv_state, m->slot_floats, context_lens,
+                                                cu_seqlens_q, state_slots, m->tok_seq, num_seqs, T, C, c.a_conv, 0, stream));
             HCHECK(mi355_hyb_attn_prepare_whole(m->q, L.k_pages, L.v_pages, m->conv, C, 0, H * c.a_dim, (H + G) * c.a_dim,
                                                 c.a_qk_norm ? f(MI355_HW_A_QNORM) : nullptr, c.a_qk_norm ? f(MI355_HW_A_KNORM) : nullptr,
                                                 slot_mapping, T, H, G, c.a_dim, c.a_vdim, c.a_v_unit, eps, dt, stream));
@@ -951,10 +952,8 @@ static int forward_enqueue(HModel* m, const uint32_t* tokens, const int64_t* pos
             // x | B | C through the convolution (bias, silu), the scan over the state slot, then the gate, the group norm and W_o
             const int C = L.ssd_channels();
             float* conv_state = m->state + L.conv_off;
-            HCHECK(mi355_hyb_conv_bias(m->conv, m->proj, ldp, L.off[P_DV], f(MI355_HW_D_CONV), f(MI355_HW_CONV_BIAS), conv_state, m->slot_floats,
-                                       context_lens, cu_seqlens_q, state_slots, m->tok_seq, num_seqs, T, C, c.d_conv, 1, stream));
-            HCHECK(mi355_hyb_conv_state_update(conv_state, m->slot_floats, m->proj, ldp, L.off[P_DV], context_lens, cu_seqlens_q, state_slots,
-                                               num_seqs, C, c.d_conv, stream));
+            HCHECK(mi355_internal_hyb_conv_step(m->conv, m->proj, ldp, L.off[P_DV], f(MI355_HW_D_CONV), f(MI355_HW_CONV_BIAS), conv_state, m->slot_floats, context_lens,
+                                                cu_seqlens_q, state_slots, m->tok_seq, num_seqs, T, C, c.d_conv, 1, stream));
             HCHECK(mi355_hyb_ssd_scan(m->o, m->state + L.state_off, m->slot_floats, m->conv, C, m->proj + L.off[P_A], ldp, f(MI355_HW_D_A_LOG),
                                       f(MI355_HW_D_DT_BIAS), f(MI355_HW_D_SKIP), context_lens, cu_seqlens_q, state_slots, num_seqs, T, c.d_heads,
                                       c.d_kv_heads, c.d_dim, c.d_vdim, stream));
@@ -984,10 +983,8 @@ static int forward_enqueue(HModel* m, const uint32_t* tokens, const int64_t* pos
         if (L.has_delta()) {
             const int C = L.conv_channels();
             float* conv_state = m->state + L.conv_off;
-            HCHECK(mi355_hyb_conv_silu(m->conv, m->proj, ldp, L.off[P_DQ], f(MI355_HW_D_CONV), conv_state, m->slot_floats, context_lens,
-                                       cu_seqlens_q, state_slots, m->tok_seq, num_seqs, T, C, c.d_conv, stream));
-            HCHECK(mi355_hyb_conv_state_update(conv_state, m->slot_floats, m->proj, ldp, L.off[P_DQ], context_lens, cu_seqlens_q,
-                                               state_slots, num_seqs, C, c.d_conv, stream));
+            HCHECK(mi355_internal_hyb_conv_step(m->conv, m->proj, ldp, L.off[P_DQ], f(MI355_HW_D_CONV), nullptr, conv_state, m->slot_floats, context_lens,
+                                                cu_seqlens_q, state_slots, m->tok_seq, num_seqs, T, C, c.d_conv, 1, stream));
             const float* decay_in = m->proj + L.off[P_A];
             int ldd = ldp;
             if (c.d_decay_channels) {

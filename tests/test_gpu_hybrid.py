@@ -391,6 +391,34 @@ def test_conv_silu_portions_and_state(lib, taps):
     assert np.abs(np.concatenate(got_b) - want_b).max() < 5e-6
 
 
+@pytest.mark.parametrize("taps,lens,act,with_bias", [(4, (1,) * 8, 1, False), (4, (0, 1, 3, 0, 1, 0), 1, True), (3, (1, 1), 0, True), (2, (2, 0), 0, False), (4, (5, 1), 1, False),
+                                                     (7, (1, 1, 1), 1, False), (1, (1,), 1, True)])
+def test_conv_and_state_in_one_launch(lib, taps, lens, act, with_bias):
+    """a step's convolution and the move of its state: one launch for decoding batches, also with sequences of no or several tokens, against the two
+    launches, bit for bit, with slots that hold anything (a sequence that starts at 0 must not read it) and nothing written beside them"""
+    _gpu()
+    rng = np.random.default_rng(taps + len(lens))
+    C, off, n, T = 301, 5, len(lens), sum(lens)
+    ldp, stride = C + 9, C * (taps - 1) + 3
+    proj, w, bias = dev(rng.standard_normal((T, ldp))), dev(rng.standard_normal((C, taps))), dev(rng.standard_normal(C))
+    cu, ctx = dev(np.concatenate([[0], np.cumsum(lens)]), np.int32), dev(np.array([k + [0, 1, 2, 40][i % 4] for i, k in enumerate(lens)]), np.int32)
+    slots = dev(rng.permutation(n + 1)[:n], np.int32)
+    ts = torch.zeros(T, dtype=torch.int32, device="cuda")
+    ok(lib.mi355_hyb_token_seq(ts.data_ptr(), cu.data_ptr(), n, _st()))
+    start = dev(rng.standard_normal((n + 1, stride)))
+    b = bias.data_ptr() if with_bias else None
+    want, ws, got, gs = torch.zeros(T, C, device="cuda"), start.clone(), torch.zeros(T, C, device="cuda"), start.clone()
+    ok(lib.mi355_hyb_conv_bias(want.data_ptr(), proj.data_ptr(), ldp, off, w.data_ptr(), b, ws.data_ptr(), stride, ctx.data_ptr(), cu.data_ptr(), slots.data_ptr(),
+                               ts.data_ptr(), n, T, C, taps, act, _st()))
+    ok(lib.mi355_hyb_conv_state_update(ws.data_ptr(), stride, proj.data_ptr(), ldp, off, ctx.data_ptr(), cu.data_ptr(), slots.data_ptr(), n, C, taps, _st()))
+    fn = lib.mi355_internal_hyb_conv_step
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32] + [ctypes.c_void_p] * 3 + [ctypes.c_int64] + [ctypes.c_void_p] * 4 + [ctypes.c_int32] * 5 + [ctypes.c_int64]
+    fn.restype = ctypes.c_int
+    ok(fn(got.data_ptr(), proj.data_ptr(), ldp, off, w.data_ptr(), b, gs.data_ptr(), stride, ctx.data_ptr(), cu.data_ptr(), slots.data_ptr(), ts.data_ptr(), n, T, C, taps,
+          act, _st()))
+    assert torch.isfinite(want).all() and torch.equal(got, want) and torch.equal(gs, ws)
+
+
 @pytest.mark.parametrize("C,T", [(1028, 1021), (12, 87383), (2048, 512), (132, 7944), (64, 49153)])
 @pytest.mark.parametrize("form", ["silu", "residual", "bias", "residual16"])
 def test_conv_rows_of_tokens(lib, C, T, form):
