@@ -1943,7 +1943,7 @@ extern "C" int mi355_internal_pa_stream_reduce_to_image(void* out, const float* 
 }
 
 // ================================================================================================
-// Prompt-step path (num_tokens >= QMP_MIN_TOKENS): the matmul is compute-bound, so it is run as a plain GEMM on the
+// Prompt-step path (num_tokens >= QMP_MIN_TOKENS, mostly from 33 on: mi355_qmm_launch): the matmul is compute-bound, so it is run as a plain GEMM on the
 // matrix cores instead of streaming the quantised weights once per 32 tokens.
 //   1. `qmp_dequant_kernel`  : repacked Q4_K / Q6_K tiles -> bf16 hi + bf16 lo, row-major [N, K] (w = hi + lo to 2^-17)
 //   2. `qmp_xsplit_kernel`   : activations (RMSNorm applied here) -> bf16 hi + lo, row-major [T, K]
@@ -1965,7 +1965,7 @@ extern "C" int mi355_internal_pa_stream_reduce_to_image(void* out, const float* 
 
 static int g_tune_qpg = 2;                                 // mi355_set_tuning(11, v): prompt-step GEMM workgroup tile: 2 (default since round 4) = 64 tokens x 256 rows, 0 = 32 x 512 (rounds 2-3), 1 / 3: A/B variants
 static int g_tune_qpg_fepi = 1;                            // mi355_set_tuning(48, 0): A/B, separate epilogue launch.  Default: the prompt-step GEMM applies the epilogue itself (Q4_K launches; store / residual / SiLU * up; round 4: +7 % on the prompt step)
-static int g_tune_qpg_min = 96;                            // mi355_set_tuning(12, n): fewest tokens that take the prompt-step GEMM (QMP_MIN_TOKENS)
+static int g_tune_qpg_min = 96;                            // mi355_set_tuning(12, n): from how many tokens on the prompt-step GEMM runs whatever the case (below: mi355_qmm_launch's `few`)
 static int g_tune_dbg = 0;                                 // mi355_set_tuning(2, v): probe / ablation modes (experiments only)
 
 #include "qmm_prefill.inc"

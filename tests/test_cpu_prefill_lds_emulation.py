@@ -14,7 +14,7 @@ from oracle import ops as O
 
 LANES = np.arange(64)
 C_, KG = LANES & 15, LANES >> 4
-QT = 2                                              # query tiles of 16 per workgroup (the kernel's PFL_QT)
+QT = 2                                              # query tiles of 16 per workgroup (the kernel's QT)
 
 
 @pytest.fixture(scope="module")
