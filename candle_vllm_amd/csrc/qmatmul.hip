@@ -2953,7 +2953,7 @@ extern "C" int mi355_internal_qmatmul_prompt(const mi355_qmm_desc* d, Mi355Promp
     const int rc = qmm_args_from_desc(d, a);
     if (rc) { io->valid = false; return rc; }
     io->ks = 0;
-    io->next = d->chain_next != 0;
+    io->next = d->chain_next != 0 && g_tune_chain;
     return mi355_qmm_launch(a, stream, io);
 }
 
