@@ -2738,11 +2738,13 @@ int mi355_qmm_launch(QmmArgs a, int64_t stream, Mi355PromptImage* io = nullptr) 
         return qmm_launch_bt<1>(a, R, wt, n_wg, NW, st);
     }
     if (a.blk_tab && !(a.B >= g_tune_qpg_min && g_tune_prefill_gemm == 1)) return (int)hipErrorNotSupported;   // only the prompt GEMM reads a block table
-    // From 33 tokens, where its kernels of one activation plane run, the prompt GEMM with K in ranges is sooner than the 32-token launches one behind the other
-    // (2048 wide, 66 tokens, us a product: q | k | v 34 -> 21, gate/up 46 -> 29, down 40 -> 26), except just above 32 tokens with a Q6_K matrix (33 tokens: 20 and 26)
-    bool q6 = false;
-    for (int s = 0; s < a.nseg; ++s) q6 = q6 || a.seg[s].type == MI355_GGML_Q6_K;
-    const bool few = a.B > (q6 ? 36 : 32) && !g_tune_exact_act && g_tune_qpg == 2 && g_tune_qpg_fepi && !a.rows_dev && g_tune_prefill_gemm == 1;
+    // Up to 95 tokens go in portions of 32.  A last portion of 1 .. 8 has the kernels that keep every activation in two bf16 planes and every weight as it is: these are
+    // often the rows that the caller reads (a prompt's last token), so they stay there.  The tokens in front of it, where they are more than one portion, take the
+    // prompt GEMM with K in ranges, of one f16 plane like the portions of 9 .. 32 and sooner than those one behind the other.  us, portions alone / with it: 41 tokens
+    // 2048 x 2048 25.7 / 17.5, 16384 x 2048 32.6 / 20.2, Q6_K 4096 x 14336 55.6 / 37.8; 65 tokens 29.3 / 21.0, 41.8 / 29.4, 70.0 / 48.5; 72 tokens 32.9 / 21.5, 47.8 / 35.3, 81.1 / 59.6
+    const int tail = a.B < g_tune_qpg_min && a.B % 32 <= 8 ? a.B % 32 : 0, head = a.B - tail;
+    const bool few = head > 32 && !g_tune_exact_act && g_tune_qpg == 2 && g_tune_qpg_fepi && !a.rows_dev && g_tune_prefill_gemm == 1;
+    int b0 = 0;
     if ((a.B >= g_tune_qpg_min && g_tune_prefill_gemm) || few) {
         // prompt step: the hand-written quantised GEMMs (qmm_prompt_gemm.inc, qmm_prefill.inc).  mi355_set_tuning(6, 2) = the first-generation path
         // (bf16 hi/lo weight image + three library GEMMs) for A/B runs; (6, 0) = stream the weights 32 tokens at a time.
@@ -2753,8 +2755,11 @@ int mi355_qmm_launch(QmmArgs a, int64_t stream, Mi355PromptImage* io = nullptr) 
         } else
 #endif
         {
-            const int rcq = qpg_launch(a, st, io, staged);
-            if (rcq != (int)hipErrorNotSupported || a.blk_tab) return rcq;
+            QmmArgs h = a;
+            h.B = head;
+            const int rcq = qpg_launch(h, st, tail ? nullptr : io, staged && !tail);
+            if (a.blk_tab || (rcq ? rcq != (int)hipErrorNotSupported : !tail)) return rcq;
+            if (rcq == 0) b0 = head;
         }
     }
     const int B = a.B;
@@ -2765,7 +2770,7 @@ int mi355_qmm_launch(QmmArgs a, int64_t stream, Mi355PromptImage* io = nullptr) 
     uint16_t* q0 = a.q_out;
     const int64_t* pos0 = a.positions;
     const int64_t* slot0 = a.slot_mapping;
-    for (int b0 = 0; b0 < B;) {
+    while (b0 < B) {
         int bn = B - b0;
         if (bn > 8) {                                         // 9..32 tokens: wide kernel, weights read once
             if (bn > 8 * QMW_MAXMT) bn = 8 * QMW_MAXMT;

@@ -308,7 +308,8 @@ int mi355_moe_scatter_combine(float* ys, const float* y_sorted, const float* wei
  *    3  decode-attention partition merge: low 4 bits 0 = separate reduce launch, 1 = in the last arriver where it pays (default),
  *       2 = always; bits 4.. = partitions per workgroup (0 = chosen per launch, else 1 | 4 | 8 | 16)
  *    5  decode-attention partition size of the step drivers (0 = their own choice: 32, or 64 for the balanced stream)
- *    6  prompt steps (from 33 tokens, 37 with a Q6_K matrix) on the hand-written quantised GEMM (1, default) or streamed like decode batches (0)
+ *    6  prompt steps (from 41 tokens; up to 95, all but the last 1 .. 8 behind whole 32s) on the hand-written quantised GEMM (1, default) or streamed
+ *       like decode batches (0)
  *    9  chained wide launches, and products of a prompt step: an epilogue stages the next mat-mul's activation image (1, default)
  *   24  "exact" activations on the 9..32-token and prompt paths: f16 hi + lo planes instead of one f16 plane (0, default)
  *   30  16-bit / GPTQ linears, bit mask of folded launches switched OFF: 1 the 1..4-token 4-bit kernel, 2 no RMSNorm on the way in,
