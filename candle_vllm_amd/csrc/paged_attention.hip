@@ -915,7 +915,8 @@ __global__ void __launch_bounds__(64 * WPB) paged_attn_mfma_kernel(const PAParam
                 den = fmaf(sm_l[w * G + g], e, den);
                 val = fmaf(sm_o[((size_t)w * G + g) * D + d], e, val);
             }
-            const float outv = (den > 0.f ? val / den : 0.f) * vs;
+            // (ONE: there is a key, so what is not above zero is a NaN score's sum, or no finite score at all, and stays NaN)
+            const float outv = (ONE || den > 0.f ? val / den : 0.f) * vs;
             const int h = hk * G + g;
             if (!ONE && p.max_partitions > 1) {
                 const int64_t pi = ((int64_t)b * p.H + h) * p.max_partitions + pslot;

@@ -89,6 +89,22 @@ def test_short_contexts(H, G, D, bs, most, fp8):
                 assert torch.isfinite(got[i]).all() and (got[i] - want[i]).abs().max() <= 2.0 ** -7 * max(want[i].abs().max().item(), 1e-3), (ps, c)
 
 
+@pytest.mark.parametrize("most", [1, 33, 146, 250, 500])
+def test_scores_that_are_no_numbers(most):
+    """a key that is NaN makes the heads over it NaN, a query that is infinite its own head, and no other"""
+    ctxs = [most, (most + 1) // 2, most]
+    k, v, bt, kv = cache(ctxs, 2, 128, 16, False, most)
+    q = torch.randn(3, 8, 128, device="cuda").bfloat16()
+    k[bt[0].long()[(most - 1) // 16], 0, 3, (most - 1) % 16, 5] = float("nan")
+    q[1, 6, 9] = float("inf")
+    for ps in (0, 32):
+        got, want = attend(q, k, v, bt, ctxs, most, ps, 16, 128 ** -0.5, 0.0, False), reference(q, kv, 128 ** -0.5, 0.0)
+        bad = torch.zeros(3, 8, dtype=torch.bool, device="cuda")
+        bad[0, :4] = bad[1, 6] = True
+        assert got[bad].isnan().all() and torch.isfinite(got[~bad]).all()
+        assert (got[~bad].double() - want[~bad]).abs().max() <= 2.0 ** -7 * want[~bad].abs().max()
+
+
 def test_probabilities_keep_more_than_bf16():
     """against 64 bits the result is off by its own rounding to bf16 (2-norm 2^-9 / sqrt(3) to 2^-8 / sqrt(3)... measured 1.6e-3) and no more"""
     k, v, bt, kv = cache([256, 200, 130, 512], 8, 128, 64, False, 1)
