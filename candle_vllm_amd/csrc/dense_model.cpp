@@ -569,8 +569,8 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
             } else {
                 int ps = choose_partition(T, Hkv, max_context_len);
                 if (ps > 0) ps = 32;   // MFMA kernel: 32-token partitions, 4 per workgroup (measured at batch 32: 32 -> 4937, 64 -> 4784, 128 -> ~4500 tok/s)
-                const int cap = ps > 0 ? mi355_internal_pa_plan(T, H, Hkv, D, c.block_size, max_context_len, 1, m->pa_cap_partitions, &ps) : max_context_len;   // as the GGUF driver
-                if (ps > 0 && mi355_host_get_partition_override() > 0) ps = mi355_host_get_partition_override();
+                int cap = ps > 0 ? mi355_internal_pa_plan(T, H, Hkv, D, c.block_size, max_context_len, 1, m->pa_cap_partitions, &ps) : max_context_len;   // as the GGUF driver
+                if (ps > 0 && mi355_host_get_partition_override() > 0) { ps = mi355_host_get_partition_override(); cap = max_context_len; }
                 if (ps > 0 && (cap + ps - 1) / ps > m->pa_cap_partitions) return (int)hipErrorInvalidValue;
                 DCHECK(mi355_paged_attention_fp8(m->attn, m->pa_sum, m->pa_max, m->pa_tmp, m->q, m->kcache[l], m->vcache[l],
                                                  block_tables, context_lens, T, H, Hkv, D, c.block_size, max_blocks,
@@ -587,9 +587,9 @@ int mi355_dense_forward(void* mp, const uint32_t* tokens, const int64_t* positio
         } else {
             int ps = choose_partition(T, Hkv, max_context_len);
             if (ps > 0 && c.kv_layout == MI355_KV_PAGED) ps = 32;   // MFMA kernel: 32-token partitions, 4 per workgroup (measured at batch 32: 32 -> 4937, 64 -> 4784, 128 -> ~4500 tok/s)
-            const int cap = ps > 0 && c.kv_layout == MI355_KV_PAGED && dt == MI355_DTYPE_BF16
+            int cap = ps > 0 && c.kv_layout == MI355_KV_PAGED && dt == MI355_DTYPE_BF16
                 ? mi355_internal_pa_plan(T, H, Hkv, D, c.block_size, max_context_len, 0, m->pa_cap_partitions, &ps) : max_context_len;   // as the GGUF driver
-            if (ps > 0 && c.kv_layout == MI355_KV_PAGED && mi355_host_get_partition_override() > 0) ps = mi355_host_get_partition_override();   // experiments: mi355_set_tuning(5, n), as the GGUF driver
+            if (ps > 0 && c.kv_layout == MI355_KV_PAGED && mi355_host_get_partition_override() > 0) { ps = mi355_host_get_partition_override(); cap = max_context_len; }   // experiments: mi355_set_tuning(5, n), as the GGUF driver
             if (ps > 0 && (cap + ps - 1) / ps > m->pa_cap_partitions) return (int)hipErrorInvalidValue;
             if (ps == 0)
                 DCHECK(mi355_paged_attention_v1(m->attn, m->q, m->kcache[l], m->vcache[l], block_tables, context_lens, T, H,

@@ -519,8 +519,8 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
         int ps = choose_partition(B, Hkv, in.ctx_cap);
         if (ps > 0) ps = 32;   // MFMA kernel: 32-token partitions, 4 per workgroup (measured at batch 32: 32 -> 4937, 64 -> 4784, 128 -> ~4500 tok/s)
         // >= 64 (sequence, kv head) pairs: the balanced LDS-DMA stream over the e4m3fn cache (round 5), as on the bf16 cache
-        const int cap = ps > 0 ? mi355_internal_pa_plan(B, H, Hkv, D, c.block_size, in.ctx_cap, 1, m->pa_cap_partitions, &ps) : in.ctx_cap;
-        if (g_host_ps_override > 0 && ps > 0) ps = g_host_ps_override;
+        int cap = ps > 0 ? mi355_internal_pa_plan(B, H, Hkv, D, c.block_size, in.ctx_cap, 1, m->pa_cap_partitions, &ps) : in.ctx_cap;
+        if (g_host_ps_override > 0 && ps > 0) { ps = g_host_ps_override; cap = in.ctx_cap; }   // (the plan's bound goes with the plan's size)
         if (ps > 0 && (cap + ps - 1) / ps > m->pa_cap_partitions) return (int)hipErrorInvalidValue;
         if (in.ctx_cap > c.max_seq) return (int)hipErrorInvalidValue;
         if (ps == 64 && B >= 9 && B <= 32 && !(H & 1) && !m->use_comm) {
@@ -555,9 +555,9 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
         int ps = choose_partition(B, Hkv, in.ctx_cap);
         if (ps > 0 && c.kv_layout == MI355_KV_PAGED) ps = 32;   // MFMA kernel: 32-token partitions, 4 per workgroup (measured at batch 32: 32 -> 4937, 64 -> 4784, 128 -> ~4500 tok/s)
         // >= 64 (sequence, kv head) pairs: 64-token stages through the balanced LDS-DMA stream (round 4: 5987 -> 6177 tok/s at batch 32)
-        const int cap = ps > 0 && c.kv_layout == MI355_KV_PAGED
+        int cap = ps > 0 && c.kv_layout == MI355_KV_PAGED
             ? mi355_internal_pa_plan(B, H, Hkv, D, c.block_size, in.ctx_cap, 0, m->pa_cap_partitions, &ps) : in.ctx_cap;
-        if (g_host_ps_override > 0 && ps > 0) ps = g_host_ps_override;
+        if (g_host_ps_override > 0 && ps > 0) { ps = g_host_ps_override; cap = in.ctx_cap; }
         const float scale = 1.0f / sqrtf((float)D);
         if (ps > 0 && (cap + ps - 1) / ps > m->pa_cap_partitions) return (int)hipErrorInvalidValue;
         if (in.ctx_cap > c.max_seq) return (int)hipErrorInvalidValue;

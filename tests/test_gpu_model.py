@@ -562,6 +562,35 @@ def test_batch12_decode_wide_path_chained_equals_unchained_equals_oracle(lib):
     assert [int(r.argmax()) for r in outs[1]] == [int(r.argmax()) for r in ref]
 
 
+@pytest.mark.parametrize("family,fp8,max_seq", [("gguf", False, 1024), ("gguf", True, 2048), ("dense", False, 1024), ("dense", True, 2048)])
+def test_partition_size_that_is_asked_for(lib, family, fp8, max_seq):
+    """mi355_set_tuning(5, n) on a batch that takes the stream by itself, with partial buffers for the model's longest sequence and no more: the step runs in
+    partitions of n over the step's own contexts.  Values as the step's own choice, to the rounding of probabilities and outputs to bf16"""
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible MI355X")
+    from candle_vllm_amd import dense_model as DM, model as M, tuning
+    from oracle import dense_llama as DL
+    B, bs, rng = 12, 64, np.random.default_rng(4)
+    dims = dict(hidden=256, n_layers=1, n_heads=8, n_kv_heads=8, head_dim=128, intermediate=256, vocab=512, rope_theta=10000.0, max_seq=max_seq, block_size=bs)
+    seqs = [{"tokens": [int(t) for t in rng.integers(0, 512, 600 - 40 * i)], "block_table": list(range(10 * i, 10 * i + 10))} for i in range(B)]
+    if family == "gguf":
+        gm = M.GGUFLLaMa(llama.LlamaConfig(**dims), max_batch=B, kv_layout=M.KV_PAGED_FP8 if fp8 else M.KV_PAGED)
+        gm.load_synthetic()
+        step = gm.forward_decode
+    else:
+        gm = DM.DenseLlama(DL.DenseConfig(**dims, kv_fp8=fp8), max_batch=B, kv_layout=M.KV_PAGED)
+        gm.load_oracle_weights(DL.make_weights(gm.cfg))
+        step = gm.forward
+    gm.alloc_kv_cache(10 * B)
+    prompt = O.prepare_prompt([dict(s, tokens=s["tokens"][:-1]) for s in seqs], bs)
+    gm.forward_prefill(prompt) if family == "gguf" else gm.forward(prompt, is_prefill=True)
+    meta = O.prepare_decode(seqs, bs)
+    own = step(meta).cpu().numpy()
+    for n in (32, 128):
+        with tuning(5, n):
+            assert _rel(step(meta).cpu().numpy(), own) < 2e-2
+
+
 def test_llama3_rope_scaling_tables_through_the_model(lib):
     """Llama-3.1-style rope_scaling: the host builds the scaled tables (mi355_rope_tables), the model swaps them in;
     decode logits must match the oracle run with the numpy restatement of the same tables -- and differ from the
