@@ -107,7 +107,7 @@ struct HModel {
     int num_blocks = 0;
     // activations (grow-only)
     int cap_t = 0, cap_out = 0;
-    size_t y_rows = 0;               // rows that `y` holds
+    bool y_one = false;              // `y` has no room for a product's sums in several ranges of K
     float *prep = nullptr, *x = nullptr, *proj = nullptr, *aux1 = nullptr, *aux2 = nullptr, *conv = nullptr, *o = nullptr, *y = nullptr, *gu = nullptr;
     void *xcopy = nullptr, *q = nullptr, *mix = nullptr, *act = nullptr, *xn = nullptr, *att = nullptr;
     int32_t* tok_seq = nullptr;
@@ -395,6 +395,11 @@ template <typename T> int grow(T*& p, size_t bytes) {
     return 0;
 }
 
+// Ranges of K that a residual product of T rows may take: 8, and RANGE_ROWS rows in all.  Of the step's own size and nothing else: what a step adds up, and in which order,
+// is not for the steps before it to say.
+constexpr int RANGE_ROWS = 4096;
+int most_ranges(const HModel* m, int T) { return m->y_one ? 1 : std::min(8, std::max(1, RANGE_ROWS / T)); }
+
 int ensure_capacity(HModel* m, int T, int n_out, int n_seqs) {
     int64_t pieces = 0;
     for (const HLayer& L : m->layers)
@@ -423,9 +428,9 @@ int ensure_capacity(HModel* m, int T, int n_out, int n_seqs) {
         HCHECK(grow(m->conv, t * (size_t)m->max_conv * 4));
         HCHECK(grow(m->o, t * (size_t)m->max_o * 4));
         HCHECK(grow(m->prep, t * (size_t)m->max_prep * 4));
-        // (room for a product's sums in several ranges of K: up to 8, and 4096 rows in all; one set of rows where the card has no more)
-        m->y_rows = std::max<size_t>(t, std::min<size_t>(8 * t, 4096));
-        if (grow(m->y, m->y_rows * W * 4)) { (void)hipGetLastError(); m->y_rows = t; HCHECK(grow(m->y, t * W * 4)); }
+        // (room for the sums of any step of up to t rows, most_ranges sets of them; where the card has no more, one set, and from then on for this model)
+        if (!m->y_one && grow(m->y, std::max<size_t>(t, std::min<size_t>(8 * t, RANGE_ROWS)) * W * 4)) { (void)hipGetLastError(); m->y_one = true; }
+        if (m->y_one) HCHECK(grow(m->y, t * W * 4));
         HCHECK(grow(m->gu, t * (size_t)m->max_ff * 2 * 4));
         HCHECK(grow(m->xcopy, t * W * 2));
         HCHECK(grow(m->q, t * (size_t)m->max_q * m->esize()));
@@ -1012,7 +1017,7 @@ static int forward_enqueue(HModel* m, const uint32_t* tokens, const int64_t* pos
         int parts = 1;
         const bool by_parts = !pair && !copies && !parallel && m->cfg.residual_form != 1 && W <= 4096 && W % 16 == 0;
         auto residual_product = [&](const void* a, int k, const void* w) -> int {
-            parts = by_parts ? mi355_internal_hyb_parts(T, W, k, dt, (int)std::min<size_t>(m->y_rows / (size_t)T, 8)) : 1;
+            parts = by_parts ? mi355_internal_hyb_parts(T, W, k, dt, most_ranges(m, T)) : 1;
             if (parts == 1) return mi355_hyb_linear(m->y, W, a, dt, k, w, nullptr, T, W, k, dt, stream);
             return mi355_internal_hyb_linear_parts(m->y, TW, parts, a, dt, k, w, T, W, k, dt, stream);
         };

@@ -1028,6 +1028,23 @@ def test_graph_replays_equal_eager_steps(lib):
     assert cap >= 1 and rep >= 15
 
 
+def test_a_step_has_the_same_bits_after_a_larger_one(lib):
+    """the number of ranges of K of a residual product is a matter of the step's size: 2100 tokens before and behind a step of 4200"""
+    _gpu()
+    from candle_vllm_amd.step_engine import StepEngine
+    cfg = {"architecture": "Sogodra", "layers": [{"type": "mingru", "mixer": {"width": 1024}, "mlp": {"ff": 4096, "kind": "dense", "limit": 1.25}}],
+           "norm": {"eps": 1e-5}, "vocab": 97, "width": 1024}
+    m, _ = build(cfg, "bfloat16", seed=5)
+    toks = np.random.default_rng(6).integers(0, cfg["vocab"], 4200).tolist()
+    eng = StepEngine(m, 8192)
+    rows = []
+    for r, n in (("a", 2100), ("b", 4200), ("c", 2100), ("d", 300), ("e", 2100)):
+        eng.feed(r, toks[:n])
+        rows.append(eng.step([r], [list(range(n))]).cpu().numpy())
+        eng.finish(r)
+    assert np.array_equal(rows[0], rows[2]) and np.array_equal(rows[0], rows[4])
+
+
 @pytest.mark.parametrize("chunk", [0, 7])
 def test_greedy_generation_through_scheduler(lib, chunk):
     """run_engine + the C++ scheduler (continuous batching, staggered arrivals, chunked prefill): every request generates exactly the
