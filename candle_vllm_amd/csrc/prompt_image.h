@@ -1,5 +1,5 @@
 // The activation image of a prompt step's next quantised product, handed from one product to the next by the model that runs them (no look-up by
-// address: the model owns the buffer and passes it to both calls).
+// address: the model owns the buffer and passes it to both calls; whether the second call's x is what the image was made of is checked).
 #pragma once
 #include <cstddef>
 #include <cstdint>
@@ -7,10 +7,11 @@
 struct Mi355PromptImage {
     uint8_t* buf = nullptr;          // device memory of the owner
     size_t bytes = 0;
-    bool valid = false;              // an image is there: of `live` rows and K columns, normalised with `norm`, in a layout of `rows` rows
+    bool valid = false;              // an image is there: of x, `live` rows and K columns, normalised with `norm`, in a layout of `rows` rows
     int32_t live = 0, rows = 0, K = 0;
     int32_t half = 0;                // which of two sets of the rows' factors it has: a product reads its own behind its GEMM, where the next image goes over the last
     const float* norm = nullptr;
+    const void* x = nullptr;         // where the call that left the image wrote its output; taken by the next call or by none
     float eps = 0.f;                 // of every norm that an image is made with (the owner's; a product's descriptor has only its own)
     bool next = false;               // the call's output is the next call's x: leave its image
     // a grouped product of a mixture's down projection (group_block_table): its sums of `ks` ranges of K instead of outputs, where that is quicker (0: outputs)

@@ -2330,7 +2330,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
             if (one) hipLaunchKernelGGL((qpg_sum_image_kernel<false>), dim3(rows), dim3(512), row_lds, st, a, C, ldp, ks, (const float*)im.row_scale, to, a.next_norm_w, io->eps);
             else hipLaunchKernelGGL((qpg_sum_image_kernel<true>), dim3(rows), dim3(512), row_lds, st, a, C, ldp, ks, (const float*)im.row_scale, to, a.next_norm_w, io->eps);
             const hipError_t e = hipGetLastError();
-            if (e == hipSuccess) { io->valid = true; io->live = T; io->rows = rows; io->K = Kn; io->half = half; io->norm = a.next_norm_w; }
+            if (e == hipSuccess) { io->valid = true; io->live = T; io->rows = rows; io->K = Kn; io->half = half; io->norm = a.next_norm_w; io->x = a.out; }
             return (int)e;
         }
     }
@@ -2660,7 +2660,7 @@ static bool qmg_wide_one_launch(int B) {
 }
 
 int mi355_qmm_launch(QmmArgs a, int64_t stream, Mi355PromptImage* io = nullptr) {
-    const bool staged = io && io->valid && io->live == a.B && io->K == a.K && io->norm == a.norm_w && a.x_dtype == MI355_DTYPE_F32 && a.ldx == a.K;
+    const bool staged = io && io->valid && io->x == a.x && io->live == a.B && io->K == a.K && io->norm == a.norm_w && a.x_dtype == MI355_DTYPE_F32 && a.ldx == a.K;
     if (io) io->valid = false;                                        // taken now or never
     {   // images staged WITHOUT backing activations (fused MoE staging) may only be consumed by the grouped 9..32-token launch they were
         // built for; any other route would read rows nobody wrote.  qw1_launch checks the remaining fields (tile height, k, norm, groups)

@@ -317,7 +317,7 @@ def test_ranges_of_k_without_room():
 class PromptImage(ctypes.Structure):
     """csrc/prompt_image.h"""
     _fields_ = [("buf", ctypes.c_void_p), ("bytes", ctypes.c_size_t), ("valid", ctypes.c_bool), ("live", ctypes.c_int32), ("rows", ctypes.c_int32),
-                ("K", ctypes.c_int32), ("half", ctypes.c_int32), ("norm", ctypes.c_void_p), ("eps", ctypes.c_float), ("next", ctypes.c_bool), ("want_parts", ctypes.c_bool),
+                ("K", ctypes.c_int32), ("half", ctypes.c_int32), ("norm", ctypes.c_void_p), ("x", ctypes.c_void_p), ("eps", ctypes.c_float), ("next", ctypes.c_bool), ("want_parts", ctypes.c_bool),
                 ("ks", ctypes.c_int32), ("ldp", ctypes.c_int32), ("parts", ctypes.c_void_p), ("scale", ctypes.c_void_p)]
 
 
@@ -354,6 +354,27 @@ def test_image_handed_on(T, hid, inter, kinds, staged):
     torch.cuda.synchronize()
     (f0, h0, x0), (f1, h1, x1) = results
     assert torch.isfinite(x0).all() and torch.equal(f0, f1) and torch.equal(h0, h1) and torch.equal(x0, x1)
+
+
+def test_image_of_other_values_is_not_taken():
+    """a product whose x is not the output that the image was made of, with the same rows, columns and norm, builds its own"""
+    rng = np.random.default_rng(8)
+    T, K = 73, 2048
+    a, b = (cv.QMatMul(blocks(rng, K, K, Q4, odd=False), Q4, "cuda") for _ in range(2))
+    x, other = (torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda() for _ in range(2))
+    norm = 1 + 0.1 * torch.randn(K, device="cuda")
+    xs, want, got = x.clone(), torch.empty(T, K, device="cuda"), torch.empty(T, K, device="cuda")
+    fn, st = cv.lib.mi355_internal_qmatmul_prompt, torch.cuda.current_stream().cuda_stream
+    fn.argtypes, fn.restype = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64], ctypes.c_int
+    room = 16384 + 256 * (K * 2 + K // 256 * 32)
+    buf = torch.zeros(room, dtype=torch.uint8, device="cuda")
+    io = PromptImage(buf.data_ptr(), room, eps=0.3)
+    d = _desc(x, [a], None, cv.EPI_RESID, xs)
+    d.chain_next, d.chain_next_k, d.chain_next_norm = 1, K, norm.data_ptr()
+    assert fn(ctypes.byref(d), ctypes.byref(io), st) == 0 and io.valid
+    assert fn(ctypes.byref(_desc(other, [b], norm, cv.EPI_STORE, got)), ctypes.byref(io), st) == 0 and not io.valid
+    assert cv.lib.mi355_qmatmul_fused(ctypes.byref(_desc(other, [b], norm, cv.EPI_STORE, want)), st) == 0
+    assert torch.equal(got, want)
 
 
 def _desc(x, ws, nw, epi, out):
