@@ -1548,7 +1548,7 @@ static int g_tune_ks_minkb = 2;                               // mi355_set_tunin
 static int g_tune_grp_ks_target = 4096;                       // mi355_set_tuning(16, n): the same for grouped launches (slots of all groups)
 static int g_tune_ks_target = 1024;                           // mi355_set_tuning(10, n): split K until a launch has n row-tile x k-split slots
 static int g_tune_wide_fuse = 0;                              // mi355_set_tuning(49, 1), probe builds only: EXPERIMENT, the 9..32-token path runs its split-K epilogue inside the GEMM launches (lost its A/B: qmm_wide1_gemm.inc)
-static inline int qmg_buf(void** p, int key, size_t need, hipStream_t st) { return mi355_scratch_get(p, key, need, st, false); }
+static inline int qmg_buf(void** p, int key, size_t need, hipStream_t st, size_t most = (size_t)-1) { return mi355_scratch_get(p, key, need, st, false, most); }
 
 template <int MT>
 static int qmg_launch(const QmmArgs& a0, hipStream_t st) {
@@ -1994,7 +1994,11 @@ static int qpw_go(const QmmArgs& r, const QpgImg& im, int n_slots, hipStream_t s
 // tile of this thread's last prompt product (tests: which kernel ran)
 static thread_local int g_qpw_last = -1, g_qpg_split_last = 1;
 extern "C" int32_t mi355_internal_last_qpw(void) { return g_qpw_last; }
-extern "C" int32_t mi355_internal_last_qpg_split(void) { return g_qpg_split_last; }   // ranges of K
+extern "C" int32_t mi355_internal_last_qpg_split(void) { return g_qpg_split_last; }   // ranges of K; 0: no launch of these kernels
+// The sums of ranges of K, and the rows of the launches that have any: what bounds their share of the kept workspace.  (4096 rows of 4096 columns are 64 MiB a range;
+// the ranges that are sooner at 8192 columns are 128 .. 252 MiB at 1088 .. 4032 rows)
+constexpr size_t QPG_PART_BYTES = (size_t)256 << 20;
+constexpr int QPG_PART_ROWS = 1024, QPG_PART_ROWS_TAB = 4096;
 // Which kernel makes a prompt product: us per k-block and round of workgroups (one per CU; the 64 x 256 tile of qmm_prefill.inc: two), a full round and
 // one that leaves most of the chip idle (it runs at a higher clock).  Both sides measured at 19 sizes of 96 .. 4096 tokens for 14 matrices of 1024 x 4096 ..
 // 28672 x 4096: with the choice 1.09 x as fast on average as with 64 x 256 tiles alone (Q4_K up to 1.34 x, Q6_K 1.92 x); 270 drawn products and 190 q | k | v of
@@ -2091,24 +2095,24 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
     }
     if (T < g_tune_qpg_min && !a.blk_tab && whole_us == 0.f) return (int)hipErrorNotSupported;
     int ks = 1;
-    if (fuse && !a.blk_tab && whole_us > 0.f && T <= 1024) {
+    if (fuse && !a.blk_tab && whole_us > 0.f && T <= QPG_PART_ROWS) {
         const int s6 = one_q6 ? n_slots : v_slots;
         float best = 0.95f * whole_us;
         for (int q = 2; q <= std::min(nkb, 16); ++q) {
             const float us = qpg_split_us(T, n_slots - s6, s6, nkb, q);
-            if (us < best) { best = us; ks = q; }
+            if (us < best && (size_t)T * ldp * 4 * q <= QPG_PART_BYTES) { best = us; ks = q; }
         }
         if (ks > 1) pick4 = pick6 = -1;
     }
     // The down product of a mixture's experts, whose sums the combining launch adds up (moe.hip): 2.6 us a k-block, one range of K after the other on
     // (blocks x 16) workgroups.  14336 -> 4096, eight experts, two per token, us: 57 tokens 145 -> 88 (three ranges), 115 147 -> 101 (four), 300 238 -> 156,
     // 994 405 -> 353 (two); 2000 698 -> 663, which the sums' way through memory uses up: up to 4096 rows.
-    const bool to_parts = io && io->want_parts && T <= 4096 && fuse && a.blk_tab && a.nseg == 1 && a.epi == MI355_EPI_STORE && !a.bias && (ldp & 3) == 0 && a.seg[0].n_rows == ldp;
+    const bool to_parts = io && io->want_parts && T <= QPG_PART_ROWS_TAB && fuse && a.blk_tab && a.nseg == 1 && a.epi == MI355_EPI_STORE && !a.bias && (ldp & 3) == 0 && a.seg[0].n_rows == ldp;
     if (to_parts) {
         float best = 0.95f * qpg_tiles_us(a.seg[0].type, T, n_slots, nkb);
         for (int q = 2; q <= std::min(nkb, 8); ++q) {
             const float us = qpg_split_us(T, all_q4 ? n_slots : 0, all_q4 ? 0 : n_slots, nkb, q);
-            if (us < best && (size_t)T * ldp * 4 * q <= (size_t)256 << 20) { best = us; ks = q; }
+            if (us < best && (size_t)T * ldp * 4 * q <= QPG_PART_BYTES) { best = us; ks = q; }
         }
     }
     // token rows of the image: whole tiles of whichever kernel reads it
@@ -2122,7 +2126,10 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
     Mi355ScratchTurn turn(MI355_SCR_QMP_WS, st);            // from the image's launch to its readers'
     auto room = [&]() {
         xa_b = (size_t)K * Tpad * 2 * parts; sf_b = (size_t)nkb * Tpad * 32; rs_b = (size_t)Tpad * 4;
-        return qmg_buf(&ws, MI355_SCR_QMP_WS, xa_b + sf_b + 2 * rs_b + c_b + 4096, st);
+        // (a buffer that grows for sums of ranges is doubled to the most that any launch of this K has for them, and no further)
+        const size_t most_rows = a.blk_tab ? QPG_PART_ROWS_TAB : QPG_PART_ROWS;
+        const size_t most = ks > 1 ? most_rows * ((size_t)K * 2 + nkb * 32 + 8) + QPG_PART_BYTES + 4096 : (size_t)-1;
+        return qmg_buf(&ws, MI355_SCR_QMP_WS, xa_b + sf_b + 2 * rs_b + c_b + 4096, st, most);
     };
     int rc = room();
     if (rc && Tpad > blk64 * 64) {                          // a full card, or a capture and a buffer that has room for the 64-token kernels' rows only
@@ -2662,6 +2669,7 @@ static bool qmg_wide_one_launch(int B) {
 int mi355_qmm_launch(QmmArgs a, int64_t stream, Mi355PromptImage* io = nullptr) {
     const bool staged = io && io->valid && io->x == a.x && io->live == a.B && io->K == a.K && io->norm == a.norm_w && a.x_dtype == MI355_DTYPE_F32 && a.ldx == a.K;
     if (io) io->valid = false;                                        // taken now or never
+    g_qpg_split_last = 0;
     {   // images staged WITHOUT backing activations (fused MoE staging) may only be consumed by the grouped 9..32-token launch they were
         // built for; any other route would read rows nobody wrote.  qw1_launch checks the remaining fields (tile height, k, norm, groups)
         QmgStream& qs0 = qmg_stream(to_stream(stream));

@@ -299,7 +299,7 @@ def test_ranges_of_k_without_room():
     b = blocks(rng, N, K, Q4)
     m = cv.QMatMul(b, Q4, "cuda")
     cv.lib.mi355_internal_scratch_limit.argtypes = [ctypes.c_int64]
-    for T, splits in ((200, 1), (80, None)):
+    for T, splits in ((200, 1), (80, 0)):
         x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
         want = product(x, b, Q4)
         torch.cuda.synchronize()
@@ -307,11 +307,36 @@ def test_ranges_of_k_without_room():
             cv.lib.mi355_internal_scratch_limit(4200000)                  # 200 tokens: image 2.2 MB, sums of a range 1.6 MB
             try:
                 got = m.forward(x)
-                assert splits is None or last_split() == splits
+                assert last_split() == splits
             finally:
                 cv.lib.mi355_internal_scratch_limit(-1)
             assert close(got, want) < TOL
             assert close(m.forward(x), want) < TOL and last_split() > 1
+
+
+def test_sums_of_ranges_are_bounded():
+    """256 MiB of sums at most, and a workspace that grows for them is not doubled beyond those and the image of 1024 tokens"""
+    from candle_vllm_amd.model import random_tiles
+    K, MiB = 14336, 1 << 20
+    tiles = random_tiles(Q4, 57344, K, "cuda", torch.Generator(device="cuda").manual_seed(1))
+    x, out = torch.randn(809, K, device="cuda"), torch.empty(809, 57344, device="cuda")
+
+    def run(tokens, rows):
+        d = cv.QmmDesc()
+        d.nseg, d.w_tiles[0], d.ggml_type[0], d.n_rows[0] = 1, tiles.data_ptr(), Q4, rows
+        d.x, d.x_dtype, d.ldx, d.k, d.num_tokens = x.data_ptr(), cv.DT_F32, K, K, tokens
+        d.epilogue, d.out, d.ldo = cv.EPI_STORE, out.data_ptr(), rows
+        assert cv.lib.mi355_qmatmul_fused(d, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return last_split()
+    with torch.cuda.stream(torch.cuda.Stream()):                          # (a workspace of its own)
+        assert run(41, 4096) > 1
+        before = torch.cuda.mem_get_info()[0]
+        ks = run(569, 32768)
+        assert ks > 1 and ks * 569 * 32768 * 4 > 128 * MiB               # twice this launch's bytes would be more than the bound
+        image = 1024 * (K * 2 + K // 256 * 32 + 8)
+        assert before - torch.cuda.mem_get_info()[0] <= image + 256 * MiB + 4 * MiB
+        assert run(809, 57344) == 1                                       # two ranges: 353 MiB
 
 
 class PromptImage(ctypes.Structure):
