@@ -442,11 +442,11 @@ __device__ __forceinline__ float4 frag4(const float* row, int k, int kend, bool 
     return f;
 }
 
-// Few tokens: a stream over the weights, as the bf16 kernel above.  A workgroup owns 16 weight rows (GLU: a gate and an up tile) and 16 MT tokens; its NW
-// waves take 16 UNR columns in turn and add their partial tiles through LDS.  Lane (m16, kg) loads four consecutive k of its row: matrix instruction j
+// Few tokens: a stream over the weights, as the bf16 kernel above.  A workgroup owns 16 weight rows (GLU: a gate and an up tile) and 16 MT tokens; its 16
+// waves take 32 columns in turn and add their partial tiles through LDS.  Lane (m16, kg) loads four consecutive k of its row: matrix instruction j
 // of a step multiplies element j of every lane, so a step is 16 columns in another order on both sides alike.
-template <int NW, int UNR, int MT, int B> __global__ __launch_bounds__(64 * NW) void linear_f32_stream_kernel(LinArgs p) {
-    constexpr int NC = B == LIN_GLU_BUILD ? 2 : 1;
+template <int MT, int B> __global__ __launch_bounds__(1024) void linear_f32_stream_kernel(LinArgs p) {
+    constexpr int NW = 16, UNR = 2, NC = B == LIN_GLU_BUILD ? 2 : 1;
     __shared__ float part[NW][NC * MT * 4][64];
     lin_batch<float, B>(p, blockIdx.x * 16);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m16 = lane & 15, kg = lane >> 4;
@@ -509,13 +509,14 @@ template <int NW, int UNR, int MT, int B> __global__ __launch_bounds__(64 * NW) 
     }
 }
 
-// More tokens: tiles of 64 MF tokens x 64 NF columns, KS groups of four waves that take the 16-wide K slices in turn (KS = 2 where the tiles are few) and
-// add up through LDS at the end.  A slice goes from global memory into registers PF slices ahead, then into one of two LDS buffers (rows of 16 + 4 floats:
+// More tokens: tiles of 64 tokens x 64 columns, KS groups of four waves that take the 16-wide K slices in turn (three where the tiles are few, two else) and
+// add up through LDS at the end.  A slice goes from global memory into registers two slices ahead, then into one of two LDS buffers (rows of 16 + 4 floats:
 // the eight rows that a ds_read_b128 serves at a time start on different banks), from where every wave multiplies its quarter by 32x32x2 instructions --
 // again with four consecutive k per lane, one to an instruction.
-template <int MF, int NF, int KS, int PF, int B> __global__ __launch_bounds__(256 * KS) void linear_f32_gemm_kernel(LinArgs p) {
-    constexpr int BM = 64 * MF, BN = 64 * NF, ROWS = BM + BN, LD = 20, NL = ROWS / 64;   // NL float4 per thread and slice
-    constexpr int TILE = KS * 2 * ROWS * LD, RED = KS > 1 ? (KS - 1) * BM * BN : 1;
+template <int KS, int B> __global__ __launch_bounds__(256 * KS) void linear_f32_gemm_kernel(LinArgs p) {
+    constexpr int BM = 64, BN = 64, ROWS = BM + BN, LD = 20, NL = ROWS / 64, PF = 2;     // NL float4 per thread and slice
+    constexpr int TILE = KS * 2 * ROWS * LD, RED = (KS - 1) * BM * BN;
+    static_assert(KS > 1);
     __shared__ float smem[TILE > RED ? TILE : RED];
     const int tid = threadIdx.x & 255, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, c32 = lane & 31, h = lane >> 5, wm = wave >> 1, wn = wave & 1;
@@ -530,7 +531,7 @@ template <int MF, int NF, int KS, int PF, int B> __global__ __launch_bounds__(25
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
         const int r = (tid >> 2) + 64 * i;
-        if (i < MF) {
+        if (i == 0) {
             ok[i] = t0 + r < p.T;
             src[i] = static_cast<const float*>(p.a) + (size_t)(ok[i] ? lin_row(p, t0 + r) : 0) * p.lda;
         } else {
@@ -542,15 +543,11 @@ template <int MF, int NF, int KS, int PF, int B> __global__ __launch_bounds__(25
     auto fetch = [&](float4 (&to)[NL], int slice) {
         const int k = 16 * slice + kq;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) to[i] = (ok[i] && k < p.K) ? frag4(src[i], k, p.K, i < MF ? p.a_vec : p.w_vec) : float4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < NL; ++i) to[i] = (ok[i] && k < p.K) ? frag4(src[i], k, p.K, i == 0 ? p.a_vec : p.w_vec) : float4{0.f, 0.f, 0.f, 0.f};
     };
-    f32x16_t acc[MF][NF];
+    f32x16_t acc;
 #pragma unroll
-    for (int m = 0; m < MF; ++m)
-#pragma unroll
-        for (int n = 0; n < NF; ++n)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[m][n][v] = 0.f;
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
     const int slices = (p.K + 15) / 16, rounds = (slices + KS - 1) / KS;   // (the last slices of a group past K are zeros)
     float* base = smem + grp * 2 * ROWS * LD;
 #pragma unroll
@@ -566,75 +563,52 @@ template <int MF, int NF, int KS, int PF, int B> __global__ __launch_bounds__(25
                 __syncthreads();
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    float4 a[MF], b[NF];
-#pragma unroll
-                    for (int m = 0; m < MF; ++m) a[m] = *reinterpret_cast<const float4*>(buf + (wm * 32 * MF + 32 * m + c32) * LD + 8 * s + 4 * h);
-#pragma unroll
-                    for (int n = 0; n < NF; ++n) b[n] = *reinterpret_cast<const float4*>(buf + (BM + wn * 32 * NF + 32 * n + c32) * LD + 8 * s + 4 * h);
+                    const float4 a = *reinterpret_cast<const float4*>(buf + (wm * 32 + c32) * LD + 8 * s + 4 * h);
+                    const float4 b = *reinterpret_cast<const float4*>(buf + (BM + wn * 32 + c32) * LD + 8 * s + 4 * h);
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-#pragma unroll
-                        for (int m = 0; m < MF; ++m)
-#pragma unroll
-                            for (int n = 0; n < NF; ++n)
-                                acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(reinterpret_cast<const float*>(&a[m])[j],
-                                                                                 reinterpret_cast<const float*>(&b[n])[j], acc[m][n], 0, 0, 0);
+                        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(reinterpret_cast<const float*>(&a)[j], reinterpret_cast<const float*>(&b)[j], acc, 0, 0, 0);
                 }
             }
         }
     }
-    if (KS > 1) {
-        __syncthreads();                                                   // every wave is done with the slices
-        if (grp)
+    __syncthreads();                                                       // every wave is done with the slices
+    if (grp)
 #pragma unroll
-            for (int m = 0; m < MF; ++m)
+        for (int v = 0; v < 16; ++v) smem[(((grp - 1) * 4 + wave) * 16 + v) * 64 + lane] = acc[v];
+    __syncthreads();
+    if (grp) return;
 #pragma unroll
-                for (int n = 0; n < NF; ++n)
+    for (int g = 0; g < KS - 1; ++g)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) smem[(((grp - 1) * 4 + wave) * MF * NF * 16 + (m * NF + n) * 16 + v) * 64 + lane] = acc[m][n][v];
-        __syncthreads();
-        if (grp) return;
+        for (int v = 0; v < 16; ++v) acc[v] += smem[((g * 4 + wave) * 16 + v) * 64 + lane];
+    const int col = n0 + wn * 32 + c32;
+    const float bias = (B != LIN_GLU_BUILD && p.bias && col < p.N) ? p.bias[col] : 0.f;
 #pragma unroll
-        for (int g = 0; g < KS - 1; ++g)
-#pragma unroll
-            for (int m = 0; m < MF; ++m)
-#pragma unroll
-                for (int n = 0; n < NF; ++n)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[m][n][v] += smem[((g * 4 + wave) * MF * NF * 16 + (m * NF + n) * 16 + v) * 64 + lane];
+    for (int v = 0; v < 16; ++v) {
+        const int t = t0 + wm * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+        if (B == LIN_GLU_BUILD) {                                           // the up column of a gate column is 16 lanes further
+            const float up = __shfl_xor(acc[v], 16);
+            if (!(c32 & 16) && col < p.N && t < p.T) lin_store_glu(p, t, (col & ~31) / 2 + (col & 15), acc[v], up);
+        } else if (col < p.N && t < p.T) lin_store<B>(p, t, col, acc[v] + bias);
     }
-#pragma unroll
-    for (int m = 0; m < MF; ++m)
-#pragma unroll
-        for (int n = 0; n < NF; ++n) {
-            const int col = n0 + wn * 32 * NF + 32 * n + c32;
-            const float bias = (B != LIN_GLU_BUILD && p.bias && col < p.N) ? p.bias[col] : 0.f;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int t = t0 + wm * 32 * MF + 32 * m + 8 * (v >> 2) + 4 * h + (v & 3);
-                if (B == LIN_GLU_BUILD) {                                   // the up column of a gate column is 16 lanes further
-                    const float up = __shfl_xor(acc[m][n][v], 16);
-                    if (!(c32 & 16) && col < p.N && t < p.T) lin_store_glu(p, t, (col & ~31) / 2 + (col & 15), acc[m][n][v], up);
-                } else if (col < p.N && t < p.T) lin_store<B>(p, t, col, acc[m][n][v] + bias);
-            }
-        }
 }
 
 // f32 products by the number of 64 x 64 tiles: under half a card's worth (and up to 32 tokens) the streaming kernel, 16 or 32 tokens to a workgroup; then the
 // tiles, three groups of waves to a tile up to two tiles per unit, two beyond.  us, the FMA kernel that took all of them before / this one / the other side of the line:
 // 2 tokens 2048 x 8192 1290 / 29;  2 tokens 32000 x 2048 396 / 55;  300 tokens x 16384 (gate/up) x 2048 412 / 198;  100 tokens 2048 x 8192 stream 102, tiles 175;
 // 200 tokens 46 and 48 (2048 x 2048);  130 tokens 3072 x 3072 tiles 70, stream 72;  500 tokens 2048 x 8192 three groups 177, two 190;  2048 tokens 9360 x 2048
-// two groups 693 (113 TFLOP/s of 157), three 744, tiles of 128 x 128 692.
+// two groups 693 (113 TFLOP/s of 157), three 744.
 template <int B> static void linear_f32_launch(const LinArgs& p, unsigned nz, hipStream_t st) {
     const int T = p.T, n = p.N, cus = mi355_num_cus();
     const int64_t cols = B == LIN_GLU_BUILD ? n / 32 : (n + 15) / 16, tiles = (int64_t)((n + 63) / 64) * ((T + 63) / 64) * nz;
     if (T <= 32 || 2 * tiles <= cus) {
-        if (T <= 16 || cols * ((T + 31) / 32) * nz < cus) linear_f32_stream_kernel<16, 2, 1, B><<<dim3((unsigned)cols, (T + 15) / 16, nz), 1024, 0, st>>>(p);
-        else linear_f32_stream_kernel<16, 2, 2, B><<<dim3((unsigned)cols, (T + 31) / 32, nz), 1024, 0, st>>>(p);
+        if (T <= 16 || cols * ((T + 31) / 32) * nz < cus) linear_f32_stream_kernel<1, B><<<dim3((unsigned)cols, (T + 15) / 16, nz), 1024, 0, st>>>(p);
+        else linear_f32_stream_kernel<2, B><<<dim3((unsigned)cols, (T + 31) / 32, nz), 1024, 0, st>>>(p);
     } else {
         const dim3 grid((n + 63) / 64, (T + 63) / 64, nz);
-        if (tiles <= 2 * cus) linear_f32_gemm_kernel<1, 1, 3, 2, B><<<grid, 768, 0, st>>>(p);
-        else linear_f32_gemm_kernel<1, 1, 2, 2, B><<<grid, 512, 0, st>>>(p);
+        if (tiles <= 2 * cus) linear_f32_gemm_kernel<3, B><<<grid, 768, 0, st>>>(p);
+        else linear_f32_gemm_kernel<2, B><<<grid, 512, 0, st>>>(p);
     }
 }
 
@@ -2903,7 +2877,7 @@ static int grouped_launch(void* out, int32_t out_dtype, int32_t ldo, const void*
         if (a_dtype != MI355_DTYPE_F32 || block_rows != 64) return -1;
         p.w_vec = (p.ldw % 4 == 0) && ((uintptr_t)w % 16 == 0) && (w_bs % 4 == 0);
         p.a_vec = (lda % 4 == 0) && ((uintptr_t)a % 16 == 0);
-        LIN_EPI2(p, (linear_f32_gemm_kernel<1, 1, 2, 2, EPI><<<dim3((n + 63) / 64, n_blocks, 1), 512, 0, st_>>>(p)));
+        LIN_EPI2(p, (linear_f32_gemm_kernel<2, EPI><<<dim3((n + 63) / 64, n_blocks, 1), 512, 0, st_>>>(p)));
         LAUNCH_OK(); return 0;
     }
     const int a_bytes = a_dtype == MI355_DTYPE_F32 ? 4 : 2;
