@@ -1943,7 +1943,7 @@ extern "C" int mi355_internal_pa_stream_reduce_to_image(void* out, const float* 
 }
 
 // ================================================================================================
-// Prompt-step path (num_tokens >= QMP_MIN_TOKENS, mostly from 33 on: mi355_qmm_launch): the matmul is compute-bound, so it is run as a plain GEMM on the
+// Prompt-step path (num_tokens >= QMP_MIN_TOKENS, mostly from 41 on: mi355_qmm_launch): the matmul is compute-bound, so it is run as a plain GEMM on the
 // matrix cores instead of streaming the quantised weights once per 32 tokens.
 //   1. `qmp_dequant_kernel`  : repacked Q4_K / Q6_K tiles -> bf16 hi + bf16 lo, row-major [N, K] (w = hi + lo to 2^-17)
 //   2. `qmp_xsplit_kernel`   : activations (RMSNorm applied here) -> bf16 hi + lo, row-major [T, K]
