@@ -24,8 +24,7 @@ def lib():
     MI355_TUNING=44:3,5:64 = the balanced LDS-DMA attention stream wherever its shapes fit); tests that scope a key with
     candle_vllm_amd.tuning() still get their own value inside the block and this one back afterwards."""
     import __graft_entry__ as ge
-    if not (os.path.exists(ge.LIB) and os.path.exists(ge.ORACLE_LIB)):
-        ge.build()
+    ge.ensure_built()
     import candle_vllm_amd
     for kv in filter(None, os.environ.get("MI355_TUNING", "").split(",")):
         k, v = kv.split(":")

@@ -16,7 +16,7 @@ import pytest
 @pytest.fixture(scope="module")
 def pal():
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     from candle_vllm_amd._lib import lib
     f = lib.mi355_internal_pal_layout
     f.restype = ctypes.c_int32

@@ -20,7 +20,7 @@ QT = 2                                              # query tiles of 16 per work
 @pytest.fixture(scope="module")
 def pal():
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     from candle_vllm_amd._lib import lib
     f = lib.mi355_internal_pal_layout
     f.restype = ctypes.c_int32

@@ -25,7 +25,7 @@ TYPES = {"default": 0, "linear": 1, "llama3": 2, "dynamic": 3, "yarn": 4}
 @pytest.mark.parametrize("name,scaling,kw", CASES, ids=[c[0] for c in CASES])
 def test_rope_tables_match_the_reference_restatement(name, scaling, kw):
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     from candle_vllm_amd._lib import lib, RopeScaling
     ref_c, ref_s = O.rope_tables_scaled(kw["theta"], kw["dim"], kw["max_seq"], scaling, kw["mpe"])
     sc = None
@@ -52,7 +52,7 @@ def test_rope_tables_match_the_reference_restatement(name, scaling, kw):
 
 def test_bad_arguments_are_rejected():
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     from candle_vllm_amd._lib import lib, RopeScaling
     buf = np.empty((4, 4), np.float32)
     sc = RopeScaling()
@@ -68,7 +68,7 @@ def test_rope_tables_match_committed_golden_rows():
     import json
     import os
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     from candle_vllm_amd._lib import lib, RopeScaling
     gold = json.load(open(os.path.join(os.path.dirname(__file__), "golden", "rope_tables.json")))
     for name, g in gold.items():
@@ -101,7 +101,7 @@ def test_rope_scaling_matches_huggingface_inverse_frequencies():
     import json
     import os
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     from candle_vllm_amd._lib import lib, RopeScaling
     gold = json.load(open(os.path.join(os.path.dirname(__file__), "golden", "rope_hf.json")))
     for name, g in gold.items():
@@ -134,7 +134,7 @@ def test_effective_max_seq_len_matches_the_reference_unit_tests():
     """`Config::effective_max_seq_len` / `apply_runtime_rope_overrides` against the reference's own tests
     (src/openai/models/mod.rs:889-918): yarn factor 4 over 262144 -> 1048576; runtime yarn factor 8 -> 2097152"""
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     from candle_vllm_amd._lib import lib, RopeScaling
     sc = RopeScaling()
     sc.type, sc.factor, sc.original_max_position_embeddings = TYPES["yarn"], 4.0, 262144.0

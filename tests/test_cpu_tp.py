@@ -78,7 +78,7 @@ def test_tp2_oracle_equals_unsharded(moe, vocab):
         pytest.skip("package not importable")
     # importing candle_vllm_amd needs the built library (symbol check); build on demand
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     cfg, W, seqs = _case(moe, vocab)
     ref_m = llama.OracleLlama(cfg, W)
     cache = ref_m.new_cache(8)
@@ -161,7 +161,7 @@ def test_tp2_dense_oracle_close_to_unsharded(gptq):
     TP=2 is not bit-identical to TP=1 in 16-bit arithmetic; it must agree to bf16 accumulation noise and pick the
     same greedy tokens."""
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     from oracle import dense_llama as DL
     cfg, W, seqs = _dense_case(gptq)
     pre, dec = _dense_run(DL.OracleDenseLlama(cfg, W, flash_layout=False), cfg, seqs)
@@ -280,7 +280,7 @@ def test_external_communicator_callbacks_two_ranks():
     communicator binds): argument passing, dtype codes, in-place sum, rank-major gather, error propagation -- through the
     same Python callbacks `test_gpu_tp2.py` uses, with the payload in host memory."""
     import __graft_entry__ as ge
-    ge.build()
+    ge.ensure_built()
     ctx = mp.get_context("spawn")
     q = ctx.Queue()
     port = _free_port()
