@@ -194,9 +194,9 @@ def last_split():
     return f()
 
 
-# K in ranges: a token in a block of its own, blocks that end inside, rows that fill neither tile nor workgroup, k-blocks that the ranges do not divide
-@pytest.mark.parametrize("kind,T,N,K", [(Q4, 41, 2048, 2048), (Q4, 64, 530, 8192), (Q4, 73, 4096, 4096), (Q4, 129, 3072, 8192), (Q4, 300, 1024, 2816), (Q4, 500, 2048, 8192),
-                                        (Q6, 41, 2048, 8192), (Q6, 64, 4100, 2048), (Q6, 95, 424, 1024), (Q6, 130, 4096, 14336), (Q6, 700, 512, 3328)])
+# K in ranges: a token in a block of its own, one to eight behind whole portions of 32 (they go in a launch of their own), blocks that end inside, rows that fill neither tile nor workgroup, k-blocks that the ranges do not divide
+@pytest.mark.parametrize("kind,T,N,K", [(Q4, 41, 2048, 2048), (Q4, 64, 530, 8192), (Q4, 65, 4096, 4096), (Q4, 73, 4096, 4096), (Q4, 129, 3072, 8192), (Q4, 300, 1024, 2816), (Q4, 500, 2048, 8192),
+                                        (Q6, 41, 2048, 8192), (Q6, 64, 4100, 2048), (Q6, 72, 2048, 8192), (Q6, 95, 424, 1024), (Q6, 130, 4096, 14336), (Q6, 700, 512, 3328)])
 def test_ranges_of_k(kind, T, N, K):
     rng = np.random.default_rng(T + N)
     b = blocks(rng, N, K, kind)
@@ -266,7 +266,7 @@ def test_gate_up_ranges_of_k(T, N, K):
     assert close(out, want) < 2 * TOL                                 # two rounded factors
 
 
-@pytest.mark.parametrize("v_kind,T", [(Q4, 41), (Q6, 41), (Q4, 161), (Q6, 320)])
+@pytest.mark.parametrize("v_kind,T", [(Q4, 41), (Q6, 41), (Q4, 72), (Q6, 66), (Q4, 161), (Q6, 320)])
 def test_qkv_ranges_of_k(v_kind, T):
     H, Hkv, D, K, block = 16, 4, 128, 2048, 16
     rng = np.random.default_rng(T)
