@@ -598,6 +598,7 @@ def main():
     # rank-0-only call would wait for its peers forever
     roofline = gm.dominant_kernel_roofline(stream, HBM_PEAK_GBS)
     if rank == 0:
+        bench_timing.progress(f"batch {B}: {out['value']} tokens/s")
         out["roofline"] = roofline
         # `roofline.frac` describes the DOMINANT launch (the best-behaved one of the step); the whole step's time-weighted fraction
         # -- every algorithmic byte of the step over the step's time -- rides next to it, in `roofline` and in the contract's `config`
@@ -606,10 +607,12 @@ def main():
         out["config"]["dominant_launch_frac_of_8TBs"] = roofline["frac"]
         if do_b32:
             out["batch32"] = bench_batch32(gm, cfg, args, perm, blocks_per_seq, stream, kv_per_tok)
+            bench_timing.progress("batch 32")
             try:
                 out["prefill"] = bench_prefill(gm, cfg, perm, blocks_per_seq)
             except Exception as e:                            # secondary number only
                 out["prefill"] = {"error": repr(e)}
+            bench_timing.progress("prompt step")
             # BASELINE's metric is "decode tokens/s @ batch=1,32 ...; achieved HBM GB/s vs peak": `value` is the batch-1 number, the
             # batch-32 number and the prompt-step number ride in `config` so that a record which keeps only the contract keys holds them
             out["config"]["batch32_tokens_per_s"] = out["batch32"]["value"]
@@ -630,13 +633,16 @@ def main():
                 out["parity"] = parity_leg(args.parity)
             except Exception as e:                            # the checker must never sink the measured number
                 out["parity"] = {"error": repr(e)}
+            bench_timing.progress("parity")
         if do_b32 and not args.no_experiments and args.legs != "none" and not args.layers:
             out["experiments"] = experiments_leg()
+            bench_timing.progress("experiments")
         if not args.no_cpu_baseline and world == 1:
             try:
                 out["cpu_baseline"] = cpu_baseline(cfg, args.cpu_steps, args.ctx)
             except Exception as e:                            # the baseline must never sink the GPU number
                 out["cpu_baseline"] = {"error": repr(e)}
+            bench_timing.progress("CPU baseline")
             try:
                 out["cpu_baseline_config0"] = cpu_baseline_config0()
             except Exception as e:

@@ -449,6 +449,7 @@ def leg_parity(name):
 def run_legs(names, parity=True):
     import gc
     import torch
+    from bench_timing import progress
     out = {}
     for n in names:
         t0 = time.time()
@@ -457,6 +458,7 @@ def run_legs(names, parity=True):
             out[n]["seconds"] = round(time.time() - t0, 1)
         except Exception as e:                                        # a secondary leg must never sink the headline
             out[n] = {"error": repr(e)}
+        progress(f"leg {n}")
         gc.collect()
         torch.cuda.empty_cache()
         if parity and "error" not in out[n] and n not in NO_PARITY_LEG:
@@ -466,6 +468,7 @@ def run_legs(names, parity=True):
                 out[n]["parity"]["seconds"] = round(time.time() - t1, 1)
             except Exception as e:                                    # the checker must never sink the measured number
                 out[n]["parity"] = {"error": repr(e)}
+            progress(f"leg {n}: parity")
             gc.collect()
             torch.cuda.empty_cache()
     return out

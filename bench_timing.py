@@ -11,7 +11,13 @@ run reported half the rate of every other run.  Now every timed number is taken 
   3. the reported value is the MEDIAN block; min, max and every block ride along, together with the library's capture / eager-step
      counters before and after the timed region (mi355_llama_graph_captures: a re-capture inside a timed block would be visible).
 """
+import sys
 import time
+
+
+def progress(what):
+    """a part of the benchmark is done: said on stderr (stdout holds the one result line), so that minutes of work are not silent"""
+    print(f"bench: {what}", file=sys.stderr, flush=True)
 
 
 def settle(step, settle_ms=300.0, agree=0.02, max_steps=4000, max_ms=6000.0, reset=None, reset_every=0, fixed_steps=0):
