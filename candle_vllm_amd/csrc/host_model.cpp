@@ -347,7 +347,7 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
                 const int nblk = tiles ? 4 * ((pairs + 255) / 256 + c.n_expert) : blk64, rows = 64 * nblk;
                 RCHECK((tiles ? mi355_internal_moe_group_tiles : mi355_moe_group_blocks)(m->p_moe_inv, m->p_moe_tab, in.moe_ids, pairs, c.n_expert, nblk + 2, st));
                 Mi355PromptImage how;
-                how.tiles = tiles ? c.n_expert : 0;
+                how.tiles = tiles ? (int16_t)c.n_expert : 0;
                 RCHECK(mi355_moe_gather_pos(m->p_moe_xg, in.xs, m->p_moe_inv, pairs, K, hid, st));
                 mi355_qmm_desc g;
                 memset(&g, 0, sizeof(g));

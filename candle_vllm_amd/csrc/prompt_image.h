@@ -16,7 +16,9 @@ struct Mi355PromptImage {
     bool next = false;               // the call's output is the next call's x: leave its image
     // a grouped product of a mixture's down projection (group_block_table): its sums of `ks` ranges of K instead of outputs, where that is quicker (0: outputs)
     bool want_parts = false;
-    int32_t tiles = 0;               // ... whose groups, so many, are whole tiles of 256 rows (mi355_internal_moe_group_tiles); -1: the kernels of such tiles whatever they take
+    // ... whose groups, so many, are whole tiles of 256 rows (mi355_internal_moe_group_tiles); -1: the kernels of such tiles whatever they take.  16 bits in what was
+    // padding: the members around it stay where callers have them (below)
+    int16_t tiles = 0;
     int32_t ks = 0, ldp = 0;
     const float* parts = nullptr;    // [ks][num_tokens][ldp], in scratch: read by the caller's next launch, in the same turn of (MI355_SCR_QMP_WS, stream)
     const float* scale = nullptr;    // [num_tokens]
@@ -24,3 +26,7 @@ struct Mi355PromptImage {
     // two sets of two floats a row, the f16 image, its sub-block sums
     static size_t need(size_t rows, size_t k) { return (size_t)MAX_ROWS * 16 + rows * (k * 2 + k / 256 * 32); }
 };
+// callers outside these sources share this layout (mi355_internal_qmatmul_prompt is exported): a new member goes behind the last or into padding
+static_assert(offsetof(Mi355PromptImage, eps) == 56 && offsetof(Mi355PromptImage, want_parts) == 61 && offsetof(Mi355PromptImage, tiles) == 62 &&
+              offsetof(Mi355PromptImage, ks) == 64 && offsetof(Mi355PromptImage, parts) == 72 && offsetof(Mi355PromptImage, scale) == 80 &&
+              sizeof(Mi355PromptImage) == 88, "the layout that callers have");

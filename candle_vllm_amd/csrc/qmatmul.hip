@@ -2310,7 +2310,7 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
     // workgroups end, 64 x 256 tiles 5.6 (4.8).  A step of 4096 tokens, eight experts and two a token, us a launch, 64 x 256 tiles over whole blocks of 64 / these: 28672 x 4096
     // 2333 / 2072, 4096 x 14336 1229 / 1280 (1340 on 64 x 256 tiles over these rows: what the first gains pays for it).
     if (big && a.blk_tab && io && io->tiles && T % 256 == 0) {
-        const float cus = (float)mi355_num_cus(), g = (float)std::max(io->tiles, 0), rows = std::max((float)(T / 256) - g, 1.f);
+        const float cus = (float)mi355_num_cus(), g = (float)std::max((int)io->tiles, 0), rows = std::max((float)(T / 256) - g, 1.f);
         const float old_us = (4.f * rows + 0.5f * g) * (float)((n_slots + 15) / 16) * (all_q4 ? 5.6f / 2.f : 4.8f);
         auto sooner = [&](int nt, float us) {
             return io->tiles < 0 || us * (std::max(rows + 0.1f * g, 1.f) * (float)((n_slots + nt - 1) / nt) + 0.5f * cus) < old_us;

@@ -359,7 +359,7 @@ def test_sums_of_ranges_are_bounded():
 class PromptImage(ctypes.Structure):
     """csrc/prompt_image.h"""
     _fields_ = [("buf", ctypes.c_void_p), ("bytes", ctypes.c_size_t), ("valid", ctypes.c_bool), ("live", ctypes.c_int32), ("rows", ctypes.c_int32),
-                ("K", ctypes.c_int32), ("half", ctypes.c_int32), ("norm", ctypes.c_void_p), ("x", ctypes.c_void_p), ("eps", ctypes.c_float), ("next", ctypes.c_bool), ("want_parts", ctypes.c_bool), ("tiles", ctypes.c_int32),
+                ("K", ctypes.c_int32), ("half", ctypes.c_int32), ("norm", ctypes.c_void_p), ("x", ctypes.c_void_p), ("eps", ctypes.c_float), ("next", ctypes.c_bool), ("want_parts", ctypes.c_bool),
                 ("ks", ctypes.c_int32), ("ldp", ctypes.c_int32), ("parts", ctypes.c_void_p), ("scale", ctypes.c_void_p)]
 
 
@@ -568,7 +568,8 @@ def test_experts_in_whole_tiles(kind, epi, counts, N, K):
     d.group_block_table = tab.data_ptr()
     fn = cv.lib.mi355_internal_qmatmul_prompt
     fn.argtypes, fn.restype = [vp, vp, ctypes.c_int64], ctypes.c_int
-    io = PromptImage(tiles=-1)
+    io = PromptImage()
+    ctypes.c_int16.from_buffer(io, PromptImage.want_parts.offset + 1).value = -1   # tiles: between want_parts and ks
     assert fn(ctypes.byref(d), ctypes.byref(io), st) == 0 and last_tile() == (20 if kind == Q4 else 21)
     live = torch.zeros(T, dtype=torch.bool, device="cuda")
     for e, c in enumerate(counts):
