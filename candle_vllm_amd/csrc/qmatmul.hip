@@ -13,7 +13,7 @@
 //   * the int4/int6 codes are unpacked IN REGISTERS to bf16 (128+q is exact in bf16: 0x4300|q) and fed
 //     straight to MFMA (v_mfma_f32_16x16x32_bf16, one MFMA = one 32-weight sub-block so the per-sub-block
 //     scale is applied to the fp32 MFMA result; Q6_K uses the K=16 MFMA for its 16-weight sub-blocks);
-//   * one token (and two of Q4_K) takes integer operands instead: qmm_digits.inc;
+//   * one token (and two of Q4_K) takes integer operands instead, x in units of its 32 columns' largest: qmm_digits.inc; the rest of this is about 3 .. 8 tokens;
 //   * activations stay fp32-accurate: x is split x = hi + lo (two bf16), hi rows and lo rows ride in the
 //     same MFMA as extra M rows (rows 0-7 hi, 8-15 lo) and are summed after scaling (error ~2^-17);
 //   * the "+128" code offset and the Q4_K minimum are folded into one term  c_j * sum_k(x)  per sub-block;

@@ -1,4 +1,4 @@
-"""Products of one and two tokens, whose x is staged as three base-256 digits of an integer in units of its 32 columns' largest exponent."""
+"""Products of one and two tokens, whose x is staged as four base-256 digits of an integer in units of its 32 columns' largest exponent."""
 import numpy as np
 import pytest
 
@@ -12,20 +12,20 @@ from tests.test_gpu_ops import bf16_dev, cv, dev          # noqa: E402,F401
 
 
 def bound(x, blocks, t, products=1):
-    """of |got - exact| per (token, row): half a unit per column -- the unit is 2^-20 of the largest exponent of the 32 --, times the weight without its minimum
+    """of |got - exact| per (token, row): a unit per column -- the unit is 2^-29 of the largest exponent of the 32 --, times the weight without its minimum
     and offset (at most 2 x the weight's scale times the largest code), and 2^-20 of all that is added for the f32 sums"""
     w = np.abs(kq.dequantize(blocks, t)).astype(np.float64)
     peak = w.reshape(len(w), -1, 32).max(axis=2, keepdims=True) * 2.0
     top = np.abs(x.astype(np.float64)).reshape(len(x), -1, 32).max(axis=2, keepdims=True)
-    unit = np.repeat(top, 32, axis=2).reshape(x.shape) * 2.0 ** -20
+    unit = np.repeat(top, 32, axis=2).reshape(x.shape) * 2.0 ** -29
     coarse = np.repeat(peak, 32, axis=2).reshape(w.shape)
-    return 0.5 * unit @ coarse.T + 2.0 ** -20 * np.abs(x.astype(np.float64)) @ coarse.T + 1e-30
+    return unit @ coarse.T + 2.0 ** -20 * np.abs(x.astype(np.float64)) @ coarse.T + 1e-30
 
 
 @pytest.mark.parametrize("t", [kq.GGML_Q4_K, kq.GGML_Q6_K])
 @pytest.mark.parametrize("T,N,K", [(1, 16, 256), (1, 40, 512), (1, 272, 2048), (1, 33, 2304), (1, 48, 14336), (2, 16, 256), (2, 40, 4096), (2, 528, 2304)])
 @pytest.mark.parametrize("spread", [0.0, 3.0])
-def test_products_within_half_a_unit(cv, t, T, N, K, spread):
+def test_products_within_a_unit(cv, t, T, N, K, spread):
     rng = np.random.default_rng(T + N + K)
     blocks = kq.quantize(rng.normal(0, 0.05, (N, K)).astype(np.float32), t)
     x = (rng.normal(size=(T, K)) * np.exp(spread * rng.normal(size=(T, K)))).astype(np.float32)
@@ -36,7 +36,26 @@ def test_products_within_half_a_unit(cv, t, T, N, K, spread):
     assert (np.abs(got - ref) <= bound(x, blocks, t)).all(), np.abs(got - ref).max()
     if spread == 0.0:
         e = np.linalg.norm(got - ref) / np.linalg.norm(ref)
-        assert e < (2e-6 if T == 1 or t == kq.GGML_Q4_K else 4e-6)      # measured 0.5e-6 .. 1.5e-6; two tokens of Q6_K have bf16 pieces: 2.8e-6
+        assert e < (5e-7 if T == 1 or t == kq.GGML_Q4_K else 4e-6)      # 2^-24 for each of a few f32 roundings; two tokens of Q6_K have bf16 pieces: 2.8e-6
+
+
+@pytest.mark.parametrize("t,T", [(kq.GGML_Q4_K, 1), (kq.GGML_Q4_K, 2), (kq.GGML_Q6_K, 1)])
+@pytest.mark.parametrize("times", [10, 30, 100, 1000])
+def test_small_columns_beside_large_ones_on_weights_of_zero(cv, t, T, times):
+    """one column of 32 is `times` the others and its weights are zero: what is left has to be as exact as two bf16 pieces of each value make it, 2^-18 of it (evenly spread:
+    2^-18 / sqrt(3) of the norm), whatever the largest of its 32 columns.  A thousand times, Q4_K: its high nibbles' offset adds 8 x 1000 x 2^-24 in f32 to sub-blocks of about 40"""
+    rng = np.random.default_rng(times + T)
+    w = np.abs(rng.normal(0, 0.05, (512, 2048))).astype(np.float32)          # (not below zero: Q4_K has no minimum then)
+    w[:, ::32] = 0.0
+    blocks = kq.quantize(w, t)
+    w = kq.dequantize(blocks, t).astype(np.float64)
+    assert (w[:, ::32] == 0.0).all()
+    x = rng.normal(size=(T, 2048)).astype(np.float32)
+    x[:, ::32] *= np.float32(times)
+    ref = x.astype(np.float64) @ w.T
+    got = cv.QMatMul(blocks, t, "cuda").forward(dev(x)).cpu().numpy().astype(np.float64)
+    e = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert e < (1.2e-5 if times == 1000 and t == kq.GGML_Q4_K else 2.2e-6), e
 
 
 @pytest.mark.parametrize("t", [kq.GGML_Q4_K, kq.GGML_Q6_K])
