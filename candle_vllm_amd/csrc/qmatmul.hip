@@ -1835,6 +1835,9 @@ static int qmg_launch(const QmmArgs& a0, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
+// ranges of K of this thread's last product of 9 .. 32 tokens (tests: which rule took it)
+static thread_local int g_qw1_split_last = 0;
+extern "C" int32_t mi355_internal_last_qw1_split(void) { return g_qw1_split_last; }
 // single-plane launcher (qmm_wide1.inc, qmm_wide1_gemm.inc): MT = m-tiles of 16 tokens (1: 9..16 tokens, 2: 17..32)
 template <int MT>
 static int qw1_launch(const QmmArgs& a0, hipStream_t st) {
@@ -1860,16 +1863,20 @@ static int qw1_launch(const QmmArgs& a0, hipStream_t st) {
         if (want < 1) want = 1;
         ks = want;
     }
-    // Where that leaves CUs idle, other numbers of ranges, of four k-blocks at least.  us of staging, GEMM and epilogue at 9 / 32 tokens on cold weights, powers of two / these:
-    //   long K: as many as stay within one workgroup per CU.  4096 x 14336 four (148 workgroups) 20.0 / 23.0, six (222) 18.4 / 21.1, seven (259: a second round) 20.5 / 24.1; Q6_K
-    //   26.6 / 28.1, 22.9 / 25.0
-    //   a few more workgroups than CUs: three, which even out over two workgroups per CU.  Q6_K 32000 x 4096 (286 workgroups) 41.6 / 46.5, 34.0 / 41.6; x 3072
-    //   34.0 / 38.5, 29.3 / 36.8; x 2048 26.3 / 29.8, two ranges 23.9 / 29.5
-    //   little more than half the CUs: three as well.  16384 x 3072 (147 workgroups) 18.1 / 20.6, 15.7 / 19.8
+    // Where that leaves CUs idle, other numbers of ranges.  us of staging, GEMM and epilogue at 9 / 32 tokens on cold weights, powers of two / these:
+    //   long K: as many as stay within one workgroup per CU, of four k-blocks at least.  4096 x 14336 four (148 workgroups) 20.0 / 23.0, six (222) 18.4 / 21.1, seven
+    //   (259: a second round) 20.5 / 24.1; Q6_K 26.6 / 28.1, 22.9 / 25.0; 9 .. 160 row-tile workgroups, 32 .. 74 k-blocks: 0.77 .. 1.02 of the time
+    //   from half the CUs to two thirds: three, two full rounds.  Gate/up 16384 x 4096 (147 workgroups) 21.1 / 24.0, 18.5 / 23.9; 14432 x 5120 (129) 22.3 / 26.0,
+    //   19.3 / 23.0; of 129 .. 170 workgroups and 12 .. 28 k-blocks 0.80 .. 0.97 of the time, at 180 1.0 .. 1.1
+    //   more workgroups than CUs: the most ranges whose rounds are no more than two (3 ranges to 4 / 3 of the CUs) or one and a half (2 ranges to 3 / 2).  Q6_K 32000 x 4096 (286)
+    //   41.6 / 46.5, 34.0 / 41.6; 257 .. 339 workgroups of 16 .. 28 k-blocks 0.75 .. 0.96 in three ranges, 380 0.82 .. 0.98 in two, and from 410 on one range is the fastest
+    //   (two 1.01 .. 1.16, three 1.04 .. 1.2 from 439 on).  Of 12 k-blocks 0.88 .. 1.01 in two; of eight 0.91 .. 0.99, but Q4_K of 17 .. 32 tokens 1.0 .. 1.06
     if (G == 1 && g_tune_ks_target > 0) {
         const int n_wg = (n_slots + QMG_NC - 1) / QMG_NC, cus = mi355_num_cus();
         if (nkb >= 32) ks = std::max(ks, std::min(cus / n_wg, nkb / 4));
-        else if (ks == 1 && ((n_wg > cus && n_wg < 2 * cus) || (2 * n_wg > cus && 3 * n_wg <= 2 * cus && nkb >= 12))) ks = std::max(1, std::min(3, nkb / 4));
+        else if (ks <= 2 && nkb >= 12 && 2 * n_wg > cus && 3 * n_wg <= 2 * cus) ks = 3;
+        else if (ks == 1 && n_wg > cus && nkb >= 16 && 3 * n_wg <= 4 * cus) ks = 3;
+        else if (ks == 1 && n_wg > cus && 2 * n_wg <= 3 * cus && (nkb >= 12 || (nkb >= 8 && (MT == 1 || a.seg[0].type == MI355_GGML_Q6_K)))) ks = 2;
     }
     // (gate/up, 256 workgroups of 16 k-blocks: a split into 2 x 8 for two workgroups per CU measured +-0.1 % on the batch-32 step, round 4)
     {   // no empty split: the kernels walk ceil(nkb / ks) k-blocks per split, and every split's partial sums are added up
@@ -1897,6 +1904,7 @@ static int qw1_launch(const QmmArgs& a0, hipStream_t st) {
     void* partp = nullptr;
     rc = qmg_buf(&partp, MI355_SCR_QMM_PART, (size_t)G * ks * BP * ldp * sizeof(float), st);
     if (rc) return rc;
+    g_qw1_split_last = ks;
     float* const part = static_cast<float*>(partp);
     static Mi355DevOnce attr_done;
     if (!attr_done.done()) {

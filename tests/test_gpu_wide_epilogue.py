@@ -111,3 +111,26 @@ def test_ranges_of_k(kind, N, K, silu):
         assert close(out, torch.nn.functional.silu(want[0]) * want[1]) < 2 * TOL
     else:
         assert close(out, want[0]) < TOL
+
+
+def last_ranges():
+    f = cv.lib.mi355_internal_last_qw1_split
+    f.restype = ctypes.c_int32
+    return f()
+
+
+# row-tile workgroups (seven tiles each) on 256 CUs: the last number that takes a rule, and the first that does not
+@pytest.mark.parametrize("wgs,nkb,T,kind,ranges", [(37, 56, 9, Q4, 6), (42, 32, 32, Q4, 6), (43, 32, 32, Q6, 5), (128, 12, 9, Q4, 2), (129, 12, 32, Q4, 3), (146, 20, 9, Q6, 3), (170, 16, 32, Q4, 3),
+                                                   (171, 16, 32, Q4, 1), (150, 11, 9, Q4, 1), (256, 16, 9, Q4, 1), (257, 16, 9, Q4, 3), (341, 16, 32, Q6, 3), (342, 16, 32, Q6, 2), (384, 16, 9, Q4, 2),
+                                                   (385, 16, 9, Q4, 1), (511, 12, 32, Q4, 1), (300, 12, 32, Q4, 2), (300, 8, 9, Q4, 2), (300, 8, 32, Q4, 1), (300, 8, 32, Q6, 2), (300, 7, 9, Q6, 1)])
+def test_number_of_ranges(wgs, nkb, T, kind, ranges):
+    from candle_vllm_amd.model import random_tiles
+    N, K = wgs * 7 * 16 - 48, 256 * nkb
+    tiles = random_tiles(kind, N, K, "cuda", torch.Generator(device="cuda").manual_seed(wgs))
+    x, out = torch.randn(T, K, device="cuda"), torch.full((T, N), float("nan"), device="cuda")
+    d = cv.QmmDesc()
+    d.nseg, d.w_tiles[0], d.ggml_type[0], d.n_rows[0] = 1, tiles.data_ptr(), kind, N
+    d.x, d.x_dtype, d.ldx, d.k, d.num_tokens = x.data_ptr(), cv.DT_F32, K, K, T
+    d.epilogue, d.out, d.ldo = cv.EPI_STORE, out.data_ptr(), N
+    go(d)
+    assert last_ranges() == ranges and torch.isfinite(out).all()
