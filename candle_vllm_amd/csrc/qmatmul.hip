@@ -1871,6 +1871,7 @@ static int qw1_launch(const QmmArgs& a0, hipStream_t st) {
     //   more workgroups than CUs: the most ranges whose rounds are no more than two (3 ranges to 4 / 3 of the CUs) or one and a half (2 ranges to 3 / 2).  Q6_K 32000 x 4096 (286)
     //   41.6 / 46.5, 34.0 / 41.6; 257 .. 339 workgroups of 16 .. 28 k-blocks 0.75 .. 0.96 in three ranges, 380 0.82 .. 0.98 in two, and from 410 on one range is the fastest
     //   (two 1.01 .. 1.16, three 1.04 .. 1.2 from 439 on).  Of 12 k-blocks 0.88 .. 1.01 in two; of eight 0.91 .. 0.99, but Q4_K of 17 .. 32 tokens 1.0 .. 1.06
+    const int ks_few = ks;
     if (G == 1 && g_tune_ks_target > 0) {
         const int n_wg = (n_slots + QMG_NC - 1) / QMG_NC, cus = mi355_num_cus();
         if (nkb >= 32) ks = std::max(ks, std::min(cus / n_wg, nkb / 4));
@@ -1879,10 +1880,9 @@ static int qw1_launch(const QmmArgs& a0, hipStream_t st) {
         else if (ks == 1 && n_wg > cus && 2 * n_wg <= 3 * cus && (nkb >= 12 || (nkb >= 8 && (MT == 1 || a.seg[0].type == MI355_GGML_Q6_K)))) ks = 2;
     }
     // (gate/up, 256 workgroups of 16 k-blocks: a split into 2 x 8 for two workgroups per CU measured +-0.1 % on the batch-32 step, round 4)
-    {   // no empty split: the kernels walk ceil(nkb / ks) k-blocks per split, and every split's partial sums are added up
-        const int kb_per = (nkb + ks - 1) / ks;
-        ks = (nkb + kb_per - 1) / kb_per;
-    }
+    // no empty split: the kernels walk ceil(nkb / ks) k-blocks per split, and every split's partial sums are added up
+    auto whole = [&](int n) { const int kb_per = (nkb + n - 1) / n; return (nkb + kb_per - 1) / kb_per; };
+    ks = whole(ks);
     QmgStream& qs = qmg_stream(st);
     const bool chained = qs.chain.valid && qs.chain.x == a.x && qs.chain.B == a.B && qs.chain.K == a.K &&
                          qs.chain.MT == MT && qs.chain.sp == 1 && qs.chain.norm_w == a.norm_w && qs.chain.st == st &&
@@ -1903,6 +1903,10 @@ static int qw1_launch(const QmmArgs& a0, hipStream_t st) {
     if (rc) return rc;
     void* partp = nullptr;
     rc = qmg_buf(&partp, MI355_SCR_QMM_PART, (size_t)G * ks * BP * ldp * sizeof(float), st);
+    if (rc && ks > whole(ks_few)) {                         // a full card, or a capture and a buffer that has room for the sums of the powers of two only
+        ks = whole(ks_few);
+        rc = qmg_buf(&partp, MI355_SCR_QMM_PART, (size_t)G * ks * BP * ldp * sizeof(float), st);
+    }
     if (rc) return rc;
     g_qw1_split_last = ks;
     float* const part = static_cast<float*>(partp);

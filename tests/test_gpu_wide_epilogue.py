@@ -134,3 +134,32 @@ def test_number_of_ranges(wgs, nkb, T, kind, ranges):
     d.epilogue, d.out, d.ldo = cv.EPI_STORE, out.data_ptr(), N
     go(d)
     assert last_ranges() == ranges and torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("kind,N,K,T,few,ranges", [(Q4, 4096, 14336, 19, 4, 6), (Q6, 32000, 4096, 32, 1, 3), (Q4, 16384, 3072, 9, 1, 3)])
+def test_no_room_for_more_sums(kind, N, K, T, few, ranges):
+    """room for the sums of the powers of two and no more: the product goes in those, on a full card and in a capture, where the buffer of an earlier product may not grow"""
+    rng = np.random.default_rng(N)
+    b = blocks(rng, N, K, kind, odd=False)
+    m = cv.QMatMul(b, kind, "cuda")
+    x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
+    want, tokens = product(x, b, kind), 16 if T <= 16 else 32
+    cv.lib.mi355_internal_scratch_limit.argtypes = [ctypes.c_int64]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        cv.lib.mi355_internal_scratch_limit(max(few * tokens * N * 4, K // 256 * 20480))   # (a k-block of the image: less than 20 KiB)
+        try:
+            got = m.forward(x)
+            assert last_ranges() == few and close(got, want) < TOL
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=torch.cuda.current_stream()):
+                captured = m.forward(x)
+        finally:
+            cv.lib.mi355_internal_scratch_limit(-1)
+        assert last_ranges() == few
+        for _ in range(3):
+            captured.zero_()
+            graph.replay()
+            assert torch.equal(captured, got)
+        assert close(m.forward(x), want) < TOL and last_ranges() == ranges
