@@ -156,6 +156,7 @@ extern "C" int32_t mi355_internal_pa_plan(int32_t num_seqs, int32_t num_heads, i
                                           int32_t kv8, int32_t slots, int32_t* partition_size);   // paged_attention.hip
 extern "C" int mi355_internal_moe_group_tiles(int32_t* pos, int32_t* block_table, const int32_t* expert_ids, int32_t num_pairs, int32_t n_expert,
                                               int32_t n_blocks, int64_t stream);                                   // moe.hip
+extern "C" int32_t mi355_internal_moe_tiles(int32_t pairs, int32_t experts, int32_t hidden, int32_t inter, int32_t down_type);   // qmatmul.hip
 extern "C" int mi355_internal_moe_combine_parts(float* ys, const float* parts, int32_t ks, int32_t rows, int32_t ldp, const float* scale, const float* weights,
                                                 const int32_t* inv, int32_t num_tokens, int32_t hidden, int32_t top_k, int64_t stream);   // moe.hip
 extern "C" int mi355_internal_qmatmul_prompt(const mi355_qmm_desc* d, Mi355PromptImage* io, int64_t stream);   // qmatmul.hip
@@ -338,12 +339,11 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
                 // per kernel for all experts.  Every expert owns whole 64-row blocks of the gathered buffers; the prompt GEMM walks a block
                 // table {expert, row end} (mi355_qmm_desc.group_block_table); rows between an expert's end and its last block's end are
                 // computed and never stored.  (Q4_K gate / up and a Q4_K or Q6_K down projection -- a Q4_K_M file; anything else takes the host-sorted path.)
-                // From 4096 rows (where the down product's sums no longer go in ranges of K) an expert owns whole tiles of 256 rows, for the
-                // kernels that unpack a weight once per 256 rows: a step of 4096 tokens of two layers, seven pairs of runs, 1.00 .. 1.06 x as fast, 1.012 at the
-                // median (sums of the kernels 10286 / 9849 us; cards at their power limit give the difference back in clocks).  Below, the tiles' empty
-                // halves take what they gain: 15.5 rounds of 64 x 256 tiles become 8.8 of 256 x 256 at 1500 tokens, by estimate 5 % less, and the ranges are lost.
+                // From 4096 rows an expert owns whole tiles of 256 rows where the kernels that unpack a weight once per 256 rows make both products sooner
+                // (mi355_internal_moe_tiles): a step of 4096 tokens of two layers, seven pairs of runs, 1.00 .. 1.06 x as fast, 1.012 at the
+                // median (sums of the kernels 10286 / 9849 us; cards at their power limit give the difference back in clocks).
                 const int blk64 = (pairs + 63) / 64 + c.n_expert;
-                const bool tiles = 64 * blk64 > 4096;
+                const bool tiles = mi355_internal_moe_tiles(pairs, c.n_expert, hid, I, L.etype[1]) != 0;
                 const int nblk = tiles ? 4 * ((pairs + 255) / 256 + c.n_expert) : blk64, rows = 64 * nblk;
                 RCHECK((tiles ? mi355_internal_moe_group_tiles : mi355_moe_group_blocks)(m->p_moe_inv, m->p_moe_tab, in.moe_ids, pairs, c.n_expert, nblk + 2, st));
                 Mi355PromptImage how;

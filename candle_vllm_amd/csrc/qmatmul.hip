@@ -2231,6 +2231,35 @@ static float qpg_tiles_us(int type, int T, int n_slots, int nkb) {
     const int wgs = ((T + 63) / 64) * ((n_slots + 15) / 16);
     return (float)nkb * (type == MI355_GGML_Q4_K ? qpw_rounds(wgs, 2 * mi355_num_cus(), 5.f, 3.4f) : qpw_rounds(wgs, mi355_num_cus(), 4.3f, 3.95f));
 }
+// us of a mixture's product over a block table: rows256 = its rows in 256s, over `groups` experts, each of which ends inside a tile.  64 x 256 tiles, or (tiles) the
+// kernels of 256 rows a tile.  A round of workgroups and k-block, the share of a tile that a group adds, what the last, part-filled round costs beyond its share, and the launches:
+// fitted to 192 steps of 3300 .. 16400 rows, 2 .. 16 experts, hidden 1024 .. 6144, 1024 .. 16384 columns each, even and uneven routing: error 10 .. 11 %
+static float qpg_tab_us(bool q4, float rows256, int groups, int n_slots, int nkb, bool tiles) {
+    const float cus = (float)mi355_num_cus(), g = (float)groups;
+    const float cols = (float)(tiles && !q4 ? (n_slots + 7) / 8 : (n_slots + 15) / 16);
+    auto us = [&](float round, float blocks, float cap, float last, float launches) { return (float)nkb * round * std::max(blocks * cols / cap + last, 1.f) + launches; };
+    if (tiles) return q4 ? us(8.8f, rows256 + 0.23f * g, cus, 0.4f, 37.f) : us(5.6f, rows256 + 0.37f * g, cus, 0.22f, 37.f);
+    return q4 ? us(5.7f, 4.f * rows256, 2.f * cus, 0.42f, 29.f) : us(5.4f, 4.f * rows256 + 0.42f * g, cus, 0.07f, 61.f);
+}
+// Whether a mixture's prompt step gives every expert whole tiles of 256 rows (mi355_internal_moe_group_tiles): where both products together, each on its sooner kernel, are 2 % or more
+// sooner by estimate than over blocks of 64.  Up to 4096 rows the down product's sums go in ranges of K, over blocks.  us of gate/up + down, blocks / whole tiles, where it picks
+// them: 8 experts of 14336 x 4096, 2100 tokens 1411 + 841 / 1212 + 830, 4096 2403 + 1356 / 2121 + 1352 (down in Q6_K 2392 + 2470 / 2266 + 1477); of 3584 columns 2100 tokens 447 + 262 /
+// 387 + 235; and where it does not: 1792 columns, 2100 tokens 215 + 122 / 257 + 138; 16 experts of 1536 x 2048, four a token, 2048 tokens 179 + 118 / 219 + 133; 4 experts of
+// 3584 x 1024, 2100 tokens 115 + 92 / 131 + 119.  What it picks is 0.3 % behind the sooner layout over those 192 steps, 0.6 % over 48 others (profiles/mixture_prompt_layouts.txt).
+extern "C" int32_t mi355_internal_moe_tiles(int32_t pairs, int32_t experts, int32_t hidden, int32_t inter, int32_t down_type) {
+    if (64 * ((int64_t)(pairs + 63) / 64 + experts) <= QPG_PART_ROWS_TAB) return 0;
+    if (!g_tune_qpg_fepi || g_tune_exact_act || g_tune_qpg != 2) return 0;                        // no such kernels
+    if ((size_t)std::max(hidden, inter) * ((size_t)256 * ((pairs + 255) / 256 + experts) + 512) * 2 >= ((size_t)1 << 32)) return 0;   // (nor 32-bit offsets into the image)
+    float us[2] = {0.f, 0.f};
+    for (int p = 0; p < 2; ++p) {
+        const bool q4 = p == 0 || down_type == MI355_GGML_Q4_K;
+        const int slots = p == 0 ? 2 * ((inter + 15) / 16) : (hidden + 15) / 16, nkb = (p == 0 ? hidden : inter) / 256;
+        const float blocks = qpg_tab_us(q4, (float)pairs / 256.f, experts, slots, nkb, false);
+        us[0] += blocks;
+        us[1] += std::min(blocks, qpg_tab_us(q4, (float)pairs / 256.f, experts, slots, nkb, true));
+    }
+    return us[1] < 0.98f * us[0];
+}
 // Few tokens: those tiles with K in ks ranges, whose sums the epilogue's launch adds up.  A workgroup walks its k-blocks at the pace of its own round trips
 // (2.3 us each, alone on its CU or not), so a product of 48 workgroups and 32 k-blocks took 95 us with most of the chip idle.  us of both launches, fitted to
 // 1 000 launches of 33 .. 1400 tokens (error 8 %): per round and k-block, 3 per round, 4 for the second launch beyond what a fused epilogue costs, and the sums'
@@ -2317,18 +2346,12 @@ static int qpg_launch(const QmmArgs& a0, hipStream_t st, Mi355PromptImage* io, c
         const QpwChoice c = qpw_pick(MI355_GGML_Q6_K, T, v_slots ? v_slots : n_slots, K, v_slots || T >= 4096 ? 0.f : c_pass);
         pick6 = c.tile; whole_us += c.us;
     }
-    // Groups in whole tiles of 256 rows, the part-filled ones (one a group, half of it empty on average: 0.6 of a tile's time) behind the others: the kernels that unpack a
-    // weight once per 256 rows where they are sooner.  us per k-block and round: 256 x 256 7.75 (Q6_K 256 x 128 4.8) and half a round until the last
-    // workgroups end, 64 x 256 tiles 5.6 (4.8).  A step of 4096 tokens, eight experts and two a token, us a launch, 64 x 256 tiles over whole blocks of 64 / these: 28672 x 4096
-    // 2333 / 2072, 4096 x 14336 1229 / 1280 (1340 on 64 x 256 tiles over these rows: what the first gains pays for it).
+    // groups in whole tiles of 256 rows: the kernels that unpack a weight once per 256 rows where they are sooner
     if (big && a.blk_tab && io && io->tiles && T % 256 == 0) {
-        const float cus = (float)mi355_num_cus(), g = (float)std::max((int)io->tiles, 0), rows = std::max((float)(T / 256) - g, 1.f);
-        const float old_us = (4.f * rows + 0.5f * g) * (float)((n_slots + 15) / 16) * (all_q4 ? 5.6f / 2.f : 4.8f);
-        auto sooner = [&](int nt, float us) {
-            return io->tiles < 0 || us * (std::max(rows + 0.1f * g, 1.f) * (float)((n_slots + nt - 1) / nt) + 0.5f * cus) < old_us;
-        };
-        if (all_q4 && epi_ok && sooner(16, 7.75f)) pick4 = 0;
-        else if (one_q6 && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID) && sooner(8, 4.8f)) pick6 = 1;
+        const float rows256 = std::max((float)(T / 256 - io->tiles), 1.f);
+        auto sooner = [&](bool q4) { return io->tiles < 0 || qpg_tab_us(q4, rows256, io->tiles, n_slots, nkb, true) < qpg_tab_us(q4, rows256, io->tiles, n_slots, nkb, false); };
+        if (all_q4 && epi_ok && sooner(true)) pick4 = 0;
+        else if (one_q6 && (a.epi == MI355_EPI_STORE || a.epi == MI355_EPI_RESID) && sooner(false)) pick6 = 1;
     }
     if (T < g_tune_qpg_min && !a.blk_tab && whole_us == 0.f) return (int)hipErrorNotSupported;
     int ks = 1;

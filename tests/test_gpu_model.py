@@ -666,3 +666,58 @@ def test_moe_decode_experts_grouped_on_the_device(lib, B):
     want = [int(e) * 2 * B + int((ids[:p] == e).sum()) for p, e in enumerate(ids)]
     assert pos.cpu().tolist() == want
     assert cnt.cpu().tolist() == [int((ids == e).sum()) for e in range(4)]
+
+
+def mixture(hid, inter, n_expert, down, max_batch, blocks_per_seq):
+    """one layer, random blocks"""
+    from candle_vllm_amd import model as M
+    from tests.fullsize_moe import _native
+    cfg = M.ModelDims(hidden=hid, n_layers=1, n_heads=8, n_kv_heads=2, head_dim=128, intermediate=inter, vocab=512, max_seq=4096, block_size=16)
+    cfg.n_expert, cfg.n_expert_used = n_expert, 2
+    gm = M.GGUFLLaMa(cfg, max_batch=max_batch, max_blocks_per_seq=blocks_per_seq, kv_layout=M.KV_FLASH)
+    rng = np.random.default_rng(hid + inter)
+
+    def f32(layer, which, a):
+        a = np.ascontiguousarray(a, np.float32)
+        M._check(M.lib.mi355_llama_set_f32(gm.h, layer, which, a.ctypes.data, a.size), "set_f32")
+
+    def q(layer, which, t, n, k):
+        b = _native(rng, t, n, k, 8.0)
+        M._check(M.lib.mi355_llama_set_qweight(gm.h, layer, which, t, b.ctypes.data, n, k), "set_qweight")
+    f32(-1, M.W_TOK_EMBD, rng.normal(0, 0.5, (512, hid)))
+    f32(-1, M.W_OUTPUT_NORM, np.ones(hid))
+    q(-1, M.W_OUTPUT, 14, 512, hid)
+    f32(0, M.W_ATTN_NORM, np.ones(hid))
+    f32(0, M.W_FFN_NORM, np.ones(hid))
+    f32(0, 12, rng.normal(0, 0.5, (n_expert, hid)))
+    for which, n, k in ((M.W_WQ, 1024, hid), (M.W_WK, 256, hid), (M.W_WV, 256, hid), (M.W_WO, hid, 1024)):
+        q(0, which, 12, n, k)
+    for which, t, n, k in ((M.W_W1, 12, inter, hid), (M.W_W3, 12, inter, hid), (M.W_W2, down, hid, inter)):
+        for e in range(n_expert):
+            b = _native(rng, t, n, k, 8.0)
+            M._check(M.lib.mi355_llama_set_moe_expert(gm.h, 0, which, e, t, b.ctypes.data, n, k), "set_moe_expert")
+    return gm
+
+
+# the kernel of the down product: whole tiles of 256 rows (20, 21), 64 x 256 tiles (-1) over either layout
+@pytest.mark.parametrize("hid,inter,down,tokens,layout,kernel", [(1024, 3584, 14, 528, 1, 21), (2048, 4096, 12, 528, 1, 20), (1024, 3584, 12, 528, 1, -1), (1024, 3584, 12, 290, 0, -1)])
+def test_moe_prompt_layouts(lib, hid, inter, down, tokens, layout, kernel):
+    """a prompt step of eight sequences, whose rows are beyond 4096, against the same sequences two at a time (blocks of 64 rows, the down product in ranges of K): the
+    host's choice, the kernel that follows from it, and every sequence's logits"""
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible MI355X")
+    from candle_vllm_amd import model as M
+    gm = mixture(hid, inter, 4, down, 8, 64)
+    gm.alloc_kv_cache(8 * 33 + 1)
+    rng = np.random.default_rng(tokens)
+    seqs = [{"tokens": [int(t) for t in rng.integers(0, 512, tokens - 7 * i)], "block_table": list(range(1 + 33 * i, 34 + 33 * i))} for i in range(8)]
+    assert M.lib.mi355_internal_moe_tiles(2 * sum(len(s["tokens"]) for s in seqs), 4, hid, inter, down) == layout
+    got = gm.forward_prefill(O.prepare_prompt(seqs, 16)).cpu().numpy().copy()
+    assert M.lib.mi355_internal_last_qpw() == kernel
+    want = []
+    for i in range(0, 8, 2):
+        want.append(gm.forward_prefill(O.prepare_prompt(seqs[i:i + 2], 16)).cpu().numpy().copy())
+        assert M.lib.mi355_internal_last_qpw() == -1
+    want = np.concatenate(want)
+    assert np.isfinite(got).all() and _rel(got, want) < 3e-3, _rel(got, want)
+    print(_rel(got, want))
