@@ -114,6 +114,7 @@ struct Model {
     // grouped experts on prompt steps: gathered rows in expert order + the permutation and its inverse
     Mi355PromptImage p_img;          // prompt steps of up to 1024 tokens: the next product's activation image (qmatmul.hip qpg_sum_image_kernel)
     float* p_moe_xg = nullptr; int32_t* p_moe_perm = nullptr; int32_t* p_moe_inv = nullptr;
+    size_t p_moe_rows = 0;           // rows of p_h, p_moe_xg and p_moe_y
     int32_t* p_moe_tab = nullptr;    // block table of the device-grouped prompt path: {expert, row end} per 64-row block
     // decode steps with many (token, slot) pairs: experts grouped on the device, `g_cap` rows per expert (host_model.cpp run_part)
     float* g_moe_xg = nullptr; float* g_moe_h = nullptr; float* g_moe_yg = nullptr; int32_t* g_moe_pos = nullptr; int32_t* g_moe_cnt = nullptr; int g_cap = 0;
@@ -343,8 +344,9 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
                 // (mi355_internal_moe_tiles): a step of 4096 tokens of two layers, seven pairs of runs, 1.00 .. 1.06 x as fast, 1.012 at the
                 // median (sums of the kernels 10286 / 9849 us; cards at their power limit give the difference back in clocks).
                 const int blk64 = (pairs + 63) / 64 + c.n_expert;
-                const bool tiles = mi355_internal_moe_tiles(pairs, c.n_expert, hid, I, L.etype[1]) != 0;
-                const int nblk = tiles ? 4 * ((pairs + 255) / 256 + c.n_expert) : blk64, rows = 64 * nblk;
+                const int tiles256 = 4 * ((pairs + 255) / 256 + c.n_expert);
+                const bool tiles = (size_t)64 * tiles256 <= m->p_moe_rows && mi355_internal_moe_tiles(pairs, c.n_expert, hid, I, L.etype[1]) != 0;
+                const int nblk = tiles ? tiles256 : blk64, rows = 64 * nblk;
                 RCHECK((tiles ? mi355_internal_moe_group_tiles : mi355_moe_group_blocks)(m->p_moe_inv, m->p_moe_tab, in.moe_ids, pairs, c.n_expert, nblk + 2, st));
                 Mi355PromptImage how;
                 how.tiles = tiles ? (int16_t)c.n_expert : 0;
@@ -934,6 +936,9 @@ extern "C" int64_t mi355_llama_kv_bytes_per_tensor(void* mp) {
            (m->cfg.kv_layout == MI355_KV_PAGED_FP8 ? 1 : 2);
 }
 
+// rows of the experts' prompt buffers (tests)
+extern "C" int64_t mi355_internal_moe_prompt_rows(void* mp) { return mp ? (int64_t)static_cast<Model*>(mp)->p_moe_rows : -1; }
+
 static int ensure_prefill_cap(Model* m, int T) {
     if (T <= m->p_cap) return 0;
     void* old[] = {m->p_xs, m->p_q, m->p_attn, m->p_h, m->p_tp_y, m->p_img.buf};
@@ -946,10 +951,32 @@ static int ensure_prefill_cap(Model* m, int T) {
     HCHECK(hipMalloc((void**)&m->p_xs, (size_t)cap * m->cfg.hidden * 4));
     HCHECK(hipMalloc((void**)&m->p_q, (size_t)cap * H * D * 2));
     HCHECK(hipMalloc((void**)&m->p_attn, (size_t)cap * H * D * 2));
-    const int KE = m->cfg.n_expert > 1 ? m->cfg.n_expert_used : 1;
-    // (+ 256 rows per expert: the device-grouped prompt path gives every expert whole tiles)
-    const size_t moe_pad = m->cfg.n_expert > 1 ? (size_t)256 * (m->cfg.n_expert + 2) : 0;
-    HCHECK(hipMalloc((void**)&m->p_h, ((size_t)cap * KE + moe_pad) * m->cfg.intermediate * 4));
+    const int E = m->cfg.n_expert, KE = E > 1 ? m->cfg.n_expert_used : 1;
+    if (E > 1) {
+        void* oldm[] = {m->p_moe_ids, m->p_moe_w, m->p_moe_y, m->p_moe_xg, m->p_moe_perm, m->p_moe_inv, m->p_moe_tab};
+        for (void* p : oldm) if (p) (void)hipFree(p);
+        m->p_moe_ids = nullptr; m->p_moe_w = nullptr; m->p_moe_y = nullptr;
+        m->p_moe_xg = nullptr; m->p_moe_perm = nullptr; m->p_moe_inv = nullptr; m->p_moe_tab = nullptr;
+    }
+    // Rows of the experts' buffers: the device-grouped prompt path gives every expert whole blocks of 64 rows, or whole tiles of 256 where a chunk can have rows enough for
+    // them and the grouping takes so many experts (eight experts of 14336: 173 MB more) -- and where the card has room
+    const size_t pairs = (size_t)cap * KE;
+    auto rows_of = [&](size_t n) {
+        float** bufs[] = {&m->p_h, E > 1 ? &m->p_moe_xg : nullptr, E > 1 ? &m->p_moe_y : nullptr};
+        m->p_moe_rows = n;
+        for (float** p : bufs) {
+            if (!p) continue;
+            const hipError_t e = hipMalloc((void**)p, n * (p == &m->p_h ? m->cfg.intermediate : m->cfg.hidden) * 4);
+            if (e == hipSuccess) continue;
+            (void)hipGetLastError();
+            *p = nullptr;
+            for (float** q : bufs) if (q && *q) { (void)hipFree(*q); *q = nullptr; }
+            return (int)e;
+        }
+        return 0;
+    };
+    const bool tiles = E > 1 && E <= 16 && 64 * ((pairs + 63) / 64 + E) > 4096;
+    if (!tiles || rows_of(pairs + (size_t)256 * E) != 0) RCHECK(rows_of(E > 1 ? pairs + (size_t)64 * (E + 2) : pairs));
     if (m->use_comm) HCHECK(hipMalloc((void**)&m->p_tp_y, (size_t)cap * m->cfg.hidden * 4));
     if (!m->use_comm && m->cfg.n_expert <= 1) {
         // (29 MiB at most for 14336 columns; without it every product builds its own image)
@@ -958,18 +985,12 @@ static int ensure_prefill_cap(Model* m, int T) {
         else { (void)hipGetLastError(); m->p_img.buf = nullptr; }
     }
     if (m->cfg.n_expert > 1) {
-        void* oldm[] = {m->p_moe_ids, m->p_moe_w, m->p_moe_y, m->p_moe_xg, m->p_moe_perm, m->p_moe_inv, m->p_moe_tab};
-        for (void* p : oldm) if (p) (void)hipFree(p);
-        m->p_moe_ids = nullptr; m->p_moe_w = nullptr; m->p_moe_y = nullptr;
-        m->p_moe_xg = nullptr; m->p_moe_perm = nullptr; m->p_moe_inv = nullptr; m->p_moe_tab = nullptr;
-        HCHECK(hipMalloc((void**)&m->p_moe_tab, ((size_t)cap * KE / 64 + 4 * m->cfg.n_expert + 8) * 8));
-        HCHECK(hipMalloc((void**)&m->p_moe_xg, ((size_t)cap * KE + moe_pad) * m->cfg.hidden * 4));
-        HCHECK(hipMemsetAsync(m->p_moe_xg, 0, ((size_t)cap * KE + moe_pad) * m->cfg.hidden * 4, 0));   // the rows no pair lands in: finite from the start
-        HCHECK(hipMalloc((void**)&m->p_moe_perm, (size_t)cap * KE * 4));
-        HCHECK(hipMalloc((void**)&m->p_moe_inv, (size_t)cap * KE * 4));
-        HCHECK(hipMalloc((void**)&m->p_moe_ids, (size_t)cap * KE * 4));
-        HCHECK(hipMalloc((void**)&m->p_moe_w, (size_t)cap * KE * 4));
-        HCHECK(hipMalloc((void**)&m->p_moe_y, ((size_t)cap * KE + moe_pad) * m->cfg.hidden * 4));
+        HCHECK(hipMalloc((void**)&m->p_moe_tab, (pairs / 64 + 4 * E + 8) * 8));
+        HCHECK(hipMemsetAsync(m->p_moe_xg, 0, m->p_moe_rows * m->cfg.hidden * 4, 0));   // the rows no pair lands in: finite from the start
+        HCHECK(hipMalloc((void**)&m->p_moe_perm, pairs * 4));
+        HCHECK(hipMalloc((void**)&m->p_moe_inv, pairs * 4));
+        HCHECK(hipMalloc((void**)&m->p_moe_ids, pairs * 4));
+        HCHECK(hipMalloc((void**)&m->p_moe_w, pairs * 4));
         HCHECK(hipDeviceSynchronize());
     }
     m->p_cap = cap;

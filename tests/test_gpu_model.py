@@ -1,6 +1,7 @@
 """GPU end-to-end parity: the C++ GGUFLLaMa decode step (eager and hipGraph replay) vs the numpy oracle on a
 tiny synthetic llama (same seeded weights), logits within the BASELINE tolerance (1e-3 relative), greedy tokens
 identical, KV cache contents equal to 1 bf16 ulp; plus the committed golden logits."""
+import ctypes
 import json
 import os
 
@@ -721,3 +722,19 @@ def test_moe_prompt_layouts(lib, hid, inter, down, tokens, layout, kernel):
     want = np.concatenate(want)
     assert np.isfinite(got).all() and _rel(got, want) < 3e-3, _rel(got, want)
     print(_rel(got, want))
+
+
+@pytest.mark.parametrize("n_expert", [4, 32])
+def test_moe_prompt_rows_follow_the_chunk(lib, n_expert):
+    """the experts' buffers have room for whole tiles of 256 rows an expert only where a chunk can have more than 4096 rows, of experts that the grouping takes"""
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible MI355X")
+    from candle_vllm_amd import model as M
+    gm = mixture(256, 256, n_expert, 12, 2, 160)
+    gm.alloc_kv_cache(161)
+    M.lib.mi355_internal_moe_prompt_rows.restype, M.lib.mi355_internal_moe_prompt_rows.argtypes = ctypes.c_int64, [ctypes.c_void_p]
+    blocks, tiles = 64 * (n_expert + 2), 256 * n_expert
+    for tokens, cap, pad in ((100, 256, blocks), (1700, 1792, blocks), (2400, 2560, tiles if n_expert <= 16 else blocks)):
+        seq = [{"tokens": [t % 512 for t in range(tokens)], "block_table": list(range(1, 161))}]
+        assert torch.isfinite(gm.forward_prefill(O.prepare_prompt(seq, 16))).all()
+        assert M.lib.mi355_internal_moe_prompt_rows(gm.h) == 2 * cap + pad
