@@ -345,40 +345,49 @@ int run_part(Model* m, int l, int part, const StepIn& in, float* logits, int64_t
                 // median (sums of the kernels 10286 / 9849 us; cards at their power limit give the difference back in clocks).
                 const int blk64 = (pairs + 63) / 64 + c.n_expert;
                 const int tiles256 = 4 * ((pairs + 255) / 256 + c.n_expert);
-                const bool tiles = (size_t)64 * tiles256 <= m->p_moe_rows && mi355_internal_moe_tiles(pairs, c.n_expert, hid, I, L.etype[1]) != 0;
-                const int nblk = tiles ? tiles256 : blk64, rows = 64 * nblk;
-                RCHECK((tiles ? mi355_internal_moe_group_tiles : mi355_moe_group_blocks)(m->p_moe_inv, m->p_moe_tab, in.moe_ids, pairs, c.n_expert, nblk + 2, st));
-                Mi355PromptImage how;
-                how.tiles = tiles ? (int16_t)c.n_expert : 0;
-                RCHECK(mi355_moe_gather_pos(m->p_moe_xg, in.xs, m->p_moe_inv, pairs, K, hid, st));
-                mi355_qmm_desc g;
-                memset(&g, 0, sizeof(g));
-                g.nseg = 2;
-                g.w_tiles[0] = L.eslab[0]; g.ggml_type[0] = L.etype[0]; g.n_rows[0] = L.erows[0];
-                g.w_tiles[1] = L.eslab[2]; g.ggml_type[1] = L.etype[2]; g.n_rows[1] = L.erows[2];
-                g.moe_expert_stride[0] = L.estride[0]; g.moe_expert_stride[1] = L.estride[2];
-                g.x = m->p_moe_xg; g.x_dtype = MI355_DTYPE_F32; g.ldx = hid; g.k = hid; g.num_tokens = rows;
-                g.norm_weight = L.ffn_norm; g.norm_eps = c.rms_eps;
-                g.epilogue = MI355_EPI_SILU_MUL; g.out = in.h; g.ldo = I;
-                g.group_block_table = m->p_moe_tab;
-                RCHECK(mi355_internal_qmatmul_prompt(&g, &how, st));
-                mi355_qmm_desc dn;
-                memset(&dn, 0, sizeof(dn));
-                dn.nseg = 1;
-                dn.w_tiles[0] = L.eslab[1]; dn.ggml_type[0] = L.etype[1]; dn.n_rows[0] = L.erows[1];
-                dn.moe_expert_stride[0] = L.estride[1];
-                dn.x = in.h; dn.x_dtype = MI355_DTYPE_F32; dn.ldx = I; dn.k = I; dn.num_tokens = rows;
-                dn.epilogue = MI355_EPI_STORE; dn.out = in.moe_y; dn.ldo = hid;
-                dn.group_block_table = m->p_moe_tab;
-                Mi355ScratchTurn turn(MI355_SCR_QMP_WS, reinterpret_cast<hipStream_t>(st));      // the product's sums lie there until the launch behind it has read them
-                Mi355PromptImage sums;
-                sums.want_parts = !tiles;
-                sums.tiles = how.tiles;
-                RCHECK(mi355_internal_qmatmul_prompt(&dn, &sums, st));
-                if (sums.ks > 1)
-                    RCHECK(mi355_internal_moe_combine_parts(in.xs, sums.parts, sums.ks, rows, sums.ldp, sums.scale, in.moe_w, m->p_moe_inv, B, hid, K, st));
-                else
-                    RCHECK(mi355_moe_scatter_combine(in.xs, in.moe_y, in.moe_w, m->p_moe_inv, B, hid, K, st));
+                bool tiles = (size_t)64 * tiles256 <= m->p_moe_rows && mi355_internal_moe_tiles(pairs, c.n_expert, hid, I, L.etype[1]) != 0;
+                for (;; tiles = false) {
+                    const int nblk = tiles ? tiles256 : blk64, rows = 64 * nblk;
+                    RCHECK((tiles ? mi355_internal_moe_group_tiles : mi355_moe_group_blocks)(m->p_moe_inv, m->p_moe_tab, in.moe_ids, pairs, c.n_expert, nblk + 2, st));
+                    Mi355PromptImage how;
+                    how.tiles = tiles ? (int16_t)c.n_expert : 0;
+                    RCHECK(mi355_moe_gather_pos(m->p_moe_xg, in.xs, m->p_moe_inv, pairs, K, hid, st));
+                    mi355_qmm_desc g;
+                    memset(&g, 0, sizeof(g));
+                    g.nseg = 2;
+                    g.w_tiles[0] = L.eslab[0]; g.ggml_type[0] = L.etype[0]; g.n_rows[0] = L.erows[0];
+                    g.w_tiles[1] = L.eslab[2]; g.ggml_type[1] = L.etype[2]; g.n_rows[1] = L.erows[2];
+                    g.moe_expert_stride[0] = L.estride[0]; g.moe_expert_stride[1] = L.estride[2];
+                    g.x = m->p_moe_xg; g.x_dtype = MI355_DTYPE_F32; g.ldx = hid; g.k = hid; g.num_tokens = rows;
+                    g.norm_weight = L.ffn_norm; g.norm_eps = c.rms_eps;
+                    g.epilogue = MI355_EPI_SILU_MUL; g.out = in.h; g.ldo = I;
+                    g.group_block_table = m->p_moe_tab;
+                    // no room for the images of the tiles' rows (a full card; a capture, which may not grow the buffer): again over blocks of 64, which need less
+                    auto no_room = [&](int rc) { return tiles && (rc == (int)hipErrorOutOfMemory || rc == (int)hipErrorStreamCaptureUnsupported); };
+                    int rc = mi355_internal_qmatmul_prompt(&g, &how, st);
+                    if (no_room(rc)) continue;
+                    RCHECK(rc);
+                    mi355_qmm_desc dn;
+                    memset(&dn, 0, sizeof(dn));
+                    dn.nseg = 1;
+                    dn.w_tiles[0] = L.eslab[1]; dn.ggml_type[0] = L.etype[1]; dn.n_rows[0] = L.erows[1];
+                    dn.moe_expert_stride[0] = L.estride[1];
+                    dn.x = in.h; dn.x_dtype = MI355_DTYPE_F32; dn.ldx = I; dn.k = I; dn.num_tokens = rows;
+                    dn.epilogue = MI355_EPI_STORE; dn.out = in.moe_y; dn.ldo = hid;
+                    dn.group_block_table = m->p_moe_tab;
+                    Mi355ScratchTurn turn(MI355_SCR_QMP_WS, reinterpret_cast<hipStream_t>(st));      // the product's sums lie there until the launch behind it has read them
+                    Mi355PromptImage sums;
+                    sums.want_parts = !tiles;
+                    sums.tiles = how.tiles;
+                    rc = mi355_internal_qmatmul_prompt(&dn, &sums, st);
+                    if (no_room(rc)) continue;
+                    RCHECK(rc);
+                    if (sums.ks > 1)
+                        RCHECK(mi355_internal_moe_combine_parts(in.xs, sums.parts, sums.ks, rows, sums.ldp, sums.scale, in.moe_w, m->p_moe_inv, B, hid, K, st));
+                    else
+                        RCHECK(mi355_moe_scatter_combine(in.xs, in.moe_y, in.moe_w, m->p_moe_inv, B, hid, K, st));
+                    break;
+                }
                 m->moe_grouped_done = true;
                 return 0;
             }

@@ -738,3 +738,27 @@ def test_moe_prompt_rows_follow_the_chunk(lib, n_expert):
         seq = [{"tokens": [t % 512 for t in range(tokens)], "block_table": list(range(1, 161))}]
         assert torch.isfinite(gm.forward_prefill(O.prepare_prompt(seq, 16))).all()
         assert M.lib.mi355_internal_moe_prompt_rows(gm.h) == 2 * cap + pad
+
+
+def test_moe_prompt_without_room_for_whole_tiles(lib):
+    """room for the images of blocks of 64 rows and not for those of whole tiles: the step goes over blocks, and over tiles again where there is room"""
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible MI355X")
+    from candle_vllm_amd import model as M
+    gm = mixture(1024, 3584, 4, 14, 8, 64)
+    gm.alloc_kv_cache(8 * 33 + 1)
+    rng = np.random.default_rng(5)
+    meta = O.prepare_prompt([{"tokens": [int(t) for t in rng.integers(0, 512, 528)], "block_table": list(range(1 + 33 * i, 34 + 33 * i))} for i in range(8)], 16)
+    gm.forward_prefill(meta)                                          # (the model's own buffers)
+    torch.cuda.synchronize()
+    rows = 64 * (2 * 8 * 528 // 64 + 4)                               # tiles: 256 * (33 + 4) of them
+    M.lib.mi355_internal_scratch_limit.argtypes = [ctypes.c_int64]
+    stream, got, kernels = torch.cuda.Stream(), [], []
+    for limit in (rows * (2 * 3584 + 14 * 32 + 8) + 8192, -1):
+        M.lib.mi355_internal_scratch_limit(limit)
+        try:
+            got.append(gm.forward_prefill(meta, stream=stream.cuda_stream).cpu().numpy().copy())
+        finally:
+            M.lib.mi355_internal_scratch_limit(-1)
+        kernels.append(M.lib.mi355_internal_last_qpw())
+    assert kernels == [-1, 21] and np.isfinite(got[0]).all() and _rel(got[0], got[1]) < 3e-3
