@@ -995,7 +995,6 @@ static int ensure_prefill_cap(Model* m, int T) {
     }
     if (m->cfg.n_expert > 1) {
         HCHECK(hipMalloc((void**)&m->p_moe_tab, (pairs / 64 + 4 * E + 8) * 8));
-        HCHECK(hipMemsetAsync(m->p_moe_xg, 0, m->p_moe_rows * m->cfg.hidden * 4, 0));   // the rows no pair lands in: finite from the start
         HCHECK(hipMalloc((void**)&m->p_moe_perm, pairs * 4));
         HCHECK(hipMalloc((void**)&m->p_moe_inv, pairs * 4));
         HCHECK(hipMalloc((void**)&m->p_moe_ids, pairs * 4));
