@@ -65,12 +65,17 @@ def test_image_for_the_next_product(T, hid, inter):
 
 
 @pytest.mark.parametrize("layout,D,rot,T", [("flash", 128, 64, 9), ("fp8", 128, 128, 32), ("paged", 72, 24, 17), ("fp8", 64, 32, 16), ("paged", 64, 64, 31)])
-def test_qkv(layout, D, rot, T):
+@pytest.mark.parametrize("bias", [False, True])
+def test_qkv(layout, D, rot, T, bias):
+    """against the general launch, and against 64 bits: q and what the cache gets, rounded to bf16 (2^-8), for an e4m3 cache once more (2^-4)"""
     H, Hkv, K, block = 6, 2, 1024, 16
     rng = np.random.default_rng(T)
-    ms = [cv.QMatMul(blocks(rng, n * D, K, t, odd=False), t, "cuda") for n, t in ((H, Q4), (Hkv, Q4), (Hkv, Q6))]
+    kinds, heads = (Q4, Q4, Q6), (H, Hkv, Hkv)
+    bs = [blocks(rng, n * D, K, t, odd=False) for n, t in zip(heads, kinds)]
+    ms = [cv.QMatMul(b, t, "cuda") for b, t in zip(bs, kinds)]
     x = torch.from_numpy(rng.normal(0, 1, (T, K)).astype(np.float32)).cuda()
     nw = torch.from_numpy(rng.uniform(0.5, 1.5, K).astype(np.float32)).cuda()
+    add = torch.from_numpy(rng.normal(0, 1, (H + 2 * Hkv) * D).astype(np.float32)).cuda()
     pos, slot = torch.from_numpy(rng.integers(0, 500, T)).cuda(), torch.from_numpy(rng.permutation(T + 64)[:T].astype(np.int64)).cuda()
     slot[::7] = -1
     ang = torch.arange(500, device="cuda").double()[:, None] * 10000.0 ** (-torch.arange(rot // 2, device="cuda").double() / (rot // 2))
@@ -83,6 +88,7 @@ def test_qkv(layout, D, rot, T):
         kc, vc = torch.zeros(n, dtype=dt, device="cuda"), torch.zeros(n, dtype=dt, device="cuda")
         d = _desc(x, ms, nw, cv.EPI_QKV_ROPE_CACHE, q.view(T, -1))
         d.out, d.ldo = None, 0
+        d.bias = add.data_ptr() if bias else None
         d.cos_table, d.sin_table, d.positions, d.slot_mapping = (v.data_ptr() for v in (cos, sin, pos, slot))
         d.q_out, d.key_cache, d.value_cache = q.data_ptr(), kc.data_ptr(), vc.data_ptr()
         d.num_heads, d.num_kv_heads, d.head_dim, d.rotary_dim, d.block_size = H, Hkv, D, rot, block
@@ -95,6 +101,20 @@ def test_qkv(layout, D, rot, T):
     for a, b, step in zip(got[0], got[1], (2.0 ** -7, 2.0 ** -3 if layout == "fp8" else 2.0 ** -7)):
         a, b = ((v.view(torch.float8_e4m3fn) if v.dtype == torch.uint8 else v).float() for v in (a, b))
         assert ((a - b).abs() <= step * torch.maximum(a.abs(), b.abs()) + 2.0 ** -9).all() and (a != b).float().mean() < 1e-2
+    xn = (x.double() * torch.rsqrt((x.double() ** 2).mean(1, keepdim=True) + 0.3) * nw.double()).float()
+    y = [(product(xn, b, t) + (a.double() if bias else 0)).view(T, -1, D) for b, t, a in zip(bs, kinds, add.split([n * D for n in heads]))]
+    c, s = ang.cos()[pos][:, None], ang.sin()[pos][:, None]
+    turned = [torch.cat([torch.stack([z[..., 0:rot:2] * c - z[..., 1:rot:2] * s, z[..., 0:rot:2] * s + z[..., 1:rot:2] * c], dim=-1).reshape(T, -1, rot), z[..., rot:]], -1) for z in y[:2]]
+    q, kc, vc = got[0]
+    blk, off, x16 = slot[slot >= 0] // block, slot[slot >= 0] % block, 16 if layout == "fp8" else 8
+    if layout == "fp8":
+        kc, vc = kc.view(torch.float8_e4m3fn).float(), vc.view(torch.float8_e4m3fn).float()
+        assert max(turned[1].abs().max(), y[2].abs().max()).item() < 448  # nothing saturates
+    kc = kc.view(-1, block, Hkv, D)[blk, off] if layout == "flash" else kc.view(-1, Hkv, D // x16, block, x16)[blk, :, :, off].reshape(-1, Hkv, D)
+    vc = vc.view(-1, block, Hkv, D)[blk, off] if layout == "flash" else vc.view(-1, Hkv, D, block)[blk, :, :, off]
+    cache_tol = TOL + 2.0 ** -8 + (2.0 ** -4 if layout == "fp8" else 0)
+    for have, want, tol in ((q.view(T, H, D), turned[0], TOL + 2.0 ** -8), (kc, turned[1][slot >= 0], cache_tol), (vc, y[2][slot >= 0], cache_tol)):
+        assert close(have, want) < tol
 
 
 @pytest.mark.parametrize("kind,N,K,silu", [(Q4, 4096, 14336, False), (Q6, 2064, 8192, False), (Q6, 32000, 2048, False), (Q4, 8192, 3072, True), (Q4, 8200, 2816, True)])
