@@ -502,17 +502,18 @@ static bool linear_flow_ok(const LinArgs& p) {
 }
 // Two row tiles per workgroup share their x, and take it where the fullest CU gets no more rows by it; a workgroup's waves and rings then follow from the units of K:
 // all of a wave's units in one ring where they fit, enough waves to keep a CU's requests going where there are more.  us on cold weights, the kernel above / this one:
-//   one tile, up to one per CU   2048 x 8192 in two ranges (8 tokens) 12.3 / 9.9, x 4096 7.9 / 6.5, x 2048 5.4 / 4.5; 4096 x 4096 11.3 / 9.6, 1024 x 512 3.7 / 3.1
-//   one tile, more               9360 x 2048 15.4 / 11.6 (1 token 13.1 / 9.8, 16 tokens 17.1 / 13.5); 12288 x 2048 16.5 / 12.1
-//   two tiles                    32000 x 2048 34.1 / 26.9; 12336 x 3072 25.6 / 18.5 (19.9 / 17.0, 30.6 / 20.5); 5120 x 5120 21.1 / 16.2
-//   gate/up pairs                16384 x 2048 19.3 / 14.7 (17.4 / 14.2); 8192 x 4096 19.8 / 16.3; 22528 x 4096 46.5 / 40.7
-// Over 154 sizes (1 .. 16 tokens, 64 .. 32000 rows, 64 .. 14336 columns) 19 % shorter on average, 1 % behind the best of ten shapes; none was slower.
+//   one tile, up to one per CU   2048 x 8192 15.9 / 14.6, x 4096 9.6 / 8.5, x 2048 6.1 / 5.2; 4096 x 4096 11.0 / 9.0, 1024 x 512 3.7 / 3.1
+//   one tile, more               9360 x 2048 15.1 / 11.7 (1 token 12.9 / 9.9, 16 tokens 16.9 / 13.7); 12288 x 2048 15.7 / 12.5
+//   two tiles                    32000 x 2048 34.9 / 28.7; 12336 x 3072 25.2 / 19.3 (20.6 / 19.3, 30.7 / 21.2); 5120 x 5120 21.0 / 18.2, 8192 x 8192 33.7 / 30.2 (32.4 / 28.9, 37.9 / 32.8)
+//   gate/up pairs                16384 x 2048 19.0 / 15.5 (17.6 / 14.8); 8192 x 4096 19.4 / 17.2; 22528 x 4096 47.4 / 42.3
+// Two tiles a workgroup and one workgroup per CU (257 .. 512 tiles): 16 waves; four waves of four units were slower than the kernel above from 6144 rows and 4096 columns on (8192 x
+// 8192 at one token 36.6).  Over 248 sizes (1 .. 16 tokens, 64 .. 32000 rows, 64 .. 14336 columns) 14 % shorter on average, none slower (profiles/layer_list_streams.txt).
 template <int B> static void linear_flow_launch(const LinArgs& p, int tiles, unsigned nz, hipStream_t st) {
     const int cus = mi355_num_cus(), units = p.K / 64, all = tiles * (int)nz;
     auto fullest = [&](int groups) { return (groups + cus - 1) / cus; };
 #define FLOW_GO(NW_, R_, PF_) linear_bf16_flow_kernel<NW_, R_, PF_, B><<<dim3((p.N + 16 * R_ - 1) / (16 * R_), 1, nz), 64 * NW_, 0, st>>>(p)
     if (B == LIN_GLU_BUILD || 2 * fullest((all + 1) / 2) <= fullest(all)) {
-        if (units > 32) FLOW_GO(4, 2, 4);
+        if (units > 32 && (B == LIN_GLU_BUILD || all > 2 * cus)) FLOW_GO(4, 2, 4);
         else if (units > 16 && (B == LIN_GLU_BUILD || all <= 2 * cus)) FLOW_GO(16, 2, 2);
         else FLOW_GO(8, 2, 2);
     } else if constexpr (B != LIN_GLU_BUILD) {
@@ -522,14 +523,17 @@ template <int B> static void linear_flow_launch(const LinArgs& p, int tiles, uns
     }
 #undef FLOW_GO
 }
-// How many waves a row tile gets and how much each has in flight.  What bounds a tile is its waves' round trips to memory, so tiles that leave compute units
-// idle get up to 16 waves; where every unit has several, fewer waves with less each, which the units take up one behind the other.  us on cold weights with
-// four waves of four steps (the only form before) / with the form chosen here, at 1, 8 and 16 tokens:
-//   up to a tile per unit   2048 x 2048 5.9 6.7 / 4.8 5.8;  2048 x 8192 21.0 22.7 / 12.2 15.4;  4096 x 4096 12.7 13.6 14.3 / 9.0 10.1 11.5;  4096 x 14336 39 42 44 / 24 30 34
-//   up to two               8192 x 1024 5.6 6.2 / 5.0 6.2;  5120 x 5120 18.2 20.1 25.5 / 15.8 20.1 25.5 (from five tokens on two steps lose: 22.5 27.3)
-//   more                    12288 x 2048 13.2 15.8 / 13.0 15.0;  32000 x 2048 29.1 36.2 / 27.6 33.4
-//   gate/up pairs           8192 x 2048 12.2 13.2 13.3 / 10.3 12.0 12.6;  16384 x 2048 17.4 19.6 / 16.9 18.4;  11264 x 4096 26.1 29.4 32.3 / 25.0 26.8 29.1
-// Below 512 columns there is nothing to split (2048 x 256 2.9 at 8 tokens with two waves of two steps, 3.0 with 16 waves), at 512 it begins to pay: 3.6 / 3.0.
+// How many waves a row tile gets and how much each has in flight, of what the kernel above leaves: f32 activations, rows that are not aligned, columns in no whole 64s.  What bounds a
+// tile is its waves' round trips to memory, so tiles that leave compute units idle get up to 16 waves; where every unit has several, fewer waves with less each, which the units
+// take up one behind the other.  us on cold weights with four waves of four steps / with the form chosen here, at 1, 8 and 16 tokens:
+//   up to a tile per unit   f32 activations 256 x 2048 8.1 7.9 8.5 / 4.9 6.7 7.8, 2048 x 2048 9.7 9.6 10.1 / 5.5 7.1 8.4, 4096 x 4096 24.5 20.8 20.7 / 12.3 14.0 16.3;
+//                           bf16 2048 x 2080 7.1 7.5 8.0 / 4.9 6.1 6.8, 2048 x 8224 22.9 23.2 25.2 / 16.1 19.2 20.9, 2048 x 2050 20.7 21.6 22.9 / 13.5 16.7 20.4
+//   up to two               f32 6144 x 2048 14.2 13.9 15.1 / 10.2 13.9 15.3; bf16 5120 x 5136 18.9 21.7 28.1 / 17.5 21.7 28.1
+//   more                    f32 16384 x 2048 18.9 21.8 26.8 / 21.3 23.1 27.5, 32000 x 2048 37.0 41.5 50.1 / 35.0 41.8 49.8; bf16 9360 x 2080 11.9 14.3 16.8 / 12.4 15.1 16.6,
+//                           32000 x 2080 29.5 35.9 41.9 / 28.5 35.4 41.7
+//   gate/up pairs (bf16)    8192 x 2080 11.2 12.1 13.0 / 10.2 11.9 12.6, 16384 x 2080 16.0 18.4 20.1 / 16.5 17.7 18.7, 11264 x 4112 31.0 35.4 39.1 / 30.3 32.8 36.9
+// Below 512 columns there is little to split: low ranks of f32 activations 4096 x 64 2.5 2.9 3.0 / 2.3 2.7 2.8, x 128 3.2 3.8 4.0 / 2.7 3.3 3.4 (2048 x 256 3.5 3.9 4.1 / 3.5 3.9 4.0);
+// at 512 it begins to pay: 2048 x 512 3.9 4.3 4.4 / 3.4 4.1 4.4.
 template <typename TA, int B> static void linear_stream_launch(const LinArgs& p, dim3 grid, hipStream_t st) {
     const int64_t tiles = (int64_t)grid.x * grid.z;
     const int cus = mi355_num_cus();
@@ -2375,10 +2379,10 @@ int mi355_hyb_linear(float* out, int32_t ldo, const void* a, int32_t a_dtype, in
     return linear_launch(out, ldo, 0, a, a_dtype, lda, 0, w, 0, bias, T, n, k, 1, dtype, stream);
 }
 // How many ranges of K a product [T, k] x [n, k] whose sums mi355_internal_hyb_norm_add_parts takes is made in, of at most `most`: few row tiles, each walking all of
-// K, leave the chip idle.  us of product and norm, one range / the picked ones (bf16 unless said): 8 tokens 2048 x 8192 17.9 / 12.3, x 4096 11.8 / 10.1,
-// 3072 x 8192 20.3 / 17.6, 4096 x 14336 32.4 / 27.9; 48 tokens 2048
+// K, leave the chip idle.  us of product and norm, one range / the picked ones (bf16 unless said): 8 tokens 2048 x 8192 17.4 / 12.3, x 4096 11.6 / 9.7,
+// 3072 x 8192 18.3 / 17.3, 4096 x 14336 30.5 / 29.6; 48 tokens 2048
 // x 8192 55 / 17, 164 53 / 21, 400 49 / 28, x 2048 15.3 / 10.8 at 48; 3072 x 8192 at 256 54 / 32; f32 8 tokens 2048 x 8192 34 / 25, 100 tokens 106 / 52.  To 16 tokens, bf16: up to two
-// row tiles per unit, 1024 columns a range (to 4 tokens one tile: 1 token 4096 x 8192 18.4 in one range, 20.4 in two); f32 up to two; beyond: the rounds of the tiles
+// row tiles per unit, 1024 columns a range (to 4 tokens one tile: 1 token 4096 x 8192 19.1 in one range or two, 21.2 in four); f32 up to two; beyond: the rounds of the tiles
 // (gt_pick) and what the sums cost the norm, over 150 sizes 1 % behind the best number.
 int32_t mi355_internal_hyb_parts(int32_t T, int32_t n, int32_t k, int32_t dtype, int32_t most) {
     const int cus = mi355_num_cus(), top = std::min(most, PARTS_MOST);

@@ -115,7 +115,8 @@ def test_linear_forms(lib, dtype, T, n, k, skew):
 # whole 64-column units on aligned rows, by the shape that takes them: one row tile per workgroup (four waves, sixteen; eight and sixteen where there are more tiles
 # than units of the chip) and two (eight waves, sixteen, four), with no unit for most waves, one to three left for a ring, and rows that fill no tile
 @pytest.mark.parametrize("T,n,k", [(8, 250, 64), (1, 17, 320), (16, 4090, 1984), (3, 1000, 2112), (8, 48, 4288), (5, 50, 6528), (4, 8323, 448), (8, 8320, 1216), (2, 9600, 2112),
-                                   (8, 4805, 128), (9, 4800, 1088), (8, 12800, 1152), (1, 4161, 2240), (12, 4170, 2560)])
+                                   (8, 4805, 128), (9, 4800, 1088), (8, 12800, 1152), (1, 4161, 2240), (12, 4170, 2560),
+                                   (3, 12400, 2240)])
 def test_bf16_streams_by_units(lib, T, n, k):
     """against 64 bits, within (k + 2) 2^-24 sum |a w| of any order; a NaN row leaves the others alone, and columns beyond n are not touched"""
     _gpu()
