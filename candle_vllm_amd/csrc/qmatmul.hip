@@ -2275,8 +2275,8 @@ static float qpg_split_us(int T, int slots4, int slots6, int nkb, int ks) {
 }
 // The same on Q6_K tiles of 256 x 128, one workgroup per CU: a weight is unpacked once per 256 tokens instead of per 64 (the 64 x 256 tile of Q6_K is bound by that: 4.3 us a k-block
 // against 2.5 of a Q4_K workgroup that shares its CU).  us with the second launch, 64 x 256 tiles / these, where it picks them: 14336 -> 4096 at 193 tokens 77 / 60,
-// 500 136 / 100, 1000 249 / 176; 8192 -> 3072 at 500 84 / 59; 4096 -> 4096 at 700 78 / 61.  70 sizes of 193 .. 1024 tokens 0.66 .. 1.0 of their time, 0.81 on
-// average.  Up to 192 tokens a quarter of a tile or more is empty and the image has no rows for it; Q4_K ranges stay on 64 x 256 tiles (500 tokens of 14336 -> 4096:
+// 500 136 / 100, 1000 249 / 176; 8192 -> 3072 at 500 84 / 59; 4096 -> 4096 at 700 78 / 61.  70 sizes of 193 .. 1024 tokens 0.64 .. 1.0 of their time, 0.80 on
+// average (profiles/q6k_prompt_ranges.txt).  Up to 192 tokens a quarter of a tile or more is empty and the image has no rows for it; Q4_K ranges stay on 64 x 256 tiles (500 tokens of 14336 -> 4096:
 // 75 us, by estimate 87 here).
 static float qpw_split_us(int T, int n_slots, int nkb, int ks) {
     return 8.f + (float)T * (float)(n_slots * 16) * 1e-6f * (2.6f + 1.25f * (float)ks) +
